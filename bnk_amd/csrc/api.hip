@@ -454,9 +454,9 @@ int bnk_init(int device_ordinal, bnk_ctx **out)
     if ((e = hipMemset(ctx->d_tally, 0, TALLY_SLOTS * TALLY_LANES * 8)) != hipSuccess) return bail("hipMemset", e);
     if ((e = hipEventCreateWithFlags(&ctx->ev_noalloc, hipEventDisableTiming)) != hipSuccess)
         return bail("hipEventCreate", e);
-    if ((e = hipHostMalloc((void **)&ctx->h_status, 64, hipHostMallocDefault)) != hipSuccess)
+    if ((e = hipHostMalloc((void **)&ctx->h_status, 128, hipHostMallocDefault)) != hipSuccess)
         return bail("hipHostMalloc", e);
-    memset(ctx->h_status, 0, 64);
+    memset(ctx->h_status, 0, 128);
     if (const char *ws = getenv("BNK_WAIT_SYNC")) ctx->wait_sync_only = ws[0] != '\0' && ws[0] != '0';
     if ((e = hipHostGetDevicePointer((void **)&ctx->d_status, ctx->h_status, 0)) != hipSuccess)
         return bail("hipHostGetDevicePointer", e);
@@ -472,6 +472,8 @@ int bnk_init(int device_ordinal, bnk_ctx **out)
     }
     ctx->filter = filter_create(ctx->stream, prop.multiProcessorCount);
     if (!ctx->filter) return bail("filter state", hipErrorOutOfMemory);
+    ctx->filter->record = reinterpret_cast<uint64_t *>(ctx->h_status + STATUS_NOTE_RECORD);
+    ctx->filter->d_record = reinterpret_cast<uint64_t *>(ctx->d_status + STATUS_NOTE_RECORD);
     if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return bail("hipStreamSynchronize", e);
     ctx->alive = true;
     *out = ctx;

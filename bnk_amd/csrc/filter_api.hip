@@ -10,7 +10,7 @@ using namespace bnk;
 namespace bnk {
 
 static hipError_t flow_table_alloc(uint32_t cap, DevBuf &slots, DevBuf &counters, DevBuf &present,
-                                   DevBuf &present_small, FlowTableDev &ft, hipStream_t s)
+                                   DevBuf &present_small, DevBuf &list, FlowTableDev &ft, hipStream_t s)
 {
     const size_t n = (size_t)cap * FLOW_REGIONS;
     // the table is kept under half full, so 8 * cap bits see at most one key per 16 bits
@@ -20,8 +20,9 @@ static hipError_t flow_table_alloc(uint32_t cap, DevBuf &slots, DevBuf &counters
     if ((e = counters.reserve(FLOW_COUNTERS * 4)) != hipSuccess) return e;
     if ((e = present.reserve(bits / 8)) != hipSuccess) return e;
     if ((e = present_small.reserve(SMALL_BITS / 8)) != hipSuccess) return e;
+    if ((e = list.reserve((size_t)cap / 2 * 4)) != hipSuccess) return e;
     ft.present_small = present_small.as<uint32_t>();
-    ft.small_ok = 1;
+    ft.list = list.as<uint32_t>();
     ft.slots = slots.as<FlowSlotMem>();
     ft.counters = counters.as<uint32_t>();
     ft.present = present.as<uint32_t>();
@@ -82,7 +83,7 @@ FilterState *filter_create(hipStream_t s, int cu_count)
     HostRuleIndex h;
     std::string err;
     build_rule_index(nullptr, 0, h, err);
-    if (flow_table_alloc(FLOW_CAP_INITIAL, f->slots, f->counters, f->present, f->present_small, f->flows, s) != hipSuccess ||
+    if (flow_table_alloc(FLOW_CAP_INITIAL, f->slots, f->counters, f->present, f->present_small, f->list, f->flows, s) != hipSuccess ||
         upload_rule_index(f, h, s) != hipSuccess) {
         filter_destroy(f);
         return nullptr;
@@ -102,45 +103,53 @@ void filter_destroy(FilterState *f)
 namespace bnk {
 
 // Makes room for n_new more distinct flows: open addressing stays below half
-// full per region, growing (and dropping tombstones) when it would not.
+// full per region, growing (and dropping tombstones) when it would not.  Most
+// packets of a note batch belong to flows the table has, so the bound on claimed
+// slots outgrows their number by a batch per call; the words the launches leave
+// behind bring it back down.  (Reading the counter from the device instead waits
+// for everything enqueued, every few calls where batches are large.)
 int flows_reserve(bnk_ctx *ctx, uint32_t n_new)
 {
     FilterState *f = ctx->filter;
     const uint64_t half = f->flows.cap / 2;
-    if (f->claimed_upper + n_new <= half) {
+    auto take = [&]() {
         f->claimed_upper += n_new;
-        f->flows.small_ok = f->claimed_upper <= SMALL_KEYS_MAX;
+        f->reserved += n_new;
+        f->reserved_at[++f->note_seq & 63u] = f->reserved;
         return BNK_OK;
+    };
+    if (f->record) {
+        const uint64_t rec = __atomic_load_n(f->record, __ATOMIC_RELAXED);
+        const uint32_t seq = (uint32_t)(rec >> 32);
+        if ((int32_t)(seq - f->table_seq) >= 0 && f->note_seq - seq < 64u)
+            f->claimed_upper = std::min(f->claimed_upper, (rec & 0xFFFFFFFFu) + f->reserved - f->reserved_at[seq & 63u]);
     }
+    if (f->claimed_upper + n_new <= half) return take();
     uint32_t c[FLOW_COUNTERS];
     HIPCHK(ctx, hipMemcpyAsync(c, f->flows.counters, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     f->claimed_upper = c[FLOW_CLAIMED];
-    if (f->claimed_upper + n_new <= half) {
-        f->claimed_upper += n_new;
-        f->flows.small_ok = f->claimed_upper <= SMALL_KEYS_MAX;
-        return BNK_OK;
-    }
-    uint64_t need = 4ull * ((uint64_t)c[FLOW_LIVE] + n_new); // at most a quarter full afterwards
+    if (f->claimed_upper + n_new <= half) return take();
+    uint64_t need = 4ull * ((uint64_t)(c[FLOW_LIVE] - c[FLOW_GONE]) + n_new); // at most a quarter full afterwards
     uint64_t cap = FLOW_CAP_INITIAL;
     while (cap < need) cap *= 2;
     if (cap > FLOW_CAP_MAX) return fail(ctx, BNK_E_NOMEM, "flow table would exceed its maximum size");
-    DevBuf ns, nc, np, nps;
+    DevBuf ns, nc, np, nps, nl;
     FlowTableDev nt{};
-    hipError_t e = flow_table_alloc((uint32_t)cap, ns, nc, np, nps, nt, ctx->stream);
+    hipError_t e = flow_table_alloc((uint32_t)cap, ns, nc, np, nps, nl, nt, ctx->stream);
     if (e == hipSuccess)
         e = launch_flow_rehash(f->flows, nt, ctx->d_status, f->max_blocks, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) {
-        ns.release(); nc.release(); np.release(); nps.release();
+        for (DevBuf *b : {&ns, &nc, &np, &nps, &nl}) b->release();
         return fail_hip(ctx, "flow table growth", e);
     }
-    f->slots.release(); f->counters.release(); f->present.release(); f->present_small.release();
-    f->slots = ns; f->counters = nc; f->present = np; f->present_small = nps;
+    for (DevBuf *b : {&f->slots, &f->counters, &f->present, &f->present_small, &f->list}) b->release();
+    f->slots = ns; f->counters = nc; f->present = np; f->present_small = nps; f->list = nl;
     f->flows = nt;
-    f->claimed_upper = (uint64_t)c[FLOW_LIVE] + n_new;
-    f->flows.small_ok = f->claimed_upper <= SMALL_KEYS_MAX;
-    return BNK_OK;
+    f->claimed_upper = c[FLOW_LIVE] - c[FLOW_GONE];
+    f->table_seq = f->note_seq;
+    return take();
 }
 
 } // namespace bnk
@@ -192,7 +201,7 @@ int run_staged(bnk_ctx *ctx, bool check, FilterArgs &a, uint8_t *h_verdict, uint
 {
     FilterState *f = ctx->filter;
     if (!check) {
-        HIPCHK(ctx, launch_filter_note(a, f->max_blocks, f->claimed_upper > 4096, ctx->stream));
+        HIPCHK(ctx, launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
     } else if (h_verdict) {
         // CheckInbound reports nothing through the status word
         a.verdict = ctx->pin.dev(h_verdict);
@@ -220,6 +229,8 @@ void base_args(bnk_ctx *ctx, uint32_t n, int64_t now_ns, FilterArgs *a)
     a->status = ctx->d_status;
     a->rules = ctx->filter->ridx;
     a->flows = ctx->filter->flows;
+    a->record = ctx->filter->d_record;
+    a->record_seq = ctx->filter->note_seq;
 }
 
 int check_device_layout(bnk_ctx *ctx, const bnk_batch *b)
@@ -269,7 +280,7 @@ int filter_batch(bnk_ctx *ctx, bool check, const bnk_batch *pkts, int64_t now_ns
             *counted = true;
         }
         HIPCHK(ctx, check ? launch_filter_check(a, f->max_blocks, ctx->stream)
-                          : launch_filter_note(a, f->max_blocks, f->claimed_upper > 4096, ctx->stream));
+                          : launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
         return BNK_OK;
     }
     Span span;
@@ -449,7 +460,7 @@ int bnk_filter_flow_count(bnk_ctx *ctx, uint32_t *count)
     HIPCHK(ctx, hipMemcpyAsync(c, ctx->filter->flows.counters, sizeof c, hipMemcpyDeviceToHost,
                                ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    *count = c[FLOW_LIVE];
+    *count = c[FLOW_LIVE] - c[FLOW_GONE];
     return BNK_OK;
     BNK_API_CATCH(ctx)
 }

@@ -8,7 +8,14 @@ namespace bnk {
 
 constexpr uint32_t FLOW_REGIONS = 6;     // protocol class (3) x top address bit (2)
 constexpr int64_t FLOW_TOMB = INT64_MIN; // expiry of a deleted (or never used) slot
-enum : uint32_t { FLOW_LIVE = 0, FLOW_CLAIMED = 1, FLOW_SWEEP = 2, FLOW_COUNTERS = 4 };
+// Words of FlowTableDev::counters: entries in the map, slots ever claimed; since the last note
+// launch, whether a sweep ran and how many entries it deleted (FLOW_LIVE still counts those);
+// and two int64, no entry of the map expires before FLOW_MIN_EXP (0: nothing known), or before
+// FLOW_NEXT_EXP if a sweep ran.
+enum : uint32_t {
+    FLOW_LIVE = 0, FLOW_CLAIMED = 1, FLOW_SWEPT = 2, FLOW_GONE = 3, FLOW_MIN_EXP = 4, FLOW_NEXT_EXP = 6, FLOW_COUNTERS = 8
+};
+constexpr int64_t FLOW_TTL_LEAST = 30000000000LL; // filter.go:108-117: nothing is stored for less
 
 // One 16-byte slot, so a probe is a single memory transaction.
 struct FlowSlotMem {
@@ -18,7 +25,9 @@ struct FlowSlotMem {
 
 struct FlowTableDev {
     FlowSlotMem *slots; // [FLOW_REGIONS * cap]
-    uint32_t *counters; // [FLOW_COUNTERS]: entries in the map, slots ever claimed, sweep flag
+    uint32_t *counters; // [FLOW_COUNTERS]
+    uint32_t *list;     // [cap / 2] the slots ever claimed, in the order they were: what walks the
+                        // whole map walks this instead of FLOW_REGIONS * cap slots
     uint32_t *present;  // [present_bits / 32] one hashed bit per key ever stored in this table:
                         // small enough to stay in L2, it answers most misses without a probe
     uint32_t *present_small; // [SMALL_BITS / 32] two hashed bits per key (a Bloom filter) in a
@@ -27,7 +36,6 @@ struct FlowTableDev {
                              // leaves the CU for a packet without a flow
     uint32_t cap;       // slots per region, a power of two
     uint32_t present_mask; // present_bits - 1 (a power of two)
-    uint32_t small_ok;  // host's call: few enough keys for present_small to be worth reading
 };
 
 constexpr uint32_t SMALL_BITS = 44u * 1024u * 8u; // 44 KiB: leaves 36 KiB of a workgroup's 80 for cut points
@@ -84,7 +92,10 @@ struct FilterArgs {
                           // packet reaching beyond it is not read, fails the parse and
                           // raises STATUS_BOUNDS.  0: the host has checked the layout
     uint32_t trim;        // bytes at the end of each packet that are not payload
-    uint32_t small_in_lds; // set by the launcher: presence questions go to the folded bitmap in LDS
+    uint32_t small_in_lds; // set by the launcher: there is LDS for present_small (a launch reads it
+                          // while the table has seen at most SMALL_KEYS_MAX keys)
+    uint64_t *record;     // note only: pinned host word that receives record_seq - 1 << 32 | slots
+    uint32_t record_seq;  // claimed by the batches up to that number, or more (see flows_reserve)
     RuleIndexDev rules;
     FlowTableDev flows;
 };
@@ -94,10 +105,9 @@ hipError_t launch_flow_clear(FlowSlotMem *p, uint32_t n, hipStream_t s);
 hipError_t launch_fill_u8(uint8_t *p, uint32_t n, uint8_t v, hipStream_t s);
 hipError_t launch_filter_check(const FilterArgs &a, uint32_t max_blocks, hipStream_t s);
 // inserts, then the reference's conditional expiry sweep
-// may_sweep: the table may hold more than 4096 entries after this batch (the
-// host's upper bound on claimed slots says so); otherwise the expiry sweep
-// cannot fire and its two launches are left out.
-hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, bool may_sweep, hipStream_t s);
+// claimed_upper: the host's upper bound on claimed slots.  Up to 4096 the
+// sweep cannot fire and its launch is left out.
+hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
 hipError_t launch_flow_rehash(const FlowTableDev &from, const FlowTableDev &to, uint32_t *status,
                               uint32_t max_blocks, hipStream_t s);
 

@@ -455,7 +455,9 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             fa.n = hi - lo;
             fa.rules = f->ridx;
             fa.flows = f->flows;
-            HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->claimed_upper > 4096, ctx->stream));
+            fa.record = f->d_record;
+            fa.record_seq = f->note_seq;
+            HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->claimed_upper, ctx->stream));
         }
         if (fits) {
             AeadArgs se{};

@@ -122,6 +122,50 @@ def test_duplicates_in_one_batch_and_sweep_threshold():
     ctx.close()
 
 
+@pytest.mark.parametrize("seed,n_flows", [(1, 4500), (2, 20000)])
+def test_sweep_with_a_wandering_clock(seed, n_flows):
+    """Device-resident note and check batches around and above 4096 entries, the clock going
+    forwards and backwards across both lifetimes: the sweep deletes exactly what the reference's
+    does in every round, also where nothing can have expired, and the table grows (and moves)
+    under way."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(seed)
+    ctx = lib.Context(0)
+    ora = O.Filter()
+    ctx.filter_set_rules([])
+    ora.set_rules([])
+    proto = np.where(rng.random(n_flows) < 0.5, 6, 17).astype(np.uint32)
+    remote = (W.CGNAT_BASE | rng.integers(0, 1 << 22, n_flows)).astype(np.uint32)
+    me = np.full(n_flows, W.CGNAT_BASE | 1, np.uint32)
+    lport, rport = (rng.integers(1, 65536, n_flows).astype(np.uint32) for _ in range(2))
+    out = W.header_records(proto, me, remote, lport, rport)
+    back = W.header_records(proto, remote, me, rport, lport)
+    now = FC.T0
+    for round_no in range(30):
+        now += int(rng.integers(-40, 60)) * FC.SEC + int(rng.integers(-1, 2))
+        for recs, check in ((out, False), (back, True)):
+            m = int(rng.integers(1, n_flows))
+            pick = np.ascontiguousarray(recs[rng.integers(0, n_flows, m)])
+            buf, off, lens = _flat(pick)
+            dev = torch.from_numpy(buf).cuda()
+            torch.cuda.synchronize()
+            b = lib.make_batch(dev, buf.nbytes, m, lib.MEM_DEVICE, stride=32, length=28)
+            if check:
+                got = torch.zeros(m, dtype=torch.uint8, device="cuda")
+                torch.cuda.synchronize()
+                ctx.filter_check_inbound(b, now, got)
+                ctx.sync()
+                assert np.array_equal(got.cpu().numpy(), ora.check_inbound_batch(buf, off, lens, now)), round_no
+            else:
+                ctx.filter_note_outbound(b, now)
+                ora.note_outbound_batch(buf, off, lens, now)
+            assert ctx.filter_flow_count() == ora.flow_count(), round_no
+    assert ctx.filter_flows() == ora.flows()
+    ctx.close()
+
+
 def test_rules_too_wide_to_expand_and_rule_edges():
     """Thousands of /0 rules over thousands of /32 cut points exceed the
     expansion budget: those rules are scanned linearly instead; verdicts must

@@ -8,6 +8,7 @@
 // one-time key; data uses blocks 1..; the MAC covers the zero-padded
 // ciphertext and one length block.
 #include "aead_lane.hpp"
+#include <math.h>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -271,6 +272,9 @@ BNK_DEV void crypt_tail_lds(Poly32 &mac, const uint32_t (&x)[16], int j, uint8_t
 struct Head {
     uint4 c0, c1;
     bool on; // the launch writes records (the same for every lane)
+    uint4 *keep0; // a run of a packet: where in LDS it leaves them instead (16 bytes, and 8 more),
+    uint2 *keep1; // and the second half of the one-time key
+    uint4 *keep_pad;
 };
 
 BNK_DEV void capture_head(Head &h, const uint8_t *c0, const uint8_t *c1)
@@ -369,10 +373,18 @@ BNK_DEV void body_generic(uint8_t *tile, uint32_t lane, const uint8_t *src, uint
 // 124 bytes, so a piece enters the ring one step later than otherwise: just
 // before it is needed, after the line that still holds the end of the piece
 // two before it has left.
-template <bool OPEN, bool ALIGNED, bool SHIFT = false>
+//
+// RUNS: the lane goes through a run of a packet instead of a whole one (see
+// aead_split_kernel).  Positions then count from src and dst, where keystream block
+// blk0 applies; a run begins with an even block, so the first one of a packet begins
+// 64 bytes before it, at the key block, with `lead` = 4 cells that are not the
+// packet's.  key_lane: the lane of the packet's first run, which hands out the
+// one-time key.
+template <bool OPEN, bool ALIGNED, bool SHIFT = false, bool RUNS = false>
 BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_t *dst, uint32_t len,
                         uint32_t len_in, const uint8_t *safe, const uint32_t (&k)[8], uint32_t n1, uint32_t n2,
-                        Poly32 &mac, uint32_t (&x)[16], Head &head)
+                        Poly32 &mac, uint32_t (&x)[16], Head &head, uint32_t blk0 = 0, uint32_t lead = 0,
+                        uint32_t key_lane = 0)
 {
     // len_in <= len: the packet's bytes in memory; the up to 15 between the two
     // are padding that counts as zeros (a sealing WireGuard launch; otherwise
@@ -392,24 +404,27 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
     uint8_t *cdst[8];
     uint32_t cfirst[8], cend[8], cend_ld[8];
     int32_t pofs[8];
-    uint32_t whole[8];
+    uint32_t before[8], whole[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) {
         const int owner = 8 * q + (int)(lane >> 3);
         csrc[q] = reinterpret_cast<const uint8_t *>(shfl64((uint64_t)(uintptr_t)(src - skew), owner)) + 16u * sub;
         cdst[q] = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)(dst - skew), owner)) + 16u * sub;
-        cfirst[q] = (uint32_t)__shfl((int)c0, owner, 64);
+        const uint32_t oc0 = (uint32_t)__shfl((int)c0, owner, 64);
+        const uint32_t olead = RUNS ? (uint32_t)__shfl((int)lead, owner, 64) : 0u;
+        cfirst[q] = oc0 + olead;
         const uint32_t olen = (uint32_t)__shfl((int)len, owner, 64);
-        cend[q] = cfirst[q] + (olen >> 4);
+        cend[q] = oc0 + (olen >> 4);
         // (a cell that is not aligned may reach into the next page: only aligned ones
         // are fetched beyond the packet's last byte)
-        cend_ld[q] = cfirst[q] + ((olen + (ALIGNED ? 15u : 0u)) >> 4);
+        cend_ld[q] = oc0 + ((olen + (ALIGNED ? 15u : 0u)) >> 4);
         if (SHIFT) {
             const uint64_t od = shfl64((uint64_t)(uintptr_t)dst, owner);
             const uint32_t skd = (uint32_t)od & 127u;
             cdst[q] = reinterpret_cast<uint8_t *>(od - skd) + 16u * sub; // my cell of the line holding the packet's first byte
             pofs[q] = (int32_t)(16u * sub) - (int32_t)skd;               // where that cell starts within the packet
-            whole[q] = olen & ~15u;                                      // bytes of it that go through the ring
+            before[q] = 16u * olead;                                     // bytes that are not the packet's
+            whole[q] = (olen & ~15u) - before[q];                        // bytes of it that go through the ring
         }
     }
     uint32_t maxsteps = steps;
@@ -422,7 +437,7 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
 
     // Lines m_lo <= m < m_hi lie wholly inside every packet of the wave: those
     // move without per-cell bounds checks.
-    uint32_t maxc0 = c0, minend = c0 + ncell;
+    uint32_t maxc0 = c0 + lead, minend = c0 + ncell;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
         const uint32_t a = (uint32_t)__shfl_xor((int)maxc0, off, 64);
@@ -430,7 +445,7 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         maxc0 = a > maxc0 ? a : maxc0;
         minend = b < minend ? b : minend;
     }
-    const uint32_t m_lo = __builtin_amdgcn_readfirstlane(maxc0) ? 1u : 0u;
+    const uint32_t m_lo = ALIGNED || RUNS ? (__builtin_amdgcn_readfirstlane(maxc0) + 7u) >> 3 : 0u;
     const uint32_t m_hi = __builtin_amdgcn_readfirstlane(minend) >> 3;
 
     // Lines are fetched one iteration ahead into registers (issue), so the
@@ -474,7 +489,7 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
     } while (0)
 #define BNK_PUT_SHIFT(q, m)                                                                 \
     do {                                                                                    \
-        const uint32_t at_##q = (uint32_t)(pofs[q] + (int32_t)(128u * (m)));                \
+        const uint32_t at_##q = (uint32_t)(pofs[q] + (int32_t)(128u * (m))) - before[q];    \
         uint8_t *const to_##q = cdst[q] + 128u * (m);                                       \
         if (at_##q < whole[q] && at_##q + 12u < whole[q]) st16a_out(to_##q, out##q);        \
         else {                                                                              \
@@ -500,22 +515,91 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
 
     uint8_t *row = tile + lane * RING_ROW;
     BNK_ISSUE_LINE(0u);
+    if (RUNS && !SHIFT) {
+        // (a run has few steps: its second line flies beside the first, in the registers that
+        // finished lines leave through)
+#define BNK_ISSUE2(q, m) out##q = BNK_LD(BNK_INSIDE_LD(q, m) ? csrc[q] + 128u * (m) : safe)
+#define BNK_COMMIT2(q, m) if (BNK_INSIDE_LD(q, m)) *BNK_SLOT(q, m) = out##q
+        BNK_EIGHT(BNK_ISSUE2, 1u);
+    }
     // keystream block 0 (the Poly1305 key) is computed while the first line flies
-    chacha_block(k, 0, n1, n2, x);
-    mac.init(x);
     ChachaShared shared;
-    chacha_shared(k, n1, n2, shared);
     // (with SHIFT a piece enters the ring, and the next one starts flying, one step later)
     constexpr uint32_t AHEAD = SHIFT ? 0u : 1u;
-    if (!SHIFT) {
+    // RUNS: a step's cells with its two keystream blocks, in one form for all of them: the lanes
+    // of a wave begin and end at different places, and a second form for the first or last step
+    // would be run behind the other.
+    auto run_step = [&](uint32_t s, const uint32_t (&ks0)[16], const uint32_t (&ks1)[16]) __attribute__((always_inline)) {
+        auto cell = [&](uint32_t kc) { return reinterpret_cast<uint4 *>(row + (((c0 + kc) & 15u) << 4)); };
+        // the packet's last 1-15 bytes end in this step
+        const uint32_t kt = len >> 4;
+        const bool tail = (len & 15u) != 0u && (len >> 7) == s;
+        if (!ALIGNED && tail) // (their cell has not come into LDS)
+            *cell(kt) = ld_partial(src + 16u * kt, len_in > 16u * kt ? len_in - 16u * kt : 0u);
+        uint4 cur = *cell(8u * s);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint32_t kc = 8u * s + j;
+            uint4 nxt = cur;
+            if (j < 7) nxt = *cell(kc + 1u);
+            if (kc >= lead && 16u * kc < len) {
+                const uint32_t (&ks)[16] = j < 4 ? ks0 : ks1;
+                uint4 v = cur;
+                const uint32_t m_in = len_in > 16u * kc ? len_in - 16u * kc : 0u, m_out = len - 16u * kc;
+                if (m_in < 16u) v = keep_bytes(v, m_in);
+                uint4 o = make_uint4(v.x ^ ks[4 * (j & 3)], v.y ^ ks[4 * (j & 3) + 1], v.z ^ ks[4 * (j & 3) + 2],
+                                     v.w ^ ks[4 * (j & 3) + 3]);
+                if (m_out < 16u) o = keep_bytes(o, m_out);
+                if (OPEN) mac.block(v.x, v.y, v.z, v.w);
+                else mac.block(o.x, o.y, o.z, o.w);
+                *cell(kc) = o;
+            }
+            cur = nxt;
+        }
+        if (tail) st_partial(dst + 16u * kt, *cell(kt), len & 15u);
+        // (see the same place in the other form)
+        if (SHIFT && (s & 1u) == 0u) *reinterpret_cast<uint4 *>(row + 256) = *reinterpret_cast<const uint4 *>(row);
+    };
+    if (RUNS) {
+        // the pair of the first step, which in the packet's first run holds the one-time key
+        uint32_t y[16];
+        chacha_block2(k, blk0, n1, n2, x, y);
+        uint32_t otk[16];
+#pragma unroll
+        for (int w = 0; w < 8; w++) otk[w] = w < 4 ? (uint32_t)__shfl((int)x[w], (int)key_lane, 64) : 0u;
+        mac.init(otk);
+        if (lead != 0u) *head.keep_pad = make_uint4(x[4], x[5], x[6], x[7]);
         BNK_COMMIT_LINE(0u);
-        BNK_ISSUE_LINE(1u);
+        if (SHIFT) {
+            BNK_ISSUE_LINE(1u);
+        } else {
+            BNK_EIGHT(BNK_COMMIT2, 1u);
+            if (2u <= maxsteps) BNK_ISSUE_LINE(2u);
+        }
+#undef BNK_ISSUE2
+#undef BNK_COMMIT2
+        wave_sync();
+        if (steps != 0u) run_step(0u, x, y);
+        if (OPEN && head.on && lead != 0u) {
+            // (the plaintext's first cells, for the packet's record; see SplitPacket)
+            *head.keep0 = *reinterpret_cast<const uint4 *>(row + (((c0 + 4u) & 15u) << 4));
+            *head.keep1 = *reinterpret_cast<const uint2 *>(row + (((c0 + 5u) & 15u) << 4));
+        }
+        wave_sync();
+    } else {
+        chacha_block(k, 0, n1, n2, x);
+        mac.init(x);
+        chacha_shared(k, n1, n2, shared);
+        if (!SHIFT) {
+            BNK_COMMIT_LINE(0u);
+            BNK_ISSUE_LINE(1u);
+        }
     }
     // iteration s: line s-1 (complete since the step before) leaves the ring,
     // line s+1 enters it, line s+2 starts flying, line s-1 goes to memory,
     // packet bytes [128s, 128s+128) are processed; the extra last iteration
     // only writes back the final line
-    for (uint32_t s = 0; s <= maxsteps + 1; s++) {
+    for (uint32_t s = RUNS ? 1u : 0u; s <= maxsteps + 1; s++) {
         if (s >= 1) {
             if (SHIFT) BNK_EIGHT(BNK_TAKE_SHIFT, s - 1);
             else BNK_EIGHT(BNK_TAKE, s - 1);
@@ -535,14 +619,19 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         if (s >= 1) {
             if (SHIFT) {
                 // whole lines of every packet of the wave: not the first, and ending within its whole cells
-                if (s - 1 >= 1u && s - 1 < m_hi) BNK_EIGHT(BNK_PUT_SHIFT_ALL, s - 1);
+                if (s - 1 >= m_lo + 1u && s - 1 < m_hi) BNK_EIGHT(BNK_PUT_SHIFT_ALL, s - 1);
                 else BNK_EIGHT(BNK_PUT_SHIFT, s - 1);
             } else if (s - 1 >= m_lo && s - 1 < m_hi) BNK_EIGHT(BNK_PUT_ALL, s - 1);
             else BNK_EIGHT(BNK_PUT, s - 1);
         }
         wave_sync();
         if (s < steps) {
-            if (8u * s + 8u <= ncell_in) {
+            if (RUNS) {
+                uint32_t y[16];
+                // (what the packet's blocks share of the first round is not kept: 13 registers)
+                chacha_block2(k, blk0 + 2u * s, n1, n2, x, y);
+                run_step(s, x, y);
+            } else if (8u * s + 8u <= ncell_in) {
                 // all eight cells of this step are whole cells of the packet: its two
                 // keystream blocks side by side
                 uint32_t y[16];
@@ -585,11 +674,11 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
                     }
                 }
             }
-            if (OPEN && s == 0) capture_head(head, row + (c0 << 4), row + (((c0 + 1u) & 15u) << 4));
+            if (OPEN && !RUNS && s == 0) capture_head(head, row + (c0 << 4), row + (((c0 + 1u) & 15u) << 4));
             // SHIFT: a step that has written the ring's first cell (every second one: the ring
             // holds a packet from its first byte) repeats it behind the ring's end
             static_assert(!SHIFT || RING_ROW >= 256u + 16u, "no room behind the ring for the copy of its first cell");
-            if (SHIFT && (s & 1u) == 0u)
+            if (SHIFT && !RUNS && (s & 1u) == 0u)
                 *reinterpret_cast<uint4 *>(row + 256) = *reinterpret_cast<const uint4 *>(row);
         }
         wave_sync();
@@ -736,6 +825,46 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
     }
 }
 
+// The window pass's sort key of packet i: its sender, 0xFFFFFFFF when the packet is
+// not authentic.
+BNK_DEV void replay_key(const AeadArgs &a, uint32_t i, uint32_t sender)
+{
+    if (!a.wg.replay_keys) return;
+    if (a.wg.replay_index_bits) {
+        a.wg.replay_keys[i - a.first] = wg_replay_pack(sender, i - a.first, a.wg.replay_index_bits);
+    } else {
+        a.wg.replay_keys[i - a.first] = sender;
+        a.wg.replay_idx[i - a.first] = i - a.first;
+    }
+}
+
+// What WireGuard does with a datagram whose tag has been checked: keepalive, IP
+// version, the trim to the IP header's total length, the sender's allowed prefix.
+// c0: the first 16 bytes of the plaintext, kept when they went through the cipher.
+BNK_DEV void decap_result(const AeadArgs &a, uint32_t i, bool have, bool reject, uint32_t len, const uint4 c0,
+                          uint32_t pr)
+{
+    uint32_t res = BNK_WG_OK, out_len = 0;
+    const uint32_t version = (c0.x >> 4) & 0xFu;
+    if (!have || reject) res = BNK_WG_AUTH_FAIL; // (no packet here: it reached beyond the output arena)
+    else if (len == 0u) res = BNK_WG_KEEPALIVE;
+    else if (len < 16u) res = BNK_WG_BAD_IP; // too short for either header
+    else if (version == 4u) {
+        const uint32_t total = __builtin_bswap32(c0.x) & 0xFFFFu;
+        const uint2 al = a.wg.allowed[pr];
+        if (len < 20u || total > len || total < 20u) res = BNK_WG_BAD_IP;
+        else if ((__builtin_bswap32(c0.w) & al.y) != (al.x & al.y)) res = BNK_WG_NOT_ALLOWED;
+        else out_len = total;
+    } else if (version == 6u) {
+        // peers own IPv4 addresses only
+        const uint32_t total = (__builtin_bswap32(c0.y) >> 16) + 40u;
+        res = (len < 40u || total > len) ? BNK_WG_BAD_IP : BNK_WG_NOT_ALLOWED;
+    } else res = BNK_WG_BAD_IP;
+    a.wg.result[i] = (uint8_t)res;
+    a.wg.out_len[i] = out_len;
+    replay_key(a, i, res != BNK_WG_AUTH_FAIL ? pr : 0xFFFFFFFFu);
+}
+
 // Tag and verdict of each lane's packet once its bytes have gone through the
 // MAC, and the zero-fill of rejected plaintexts.
 // Returns whether the lane's packet was rejected.
@@ -761,38 +890,7 @@ BNK_DEV bool lane_finish(const AeadArgs &a, uint32_t lane, bool have, uint32_t i
             if (a.verdict) a.verdict[i] = reject ? 0 : 1;
         }
     }
-    if (OPEN && decap) {
-        // what WireGuard does with an opened datagram: keepalive, IP version, the
-        // trim to the IP header's total length, the sender's allowed prefix (the
-        // header's first 16 bytes were kept when they went through the cipher)
-        uint32_t res = BNK_WG_OK, out_len = 0;
-        const uint32_t version = (head.c0.x >> 4) & 0xFu;
-        if (!have || reject) res = BNK_WG_AUTH_FAIL; // (no packet here: it reached beyond the output arena)
-        else if (len == 0u) res = BNK_WG_KEEPALIVE;
-        else if (len < 16u) res = BNK_WG_BAD_IP; // too short for either header
-        else if (version == 4u) {
-            const uint32_t total = __builtin_bswap32(head.c0.x) & 0xFFFFu;
-            const uint2 al = a.wg.allowed[pr];
-            if (len < 20u || total > len || total < 20u) res = BNK_WG_BAD_IP;
-            else if ((__builtin_bswap32(head.c0.w) & al.y) != (al.x & al.y)) res = BNK_WG_NOT_ALLOWED;
-            else out_len = total;
-        } else if (version == 6u) {
-            // peers own IPv4 addresses only
-            const uint32_t total = (__builtin_bswap32(head.c0.y) >> 16) + 40u;
-            res = (len < 40u || total > len) ? BNK_WG_BAD_IP : BNK_WG_NOT_ALLOWED;
-        } else res = BNK_WG_BAD_IP;
-        a.wg.result[i] = (uint8_t)res;
-        a.wg.out_len[i] = out_len;
-        if (a.wg.replay_keys) {
-            const uint32_t sender = res != BNK_WG_AUTH_FAIL ? pr : 0xFFFFFFFFu;
-            if (a.wg.replay_index_bits) {
-                a.wg.replay_keys[i - a.first] = wg_replay_pack(sender, i - a.first, a.wg.replay_index_bits);
-            } else {
-                a.wg.replay_keys[i - a.first] = sender;
-                a.wg.replay_idx[i - a.first] = i - a.first;
-            }
-        }
-    }
+    if (OPEN && decap) decap_result(a, i, have, reject, len, head.c0, pr);
     if (OPEN && record) {
         // bytes 0-23 of the plaintext, its length, 1 if it is authentic: the lanes'
         // records lie side by side
@@ -822,29 +920,39 @@ BNK_DEV bool lane_finish(const AeadArgs &a, uint32_t lane, bool have, uint32_t i
     return reject;
 }
 
-// A lane per packet.  SHORT_ONLY: the launch for batches in which every wave
-// takes the short path (see aead_short_kernel).
-template <bool OPEN, bool SHORT_ONLY>
-BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t t = blockIdx.x * LANE_BLOCK + threadIdx.x;
-    const uint32_t t_end = a.n;
+// One packet of a launch as its own lane sees it.
+struct LanePacket {
+    uint32_t i;        // its index in the batch
+    uint32_t pr;       // row of the key table
+    uint32_t len;      // bytes through the cipher, 0 without a packet
+    uint32_t len_in;   // of which in memory (the rest is padding that counts as zeros)
+    uint32_t wg_res;   // decapsulating: what its header said
+    uint64_t ctr;
+    const uint8_t *src; // the AEAD data, null without a packet
+    uint8_t *dst;
+    uint4 k0, k1;      // its key
+    bool in_batch, skipped, bad_peer, too_short, outside;
+    bool have;         // there is a packet to seal or open
+};
 
-    // ---- this lane's packet ----
-    // Straight-line code: every load below is issued whether or not the lane
-    // has a packet (from packet 0's entries or from `safe` when it has none or
-    // the array is absent), because a load under a branch makes the wave wait
-    // for it where the branch closes, and these form a chain (order -> lengths,
-    // offsets, peer -> key) that the first data loads should not queue behind.
-    // Worth 2 % on batches with every per-packet array present (the relay), a
-    // wash elsewhere.
+// Packet number t of the launch.
+// Straight-line code: every load below is issued whether or not the lane
+// has a packet (from packet 0's entries or from `safe` when it has none or
+// the array is absent), because a load under a branch makes the wave wait
+// for it where the branch closes, and these form a chain (order -> lengths,
+// offsets, peer -> key) that the first data loads should not queue behind.
+// Worth 2 % on batches with every per-packet array present (the relay), a
+// wash elsewhere.
+template <bool OPEN>
+BNK_DEV LanePacket lane_packet(const AeadArgs &a, uint32_t t, bool in_batch)
+{
+    LanePacket p;
     const uint32_t *safe32 = a.keys;
     const uint64_t *safe64 = reinterpret_cast<const uint64_t *>(a.keys);
-    const bool in_batch = t < t_end;
+    p.in_batch = in_batch;
     const uint32_t tt = in_batch ? t : 0u;
     const uint32_t ord = *(a.order ? a.order + tt : safe32);
-    const uint32_t i = a.first + (a.order ? ord : tt);
+    const uint32_t i = p.i = a.first + (a.order ? ord : tt);
     const uint32_t len_ld = *(a.lens ? a.lens + i : safe32);
     const uint32_t peer_ld = *(a.peer ? a.peer + i : safe32);
     const uint8_t skip_ld = *(a.skip ? a.skip + i : reinterpret_cast<const uint8_t *>(a.keys));
@@ -898,92 +1006,107 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
     // the sums below would wrap is beyond any arena
     const bool wraps = len > MAX_PACKET_BYTES;
     if (encap && !wraps) len += wg_padding(len, a.wg.mtu);
-    const uint32_t pr = decap ? wg_peer : a.peer ? peer_ld : 0u;
-    const bool skipped = (a.skip != nullptr && skip_ld != 0) || wg_res != BNK_WG_OK;
-    const bool bad_peer = pr >= a.n_peers;
-    const bool too_short = OPEN && len < 16u;
+    p.wg_res = wg_res;
+    p.pr = decap ? wg_peer : a.peer ? peer_ld : 0u;
+    p.skipped = (a.skip != nullptr && skip_ld != 0) || wg_res != BNK_WG_OK;
+    p.bad_peer = p.pr >= a.n_peers;
+    p.too_short = OPEN && len < 16u;
     const uint64_t in_at = (a.in_off ? in_off_ld : (uint64_t)i * a.in_stride) + a.in_skip;
     const uint64_t out_at = (a.out_off ? out_off_ld : (uint64_t)i * a.out_stride) + a.out_skip;
     // seal reads len and writes len + 16, open reads len (tag included) and writes len - 16
-    const bool outside = beyond_arena(in_at, len, a.in_limit) ||
-                         beyond_arena(out_at, OPEN ? (too_short ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
-                         (wraps && (a.in_limit | a.out_limit) != 0);
-    const uint64_t ctr = decap ? wg_ctr : a.counters ? ctr_ld : a.counter0 + i;
+    p.outside = beyond_arena(in_at, len, a.in_limit) ||
+                beyond_arena(out_at, OPEN ? (p.too_short ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
+                (wraps && (a.in_limit | a.out_limit) != 0);
+    p.ctr = decap ? wg_ctr : a.counters ? ctr_ld : a.counter0 + i;
     // a keypair that has used up its nonces sends nothing more (wireguard-go device/send.go)
-    const bool spent = encap && ctr >= WG_REJECT_AFTER_MESSAGES;
-    const bool have = in_batch && !skipped && !bad_peer && !too_short && !outside && !spent;
+    const bool spent = encap && p.ctr >= WG_REJECT_AFTER_MESSAGES;
+    p.have = in_batch && !p.skipped && !p.bad_peer && !p.too_short && !p.outside && !spent;
     // the key table has at least one row
-    const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * (bad_peer ? 0u : pr));
-    const uint4 k0 = kp[0], k1 = kp[1];
+    const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * (p.bad_peer ? 0u : p.pr));
+    p.k0 = kp[0];
+    p.k1 = kp[1];
     if (OPEN) len -= 16u;
-    len = have ? len : 0u;
-    const uint32_t len_in = encap ? min(len_plain, len) : len; // bytes of it in memory
-    const uint8_t *src = have ? a.in + in_at : nullptr;
-    uint8_t *dst = have ? a.out + out_at : nullptr;
-    const bool lane_lines = (((uintptr_t)src | (uintptr_t)dst) & 15u) == 0 &&
-                            (((uintptr_t)src ^ (uintptr_t)dst) & 127u) == 0;
+    p.len = p.have ? len : 0u;
+    p.len_in = encap ? min(len_plain, p.len) : p.len;
+    p.src = p.have ? a.in + in_at : nullptr;
+    p.dst = p.have ? a.out + out_at : nullptr;
+    return p;
+}
+
+// What those checks leave behind for the packet, and the header of a datagram
+// that is sent.
+template <bool OPEN>
+BNK_DEV void lane_packet_report(const AeadArgs &a, const LanePacket &p)
+{
+    if (OPEN && a.wg.mode == WG_FUSE_DECAP && p.in_batch) {
+        const bool ok = p.wg_res == BNK_WG_OK;
+        a.wg.peer_out[p.i] = ok ? p.pr : 0xFFFFFFFFu;
+        a.wg.counter_out[p.i] = ok ? p.ctr : 0ull;
+        if (!ok) {
+            a.wg.result[p.i] = (uint8_t)p.wg_res;
+            a.wg.out_len[p.i] = 0;
+            replay_key(a, p.i, 0xFFFFFFFFu);
+        }
+    }
+    if (p.in_batch && !p.skipped && (p.bad_peer || p.too_short || p.outside)) {
+        if (p.bad_peer) status_raise(a.status, STATUS_PEER_RANGE);
+        else if (p.outside) status_raise(a.status, STATUS_BOUNDS);
+        if (OPEN && a.verdict) a.verdict[p.i] = 0;
+    }
+    if (!OPEN && a.wg.mode == WG_FUSE_ENCAP && p.in_batch && !p.skipped) {
+        // the transport header: type 4, the receiver's index, the counter
+        if (p.have)
+            st16(p.dst - 16, make_uint4(4u, a.wg.remote_index[p.pr], (uint32_t)p.ctr, (uint32_t)(p.ctr >> 32)));
+        a.wg.wire_len[p.i] = p.have ? 16u + p.len + 16u : 0u;
+    }
+}
+
+// A lane per packet.  SHORT_ONLY: the launch for batches in which every wave
+// takes the short path (see aead_short_kernel).
+template <bool OPEN, bool SHORT_ONLY>
+BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t t = blockIdx.x * LANE_BLOCK + threadIdx.x;
+    const LanePacket p = lane_packet<OPEN>(a, t, t < a.n);
+    const bool lane_lines = (((uintptr_t)p.src | (uintptr_t)p.dst) & 15u) == 0 &&
+                            (((uintptr_t)p.src ^ (uintptr_t)p.dst) & 127u) == 0;
     // which launch does this wave's packets: nothing has been written so far
     const bool all_lines = __ballot(!lane_lines) == 0ull;
-    const bool all_short = all_lines && __ballot(len > 64u * SHORT_BLOCKS) == 0ull;
+    const bool all_short = all_lines && __ballot(p.len > 64u * SHORT_BLOCKS) == 0ull;
     if (SHORT_ONLY && !all_short) {
         // (the host launches this kernel only where no wave can come here)
         status_raise(a.status, STATUS_INTERNAL);
         return;
     }
-    // what the checks above leave behind per packet
-    if (decap && in_batch) {
-        const bool ok = wg_res == BNK_WG_OK;
-        a.wg.peer_out[i] = ok ? wg_peer : 0xFFFFFFFFu;
-        a.wg.counter_out[i] = ok ? wg_ctr : 0ull;
-        if (!ok) {
-            a.wg.result[i] = (uint8_t)wg_res;
-            a.wg.out_len[i] = 0;
-            if (a.wg.replay_keys) {
-                if (a.wg.replay_index_bits) {
-                    a.wg.replay_keys[i - a.first] = wg_replay_pack(0xFFFFFFFFu, i - a.first, a.wg.replay_index_bits);
-                } else {
-                    a.wg.replay_keys[i - a.first] = 0xFFFFFFFFu;
-                    a.wg.replay_idx[i - a.first] = i - a.first;
-                }
-            }
-        }
-    }
-    if (in_batch && !skipped && (bad_peer || too_short || outside)) {
-        if (bad_peer) status_raise(a.status, STATUS_PEER_RANGE);
-        else if (outside) status_raise(a.status, STATUS_BOUNDS);
-        if (OPEN && a.verdict) a.verdict[i] = 0;
-    }
-    if (encap && in_batch && !skipped) {
-        // the transport header: type 4, the receiver's index, the counter
-        if (have) st16(dst - 16, make_uint4(4u, a.wg.remote_index[pr], (uint32_t)ctr, (uint32_t)(ctr >> 32)));
-        a.wg.wire_len[i] = have ? 16u + len + 16u : 0u;
-    }
-    const uint32_t k[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    lane_packet_report<OPEN>(a, p);
+    const uint32_t k[8] = {p.k0.x, p.k0.y, p.k0.z, p.k0.w, p.k1.x, p.k1.y, p.k1.z, p.k1.w};
 
-    const uint32_t n1 = (uint32_t)ctr, n2 = (uint32_t)(ctr >> 32);
+    const uint32_t n1 = (uint32_t)p.ctr, n2 = (uint32_t)(p.ctr >> 32);
     uint32_t x[16];
     Poly32 mac; // keyed from keystream block 0 inside the body, once its first loads are out
 
+    const bool decap = OPEN && a.wg.mode == WG_FUSE_DECAP;
     const uint8_t *safe = reinterpret_cast<const uint8_t *>(a.keys);
     Head head;
     head.on = OPEN && (a.heads != nullptr || decap);
     head.c0 = head.c1 = make_uint4(0, 0, 0, 0);
-    if (SHORT_ONLY) body_short<OPEN, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head);
-    else if (all_short) body_short<OPEN>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head);
+    if (SHORT_ONLY) body_short<OPEN, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
+    else if (all_short) body_short<OPEN>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
     else if (!all_lines) {
-        if (__ballot(((uintptr_t)dst & 3u) != 0) == 0ull)
-            body_lines<OPEN, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head);
-        else body_lines<OPEN, false>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head);
+        if (__ballot(((uintptr_t)p.dst & 3u) != 0) == 0ull)
+            body_lines<OPEN, false, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
+        else body_lines<OPEN, false>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
     }
-    else body_lines<OPEN, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head);
+    else body_lines<OPEN, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
 
-    const bool reject = lane_finish<OPEN>(a, lane, have, i, len, src, dst, mac, head,
-                                          in_batch && a.heads ? a.heads + 32ull * t : nullptr,
-                                          decap && in_batch && wg_res == BNK_WG_OK, pr);
+    const bool reject = lane_finish<OPEN>(a, lane, p.have, p.i, p.len, p.src, p.dst, mac, head,
+                                          p.in_batch && a.heads ? a.heads + 32ull * t : nullptr,
+                                          decap && p.in_batch && p.wg_res == BNK_WG_OK, p.pr);
     if (OPEN && a.tally) {
         // a plain open counting its own verdicts: verdict 1 exactly where the lane had a packet
         // whose tag verified
-        const unsigned long long ok = __ballot(have && !reject), all = __ballot(in_batch);
+        const unsigned long long ok = __ballot(p.have && !reject), all = __ballot(p.in_batch);
         if (lane == 0u) {
             tally_bump(a.tally, TALLY_OPENED, (uint32_t)__popcll(ok));
             tally_bump(a.tally, TALLY_REJECTED, (uint32_t)__popcll(all & ~ok));
@@ -1012,6 +1135,223 @@ void aead_short_kernel(AeadArgs a)
 {
     __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * SHORT_ROW];
     wave_main<OPEN, true>(a, tile_all[threadIdx.x >> 6]);
+}
+
+// A few lanes per packet, for batches between the two: too few packets to fill
+// the chip with one per lane (then a launch lasts as long as one lane needs for the
+// longest packet, 70 us at 1420 bytes), too many to spend a wave on each.  A wave
+// takes `a.split` packets and deals them out to its 64 lanes in runs of q pieces of
+// 128 bytes, a lane a run, q as small as the lanes allow and the same for all of the
+// wave's packets: its lanes are done at the same time whatever mix of lengths it holds,
+// so no grouping by length comes before.  A lane goes through its run as the launch
+// above goes through a packet (body_lines); its share of the tag is lifted to its
+// place (split_value in aead_lane.hpp), added to the packet's in LDS, and the lane
+// of the packet's first run finishes it.
+//
+// A piece is a pair of keystream blocks from an even one on: block 0, the one-time
+// key, comes out of the first piece's pair, whose other half is the packet's first 64
+// bytes, so no lane computes a block for the key alone.  What splitting costs is the
+// lift, some fourteen field multiplications per lane (0.8 of a ChaCha20 block).
+constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
+constexpr uint32_t SPLIT_MAX_RUNS = 32;    // per packet (split_join)
+
+struct SplitPacket {
+    // what the lanes of the packet read before they start; then the second half of its one-time key
+    union {
+        struct {
+            const uint8_t *src;
+            uint64_t ctr;
+        } from;
+        uint4 pad;
+    };
+    uint8_t *dst;
+    // the same; then bytes 16-23 of the plaintext (open)
+    union {
+        struct {
+            uint32_t len_in, start; // start: lane of the first run
+        } deal;
+        uint2 head1;
+    };
+    uint4 tag, head0; // open: what came with the packet; bytes 0-15 of the plaintext
+    uint32_t len, pr;
+    uint32_t sum[5];  // the tag polynomial, limb by limb
+    uint32_t unused;
+};
+
+template <bool OPEN>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void aead_split_kernel(AeadArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t tile[64 * RING_ROW];
+    __shared__ SplitPacket sh[SPLIT_MAX_PACKETS];
+    static_assert(8 * (sizeof(tile) + sizeof(sh)) <= 160 * 1024, "two waves per SIMD");
+    const uint32_t lane = threadIdx.x;
+    const uint32_t first = blockIdx.x * a.split;
+    const uint32_t count = min(a.split, a.n - first);
+    const bool decap = OPEN && a.wg.mode == WG_FUSE_DECAP;
+
+    // ---- the packets, a lane each, and how they are dealt out ----
+    uint32_t q, lanes;
+    {
+        const LanePacket p = lane_packet<OPEN>(a, first + lane, lane < count);
+        // (the last things a packet is asked for fly while the pieces are dealt out)
+        const uint4 tag = ld16(OPEN && p.have ? p.src + p.len : reinterpret_cast<const uint8_t *>(a.keys));
+        const uint32_t pieces = p.have ? ((p.len + 63u) >> 6) / 2u + 1u : 0u;
+        uint32_t total = pieces, most = pieces;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+            total += (uint32_t)__shfl_xor((int)total, off, 64);
+            most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
+        }
+        uint32_t runs;
+        for (q = max(max((total + 63u) / 64u, (most + SPLIT_MAX_RUNS - 1u) / SPLIT_MAX_RUNS), 1u);; q++) {
+            lanes = runs = (pieces + q - 1u) / q;
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) lanes += (uint32_t)__shfl_xor((int)lanes, off, 64);
+            if (lanes <= 64u) break; // (at q = most every packet has one run)
+        }
+        q = __builtin_amdgcn_readfirstlane(q);
+        lanes = __builtin_amdgcn_readfirstlane(lanes);
+        uint32_t upto = runs;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)upto, off, 64);
+            if ((int)lane >= off) upto += o;
+        }
+        lane_packet_report<OPEN>(a, p);
+        if (OPEN && p.in_batch && !p.have) {
+            const uint4 zero = make_uint4(0, 0, 0, 0);
+            if (decap && p.wg_res == BNK_WG_OK) decap_result(a, p.i, false, false, 0u, zero, p.pr);
+            if (a.heads) {
+                st16a(a.heads + 32ull * (first + lane), zero);
+                st16a(a.heads + 32ull * (first + lane) + 16, zero);
+            }
+        }
+        if (lane < SPLIT_MAX_PACKETS) {
+            SplitPacket &to = sh[lane];
+            to.from.src = p.src;
+            to.from.ctr = p.ctr;
+            to.dst = p.dst;
+            to.deal.len_in = p.len_in;
+            to.deal.start = upto - runs;
+            to.tag = tag;
+            to.head0 = make_uint4(0, 0, 0, 0);
+            to.len = p.len;
+            to.pr = p.have ? p.pr : 0u;
+#pragma unroll
+            for (int l = 0; l < 5; l++) to.sum[l] = 0u;
+        }
+    }
+    wave_sync();
+
+    // ---- my run: number `run` of packet pk ----
+    const bool on = lane < lanes;
+    uint32_t pk = 0;
+#pragma unroll
+    for (uint32_t step = SPLIT_MAX_PACKETS / 2u; step; step >>= 1)
+        if (pk + step < count && sh[pk + step].deal.start <= lane) pk += step;
+    SplitPacket &my = sh[pk];
+    const uint32_t run = on ? lane - my.deal.start : 0u;
+    const uint32_t lead = on && run == 0u ? 4u : 0u;
+    // (a packet's bytes count from 64 before it, where its key block lies)
+    const uint32_t begin = run * q * 128u;
+    const uint32_t plen = on ? my.len + 64u : 0u, plen_in = on ? my.deal.len_in + 64u : 0u;
+    const uint32_t len = min(plen - begin, q * 128u);
+    const uint32_t len_in = plen_in > begin ? min(plen_in - begin, len) : 0u;
+    const uint8_t *src = on ? my.from.src - 64 + begin : nullptr;
+    uint8_t *dst = on ? my.dst - 64 + begin : nullptr;
+    const uint64_t ctr = on ? my.from.ctr : 0u;
+    const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * (on ? my.pr : 0u));
+    const uint4 k0 = kp[0], k1 = kp[1];
+    const uint32_t k[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+    const uint32_t n1 = (uint32_t)ctr, n2 = (uint32_t)(ctr >> 32);
+    const uint8_t *safe = reinterpret_cast<const uint8_t *>(a.keys);
+    uint32_t x[16];
+    Poly32 mac;
+    Head head;
+    head.on = OPEN && (a.heads != nullptr || decap);
+    head.keep0 = &my.head0;
+    head.keep1 = &my.head1;
+    head.keep_pad = &my.pad;
+    wave_sync(); // every lane has read what it starts with
+    const bool lane_lines = (((uintptr_t)src | (uintptr_t)dst) & 15u) == 0 && (((uintptr_t)src ^ (uintptr_t)dst) & 127u) == 0;
+    if (__ballot(!lane_lines) == 0ull)
+        body_lines<OPEN, true, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+    else if (__ballot(((uintptr_t)dst & 3u) != 0) == 0ull)
+        body_lines<OPEN, false, true, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+    else
+        body_lines<OPEN, false, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+
+    // ---- my share of the tag, lifted over the cells behind my run ----
+    {
+        const uint32_t e = on ? ((plen + 15u) >> 4) - ((begin + len + 15u) >> 4) : 0u;
+        Fe26 term = split_value(mac), pw = fe_clamped_r(mac.r0, mac.r1, mac.r2, mac.r3);
+        for (uint32_t b = 0;; b++) {
+            term = fe_select(((e >> b) & 1u) != 0u, fe_mul(term, pw), term);
+            if (__ballot((e >> b) > 1u) == 0ull) break;
+            pw = fe_sqr(pw);
+        }
+        if (on) {
+            atomicAdd(&my.sum[0], term.v0);
+            atomicAdd(&my.sum[1], term.v1);
+            atomicAdd(&my.sum[2], term.v2);
+            atomicAdd(&my.sum[3], term.v3);
+            atomicAdd(&my.sum[4], term.v4);
+        }
+    }
+    wave_sync();
+
+    // ---- the lane of the packet's first run finishes it ----
+    bool reject = false;
+    if (lead != 0u) {
+        const uint32_t sum[5] = {my.sum[0], my.sum[1], my.sum[2], my.sum[3], my.sum[4]};
+        const uint4 pad = my.pad;
+        mac.pad0 = pad.x; mac.pad1 = pad.y; mac.pad2 = pad.z; mac.pad3 = pad.w;
+        split_join(mac, sum);
+        // LE64(len(aad) = 0) || LE64(len(ciphertext))
+        mac.block(0, 0, plen - 64u, 0);
+        uint32_t tag[4];
+        mac.finish(tag);
+        if (!OPEN) {
+            st16(dst + plen, make_uint4(tag[0], tag[1], tag[2], tag[3]));
+        } else {
+            const uint4 tg = my.tag;
+            // all 16 bytes are compared, no early exit
+            reject = ((tg.x ^ tag[0]) | (tg.y ^ tag[1]) | (tg.z ^ tag[2]) | (tg.w ^ tag[3])) != 0u;
+            const uint32_t i = a.first + first + pk; // (these launches have no order[])
+            const uint4 c0 = my.head0;
+            if (a.verdict) a.verdict[i] = reject ? 0 : 1;
+            if (decap) decap_result(a, i, true, reject, plen - 64u, c0, my.pr);
+            if (a.heads) {
+                uint8_t *record = a.heads + 32ull * (first + pk);
+                const uint2 c1 = my.head1;
+                st16a(record, c0);
+                st16a(record + 16, make_uint4(c1.x, c1.y, plen - 64u, reject ? 0u : 1u));
+            }
+        }
+    }
+    if (OPEN) {
+        unsigned long long rej = __ballot(reject);
+        if (a.tally) {
+            const uint32_t ok = (uint32_t)__popcll(__ballot(lead != 0u && !reject));
+            if (lane == 0u) {
+                tally_bump(a.tally, TALLY_OPENED, ok);
+                tally_bump(a.tally, TALLY_REJECTED, count - ok);
+            }
+        }
+        if (rej != 0ull) {
+            // (the plaintext was stored by other lanes of this wave, see lane_finish)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            while (rej != 0ull) {
+                const int r = __ffsll((long long)rej) - 1;
+                rej &= rej - 1ull;
+                uint8_t *d = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)dst, r)) + 64;
+                const uint32_t L = (uint32_t)__shfl((int)plen, r, 64) - 64u;
+                for (uint32_t pos = 16u * lane; pos + 16u <= L; pos += 1024u)
+                    st16(d + pos, make_uint4(0, 0, 0, 0));
+                if (lane < (L & 15u)) st8(d + (L & ~15u) + lane, 0);
+            }
+        }
+    }
 }
 
 // One wave = one packet, for batches too small to fill the chip with a packet
@@ -1059,6 +1399,10 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     const uint8_t *src = a.in + (a.in_off ? in_off_ld : (uint64_t)i * a.in_stride) + a.in_skip;
     uint8_t *dst = a.out + (a.out_off ? out_off_ld : (uint64_t)i * a.out_stride) + a.out_skip;
     const bool skipped = a.skip != nullptr && skip_ld != 0;
+    auto refuse = [&]() {
+        a.verdict[i] = 0;
+        if (a.tally) tally_bump(a.tally, TALLY_REJECTED, 1u);
+    };
     uint64_t ctr = 0;
     if (!WG) {
         // (framing launches only run on layouts the host has checked)
@@ -1069,7 +1413,7 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
             (len > MAX_PACKET_BYTES && (a.in_limit | a.out_limit) != 0)) {
             if (lane == 0 && !skipped) {
                 status_raise(a.status, STATUS_BOUNDS);
-                if (OPEN) a.verdict[i] = 0;
+                if (OPEN) refuse();
             }
             return;
         }
@@ -1141,12 +1485,12 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         if (pr >= a.n_peers) {
             if (lane == 0) {
                 status_raise(a.status, STATUS_PEER_RANGE);
-                if (OPEN) a.verdict[i] = 0;
+                if (OPEN) refuse();
             }
             return;
         }
         if (OPEN && len < 16u) {
-            if (lane == 0) a.verdict[i] = 0;
+            if (lane == 0) refuse();
             return;
         }
         if (OPEN) len -= 16u;
@@ -1231,7 +1575,8 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         no_head.on = false;
         body_generic<OPEN>(tile_all[threadIdx.x >> 6], lane, have ? src : nullptr, have ? dst : nullptr,
                            have ? len : 0u, reinterpret_cast<const uint8_t *>(a.keys), k, n1, n2, mac, x, no_head);
-        lane_finish<OPEN>(a, lane, have, i, len, have ? src : nullptr, have ? dst : nullptr, mac, no_head, nullptr);
+        const bool bad = lane_finish<OPEN>(a, lane, have, i, len, have ? src : nullptr, have ? dst : nullptr, mac, no_head, nullptr);
+        if (OPEN && have && a.tally) tally_bump(a.tally, bad ? TALLY_REJECTED : TALLY_OPENED, 1u);
         return;
     }
 
@@ -1306,7 +1651,10 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         // all 16 bytes are compared, no early exit
         reject = ((want_tag.x ^ tag[0]) | (want_tag.y ^ tag[1]) | (want_tag.z ^ tag[2]) |
                   (want_tag.w ^ tag[3])) != 0;
-        if (!WG && lane == 0) a.verdict[i] = reject ? 0 : 1;
+        if (!WG && lane == 0) {
+            a.verdict[i] = reject ? 0 : 1;
+            if (a.tally) tally_bump(a.tally, reject ? TALLY_REJECTED : TALLY_OPENED, 1u);
+        }
     }
     if (WG && OPEN) {
         // ---- what wireguard-go checks once a packet is authentic: keepalive, IP
@@ -1362,16 +1710,72 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     }
 }
 
-// A lane per packet takes about 20 us + 43 ns per byte of the longest packet
-// however few packets there are, a wave per packet about 17 us + 2.7 to 3.3 ns
-// per packet (200 to 1420 bytes): measured crossovers 3,000 packets of 60
-// bytes, 4,800 of 200, 16,400 of 1420.  With the common length known the rule
-// below stays just under them; without it the caller's threshold stands alone.
+// Which launch?  Packets in GPU memory (us per launch of n packets in a row, all of
+// them resident at once; seal and open within 2 us of each other):
+//   a wave per packet   9 + 4.2 per 1000 packets at 1420 bytes, 3.3 at 60
+//   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2)
+//   a lane per packet   5 + 2.75 per ChaCha20 block of the longest packet, and 20 more
+//                       for the grouping where lengths vary
+// so 4096 packets x 1420 take 21 / 18 / 71 us, 16384 66 / 26 / 71, and 24000 packets of 1
+// to 1420 bytes - / 35 / 97.
+//
+// Packets in host memory (over_link): a wave per packet reads them where they are, the
+// others fetch the whole span first: about 17 us + 2.7 to 3.3 ns per packet (200 to 1420
+// bytes) against a lane per packet: measured crossovers 3,000 packets of 60 bytes, 4,800 of
+// 200, 16,400 of 1420.  With the common length known the rule stays just under them;
+// without it the caller's threshold stands alone.
 bool aead_runs_spread(const AeadArgs &a)
 {
-    if (a.lens) return a.n <= a.spread_max;
-    const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
-    return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
+    if (a.over_link) {
+        if (a.lens) return a.n <= a.spread_max;
+        const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
+        return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
+    }
+    const uint64_t most = 4ull * a.spread_max / 5; // 3276 by default
+    if (a.lens) return a.n <= most;
+    return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);
+}
+
+// Packets per wave of the launch that splits packets over lanes, 0 where a launch of
+// a lane per packet is the better one.
+//
+// How many: n / 2048 of them fill the chip with waves once and say how many pieces a run
+// must hold; what decides the cost is then how many of a wave's 64 lanes have a run, so the
+// wave takes as many more as still fit at that length (16384 packets x 1420: 10 instead of 8,
+// 38 us a pair of launches instead of 46 with three streams at work, 58 on one stream either
+// way).  Where the host does not know the lengths the room per packet in the arena stands for
+// their mean, with a margin for how much of it a wave may get: beyond 64 lanes all of a wave's
+// runs get longer (24000 packets of 1 to 1420 bytes, 15 per wave instead of 12: 39 us instead
+// of 47 on three streams, 70 instead of 63 on one).
+//
+// Where it ends: on one stream it is ahead up to where lanes fill the chip (65536 x 1420: 121
+// us a pair against 145), but it does half as much work again, and with several streams at
+// work the launches of a lane per packet overlap: 16384 x 1420 38 us against 50, x 600 25
+// against 27, 32768 x 1420 66 against 55.  Where lengths vary the other choice has the
+// grouping ahead of it as well: 40000 packets of 1 to 1420 bytes 61 us against 83, 57344 84
+// against 87, 65536 97 against 89.
+static uint32_t split_packets(const AeadArgs &a)
+{
+    // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
+    if (a.spread_max == 0 || a.order || aead_runs_spread(a)) return 0;
+    const uint32_t per = (a.n + 2047u) / 2048u;
+    if (per > (a.lens ? 28u : 12u)) return 0;
+    const uint32_t room = a.lens ? (uint32_t)std::min<uint64_t>(a.in_bytes / a.n, 1500u) : a.len;
+    const uint32_t blocks = (room + 63u) / 64u, pieces = blocks / 2u + 1u;
+    auto fits = [&](uint32_t k, uint32_t q) {
+        if (!a.lens) return k * ((pieces + q - 1u) / q) <= 64u;
+        const double mean = (double)room / (128.0 * q) + 1.0;
+        return k * mean + 0.3 * mean * sqrt((double)k) <= 64.0;
+    };
+    uint32_t q = 1, k = per;
+    while (q < pieces && !fits(k, q)) q++;
+    while (k < SPLIT_MAX_PACKETS && fits(k + 1u, q)) k++;
+    return a.lens || 150u + 920u * q < 275u * (blocks + 1u) ? k : 0u;
+}
+
+bool aead_wants_order(const AeadArgs &a)
+{
+    return a.lens && a.n > 64 && !aead_runs_spread(a) && split_packets(a) == 0;
 }
 
 // Can the host tell that every wave of the launch takes the short path?  One
@@ -1396,9 +1800,13 @@ static bool every_wave_short(const AeadArgs &a, bool open)
 }
 
 template <bool OPEN>
-static hipError_t launch_wave(const AeadArgs &a, hipStream_t s)
+static hipError_t launch_wave(const AeadArgs &args, hipStream_t s)
 {
-    if (every_wave_short(a, OPEN))
+    AeadArgs a = args;
+    a.split = split_packets(a);
+    if (a.split)
+        hipLaunchKernelGGL(aead_split_kernel<OPEN>, dim3((a.n + a.split - 1u) / a.split), dim3(64), 0, s, a);
+    else if (every_wave_short(a, OPEN))
         hipLaunchKernelGGL(aead_short_kernel<OPEN>, dim3((a.n + LANE_BLOCK - 1u) / LANE_BLOCK), dim3(LANE_BLOCK), 0, s, a);
     else
         hipLaunchKernelGGL(aead_wave_kernel<OPEN>, dim3((a.n + LANE_BLOCK - 1u) / LANE_BLOCK), dim3(LANE_BLOCK), 0, s, a);

@@ -420,6 +420,25 @@ BNK_DEV Fe26 fe_select(bool take_a, const Fe26 &a, const Fe26 &b)
                 take_a ? a.v3 : b.v3, take_a ? a.v4 : b.v4};
 }
 
+// Column sums below 2^61 as an element.
+BNK_DEV Fe26 fe_carry(uint64_t d0, uint64_t d1, uint64_t d2, uint64_t d3, uint64_t d4)
+{
+    Fe26 o;
+    uint64_t c;
+    c = d0 >> 26; o.v0 = (uint32_t)d0 & 0x3ffffffu; d1 += c;
+    c = d1 >> 26; o.v1 = (uint32_t)d1 & 0x3ffffffu; d2 += c;
+    c = d2 >> 26; o.v2 = (uint32_t)d2 & 0x3ffffffu; d3 += c;
+    c = d3 >> 26; o.v3 = (uint32_t)d3 & 0x3ffffffu; d4 += c;
+    c = d4 >> 26; o.v4 = (uint32_t)d4 & 0x3ffffffu;
+    // c < 2^36: times five it still fits 64 bits, and two more carries settle it
+    c = (uint64_t)o.v0 + c * 5;
+    o.v0 = (uint32_t)c & 0x3ffffffu;
+    c = (uint64_t)o.v1 + (c >> 26);
+    o.v1 = (uint32_t)c & 0x3ffffffu;
+    o.v2 += (uint32_t)(c >> 26);
+    return o;
+}
+
 // a * b mod 2^130 - 5.  a's limbs below 2^28, b's below 2^27: a product is
 // below 2^28 * 5 * 2^27 < 2^58 and five of them stay below 2^61.
 BNK_DEV Fe26 fe_mul(const Fe26 &a, const Fe26 &b)
@@ -435,20 +454,18 @@ BNK_DEV Fe26 fe_mul(const Fe26 &a, const Fe26 &b)
                   (uint64_t)a.v3 * b.v0 + (uint64_t)a.v4 * s4;
     uint64_t d4 = (uint64_t)a.v0 * b.v4 + (uint64_t)a.v1 * b.v3 + (uint64_t)a.v2 * b.v2 +
                   (uint64_t)a.v3 * b.v1 + (uint64_t)a.v4 * b.v0;
-    Fe26 o;
-    uint64_t c;
-    c = d0 >> 26; o.v0 = (uint32_t)d0 & 0x3ffffffu; d1 += c;
-    c = d1 >> 26; o.v1 = (uint32_t)d1 & 0x3ffffffu; d2 += c;
-    c = d2 >> 26; o.v2 = (uint32_t)d2 & 0x3ffffffu; d3 += c;
-    c = d3 >> 26; o.v3 = (uint32_t)d3 & 0x3ffffffu; d4 += c;
-    c = d4 >> 26; o.v4 = (uint32_t)d4 & 0x3ffffffu;
-    // c < 2^36: times five it still fits 64 bits, and two more carries settle it
-    c = (uint64_t)o.v0 + c * 5;
-    o.v0 = (uint32_t)c & 0x3ffffffu;
-    c = (uint64_t)o.v1 + (c >> 26);
-    o.v1 = (uint32_t)c & 0x3ffffffu;
-    o.v2 += (uint32_t)(c >> 26);
-    return o;
+    return fe_carry(d0, d1, d2, d3, d4);
+}
+
+// a * a, a's limbs below 2^27: 15 products instead of 25.
+BNK_DEV Fe26 fe_sqr(const Fe26 &a)
+{
+    const uint32_t s3 = a.v3 * 5, s4 = a.v4 * 5, t0 = a.v0 * 2, t1 = a.v1 * 2, t2 = a.v2 * 2, t3 = a.v3 * 2;
+    return fe_carry((uint64_t)a.v0 * a.v0 + (uint64_t)t1 * s4 + (uint64_t)t2 * s3,
+                    (uint64_t)t0 * a.v1 + (uint64_t)t2 * s4 + (uint64_t)a.v3 * s3,
+                    (uint64_t)t0 * a.v2 + (uint64_t)a.v1 * a.v1 + (uint64_t)t3 * s4,
+                    (uint64_t)t0 * a.v3 + (uint64_t)t1 * a.v2 + (uint64_t)a.v4 * s4,
+                    (uint64_t)t0 * a.v4 + (uint64_t)t1 * a.v3 + (uint64_t)a.v2 * a.v2);
 }
 
 // One lane's share of the tag polynomial: its k (0..4) cells m[4t .. 4t+3]
@@ -468,7 +485,7 @@ BNK_DEV Fe26 spread_term(const Fe26 &r, const uint32_t (&m)[16], uint32_t k, uin
     for (uint32_t b = 0; (1u << b) <= e_max; b++) {
         const Fe26 nl = fe_mul(lift, pw);
         lift = fe_select(((e >> b) & 1u) != 0, nl, lift);
-        pw = fe_mul(pw, pw);
+        pw = fe_sqr(pw);
     }
     return fe_mul(acc, lift);
 }
@@ -514,5 +531,40 @@ BNK_DEV uint32_t spread_e_max(uint32_t len)
     return cd > 4u ? cd - 3u : 1u;
 }
 constexpr uint32_t SPREAD_MAX_LEN = 63u * 64u; // data blocks on lanes 1..63
+
+// ---------------------------------------------------------------------------
+// One packet split over a few lanes, a run of consecutive blocks each: every
+// lane evaluates its own cells from zero by Horner's rule in radix 2^32 (r is
+// clamped, Poly32), and its result is lifted by r^(cells after its last one) and
+// added to the others' in radix 2^26, where powers of r can be multiplied.
+// ---------------------------------------------------------------------------
+
+// The accumulator of one lane as a field element (limbs below 2^27).
+BNK_DEV Fe26 split_value(const Poly32 &p)
+{
+    return Fe26{p.h0 & 0x3ffffffu, funnel(p.h1, p.h0, 26) & 0x3ffffffu, funnel(p.h2, p.h1, 20) & 0x3ffffffu,
+                funnel(p.h3, p.h2, 14) & 0x3ffffffu, (p.h3 >> 8) | (p.h4 << 24)};
+}
+
+// The sum of up to 32 lifted terms (limb by limb, each below 2^32) back into the
+// accumulator: the length block and the pad follow as for a packet of one lane.
+BNK_DEV void split_join(Poly32 &p, const uint32_t (&sum)[5])
+{
+    uint64_t t0 = sum[0], t1 = sum[1], t2 = sum[2], t3 = sum[3], t4 = sum[4];
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+        t1 += t0 >> 26; t0 &= 0x3ffffffu;
+        t2 += t1 >> 26; t1 &= 0x3ffffffu;
+        t3 += t2 >> 26; t2 &= 0x3ffffffu;
+        t4 += t3 >> 26; t3 &= 0x3ffffffu;
+        t0 += (t4 >> 26) * 5; t4 &= 0x3ffffffu;
+    }
+    uint64_t w = t0 + (t1 << 26);
+    p.h0 = (uint32_t)w; w = (w >> 32) + (t2 << 20);
+    p.h1 = (uint32_t)w; w = (w >> 32) + (t3 << 14);
+    p.h2 = (uint32_t)w; w = (w >> 32) + (t4 << 8);
+    p.h3 = (uint32_t)w;
+    p.h4 = (uint32_t)(w >> 32); // at most 4
+}
 
 } // namespace bnk

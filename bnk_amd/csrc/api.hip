@@ -71,7 +71,7 @@ int aead_batch_host_chunked(bnk_ctx *ctx, bool open, const bnk_batch *in, const 
         AeadArgs c = a;
         c.first = lo;
         c.n = hi - lo;
-        if (a.lens && c.n > 64) {
+        if (aead_wants_order(c)) {
             HIPCHK(ctx, launch_length_sort(a.lens + lo, c.n, open ? 16 : 0, ctx->order.as<uint32_t>() + lo,
                                            ctx->hist.as<uint32_t>(), ctx->cursor.as<uint32_t>(), ctx->stream));
             c.order = ctx->order.as<uint32_t>() + lo;
@@ -107,6 +107,7 @@ int aead_batch_host_direct(bnk_ctx *ctx, bool open, const bnk_batch *in, const b
     if (rc) return rc;
     // A launch of a wave per packet reads every packet where it lies, so only the
     // packets' own bytes count; a lane per packet first fetches the whole span.
+    a.over_link = true;
     a.lens = in->lens; // (for aead_runs_spread only whether there is one matters; set properly below)
     const uint64_t moved = aead_runs_spread(a) ? host_payload_bytes(in) : sin.size();
     if (moved > DIRECT_MAX_BYTES) return 1;
@@ -146,7 +147,7 @@ int aead_batch_host_direct(bnk_ctx *ctx, bool open, const bnk_batch *in, const b
     if (in->lens) {
         memcpy(p_lens, in->lens, (size_t)n * 4);
         a.lens = stage.dev(p_lens);
-        if (n > 64 && !aead_runs_spread(a)) {
+        if (aead_wants_order(a)) {
             // lanes of a wave should run equal block counts: longest first
             const uint32_t tag = open ? 16 : 0;
             auto blocks = [&](uint32_t i) {
@@ -221,6 +222,7 @@ int aead_batch(bnk_ctx *ctx, bool open, const bnk_batch *in, const bnk_batch *ou
     a.in_stride = in->stride;
     a.out_stride = out->stride;
     a.len = in->len;
+    a.in_bytes = in->bytes;
 
     if (in->mem == BNK_MEM_DEVICE) {
         rc = aead_device_layout_check(ctx, open, in, out);
@@ -241,7 +243,7 @@ int aead_batch(bnk_ctx *ctx, bool open, const bnk_batch *in, const bnk_batch *ou
         if (sort_scratch) {
             // the caller's scratch instead of the context's grow-only buffers
             a.order = nullptr;
-            if (a.lens && n > 64 && !aead_runs_spread(a)) {
+            if (aead_wants_order(a)) {
                 // the histogram keeps its place from call to call: it is left all zeros by each grouping
                 uint32_t *hist = sort_scratch, *cursor = hist + LEN_BINS, *order = cursor + LEN_CURSOR_WORDS;
                 HIPCHK(ctx, launch_length_sort(a.lens, n, open ? 16 : 0, order, hist, cursor, ctx->stream));
@@ -251,12 +253,10 @@ int aead_batch(bnk_ctx *ctx, bool open, const bnk_batch *in, const bnk_batch *ou
             rc = maybe_sort(ctx, &a, open ? 16 : 0);
             if (rc) return rc;
         }
-        // the verdicts are counted by the launch itself where a lane has a packet, else by a
-        // launch behind it
-        const bool count = open && ctx->tally_on.load(std::memory_order_relaxed);
-        if (count && !aead_runs_spread(a)) a.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
+        // (the launch counts its own verdicts)
+        if (open && ctx->tally_on.load(std::memory_order_relaxed))
+            a.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
         HIPCHK(ctx, open ? launch_aead_open(a, ctx->stream) : launch_aead_seal(a, ctx->stream));
-        if (count && !a.tally) return tally_results(ctx, TALLY_OPEN, verdict, n, BNK_MEM_DEVICE);
         return BNK_OK;
     }
     if (sort_scratch) return fail(ctx, BNK_E_INVAL, "this entry point takes device-resident batches only");

@@ -263,7 +263,7 @@ inline int stage_host(bnk_ctx *ctx, const bnk_batch *in, const bnk_batch *out, i
 inline int maybe_sort(bnk_ctx *ctx, AeadArgs *a, uint32_t tag_bytes)
 {
     a->order = nullptr;
-    if (!a->lens || a->n <= 64 || aead_runs_spread(*a)) return BNK_OK;
+    if (!aead_wants_order(*a)) return BNK_OK;
     HIPCHK(ctx, ctx->order.reserve((size_t)a->n * 4));
     HIPCHK(ctx, ctx->hist.reserve(LEN_BINS * 4));
     HIPCHK(ctx, ctx->cursor.reserve(LEN_CURSOR_WORDS * 4));

@@ -109,7 +109,10 @@ struct AeadArgs {
                                // has checked the layout
     uint32_t first;            // the launch covers packets first .. first+n-1; order[] is relative to first
     uint32_t spread_max;       // launches of at most this many packets run one wave per packet
-    unsigned long long *tally; // open, a lane per packet, or nullptr: the launch counts its own verdicts
+    uint64_t in_bytes;         // size of the input arena (a hint: how long packets may be on average)
+    bool over_link;            // packets lie in host memory: a wave per packet reads them there
+    uint32_t split;            // set by the launcher: packets per wave of aead_split_kernel
+    unsigned long long *tally; // open without framing, or nullptr: the launch counts its own verdicts
                                // here (TALLY_OPENED / TALLY_REJECTED, see tally_bump)
     WgFuse wg;                 // only with aead_runs_spread(); mode 0: plain AEAD
 };
@@ -163,6 +166,8 @@ __device__ inline void status_raise(uint32_t *status, uint32_t condition)
 // True when the launch will run one wave per packet (then order[] is not used
 // and callers need not build it).
 bool aead_runs_spread(const AeadArgs &a);
+// True when the launch would run faster with order[] (a lane per packet, lengths vary).
+bool aead_wants_order(const AeadArgs &a);
 hipError_t launch_aead_seal(const AeadArgs &a, hipStream_t s);
 hipError_t launch_aead_open(const AeadArgs &a, hipStream_t s);
 

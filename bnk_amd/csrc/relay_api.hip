@@ -35,6 +35,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
     // ---- where everything lives on the device ----
     AeadArgs op{};
     op.spread_max = ctx->spread_max;
+    op.in_bytes = in->bytes;
     op.keys = ctx->d_keys[BNK_KEYS_RECV];
     op.n_peers = ctx->n_keys[BNK_KEYS_RECV];
     op.status = ctx->d_status;
@@ -81,6 +82,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
                 h_verdict = (uint8_t *)(p_peer_out + n);
                 if (in->lens) { memcpy(p_lens, in->lens, (size_t)n * 4); op.lens = ctx->pin.dev(p_lens); }
                 const uint32_t mis = (uint32_t)((uintptr_t)(d_ring_in + sin.lo) & 127u);
+                op.over_link = true;
                 if (aead_runs_spread(op)) {
                     // a wave per packet reads the ring itself (see aead_batch_host_direct)
                     op.in = d_ring_in + sin.lo;
@@ -240,7 +242,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         o.out_stride = in->stride;
         o.verdict = ctx->r_auth.as<uint8_t>();
         o.order = nullptr;
-        if (o.lens && m > 64 && !aead_runs_spread(o)) {
+        if (aead_wants_order(o)) {
             HIPCHK(ctx, launch_length_sort(o.lens + lo, m, 16, ctx->order.as<uint32_t>() + lo,
                                            ctx->hist.as<uint32_t>(), ctx->cursor.as<uint32_t>(), ctx->stream));
             o.order = ctx->order.as<uint32_t>() + lo;
@@ -284,6 +286,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         // ---- 4. re-seal the survivors under the outbound keys ----
         AeadArgs se{};
         se.spread_max = ctx->spread_max;
+        se.in_bytes = in->bytes;
         se.keys = ctx->d_keys[BNK_KEYS_SEND];
         se.n_peers = n_peers_out;
         se.status = ctx->d_status;

@@ -292,6 +292,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
     // qualifies for it, else a plain launch over per-packet padded lengths.
     AeadArgs probe{};
     probe.spread_max = ctx->spread_max;
+    probe.over_link = host; // (how a batch that is read in place would run)
     probe.n = n;
     probe.len = slots->len;
     probe.lens = slots->lens; // only whether there is one matters here
@@ -462,6 +463,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         if (fits) {
             AeadArgs se{};
             se.spread_max = ctx->spread_max;
+            se.over_link = ring_out != nullptr;
             se.keys = ctx->d_keys[BNK_KEYS_SEND];
             se.n_peers = pe.n;
             se.status = ctx->d_status;
@@ -487,6 +489,8 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         }
         AeadArgs se{};
         se.spread_max = ctx->spread_max;
+        se.over_link = ring_out != nullptr;
+        se.in_bytes = slots->bytes;
         se.keys = ctx->d_keys[BNK_KEYS_SEND];
         se.n_peers = pe.n;
         se.status = ctx->d_status;
@@ -520,7 +524,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         }
         // (padding never changes a packet's number of 64-byte blocks, so the plaintext
         // lengths group the packets as the padded ones would)
-        if (slots->lens && se.n > 64 && !aead_runs_spread(se)) {
+        if (slots->lens && aead_wants_order(se)) {
             HIPCHK(ctx, launch_length_sort(se.lens + lo, se.n, 0, ctx->order.as<uint32_t>() + lo,
                                            ctx->hist.as<uint32_t>(), ctx->cursor.as<uint32_t>(), ctx->stream));
             se.order = ctx->order.as<uint32_t>() + lo;
@@ -650,6 +654,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     // qualifies for it, else a plain launch over per-packet ciphertext lengths.
     AeadArgs probe{};
     probe.spread_max = ctx->spread_max;
+    probe.over_link = host; // (how a batch that is read in place would run)
     probe.n = n;
     probe.len = wire->len;
     probe.lens = wire->lens; // only whether there is one matters here
@@ -860,6 +865,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         if (fits) {
             AeadArgs op{};
             op.spread_max = ctx->spread_max;
+            op.over_link = direct;
             op.keys = ctx->d_keys[BNK_KEYS_RECV];
             op.n_peers = pe.n;
             op.status = ctx->d_status;
@@ -889,6 +895,8 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         }
         AeadArgs op{};
         op.spread_max = ctx->spread_max;
+        op.over_link = direct;
+        op.in_bytes = wire->bytes;
         op.keys = ctx->d_keys[BNK_KEYS_RECV];
         op.n_peers = pe.n;
         op.status = ctx->d_status;
@@ -925,7 +933,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
                 op.wg.replay_idx = rsc.idx;
                 op.wg.replay_index_bits = wg_replay_index_bits(op.n, pe.n);
             }
-            if (wire->lens && op.n > 64) {
+            if (wire->lens && aead_wants_order(op)) {
                 // (32 bytes of every datagram are header and tag)
                 HIPCHK(ctx, launch_length_sort(wb.lens + lo, op.n, 32, ctx->order.as<uint32_t>() + lo,
                                                ctx->hist.as<uint32_t>(), ctx->cursor.as<uint32_t>(), ctx->stream));
@@ -942,7 +950,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         op.verdict = d_auth;
         // (the datagram's own bounds were checked by the parse)
         op.skip = d_result; // BNK_WG_OK is 0: header failures are not opened
-        if (wire->lens && op.n > 64 && !aead_runs_spread(op)) {
+        if (wire->lens && aead_wants_order(op)) {
             HIPCHK(ctx, launch_length_sort(d_ctlen + lo, op.n, 16, ctx->order.as<uint32_t>() + lo,
                                            ctx->hist.as<uint32_t>(), ctx->cursor.as<uint32_t>(), ctx->stream));
             op.order = ctx->order.as<uint32_t>() + lo;

@@ -245,3 +245,73 @@ def test_length_grouping_on_either_side_of_its_launch_shapes(n):
             ctx.sync()
             bad = np.flatnonzero(d_sealed.cpu().numpy() != want)
             assert bad.size == 0, f"lengths up to {top}: first differing byte at {bad[:4]}"
+
+
+@pytest.mark.parametrize("n,length,kind", [(3277, 1500, "mixed"), (20011, 9000, "mixed"), (32769, 200, "mixed"),
+                                           (57344, 300, "mixed"), (57345, 300, "mixed"), (4097, 1420, "one"),
+                                           (2049, 257, "one"), (24576, 576, "one"), (5000, 4100, "one")])
+def test_packets_split_over_lanes_match_the_oracle(n, length, kind):
+    """Batches too large for a wave per packet and too small for a lane per packet, sealed and
+    opened in place: each packet is dealt out to several lanes in runs of 128-byte pieces (one
+    to seventy pieces a packet here, one to nine a run), packets of no and of one byte among
+    them, at sizes on both sides of where that launch begins and ends."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    dev = torch.device("cuda:0")
+    n_peers = 7
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    if kind == "one":
+        lens = np.full(n, length, np.uint32)
+        room = np.full(n, length + 16 + (n % 5), np.int64)  # a stride of any alignment
+    else:
+        lens = np.where(rng.random(n) < 0.05, rng.integers(0, 2, n), rng.integers(0, length + 1, n)).astype(np.uint32)
+        room = ((lens.astype(np.int64) + 16 + 15) // 16) * 16 + 16 * rng.integers(0, 3, n)
+    off = np.concatenate([[0], np.cumsum(room)[:-1]]).astype(np.uint64)
+    total = int(room.sum()) + 16
+    plain = rng.integers(0, 256, total, dtype=np.uint8)
+    peer = rng.integers(0, n_peers, n).astype(np.uint32)
+    ctrs = rng.integers(0, 1 << 63, n, dtype=np.uint64)
+    want = plain.copy()
+    O.seal_batch(keys, peer, ctrs, plain, off, lens, want, off, 8)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    arena, d_peer, d_ctr = d(plain), d(peer.astype(np.int32)), d(ctrs.astype(np.int64))
+    shape = {"stride": int(room[0])} if kind == "one" else {"offsets": d(off.astype(np.int64))}
+    size = {"length": length} if kind == "one" else {"lens": d(lens.astype(np.int32))}
+    size_ct = {"length": length + 16} if kind == "one" else {"lens": d((lens + 16).astype(np.int32))}
+    forged = rng.permutation(n)[:50]
+    pos = off[forged].astype(np.int64) + rng.integers(0, lens[forged].astype(np.int64) + 16)
+    d_v = torch.full((n,), 9, dtype=torch.uint8, device=dev)
+    torch.cuda.synchronize()
+    with lib.Context(0) as ctx:
+        ctx.keys_set(lib.KEYS_SEND, keys)
+        ctx.keys_set(lib.KEYS_RECV, keys)
+        out = lib.make_batch(arena, total, n, lib.MEM_DEVICE, **shape)
+        ctx.seal(lib.make_batch(arena, total, n, lib.MEM_DEVICE, peer=d_peer, counters=d_ctr, **shape, **size), out)
+        ctx.sync()
+        got = arena.cpu().numpy()
+        bad = np.flatnonzero(got != want)
+        assert bad.size == 0, "first differing byte at %r" % bad[:4]
+        arena[d(pos)] ^= 0x10
+        torch.cuda.synchronize()
+        ctx.counters_reset()
+        ctx.open(lib.make_batch(arena, total, n, lib.MEM_DEVICE, peer=d_peer, counters=d_ctr, **shape, **size_ct), out, d_v)
+        ctx.sync()
+        counts = ctx.counters()
+    exp_v = np.ones(n, np.uint8)
+    exp_v[forged] = 0
+    assert np.array_equal(d_v.cpu().numpy(), exp_v)
+    assert (counts["opened"], counts["rejected"]) == (n - 50, 50)
+    # plaintexts back in place, rejected ones cleared, tags and gaps as they were
+    expect = want.copy()
+    expect[pos] ^= 0x10
+    at, length64 = off.astype(np.int64), lens.astype(np.int64)
+    inside = np.zeros(total + 1, np.int32)
+    np.add.at(inside, at, 1)
+    np.add.at(inside, at + length64, -1)
+    data = np.cumsum(inside[:-1]) > 0
+    expect[data] = plain[data]
+    for i in forged:
+        expect[at[i]:at[i] + length64[i]] = 0
+    assert np.array_equal(arena.cpu().numpy(), expect)

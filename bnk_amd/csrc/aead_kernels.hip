@@ -1103,6 +1103,11 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
     const bool reject = lane_finish<OPEN>(a, lane, p.have, p.i, p.len, p.src, p.dst, mac, head,
                                           p.in_batch && a.heads ? a.heads + 32ull * t : nullptr,
                                           decap && p.in_batch && p.wg_res == BNK_WG_OK, p.pr);
+    if (!OPEN && a.tally) {
+        // an encapsulating launch counting what it sends
+        const unsigned long long sent = __ballot(p.have);
+        if (lane == 0u) tally_bump(a.tally, TALLY_SEALED, (uint32_t)__popcll(sent));
+    }
     if (OPEN && a.tally) {
         // a plain open counting its own verdicts: verdict 1 exactly where the lane had a packet
         // whose tag verified
@@ -1218,6 +1223,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             if ((int)lane >= off) upto += o;
         }
         lane_packet_report<OPEN>(a, p);
+        if (!OPEN && a.tally) {
+            const unsigned long long sent = __ballot(p.have);
+            if (lane == 0u) tally_bump(a.tally, TALLY_SEALED, (uint32_t)__popcll(sent));
+        }
         if (OPEN && p.in_batch && !p.have) {
             const uint4 zero = make_uint4(0, 0, 0, 0);
             if (decap && p.wg_res == BNK_WG_OK) decap_result(a, p.i, false, false, 0u, zero, p.pr);
@@ -1726,6 +1735,8 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
 // without it the caller's threshold stands alone.
 bool aead_runs_spread(const AeadArgs &a)
 {
+    // (framing behind a header: the host has not seen that every packet fits 63 blocks)
+    if (a.wg.mode != WG_FUSE_OFF && a.in_skip != 0u && !a.over_link) return false;
     if (a.over_link) {
         if (a.lens) return a.n <= a.spread_max;
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
@@ -1754,6 +1765,12 @@ bool aead_runs_spread(const AeadArgs &a)
 // against 27, 32768 x 1420 66 against 55.  Where lengths vary the other choice has the
 // grouping ahead of it as well: 40000 packets of 1 to 1420 bytes 61 us against 83, 57344 84
 // against 87, 65536 97 against 89.
+//
+// Up to 10240 packets whose lengths the host does not know, five per wave: whatever mix of
+// up to 1471 bytes they are, a piece is then all that a run ever holds, and the launch lasts
+// as long as that (3400 packets of 1 to 1420 bytes 46 -> 32 us a pair against as many as fit on
+// average, 10000 51 -> 40).
+constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
 static uint32_t split_packets(const AeadArgs &a)
 {
     // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
@@ -1768,6 +1785,7 @@ static uint32_t split_packets(const AeadArgs &a)
         return k * mean + 0.3 * mean * sqrt((double)k) <= 64.0;
     };
     uint32_t q = 1, k = per;
+    if (a.lens && per <= SPLIT_ALWAYS_ONE) return std::max(per, SPLIT_ALWAYS_ONE);
     while (q < pieces && !fits(k, q)) q++;
     while (k < SPLIT_MAX_PACKETS && fits(k + 1u, q)) k++;
     return a.lens || 150u + 920u * q < 275u * (blocks + 1u) ? k : 0u;

@@ -462,9 +462,11 @@ int aead_batch(bnk_ctx *ctx, bool open, const bnk_batch *in, const bnk_batch *ou
 // bnk_wg_encap_batch (wg_api.hip), with NoteOutbound at *note_now on the plaintexts first
 // when note_now is given; and bnk_wg_decap_batch, with CheckInbound at *check_now on the
 // delivered packets afterwards when check_now is given.  The context lock is held.
-int wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint32_t *wire_len, const int64_t *note_now);
+// *counted: whether the call's own launches count for bnk_counters_get (else the caller does it)
+int wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint32_t *wire_len, const int64_t *note_now,
+                  bool *counted = nullptr);
 int wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out, uint8_t *result, uint32_t *out_len,
-                  uint32_t *peer, uint64_t *counter, const int64_t *check_now);
+                  uint32_t *peer, uint64_t *counter, const int64_t *check_now, bool *counted = nullptr);
 
 // The file-scope device scratch of the entry point that allocates nothing
 // (noalloc_api.hip): looks up its address on `device` (which must be current).

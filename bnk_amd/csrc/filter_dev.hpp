@@ -85,6 +85,8 @@ struct FilterArgs {
                           // delivered these packets; a denied packet's BNK_WG_OK becomes BNK_WG_FILTERED
     unsigned long long *tally; // check only, or nullptr: the launch counts its verdicts here
                           // (TALLY_ALLOWED / TALLY_DENIED, see tally_bump)
+    unsigned long long *wg_tally; // with wg_result, or nullptr: the launch counts the results here as
+                          // it leaves them (decap_slot, and TALLY_ALLOWED for what was delivered)
     uint32_t *status;
     int64_t now;
     uint32_t n, stride, len;

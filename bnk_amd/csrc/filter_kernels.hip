@@ -268,31 +268,112 @@ BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, uint32_t lane, uint32_t iv
 constexpr uint32_t LDS_BOUNDS_MAX = 24576; // 96 KiB of cut points
 constexpr uint32_t FILTER_THREADS = 1024; // one copy of the index serves 16 waves
 
+// Where the three tables lie in a workgroup's LDS, in words, each on a 16-byte boundary:
+// the small presence bitmap, the jump table, the cut points.
+constexpr uint32_t LDS_SMALL_WORDS = SMALL_BITS / 32u;
+constexpr uint32_t LDS_JUMP_WORDS = (JUMP_BUCKETS + 2u) / 2u;
+constexpr uint32_t LDS_JUMP_ROOM = (LDS_JUMP_WORDS + 3u) & ~3u;
+
+// What a lane reads of a packet before anything is decided about it.
+struct RawHeader {
+    u32x4 a;        // bytes 0-15
+    u32x2 b;        // bytes 16-23, or 12-19 of a packet too short for those
+    uint32_t len;   // of the packet, without what is trimmed off
+    uint32_t i;     // the packet
+    bool ok;        // there is a packet to look at
+    uint8_t result; // what a decapsulating call said about it so far
+};
+
+// The loads of one packet, every one issued whether or not it is needed (from `safe`, 32
+// readable bytes, where it is not: a load under a branch is waited for where the branch
+// closes), so that they fly while the tables are staged or another packet is looked up.
+BNK_DEV RawHeader fetch_header(const FilterArgs &a, uint32_t t)
+{
+    RawHeader r;
+    const bool in = t < a.n;
+    const uint32_t tt = in ? t : 0u;
+    const uint8_t *const safe = reinterpret_cast<const uint8_t *>(a.flows.counters);
+    r.i = tt;
+    r.result = *(a.wg_result ? a.wg_result + tt : safe);
+    if (a.heads) {
+        // whoever wrote the records has checked the packets against the arena
+        r.a = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt);
+        const u32x4 r1 = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt + 16);
+        if (a.order) r.i = a.order[tt];
+        r.b = u32x2{r1.x, r1.y};
+        r.len = r1.z;
+        r.ok = in && r1.w != 0u && r.len >= 20u;
+        // (a record holds bytes 16-23 where the packet has them)
+        if (r.len < 24u) r.b = u32x2{0u, r1.x};
+        return r;
+    }
+    const uint8_t gate = *(a.gate ? a.gate + tt : safe);
+    const uint32_t len_ld = *(a.lens ? a.lens + tt : reinterpret_cast<const uint32_t *>(safe));
+    const uint64_t off_ld = *(a.off ? a.off + tt : reinterpret_cast<const uint64_t *>(safe));
+    const uint32_t len = a.lens ? len_ld : a.len;
+    const uint64_t at = a.off ? off_ld : (uint64_t)tt * a.stride;
+    r.len = len - (len >= a.trim ? a.trim : len);
+    r.ok = in && !(a.gate && gate == 0);
+    if (r.ok && beyond_arena(at, len, a.limit)) {
+        status_raise(a.status, STATUS_BOUNDS);
+        r.ok = false;
+    }
+    r.ok = r.ok && r.len >= 20u;
+    const uint8_t *const p = r.ok ? a.pkts + at : safe;
+    r.a = *reinterpret_cast<const u32x4_unaligned *>(p);
+    r.b = *reinterpret_cast<const u32x2_unaligned *>(p + (r.ok && r.len < 24u ? 12 : 16));
+    return r;
+}
+
 // filter.go:121-147 for a batch; enforcement is on (the host short-circuits
 // allow-all mode).
 __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterArgs a)
 {
-    extern __shared__ uint32_t lds[]; // the cut points when they fit, then the small presence bitmap
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     const RuleIndexDev ri = a.rules;
     const bool in_lds = ri.n_bounds <= LDS_BOUNDS_MAX;
-    const bool small = a.small_in_lds != 0u && a.flows.counters[FLOW_CLAIMED] <= SMALL_KEYS_MAX;
     const bool jumps = in_lds && ri.jump != nullptr;
-    constexpr uint32_t JUMP_WORDS = (JUMP_BUCKETS + 2u) / 2u;
-    uint32_t *lb = lds, *ljw = lds + ri.n_bounds;
-    uint32_t *lsmall = lds + (in_lds ? ri.n_bounds + (jumps ? JUMP_WORDS : 0u) : 0u);
+    const bool small = a.small_in_lds != 0u && a.flows.counters[FLOW_CLAIMED] <= SMALL_KEYS_MAX;
+    uint32_t *lsmall = lds, *ljw = lds + (a.small_in_lds ? LDS_SMALL_WORDS : 0u), *lb = ljw + (jumps ? LDS_JUMP_ROOM : 0u);
     const uint16_t *lj = reinterpret_cast<const uint16_t *>(ljw);
-    if (in_lds)
-        for (uint32_t q = threadIdx.x; q < ri.n_bounds; q += FILTER_THREADS) lb[q] = ri.bounds[q];
-    if (jumps)
-        for (uint32_t q = threadIdx.x; q < JUMP_WORDS; q += FILTER_THREADS)
-            ljw[q] = reinterpret_cast<const uint32_t *>(ri.jump)[q];
-    if (small)
-        for (uint32_t q = threadIdx.x; q < SMALL_BITS / 32u; q += FILTER_THREADS)
-            lsmall[q] = a.flows.present_small[q];
-    __syncthreads();
     const uint32_t stride = gridDim.x * FILTER_THREADS;
     const uint32_t lane = threadIdx.x & 63u;
+    // The first packet's header flies while the tables are staged, and theirs is one trip: 16
+    // bytes per lane and load, all of them in flight together.  (2^22 packets 75 -> 72 us
+    // against staging word by word, each waited for, and every header where it is parsed.)
+    RawHeader next = fetch_header(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
+    {
+        constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = (SMALL_QUADS + FILTER_THREADS - 1u) / FILTER_THREADS;
+        static_assert(LDS_SMALL_WORDS % 4u == 0u, "whole quads");
+        const uint4 *const s4 = reinterpret_cast<const uint4 *>(a.flows.present_small);
+        const uint4 *const b4 = reinterpret_cast<const uint4 *>(ri.bounds), *const j4 = reinterpret_cast<const uint4 *>(ri.jump);
+        const uint32_t bq = in_lds ? ri.n_bounds / 4u : 0u, jq = jumps ? LDS_JUMP_WORDS / 4u : 0u;
+        const uint32_t t = threadIdx.x;
+        uint4 sv[SMALL_PER], bv[2], jv;
+        uint32_t btail = 0, jtail = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < SMALL_PER; j++) sv[j] = s4[min(t + j * FILTER_THREADS, SMALL_QUADS - 1u)];
+#pragma unroll
+        for (uint32_t j = 0; j < 2u; j++) bv[j] = *(t + j * FILTER_THREADS < bq ? b4 + t + j * FILTER_THREADS : s4);
+        jv = *(t < jq ? j4 + t : s4);
+        if (in_lds && t < (ri.n_bounds & 3u)) btail = ri.bounds[4u * bq + t];
+        if (jumps && t < (LDS_JUMP_WORDS & 3u)) jtail = reinterpret_cast<const uint32_t *>(ri.jump)[4u * jq + t];
+        if (a.small_in_lds) {
+#pragma unroll
+            for (uint32_t j = 0; j < SMALL_PER; j++)
+                if (t + j * FILTER_THREADS < SMALL_QUADS) reinterpret_cast<uint4 *>(lsmall)[t + j * FILTER_THREADS] = sv[j];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 2u; j++)
+            if (t + j * FILTER_THREADS < bq) reinterpret_cast<uint4 *>(lb)[t + j * FILTER_THREADS] = bv[j];
+        if (t < jq) reinterpret_cast<uint4 *>(ljw)[t] = jv;
+        if (in_lds && t < (ri.n_bounds & 3u)) lb[4u * bq + t] = btail;
+        if (jumps && t < (LDS_JUMP_WORDS & 3u)) ljw[4u * jq + t] = jtail;
+        for (uint32_t q = t + 2u * FILTER_THREADS; q < bq; q += FILTER_THREADS) reinterpret_cast<uint4 *>(lb)[q] = b4[q];
+    }
+    __syncthreads();
     uint32_t n_pass = 0, n_drop = 0; // this wave's verdicts (the same in every lane)
+    uint32_t n_result = 0;           // with wg_tally: how often lane v's value v came out as the result
     if (blockIdx.x == 0u && threadIdx.x == 0u) {
         // (what this batch refreshes expires no earlier than this: news only if the clock went back)
         const int64_t from = a.now + FLOW_TTL_LEAST;
@@ -305,33 +386,13 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     for (uint32_t i0 = blockIdx.x * FILTER_THREADS + (threadIdx.x & ~63u); i0 < a.n; i0 += stride) {
         // t: this lane's place in the sweep; i: the packet it answers for
         const uint32_t t = i0 + lane;
-        uint32_t i = t;
-        bool valid;
+        const RawHeader raw = next;
+        next = fetch_header(a, t + stride);
+        const uint32_t i = raw.i;
         Parsed h{};
-        if (a.heads) {
-            valid = t < a.n;
-            const uint32_t tt = valid ? t : 0u;
-            const u32x4 r0 = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt);
-            const u32x4 r1 = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt + 16);
-            if (a.order) i = a.order[tt];
-            // whoever wrote the records has checked the packets against the arena
-            const uint32_t plen = r1.z;
-            valid = valid && r1.w != 0u && plen >= 20u &&
-                    parse_words(r0, r1.x, r1.y, plen >= 24u, plen, h, PacketAt{a.pkts, a.off, a.stride, i});
-        } else {
-            valid = t < a.n && !(a.gate && a.gate[t] == 0);
-            if (valid) {
-                const uint32_t len = a.lens ? a.lens[t] : a.len;
-                const uint32_t plen = len - (len >= a.trim ? a.trim : len);
-                const uint64_t at = a.off ? a.off[t] : (uint64_t)t * a.stride;
-                if (beyond_arena(at, len, a.limit)) {
-                    status_raise(a.status, STATUS_BOUNDS);
-                    valid = false;
-                } else {
-                    valid = parse_packet(a.pkts + at, plen, h, PacketAt{a.pkts, a.off, a.stride, t});
-                }
-            }
-        }
+        const bool wide = raw.len >= 24u;
+        const bool valid = raw.ok && parse_words(raw.a, wide ? raw.b.x : raw.b.y, raw.b.y, wide, raw.len, h,
+                                                 PacketAt{a.pkts, a.off, a.stride, i});
         uint32_t key = 0, iv = 0;
         bool maybe = false;
         FlowSlot s{};
@@ -395,8 +456,10 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         if (t < a.n) {
             a.verdict[i] = pass;
             // a packet WireGuard delivered and this filter denied (BNK_WG_OK is 0)
-            if (a.wg_result && !pass && a.wg_result[i] == 0) a.wg_result[i] = BNK_WG_FILTERED;
+            if (a.wg_result && !pass && raw.result == BNK_WG_OK) a.wg_result[i] = BNK_WG_FILTERED;
         }
+        if (a.wg_tally)
+            tally_vote(!pass && raw.result == BNK_WG_OK ? (uint32_t)BNK_WG_FILTERED : raw.result, t < a.n, lane, n_result);
         if (a.tally) {
             const unsigned long long in = __ballot(t < a.n), ok = __ballot(t < a.n && pass != 0);
             n_pass += (uint32_t)__popcll(ok);
@@ -406,6 +469,11 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     if (a.tally && lane == 0u) {
         tally_bump(a.tally, TALLY_ALLOWED, n_pass);
         tally_bump(a.tally, TALLY_DENIED, n_drop);
+    }
+    if (a.wg_tally && lane < 16u && n_result != 0u && decap_slot(lane) != TALLY_NONE) {
+        tally_bump(a.wg_tally, decap_slot(lane), n_result);
+        // CheckInbound behind a decapsulating call saw exactly what was delivered
+        if (lane == BNK_WG_OK) tally_bump(a.wg_tally, TALLY_ALLOWED, n_result);
     }
 }
 
@@ -620,9 +688,7 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
 {
     if (args.n == 0) return hipSuccess;
     FilterArgs a = args;
-    uint32_t lds = a.rules.n_bounds <= LDS_BOUNDS_MAX
-                       ? a.rules.n_bounds * 4u + (a.rules.jump ? (JUMP_BUCKETS + 2u) * 2u : 0u)
-                       : 0u;
+    uint32_t lds = a.rules.n_bounds <= LDS_BOUNDS_MAX ? a.rules.n_bounds * 4u + (a.rules.jump ? LDS_JUMP_ROOM * 4u : 0u) : 0u;
     // the small bitmap rides along while two workgroups still fit a CU's 160 KiB
     a.small_in_lds = lds + SMALL_BITS / 8u <= 80u * 1024u ? 1u : 0u;
     if (a.small_in_lds) lds += SMALL_BITS / 8u;
@@ -630,7 +696,7 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
         // more dynamic LDS than the default limit: opt in (gfx950 has 160 KiB per CU)
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(filter_check_kernel),
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(LDS_BOUNDS_MAX * 4u + (JUMP_BUCKETS + 2u) * 2u));
+                                           (int)(LDS_BOUNDS_MAX * 4u + LDS_JUMP_ROOM * 4u));
         if (e != hipSuccess) return e;
     }
     // one index copy per workgroup: as many workgroups per CU as their LDS allows, two at most

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/bnkhip.h"
+
 namespace bnk {
 
 // WireGuard pads the plaintext with zeros to a multiple of 16, never beyond the
@@ -112,8 +114,9 @@ struct AeadArgs {
     uint64_t in_bytes;         // size of the input arena (a hint: how long packets may be on average)
     bool over_link;            // packets lie in host memory: a wave per packet reads them there
     uint32_t split;            // set by the launcher: packets per wave of aead_split_kernel
-    unsigned long long *tally; // open without framing, or nullptr: the launch counts its own verdicts
-                               // here (TALLY_OPENED / TALLY_REJECTED, see tally_bump)
+    unsigned long long *tally; // or nullptr: an open without framing counts its own verdicts here
+                               // (TALLY_OPENED / TALLY_REJECTED, see tally_bump), an encapsulating
+                               // launch over a device-resident batch what it sends (TALLY_SEALED)
     WgFuse wg;                 // only with aead_runs_spread(); mode 0: plain AEAD
 };
 
@@ -135,11 +138,42 @@ enum TallySlot {
 };
 constexpr int TALLY_SLOTS = 16;
 constexpr uint32_t TALLY_LANES = 64;
+constexpr uint32_t TALLY_NONE = 0xFF;
+// the counter a decapsulating call's result feeds
+// (everything but a bad header, an unknown index and a failed tag was authentic)
+__host__ __device__ inline uint32_t decap_slot(uint32_t result)
+{
+    switch (result) {
+    case BNK_WG_OK: return TALLY_DELIVERED;
+    case BNK_WG_KEEPALIVE: return TALLY_KEEPALIVE;
+    case BNK_WG_BAD_HEADER: return TALLY_BAD_HEADER;
+    case BNK_WG_UNKNOWN_INDEX: return TALLY_UNKNOWN_INDEX;
+    case BNK_WG_AUTH_FAIL: return TALLY_REJECTED;
+    case BNK_WG_BAD_IP: return TALLY_BAD_IP;
+    case BNK_WG_NOT_ALLOWED: return TALLY_NOT_ALLOWED;
+    case BNK_WG_FILTERED: return TALLY_DENIED;
+    case BNK_WG_REPLAY: return TALLY_REPLAYED;
+    default: return TALLY_NONE;
+    }
+}
 static_assert(TALLY_RELAYED < TALLY_SLOTS, "slots");
 #if defined(__HIPCC__)
 __device__ inline void tally_bump(unsigned long long *tally, uint32_t slot, uint32_t k)
 {
     if (k != 0u) atomicAdd(&tally[slot * TALLY_LANES + (blockIdx.x & (TALLY_LANES - 1u))], (unsigned long long)k);
+}
+
+// The lanes of a wave vote per distinct value below 16 and lane v adds value v's votes to `mine`.
+__device__ __forceinline__ void tally_vote(uint32_t v, bool valid, uint32_t lane, uint32_t &mine)
+{
+    unsigned long long todo = __ballot(valid && v < 16u);
+    while (todo != 0ull) {
+        const int leader = __ffsll((long long)todo) - 1;
+        const uint32_t lv = (uint32_t)__builtin_amdgcn_readlane((int)v, leader);
+        const unsigned long long same = __ballot(valid && v == lv);
+        if (lane == lv) mine += (uint32_t)__popcll(same);
+        todo &= ~same;
+    }
 }
 #endif
 

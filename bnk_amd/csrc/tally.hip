@@ -7,10 +7,11 @@
 // result), and the counts are a histogram of those bytes, taken where they lie:
 // on the host for a host batch (the bytes have just come back); for a
 // device-resident one by the launch that writes them where it is the last to
-// touch them (a plain open, a CheckInbound on its own: a vote per wave and two
-// atomics, see tally_bump), else by one small launch behind the batch's own work
-// (the framing calls, whose results the window pass and the filter still change,
-// and the relay).
+// touch them (a plain open, a CheckInbound on its own or behind a decapsulating
+// call, an encapsulating seal that does its own framing: a vote per wave and one
+// or two atomics, see tally_bump), else by one small launch behind the batch's own
+// work (a decapsulating call without the filter, whose results the window pass
+// still changes, and the relay).
 #include "api_common.hpp"
 #include "kernels.hpp"
 
@@ -24,7 +25,7 @@ struct TallyMap {
     uint8_t also[16]; // a second counter the same value feeds
 };
 
-constexpr uint8_t NONE = 0xFF;
+constexpr uint8_t NONE = TALLY_NONE;
 
 TallyMap map_of(TallyKind kind)
 {
@@ -42,16 +43,7 @@ TallyMap map_of(TallyKind kind)
         break;
     case TALLY_DECAP:
     case TALLY_DECAP_CHECK:
-        // (everything but a bad header, an unknown index and a failed tag was authentic)
-        m.slot[BNK_WG_OK] = TALLY_DELIVERED;
-        m.slot[BNK_WG_KEEPALIVE] = TALLY_KEEPALIVE;
-        m.slot[BNK_WG_BAD_HEADER] = TALLY_BAD_HEADER;
-        m.slot[BNK_WG_UNKNOWN_INDEX] = TALLY_UNKNOWN_INDEX;
-        m.slot[BNK_WG_AUTH_FAIL] = TALLY_REJECTED;
-        m.slot[BNK_WG_BAD_IP] = TALLY_BAD_IP;
-        m.slot[BNK_WG_NOT_ALLOWED] = TALLY_NOT_ALLOWED;
-        m.slot[BNK_WG_FILTERED] = TALLY_DENIED;
-        m.slot[BNK_WG_REPLAY] = TALLY_REPLAYED;
+        for (uint32_t v = 0; v < 16u; v++) m.slot[v] = (uint8_t)decap_slot(v);
         // CheckInbound behind a decapsulating call saw exactly what was delivered
         if (kind == TALLY_DECAP_CHECK) m.also[BNK_WG_OK] = TALLY_ALLOWED;
         break;
@@ -72,18 +64,6 @@ TallyMap map_of(TallyKind kind)
 // add into the block's 16 LDS words, and the block issues one global atomic per
 // value that occurred: a few hundred atomics for a batch of a million.
 constexpr uint32_t TALLY_PER_THREAD = 16;
-
-__device__ __forceinline__ void tally_vote(uint32_t v, bool valid, uint32_t lane, uint32_t &mine)
-{
-    unsigned long long todo = __ballot(valid && v < 16u);
-    while (todo != 0ull) {
-        const int leader = __ffsll((long long)todo) - 1;
-        const uint32_t lv = (uint32_t)__builtin_amdgcn_readlane((int)v, leader);
-        const unsigned long long same = __ballot(valid && v == lv);
-        if (lane == lv) mine += (uint32_t)__popcll(same);
-        todo &= ~same;
-    }
-}
 
 __global__ __launch_bounds__(256) void tally_kernel(const uint8_t *res, uint32_t n, TallyMap map,
                                                     unsigned long long *counters)

@@ -1404,3 +1404,66 @@ def test_short_uniform_tunnel_batches_device_resident(plen):
         ok = np.flatnonzero(want == 0)
         assert np.array_equal(got[ok, 16:16 + plen], plain[ok])
         assert not got[5, 16:16 + padded].any()  # a rejected packet's plaintext is cleared
+
+
+@pytest.mark.parametrize("n", [1, 5, 6, 64, 700, 3277])
+@pytest.mark.parametrize("misalign", [False, True])
+def test_small_device_batches_do_their_own_framing(n, misalign):
+    """A device-resident batch too small for a lane per packet, whose lengths only the device
+    has: encapsulated and decapsulated by launches that split the packets over lanes, packets
+    of nothing and packets beyond 63 ChaCha20 blocks among them; and counted there."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(97 + n)
+    peers = _peers(rng)
+    back = [(p[1], p[0], p[2], p[3]) for p in peers]  # the other end
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    lens = rng.choice([0, 20, 40, 63, 64, 65, 127, 128, 129, 576, 1399, 1420, 1471, 4033, 9000], n).astype(np.uint32)
+    peer = rng.integers(0, N_PEERS, n).astype(np.uint32)
+    off, total = _layout(rng, 16 + lens.astype(np.int64) + 15 + 16, misalign)
+    arena = np.full(total, 0xEE, np.uint8)
+    want, ctr = arena.copy(), np.zeros(N_PEERS, np.uint64)
+    wire_len, forged = np.zeros(n, np.uint32), np.zeros(n, bool)
+    expect = []
+    for i in range(n):
+        p, at = int(peer[i]), int(off[i])
+        pt = _inner(rng, peers, p, int(lens[i]))
+        arena[at + 16:at + 16 + len(pt)] = np.frombuffer(pt, np.uint8)
+        w = O.wg_encap(pt, 0, keys[p].tobytes(), peers[p][1], int(ctr[p]))
+        ctr[p] += 1
+        want[at:at + len(w)] = np.frombuffer(w, np.uint8)
+        wire_len[i] = len(w)
+        forged[i] = i % 11 == 3
+        w = w[:-1] + bytes([w[-1] ^ 1]) if forged[i] else w
+        expect.append(O.wg_decap(w, back, keys))
+    dev = torch.device("cuda:0")
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    ctx = _ctx(peers, keys_send=keys, keys_recv=keys)
+    d_arena, d_off, d_lens = d(arena), d(off.astype(np.int64)), d(lens.astype(np.int32))
+    d_peer, d_wlen = d(peer.astype(np.int32)), torch.zeros(n, dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    ctx.wg_encap(lib.make_batch(d_arena, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens, peer=d_peer), 0, d_wlen)
+    ctx.sync()
+    assert np.array_equal(d_wlen.cpu().numpy().astype(np.uint32), wire_len)
+    assert np.array_equal(d_arena.cpu().numpy(), want)
+    assert ctx.counters()["sealed"] == n
+    assert np.array_equal(ctx.wg_send_counters(N_PEERS), ctr)
+    ctx.wg_peers_set(back)
+    for i in np.flatnonzero(forged):
+        want[int(off[i]) + int(wire_len[i]) - 1] ^= 1
+    d_wire, d_out = d(want), torch.full((total,), 0x55, dtype=torch.uint8, device=dev)
+    res = torch.zeros(n, dtype=torch.uint8, device=dev)
+    olen, gp = (torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(2))
+    gc = torch.zeros(n, dtype=torch.int64, device=dev)
+    torch.cuda.synchronize()
+    ctx.wg_decap(lib.make_batch(d_wire, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_wlen),
+                 lib.make_batch(d_out, total, n, lib.MEM_DEVICE, offsets=d_off), res, olen, gp, gc)
+    ctx.sync()
+    assert res.cpu().tolist() == [e[0] for e in expect]
+    assert olen.cpu().tolist() == [len(e[1]) for e in expect]
+    assert gp.cpu().tolist() == peer.tolist() and gc.cpu().tolist() == [e[3] for e in expect]
+    got = d_out.cpu().numpy()
+    for i, e in enumerate(expect):
+        assert got[int(off[i]):int(off[i]) + len(e[1])].tobytes() == e[1], i
+    ctx.close()

@@ -1,4 +1,5 @@
 // C ABI entry points of the packet filter (see include/bnkhip.h).
+#include <chrono>
 #include <stdio.h>
 
 #include "api_common.hpp"
@@ -106,8 +107,12 @@ namespace bnk {
 // full per region, growing (and dropping tombstones) when it would not.  Most
 // packets of a note batch belong to flows the table has, so the bound on claimed
 // slots outgrows their number by a batch per call; the words the launches leave
-// behind bring it back down.  (Reading the counter from the device instead waits
-// for everything enqueued, every few calls where batches are large.)
+// behind bring it back down.  Where the next batch may not fit while this one is
+// still on its way, a launch behind this one's leaves its number and the slots
+// claimed (FilterArgs::record_after), and the next call waits for that word alone.
+// (Reading the counter from the device instead waits for everything enqueued: with
+// 2^18 packets, or 3000 in the first table, every call through a tunnel stood
+// behind the whole one before it, 40 us in which the GPU had nothing to do.)
 int flows_reserve(bnk_ctx *ctx, uint32_t n_new)
 {
     FilterState *f = ctx->filter;
@@ -116,15 +121,23 @@ int flows_reserve(bnk_ctx *ctx, uint32_t n_new)
         f->claimed_upper += n_new;
         f->reserved += n_new;
         f->reserved_at[++f->note_seq & 63u] = f->reserved;
+        f->record_after = f->record != nullptr && f->claimed_upper + n_new > f->flows.cap / 2;
         return BNK_OK;
     };
-    if (f->record) {
+    auto lower = [&]() {
         const uint64_t rec = __atomic_load_n(f->record, __ATOMIC_RELAXED);
         const uint32_t seq = (uint32_t)(rec >> 32);
         if ((int32_t)(seq - f->table_seq) >= 0 && f->note_seq - seq < 64u)
             f->claimed_upper = std::min(f->claimed_upper, (rec & 0xFFFFFFFFu) + f->reserved - f->reserved_at[seq & 63u]);
-    }
+        return seq == f->note_seq;
+    };
+    if (f->record) lower();
     if (f->claimed_upper + n_new <= half) return take();
+    if (f->record_after) {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+        while (!lower() && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
+        if (f->claimed_upper + n_new <= half) return take();
+    }
     uint32_t c[FLOW_COUNTERS];
     HIPCHK(ctx, hipMemcpyAsync(c, f->flows.counters, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -231,6 +244,7 @@ void base_args(bnk_ctx *ctx, uint32_t n, int64_t now_ns, FilterArgs *a)
     a->flows = ctx->filter->flows;
     a->record = ctx->filter->d_record;
     a->record_seq = ctx->filter->note_seq;
+    a->record_after = ctx->filter->record_after;
 }
 
 int check_device_layout(bnk_ctx *ctx, const bnk_batch *b)

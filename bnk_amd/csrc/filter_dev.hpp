@@ -98,6 +98,8 @@ struct FilterArgs {
                           // while the table has seen at most SMALL_KEYS_MAX keys)
     uint64_t *record;     // note only: pinned host word that receives record_seq - 1 << 32 | slots
     uint32_t record_seq;  // claimed by the batches up to that number, or more (see flows_reserve)
+    bool record_after;    // note only: and record_seq << 32 | slots once this launch, the last of its
+                          // batch, has ended
     RuleIndexDev rules;
     FlowTableDev flows;
 };

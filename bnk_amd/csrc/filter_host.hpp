@@ -177,6 +177,7 @@ struct FilterState {
     uint32_t note_seq = 0, table_seq = 0;            // newest batch; newest batch before the current table
     uint64_t reserved = 0;                           // sum of n_new over all batches
     uint64_t reserved_at[64] = {0};                  // that sum as of batch (number & 63)
+    bool record_after = false;                       // the newest batch's number follows its launch into *record
     uint32_t max_blocks = 2048;
     void release()
     {

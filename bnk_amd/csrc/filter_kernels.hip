@@ -557,6 +557,13 @@ __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
     }
 }
 
+// (FilterArgs::record_after)
+__global__ void note_record_kernel(uint64_t *record, uint32_t seq, const uint32_t *counters)
+{
+    const uint32_t claimed = __hip_atomic_load(&counters[FLOW_CLAIMED], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(record, (uint64_t)seq << 32 | claimed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // filter.go:202-207: above 4096 entries, delete those with now.After(exp); there
 // is nothing to delete while no entry can have expired.  Nothing this launch
 // decides by changes while it runs: what it deletes and the bound it finds over
@@ -712,6 +719,8 @@ hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t
 {
     if (a.n == 0) return hipSuccess;
     hipLaunchKernelGGL(filter_note_kernel, dim3(grid_for(a.n, max_blocks)), dim3(256), 0, s, a);
+    if (a.record && a.record_after)
+        hipLaunchKernelGGL(note_record_kernel, dim3(1), dim3(1), 0, s, a.record, a.record_seq, a.flows.counters);
     // filter.go:202: no sweep while the map holds at most 4096 entries
     if (claimed_upper <= 4096u) return hipGetLastError();
     const uint32_t most = (uint32_t)(claimed_upper < a.flows.cap / 2u ? claimed_upper : a.flows.cap / 2u);

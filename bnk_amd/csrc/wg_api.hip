@@ -469,6 +469,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             fa.flows = f->flows;
             fa.record = f->d_record;
             fa.record_seq = f->note_seq;
+            fa.record_after = f->record_after && hi == n;
             HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->claimed_upper, ctx->stream));
         }
         if (fits) {

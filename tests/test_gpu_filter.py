@@ -315,3 +315,35 @@ def test_apply_netmap_json_end_to_end():
     ctx.filter_apply_netmap_json(json.dumps({"self_id": 2, "peers": []}))
     assert ctx.filter_check_inbound_ptrs([W.tcp(a, b, 1, 8888)], FC.T0).tolist() == [1]
     ctx.close()
+
+
+@pytest.mark.parametrize("n,distinct", [(3000, 900), (4096, 30000), (700, 5000)])
+def test_note_batches_in_a_row_while_the_table_is_nearly_full(n, distinct):
+    """Device-resident NoteOutbound batches enqueued without waiting, of flows that the table
+    mostly has (the bound on claimed slots then stands in the way of the next batch while this
+    one is on its way) or mostly has not (the table grows in between): the oracle's table."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    flows = np.zeros((distinct, 28), np.uint8)
+    flows[:, 0], flows[:, 3], flows[:, 8], flows[:, 9] = 0x45, 28, 64, np.where(np.arange(distinct) % 3, 6, 17)
+    flows[:, 12:16] = (100, 64, 0, 1)
+    flows[:, 16:24] = rng.integers(0, 256, (distinct, 8))
+    flows[:, 22:24] = np.arange(distinct, dtype=np.uint16).view(np.uint8).reshape(-1, 2)
+    ctx, ora = lib.Context(0), O.Filter()
+    rules = [([(0, 0)], "icmp", [])]
+    ctx.filter_set_rules(rules)
+    ora.set_rules(rules)
+    dev = torch.device("cuda:0")
+    picks = [rng.integers(0, distinct, n) for _ in range(24)]
+    device = [torch.from_numpy(np.ascontiguousarray(flows[p])).to(dev) for p in picks]
+    torch.cuda.synchronize()
+    for k, (p, d) in enumerate(zip(picks, device)):
+        now = FC.T0 + k * 1_000_000
+        ctx.filter_note_outbound(lib.make_batch(d, n * 28, n, lib.MEM_DEVICE, stride=28, length=28), now)
+        rec = flows[p]
+        ora.note_outbound_batch(rec.reshape(-1).copy(), np.arange(n, dtype=np.uint64) * 28, np.full(n, 28, np.uint32), now)
+    ctx.sync()
+    assert ctx.filter_flows() == ora.flows()
+    ctx.close()

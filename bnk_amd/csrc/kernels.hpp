@@ -258,10 +258,12 @@ hipError_t launch_peer_rank_counting(const uint32_t *peer, void *tmp, uint64_t *
 // host memory).
 hipError_t launch_pull(const void *src, void *dst, uint64_t bytes, hipStream_t s);
 
-// launch_wg_keys + launch_peer_rank for at most PEER_RANK_SMALL_MAX packets in
+// launch_wg_keys + launch_peer_rank for the batches peer_rank_one_block names in
 // one launch, straight from the peer array (null: every packet is peer 0).  A
 // peer index beyond the table sets STATUS_PEER_RANGE and gets no counter.
-constexpr uint32_t PEER_RANK_SMALL_MAX = 1024;
+constexpr uint32_t PEER_RANK_SMALL_MAX = 1024; // a packet a thread
+constexpr uint32_t PEER_RANK_BLOCK_MAX = 4096; // four
+bool peer_rank_one_block(uint32_t n, uint32_t n_keys);
 hipError_t launch_peer_rank_small(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
                                   uint64_t *ctr_out, bool advance, uint64_t ctr_limit, uint32_t *status,
                                   hipStream_t s);

@@ -137,9 +137,9 @@ size_t relay_sort_tmp_bytes(uint32_t n, uint32_t n_keys)
     return std::max(bytes, rows * plan.cols * 4u + (size_t)plan.cols * 8u);
 }
 
-__global__ void peer_rank_small_kernel(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
-                                       uint64_t *ctr_out, int advance, int no_peer_ok, unsigned bits,
-                                       uint64_t ctr_limit, uint32_t *status);
+static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
+                                             uint64_t *ctr_out, bool advance, bool no_peer_ok, uint64_t ctr_limit,
+                                             uint32_t *status, hipStream_t s);
 
 static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &plan, void *tmp,
                                          uint64_t *ctr_base, uint32_t n_keys, uint32_t n, uint64_t *ctr_out,
@@ -155,16 +155,14 @@ hipError_t launch_relay_assign(const uint8_t *auth, const uint8_t *pass, const u
     if (n == 0) return hipSuccess;
     const dim3 grid((n + 255u) / 256u);
     const RankPlan plan = rank_plan(n, n_peers_out);
-    const bool counting = n > PEER_RANK_SMALL_MAX && plan.fits && plan.bytes <= sort_tmp_bytes;
+    const bool one_block = peer_rank_one_block(n, n_peers_out);
+    const bool counting = !one_block && plan.fits && plan.bytes <= sort_tmp_bytes;
     hipLaunchKernelGGL(relay_verdict_kernel, grid, dim3(256), 0, s, auth, pass, peer_out, n_peers_out,
                        n, keys, counting ? (uint32_t *)nullptr : idx, verdict, ctr_out, status);
-    if (n <= PEER_RANK_SMALL_MAX) {
-        // keys[] is the peer of each survivor and all ones for the rest
-        hipLaunchKernelGGL(peer_rank_small_kernel, dim3(1), dim3(PEER_RANK_SMALL_MAX), 0, s, keys, n_peers_out,
-                           n, const_cast<uint64_t *>(ctr_base_out), ctr_out, advance ? 1 : 0, 1,
-                           key_bits(n_peers_out), 0ull, status);
-        return hipGetLastError();
-    }
+    // (keys[] is the peer of each survivor and all ones for the rest)
+    if (one_block)
+        return launch_peer_rank_one_block(keys, n_peers_out, n, const_cast<uint64_t *>(ctr_base_out), ctr_out, advance,
+                                          true, 0ull, status, s);
     if (counting)
         return launch_peer_rank_table(keys, plan, sort_tmp, const_cast<uint64_t *>(ctr_base_out), n_peers_out, n,
                                       ctr_out, advance, 0ull, true, nullptr, s);
@@ -217,15 +215,98 @@ __global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
     if (advance && valid && last) ctr_base[key[0]] = ctr_add(mine, 1u, ctr_limit);
 }
 
+// The same for up to PEER_RANK_BLOCK_MAX packets, four a thread, peer and position sorted as
+// one word; position p of the sorted batch is thread p % PEER_BLOCK_THREADS's.  (The counting
+// form's three launches cost four to six microseconds each at any size: 3000 packets 16 us,
+// here 9.)
+constexpr uint32_t PEER_BLOCK_THREADS = 1024, PEER_BLOCK_ITEMS = PEER_RANK_BLOCK_MAX / PEER_BLOCK_THREADS;
+constexpr unsigned PEER_BLOCK_INDEX_BITS = 12;
+static_assert(PEER_RANK_BLOCK_MAX == 1u << PEER_BLOCK_INDEX_BITS && PEER_RANK_BLOCK_MAX % PEER_BLOCK_THREADS == 0, "packed keys");
+__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
+    const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
+    int advance, int no_peer_ok, unsigned bits, uint64_t ctr_limit, uint32_t *status)
+{
+    using Sort = rocprim::block_radix_sort<uint32_t, PEER_BLOCK_THREADS, PEER_BLOCK_ITEMS>;
+    using Scan = rocprim::block_scan<uint32_t, PEER_BLOCK_THREADS>;
+    __shared__ union {
+        typename Sort::storage_type sort;
+        typename Scan::storage_type scan;
+    } tmp;
+    __shared__ uint32_t sk[PEER_RANK_BLOCK_MAX + 1];
+    __shared__ uint32_t start[PEER_RANK_BLOCK_MAX];
+    const uint32_t t = threadIdx.x;
+    const uint32_t none = (1u << bits) - 1u; // above every peer
+    uint32_t word[PEER_BLOCK_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+        const uint32_t i = t * PEER_BLOCK_ITEMS + j;
+        uint32_t key = NO_PEER;
+        if (i < n) {
+            key = peer ? peer[i] : 0u;
+            if (key >= n_keys && !(no_peer_ok && key == NO_PEER)) status_raise(status, STATUS_PEER_RANGE);
+        }
+        word[j] = (key < n_keys ? key : none) << PEER_BLOCK_INDEX_BITS | i;
+    }
+    Sort().sort_to_striped(word, tmp.sort, PEER_BLOCK_INDEX_BITS, PEER_BLOCK_INDEX_BITS + bits);
+#pragma unroll
+    for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) sk[j * PEER_BLOCK_THREADS + t] = word[j] >> PEER_BLOCK_INDEX_BITS;
+    if (t == 0) sk[PEER_RANK_BLOCK_MAX] = NO_PEER;
+    __syncthreads();
+    {
+        uint32_t upto[PEER_BLOCK_ITEMS], ahead = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+            const uint32_t p = t * PEER_BLOCK_ITEMS + j;
+            upto[j] = p != 0u && sk[p - 1u] != sk[p] ? p : 0u;
+            if (j) upto[j] = max(upto[j - 1u], upto[j]);
+        }
+        Scan().exclusive_scan(upto[PEER_BLOCK_ITEMS - 1u], ahead, 0u, tmp.scan, rocprim::maximum<uint32_t>());
+#pragma unroll
+        for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) start[t * PEER_BLOCK_ITEMS + j] = max(ahead, upto[j]);
+    }
+    __syncthreads();
+    uint64_t mine[PEER_BLOCK_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+        const uint32_t p = j * PEER_BLOCK_THREADS + t, key = word[j] >> PEER_BLOCK_INDEX_BITS;
+        mine[j] = 0;
+        if (key == none) continue;
+        mine[j] = ctr_add(ctr_base[key], p - start[p], ctr_limit);
+        ctr_out[word[j] & (PEER_RANK_BLOCK_MAX - 1u)] = mine[j];
+    }
+    __syncthreads(); // every base has been read
+#pragma unroll
+    for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+        const uint32_t p = j * PEER_BLOCK_THREADS + t, key = word[j] >> PEER_BLOCK_INDEX_BITS;
+        if (advance && key != none && sk[p + 1u] != key) ctr_base[key] = ctr_add(mine[j], 1u, ctr_limit);
+    }
+}
+
+bool peer_rank_one_block(uint32_t n, uint32_t n_keys)
+{
+    return n <= PEER_RANK_SMALL_MAX || (n <= PEER_RANK_BLOCK_MAX && key_bits(n_keys) + PEER_BLOCK_INDEX_BITS <= 32u);
+}
+
+static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
+                                             uint64_t *ctr_out, bool advance, bool no_peer_ok, uint64_t ctr_limit,
+                                             uint32_t *status, hipStream_t s)
+{
+    if (n <= PEER_RANK_SMALL_MAX)
+        hipLaunchKernelGGL(peer_rank_small_kernel, dim3(1), dim3(PEER_RANK_SMALL_MAX), 0, s, peer, n_keys, n,
+                           ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status);
+    else
+        hipLaunchKernelGGL(peer_rank_block_kernel, dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, peer, n_keys, n,
+                           ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status);
+    return hipGetLastError();
+}
+
 hipError_t launch_peer_rank_small(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
                                   uint64_t *ctr_out, bool advance, uint64_t ctr_limit, uint32_t *status,
                                   hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    if (n > PEER_RANK_SMALL_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(peer_rank_small_kernel, dim3(1), dim3(PEER_RANK_SMALL_MAX), 0, s, peer, n_keys, n,
-                       ctr_base, ctr_out, advance ? 1 : 0, 0, key_bits(n_keys), ctr_limit, status);
-    return hipGetLastError();
+    if (!peer_rank_one_block(n, n_keys)) return hipErrorInvalidValue;
+    return launch_peer_rank_one_block(peer, n_keys, n, ctr_base, ctr_out, advance, false, ctr_limit, status, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -408,7 +489,7 @@ static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &p
 bool peer_rank_counts(uint32_t n, uint32_t n_keys, size_t tmp_bytes)
 {
     const RankPlan plan = rank_plan(n, n_keys);
-    return n > PEER_RANK_SMALL_MAX && plan.fits && plan.bytes <= tmp_bytes;
+    return !peer_rank_one_block(n, n_keys) && plan.fits && plan.bytes <= tmp_bytes;
 }
 
 hipError_t launch_peer_rank_counting(const uint32_t *peer, void *tmp, uint64_t *ctr_base, uint32_t n_keys, uint32_t n,

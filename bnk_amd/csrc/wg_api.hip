@@ -426,7 +426,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
 
     // counters in batch order per peer, advancing the peers' send counters:
     // needs the peer array only, so it runs ahead of the packet bytes
-    if (n <= PEER_RANK_SMALL_MAX) {
+    if (peer_rank_one_block(n, pe.n)) {
         HIPCHK(ctx, launch_peer_rank_small(d_peer, pe.n, n, pe.send_ctr, d_ctr, true, WG_REJECT_AFTER_MESSAGES,
                                            ctx->d_status, ctx->stream));
     } else if (d_peer && peer_rank_counts(n, pe.n, tmp_bytes)) {
@@ -811,7 +811,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     const bool replay = ctx->wg_replay_on;
     WgReplayDev rpd{ctx->wg_replay, pe.n};
     WgReplayScratch rsc{};
-    if (replay && n > WG_REPLAY_SMALL_MAX) {
+    if (replay && !wg_replay_one_block(n, pe.n)) {
         const uint32_t biggest = chunked ? hp.per : n;
         for (DevBuf *buf : {&ctx->r_keys, &ctx->r_idx, &ctx->r_skeys, &ctx->r_sidx})
             HIPCHK(ctx, buf->reserve((size_t)biggest * 4));
@@ -845,7 +845,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     auto replay_range = [&](uint32_t lo, uint32_t hi, bool keys_from_open = false) -> int {
         if (!replay) return BNK_OK;
         WgReplayScratch c = rsc;
-        c.table_slots = hi - lo > WG_REPLAY_SMALL_MAX ? wg_replay_table_slots(hi - lo) : 0;
+        c.table_slots = wg_replay_one_block(hi - lo, pe.n) ? 0 : wg_replay_table_slots(hi - lo);
         if (c.table_slots) c.parity = ctx->wg_replay_parity++ & 1u;
         c.keys_ready = keys_from_open;
         HIPCHK(ctx, launch_wg_replay(d_result + lo, d_out_len + lo, d_peer + lo, d_counter + lo, hi - lo, rpd, c,
@@ -949,7 +949,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
             op.wg.peer_out = d_peer;
             op.wg.counter_out = d_counter;
             // the window pass sorts the authentic packets by peer: its keys come from here
-            const bool keys_here = replay && op.n > WG_REPLAY_SMALL_MAX;
+            const bool keys_here = replay && !wg_replay_one_block(op.n, pe.n);
             if (keys_here) {
                 op.wg.replay_keys = rsc.keys;
                 op.wg.replay_idx = rsc.idx;

@@ -43,13 +43,15 @@ hipError_t launch_wg_encap_prep(const WgBatch &b, uint8_t *hdr_base, const WgPee
 constexpr uint32_t WG_REPLAY_BLOCKS = 128;
 constexpr uint32_t WG_REPLAY_WORDS = 1 + WG_REPLAY_BLOCKS;
 constexpr uint32_t WG_REPLAY_SMALL_MAX = 1024; // at most this many packets: one launch of one block
+constexpr uint32_t WG_REPLAY_BLOCK_MAX = 4096; // and up to here as well, four packets a thread, where
+bool wg_replay_one_block(uint32_t n, uint32_t n_peers); // this says so (of any n)
 
 struct WgReplayDev {
     uint64_t *state; // [n_peers][WG_REPLAY_WORDS]
     uint32_t n_peers;
 };
 
-// Device scratch of one replay pass over n packets (beyond WG_REPLAY_SMALL_MAX).
+// Device scratch of one replay pass over n packets (not needed where wg_replay_one_block).
 struct WgReplayScratch {
     uint32_t *keys, *idx, *skeys, *sidx;   // n words each
     uint64_t *sctr, *sval, *pmax;          // n each

@@ -426,38 +426,12 @@ __global__ __launch_bounds__(256) void replay_late_advance_kernel(const uint32_t
     advance_window(state + (size_t)key * WG_REPLAY_WORDS, last);
 }
 
-// Sets the bit of every packet that reached the bit test and still lies in the
-// window its peer ends the batch with.  Neighbours in sorted order mostly
-// share their peer and their block of 64 counters: a lane whose left neighbour
-// differs gathers the bits of the lanes behind it that agree with it and
-// issues one atomic for all of them.
-//
-// The same launch leaves the first-occurrence table empty for the next pass
-// (nothing to do when this pass had no late packet, the usual case) and clears
-// the flag word the next pass will use (nobody reads that one now).
-__global__ __launch_bounds__(256) void replay_mark_kernel(const uint32_t *skeys, const uint64_t *sctr,
-                                                          const uint8_t *cls, uint64_t *state, uint32_t n,
-                                                          uint32_t *table, uint32_t slots, uint32_t *flags,
-                                                          uint32_t parity)
+// Sets `bit` of `block` in the window of peer `key` for every lane that has one (key NO_PEER:
+// none).  A lane whose left neighbour differs gathers the bits of the lanes behind it that
+// agree with it in peer and block and issues one atomic for all of them.
+__device__ __forceinline__ void mark_bits(uint64_t *state, uint32_t key, uint64_t block, uint64_t bit)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) flags[parity ^ 1u] = 0u;
-    if (flags[parity] != 0u)
-        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < slots; i += gridDim.x * 256u) table[i] = HASH_EMPTY;
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
     const uint32_t lane = threadIdx.x & 63u;
-    uint32_t key = NO_PEER;
-    uint64_t block = ~0ull, bit = 0;
-    if (p < n && cls[p] != RP_NONE) {
-        key = skeys[p];
-        const uint64_t c = sctr[p];
-        const uint64_t final_last = state[(size_t)key * WG_REPLAY_WORDS];
-        if ((final_last >> 6) - (c >> 6) < WG_REPLAY_BLOCKS) { // else its slot now belongs to a later block
-            block = c >> 6;
-            bit = 1ull << (c & 63u);
-        } else {
-            key = NO_PEER;
-        }
-    }
     // runs of equal (peer, block) among neighbouring lanes
     const uint32_t pkey = (uint32_t)__shfl_up((int)key, 1, 64);
     const uint32_t pblo = (uint32_t)__shfl_up((int)(uint32_t)block, 1, 64);
@@ -479,6 +453,38 @@ __global__ __launch_bounds__(256) void replay_mark_kernel(const uint32_t *skeys,
         atomicOr(reinterpret_cast<unsigned long long *>(
                      &state[(size_t)key * WG_REPLAY_WORDS + 1u + (block & (WG_REPLAY_BLOCKS - 1u))]),
                  (unsigned long long)acc);
+}
+
+// Sets the bit of every packet that reached the bit test and still lies in the
+// window its peer ends the batch with.  Neighbours in sorted order mostly
+// share their peer and their block of 64 counters.
+//
+// The same launch leaves the first-occurrence table empty for the next pass
+// (nothing to do when this pass had no late packet, the usual case) and clears
+// the flag word the next pass will use (nobody reads that one now).
+__global__ __launch_bounds__(256) void replay_mark_kernel(const uint32_t *skeys, const uint64_t *sctr,
+                                                          const uint8_t *cls, uint64_t *state, uint32_t n,
+                                                          uint32_t *table, uint32_t slots, uint32_t *flags,
+                                                          uint32_t parity)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) flags[parity ^ 1u] = 0u;
+    if (flags[parity] != 0u)
+        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < slots; i += gridDim.x * 256u) table[i] = HASH_EMPTY;
+    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
+    uint32_t key = NO_PEER;
+    uint64_t block = ~0ull, bit = 0;
+    if (p < n && cls[p] != RP_NONE) {
+        key = skeys[p];
+        const uint64_t c = sctr[p];
+        const uint64_t final_last = state[(size_t)key * WG_REPLAY_WORDS];
+        if ((final_last >> 6) - (c >> 6) < WG_REPLAY_BLOCKS) { // else its slot now belongs to a later block
+            block = c >> 6;
+            bit = 1ull << (c & 63u);
+        } else {
+            key = NO_PEER;
+        }
+    }
+    mark_bits(state, key, block, bit);
 }
 
 unsigned key_bits(uint32_t n_keys)
@@ -582,6 +588,166 @@ __global__ __launch_bounds__(SMALL) void replay_small_kernel(uint8_t *result, ui
     }
 }
 
+// The whole pass for a batch between that and WG_REPLAY_BLOCK_MAX packets in one workgroup, four
+// packets a thread, with the steps of the large form (below a few thousand packets its eight
+// launches take four microseconds each, mostly for being launches: 3000 packets 31 us, here
+// 15, and as much again for the host to launch them).  Position p of the sorted batch is thread p % BLOCK_THREADS's, so that neighbours in
+// order are neighbours in a wave; only the running maximum goes over four in a row per thread.
+constexpr uint32_t BLOCK_THREADS = 1024, BLOCK_ITEMS = WG_REPLAY_BLOCK_MAX / BLOCK_THREADS;
+constexpr unsigned BLOCK_INDEX_BITS = 12;
+static_assert(WG_REPLAY_BLOCK_MAX == 1u << BLOCK_INDEX_BITS && WG_REPLAY_BLOCK_MAX % BLOCK_THREADS == 0, "packed keys");
+constexpr uint32_t BLOCK_TABLE = 2u * WG_REPLAY_BLOCK_MAX;
+__global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *result, uint32_t *out_len,
+                                                                     const uint32_t *peer, const uint64_t *counter,
+                                                                     uint32_t n_peers, uint32_t n, uint64_t *state,
+                                                                     unsigned bits)
+{
+    using Sort = rocprim::block_radix_sort<uint32_t, BLOCK_THREADS, BLOCK_ITEMS>;
+    using ScanMax = rocprim::block_scan<RunMax, BLOCK_THREADS>;
+    __shared__ union {
+        typename Sort::storage_type sort;
+        typename ScanMax::storage_type scan;
+        uint32_t table[BLOCK_TABLE];
+    } tmp;
+    __shared__ uint32_t sk[WG_REPLAY_BLOCK_MAX + 1];
+    __shared__ uint64_t sc[WG_REPLAY_BLOCK_MAX];
+    __shared__ uint64_t smax[WG_REPLAY_BLOCK_MAX];
+    const uint32_t t = threadIdx.x;
+    const uint32_t none = (1u << bits) - 1u; // above every peer
+    uint32_t word[BLOCK_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        const uint32_t i = t * BLOCK_ITEMS + j;
+        uint32_t key = none;
+        if (i < n) {
+            const uint32_t p = peer[i];
+            if (replay_subject(result[i]) && p < n_peers) key = p;
+        }
+        word[j] = key << BLOCK_INDEX_BITS | i;
+    }
+    // stable: a peer's packets stay in batch order
+    Sort().sort_to_striped(word, tmp.sort, BLOCK_INDEX_BITS, BLOCK_INDEX_BITS + bits);
+    uint64_t c[BLOCK_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        const uint32_t key = word[j] >> BLOCK_INDEX_BITS;
+        c[j] = key != none ? counter[word[j] & (WG_REPLAY_BLOCK_MAX - 1u)] : 0;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        sk[j * BLOCK_THREADS + t] = word[j] >> BLOCK_INDEX_BITS;
+        sc[j * BLOCK_THREADS + t] = c[j];
+    }
+    if (t == 0) sk[WG_REPLAY_BLOCK_MAX] = NO_PEER;
+    __syncthreads();
+    {
+        // (a counter the filter turns away outright never moves last)
+        RunMax upto[BLOCK_ITEMS];
+#pragma unroll
+        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+            const uint64_t v = sc[t * BLOCK_ITEMS + j];
+            upto[j] = RunMax{sk[t * BLOCK_ITEMS + j], v < WG_REJECT_AFTER_MESSAGES ? v : 0};
+            if (j) upto[j] = RunMaxOp()(upto[j - 1u], upto[j]);
+        }
+        RunMax ahead;
+        ScanMax().exclusive_scan(upto[BLOCK_ITEMS - 1u], ahead, RunMax{NO_PEER, 0}, tmp.scan, RunMaxOp());
+#pragma unroll
+        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) smax[t * BLOCK_ITEMS + j] = RunMaxOp()(ahead, upto[j]).v;
+    }
+    __syncthreads();
+    uint8_t cls[BLOCK_ITEMS];
+    bool any_late = false;
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        const uint32_t p = j * BLOCK_THREADS + t, key = word[j] >> BLOCK_INDEX_BITS;
+        cls[j] = RP_NONE;
+        if (key == none) continue;
+        const uint64_t *st = state + (size_t)key * WG_REPLAY_WORDS;
+        const uint64_t last0 = st[0];
+        uint64_t last = last0;
+        if (p != 0u && sk[p - 1u] == key && smax[p - 1u] > last) last = smax[p - 1u];
+        if (reaches_bit_test(c[j], last)) cls[j] = c[j] > last ? RP_AHEAD : RP_LATE;
+        if (cls[j] == RP_LATE && c[j] <= last0 && seen_before(st, c[j])) cls[j] = RP_SEEN;
+        any_late |= cls[j] == RP_LATE;
+    }
+    bool repeat[BLOCK_ITEMS];
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) repeat[j] = false;
+    // (the windows have been read as the batch found them behind this)
+    if (__syncthreads_or(any_late)) {
+        // The first of the late packets that carry a counter, by table as in the large form.
+        constexpr uint32_t mask = BLOCK_TABLE - 1u;
+        for (uint32_t h = t; h < BLOCK_TABLE; h += BLOCK_THREADS) tmp.table[h] = HASH_EMPTY;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+            if (cls[j] != RP_LATE) continue;
+            const uint32_t p = j * BLOCK_THREADS + t, key = word[j] >> BLOCK_INDEX_BITS;
+            for (uint32_t h = table_home(key, c[j], mask);; h = (h + 1u) & mask) {
+                const uint32_t old = atomicCAS(&tmp.table[h], HASH_EMPTY, p);
+                if (old == HASH_EMPTY) break;
+                if (sk[old] == key && sc[old] == c[j]) {
+                    atomicMin(&tmp.table[h], p);
+                    break;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+            if (cls[j] != RP_LATE) continue;
+            const uint32_t p = j * BLOCK_THREADS + t, key = word[j] >> BLOCK_INDEX_BITS;
+            for (uint32_t h = table_home(key, c[j], mask);; h = (h + 1u) & mask) {
+                const uint32_t at = tmp.table[h];
+                if (at == HASH_EMPTY) break; // cannot happen: it was entered
+                if (sk[at] == key && sc[at] == c[j]) {
+                    repeat[j] = at != p;
+                    break;
+                }
+            }
+            if (repeat[j] || c[j] == 0u) continue; // (counter 0 is never ahead of anything)
+            // Or an earlier packet that was ahead when it came raised the run's maximum to
+            // exactly c: the first position of the run that reaches c carried it.
+            uint32_t lo = 0, hi = p;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) / 2u;
+                if (sk[mid] == key && smax[mid] >= c[j]) hi = mid;
+                else lo = mid + 1u;
+            }
+            repeat[j] = hi < p && smax[hi] == c[j];
+        }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        const uint32_t p = j * BLOCK_THREADS + t, key = word[j] >> BLOCK_INDEX_BITS;
+        if (key == none) continue;
+        if (cls[j] == RP_NONE || cls[j] == RP_SEEN || repeat[j]) {
+            const uint32_t i = word[j] & (WG_REPLAY_BLOCK_MAX - 1u);
+            result[i] = BNK_WG_REPLAY;
+            out_len[i] = 0;
+        }
+        if (sk[p + 1u] != key) advance_window(state + (size_t)key * WG_REPLAY_WORDS, smax[p]);
+    }
+    // (see replay_small_kernel)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __syncthreads(); // the cleared blocks are in place before bits go in
+#pragma unroll
+    for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+        uint32_t key = NO_PEER;
+        uint64_t block = ~0ull, bit = 0;
+        if (cls[j] != RP_NONE) {
+            const uint32_t k = word[j] >> BLOCK_INDEX_BITS;
+            const uint64_t final_last = *reinterpret_cast<volatile uint64_t *>(state + (size_t)k * WG_REPLAY_WORDS);
+            if ((final_last >> 6) - (c[j] >> 6) < WG_REPLAY_BLOCKS) {
+                key = k;
+                block = c[j] >> 6;
+                bit = 1ull << (c[j] & 63u);
+            }
+        }
+        mark_bits(state, key, block, bit);
+    }
+}
+
 __global__ __launch_bounds__(256) void replay_reset_kernel(uint64_t *state, const uint8_t *flags, uint32_t n_peers)
 {
     const uint32_t total = n_peers * WG_REPLAY_WORDS;
@@ -626,6 +792,11 @@ uint32_t wg_replay_table_slots(uint32_t n)
     return s;
 }
 
+bool wg_replay_one_block(uint32_t n, uint32_t n_peers)
+{
+    return n <= WG_REPLAY_SMALL_MAX || (n <= WG_REPLAY_BLOCK_MAX && key_bits(n_peers) + BLOCK_INDEX_BITS <= 32u);
+}
+
 hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *peer, const uint64_t *counter,
                             uint32_t n, const WgReplayDev &rp, const WgReplayScratch &sc, hipStream_t s)
 {
@@ -638,6 +809,11 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
     if (n <= WG_REPLAY_SMALL_MAX) {
         hipLaunchKernelGGL(replay_small_kernel<WG_REPLAY_SMALL_MAX>, dim3(1), dim3(WG_REPLAY_SMALL_MAX), 0, s,
                            result, out_len, peer, counter, rp.n_peers, n, rp.state, key_bits(rp.n_peers));
+        return hipGetLastError();
+    }
+    if (wg_replay_one_block(n, rp.n_peers)) {
+        hipLaunchKernelGGL(replay_block_kernel, dim3(1), dim3(BLOCK_THREADS), 0, s, result, out_len, peer, counter,
+                           rp.n_peers, n, rp.state, key_bits(rp.n_peers));
         return hipGetLastError();
     }
     const dim3 grid((n + 255u) / 256u);

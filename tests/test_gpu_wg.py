@@ -1406,7 +1406,7 @@ def test_short_uniform_tunnel_batches_device_resident(plen):
         assert not got[5, 16:16 + padded].any()  # a rejected packet's plaintext is cleared
 
 
-@pytest.mark.parametrize("n", [1, 5, 6, 64, 700, 3277])
+@pytest.mark.parametrize("n", [1, 5, 6, 64, 700, 1025, 3277, 4096, 4097])
 @pytest.mark.parametrize("misalign", [False, True])
 def test_small_device_batches_do_their_own_framing(n, misalign):
     """A device-resident batch too small for a lane per packet, whose lengths only the device

@@ -106,7 +106,8 @@ def _expect(wires, rx, keys, filters):
     return res, olen, peer, ctr
 
 
-@pytest.mark.parametrize("mode", ["host_fused", "host_unfused", "device_large", "device_separate", "ring_fused"])
+@pytest.mark.parametrize("mode", ["host_fused", "host_unfused", "device_large", "device_separate", "ring_fused",
+                                  "device_block"])
 def test_replay_windows_match_the_sequential_filter(mode):
     import torch
     from bnk_amd import lib
@@ -118,7 +119,7 @@ def test_replay_windows_match_the_sequential_filter(mode):
     last = [0] * P
     sizes = {"host_fused": [1, 64, 300, 1024, 700], "host_unfused": [300, 1024, 2000, 150],
              "device_large": [5000, 1025, 9000, 3000], "device_separate": [3000, 1025, 6000],
-             "ring_fused": [128, 900, 128]}[mode]
+             "ring_fused": [128, 900, 128], "device_block": [1025, 4096, 2047, 4097, 4095]}[mode]
     seen = set()
     with lib.Context(0) as ctx:
         ctx.keys_set(lib.KEYS_RECV, keys)
@@ -131,7 +132,7 @@ def test_replay_windows_match_the_sequential_filter(mode):
             arena, offs, lens, wires, last = _batch(rng, tx, keys, n, last, near_limit=(b == 2))
             want = _expect(wires, rx, keys, filters)
             total = arena.nbytes
-            if mode in ("device_large", "device_separate"):
+            if mode.startswith("device"):
                 d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
                 d_arena, d_out = d(arena), torch.zeros(total, dtype=torch.uint8, device="cuda:0")
                 res = torch.zeros(n, dtype=torch.uint8, device="cuda:0")

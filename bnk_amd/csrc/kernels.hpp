@@ -253,6 +253,12 @@ hipError_t launch_peer_rank_counting(const uint32_t *peer, void *tmp, uint64_t *
                                      uint64_t *ctr_out, bool advance, uint64_t ctr_limit, uint32_t *status,
                                      hipStream_t s);
 
+// sorted[] = words[] in ascending order of words[i] >> shift, stably; a key beyond n_peers counts
+// as n_peers.  For the batches peer_sort_tmp_bytes gives a size for (else 0): tmp holds that much.
+size_t peer_sort_tmp_bytes(uint32_t n, uint32_t n_peers);
+hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n, uint32_t n_peers, unsigned shift,
+                            void *tmp, hipStream_t s);
+
 // Copy of a byte span whose two ends share their alignment within 16 bytes,
 // one aligned 16-byte piece per lane (used to fetch small spans of pinned
 // host memory).

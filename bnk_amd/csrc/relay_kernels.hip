@@ -99,6 +99,9 @@ constexpr uint32_t RANK_ROW_STEP = 256; // 64 lanes x 16 bytes
 constexpr uint32_t RANK_ROW_STEPS = RANK_TABLE_MAX_KEYS / RANK_ROW_STEP;
 constexpr uint32_t TILE_RUNS_MAX = 32;
 constexpr size_t RANK_TABLE_MAX_BYTES = 64u << 20;
+// Sorting by peer (launch_peer_sort): up to this many keys.  With 4001 of them a tile's row is
+// longer than the tile and it is the library's radix sort or this within 3 % either way.
+constexpr uint32_t PEER_SORT_MAX_KEYS = 2048;
 
 struct RankPlan {
     uint32_t runs;  // runs of 64 packets per tile
@@ -111,9 +114,12 @@ struct RankPlan {
 static RankPlan rank_plan(uint32_t n, uint32_t n_keys)
 {
     RankPlan p{};
-    // about 2048 tiles (a wave each: enough to keep every CU busy), as long as a wave
+    // about 1024 tiles (a wave each: enough to keep every CU busy; with 2048 the table of a
+    // thousand peers is longer than the batch: counters and window sort of 2^17 packets 8 us
+    // more, of 2^18 6), 2048 for large batches (2^20: 5 us less), as long as a wave
     // can hold its tile's keys in registers
-    p.runs = std::min<uint32_t>(TILE_RUNS_MAX, std::max<uint32_t>(1u, (n + 64u * 2048u - 1u) / (64u * 2048u)));
+    const uint32_t run_packets = 64u * (n <= 1u << 19 ? 1024u : 2048u);
+    p.runs = std::min<uint32_t>(TILE_RUNS_MAX, std::max<uint32_t>(1u, (n + run_packets - 1u) / run_packets));
     p.tiles = (n + 64u * p.runs - 1u) / (64u * p.runs);
     p.cols = (n_keys + RANK_ROW_STEP - 1u) / RANK_ROW_STEP * RANK_ROW_STEP;
     p.bytes = ((size_t)p.tiles + 1u) * p.cols * 4u + (size_t)p.cols * 8u;
@@ -323,9 +329,16 @@ hipError_t launch_peer_rank_small(const uint32_t *peer, uint32_t n_keys, uint32_
 // Three launches over the keys, against eight (two of them passes over
 // key-index pairs) for the sort.
 // ---------------------------------------------------------------------------
+// (shift: the key of a packet is keys[i] >> shift, the last key standing for all beyond it; 0:
+// keys[i] itself, and one beyond the table has none)
+__device__ __forceinline__ uint32_t rank_key(uint32_t word, unsigned shift, uint32_t n_keys)
+{
+    return shift ? min(word >> shift, n_keys - 1u) : word;
+}
+
 __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
                                                         uint32_t cols, uint32_t runs, uint32_t *table,
-                                                        uint32_t *status)
+                                                        uint32_t *status, unsigned shift)
 {
     __shared__ __attribute__((aligned(16))) uint32_t cnt[RANK_TABLE_MAX_KEYS];
     const uint32_t lane = threadIdx.x;
@@ -337,7 +350,7 @@ __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, ui
 #pragma unroll
     for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
         const uint32_t i = first + r * 64u + lane;
-        key[r] = r < runs && i < n ? keys[i] : NO_PEER;
+        key[r] = r < runs && i < n ? rank_key(keys[i], shift, n_keys) : NO_PEER;
     }
     __syncthreads();
 #pragma unroll
@@ -402,6 +415,7 @@ __global__ __launch_bounds__(SCAN_PEERS * SCAN_PARTS) void rank_scan_kernel(uint
         // the peer's counter as the batch found it stays behind for the assigning launch;
         // the counter itself moves past what the batch takes
         total[key] = run;
+        if (ctr_base == nullptr) return;
         const uint64_t was = ctr_base[key];
         base_was[key] = was;
         if (advance && run != 0u) ctr_base[key] = ctr_add(was, run, ctr_limit);
@@ -468,6 +482,105 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
     }
 }
 
+// The third launch when the batch is to be sorted by key, stably (three launches where the
+// library's radix sort takes five to nine with its memsets: a tunnel pass of 16000 packets of
+// 100 bytes 100 -> 92 us, 2^17 151 -> 133, 2^18 201 -> 184, 2^20 472 -> 457): a packet's place is where its
+// key's packets begin (every tile scans the totals for itself) plus its rank among them.
+__global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, uint32_t n, uint32_t n_keys,
+                                                        uint32_t cols, uint32_t runs, const uint32_t *table,
+                                                        const uint32_t *total, unsigned bits, unsigned shift,
+                                                        uint32_t *sorted)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t before[RANK_TABLE_MAX_KEYS];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t first = blockIdx.x * runs * 64u;
+    uint32_t word[TILE_RUNS_MAX];
+#pragma unroll
+    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
+        const uint32_t i = first + r * 64u + lane;
+        word[r] = r < runs && i < n ? words[i] : 0u;
+    }
+    {
+        const uint4 *const row = reinterpret_cast<const uint4 *>(table + (size_t)blockIdx.x * cols);
+        const uint4 *const tot = reinterpret_cast<const uint4 *>(total);
+        uint32_t base = 0;
+        for (uint32_t q = 0; q < cols / RANK_ROW_STEP; q++) {
+            // (columns beyond the keys hold nothing that was written)
+            const uint32_t c = (q * 64u + lane) * 4u;
+            uint4 t = tot[q * 64u + lane], v = row[q * 64u + lane];
+            if (c >= n_keys) t.x = 0;
+            if (c + 1u >= n_keys) t.y = 0;
+            if (c + 2u >= n_keys) t.z = 0;
+            if (c + 3u >= n_keys) t.w = 0;
+            const uint32_t mine = t.x + t.y + t.z + t.w;
+            uint32_t inc = mine;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t o = (uint32_t)__shfl_up((int)inc, off, 64);
+                if ((int)lane >= off) inc += o;
+            }
+            const uint32_t s0 = base + inc - mine;
+            v.x += s0;
+            v.y += s0 + t.x;
+            v.z += s0 + t.x + t.y;
+            v.w += s0 + t.x + t.y + t.z;
+            reinterpret_cast<uint4 *>(before)[q * 64u + lane] = v;
+            base += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
+        if (r < runs) { // uniform
+            const bool valid = first + r * 64u + lane < n;
+            const uint32_t kk = rank_key(word[r], shift, n_keys);
+            unsigned long long same = __ballot(valid);
+            for (unsigned b = 0; b < bits; b++) {
+                const unsigned long long m = __ballot((kk >> b) & 1u);
+                same &= ((kk >> b) & 1u) ? m : ~m;
+            }
+            if (valid) {
+                const uint32_t lower = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+                const uint32_t at = before[kk];
+                sorted[at + lower] = word[r];
+                // (see rank_assign_kernel)
+                if (lower == 0u) before[kk] = at + (uint32_t)__popcll(same);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// One key more than there are peers: the packets without one, last.
+static RankPlan sort_plan(uint32_t n, uint32_t n_peers)
+{
+    RankPlan p = rank_plan(n, n_peers + 1u);
+    p.fits = p.fits && n_peers + 1u <= PEER_SORT_MAX_KEYS;
+    return p;
+}
+
+size_t peer_sort_tmp_bytes(uint32_t n, uint32_t n_peers)
+{
+    const RankPlan p = sort_plan(n, n_peers);
+    return p.fits ? p.bytes : 0;
+}
+
+hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n, uint32_t n_peers, unsigned shift,
+                            void *tmp, hipStream_t s)
+{
+    const RankPlan plan = sort_plan(n, n_peers);
+    const uint32_t n_keys = n_peers + 1u;
+    uint32_t *table = static_cast<uint32_t *>(tmp), *total = table + (size_t)plan.tiles * plan.cols;
+    hipLaunchKernelGGL(rank_count_kernel, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+                       (uint32_t *)nullptr, shift);
+    hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS), dim3(SCAN_PEERS * SCAN_PARTS), 0, s,
+                       table, plan.tiles, n_keys, plan.cols, total, (uint64_t *)nullptr, (uint64_t *)nullptr, 0, 0ull);
+    hipLaunchKernelGGL(rank_place_kernel, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+                       total, key_bits(n_keys), shift, sorted);
+    return hipGetLastError();
+}
+
 static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &plan, void *tmp,
                                          uint64_t *ctr_base, uint32_t n_keys, uint32_t n, uint64_t *ctr_out,
                                          bool advance, uint64_t ctr_limit, bool zero_others, uint32_t *status,
@@ -477,7 +590,7 @@ static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &p
     uint32_t *total = table + (size_t)plan.tiles * plan.cols;
     uint64_t *base_was = reinterpret_cast<uint64_t *>(total + plan.cols);
     hipLaunchKernelGGL(rank_count_kernel, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
-                       table, status);
+                       table, status, 0u);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS),
                        dim3(SCAN_PEERS * SCAN_PARTS), 0, s, table, plan.tiles, n_keys, plan.cols, total, ctr_base,
                        base_was, advance ? 1 : 0, ctr_limit);

@@ -782,7 +782,7 @@ size_t wg_replay_tmp_bytes(uint32_t n, uint32_t n_peers)
                                                 (const uint32_t *)nullptr, (uint32_t *)nullptr, (size_t)n, 0,
                                                 key_bits(n_peers));
     b = ((size_t)(n + SEG_BLOCK - 1u) / SEG_BLOCK) * 12u + 16u; // the scan's block carries
-    return std::max(std::max(a, b), c);
+    return std::max(std::max(a, b), std::max(c, peer_sort_tmp_bytes(n, n_peers)));
 }
 
 uint32_t wg_replay_table_slots(uint32_t n)
@@ -829,8 +829,11 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
         if (!sc.keys_ready)
             hipLaunchKernelGGL(replay_keys_packed_kernel, grid, dim3(256), 0, s, result, peer, rp.n_peers, n,
                                index_bits, sc.keys);
-        e = rocprim::radix_sort_keys<SortConfig>(sc.tmp, bytes, sc.keys, sc.idx, (size_t)n, index_bits,
-                                                 index_bits + peer_bits, s);
+        const size_t counting = peer_sort_tmp_bytes(n, rp.n_peers);
+        e = counting != 0 && counting <= sc.tmp_bytes
+                ? launch_peer_sort(sc.keys, sc.idx, n, rp.n_peers, index_bits, sc.tmp, s)
+                : rocprim::radix_sort_keys<SortConfig>(sc.tmp, bytes, sc.keys, sc.idx, (size_t)n, index_bits,
+                                                       index_bits + peer_bits, s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(replay_unpack_kernel, dim3(seg_blocks), dim3(SEG_BLOCK), 0, s, sc.idx, counter, n,
                            index_bits, peer_bits, sc.skeys, sc.sidx, sc.sctr, sc.sval, carry_x, carry_open);

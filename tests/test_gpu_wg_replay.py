@@ -310,6 +310,46 @@ def test_window_pass_with_more_peers_than_a_packed_sort_key_holds():
         assert np.array_equal(olen.cpu().numpy() != 0, want == lib.WG_OK)
 
 
+@pytest.mark.parametrize("n_peers,n_total", [(255, 66000), (2047, 66000), (2048, 66000), (3, 530000)])
+def test_window_pass_sorted_by_counting_and_where_that_ends(n_peers, n_total):
+    """A key more than there are peers fills the counting sort's row of 256 or the last of the
+    rows it is used for, or goes beyond them; tiles of one run and of several, the last one
+    ragged; some tags forged, so that packets without a sender take part."""
+    import torch
+    from bnk_amd import lib
+    rng = np.random.default_rng(n_peers)
+    tx = [(10 + 3 * i, 500000 + 5 * i, 0x64400000 + i, 0xFFFFFFFF) for i in range(n_peers)]
+    rx = [(p[1], p[0], p[2], p[3]) for p in tx]
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    jump_rows = rng.choice(n_peers, max(1, n_peers // 8), replace=False)
+    with lib.Context(0) as txc, lib.Context(0) as rxc:
+        txc.keys_set(lib.KEYS_SEND, keys)
+        txc.wg_peers_set(tx)
+        rxc.keys_set(lib.KEYS_RECV, keys)
+        rxc.wg_peers_set(rx)
+        wire, stride, wire_len, peer, ctr = _traffic(txc, tx, n_total // 3, n_total // 5, n_total, 40, jump_rows, rng)
+        forged = rng.choice(n_total, n_total // 50, replace=False)
+        wire.reshape(-1)[forged.astype(np.int64) * stride + wire_len - 1] ^= 1
+        good = np.ones(n_total, bool)
+        good[forged] = False
+        want = np.full(n_total, lib.WG_AUTH_FAIL, np.uint8)
+        want[good] = _window_expectation(peer[good], ctr[good], n_peers)
+        d_wire = torch.from_numpy(np.ascontiguousarray(wire)).to("cuda:0")
+        d_out = torch.zeros(wire.nbytes, dtype=torch.uint8, device="cuda:0")
+        res = torch.zeros(n_total, dtype=torch.uint8, device="cuda:0")
+        olen, gp = (torch.zeros(n_total, dtype=torch.int32, device="cuda:0") for _ in range(2))
+        gc = torch.zeros(n_total, dtype=torch.int64, device="cuda:0")
+        torch.cuda.synchronize()
+        rxc.wg_decap(lib.make_batch(d_wire, wire.nbytes, n_total, lib.MEM_DEVICE, stride=stride, length=wire_len),
+                     lib.make_batch(d_out, wire.nbytes, n_total, lib.MEM_DEVICE, stride=stride), res, olen, gp, gc)
+        rxc.sync()
+        assert np.array_equal(gp.cpu().numpy().astype(np.uint32), peer)
+        got = res.cpu().numpy()
+        bad = np.flatnonzero(got != want)
+        assert bad.size == 0, f"result differs at {bad[:5]}: got {got[bad[:5]]} want {want[bad[:5]]}"
+        assert (want == lib.WG_REPLAY).sum() > 1000 and (want == lib.WG_OK).sum() > 1000
+
+
 def test_window_pass_of_a_host_batch_that_goes_through_in_chunks():
     """A host batch beyond the size that runs in one piece is cut into chunks,
     each with a window pass of its own continuing the one before: results are

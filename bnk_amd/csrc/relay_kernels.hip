@@ -329,13 +329,13 @@ hipError_t launch_peer_rank_small(const uint32_t *peer, uint32_t n_keys, uint32_
 // Three launches over the keys, against eight (two of them passes over
 // key-index pairs) for the sort.
 // ---------------------------------------------------------------------------
-// (shift: the key of a packet is keys[i] >> shift, the last key standing for all beyond it; 0:
-// keys[i] itself, and one beyond the table has none)
+// SHIFTED: the key of a packet is keys[i] >> shift, the last key standing for all beyond it.
 __device__ __forceinline__ uint32_t rank_key(uint32_t word, unsigned shift, uint32_t n_keys)
 {
-    return shift ? min(word >> shift, n_keys - 1u) : word;
+    return min(word >> shift, n_keys - 1u);
 }
 
+template <bool SHIFTED>
 __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
                                                         uint32_t cols, uint32_t runs, uint32_t *table,
                                                         uint32_t *status, unsigned shift)
@@ -350,11 +350,12 @@ __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, ui
 #pragma unroll
     for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
         const uint32_t i = first + r * 64u + lane;
-        key[r] = r < runs && i < n ? rank_key(keys[i], shift, n_keys) : NO_PEER;
+        key[r] = r < runs && i < n ? keys[i] : NO_PEER;
     }
     __syncthreads();
 #pragma unroll
     for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
+        if (SHIFTED && r < runs && first + r * 64u + lane < n) key[r] = rank_key(key[r], shift, n_keys);
         if (key[r] < n_keys) atomicAdd(&cnt[key[r]], 1u);
         // (keys straight from a caller's peer array: one beyond the table gets no counter and is reported)
         else if (status && r < runs && first + r * 64u + lane < n) status_raise(status, STATUS_PEER_RANGE);
@@ -572,7 +573,7 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
     const RankPlan plan = sort_plan(n, n_peers);
     const uint32_t n_keys = n_peers + 1u;
     uint32_t *table = static_cast<uint32_t *>(tmp), *total = table + (size_t)plan.tiles * plan.cols;
-    hipLaunchKernelGGL(rank_count_kernel, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+    hipLaunchKernelGGL(rank_count_kernel<true>, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
                        (uint32_t *)nullptr, shift);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS), dim3(SCAN_PEERS * SCAN_PARTS), 0, s,
                        table, plan.tiles, n_keys, plan.cols, total, (uint64_t *)nullptr, (uint64_t *)nullptr, 0, 0ull);
@@ -589,7 +590,7 @@ static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &p
     uint32_t *table = static_cast<uint32_t *>(tmp);
     uint32_t *total = table + (size_t)plan.tiles * plan.cols;
     uint64_t *base_was = reinterpret_cast<uint64_t *>(total + plan.cols);
-    hipLaunchKernelGGL(rank_count_kernel, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
+    hipLaunchKernelGGL(rank_count_kernel<false>, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
                        table, status, 0u);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS),
                        dim3(SCAN_PEERS * SCAN_PARTS), 0, s, table, plan.tiles, n_keys, plan.cols, total, ctr_base,

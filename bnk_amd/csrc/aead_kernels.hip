@@ -1766,7 +1766,12 @@ bool aead_runs_spread(const AeadArgs &a)
 // work the launches of a lane per packet overlap: 16384 x 1420 38 us against 50, x 600 25
 // against 27, 32768 x 1420 66 against 55.  Where lengths vary the other choice has the
 // grouping ahead of it as well: 40000 packets of 1 to 1420 bytes 61 us against 83, 57344 84
-// against 87, 65536 97 against 89.
+// against 87, 65536 97 against 89.  Short packets end it earlier, since a lane each is then
+// done in no time (pairs with three streams at work, slots of a multiple of 128 bytes): 32000
+// of 1 to 44 bytes 16 us against 18, 40000 19.0 against 18.5, 48000 22 against 19; 1 to 200
+// bytes 40000 27 against 28, 48000 33 against 27; 1 to 400 bytes 48000 40 against 44, 57000 47
+// against 46.  (Back to back without gaps they hold out longer, 1 to 200 bytes 29 against 35 at
+// 57000, but the host sees the room alone.)
 //
 // Up to 10240 packets whose lengths the host does not know, five per wave: whatever mix of
 // up to 1471 bytes they are, a piece is then all that a run ever holds, and the launch lasts
@@ -1778,8 +1783,8 @@ static uint32_t split_packets(const AeadArgs &a)
     // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
     if (a.spread_max == 0 || a.order || aead_runs_spread(a)) return 0;
     const uint32_t per = (a.n + 2047u) / 2048u;
-    if (per > (a.lens ? 28u : 12u)) return 0;
     const uint32_t room = a.lens ? (uint32_t)std::min<uint64_t>(a.in_bytes / a.n, 1500u) : a.len;
+    if (per > (!a.lens ? 12u : room < 256u ? 18u : 27u)) return 0;
     const uint32_t blocks = (room + 63u) / 64u, pieces = blocks / 2u + 1u;
     auto fits = [&](uint32_t k, uint32_t q) {
         if (!a.lens) return k * ((pieces + q - 1u) / q) <= 64u;

@@ -972,7 +972,7 @@ BNK_DEV LanePacket lane_packet(const AeadArgs &a, uint32_t t, bool in_batch)
         const uint64_t at = a.in_off ? in_off_ld : (uint64_t)i * a.in_stride;
         // the datagram where it is read, and the plaintext where it would be written
         const bool beyond = beyond_arena(at, len, a.in_limit) ||
-                            beyond_arena((a.out_off ? out_off_ld : (uint64_t)i * a.out_stride) + a.out_skip,
+                            beyond_arena(a.out_off ? out_off_ld : (uint64_t)i * a.out_stride, a.out_skip,
                                          len >= 32u ? len - 32u : 0u, a.out_limit);
         if (in_batch && beyond) status_raise(a.status, STATUS_BOUNDS);
         if (beyond || len < 32u) wg_res = BNK_WG_BAD_HEADER;
@@ -1011,11 +1011,11 @@ BNK_DEV LanePacket lane_packet(const AeadArgs &a, uint32_t t, bool in_batch)
     p.skipped = (a.skip != nullptr && skip_ld != 0) || wg_res != BNK_WG_OK;
     p.bad_peer = p.pr >= a.n_peers;
     p.too_short = OPEN && len < 16u;
-    const uint64_t in_at = (a.in_off ? in_off_ld : (uint64_t)i * a.in_stride) + a.in_skip;
-    const uint64_t out_at = (a.out_off ? out_off_ld : (uint64_t)i * a.out_stride) + a.out_skip;
+    const uint64_t in_at = a.in_off ? in_off_ld : (uint64_t)i * a.in_stride;
+    const uint64_t out_at = a.out_off ? out_off_ld : (uint64_t)i * a.out_stride;
     // seal reads len and writes len + 16, open reads len (tag included) and writes len - 16
-    p.outside = beyond_arena(in_at, len, a.in_limit) ||
-                beyond_arena(out_at, OPEN ? (p.too_short ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
+    p.outside = beyond_arena(in_at, a.in_skip, len, a.in_limit) ||
+                beyond_arena(out_at, a.out_skip, OPEN ? (p.too_short ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
                 (wraps && (a.in_limit | a.out_limit) != 0);
     p.ctr = decap ? wg_ctr : a.counters ? ctr_ld : a.counter0 + i;
     // a keypair that has used up its nonces sends nothing more (wireguard-go device/send.go)
@@ -1028,8 +1028,8 @@ BNK_DEV LanePacket lane_packet(const AeadArgs &a, uint32_t t, bool in_batch)
     if (OPEN) len -= 16u;
     p.len = p.have ? len : 0u;
     p.len_in = encap ? min(len_plain, p.len) : p.len;
-    p.src = p.have ? a.in + in_at : nullptr;
-    p.dst = p.have ? a.out + out_at : nullptr;
+    p.src = p.have ? a.in + in_at + a.in_skip : nullptr;
+    p.dst = p.have ? a.out + out_at + a.out_skip : nullptr;
     return p;
 }
 
@@ -1415,10 +1415,11 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     uint64_t ctr = 0;
     if (!WG) {
         // (framing launches only run on layouts the host has checked)
-        const uint64_t in_at = (uint64_t)(src - a.in), out_at = (uint64_t)(dst - a.out);
+        const uint64_t in_at = a.in_off ? in_off_ld : (uint64_t)i * a.in_stride;
+        const uint64_t out_at = a.out_off ? out_off_ld : (uint64_t)i * a.out_stride;
         const bool short_ct = OPEN && len < 16u;
-        if (beyond_arena(in_at, len, a.in_limit) ||
-            beyond_arena(out_at, OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
+        if (beyond_arena(in_at, a.in_skip, len, a.in_limit) ||
+            beyond_arena(out_at, a.out_skip, OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
             (len > MAX_PACKET_BYTES && (a.in_limit | a.out_limit) != 0)) {
             if (lane == 0 && !skipped) {
                 status_raise(a.status, STATUS_BOUNDS);

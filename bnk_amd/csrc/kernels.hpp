@@ -190,6 +190,13 @@ __host__ __device__ inline bool beyond_arena(uint64_t off, uint64_t len, uint64_
 {
     return limit != 0 && (off > limit || len > limit - off);
 }
+// The same for the `len` bytes that begin `skip` bytes behind a packet's offset word (room for a
+// header): all of [off, off + skip + len) counts, and off + skip is not formed, which an offset
+// word close to 2^64 would carry around to the arena's first bytes.
+__host__ __device__ inline bool beyond_arena(uint64_t off, uint32_t skip, uint64_t len, uint64_t limit)
+{
+    return beyond_arena(off, skip + len, limit);
+}
 #if defined(__HIPCC__)
 __device__ inline void status_raise(uint32_t *status, uint32_t condition)
 {

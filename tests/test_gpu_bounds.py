@@ -339,6 +339,47 @@ def test_framing_skips_slots_outside_the_arena(n):
         assert np.array_equal(got, expect)
 
 
+@pytest.mark.parametrize("n,spread_max", [(500, 4096), (5000, 4096), (500, 0)])
+def test_slot_offsets_that_wrap_are_outside_the_arena(n, spread_max):
+    """A slot's packet lies 16 bytes behind its offset word: a word just below 2^64 must not
+    carry around to the arena's first bytes.  Its slot is refused like any other outside the
+    arena, and nothing lands ahead of the arena or in the slot that lies there."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    key = rng.integers(0, 256, (1, 32), dtype=np.uint8)
+    lens = rng.choice([0, 20, 100, 1400], n).astype(np.uint32)
+    slot = (16 + lens.astype(np.int64) + 15 + 16 + 15) & ~15
+    off = np.concatenate([[0], np.cumsum(slot)[:-1]]).astype(np.uint64)
+    total = int(slot.sum())
+    arena = rng.integers(0, 256, total, dtype=np.uint8)
+    off_b = off.copy()
+    bad = np.array([1, 2, n // 2, n - 2, n - 1])
+    off_b[bad] = [2**64 - 16, 2**64 - 1, 2**64 - 15, 2**64 - 48, 2**64 - 17]
+    want, want_len = arena.copy(), np.zeros(n, np.uint32)
+    for i in range(n):
+        if i in bad:
+            continue
+        o = int(off[i])
+        dg = O.wg_encap(arena[o + 16:o + 16 + int(lens[i])].tobytes(), 1420, key[0].tobytes(), 77, i)
+        want[o:o + len(dg)] = np.frombuffer(dg, np.uint8)
+        want_len[i] = len(dg)
+    with lib.Context(0) as ctx:
+        ctx.set_spread_max_packets(spread_max)
+        ctx.keys_set(lib.KEYS_SEND, key)
+        ctx.wg_peers_set([(5, 77, 0x64400001, 0xFFFFFFFF)])
+        slots = Banded(arena)
+        d_off, d_lens = _dev(off_b.view(np.int64)), _dev(lens.astype(np.int32))
+        d_wl = torch.full((n,), 77, dtype=torch.int32, device="cuda:0")
+        torch.cuda.synchronize()
+        ctx.wg_encap(lib.make_batch(slots.ptr, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens), 1420, d_wl)
+        _expect_inval(ctx)
+        assert slots.guards_intact()
+        assert np.array_equal(d_wl.cpu().numpy().astype(np.uint32), want_len)
+        assert np.array_equal(slots.arena(), want)
+
+
 def test_relay_skips_packets_outside_the_arenas():
     import torch
     from bnk_amd import lib

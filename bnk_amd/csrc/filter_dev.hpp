@@ -93,6 +93,7 @@ struct FilterArgs {
     uint64_t limit;       // arena size for device-resident batches with per-packet arrays: a
                           // packet reaching beyond it is not read, fails the parse and
                           // raises STATUS_BOUNDS.  0: the host has checked the layout
+    uint32_t ahead;       // note only: bytes of the arena that lie ahead of pkts (with limit)
     uint32_t trim;        // bytes at the end of each packet that are not payload
     uint32_t small_in_lds; // set by the launcher: there is LDS for present_small (a launch reads it
                           // while the table has seen at most SMALL_KEYS_MAX keys)

@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.n; i += stride) {
         const uint64_t at = a.off ? a.off[i] : (uint64_t)i * a.stride;
         const uint32_t len = a.lens ? a.lens[i] : a.len;
-        if (beyond_arena(at, len, a.limit)) {
+        if (beyond_arena(at, a.ahead, len, a.limit)) {
             status_raise(a.status, STATUS_BOUNDS);
             continue;
         }

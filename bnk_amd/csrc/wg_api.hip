@@ -462,6 +462,9 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             fa.lens = b.lens ? b.lens + lo : nullptr;
             fa.stride = slots->stride;
             fa.len = slots->len;
+            // (the header's room counts: a slot begins where the arena does)
+            fa.limit = b.limit;
+            fa.ahead = 16;
             fa.status = ctx->d_status;
             fa.now = *note_now;
             fa.n = hi - lo;

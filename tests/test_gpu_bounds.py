@@ -380,6 +380,56 @@ def test_slot_offsets_that_wrap_are_outside_the_arena(n, spread_max):
         assert np.array_equal(slots.arena(), want)
 
 
+@pytest.mark.parametrize("n", [300, 5000])
+def test_noting_ahead_of_encap_skips_slots_outside_the_arena(n):
+    """NoteOutbound within the sending call looks at a packet only where it lies in the arena.
+    Behind the arena lie slots with packets as good as any: they are neither sent nor noted."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    key = rng.integers(0, 256, (1, 32), dtype=np.uint8)
+    now, length, slot = W.T0_NS, 60, 112
+    rec = np.zeros((n + 3, slot), np.uint8)
+    rec[:, 16] = 0x45
+    rec[:, 19] = length
+    rec[:, 25] = 17
+    rec[:, 28:32] = [100, 64, 0, 1]
+    rec[:, 32:36] = [100, 64, 9, 9]
+    rec[:, 36:40] = np.stack([np.arange(n + 3) >> 8, np.arange(n + 3) & 255, np.full(n + 3, 0), np.full(n + 3, 53)], 1)
+    off = np.arange(n, dtype=np.uint64) * slot
+    bad = np.array([1, n // 2, n - 1])
+    # behind the arena, half in it (16 bytes of the packet), and by a word that wraps
+    off_b = off.copy()
+    off_b[bad] = [n * slot + slot, n * slot - 32, 2**64 - 16]
+    good = np.setdiff1d(np.arange(n), bad)
+    rules = [([(0, 0)], "tcp", [(0, 0)])]
+    ora = O.Filter()
+    ora.set_rules(rules)
+    inner = np.ascontiguousarray(rec[good, 16:16 + length]).reshape(-1)
+    ora.note_outbound_batch(inner, np.arange(good.size, dtype=np.uint64) * length, np.full(good.size, length, np.uint32), now)
+    want_len = np.zeros(n, np.uint32)
+    want_len[good] = 16 + 64 + 16
+    with lib.Context(0) as ctx:
+        ctx.keys_set(lib.KEYS_SEND, key)
+        ctx.wg_peers_set([(5, 77, 0x64400001, 0xFFFFFFFF)])
+        ctx.filter_set_rules(rules)
+        slots = Banded(rec.reshape(-1))
+        d_off, d_lens = _dev(off_b.view(np.int64)), _dev(np.full(n, length, np.int32))
+        d_wl = torch.full((n,), 77, dtype=torch.int32, device="cuda:0")
+        torch.cuda.synchronize()
+        ctx.wg_note_encap(lib.make_batch(slots.ptr, n * slot, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens), 1420, now, d_wl)
+        _expect_inval(ctx)
+        assert np.array_equal(d_wl.cpu().numpy().astype(np.uint32), want_len)
+        assert slots.guards_intact() and np.array_equal(slots.arena()[n * slot:], rec[n:].reshape(-1))
+        assert ctx.filter_flows() == ora.flows()
+        # an arena that ends within the first header's room
+        ctx.wg_note_encap(lib.make_batch(slots.ptr, 8, 1, lib.MEM_DEVICE, offsets=_dev(off[n // 2:n // 2 + 1].view(np.int64) * 0),
+                                         lens=_dev(np.full(1, length, np.int32))), 1420, now + 1, d_wl)
+        _expect_inval(ctx)
+        assert ctx.filter_flows() == ora.flows()
+
+
 def test_relay_skips_packets_outside_the_arenas():
     import torch
     from bnk_amd import lib

@@ -1,0 +1,101 @@
+// Which AEAD launch a batch gets: a wave per packet, a few lanes per packet or a lane per packet.
+// Host code, of sizes and kinds of memory only (tests/cpp/route_test.cpp runs it without a GPU).
+#pragma once
+#include <math.h>
+
+#include <algorithm>
+
+#include "kernels.hpp"
+
+namespace bnk {
+
+// Which launch?  Packets in GPU memory (us per launch of n packets in a row, all of
+// them resident at once; seal and open within 2 us of each other):
+//   a wave per packet   9 + 4.2 per 1000 packets at 1420 bytes, 3.3 at 60
+//   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2)
+//   a lane per packet   5 + 2.75 per ChaCha20 block of the longest packet, and 20 more
+//                       for the grouping where lengths vary
+// so 4096 packets x 1420 take 21 / 18 / 71 us, 16384 66 / 26 / 71, and 24000 packets of 1
+// to 1420 bytes - / 35 / 97.
+//
+// Packets in host memory (over_link): a wave per packet reads them where they are, the
+// others fetch the whole span first: about 17 us + 2.7 to 3.3 ns per packet (200 to 1420
+// bytes) against a lane per packet: measured crossovers 3,000 packets of 60 bytes, 4,800 of
+// 200, 16,400 of 1420.  With the common length known the rule stays just under them;
+// without it the caller's threshold stands alone.
+//
+// True when the launch will run one wave per packet (then order[] is not used and callers need
+// not build it).
+inline bool aead_runs_spread(const AeadArgs &a)
+{
+    // (framing behind a header: the host has not seen that every packet fits 63 blocks)
+    if (a.wg.mode != WG_FUSE_OFF && a.in_skip != 0u && !a.over_link) return false;
+    if (a.over_link) {
+        if (a.lens) return a.n <= a.spread_max;
+        const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
+        return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
+    }
+    // 3072 by default: beyond it the wave-per-packet launch goes over the chip once more (a pair
+    // of launches of 3000 packets of 1 to 1420 bytes 31 us against 32 split, of 3200 42 against 32)
+    const uint64_t most = 3ull * a.spread_max / 4;
+    if (a.lens) return a.n <= most;
+    return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);
+}
+
+// Packets per wave of the launch that splits packets over lanes, 0 where a launch of
+// a lane per packet is the better one.
+//
+// How many: n / 2048 of them fill the chip with waves once and say how many pieces a run
+// must hold; what decides the cost is then how many of a wave's 64 lanes have a run, so the
+// wave takes as many more as still fit at that length (16384 packets x 1420: 10 instead of 8,
+// 38 us a pair of launches instead of 46 with three streams at work, 58 on one stream either
+// way).  Where the host does not know the lengths the room per packet in the arena stands for
+// their mean, with a margin for how much of it a wave may get: beyond 64 lanes all of a wave's
+// runs get longer (24000 packets of 1 to 1420 bytes, 15 per wave instead of 12: 39 us instead
+// of 47 on three streams, 70 instead of 63 on one).
+//
+// Where it ends: on one stream it is ahead up to where lanes fill the chip (65536 x 1420: 121
+// us a pair against 145), but it does half as much work again, and with several streams at
+// work the launches of a lane per packet overlap: 16384 x 1420 38 us against 50, x 600 25
+// against 27, 32768 x 1420 66 against 55.  Where lengths vary the other choice has the
+// grouping ahead of it as well: 40000 packets of 1 to 1420 bytes 61 us against 83, 57344 84
+// against 87, 65536 97 against 89.  Short packets end it earlier, since a lane each is then
+// done in no time (pairs with three streams at work, slots of a multiple of 128 bytes): 32000
+// of 1 to 44 bytes 16 us against 18, 40000 19.0 against 18.5, 48000 22 against 19; 1 to 200
+// bytes 40000 27 against 28, 48000 33 against 27; 1 to 400 bytes 48000 40 against 44, 57000 47
+// against 46.  (Back to back without gaps they hold out longer, 1 to 200 bytes 29 against 35 at
+// 57000, but the host sees the room alone.)
+//
+// Up to 10240 packets whose lengths the host does not know, five per wave: whatever mix of
+// up to 1471 bytes they are, a piece is then all that a run ever holds, and the launch lasts
+// as long as that (3400 packets of 1 to 1420 bytes 46 -> 32 us a pair against as many as fit on
+// average, 10000 51 -> 40).
+constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
+constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
+inline uint32_t aead_split_packets(const AeadArgs &a)
+{
+    // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
+    if (a.spread_max == 0 || a.order || aead_runs_spread(a)) return 0;
+    const uint32_t per = (a.n + 2047u) / 2048u;
+    const uint32_t room = a.lens ? (uint32_t)std::min<uint64_t>(a.in_bytes / a.n, 1500u) : a.len;
+    if (per > (!a.lens ? 12u : room < 256u ? 18u : 27u)) return 0;
+    const uint32_t blocks = (room + 63u) / 64u, pieces = blocks / 2u + 1u;
+    auto fits = [&](uint32_t k, uint32_t q) {
+        if (!a.lens) return k * ((pieces + q - 1u) / q) <= 64u;
+        const double mean = (double)room / (128.0 * q) + 1.0;
+        return k * mean + 0.3 * mean * sqrt((double)k) <= 64.0;
+    };
+    uint32_t q = 1, k = per;
+    if (a.lens && per <= SPLIT_ALWAYS_ONE) return std::max(per, SPLIT_ALWAYS_ONE);
+    while (q < pieces && !fits(k, q)) q++;
+    while (k < SPLIT_MAX_PACKETS && fits(k + 1u, q)) k++;
+    return a.lens || 150u + 920u * q < 275u * (blocks + 1u) ? k : 0u;
+}
+
+// True when the launch would run faster with order[] (a lane per packet, lengths vary).
+inline bool aead_wants_order(const AeadArgs &a)
+{
+    return a.lens && a.n > 64 && !aead_runs_spread(a) && aead_split_packets(a) == 0;
+}
+
+} // namespace bnk

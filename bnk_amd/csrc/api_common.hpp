@@ -10,6 +10,7 @@
 #include <new>
 #include <string>
 
+#include "aead_route.hpp"
 #include "ctx.hpp"
 
 namespace bnk {

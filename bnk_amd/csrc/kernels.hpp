@@ -204,11 +204,7 @@ __device__ inline void status_raise(uint32_t *status, uint32_t condition)
 }
 #endif
 
-// True when the launch will run one wave per packet (then order[] is not used
-// and callers need not build it).
-bool aead_runs_spread(const AeadArgs &a);
-// True when the launch would run faster with order[] (a lane per packet, lengths vary).
-bool aead_wants_order(const AeadArgs &a);
+// (which of the AEAD kernels they launch: aead_route.hpp)
 hipError_t launch_aead_seal(const AeadArgs &a, hipStream_t s);
 hipError_t launch_aead_open(const AeadArgs &a, hipStream_t s);
 

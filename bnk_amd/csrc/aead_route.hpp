@@ -28,8 +28,9 @@ namespace bnk {
 // not build it).
 inline bool aead_runs_spread(const AeadArgs &a)
 {
-    // (framing behind a header: the host has not seen that every packet fits 63 blocks)
-    if (a.wg.mode != WG_FUSE_OFF && a.in_skip != 0u && !a.over_link) return false;
+    // (framing behind a header: the host has not seen that every packet fits 63 blocks, and the
+    // wave-per-packet kernel does that framing for no other)
+    if (a.wg.mode != WG_FUSE_OFF && a.in_skip != 0u) return false;
     if (a.over_link) {
         if (a.lens) return a.n <= a.spread_max;
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;

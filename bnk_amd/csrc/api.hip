@@ -131,6 +131,7 @@ int aead_batch_host_direct(bnk_ctx *ctx, bool open, const bnk_batch *in, const b
     if (aead_runs_spread(a)) {
         a.in = d_in + sin.lo;
     } else {
+        a.over_link = false;
         const uint32_t mis = (uint32_t)((uintptr_t)(d_in + sin.lo) & 127u);
         HIPCHK(ctx, ctx->in_arena.reserve(sin.size() + 160));
         HIPCHK(ctx, launch_pull(d_in + sin.lo, ctx->in_arena.as<uint8_t>() + mis, sin.size(), ctx->stream));

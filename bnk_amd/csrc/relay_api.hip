@@ -87,6 +87,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
                     // a wave per packet reads the ring itself (see aead_batch_host_direct)
                     op.in = d_ring_in + sin.lo;
                 } else {
+                    op.over_link = false;
                     HIPCHK(ctx, ctx->in_arena.reserve(sin.size() + 160));
                     HIPCHK(ctx, launch_pull(d_ring_in + sin.lo, ctx->in_arena.as<uint8_t>() + mis, sin.size(), ctx->stream));
                     op.in = ctx->in_arena.as<uint8_t>() + mis;

@@ -408,6 +408,8 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         d_wire_len = wire_len;
     }
 
+    const bool over_link = ring_out != nullptr && wave_per_packet; // (else they have been fetched)
+
     for (DevBuf *buf : {&ctx->r_keys, &ctx->r_idx, &ctx->r_skeys, &ctx->r_sidx, &ctx->wg_padded})
         HIPCHK(ctx, buf->reserve((size_t)n * 4));
     HIPCHK(ctx, ctx->r_ctr_out.reserve((size_t)n * 8));
@@ -478,7 +480,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         if (fits) {
             AeadArgs se{};
             se.spread_max = ctx->spread_max;
-            se.over_link = ring_out != nullptr;
+            se.over_link = over_link;
             se.keys = ctx->d_keys[BNK_KEYS_SEND];
             se.n_peers = pe.n;
             se.status = ctx->d_status;
@@ -504,7 +506,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         }
         AeadArgs se{};
         se.spread_max = ctx->spread_max;
-        se.over_link = ring_out != nullptr;
+        se.over_link = over_link;
         se.in_bytes = slots->bytes;
         se.keys = ctx->d_keys[BNK_KEYS_SEND];
         se.n_peers = pe.n;
@@ -795,6 +797,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         d_peer = peer;
         d_counter = counter;
     }
+    const bool over_link = direct && wave_per_packet; // (else they have been fetched)
     HIPCHK(ctx, ctx->wg_ctlen.reserve((size_t)n * 4));
     HIPCHK(ctx, ctx->r_auth.reserve(n));
     if (wire->lens) {
@@ -891,7 +894,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         if (fits) {
             AeadArgs op{};
             op.spread_max = ctx->spread_max;
-            op.over_link = direct;
+            op.over_link = over_link;
             op.keys = ctx->d_keys[BNK_KEYS_RECV];
             op.n_peers = pe.n;
             op.status = ctx->d_status;
@@ -921,7 +924,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         }
         AeadArgs op{};
         op.spread_max = ctx->spread_max;
-        op.over_link = direct;
+        op.over_link = over_link;
         op.in_bytes = wire->bytes;
         op.keys = ctx->d_keys[BNK_KEYS_RECV];
         op.n_peers = pe.n;

@@ -1,10 +1,10 @@
 // CPU check of the host-side rules around a launch (bnk_amd/csrc): which packets lie in the
-// arena.  Prints PASS/FAIL lines; exit status is the number of failures.
+// arena and which AEAD launch a batch gets.  Prints PASS/FAIL lines; exit status is the number of failures.
 #include <stdio.h>
 
 #include <initializer_list>
 
-#include "../../bnk_amd/csrc/kernels.hpp"
+#include "../../bnk_amd/csrc/aead_route.hpp"
 
 using namespace bnk;
 
@@ -33,9 +33,55 @@ static void arena_bounds()
     expect(!beyond_arena(top, 16u, 100u, 0), "limit 0 checks nothing");
 }
 
+// Framing behind a header is never a wave per packet's work, whichever way the launch is asked:
+// with the lengths at hand or without, over the link or not.
+static void framing_behind_a_header()
+{
+    const uint32_t lens[1] = {0};
+    for (uint32_t spread_max : {0u, 64u, 2000u, 4096u, 1u << 20})
+        for (uint32_t n : {1u, 64u, 200u, 4096u, 16384u})
+            for (uint32_t len : {0u, 60u, 1420u, 5000u})
+                for (int k = 0; k < 8; k++) {
+                    AeadArgs a{};
+                    a.spread_max = spread_max;
+                    a.n = n;
+                    a.len = len;
+                    a.in_bytes = (uint64_t)n * (len + 32u);
+                    a.lens = k & 1 ? lens : nullptr;
+                    a.over_link = (k & 2) != 0;
+                    a.wg.mode = k & 4 ? WG_FUSE_ENCAP : WG_FUSE_DECAP;
+                    a.in_skip = 16;
+                    expect(!aead_runs_spread(a), "framing behind a header by a lane per packet or a run of one");
+                }
+}
+
+// A batch that is not a wave per packet's work over the link is fetched into device memory and
+// asked about again there: the answer stays.
+static void fetched_batches_stay_with_the_lanes()
+{
+    const uint32_t lens[1] = {0};
+    for (uint32_t spread_max : {0u, 1u, 3u, 64u, 2000u, 4096u, 16384u})
+        for (uint32_t n = 1; n <= 65536; n += 1 + n / 7)
+            for (uint32_t len : {0u, 60u, 200u, 600u, 1420u, 5000u, 65535u})
+                for (int k = 0; k < 2; k++) {
+                    AeadArgs a{};
+                    a.spread_max = spread_max;
+                    a.n = n;
+                    a.len = len;
+                    a.in_bytes = (uint64_t)n * (len + 16u);
+                    a.lens = k ? lens : nullptr;
+                    a.over_link = true;
+                    const bool there = aead_runs_spread(a);
+                    a.over_link = false;
+                    expect(there || !aead_runs_spread(a), "a fetched batch stays with the lanes");
+                }
+}
+
 int main()
 {
     arena_bounds();
+    fetched_batches_stay_with_the_lanes();
+    framing_behind_a_header();
     if (!failures) printf("PASS launch rules\n");
     return failures;
 }

@@ -362,6 +362,49 @@ def test_decap_in_place(mem, n, spread_max):
     ctx.close()
 
 
+@pytest.mark.parametrize("n,spread_max,length", [(200, 64, 5000), (65, 64, 4033), (256, 64, 4500), (900, 512, 4040)])
+def test_uniform_long_packets_in_rings_with_a_lowered_knob(n, spread_max, length):
+    """Packets of one length beyond 63 blocks, more of them than the knob allows a wave each and
+    no more than four times that: both directions work, with the bytes of any other setting."""
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    peers = _peers(rng)
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    peer = rng.integers(0, N_PEERS, n).astype(np.uint32)
+    stride = (16 + length + 15 + 16 + 15) & ~15
+    ctx = _ctx(peers, keys, keys)
+    ctx.set_spread_max_packets(spread_max)
+    ring, out = ctx.ring_alloc(n * stride), ctx.ring_alloc(n * stride)
+    ring[:] = 0xEE
+    out[:] = 0x77
+    want, nxt = np.array(ring), np.zeros(N_PEERS, np.int64)
+    plains = []
+    for i in range(n):
+        p = int(peer[i])
+        plains.append(_inner(rng, peers, p, length))
+        ring[i * stride + 16:i * stride + 16 + length] = np.frombuffer(plains[-1], np.uint8)
+        # (one context is both ends: what goes out names the index it comes in under)
+        w = O.wg_encap(plains[-1], 8000, keys[p].tobytes(), peers[p][1], int(nxt[p]))
+        want[i * stride:i * stride + len(w)] = np.frombuffer(w, np.uint8)
+        nxt[p] += 1
+    wire_len = np.zeros(n, np.uint32)
+    ctx.wg_encap(lib.make_batch(ring, n * stride, n, lib.MEM_HOST, stride=stride, length=length, peer=peer), 8000, wire_len)
+    assert (wire_len == 32 + (length + 15) // 16 * 16).all()
+    assert np.array_equal(np.array(ring), want)
+    ctx.wg_peers_set([(b, a, c, d) for a, b, c, d in peers])
+    res, olen = np.full(n, 99, np.uint8), np.zeros(n, np.uint32)
+    gp, gc = np.zeros(n, np.uint32), np.zeros(n, np.uint64)
+    ctx.wg_decap(lib.make_batch(ring, n * stride, n, lib.MEM_HOST, stride=stride, length=int(wire_len[0])),
+                 lib.make_batch(out, n * stride, n, lib.MEM_HOST, stride=stride), res, olen, gp, gc)
+    assert (res == 0).all() and (olen == length).all() and np.array_equal(gp, peer)
+    got = np.array(out).reshape(n, stride)
+    assert all(np.array_equal(got[i, :length], np.frombuffer(plains[i], np.uint8)) for i in range(n))
+    ctx.ring_free(ring)
+    ctx.ring_free(out)
+    ctx.close()
+
+
 def _decap_cases(rng, peers, keys, n):
     """Datagrams as the remote peers would send them, most of them damaged in
     one of the ways the receive path must tell apart."""

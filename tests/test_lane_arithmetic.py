@@ -18,7 +18,8 @@ def test_lane_arithmetic_on_cpu():
 
 
 def test_rules_around_a_launch_on_cpu():
-    """tests/cpp/route_test.cpp: what counts as inside an arena."""
+    """tests/cpp/route_test.cpp: what counts as inside an arena, and which launch a batch
+    gets."""
     subprocess.run(["make", "-s", "-C", os.path.join(HERE, "cpp"), "route_test"], check=True)
     r = subprocess.run([os.path.join(HERE, "cpp", "route_test")], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr

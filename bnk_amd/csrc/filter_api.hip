@@ -208,12 +208,29 @@ int stage_headers(bnk_ctx *ctx, uint32_t n, GetPtr ptr_of, GetLen len_of, Filter
     return BNK_OK;
 }
 
+// Room for what a note batch may add, and what its launch has to know about the table.  The
+// batch gets its number here, and the next call may wait for the word that carries it: so this
+// comes last, behind every check and copy that could still turn the call away.
+int note_ready(bnk_ctx *ctx, FilterArgs *a)
+{
+    int rc = flows_reserve(ctx, a->n);
+    if (rc) return rc;
+    const FilterState *f = ctx->filter;
+    a->flows = f->flows;
+    a->record = f->d_record;
+    a->record_seq = f->note_seq;
+    a->record_after = f->record_after;
+    return BNK_OK;
+}
+
 // Runs a staged host batch and brings the verdicts (check) or the overflow
 // flag (note) back.
 int run_staged(bnk_ctx *ctx, bool check, FilterArgs &a, uint8_t *h_verdict, uint8_t *verdict)
 {
     FilterState *f = ctx->filter;
     if (!check) {
+        int nrc = note_ready(ctx, &a);
+        if (nrc) return nrc;
         HIPCHK(ctx, launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
     } else if (h_verdict) {
         // CheckInbound reports nothing through the status word
@@ -242,9 +259,6 @@ void base_args(bnk_ctx *ctx, uint32_t n, int64_t now_ns, FilterArgs *a)
     a->status = ctx->d_status;
     a->rules = ctx->filter->ridx;
     a->flows = ctx->filter->flows;
-    a->record = ctx->filter->d_record;
-    a->record_seq = ctx->filter->note_seq;
-    a->record_after = ctx->filter->record_after;
 }
 
 int check_device_layout(bnk_ctx *ctx, const bnk_batch *b)
@@ -273,10 +287,6 @@ int filter_batch(bnk_ctx *ctx, bool check, const bnk_batch *pkts, int64_t now_ns
         else HIPCHK(ctx, launch_fill_u8(verdict, n, 1, ctx->stream));
         return BNK_OK;
     }
-    if (!check) {
-        rc = flows_reserve(ctx, n);
-        if (rc) return rc;
-    }
     FilterArgs a;
     base_args(ctx, n, now_ns, &a);
     if (pkts->mem == BNK_MEM_DEVICE) {
@@ -293,6 +303,7 @@ int filter_batch(bnk_ctx *ctx, bool check, const bnk_batch *pkts, int64_t now_ns
             a.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
             *counted = true;
         }
+        if (!check && (rc = note_ready(ctx, &a))) return rc;
         HIPCHK(ctx, check ? launch_filter_check(a, f->max_blocks, ctx->stream)
                           : launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
         return BNK_OK;
@@ -322,15 +333,10 @@ int filter_ptrs(bnk_ctx *ctx, bool check, const uint8_t *const *pkts, const uint
         if (check) memset(verdict, 1, n);
         return BNK_OK;
     }
-    int rc;
-    if (!check) {
-        rc = flows_reserve(ctx, n);
-        if (rc) return rc;
-    }
     FilterArgs a;
     base_args(ctx, n, now_ns, &a);
     uint8_t *h_verdict = nullptr;
-    rc = stage_headers(
+    int rc = stage_headers(
         ctx, n, [&](uint32_t i) { return pkts[i]; }, [&](uint32_t i) { return lens[i]; }, &a, &h_verdict);
     if (rc) return rc;
     return run_staged(ctx, check, a, h_verdict, verdict);

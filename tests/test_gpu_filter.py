@@ -347,3 +347,41 @@ def test_note_batches_in_a_row_while_the_table_is_nearly_full(n, distinct):
     ctx.sync()
     assert ctx.filter_flows() == ora.flows()
     ctx.close()
+
+
+def test_a_refused_note_batch_leaves_nothing_to_wait_for():
+    """While the table is nearly full a NoteOutbound waits for a word that the batch before it
+    leaves behind.  A batch that is refused launches nothing, so it must not be that batch: the
+    call behind it would sit out its whole wait (20 ms) with the context locked."""
+    import time
+    import torch
+    from bnk_amd import lib
+    n = 3000
+    flows = np.zeros((n, 28), np.uint8)
+    flows[:, 0], flows[:, 3], flows[:, 8], flows[:, 9] = 0x45, 28, 64, 17
+    flows[:, 12:16] = (100, 64, 0, 1)
+    flows[:, 22:24] = (np.arange(n, dtype=np.uint16) % 900).view(np.uint8).reshape(-1, 2)
+    ctx = lib.Context(0)
+    ctx.filter_set_rules([([(0, 0)], "icmp", [])])
+    d = torch.from_numpy(flows).to("cuda:0")
+    torch.cuda.synchronize()
+    good = lib.make_batch(d, n * 28, n, lib.MEM_DEVICE, stride=28, length=28)
+    host = np.ascontiguousarray(flows[:100])
+    off = np.full(n, 28 * 100, np.uint64)
+    refused = [lib.make_batch(d, n * 28 - 1, n, lib.MEM_DEVICE, stride=28, length=28),
+               lib.make_batch(host, host.nbytes, n, lib.MEM_HOST, offsets=off, lens=np.full(n, 28, np.uint32))]
+    ctx.filter_note_outbound(good, FC.T0)
+    ctx.sync()
+    for bad in refused:
+        took = []
+        for k in range(6):
+            with pytest.raises(lib.BnkError) as ei:
+                ctx.filter_note_outbound(bad, FC.T0 + k)
+            assert ei.value.code == lib.E_INVAL
+            t = time.perf_counter()
+            ctx.filter_note_outbound(good, FC.T0 + k)
+            took.append(time.perf_counter() - t)
+            ctx.sync()
+        assert min(took) < 0.010, took
+    assert ctx.filter_flow_count() == 900
+    ctx.close()

@@ -118,31 +118,23 @@ int flows_reserve(bnk_ctx *ctx, uint32_t n_new)
     FilterState *f = ctx->filter;
     const uint64_t half = f->flows.cap / 2;
     auto take = [&]() {
-        f->claimed_upper += n_new;
-        f->reserved += n_new;
-        f->reserved_at[++f->note_seq & 63u] = f->reserved;
-        f->record_after = f->record != nullptr && f->claimed_upper + n_new > f->flows.cap / 2;
+        f->bound.take(n_new);
+        f->record_after = f->record != nullptr && f->bound.upper + n_new > f->flows.cap / 2;
         return BNK_OK;
     };
-    auto lower = [&]() {
-        const uint64_t rec = __atomic_load_n(f->record, __ATOMIC_RELAXED);
-        const uint32_t seq = (uint32_t)(rec >> 32);
-        if ((int32_t)(seq - f->table_seq) >= 0 && f->note_seq - seq < 64u)
-            f->claimed_upper = std::min(f->claimed_upper, (rec & 0xFFFFFFFFu) + f->reserved - f->reserved_at[seq & 63u]);
-        return seq == f->note_seq;
-    };
+    auto lower = [&]() { return f->bound.lower(__atomic_load_n(f->record, __ATOMIC_RELAXED)); };
     if (f->record) lower();
-    if (f->claimed_upper + n_new <= half) return take();
+    if (f->bound.upper + n_new <= half) return take();
     if (f->record_after) {
         const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
         while (!lower() && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
-        if (f->claimed_upper + n_new <= half) return take();
+        if (f->bound.upper + n_new <= half) return take();
     }
     uint32_t c[FLOW_COUNTERS];
     HIPCHK(ctx, hipMemcpyAsync(c, f->flows.counters, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    f->claimed_upper = c[FLOW_CLAIMED];
-    if (f->claimed_upper + n_new <= half) return take();
+    f->bound.upper = c[FLOW_CLAIMED];
+    if (f->bound.upper + n_new <= half) return take();
     uint64_t need = 4ull * ((uint64_t)(c[FLOW_LIVE] - c[FLOW_GONE]) + n_new); // at most a quarter full afterwards
     uint64_t cap = FLOW_CAP_INITIAL;
     while (cap < need) cap *= 2;
@@ -160,8 +152,7 @@ int flows_reserve(bnk_ctx *ctx, uint32_t n_new)
     for (DevBuf *b : {&f->slots, &f->counters, &f->present, &f->present_small, &f->list}) b->release();
     f->slots = ns; f->counters = nc; f->present = np; f->present_small = nps; f->list = nl;
     f->flows = nt;
-    f->claimed_upper = c[FLOW_LIVE] - c[FLOW_GONE];
-    f->table_seq = f->note_seq;
+    f->bound.upper = c[FLOW_LIVE] - c[FLOW_GONE];
     return take();
 }
 
@@ -218,7 +209,7 @@ int note_ready(bnk_ctx *ctx, FilterArgs *a)
     const FilterState *f = ctx->filter;
     a->flows = f->flows;
     a->record = f->d_record;
-    a->record_seq = f->note_seq;
+    a->record_seq = f->bound.seq;
     a->record_after = f->record_after;
     return BNK_OK;
 }
@@ -231,7 +222,7 @@ int run_staged(bnk_ctx *ctx, bool check, FilterArgs &a, uint8_t *h_verdict, uint
     if (!check) {
         int nrc = note_ready(ctx, &a);
         if (nrc) return nrc;
-        HIPCHK(ctx, launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
+        HIPCHK(ctx, launch_filter_note(a, f->max_blocks, f->bound.upper, ctx->stream));
     } else if (h_verdict) {
         // CheckInbound reports nothing through the status word
         a.verdict = ctx->pin.dev(h_verdict);
@@ -305,7 +296,7 @@ int filter_batch(bnk_ctx *ctx, bool check, const bnk_batch *pkts, int64_t now_ns
         }
         if (!check && (rc = note_ready(ctx, &a))) return rc;
         HIPCHK(ctx, check ? launch_filter_check(a, f->max_blocks, ctx->stream)
-                          : launch_filter_note(a, f->max_blocks, f->claimed_upper, ctx->stream));
+                          : launch_filter_note(a, f->max_blocks, f->bound.upper, ctx->stream));
         return BNK_OK;
     }
     Span span;

@@ -8,6 +8,7 @@
 
 #include "ctx.hpp"
 #include "filter_dev.hpp"
+#include "flow_bound.hpp"
 
 namespace bnk {
 
@@ -169,14 +170,8 @@ struct FilterState {
     RuleIndexDev ridx{};
     DevBuf slots, counters, present, present_small, list;
     FlowTableDev flows{};
-    uint64_t claimed_upper = 0; // host bound on slots ever claimed in the current table
-    // What brings that bound down again without waiting for the stream: every note batch has a
-    // number, its launch leaves (the number before << 32 | slots claimed so far) in *record as it
-    // starts, and reserved_at[] knows how much the batches after that number may have added.
-    uint64_t *record = nullptr, *d_record = nullptr; // pinned host word, owned by the context
-    uint32_t note_seq = 0, table_seq = 0;            // newest batch; newest batch before the current table
-    uint64_t reserved = 0;                           // sum of n_new over all batches
-    uint64_t reserved_at[64] = {0};                  // that sum as of batch (number & 63)
+    FlowBound bound;                                 // on slots ever claimed in the current table
+    uint64_t *record = nullptr, *d_record = nullptr; // its pinned host word, owned by the context
     bool record_after = false;                       // the newest batch's number follows its launch into *record
     uint32_t max_blocks = 2048;
     void release()

@@ -473,9 +473,9 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             fa.rules = f->ridx;
             fa.flows = f->flows;
             fa.record = f->d_record;
-            fa.record_seq = f->note_seq;
+            fa.record_seq = f->bound.seq;
             fa.record_after = f->record_after && hi == n;
-            HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->claimed_upper, ctx->stream));
+            HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->bound.upper, ctx->stream));
         }
         if (fits) {
             AeadArgs se{};

@@ -1,10 +1,13 @@
 // CPU check of the host-side rules around a launch (bnk_amd/csrc): which packets lie in the
-// arena and which AEAD launch a batch gets.  Prints PASS/FAIL lines; exit status is the number of failures.
+// arena, which AEAD launch a batch gets, how many flow table slots may be claimed.  Prints PASS/FAIL lines; exit status is the number of failures.
 #include <stdio.h>
 
+#include <deque>
 #include <initializer_list>
+#include <random>
 
 #include "../../bnk_amd/csrc/aead_route.hpp"
+#include "../../bnk_amd/csrc/flow_bound.hpp"
 
 using namespace bnk;
 
@@ -77,11 +80,46 @@ static void fetched_batches_stay_with_the_lanes()
                 }
 }
 
+// The bound on claimed slots against a model of the launches: never below what is claimed, back
+// down to it once the batches have run, however many batches there have been (the numbers wrap at
+// 2^32, and a table may stay as it is for longer than 2^31 of them).
+static void claimed_slots(uint32_t first_seq)
+{
+    std::mt19937 rng(first_seq | 1u);
+    FlowBound b;
+    b.seq = first_seq;
+    b.at[first_seq & 63u] = 0;
+    uint64_t record = (uint64_t)first_seq << 32; // (batch first_seq found an empty table)
+    uint64_t claimed = 0;
+    struct Batch { uint32_t seq; uint64_t claims; };
+    std::deque<Batch> on_the_way;
+    for (int k = 0; k < 4000; k++) {
+        const uint32_t n = 1u + rng() % 3000u;
+        b.lower(record);
+        b.take(n);
+        on_the_way.push_back({b.seq, rng() % 4u ? 0u : rng() % (n + 1u)});
+        uint64_t may = claimed;
+        for (const Batch &o : on_the_way) may += o.claims;
+        expect(b.upper >= may, "no fewer slots than are claimed");
+        // some of the batches run, each leaving its record as it starts
+        while (!on_the_way.empty() && (on_the_way.size() > 40u || rng() % 3u)) {
+            record = (uint64_t)(on_the_way.front().seq - 1u) << 32 | claimed;
+            claimed += on_the_way.front().claims;
+            on_the_way.pop_front();
+        }
+        if (k % 500 == 250) claimed -= claimed / 3u; // the table grows and drops what is not in the map
+    }
+    record = (uint64_t)b.seq << 32 | claimed;
+    expect(b.lower(record), "the newest batch's record is known for it");
+    expect(b.upper == claimed, "and brings the bound down to what is claimed");
+}
+
 int main()
 {
     arena_bounds();
     fetched_batches_stay_with_the_lanes();
     framing_behind_a_header();
+    for (uint32_t first_seq : {0u, 1000u, 0x7FFFFFFFu - 2000u, 0x80000001u, 0xFFFFFFFFu - 2000u}) claimed_slots(first_seq);
     if (!failures) printf("PASS launch rules\n");
     return failures;
 }

@@ -50,7 +50,7 @@ inline bool aead_runs_spread(const AeadArgs &a)
 // must hold; what decides the cost is then how many of a wave's 64 lanes have a run, so the
 // wave takes as many more as still fit at that length (16384 packets x 1420: 10 instead of 8,
 // 38 us a pair of launches instead of 46 with three streams at work, 58 on one stream either
-// way).  Where the host does not know the lengths the room per packet in the arena stands for
+// way).  Where the lengths vary the room per packet (aead_room) stands for
 // their mean, with a margin for how much of it a wave may get: beyond 64 lanes all of a wave's
 // runs get longer (24000 packets of 1 to 1420 bytes, 15 per wave instead of 12: 39 us instead
 // of 47 on three streams, 70 instead of 63 on one).
@@ -67,10 +67,36 @@ inline bool aead_runs_spread(const AeadArgs &a)
 // against 46.  (Back to back without gaps they hold out longer, 1 to 200 bytes 29 against 35 at
 // 57000, but the host sees the room alone.)
 //
+// A host batch has the chip to itself and its grouping in the call's way, so short packets do not
+// end it there: calls on pinned rings, a lane per packet against split, 38000 of 1 to 100 bytes
+// sealed 258 us against 234, through the tunnel 366 out and 403 in against 320 and 317, 50000 340
+// against 301 and 461 and 521 against 419 and 415; 40000 of 1 to 200 bytes 345 against 334; only
+// 54000 of 1 to 60 bytes are sealed in 275 against 281, with 408 and 417 against 398 and 395
+// through the tunnel.
+//
 // Up to 10240 packets whose lengths the host does not know, five per wave: whatever mix of
 // up to 1471 bytes they are, a piece is then all that a run ever holds, and the launch lasts
 // as long as that (3400 packets of 1 to 1420 bytes 46 -> 32 us a pair against as many as fit on
 // average, 10000 51 -> 40).
+// Room per packet: what the batch's packets take up on average in an arena that just holds them,
+// as far as the host can tell.  From the lengths themselves where it has them (16 bytes more, for
+// a tag and for the gaps between slots); of a batch in GPU memory it knows the stride, or else
+// only the arena, which may hold far more than the batch: room is then too large, and a wave gets
+// fewer packets than would fit.
+constexpr uint32_t SPLIT_ROOM_MAX = 1500; // beyond it one rule holds
+inline uint32_t aead_room(const bnk_batch &b)
+{
+    if (!b.lens || b.n == 0) return 0;
+    uint64_t all = b.bytes;
+    if (b.mem == BNK_MEM_HOST) {
+        all = 16ull * b.n;
+        for (uint32_t i = 0; i < b.n; i++) all += b.lens[i];
+    } else if (!b.offsets) {
+        all = std::min(all, (uint64_t)b.n * b.stride);
+    }
+    return (uint32_t)std::min<uint64_t>(all / b.n, SPLIT_ROOM_MAX);
+}
+
 constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
 constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
 inline uint32_t aead_split_packets(const AeadArgs &a)
@@ -78,8 +104,8 @@ inline uint32_t aead_split_packets(const AeadArgs &a)
     // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
     if (a.spread_max == 0 || a.order || aead_runs_spread(a)) return 0;
     const uint32_t per = (a.n + 2047u) / 2048u;
-    const uint32_t room = a.lens ? (uint32_t)std::min<uint64_t>(a.in_bytes / a.n, 1500u) : a.len;
-    if (per > (!a.lens ? 12u : room < 256u ? 18u : 27u)) return 0;
+    const uint32_t room = a.lens ? std::min(a.room, SPLIT_ROOM_MAX) : a.len;
+    if (per > (!a.lens ? 12u : room < 256u && !a.host_batch ? 18u : 27u)) return 0;
     const uint32_t blocks = (room + 63u) / 64u, pieces = blocks / 2u + 1u;
     auto fits = [&](uint32_t k, uint32_t q) {
         if (!a.lens) return k * ((pieces + q - 1u) / q) <= 64u;

@@ -223,7 +223,8 @@ int aead_batch(bnk_ctx *ctx, bool open, const bnk_batch *in, const bnk_batch *ou
     a.in_stride = in->stride;
     a.out_stride = out->stride;
     a.len = in->len;
-    a.in_bytes = in->bytes;
+    a.room = aead_room(*in);
+    a.host_batch = in->mem == BNK_MEM_HOST;
 
     if (in->mem == BNK_MEM_DEVICE) {
         rc = aead_device_layout_check(ctx, open, in, out);

@@ -111,7 +111,8 @@ struct AeadArgs {
                                // has checked the layout
     uint32_t first;            // the launch covers packets first .. first+n-1; order[] is relative to first
     uint32_t spread_max;       // launches of at most this many packets run one wave per packet
-    uint64_t in_bytes;         // size of the input arena (a hint: how long packets may be on average)
+    uint32_t room;             // with lens: bytes of an arena per packet (a hint, see aead_room)
+    bool host_batch;           // the call waits for its launch: no other has the chip meanwhile
     bool over_link;            // packets lie in host memory: a wave per packet reads them there
     uint32_t split;            // set by the launcher: packets per wave of aead_split_kernel
     unsigned long long *tally; // or nullptr: an open without framing counts its own verdicts here

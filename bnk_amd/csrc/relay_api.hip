@@ -35,7 +35,8 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
     // ---- where everything lives on the device ----
     AeadArgs op{};
     op.spread_max = ctx->spread_max;
-    op.in_bytes = in->bytes;
+    op.room = aead_room(*in);
+    op.host_batch = host;
     op.keys = ctx->d_keys[BNK_KEYS_RECV];
     op.n_peers = ctx->n_keys[BNK_KEYS_RECV];
     op.status = ctx->d_status;
@@ -287,7 +288,8 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         // ---- 4. re-seal the survivors under the outbound keys ----
         AeadArgs se{};
         se.spread_max = ctx->spread_max;
-        se.in_bytes = in->bytes;
+        se.room = op.room;
+        se.host_batch = host;
         se.keys = ctx->d_keys[BNK_KEYS_SEND];
         se.n_peers = n_peers_out;
         se.status = ctx->d_status;

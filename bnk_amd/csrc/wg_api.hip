@@ -409,6 +409,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
     }
 
     const bool over_link = ring_out != nullptr && wave_per_packet; // (else they have been fetched)
+    const uint32_t room = aead_room(*slots);
 
     for (DevBuf *buf : {&ctx->r_keys, &ctx->r_idx, &ctx->r_skeys, &ctx->r_sidx, &ctx->wg_padded})
         HIPCHK(ctx, buf->reserve((size_t)n * 4));
@@ -507,7 +508,8 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         AeadArgs se{};
         se.spread_max = ctx->spread_max;
         se.over_link = over_link;
-        se.in_bytes = slots->bytes;
+        se.room = room;
+        se.host_batch = host;
         se.keys = ctx->d_keys[BNK_KEYS_SEND];
         se.n_peers = pe.n;
         se.status = ctx->d_status;
@@ -798,6 +800,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         d_counter = counter;
     }
     const bool over_link = direct && wave_per_packet; // (else they have been fetched)
+    const uint32_t room = aead_room(*wire);
     HIPCHK(ctx, ctx->wg_ctlen.reserve((size_t)n * 4));
     HIPCHK(ctx, ctx->r_auth.reserve(n));
     if (wire->lens) {
@@ -925,7 +928,8 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         AeadArgs op{};
         op.spread_max = ctx->spread_max;
         op.over_link = over_link;
-        op.in_bytes = wire->bytes;
+        op.room = room;
+        op.host_batch = host;
         op.keys = ctx->d_keys[BNK_KEYS_RECV];
         op.n_peers = pe.n;
         op.status = ctx->d_status;

@@ -5,6 +5,7 @@
 #include <deque>
 #include <initializer_list>
 #include <random>
+#include <vector>
 
 #include "../../bnk_amd/csrc/aead_route.hpp"
 #include "../../bnk_amd/csrc/flow_bound.hpp"
@@ -49,7 +50,7 @@ static void framing_behind_a_header()
                     a.spread_max = spread_max;
                     a.n = n;
                     a.len = len;
-                    a.in_bytes = (uint64_t)n * (len + 32u);
+                    a.room = len + 32u;
                     a.lens = k & 1 ? lens : nullptr;
                     a.over_link = (k & 2) != 0;
                     a.wg.mode = k & 4 ? WG_FUSE_ENCAP : WG_FUSE_DECAP;
@@ -71,13 +72,68 @@ static void fetched_batches_stay_with_the_lanes()
                     a.spread_max = spread_max;
                     a.n = n;
                     a.len = len;
-                    a.in_bytes = (uint64_t)n * (len + 16u);
+                    a.room = len + 16u;
                     a.lens = k ? lens : nullptr;
                     a.over_link = true;
                     const bool there = aead_runs_spread(a);
                     a.over_link = false;
                     expect(there || !aead_runs_spread(a), "a fetched batch stays with the lanes");
                 }
+}
+
+// The room per packet is the batch's, not its arena's: a batch in a corner of a large ring and a
+// piece of a larger batch go the way of the same packets in an arena that just holds them.
+static void room_per_packet()
+{
+    for (uint32_t longest : {44u, 200u, 400u, 1420u})
+        for (uint32_t n : {5000u, 12000u, 24000u, 36864u, 36865u, 48000u, 55296u, 60000u}) {
+            std::vector<uint32_t> lens(n);
+            uint64_t sum = 0;
+            for (uint32_t i = 0; i < n; i++) sum += lens[i] = 1u + i % longest;
+            std::vector<uint64_t> offsets(n, 0);
+            bnk_batch fits{}, corner{}, strided{}, unknown{};
+            fits.n = n;
+            fits.mem = BNK_MEM_HOST;
+            fits.lens = lens.data();
+            fits.offsets = offsets.data();
+            fits.bytes = sum + 16ull * n;
+            corner = fits;
+            corner.bytes = 1ull << 32;
+            expect(aead_room(fits) == aead_room(corner) && aead_room(fits) == (sum + 16ull * n) / n, "a corner of a large ring");
+            strided = fits;
+            strided.mem = BNK_MEM_DEVICE;
+            strided.lens = (const uint32_t *)16; // (nobody reads it here)
+            strided.offsets = nullptr;
+            strided.stride = longest + 16u;
+            strided.bytes = 1ull << 32;
+            expect(aead_room(strided) == longest + 16u, "a stride in a large arena");
+            unknown = strided;
+            unknown.offsets = (const uint64_t *)16;
+            expect(aead_room(unknown) == SPLIT_ROOM_MAX, "an arena is all there is to go by");
+            unknown.bytes = (uint64_t)n * 100u;
+            expect(aead_room(unknown) == 100u, "and is the batch's when it just holds it");
+
+            AeadArgs a{};
+            a.spread_max = SPREAD_MAX_PACKETS;
+            a.lens = lens.data();
+            a.room = aead_room(corner);
+            for (uint32_t pieces : {1u, 2u, 5u}) {
+                a.n = n / pieces;
+                bnk_batch alone = fits;
+                alone.n = a.n;
+                alone.bytes = 0;
+                for (uint32_t i = 0; i < a.n; i++) alone.bytes += lens[i] + 16u;
+                AeadArgs b = a;
+                b.room = aead_room(alone);
+                expect((aead_split_packets(a) != 0) == (aead_split_packets(b) != 0) && aead_wants_order(a) == aead_wants_order(b),
+                       "a piece goes the way of the batch it is");
+            }
+            // (short packets in numbers are a lane's work each wherever they lie)
+            a.n = n;
+            if (longest <= 200u && n > 36864u) expect(aead_wants_order(a), "short packets, many");
+            a.host_batch = true;
+            if (n > 5000u && n <= 55296u) expect(aead_split_packets(a) != 0, "a host batch of any lengths is split");
+        }
 }
 
 // The bound on claimed slots against a model of the launches: never below what is claimed, back
@@ -119,6 +175,7 @@ int main()
     arena_bounds();
     fetched_batches_stay_with_the_lanes();
     framing_behind_a_header();
+    room_per_packet();
     for (uint32_t first_seq : {0u, 1000u, 0x7FFFFFFFu - 2000u, 0x80000001u, 0xFFFFFFFFu - 2000u}) claimed_slots(first_seq);
     if (!failures) printf("PASS launch rules\n");
     return failures;

@@ -1206,8 +1206,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
             total += (uint32_t)__shfl_xor((int)total, off, 64);
             most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
         }
+        // A packet that lands on itself, but not where it is (a datagram's plaintext at the datagram's
+        // own offset, 16 bytes ahead of its ciphertext): its runs would overwrite each other's bytes.
+        // A lane that goes through it alone reads ahead of what it writes, so such a wave deals out
+        // whole packets.
+        const int64_t shift = (int64_t)((uint64_t)(uintptr_t)p.dst - (uint64_t)(uintptr_t)p.src), reach = (int64_t)p.len + 16;
+        const bool onto_itself = __ballot(shift != 0 && shift < reach && -shift < reach) != 0ull;
         uint32_t runs;
-        for (q = max(max((total + 63u) / 64u, (most + SPLIT_MAX_RUNS - 1u) / SPLIT_MAX_RUNS), 1u);; q++) {
+        for (q = max(onto_itself ? most : max((total + 63u) / 64u, (most + SPLIT_MAX_RUNS - 1u) / SPLIT_MAX_RUNS), 1u);; q++) {
             lanes = runs = (pieces + q - 1u) / q;
 #pragma unroll
             for (int off = 32; off >= 1; off >>= 1) lanes += (uint32_t)__shfl_xor((int)lanes, off, 64);

@@ -249,7 +249,8 @@ int bnk_keys_set(bnk_ctx *ctx, int which, const uint8_t *keys32,
  * written at the packet's position in `out` (only base, bytes, mem, offsets,
  * stride of `out` are read).  Keys come from BNK_KEYS_SEND.  in and out may
  * be the same arena at the same offsets (in place), as wireguard-go's
- * AEAD.Seal(header, nonce, plaintext, nil) is. */
+ * AEAD.Seal(header, nonce, plaintext, nil) is; no other overlap is promised to
+ * work, here or in bnk_aead_open_batch. */
 int bnk_aead_seal_batch(bnk_ctx *ctx, const bnk_batch *in,
                         const bnk_batch *out);
 
@@ -404,7 +405,10 @@ int bnk_wg_encap_batch(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu,
  * total length, is out_len[i] bytes at out's offset i.  For every result but
  * BAD_HEADER/UNKNOWN_INDEX peer[i] and counter[i] name the sender and the
  * nonce counter; otherwise peer[i] = 0xFFFFFFFF.  A failed open leaves zeros in
- * `out`, like the AEAD entry points.
+ * `out`, like the AEAD entry points.  `wire` and `out` are disjoint, or the same
+ * arena with every out offset 16 above its datagram's, the plaintext landing
+ * where its ciphertext was (in place, as wireguard-go opens); no other overlap
+ * is promised to work.
  * Every authentic packet (any result but BAD_HEADER, UNKNOWN_INDEX, AUTH_FAIL)
  * goes through its peer's anti-replay window (RFC 6479, 8128 counters, kept on
  * the device per row of the peer table) in batch order, before the keepalive,

@@ -405,6 +405,49 @@ def test_uniform_long_packets_in_rings_with_a_lowered_knob(n, spread_max, length
     ctx.close()
 
 
+@pytest.mark.parametrize("n,length", [(300, 9000), (700, 1400), (41, 2600)])
+@pytest.mark.parametrize("ahead", [0, 16])
+@pytest.mark.parametrize("misalign", [False, True])
+def test_device_decap_onto_its_own_datagrams(n, length, ahead, misalign):
+    """Device-resident batches whose plaintexts land in the arena they are read from: where their
+    ciphertexts were (in place), or 16 bytes ahead, at the datagrams' own offsets.  At 9000 bytes
+    a packet's runs are six pieces of 128 bytes long."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n + ahead)
+    peers = _peers(rng)
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    sender = rng.integers(0, N_PEERS, n)
+    plains = [_inner(rng, peers, int(p), length - int(rng.integers(0, 40))) for p in sender]
+    wires = [O.wg_encap(pt, 0, keys[int(p)].tobytes(), peers[int(p)][0], i) for i, (p, pt) in enumerate(zip(sender, plains))]
+    lens = np.array([len(w) for w in wires], np.uint32)
+    off, total = _layout(rng, lens, misalign)
+    arena = np.full(total, 0xEE, np.uint8)
+    for o, w in zip(off, wires):
+        arena[int(o):int(o) + len(w)] = np.frombuffer(w, np.uint8)
+    want = arena.copy()
+    for o, w, pt in zip(off, wires, plains):
+        at = int(o) + 16 - ahead
+        want[at:at + len(w) - 32] = np.frombuffer(pt + bytes(len(w) - 32 - len(pt)), np.uint8)
+    dev = torch.device("cuda:0")
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)  # noqa: E731
+    ctx = _ctx(peers, keys_recv=keys)
+    buf, d_off, d_lens, d_out = d(arena), d(off.astype(np.int64)), d(lens.astype(np.int32)), d(off.astype(np.int64) + 16 - ahead)
+    res = torch.full((n,), 99, dtype=torch.uint8, device=dev)
+    olen, gp = (torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(2))
+    gc = torch.zeros(n, dtype=torch.int64, device=dev)
+    torch.cuda.synchronize()
+    ctx.wg_decap(lib.make_batch(buf, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens),
+                 lib.make_batch(buf, total, n, lib.MEM_DEVICE, offsets=d_out), res, olen, gp, gc)
+    ctx.sync()
+    assert res.cpu().tolist() == [0] * n
+    assert olen.cpu().tolist() == [len(p) for p in plains]
+    bad = np.flatnonzero(buf.cpu().numpy() != want)
+    assert bad.size == 0, f"first differing byte at {bad[:5]}"
+    ctx.close()
+
+
 def _decap_cases(rng, peers, keys, n):
     """Datagrams as the remote peers would send them, most of them damaged in
     one of the ways the receive path must tell apart."""

@@ -612,9 +612,11 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         // everything, which lands behind the first seven of those loads (the eighth is shared
         // by the two forms of the line and issued after them) and makes the wave sit out their
         // whole way to memory and back in every step: 5 % of a sealing launch.  (The opening
-        // code comes out without that wait, and with this one it is 1 % slower.
-        // tests/test_kernel_isa.py looks for the pattern in both.)
-        if (!OPEN) __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+        // code of a lane per packet comes out without that wait, and with this one it is 1 %
+        // slower; that of a run per lane does not, but a run has few steps: 24000 packets of 1 to
+        // 1420 bytes, a pair of launches 39.6 -> 39.4 us.  tests/test_kernel_isa.py looks for the
+        // pattern in all four.)
+        if (!OPEN || RUNS) __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
         if (s + AHEAD + 1u <= maxsteps) BNK_ISSUE_LINE(s + AHEAD + 1u);
         if (s >= 1) {
             if (SHIFT) {

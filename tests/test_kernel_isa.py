@@ -18,6 +18,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "..", "bnk_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 WAVE_KERNELS = ("_ZN3bnk16aead_wave_kernelILb0EEEvNS_8AeadArgsE", "_ZN3bnk16aead_wave_kernelILb1EEEvNS_8AeadArgsE")
+# the same loop over a run of a packet, with a few lanes per packet
+SPLIT_KERNELS = tuple("_ZN3bnk17aead_split_kernelILb%dEEEvNS_8AeadArgsE" % o for o in (0, 1))
 # seal, open, seal + framing, open + framing of a small batch: a wave per packet
 SPREAD_KERNELS = tuple("_ZN3bnk18aead_spread_kernelILb%dELb%dEEEvNS_8AeadArgsE" % (o, w) for w in (0, 1) for o in (0, 1))
 
@@ -41,7 +43,7 @@ def _body(listing, name):
     return listing[i:listing.index("s_endpgm", i)].split("\n")
 
 
-@pytest.mark.parametrize("name", WAVE_KERNELS)
+@pytest.mark.parametrize("name", WAVE_KERNELS + SPLIT_KERNELS)
 def test_no_wait_for_everything_among_the_loads_of_a_line(listing, name):
     lines = _body(listing, name)
     assert sum("global_load_dwordx4" in x for x in lines) >= 24, "not the kernel this test was written for"
@@ -55,7 +57,7 @@ def test_no_wait_for_everything_among_the_loads_of_a_line(listing, name):
     assert not bad, "s_waitcnt vmcnt(0) between the loads of a line at listing lines %r of %s" % (bad, name)
 
 
-@pytest.mark.parametrize("name", WAVE_KERNELS)
+@pytest.mark.parametrize("name", WAVE_KERNELS + SPLIT_KERNELS)
 def test_the_wave_kernels_spill_nothing(listing, name):
     meta = listing[listing.index(".name:           " + name):]
     meta = meta[:meta.index(".wavefront_size")]

@@ -13,6 +13,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "../../include/bnkhip.h"
+#include "block_sort.hpp"
 #include "kernels.hpp"
 
 namespace bnk {
@@ -224,28 +225,25 @@ __global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
 // The same for up to PEER_RANK_BLOCK_MAX packets, four a thread, peer and position sorted as
 // one word; position p of the sorted batch is thread p % PEER_BLOCK_THREADS's.  (The counting
 // form's three launches cost four to six microseconds each at any size: 3000 packets 16 us,
-// here 9.)
-constexpr uint32_t PEER_BLOCK_THREADS = 1024, PEER_BLOCK_ITEMS = PEER_RANK_BLOCK_MAX / PEER_BLOCK_THREADS;
+// here 8.)
+constexpr uint32_t PEER_BLOCK_THREADS = BLOCK_SORT_THREADS, PEER_BLOCK_ITEMS = BLOCK_SORT_ITEMS;
 constexpr unsigned PEER_BLOCK_INDEX_BITS = 12;
-static_assert(PEER_RANK_BLOCK_MAX == 1u << PEER_BLOCK_INDEX_BITS && PEER_RANK_BLOCK_MAX % PEER_BLOCK_THREADS == 0, "packed keys");
+static_assert(PEER_RANK_BLOCK_MAX == 1u << PEER_BLOCK_INDEX_BITS && PEER_RANK_BLOCK_MAX == BLOCK_SORT_WORDS, "packed keys");
 __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
     const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
     int advance, int no_peer_ok, unsigned bits, uint64_t ctr_limit, uint32_t *status)
 {
-    using Sort = rocprim::block_radix_sort<uint32_t, PEER_BLOCK_THREADS, PEER_BLOCK_ITEMS>;
-    using Scan = rocprim::block_scan<uint32_t, PEER_BLOCK_THREADS>;
-    __shared__ union {
-        typename Sort::storage_type sort;
-        typename Scan::storage_type scan;
-    } tmp;
+    constexpr uint32_t ROWS = PEER_RANK_BLOCK_MAX / 64u;
+    static_assert(ROWS == 64u, "a lane per row");
+    __shared__ BlockSortShared sort;
     __shared__ uint32_t sk[PEER_RANK_BLOCK_MAX + 1];
-    __shared__ uint32_t start[PEER_RANK_BLOCK_MAX];
-    const uint32_t t = threadIdx.x;
+    __shared__ uint32_t last_head[ROWS];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t none = (1u << bits) - 1u; // above every peer
     uint32_t word[PEER_BLOCK_ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
-        const uint32_t i = t * PEER_BLOCK_ITEMS + j;
+        const uint32_t i = block_sort_place(j);
         uint32_t key = NO_PEER;
         if (i < n) {
             key = peer ? peer[i] : 0u;
@@ -253,31 +251,44 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
         }
         word[j] = (key < n_keys ? key : none) << PEER_BLOCK_INDEX_BITS | i;
     }
-    Sort().sort_to_striped(word, tmp.sort, PEER_BLOCK_INDEX_BITS, PEER_BLOCK_INDEX_BITS + bits);
+    block_sort(word, PEER_BLOCK_INDEX_BITS, bits, sort);
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) sk[j * PEER_BLOCK_THREADS + t] = word[j] >> PEER_BLOCK_INDEX_BITS;
     if (t == 0) sk[PEER_RANK_BLOCK_MAX] = NO_PEER;
     __syncthreads();
-    {
-        uint32_t upto[PEER_BLOCK_ITEMS], ahead = 0;
+    // where a position's run begins: the head at or before it in its row of 64, else the last
+    // head of the rows before
+    uint32_t start[PEER_BLOCK_ITEMS];
 #pragma unroll
-        for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
-            const uint32_t p = t * PEER_BLOCK_ITEMS + j;
-            upto[j] = p != 0u && sk[p - 1u] != sk[p] ? p : 0u;
-            if (j) upto[j] = max(upto[j - 1u], upto[j]);
-        }
-        Scan().exclusive_scan(upto[PEER_BLOCK_ITEMS - 1u], ahead, 0u, tmp.scan, rocprim::maximum<uint32_t>());
-#pragma unroll
-        for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) start[t * PEER_BLOCK_ITEMS + j] = max(ahead, upto[j]);
+    for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+        const uint32_t p = j * PEER_BLOCK_THREADS + t;
+        const unsigned long long heads = __ballot(p == 0u || sk[p - 1u] != sk[p]);
+        const unsigned long long upto = heads & (~0ull >> (63u - lane));
+        start[j] = upto ? p - lane + 63u - (uint32_t)__clzll((long long)upto) : NO_PEER;
+        if (lane == 63u) last_head[p >> 6] = upto ? start[j] : 0u;
     }
     __syncthreads();
+    {
+        uint32_t back = last_head[lane];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)back, off, 64);
+            if ((int)lane >= off) back = max(back, o);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
+            const uint32_t row = j * (PEER_BLOCK_THREADS / 64u) + wave;
+            const uint32_t handed = (uint32_t)__shfl((int)back, (int)(row ? row - 1u : 0u), 64);
+            if (start[j] == NO_PEER) start[j] = handed; // (the first row begins with a head)
+        }
+    }
     uint64_t mine[PEER_BLOCK_ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
         const uint32_t p = j * PEER_BLOCK_THREADS + t, key = word[j] >> PEER_BLOCK_INDEX_BITS;
         mine[j] = 0;
         if (key == none) continue;
-        mine[j] = ctr_add(ctr_base[key], p - start[p], ctr_limit);
+        mine[j] = ctr_add(ctr_base[key], p - start[j], ctr_limit);
         ctr_out[word[j] & (PEER_RANK_BLOCK_MAX - 1u)] = mine[j];
     }
     __syncthreads(); // every base has been read

@@ -40,6 +40,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "../../include/bnkhip.h"
+#include "block_sort.hpp"
 #include "kernels.hpp"
 #include "wg_dev.hpp"
 
@@ -591,22 +592,21 @@ __global__ __launch_bounds__(SMALL) void replay_small_kernel(uint8_t *result, ui
 // The whole pass for a batch between that and WG_REPLAY_BLOCK_MAX packets in one workgroup, four
 // packets a thread, with the steps of the large form (below a few thousand packets its eight
 // launches take four microseconds each, mostly for being launches: 3000 packets 31 us, here
-// 15, and as much again for the host to launch them).  Position p of the sorted batch is thread p % BLOCK_THREADS's, so that neighbours in
-// order are neighbours in a wave; only the running maximum goes over four in a row per thread.
-constexpr uint32_t BLOCK_THREADS = 1024, BLOCK_ITEMS = WG_REPLAY_BLOCK_MAX / BLOCK_THREADS;
+// 15, and as much again for the host to launch them).  Position p of the sorted batch is thread
+// p % BLOCK_THREADS's, so that neighbours in order are neighbours in a wave; only the running
+// maximum goes over four in a row per thread.
+constexpr uint32_t BLOCK_THREADS = BLOCK_SORT_THREADS, BLOCK_ITEMS = BLOCK_SORT_ITEMS;
 constexpr unsigned BLOCK_INDEX_BITS = 12;
-static_assert(WG_REPLAY_BLOCK_MAX == 1u << BLOCK_INDEX_BITS && WG_REPLAY_BLOCK_MAX % BLOCK_THREADS == 0, "packed keys");
+static_assert(WG_REPLAY_BLOCK_MAX == 1u << BLOCK_INDEX_BITS && WG_REPLAY_BLOCK_MAX == BLOCK_SORT_WORDS, "packed keys");
 constexpr uint32_t BLOCK_TABLE = 2u * WG_REPLAY_BLOCK_MAX;
 __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *result, uint32_t *out_len,
                                                                      const uint32_t *peer, const uint64_t *counter,
                                                                      uint32_t n_peers, uint32_t n, uint64_t *state,
                                                                      unsigned bits)
 {
-    using Sort = rocprim::block_radix_sort<uint32_t, BLOCK_THREADS, BLOCK_ITEMS>;
-    using ScanMax = rocprim::block_scan<RunMax, BLOCK_THREADS>;
+    static_assert(BLOCK_THREADS == SEG_BLOCK, "seg_block_scan");
     __shared__ union {
-        typename Sort::storage_type sort;
-        typename ScanMax::storage_type scan;
+        BlockSortShared sort;
         uint32_t table[BLOCK_TABLE];
     } tmp;
     __shared__ uint32_t sk[WG_REPLAY_BLOCK_MAX + 1];
@@ -617,7 +617,7 @@ __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *re
     uint32_t word[BLOCK_ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
-        const uint32_t i = t * BLOCK_ITEMS + j;
+        const uint32_t i = block_sort_place(j);
         uint32_t key = none;
         if (i < n) {
             const uint32_t p = peer[i];
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *re
         word[j] = key << BLOCK_INDEX_BITS | i;
     }
     // stable: a peer's packets stay in batch order
-    Sort().sort_to_striped(word, tmp.sort, BLOCK_INDEX_BITS, BLOCK_INDEX_BITS + bits);
+    block_sort(word, BLOCK_INDEX_BITS, bits, tmp.sort);
     uint64_t c[BLOCK_ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
@@ -641,18 +641,26 @@ __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *re
     if (t == 0) sk[WG_REPLAY_BLOCK_MAX] = NO_PEER;
     __syncthreads();
     {
-        // (a counter the filter turns away outright never moves last)
-        RunMax upto[BLOCK_ITEMS];
+        // The running maximum of a peer's counters, up to and with each position (a counter the
+        // filter turns away outright never moves last): four positions in a row per thread, and
+        // the threads' last runs handed on.
+        uint64_t v[BLOCK_ITEMS], run = 0;
+        bool head[BLOCK_ITEMS], any = false;
 #pragma unroll
         for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
-            const uint64_t v = sc[t * BLOCK_ITEMS + j];
-            upto[j] = RunMax{sk[t * BLOCK_ITEMS + j], v < WG_REJECT_AFTER_MESSAGES ? v : 0};
-            if (j) upto[j] = RunMaxOp()(upto[j - 1u], upto[j]);
+            const uint32_t p = t * BLOCK_ITEMS + j;
+            const uint64_t counter_here = sc[p];
+            v[j] = counter_here < WG_REJECT_AFTER_MESSAGES ? counter_here : 0;
+            head[j] = p == 0u || sk[p - 1u] != sk[p];
+            any |= head[j];
+            run = head[j] || v[j] > run ? v[j] : run;
         }
-        RunMax ahead;
-        ScanMax().exclusive_scan(upto[BLOCK_ITEMS - 1u], ahead, RunMax{NO_PEER, 0}, tmp.scan, RunMaxOp());
+        run = seg_block_scan(run, any).prev;
 #pragma unroll
-        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) smax[t * BLOCK_ITEMS + j] = RunMaxOp()(ahead, upto[j]).v;
+        for (uint32_t j = 0; j < BLOCK_ITEMS; j++) {
+            run = head[j] || v[j] > run ? v[j] : run;
+            smax[t * BLOCK_ITEMS + j] = run;
+        }
     }
     __syncthreads();
     uint8_t cls[BLOCK_ITEMS];

@@ -471,3 +471,72 @@ def test_window_pass_with_few_and_many_senders(peers, monkeypatch):
             assert bad.size == 0, f"batch {b}: result differs at {bad[:5]}: got {got[bad[:5]]} want {want[0][bad[:5]]}"
             assert np.array_equal(olen.cpu().numpy().astype(np.uint32), want[1])
             assert (want[0] == lib.WG_REPLAY).sum() > 50
+
+
+@pytest.mark.parametrize("n_peers,n", [(1, 1025), (2, 4096), (127, 4095), (254, 4096), (255, 3000), (256, 4096),
+                                       (4097, 2048), (65534, 4096), (70000, 1026)])
+def test_counters_and_windows_of_one_workgroup_over_the_peers_digits(n_peers, n):
+    """1025 to 4096 packets take their send counters and go through their windows in one
+    workgroup each, sorted by sender eight bits at a time at most: tables of one, two and three
+    passes and their edges, counters against the count of earlier packets of the peer, windows
+    (repeats, old packets, jumps) against the sequential filter."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n_peers + n)
+    tx = [(10 + 3 * i, 500000 + 5 * i, 0x64400000 + i, 0xFFFFFFFF) for i in range(n_peers)]
+    rx = [(p[1], p[0], p[2], p[3]) for p in tx]
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    # the table's ends, a crowd at one of them and everything between
+    peer = rng.integers(0, n_peers, n).astype(np.uint32)
+    peer[:n // 4] = n_peers - 1
+    peer[n // 4:n // 3] = rng.integers(0, min(n_peers, 5), n // 3 - n // 4)
+    rng.shuffle(peer)
+    slot, length = 96, 40
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    with lib.Context(0) as txc, lib.Context(0) as rxc:
+        txc.keys_set(lib.KEYS_SEND, keys)
+        txc.wg_peers_set(tx)
+        rxc.keys_set(lib.KEYS_RECV, keys)
+        rxc.wg_peers_set(rx)
+        first = {int(p): 9000 + int(p) % 7 for p in rng.choice(n_peers, min(n_peers, 40), replace=False)}
+        for p, c in first.items():
+            txc.wg_send_counter_set(p, c)
+        wires, ctrs, nxt = [], [], np.array([first.get(p, 0) for p in range(n_peers)], np.uint64)
+        for _ in range(2):
+            rows = rng.integers(0, 256, (n, slot), dtype=np.uint8)
+            rows[:, 16], rows[:, 18], rows[:, 19] = 0x45, 0, length
+            rows[:, 28:32] = np.array([t[2] for t in tx], np.uint32)[peer].astype(">u4").view(np.uint8).reshape(n, 4)
+            want = np.zeros(n, np.uint64)
+            for i in range(n):
+                want[i] = nxt[peer[i]]
+                nxt[peer[i]] += 1
+            buf, wl = d(rows.reshape(-1)), torch.zeros(n, dtype=torch.int32, device="cuda:0")
+            torch.cuda.synchronize()
+            txc.wg_encap(lib.make_batch(buf, n * slot, n, lib.MEM_DEVICE, stride=slot, length=length, peer=d(peer.view(np.int32))), 1420, wl)
+            txc.sync()
+            assert (wl == 80).all()
+            wires.append(buf.cpu().numpy().reshape(n, slot))
+            got = wires[-1][:, 8:16].copy().view("<u8").reshape(-1)
+            assert np.array_equal(got, want)
+            ctrs.append(want)
+        assert np.array_equal(txc.wg_send_counters(n_peers), nxt)
+        # one batch of each half and of both again, in any order
+        both, who, ctr = np.concatenate(wires), np.concatenate([peer, peer]), np.concatenate(ctrs)
+        filters = {}
+        for _ in range(2):
+            pick = rng.integers(0, 2 * n, n)
+            want = np.array([lib.WG_OK if filters.setdefault(int(who[i]), O.ReplayFilter()).validate(int(ctr[i])) else lib.WG_REPLAY
+                             for i in pick], np.uint8)
+            wire, out = d(both[pick].reshape(-1)), torch.zeros(n * slot, dtype=torch.uint8, device="cuda:0")
+            res = torch.full((n,), 99, dtype=torch.uint8, device="cuda:0")
+            olen, gp = (torch.zeros(n, dtype=torch.int32, device="cuda:0") for _ in range(2))
+            gc = torch.zeros(n, dtype=torch.int64, device="cuda:0")
+            torch.cuda.synchronize()
+            rxc.wg_decap(lib.make_batch(wire, n * slot, n, lib.MEM_DEVICE, stride=slot, length=80),
+                         lib.make_batch(out, n * slot, n, lib.MEM_DEVICE, stride=slot), res, olen, gp, gc)
+            rxc.sync()
+            assert np.array_equal(gc.cpu().numpy().view(np.uint64), ctr[pick])
+            assert np.array_equal(res.cpu().numpy(), want)
+            assert np.array_equal(olen.cpu().numpy(), np.where(want == lib.WG_OK, length, 0))
+            assert len(np.unique(want)) == 2

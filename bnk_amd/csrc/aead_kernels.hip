@@ -1422,11 +1422,12 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     uint64_t ctr = 0;
     if (!WG) {
         // (framing launches only run on layouts the host has checked)
-        const uint64_t in_at = a.in_off ? in_off_ld : (uint64_t)i * a.in_stride;
-        const uint64_t out_at = a.out_off ? out_off_ld : (uint64_t)i * a.out_stride;
+        // (a launch that checks has no skip here: the kernel that framed the packets has looked
+        // at their raw offsets.  Taking skip and offset apart costs a launch of 2900 packets 1 %.)
+        const uint64_t in_at = (uint64_t)(src - a.in), out_at = (uint64_t)(dst - a.out);
         const bool short_ct = OPEN && len < 16u;
-        if (beyond_arena(in_at, a.in_skip, len, a.in_limit) ||
-            beyond_arena(out_at, a.out_skip, OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
+        if (beyond_arena(in_at, len, a.in_limit) ||
+            beyond_arena(out_at, OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
             (len > MAX_PACKET_BYTES && (a.in_limit | a.out_limit) != 0)) {
             if (lane == 0 && !skipped) {
                 status_raise(a.status, STATUS_BOUNDS);

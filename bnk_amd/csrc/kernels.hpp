@@ -92,10 +92,11 @@ struct AeadArgs {
     const uint64_t *counters;  // or nullptr: counter0 + i
     const uint32_t *order;     // or nullptr: lane t handles packet t
     uint8_t *verdict;          // open only
-    uint8_t *heads;            // open by aead_wave_kernel only, or nullptr: one 32-byte record per
-                               // lane of the launch, in launch order (record t belongs to packet
-                               // first + order[t], or first + t without order[]): bytes 0-23 of the
-                               // plaintext, then its length and 1 if it is authentic (two words)
+    uint8_t *heads;            // open by a lane per packet or a few, or nullptr: one 32-byte record
+                               // per packet of the launch, in launch order (record t belongs to
+                               // packet first + order[t], or first + t without order[]): bytes 0-23
+                               // of the plaintext, then its length and 1 if it is authentic (two
+                               // words)
     const uint8_t *skip;       // or nullptr; skip[i] != 0 leaves packet i alone
     uint32_t *status;          // device status word, bit 0 = peer out of range
     uint64_t counter0;
@@ -110,7 +111,7 @@ struct AeadArgs {
                                // alone, gets verdict 0 and raises STATUS_BOUNDS.  0: the host
                                // has checked the layout
     uint32_t first;            // the launch covers packets first .. first+n-1; order[] is relative to first
-    uint32_t spread_max;       // launches of at most this many packets run one wave per packet
+    uint32_t spread_max;       // bnk_set_spread_max_packets (aead_runs_spread)
     uint32_t room;             // with lens: bytes of an arena per packet (a hint, see aead_room)
     bool host_batch;           // the call waits for its launch: no other has the chip meanwhile
     bool over_link;            // packets lie in host memory: a wave per packet reads them there
@@ -118,7 +119,7 @@ struct AeadArgs {
     unsigned long long *tally; // or nullptr: an open without framing counts its own verdicts here
                                // (TALLY_OPENED / TALLY_REJECTED, see tally_bump), an encapsulating
                                // launch over a device-resident batch what it sends (TALLY_SEALED)
-    WgFuse wg;                 // only with aead_runs_spread(); mode 0: plain AEAD
+    WgFuse wg;                 // mode 0: plain AEAD
 };
 
 // Below this many packets a wave per packet finishes sooner than a lane per

@@ -1553,3 +1553,46 @@ def test_small_device_batches_do_their_own_framing(n, misalign):
     for i, e in enumerate(expect):
         assert got[int(off[i]):int(off[i]) + len(e[1])].tobytes() == e[1], i
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [4097, 9000, 16384])
+def test_uniform_device_batches_between_the_small_and_the_large_launches(n):
+    """4097 to 16384 device-resident packets of one MTU-sized length (a range in which encapsulating
+    was once refused, by two rules that named different launches): every datagram against the
+    oracle's, then back to the packets it came from."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    peers = _peers(rng)
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    peer = rng.integers(0, N_PEERS, n).astype(np.uint32)
+    length, stride = 1400, 1456
+    rows = rng.integers(0, 256, (n, stride), dtype=np.uint8)
+    rows[:, 16], rows[:, 18], rows[:, 19] = 0x45, length >> 8, length & 255
+    rows[:, 28:32] = np.array([p[2] for p in peers], np.uint32)[peer].astype(">u4").view(np.uint8).reshape(n, 4)
+    want, nxt = rows.copy(), np.zeros(N_PEERS, np.int64)
+    for i in range(n):
+        p = int(peer[i])
+        w = O.wg_encap(rows[i, 16:16 + length].tobytes(), MTU, keys[p].tobytes(), peers[p][1], int(nxt[p]))
+        want[i, :len(w)] = np.frombuffer(w, np.uint8)
+        nxt[p] += 1
+    dev = torch.device("cuda:0")
+    ctx = _ctx(peers, keys, keys)
+    buf, d_peer = torch.from_numpy(rows.reshape(-1)).to(dev), torch.from_numpy(peer.view(np.int32)).to(dev)
+    wl = torch.zeros(n, dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    ctx.wg_encap(lib.make_batch(buf, n * stride, n, lib.MEM_DEVICE, stride=stride, length=length, peer=d_peer), MTU, wl)
+    ctx.sync()
+    assert (wl == 1440).all() and np.array_equal(buf.cpu().numpy().reshape(n, stride), want)
+    ctx.wg_peers_set([(b, a, c, d) for a, b, c, d in peers])
+    out, res = torch.zeros(n * stride, dtype=torch.uint8, device=dev), torch.full((n,), 99, dtype=torch.uint8, device=dev)
+    olen, gp = (torch.zeros(n, dtype=torch.int32, device=dev) for _ in range(2))
+    gc = torch.zeros(n, dtype=torch.int64, device=dev)
+    torch.cuda.synchronize()
+    ctx.wg_decap(lib.make_batch(buf, n * stride, n, lib.MEM_DEVICE, stride=stride, length=1440),
+                 lib.make_batch(out, n * stride, n, lib.MEM_DEVICE, stride=stride), res, olen, gp, gc)
+    ctx.sync()
+    assert (res == 0).all() and (olen == length).all() and np.array_equal(gp.cpu().numpy().view(np.uint32), peer)
+    assert np.array_equal(out.cpu().numpy().reshape(n, stride)[:, :length], rows[:, 16:16 + length])
+    ctx.close()

@@ -3,8 +3,8 @@ point of a context.  They are an addition (the reference's filter drops
 without counting, internal/filter/filter.go:100-145), so what is checked is
 that they are the histogram of the result bytes the calls return -- which the
 other tests pin against the oracle -- for host batches (counted on the host)
-and device-resident ones (counted by a launch behind the batch) alike, that a
-failed call counts nothing, and that merged calls count once."""
+and device-resident ones (counted by the launch itself, or by one behind it)
+alike, that a failed call counts nothing, and that merged calls count once."""
 import threading
 
 import numpy as np
@@ -78,6 +78,49 @@ def test_seal_open_counts_host_and_device_and_reset():
                  lib.make_batch(d_back, back.nbytes, n - 8, lib.MEM_DEVICE, stride=stride), d_verdict[5:])
         late = int((forged >= n - 8).sum())
         assert ctx.counters() == {**ZERO, "opened": n - 8 - (7 - late), "rejected": 7 - late}
+
+
+@pytest.mark.parametrize("n,spread_max", [(300, 4096), (5000, 4096), (700, 0), (60000, 4096)])
+def test_an_open_counts_every_way_to_be_refused(n, spread_max):
+    """The launches of a wave, a few lanes and a lane per packet count their own verdicts: forged
+    packets, packets too short for a tag, beyond the arena or of no peer, long ones among them."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    keys = rng.integers(0, 256, (4, 32), dtype=np.uint8)
+    peer = rng.integers(0, 4, n).astype(np.uint32)
+    ctr = np.arange(n, dtype=np.uint64)
+    lens = rng.choice([0, 1, 60, 300], n).astype(np.uint32)
+    lens[::97] = 4500  # beyond 63 blocks
+    slot = (lens.astype(np.int64) + 16 + 15) & ~15
+    off = (np.cumsum(slot) - slot).astype(np.uint64)
+    total = int(slot.sum())
+    plain, sealed = rng.integers(0, 256, total, dtype=np.uint8), np.zeros(total, np.uint8)
+    O.seal_batch(keys, peer, ctr, plain, off, lens, sealed, off, 4)
+    ct = lens + np.uint32(16)
+    way = rng.choice(8, n)
+    for i in np.flatnonzero(way == 1):
+        sealed[int(off[i]) + int(ct[i]) - 1] ^= 1
+    ct[way == 2] = rng.integers(0, 16, int((way == 2).sum()))
+    off_b, peer_b = off.copy(), peer.copy()
+    off_b[way == 3] = total + 16
+    peer_b[way == 4] = 4
+    want = ((way == 0) | (way > 4)).astype(np.uint8)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    with lib.Context(0) as ctx:
+        ctx.set_spread_max_packets(spread_max)
+        ctx.keys_set(lib.KEYS_RECV, keys)
+        d_in, d_out = d(sealed), torch.zeros(total, dtype=torch.uint8, device="cuda:0")
+        verdict = torch.full((n,), 9, dtype=torch.uint8, device="cuda:0")
+        d_off, d_ct, d_peer, d_ctr = d(off_b.view(np.int64)), d(ct.view(np.int32)), d(peer_b.view(np.int32)), d(ctr.view(np.int64))
+        torch.cuda.synchronize()
+        ctx.open(lib.make_batch(d_in, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_ct, peer=d_peer, counters=d_ctr),
+                 lib.make_batch(d_out, total, n, lib.MEM_DEVICE, offsets=d(off.view(np.int64))), verdict)
+        with pytest.raises(lib.BnkError):
+            ctx.sync()
+        assert np.array_equal(verdict.cpu().numpy(), want)
+        assert ctx.counters() == {**ZERO, "opened": int(want.sum()), "rejected": int(n - want.sum())}
 
 
 def test_merged_calls_count_once_each():

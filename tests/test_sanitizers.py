@@ -4,7 +4,8 @@ detector (README.md:79) and fuzzes the parser that reads datagrams from the
 network (internal/disco/fuzz_test.go:6-15); here:
 
   AddressSanitizer + UndefinedBehaviorSanitizer (any report ends the program)
-      the kernels' lane arithmetic compiled for the host, the replay window,
+      the kernels' lane arithmetic compiled for the host, the rules around a launch,
+      the replay window,
       the Bind mirror over loopback, the filter-call coalescer, each with the C
       oracle's sources built the same way where they link it;
       the oracle's own Python tests against oracle/san/libbnkoracle.so;
@@ -35,6 +36,7 @@ def _run(path, *args, timeout=300):
 def test_host_code_under_address_and_undefined_behaviour_sanitizers():
     subprocess.run(["make", "-s", "-C", CPP, "san"], check=True)
     assert "PASS lane arithmetic" in _run(os.path.join(CPP, "san", "lane_test"))
+    assert "PASS launch rules" in _run(os.path.join(CPP, "san", "route_test"))
     assert "ok" in _run(os.path.join(CPP, "san", "replay_test"))
     assert "ok" in _run(os.path.join(CPP, "san", "coalesce_test"))
     assert "ok" in _run(os.path.join(CPP, "san", "bind_test"))

@@ -534,8 +534,12 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         // the packet's last 1-15 bytes end in this step
         const uint32_t kt = len >> 4;
         const bool tail = (len & 15u) != 0u && (len >> 7) == s;
-        if (!ALIGNED && tail) // (their cell has not come into LDS)
-            *cell(kt) = ld_partial(src + 16u * kt, len_in > 16u * kt ? len_in - 16u * kt : 0u);
+        if (!ALIGNED && tail) { // (their cell has not come into LDS)
+            // (where its bytes lie is worked out here and not ahead of the loop, which has no registers for it)
+            uint32_t kt_here = kt;
+            asm volatile("" : "+v"(kt_here));
+            *cell(kt_here) = ld_partial(src + 16u * kt_here, len_in > 16u * kt_here ? len_in - 16u * kt_here : 0u);
+        }
         uint4 cur = *cell(8u * s);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -655,7 +659,8 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
             } else {
 #pragma unroll 1
                 for (uint32_t h = 0; h < 2; h++) {
-                    const uint32_t b = 2u * s + h;
+                    uint32_t b = 2u * s + h;
+                    if (!ALIGNED) asm volatile("" : "+v"(b)); // (as in run_step)
                     if (64u * b < len) {
                         chacha_block(k, b + 1, n1, n2, x);
 #pragma unroll
@@ -754,6 +759,8 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         chacha_block2_shared(k, shared, 0, n1, n2, x, y);
     }
     mac.init(x);
+    // (the second half of the one-time key waits behind the lane's cells: four registers)
+    if (LEAN) *reinterpret_cast<uint4 *>(tile + lane * SHORT_ROW + 128u) = make_uint4(x[4], x[5], x[6], x[7]);
 #pragma unroll
     for (int q = 0; q < 8; q++)
         if (jcell[q] < nld[q]) *reinterpret_cast<uint4 *>(rows + 8u * q * SHORT_ROW + (jcell[q] << 4)) = pre[0][q];
@@ -770,7 +777,16 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const uint32_t kc = 4u * b + j;
-            if (kc < ncell_in) crypt_cell_v<OPEN>(mac, ks, j, v[j], row + (kc << 4));
+            if (LEAN && kc == 0u) {
+                // (the packet's first cell: the MAC has nothing to multiply yet)
+                uint4 c = v[0];
+                if (len_in < 16u) c = keep_bytes(c, len_in);
+                uint4 o = make_uint4(c.x ^ ks[0], c.y ^ ks[1], c.z ^ ks[2], c.w ^ ks[3]);
+                if (len < 16u) o = keep_bytes(o, len);
+                mac.start(OPEN ? c.x : o.x, OPEN ? c.y : o.y, OPEN ? c.z : o.z, OPEN ? c.w : o.w);
+                if (len < 16u) st_partial(dst, o, len);
+                *reinterpret_cast<uint4 *>(row) = o;
+            } else if (kc < ncell_in) crypt_cell_v<OPEN>(mac, ks, j, v[j], row + (kc << 4));
             else if (kc < ncell || (kc == ncell && (len & 15u))) {
                 const uint32_t m_out = kc < ncell ? 16u : len & 15u;
                 const uint32_t m_in = len_in > 16u * kc ? min(len_in - 16u * kc, m_out) : 0u;
@@ -793,6 +809,10 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         crypt_block(1, x, v);
     }
     if (OPEN) capture_head(head, row, row + 16);
+    if (LEAN) {
+        const uint4 pad = *reinterpret_cast<const uint4 *>(row + 128);
+        mac.pad0 = pad.x; mac.pad1 = pad.y; mac.pad2 = pad.z; mac.pad3 = pad.w;
+    }
     wave_sync();
     if (LEAN) {
 #pragma unroll
@@ -1066,11 +1086,11 @@ BNK_DEV void lane_packet_report(const AeadArgs &a, const LanePacket &p)
 // A lane per packet.  SHORT_ONLY: the launch for batches in which every wave
 // takes the short path (see aead_short_kernel).
 template <bool OPEN, bool SHORT_ONLY>
-BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
+BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile, uint2 *aside)
 {
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t t = blockIdx.x * LANE_BLOCK + threadIdx.x;
-    const LanePacket p = lane_packet<OPEN>(a, t, t < a.n);
+    LanePacket p = lane_packet<OPEN>(a, t, t < a.n);
     const bool lane_lines = (((uintptr_t)p.src | (uintptr_t)p.dst) & 15u) == 0 &&
                             (((uintptr_t)p.src ^ (uintptr_t)p.dst) & 127u) == 0;
     // which launch does this wave's packets: nothing has been written so far
@@ -1093,6 +1113,8 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
     Head head;
     head.on = OPEN && (a.heads != nullptr || decap);
     head.c0 = head.c1 = make_uint4(0, 0, 0, 0);
+    // (which packet it is and whose comes up again only at the end)
+    if (OPEN && !SHORT_ONLY) aside[lane] = make_uint2(p.i, p.pr);
     if (SHORT_ONLY) body_short<OPEN, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
     else if (all_short) body_short<OPEN>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
     else if (!all_lines) {
@@ -1102,6 +1124,11 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile)
     }
     else body_lines<OPEN, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
 
+    if (OPEN && !SHORT_ONLY) {
+        wave_sync();
+        p.i = aside[lane].x;
+        p.pr = aside[lane].y;
+    }
     const bool reject = lane_finish<OPEN>(a, lane, p.have, p.i, p.len, p.src, p.dst, mac, head,
                                           p.in_batch && a.heads ? a.heads + 32ull * t : nullptr,
                                           decap && p.in_batch && p.wg_res == BNK_WG_OK, p.pr);
@@ -1125,8 +1152,9 @@ template <bool OPEN>
 __global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void aead_wave_kernel(AeadArgs a)
 {
     __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * RING_ROW];
+    __shared__ uint2 aside[OPEN ? LANE_KERNEL_WAVES : 1][OPEN ? 64 : 1];
     static_assert(RING_ROW >= LDS_ROW && RING_ROW >= SHORT_ROW, "the other paths reuse the tile");
-    wave_main<OPEN, false>(a, tile_all[threadIdx.x >> 6]);
+    wave_main<OPEN, false>(a, tile_all[threadIdx.x >> 6], aside[OPEN ? threadIdx.x >> 6 : 0]);
 }
 
 // Batches in which the host can tell that every wave takes the short path
@@ -1141,7 +1169,7 @@ __global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHOR
 void aead_short_kernel(AeadArgs a)
 {
     __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * SHORT_ROW];
-    wave_main<OPEN, true>(a, tile_all[threadIdx.x >> 6]);
+    wave_main<OPEN, true>(a, tile_all[threadIdx.x >> 6], nullptr);
 }
 
 // A few lanes per packet, for batches between the two: too few packets to fill

@@ -286,6 +286,11 @@ struct Poly26 {
 // r1..r3, so a product that lands at 2^128 or above folds back exactly with
 // s_j = r_j + r_j/4 = 5*r_j/4 (2^130 = 5 mod p).  Message words are used as
 // they are: no limb extraction, 20 multiplies per block.
+//
+// The accumulator holds h + m, the cell that came last not yet multiplied: a
+// step multiplies by r and adds the next cell, whose words are what the columns
+// of the product start from (a multiply-add takes them for nothing), and the tag
+// takes one more multiplication.  h below is that sum.
 struct Poly32 {
     uint32_t r0, r1, r2, r3;
     uint32_t s1, s2, s3;
@@ -302,10 +307,45 @@ struct Poly32 {
         pad0 = x[4]; pad1 = x[5]; pad2 = x[6]; pad3 = x[7];
     }
 
+    // h = h * r + (w0, w1, w2, w3, top), top 0 or 1.
+    //
+    // One carry chain per cell: each column's upper half is added into the next
+    // column as it is, and what lies at and above 2^130 (known from the top column
+    // and the upper half below it, before any carry) goes in at the bottom of the
+    // same chain.  h4 stays below 6: (e4 & 3) and the chain's last carry and `top`.
+    BNK_DEV void mul_add(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t top)
+    {
+        // h_i < 2^32, r_j < 2^28, s_j < 1.25 * 2^28, h4 * s_j < 2^31: a column stays
+        // below 2^62 + 2^60 + 2^33
+        const uint64_t d3 = (uint64_t)h0 * r3 + w3 + (uint64_t)h1 * r2 + (uint64_t)h2 * r1 + (uint64_t)h3 * r0 +
+                            (uint64_t)h4 * s3;
+        // the column at 2^128: d3 < 4 * 2^60 + small, so its upper half is at most 2^30, and
+        // h4 * r0 < 5 * 2^28: the sum stays below 2.3 * 2^30, and its part above 2^130 times
+        // five below 2^32
+        const uint32_t e4 = h4 * r0 + (uint32_t)(d3 >> 32);
+        const uint64_t d0 = (uint64_t)h0 * r0 + w0 + (uint64_t)h1 * s3 + (uint64_t)h2 * s2 + (uint64_t)h3 * s1;
+        const uint64_t d1 = (uint64_t)h0 * r1 + w1 + (uint64_t)h1 * r0 + (uint64_t)h2 * s3 + (uint64_t)h3 * s2 +
+                            (uint64_t)h4 * s1;
+        const uint64_t d2 = (uint64_t)h0 * r2 + w2 + (uint64_t)h1 * r1 + (uint64_t)h2 * r0 + (uint64_t)h3 * s3 +
+                            (uint64_t)h4 * s2;
+        uint32_t c;
+        h0 = addc32((uint32_t)d0, (e4 >> 2) * 5u, 0, c);
+        h1 = addc32((uint32_t)d1, (uint32_t)(d0 >> 32), c, c);
+        h2 = addc32((uint32_t)d2, (uint32_t)(d1 >> 32), c, c);
+        h3 = addc32((uint32_t)d3, (uint32_t)(d2 >> 32), c, c);
+        h4 = (e4 & 3u) + top + c;
+    }
+
+    // The first block: nothing to multiply yet.
+    BNK_DEV void start(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3)
+    {
+        h0 = w0; h1 = w1; h2 = w2; h3 = w3; h4 = 1u;
+    }
+
     // One full 16-byte block (little-endian words w0..w3) with bit 128 set.
     // Additions go 32 bits at a time with an explicit carry (add-with-carry
     // instructions on the GPU; written as 64-bit sums the compiler builds each
-    // zero-extended operand with a move first: 68 instructions a block against 47).
+    // zero-extended operand with a move first).
     // The block runs at raised wave priority for the same reason as the rotates of
     // ChaCha20: nearly all of it is multiplies and carries, which a SIMD takes
     // from one wave at a time.
@@ -314,39 +354,7 @@ struct Poly32 {
 #if defined(__HIP_DEVICE_COMPILE__)
         __builtin_amdgcn_s_setprio(1);
 #endif
-        uint32_t c;
-        const uint32_t a0 = addc32(h0, w0, 0, c);
-        const uint32_t a1 = addc32(h1, w1, c, c);
-        const uint32_t a2 = addc32(h2, w2, c, c);
-        const uint32_t a3 = addc32(h3, w3, c, c);
-        const uint32_t a4 = h4 + 1u + c; // at most 9
-
-        // a_i < 2^32, r_j < 2^28, s_j < 1.25 * 2^28: four terms stay below 2^63,
-        // and a4 * s_j below 2^32
-        const uint64_t d0 = (uint64_t)a0 * r0 + (uint64_t)a1 * s3 + (uint64_t)a2 * s2 + (uint64_t)a3 * s1;
-        const uint64_t d1 = (uint64_t)a0 * r1 + (uint64_t)a1 * r0 + (uint64_t)a2 * s3 + (uint64_t)a3 * s2 +
-                            (uint64_t)a4 * s1;
-        const uint64_t d2 = (uint64_t)a0 * r2 + (uint64_t)a1 * r1 + (uint64_t)a2 * r0 + (uint64_t)a3 * s3 +
-                            (uint64_t)a4 * s2;
-        const uint64_t d3 = (uint64_t)a0 * r3 + (uint64_t)a1 * r2 + (uint64_t)a2 * r1 + (uint64_t)a3 * r0 +
-                            (uint64_t)a4 * s3;
-        uint32_t e4 = a4 * r0; // stays at 2^128; below 2^32 because a4 <= 9
-
-        // each column's upper half goes into the next column
-        const uint32_t l1 = addc32((uint32_t)d1, (uint32_t)(d0 >> 32), 0, c);
-        const uint32_t u1 = (uint32_t)(d1 >> 32) + c;
-        const uint32_t l2 = addc32((uint32_t)d2, u1, 0, c);
-        const uint32_t u2 = (uint32_t)(d2 >> 32) + c;
-        const uint32_t l3 = addc32((uint32_t)d3, u2, 0, c);
-        const uint32_t u3 = (uint32_t)(d3 >> 32) + c;
-        e4 += u3;
-        // everything at and above 2^130 comes back times 5
-        const uint32_t f = (e4 >> 2) * 5u;
-        h0 = addc32((uint32_t)d0, f, 0, c);
-        h1 = addc32(l1, 0, c, c);
-        h2 = addc32(l2, 0, c, c);
-        h3 = addc32(l3, 0, c, c);
-        h4 = (e4 & 3u) + c;
+        mul_add(w0, w1, w2, w3, 1u);
 #if defined(__HIP_DEVICE_COMPILE__)
         __builtin_amdgcn_s_setprio(0);
 #endif
@@ -355,6 +363,7 @@ struct Poly32 {
     // tag = ((h mod 2^130-5) + s) mod 2^128 as four little-endian words
     BNK_DEV void finish(uint32_t (&tag)[4])
     {
+        mul_add(0, 0, 0, 0, 0); // the last cell's multiplication
         // h < 2^130 + small: h >= p  <=>  h + 5 >= 2^130
         uint64_t t;
         t = (uint64_t)h0 + 5u;         const uint32_t g0 = (uint32_t)t;

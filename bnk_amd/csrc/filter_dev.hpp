@@ -67,6 +67,7 @@ struct RuleIndexDev {
     uint32_t n_bounds;
     uint32_t top_step;      // largest power of two < n_bounds (0 when n_bounds == 1)
     uint32_t n_wide;
+    bool long_lists;        // some interval's list is longer than a block
 };
 
 struct FilterArgs {

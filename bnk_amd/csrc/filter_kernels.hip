@@ -170,31 +170,37 @@ BNK_DEV uint32_t interval_of(Ptr bounds, uint32_t n, uint32_t top_step, uint32_t
 
 // The same with the jump table: only the cut points of src's address bucket
 // are searched (a handful instead of thirteen halvings for 8192 cut points).
+// Every lane of the wave must call it: the lanes halve together until the last of them
+// is there (a lane that is keeps its answer), so the loop is a vote and a few selects
+// instead of a mask that shrinks lane by lane.  valid: false asks for 0.
 BNK_DEV uint32_t interval_of_jump(const uint32_t *bounds, const uint16_t *jump, uint32_t jump_lo,
-                                  uint32_t jump_shift, uint32_t src)
+                                  uint32_t jump_shift, uint32_t src, bool valid)
 {
-    if (src < jump_lo) return 0; // below bounds[1]
+    const bool in = valid & (src >= jump_lo); // (else below bounds[1])
     uint32_t b = (src - jump_lo) >> jump_shift;
-    b = b < JUMP_BUCKETS ? b : JUMP_BUCKETS - 1u;
-    uint32_t lo = jump[b], hi = jump[b + 1u] + 1u; // the answer lies in [lo, hi)
-    if (b == JUMP_BUCKETS - 1u) {
-        // the last bucket also takes everything above the last cut point
-        hi = jump[JUMP_BUCKETS] + 1u;
-    }
-    while (hi - lo > 1u) {
+    b = b < JUMP_BUCKETS ? b : JUMP_BUCKETS - 1u; // the last bucket also takes everything above the last cut point
+    const uint32_t first = jump[b], last = jump[b + 1u];
+    uint32_t lo = in ? first : 0u, hi = in ? last + 1u : 1u; // the answer lies in [lo, hi)
+    while (__ballot(hi - lo > 1u) != 0ull) {
         const uint32_t mid = (lo + hi) >> 1;
-        if (bounds[mid] <= src) lo = mid;
-        else hi = mid;
+        const bool up = (bounds[mid] <= src) | (mid == lo);
+        lo = up ? mid : lo;
+        hi = up ? hi : mid;
     }
     return lo;
 }
 
-// One word holds a range: key_lo << 14 | key_hi - key_lo.
-BNK_DEV bool in_range(uint32_t e, uint32_t key) { return key - (e >> 14) <= (e & RANGE_MAX_SPAN); }
-
-BNK_DEV bool quad_hit(uint4 v, uint32_t key)
+// One word holds a range: key_lo << 14 | key_hi - key_lo.  How far the key lies beyond it, 0 in it.
+BNK_DEV uint32_t range_miss(uint32_t e, uint32_t key)
 {
-    return in_range(v.x, key) || in_range(v.y, key) || in_range(v.z, key) || in_range(v.w, key);
+    return __builtin_elementwise_sub_sat(key - (e >> 14), e & RANGE_MAX_SPAN);
+}
+
+// 0 if one of the four has the key.  (As a chain of comparisons the compiler tests one word,
+// branches, and fetches the next ones only then.)
+BNK_DEV uint32_t quad_miss(uint4 v, uint32_t key)
+{
+    return min(min(range_miss(v.x, key), range_miss(v.y, key)), min(range_miss(v.z, key), range_miss(v.w, key)));
 }
 
 // Value of x in lane J of this lane's quad (lanes 4k .. 4k+3).
@@ -202,6 +208,13 @@ template <int J>
 BNK_DEV uint32_t quad_bcast(uint32_t x)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, J | J << 2 | J << 4 | J << 6, 0xF, 0xF, true);
+}
+
+// Value of x in lane A, B, C or D of the quad, for its first to fourth lane.
+template <int A, int B, int C, int D>
+BNK_DEV uint32_t quad_perm(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, A | B << 2 | C << 4 | D << 6, 0xF, 0xF, true);
 }
 
 // A list of more than 16 pieces: head is the first quad of the interval's own
@@ -218,7 +231,7 @@ BNK_DEV bool long_list_hit(const RuleIndexDev &ri, uint32_t first, uint32_t nblk
     }
     const uint4 *b = ob + 4u * lo;
     const uint4 w0 = b[0], w1 = b[1], w2 = b[2], w3 = b[3];
-    return quad_hit(w0, key) || quad_hit(w1, key) || quad_hit(w2, key) || quad_hit(w3, key);
+    return min(min(quad_miss(w0, key), quad_miss(w1, key)), min(quad_miss(w2, key), quad_miss(w3, key))) == 0u;
 }
 
 // Rule lookup for the four packets of a quad of lanes at once; every lane of the
@@ -229,33 +242,47 @@ BNK_DEV bool long_list_hit(const RuleIndexDev &ri, uint32_t first, uint32_t nblk
 // packet's block together, 16 bytes each, which the memory pipeline sees as a
 // single 64-byte access, and do that for each of their four packets in turn.
 // Each lane tests its 16 bytes against the key of the packet they belong to and
-// the verdicts are gathered per quad with a wave-wide vote.
-BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, uint32_t lane, uint32_t iv, uint32_t src, uint32_t key)
+// the answers are gathered within the quad.
+struct QuadBlocks {
+    uint4 p0, p1, p2, p3; // the lane's 16 bytes of the blocks of its quad's four packets
+};
+// SMALL: there are at most 2^16 intervals (a byte offset among their blocks has 32 bits).
+template <bool SMALL>
+BNK_DEV const uint4 *rules_block(const RuleIndexDev &ri, uint32_t iv)
 {
-    const uint32_t part = lane & 3u, qshift = lane & ~3u;
-    const uint32_t *mine = ri.ranges + part * 4u;
-    const uint32_t iv0 = quad_bcast<0>(iv), iv1 = quad_bcast<1>(iv), iv2 = quad_bcast<2>(iv), iv3 = quad_bcast<3>(iv);
-    const uint4 p0 = *reinterpret_cast<const uint4 *>(mine + (size_t)iv0 * RANGE_BLOCK);
-    const uint4 p1 = *reinterpret_cast<const uint4 *>(mine + (size_t)iv1 * RANGE_BLOCK);
-    const uint4 p2 = *reinterpret_cast<const uint4 *>(mine + (size_t)iv2 * RANGE_BLOCK);
-    const uint4 p3 = *reinterpret_cast<const uint4 *>(mine + (size_t)iv3 * RANGE_BLOCK);
-    const unsigned long long h0 = __ballot(quad_hit(p0, quad_bcast<0>(key)));
-    const unsigned long long h1 = __ballot(quad_hit(p1, quad_bcast<1>(key)));
-    const unsigned long long h2 = __ballot(quad_hit(p2, quad_bcast<2>(key)));
-    const unsigned long long h3 = __ballot(quad_hit(p3, quad_bcast<3>(key)));
-    const unsigned long long hm = part == 0u ? h0 : part == 1u ? h1 : part == 2u ? h2 : h3;
-    bool hit = ((hm >> qshift) & 0xFull) != 0ull;
-    // a long list shows in the first word of its block, which the quad's first
-    // lane holds for round j as p<j>; the votes are taken by all lanes together
-    const unsigned long long l0 = __ballot(part == 0u && p0.x == RANGE_LONG);
-    const unsigned long long l1 = __ballot(part == 0u && p1.x == RANGE_LONG);
-    const unsigned long long l2 = __ballot(part == 0u && p2.x == RANGE_LONG);
-    const unsigned long long l3 = __ballot(part == 0u && p3.x == RANGE_LONG);
-    const unsigned long long lm = part == 0u ? l0 : part == 1u ? l1 : part == 2u ? l2 : l3;
-    if ((lm >> qshift) & 1ull) {
-        // rare: fetch the pointer words myself (the line is in L1 by now)
-        const uint4 head = *reinterpret_cast<const uint4 *>(ri.ranges + (size_t)iv * RANGE_BLOCK);
-        hit = long_list_hit(ri, head.y, head.z, key);
+    const uint8_t *const blocks = reinterpret_cast<const uint8_t *>(ri.ranges);
+    return reinterpret_cast<const uint4 *>(blocks + (SMALL ? iv * (RANGE_BLOCK * 4u) : (size_t)iv * (RANGE_BLOCK * 4u)));
+}
+
+template <bool SMALL>
+BNK_DEV QuadBlocks rules_fetch_quad(const RuleIndexDev &ri, uint32_t lane, uint32_t iv)
+{
+    const uint32_t part = lane & 3u;
+    return QuadBlocks{rules_block<SMALL>(ri, quad_bcast<0>(iv))[part], rules_block<SMALL>(ri, quad_bcast<1>(iv))[part],
+                      rules_block<SMALL>(ri, quad_bcast<2>(iv))[part], rules_block<SMALL>(ri, quad_bcast<3>(iv))[part]};
+}
+
+template <bool SMALL>
+BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint32_t lane, uint32_t iv, uint32_t src, uint32_t key)
+{
+    const uint32_t part = lane & 3u;
+    // packet j of the quad in the lane's own 16 bytes, and of all that the quad's lanes find the
+    // least for the lane's own packet: two exchanges, in which a lane hands over what it has
+    // found for its neighbours' packets
+    const uint32_t m0 = quad_miss(q.p0, quad_bcast<0>(key)), m1 = quad_miss(q.p1, quad_bcast<1>(key)),
+                   m2 = quad_miss(q.p2, quad_bcast<2>(key)), m3 = quad_miss(q.p3, quad_bcast<3>(key));
+    const bool odd = (part & 1u) != 0u, upper = (part & 2u) != 0u;
+    const uint32_t lo = min(odd ? m1 : m0, quad_perm<1, 0, 3, 2>(odd ? m0 : m1)),
+                   hi = min(odd ? m3 : m2, quad_perm<1, 0, 3, 2>(odd ? m2 : m3));
+    bool hit = min(upper ? hi : lo, quad_perm<2, 3, 0, 1>(upper ? lo : hi)) == 0u;
+    if (ri.long_lists) {
+        // it shows in the first word of the block, which the quad's first lane holds for packet j
+        // as p<j>.x
+        const bool far = (q.p0.x == RANGE_LONG) | (q.p1.x == RANGE_LONG) | (q.p2.x == RANGE_LONG) | (q.p3.x == RANGE_LONG);
+        if (__ballot(far & (part == 0u)) != 0ull) {
+            const uint4 head = *rules_block<SMALL>(ri, iv); // (the line is in L1 by now)
+            if (head.x == RANGE_LONG) hit = long_list_hit(ri, head.y, head.z, key);
+        }
     }
     if (!hit)
         for (uint32_t w = 0; w < ri.n_wide; w++) {
@@ -277,17 +304,25 @@ constexpr uint32_t LDS_JUMP_ROOM = (LDS_JUMP_WORDS + 3u) & ~3u;
 // What a lane reads of a packet before anything is decided about it.
 struct RawHeader {
     u32x4 a;        // bytes 0-15
-    u32x2 b;        // bytes 16-23, or 12-19 of a packet too short for those
+    uint32_t ports; // bytes 20-23, of a packet that has them
     uint32_t len;   // of the packet, without what is trimmed off
     uint32_t i;     // the packet
     bool ok;        // there is a packet to look at
     uint8_t result; // what a decapsulating call said about it so far
 };
 
+// Where a launch finds its headers: in packets of one length at one stride and nothing else to
+// look at; in packets with per-packet arrays, whichever of them there are; in the records of
+// FilterArgs::heads.  A launch is compiled for one of them: with all three in one kernel its
+// arguments do not fit the scalar registers and are fetched out of vector registers lane by
+// lane wherever they are used (2^22 plain headers: 510 vector and 280 scalar instructions per
+// 64 packets).
+enum HeaderFrom { FROM_PLAIN, FROM_ARRAYS, FROM_RECORDS };
+
 // The loads of one packet, every one issued whether or not the lane needs it (from `safe`, 32
 // readable bytes, where it does not: a load under a branch is waited for where the branch
-// closes).  The per-packet arrays are looked at only if the launch has one at all: four loads
-// from `safe` per packet cost a launch over plain records 4 us in 77 (2^22 packets).
+// closes).
+template <int FROM>
 BNK_DEV RawHeader fetch_header(const FilterArgs &a, uint32_t t)
 {
     RawHeader r;
@@ -296,22 +331,20 @@ BNK_DEV RawHeader fetch_header(const FilterArgs &a, uint32_t t)
     const uint8_t *const safe = reinterpret_cast<const uint8_t *>(a.flows.counters);
     r.i = tt;
     r.result = 0;
-    if (a.heads) {
+    if (FROM == FROM_RECORDS) {
         // whoever wrote the records has checked the packets against the arena
         r.a = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt);
         const u32x4 r1 = *reinterpret_cast<const u32x4 *>(a.heads + 32ull * tt + 16);
         if (a.order) r.i = a.order[tt];
-        r.b = u32x2{r1.x, r1.y};
+        r.ports = r1.y;
         r.len = r1.z;
         r.ok = in && r1.w != 0u && r.len >= 20u;
-        // (a record holds bytes 16-23 where the packet has them)
-        if (r.len < 24u) r.b = u32x2{0u, r1.x};
         return r;
     }
     uint32_t len = a.len;
     uint64_t at = (uint64_t)tt * a.stride;
     bool open = true;
-    if (a.gate || a.lens || a.off || a.wg_result) { // (the same for the whole launch)
+    if (FROM == FROM_ARRAYS) {
         r.result = *(a.wg_result ? a.wg_result + tt : safe);
         const uint8_t gate = *(a.gate ? a.gate + tt : safe);
         const uint32_t len_ld = *(a.lens ? a.lens + tt : reinterpret_cast<const uint32_t *>(safe));
@@ -322,37 +355,64 @@ BNK_DEV RawHeader fetch_header(const FilterArgs &a, uint32_t t)
     }
     r.len = len - (len >= a.trim ? a.trim : len);
     r.ok = in && open;
-    if (r.ok && beyond_arena(at, len, a.limit)) {
+    if (FROM == FROM_ARRAYS && r.ok && beyond_arena(at, len, a.limit)) {
         status_raise(a.status, STATUS_BOUNDS);
         r.ok = false;
     }
     r.ok = r.ok && r.len >= 20u;
     const uint8_t *const p = r.ok ? a.pkts + at : safe;
     r.a = *reinterpret_cast<const u32x4_unaligned *>(p);
-    r.b = *reinterpret_cast<const u32x2_unaligned *>(p + (r.ok && r.len < 24u ? 12 : 16));
+    r.ports = ld32u(p + (r.len >= 24u ? 20u : 12u));
     return r;
 }
 
+// filter.go:71-106 on what was fetched (parse_words without its branches): every lane goes
+// through all of it, and only a header with options takes a look at the packet itself.
+template <int FROM>
+BNK_DEV bool parse_fetched(const FilterArgs &a, const RawHeader &r, Parsed &o)
+{
+    const uint32_t ihl = (r.a.x & 0xFu) * 4u;
+    o.proto = (r.a.z >> 8) & 0xFFu;
+    o.src = __builtin_bswap32(r.a.w);
+    const bool ports = (o.proto == 6u) | (o.proto == 17u);
+    const bool ok = r.ok & (((r.a.x >> 4) & 0xFu) == 4u) & (ihl >= 20u) & (ports | (o.proto == 1u)) &
+                    (r.len >= ihl + (ports ? 4u : 1u));
+    uint32_t w = r.ports; // (with ports behind 20 bytes of header the packet has 24)
+    if (ok && ports && ihl != 20u) w = ld32u(PacketAt{a.pkts, FROM == FROM_PLAIN ? nullptr : a.off, a.stride, r.i}.get() + ihl);
+    w = ports ? __builtin_bswap32(w) : 0u;
+    o.sport = w >> 16;
+    o.dport = w & 0xFFFFu;
+    return ok;
+}
+
 // filter.go:121-147 for a batch; enforcement is on (the host short-circuits
-// allow-all mode).
+// allow-all mode).  JUMPS: the cut points and the jump table are in LDS.
+template <int FROM, bool JUMPS>
 __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     const RuleIndexDev ri = a.rules;
-    const bool in_lds = ri.n_bounds <= LDS_BOUNDS_MAX;
-    const bool jumps = in_lds && ri.jump != nullptr;
+    const bool in_lds = JUMPS || ri.n_bounds <= LDS_BOUNDS_MAX;
+    constexpr bool jumps = JUMPS;
     const bool small = a.small_in_lds != 0u && a.flows.counters[FLOW_CLAIMED] <= SMALL_KEYS_MAX;
     uint32_t *lsmall = lds, *ljw = lds + (a.small_in_lds ? LDS_SMALL_WORDS : 0u), *lb = ljw + (jumps ? LDS_JUMP_ROOM : 0u);
     const uint16_t *lj = reinterpret_cast<const uint16_t *>(ljw);
     const uint32_t stride = gridDim.x * FILTER_THREADS;
     const uint32_t lane = threadIdx.x & 63u;
     // The first packet's header flies while the tables are staged, and theirs is one trip: 16
-    // bytes per lane and load, all of them in flight together.  A call of 2^22 packets on 4096
-    // rules and 65,536 flows takes 74.1 us, on 64 rules and 500 flows 57.0; 2^14 packets 10.6 and
-    // 8.8.  Staging word by word, each waited for, with every header where it is parsed: 77.2 and
-    // 59.2; 11.5 and 9.4.  Later headers fetched ahead of the packet before them instead of
-    // behind it: 12 registers more, 75.5 and 60.0; 11.2 and 9.4.
-    RawHeader raw = fetch_header(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
+    // bytes per lane and load, all of them in flight together (word by word, each waited for:
+    // 3 us more for 2^22 packets, 1 for 2^14).
+    //
+    // What bounds the launch: 8 waves per SIMD, of whose time half is spent waiting for memory
+    // (a packet's rule list, presence word and flow slot come from L2 and beyond, one behind the
+    // other) and a third waiting to issue, half of the VALU's slots taken.  So both count, the
+    // instructions and the order in which memory is asked: 2^22 plain headers on 4096 rules and
+    // 65,536 flows took 79.3 us with 510 vector and 280 scalar instructions per 64 packets, the
+    // rule lists fetched a word at a time as the tests before it failed; compiled per kind of
+    // launch, without branches in the parse and the tests, and with the loads ahead of what
+    // waits for them 355 and 111, and 67.4.  The next header ahead of the flow's look-up as
+    // well: 72 (its loads queue ahead of the look-up's).
+    RawHeader raw = fetch_header<FROM>(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
     {
         constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = (SMALL_QUADS + FILTER_THREADS - 1u) / FILTER_THREADS;
         static_assert(LDS_SMALL_WORDS % 4u == 0u, "whole quads");
@@ -385,7 +445,7 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     __syncthreads();
     uint32_t n_pass = 0, n_drop = 0; // this wave's verdicts (the same in every lane)
     uint32_t n_result = 0;           // with wg_tally: how often lane v's value v came out as the result
-    if (blockIdx.x == 0u && threadIdx.x == 0u) {
+    if (blockIdx.x == 0u && threadIdx.x == FILTER_THREADS - 64u) { // (the wave of a small batch that has nothing else to do)
         // (what this batch refreshes expires no earlier than this: news only if the clock went back)
         const int64_t from = a.now + FLOW_TTL_LEAST;
         for (const uint32_t w : {FLOW_MIN_EXP, FLOW_NEXT_EXP}) {
@@ -399,34 +459,29 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         const uint32_t t = i0 + lane;
         const uint32_t i = raw.i;
         Parsed h{};
-        const bool wide = raw.len >= 24u;
-        const bool valid = raw.ok && parse_words(raw.a, wide ? raw.b.x : raw.b.y, raw.b.y, wide, raw.len, h,
-                                                 PacketAt{a.pkts, a.off, a.stride, i});
-        uint32_t key = 0, iv = 0;
-        bool maybe = false;
-        FlowSlot s{};
-        if (valid) {
-            key = proto_class(h.proto) << 16 | h.dport;
-            iv = jumps    ? interval_of_jump(lb, lj, ri.jump_lo, ri.jump_shift, h.src)
-                 : in_lds ? interval_of(lb, ri.n_bounds, ri.top_step, h.src)
-                          : interval_of(ri.bounds, ri.n_bounds, ri.top_step, h.src);
-            // return traffic: remote = src, remotePort = srcPort, localPort = dstPort.
-            // A clear presence bit means the key was never stored: no probe
-            // needed.  The bits come from LDS when the small bitmap is in use;
-            // otherwise the word is fetched alongside the rule list, not after it.
-            s = flow_slot(a.flows, h.src, h.sport, h.dport, h.proto);
-            if (small) {
-                maybe = ((lsmall[s.sbit0 >> 5] >> (s.sbit0 & 31u)) & (lsmall[s.sbit1 >> 5] >> (s.sbit1 & 31u)) & 1u) != 0u;
-                // one in eleven keys that were never stored passes the small
-                // filter; the large one (a word from L2) turns nine in ten of
-                // those away before they cost a 128-byte line of the table
-                if (maybe) maybe = ((a.flows.present[s.bit >> 5] >> (s.bit & 31u)) & 1u) != 0u;
-            } else {
-                maybe = ((a.flows.present[s.bit >> 5] >> (s.bit & 31u)) & 1u) != 0u;
-            }
-        }
+        const bool valid = parse_fetched<FROM>(a, raw, h);
+        const uint32_t key = proto_class(h.proto) << 16 | h.dport;
+        const uint32_t iv = JUMPS    ? interval_of_jump(lb, lj, ri.jump_lo, ri.jump_shift, h.src, valid)
+                            : !valid ? 0u
+                            : in_lds ? interval_of(lb, ri.n_bounds, ri.top_step, h.src)
+                                     : interval_of(ri.bounds, ri.n_bounds, ri.top_step, h.src);
+        // What the packet waits for is asked for in the order it is needed, with nothing waited for
+        // in between: its rule list, then the word that says whether its flow was ever stored.
+        const QuadBlocks blocks = rules_fetch_quad<JUMPS>(ri, lane, iv);
+        // return traffic: remote = src, remotePort = srcPort, localPort = dstPort.
+        // A clear presence bit means the key was never stored: no probe
+        // needed.  The small bitmap is in LDS where it is in use:
+        // one in eleven keys that were never stored passes it; the large one
+        // turns nine in ten of those away before they cost a 128-byte line of the table.
+        const FlowSlot s = flow_slot(a.flows, h.src, h.sport, h.dport, h.proto);
+        bool maybe = valid;
+        if (small)
+            maybe &= ((lsmall[s.sbit0 >> 5] >> (s.sbit0 & 31u)) & (lsmall[s.sbit1 >> 5] >> (s.sbit1 & 31u)) & 1u) != 0u;
+        const uint32_t present = a.flows.present[maybe ? s.bit >> 5 : 0u];
+        asm volatile("" ::: "memory"); // (both are on their way before either is waited for)
+        maybe &= ((present >> (s.bit & 31u)) & 1u) != 0u;
         uint8_t pass = 0;
-        if (rules_match_quad(ri, lane, iv, h.src, key)) {
+        if (rules_match_quad<JUMPS>(ri, blocks, lane, iv, h.src, key)) {
             pass = valid ? 1 : 0;
         } else if (valid) {
             for (uint32_t probe = 0; maybe && probe < a.flows.cap; probe++) {
@@ -465,22 +520,22 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         if (t < a.n) {
             a.verdict[i] = pass;
             // a packet WireGuard delivered and this filter denied (BNK_WG_OK is 0)
-            if (a.wg_result && !pass && raw.result == BNK_WG_OK) a.wg_result[i] = BNK_WG_FILTERED;
+            if (FROM == FROM_ARRAYS && a.wg_result && !pass && raw.result == BNK_WG_OK) a.wg_result[i] = BNK_WG_FILTERED;
         }
-        if (a.wg_tally)
+        if (FROM == FROM_ARRAYS && a.wg_tally)
             tally_vote(!pass && raw.result == BNK_WG_OK ? (uint32_t)BNK_WG_FILTERED : raw.result, t < a.n, lane, n_result);
         if (a.tally) {
             const unsigned long long in = __ballot(t < a.n), ok = __ballot(t < a.n && pass != 0);
             n_pass += (uint32_t)__popcll(ok);
             n_drop += (uint32_t)__popcll(in & ~ok);
         }
-        raw = fetch_header(a, t + stride);
+        raw = fetch_header<FROM>(a, t + stride);
     }
     if (a.tally && lane == 0u) {
         tally_bump(a.tally, TALLY_ALLOWED, n_pass);
         tally_bump(a.tally, TALLY_DENIED, n_drop);
     }
-    if (a.wg_tally && lane < 16u && n_result != 0u && decap_slot(lane) != TALLY_NONE) {
+    if (FROM == FROM_ARRAYS && a.wg_tally && lane < 16u && n_result != 0u && decap_slot(lane) != TALLY_NONE) {
         tally_bump(a.wg_tally, decap_slot(lane), n_result);
         // CheckInbound behind a decapsulating call saw exactly what was delivered
         if (lane == BNK_WG_OK) tally_bump(a.wg_tally, TALLY_ALLOWED, n_result);
@@ -501,8 +556,12 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
 // in a tunnel's slots, 16,384 flows, 11.9 and 32.1.
 __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
 {
-    const uint32_t stride = gridDim.x * 256u;
-    if (blockIdx.x == 0u && threadIdx.x == 0u) {
+    const uint32_t stride = (gridDim.x - 1u) * 256u;
+    // The launch's first workgroup has no packets: its few dependent reads, an atomic and a store
+    // to the host would otherwise be one wave's way to its first packet, and the whole launch waits
+    // for the slowest wave.
+    if (blockIdx.x == 0u) {
+        if (threadIdx.x != 0u) return;
         // What the last sweep left behind is folded in here, so that the next one can read the
         // entry count and the bound without anybody changing them meanwhile.
         uint32_t *c = a.flows.counters;
@@ -520,8 +579,9 @@ __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
         if (a.record)
             __hip_atomic_store(a.record, (uint64_t)(a.record_seq - 1u) << 32 | atomicAdd(&c[FLOW_CLAIMED], 0u),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
     }
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < a.n; i += stride) {
+    for (uint32_t i = (blockIdx.x - 1u) * 256u + threadIdx.x; i < a.n; i += stride) {
         const uint64_t at = a.off ? a.off[i] : (uint64_t)i * a.stride;
         const uint32_t len = a.lens ? a.lens[i] : a.len;
         if (beyond_arena(at, a.ahead, len, a.limit)) {
@@ -712,10 +772,15 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
     // the small bitmap rides along while two workgroups still fit a CU's 160 KiB
     a.small_in_lds = lds + SMALL_BITS / 8u <= 80u * 1024u ? 1u : 0u;
     if (a.small_in_lds) lds += SMALL_BITS / 8u;
+    const bool jumps = a.rules.n_bounds <= LDS_BOUNDS_MAX && a.rules.jump != nullptr;
+    const bool arrays = a.gate || a.lens || a.off || a.wg_result || a.limit != 0;
+    void (*const kernels[3][2])(FilterArgs) = {{filter_check_kernel<FROM_PLAIN, false>, filter_check_kernel<FROM_PLAIN, true>},
+                                               {filter_check_kernel<FROM_ARRAYS, false>, filter_check_kernel<FROM_ARRAYS, true>},
+                                               {filter_check_kernel<FROM_RECORDS, false>, filter_check_kernel<FROM_RECORDS, true>}};
+    void (*const kernel)(FilterArgs) = kernels[a.heads ? FROM_RECORDS : arrays ? FROM_ARRAYS : FROM_PLAIN][jumps];
     if (lds > 48u * 1024u) {
         // more dynamic LDS than the default limit: opt in (gfx950 has 160 KiB per CU)
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(filter_check_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(LDS_BOUNDS_MAX * 4u + LDS_JUMP_ROOM * 4u));
         if (e != hipSuccess) return e;
     }
@@ -724,14 +789,14 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
     uint32_t blocks = (a.n + FILTER_THREADS - 1u) / FILTER_THREADS;
     const uint32_t cap = (max_blocks / 8u) * per_cu; // max_blocks is 8 per CU
     if (blocks > cap) blocks = cap;
-    hipLaunchKernelGGL(filter_check_kernel, dim3(blocks), dim3(FILTER_THREADS), lds, s, a);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(FILTER_THREADS), lds, s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(filter_note_kernel, dim3(grid_for(a.n, max_blocks)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(filter_note_kernel, dim3(grid_for(a.n, max_blocks) + 1u), dim3(256), 0, s, a);
     if (a.record && a.record_after)
         hipLaunchKernelGGL(note_record_kernel, dim3(1), dim3(1), 0, s, a.record, a.record_seq, a.flows.counters);
     // filter.go:202: no sweep while the map holds at most 4096 entries

@@ -385,3 +385,75 @@ def test_a_refused_note_batch_leaves_nothing_to_wait_for():
         assert min(took) < 0.010, took
     assert ctx.filter_flow_count() == 900
     ctx.close()
+
+
+@pytest.mark.parametrize("rules", ["few", "long", "many"])
+@pytest.mark.parametrize("n", [1, 63, 65, 1025, 5000])
+def test_every_form_of_a_device_batch(rules, n):
+    """CheckInbound on plain records of one length and stride, and on per-packet offsets and
+    lengths: headers with options, without ports, of other protocols and versions, cut off
+    anywhere, against rules whose lists fit a block, do not, and whose cut points fill more than
+    LDS holds; replies to noted flows among them."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n * 7 + len(rules))
+    base = W.CGNAT_BASE
+    if rules == "few":
+        table = [([(base | i << 8, 24)], "tcp" if i % 3 else "udp", [(20 * i, 20 * i + 30)]) for i in range(60)]
+    elif rules == "long":
+        table = [([(base, 16)], "tcp", [(3 * i, 3 * i + 1) for i in range(9, 49)]),
+                 ([(base | 0x700, 24)], "udp", [(50 * i, 50 * i + 20) for i in range(20)]), ([(base, 12)], "icmp", [])]
+    else:
+        table = [([(base | 2 * i, 32)], "tcp" if i & 1 else "udp", [(i % 900, i % 900 + 400)]) for i in range(13000)]
+    ctx, ora = lib.Context(0), O.Filter()
+    ctx.filter_set_rules(table)
+    ora.set_rules(table)
+    proto = rng.choice([6, 6, 17, 1, 2], n).astype(np.uint8)
+    src = (base | rng.integers(0, 1 << 15, n)).astype(np.uint32)
+    src[::9] = rng.integers(0, 1 << 32, n, dtype=np.uint64)[::9].astype(np.uint32)
+    me = np.full(n, base | 1, np.uint32)
+    sport, dport = (rng.integers(0, 1400, n).astype(np.uint32) for _ in range(2))
+    rec = W.header_records(proto, src, me, sport, dport)[:, :28]
+    # every fourth packet answers a flow
+    k = np.arange(0, n, 4)
+    out = np.ascontiguousarray(W.header_records(proto[k], me[k], src[k], dport[k], sport[k])[:, :28])
+    offs = np.arange(k.size, dtype=np.uint64) * 28
+    ora.note_outbound_batch(out.reshape(-1), offs, np.full(k.size, 28, np.uint32), FC.T0)
+    d_out = torch.from_numpy(out).to("cuda:0")
+    torch.cuda.synchronize()
+    ctx.filter_note_outbound(lib.make_batch(d_out, out.nbytes, k.size, lib.MEM_DEVICE, stride=28, length=28), FC.T0)
+    # some are not what they seem: other versions, options
+    rec = rec.copy()
+    rec[::13, 0] = rng.choice([0x65, 0x44, 0x4F, 0x46], rec[::13].shape[0])
+
+    def compare(arena, at, sizes, now, **layout):
+        want = ora.check_inbound_batch(arena, at, sizes, now)
+        d = torch.from_numpy(np.concatenate([arena, np.zeros(16, np.uint8)])).to("cuda:0")
+        arrays = {a: torch.from_numpy(v).to("cuda:0") for a, v in layout.items() if isinstance(v, np.ndarray)}
+        got = torch.full((n,), 9, dtype=torch.uint8, device="cuda:0")
+        torch.cuda.synchronize()
+        ctx.filter_check_inbound(lib.make_batch(d, arena.nbytes, n, lib.MEM_DEVICE, **{**layout, **arrays}), now, got)
+        ctx.sync()
+        assert np.array_equal(got.cpu().numpy(), want)
+        return want
+
+    passed = []
+    for j, (stride, length) in enumerate([(28, 28), (41, 28), (64, 24), (28, 23), (64, 64)]):
+        arena = np.zeros(n * stride, np.uint8)
+        arena.reshape(n, stride)[:, :min(stride, 28)] = rec[:, :min(stride, 28)]
+        full = np.full(n, length, np.uint32)
+        passed.append(compare(arena, np.arange(n, dtype=np.uint64) * stride, full, FC.T0 + j + 1, stride=stride, length=length))
+    lens = rng.integers(0, 70, n).astype(np.uint32)
+    lens[::3] = 28
+    ends = np.cumsum(lens + rng.integers(0, 5, n)).astype(np.int64)
+    off = (ends - lens).astype(np.uint64)
+    arena = rng.integers(0, 256, int(ends[-1]) + 1, dtype=np.uint8)
+    for i in range(n):
+        m = min(int(lens[i]), 28)
+        arena[int(off[i]):int(off[i]) + m] = rec[i, :m]
+    passed.append(compare(arena, off, lens, FC.T0 + 9, offsets=off.astype(np.int64), lens=lens.astype(np.int32)))
+    if n >= 1000:
+        assert 0.05 < np.concatenate(passed).mean() < 0.95
+    assert ctx.filter_flows() == ora.flows()
+    ctx.close()

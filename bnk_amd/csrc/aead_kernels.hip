@@ -66,6 +66,13 @@ BNK_DEV void st16a_out(uint8_t *p, uint4 v)
 
 BNK_DEV uint8_t ld8(const uint8_t *p) { return *reinterpret_cast<const BNK_GLOBAL uint8_t *>((uintptr_t)p); }
 BNK_DEV void st8(uint8_t *p, uint8_t v) { *reinterpret_cast<BNK_GLOBAL uint8_t *>((uintptr_t)p) = v; }
+BNK_DEV void st8a(uint8_t *p, uint2 v)
+{
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 t = {v.x, v.y};
+    *reinterpret_cast<BNK_GLOBAL u32x2 *>((uintptr_t)p) = t;
+}
+BNK_DEV void st2a(uint8_t *p, uint16_t v) { *reinterpret_cast<BNK_GLOBAL uint16_t *>((uintptr_t)p) = v; }
 BNK_DEV void st4a(uint8_t *p, uint32_t v) { *reinterpret_cast<BNK_GLOBAL uint32_t *>((uintptr_t)p) = v; }
 
 typedef uint32_t __attribute__((aligned(1))) u32_unaligned;
@@ -191,18 +198,9 @@ constexpr uint32_t WAVES_PER_BLOCK = 4;
 #define LANE_KERNEL_WAVES 1
 constexpr uint32_t LANE_BLOCK = 64u * LANE_KERNEL_WAVES;
 // Short path: a wave whose packets all have at most SHORT_BLOCKS data blocks
-// (128 plaintext bytes: at most eight cells, in at most two lines) brings each
-// packet in whole, computes it in one go and writes it back, with rows that
-// hold the packet's cells from its first one.  Straight-line code, every load
-// of the wave in flight at once: 2^20 x 60 bytes seal in 101 us against 113 us
-// through the ring.  (Running such waves three to a SIMD on smaller rows was
-// tried too: the 168 registers that allows cost the long packets 15 % and the
-// short ones gained nothing.)
+// (128 plaintext bytes) brings each packet in whole, computes it in one go and
+// writes it back.  Straight-line code, every load of the wave in flight at once.
 constexpr uint32_t SHORT_BLOCKS = 2;
-constexpr uint32_t SHORT_ROW = 144;          // 8 cells + 16 pad
-#ifndef SHORT_WAVES_PER_SIMD
-#define SHORT_WAVES_PER_SIMD 3
-#endif
 
 // v: the cell's 16 bytes, read from `cell` beforehand (before the keystream block was
 // computed, so that the LDS read is not waited for)
@@ -509,7 +507,13 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         if ((m) >= m_lo && (m) < m_hi) BNK_EIGHT(OP##_ALL, m);                              \
         else BNK_EIGHT(OP, m);                                                              \
     } while (0)
-#define BNK_ISSUE_LINE(m) BNK_LINE(BNK_ISSUE, m)
+// (the empty asm ends one of the two forms differently from the other: the compiler would
+// otherwise make one load of the last of both, behind their join and a wait for the other seven)
+#define BNK_ISSUE_LINE(m)                                                                   \
+    do {                                                                                    \
+        if ((m) >= m_lo && (m) < m_hi) { BNK_EIGHT(BNK_ISSUE_ALL, m); asm volatile(""); }   \
+        else BNK_EIGHT(BNK_ISSUE, m);                                                       \
+    } while (0)
 #define BNK_COMMIT_LINE(m) BNK_LINE(BNK_COMMIT, m)
     uint4 out0 = pre0, out1 = pre0, out2 = pre0, out3 = pre0, out4 = pre0, out5 = pre0, out6 = pre0, out7 = pre0;
 
@@ -711,45 +715,55 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
 #undef BNK_COMMIT_LINE
 }
 
-// Short path (see SHORT_BLOCKS): cell j of a packet lives at row + 16 j.  Same
-// cooperative movement as body_lines: eight adjacent lanes per aligned
-// 128-byte line, only cells of the packet read into LDS or written back.
-// LEAN (the launch that holds more such waves per SIMD): where each cell goes is
-// worked out again after the cipher instead of being kept in registers across it.
-template <bool OPEN, bool LEAN = false>
-BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_t *dst, uint32_t len,
+// A lane's row on the short path: a packet's cells and 16 bytes more.
+template <int CELLS>
+constexpr uint32_t short_row() { return 16u * CELLS + 16u; }
+
+// Short path (see SHORT_BLOCKS), every packet of the wave 16-byte aligned in source and
+// destination and at most 16 * CELLS bytes long: CELLS adjacent lanes per packet move its cells,
+// whatever lines they lie in (the packets of a batch of such packets lie side by side, so what a
+// load leaves of a line the next lanes' or the next load's packets take), and cell j of a packet
+// lives at row + 16 j of its lane's row, the second half of the one-time key behind the cells.
+// Where each cell goes is worked out again after the cipher instead of being kept in registers
+// across it.
+//
+// What bounds such a wave is vector issue (two ChaCha20 blocks and five cells of Poly1305 for a
+// packet of 60 bytes), next to it the number of its memory instructions.  Eight lanes per 128-byte
+// line, two lines per packet that might reach into a second, took twice the loads and stores and
+// more registers, and asked for source and destination at the same place of a line; pairs of
+// launches of 2^20 packets, us before and now:
+//   60 bytes in slots of 80 / 96 / 1536      153 / 159 / 164      123 / 129 / 139
+//   60 from slots of 96 to slots of 112      228 (no short path)  127
+//   100 in 128, 124 in 144 / 2048            187, 213 / 251       179, 185 / 238
+//   1 to 60, 1 to 128 bytes (two to a SIMD)  217, 266             186, 230
+//
+// Sealing, the tag is put behind the packet's bytes in its row and leaves with them: what an
+// owner stores for itself are the last 1 to 15 bytes of the two together (a tag and a
+// packet's last bytes by their owner are four scattered stores at 60 bytes).  `have`: the lane has
+// a packet, be it an empty one.
+template <bool OPEN, int CELLS>
+BNK_DEV void body_short(uint8_t *tile, uint32_t lane, bool have, const uint8_t *src, uint8_t *dst, uint32_t len,
                         uint32_t len_in, const uint8_t *safe, const uint32_t (&k)[8], uint32_t n1, uint32_t n2,
                         Poly32 &mac, uint32_t (&x)[16], Head &head)
 {
+    static_assert(CELLS == 4 || CELLS == 8, "one data block or two");
+    constexpr uint32_t ROW = short_row<CELLS>();
+    constexpr int PER = 64 / CELLS; // packets per load
     const uint32_t ncell_in = len_in >> 4; // see body_lines
-    const uint32_t skew = (uint32_t)(uintptr_t)src & 127u;
-    const uint32_t c0 = skew >> 4;
-    const uint32_t ncell = len >> 4;           // whole cells, stored cooperatively
-    const uint32_t sub = lane & 7u;
-    // does any packet of the wave reach into a second line?
-    const bool two = __ballot(c0 + ((len + 15u) >> 4) > 8u) != 0ull;
-    uint8_t *rows = tile + (lane >> 3) * SHORT_ROW;
-    uint4 pre[2][8];
-    uint32_t jcell[8], nst[8], nld[8]; // my cell's index in the owner's packet for line 0; its cell counts
-    const uint8_t *csrc[8];
-    uint8_t *cdst[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const int owner = 8 * q + (int)(lane >> 3);
-        csrc[q] = reinterpret_cast<const uint8_t *>(shfl64((uint64_t)(uintptr_t)(src - skew), owner)) + 16u * sub;
-        cdst[q] = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)(dst - skew), owner)) + 16u * sub;
-        const uint32_t olen = (uint32_t)__shfl((int)len, owner, 64);
-        jcell[q] = sub - (uint32_t)__shfl((int)c0, owner, 64); // wraps below zero for cells before the packet
-        nst[q] = olen >> 4;
-        nld[q] = (olen + 15u) >> 4;
-    }
+    const uint32_t ncell = len >> 4;       // whole cells, stored cooperatively
+    const uint32_t sub = lane % CELLS;
+    uint8_t *const move = tile + (lane / CELLS) * ROW + 16u * sub; // my cell of load 0's packet
+    uint4 pre[CELLS];
+    uint32_t mine = 0; // bit q: my cell is the packet's
     // unconditional loads, from a harmless address when the cell is not the
     // packet's (a load under a branch is waited for where the branch closes)
 #pragma unroll
-    for (int q = 0; q < 8; q++) pre[0][q] = ld16a(jcell[q] < nld[q] ? csrc[q] : safe);
-    if (two) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) pre[1][q] = ld16a(jcell[q] + 8u < nld[q] ? csrc[q] + 128u : safe);
+    for (int q = 0; q < CELLS; q++) {
+        const int owner = PER * q + (int)(lane / CELLS);
+        const uint8_t *at = reinterpret_cast<const uint8_t *>(shfl64((uint64_t)(uintptr_t)src, owner)) + 16u * sub;
+        const bool in = 16u * sub < (uint32_t)__shfl((int)len, owner, 64);
+        mine |= in ? 1u << q : 0u;
+        pre[q] = ld16a(in ? at : safe);
     }
     // keystream blocks 0 (the Poly1305 key) and 1 side by side while the loads fly
     uint32_t y[16];
@@ -759,49 +773,37 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         chacha_block2_shared(k, shared, 0, n1, n2, x, y);
     }
     mac.init(x);
-    // (the second half of the one-time key waits behind the lane's cells: four registers)
-    if (LEAN) *reinterpret_cast<uint4 *>(tile + lane * SHORT_ROW + 128u) = make_uint4(x[4], x[5], x[6], x[7]);
+    uint8_t *row = tile + lane * ROW;
+    *reinterpret_cast<uint4 *>(row + 16 * CELLS) = make_uint4(x[4], x[5], x[6], x[7]);
 #pragma unroll
-    for (int q = 0; q < 8; q++)
-        if (jcell[q] < nld[q]) *reinterpret_cast<uint4 *>(rows + 8u * q * SHORT_ROW + (jcell[q] << 4)) = pre[0][q];
-    if (two) {
-#pragma unroll
-        for (int q = 0; q < 8; q++)
-            if (jcell[q] + 8u < nld[q])
-                *reinterpret_cast<uint4 *>(rows + 8u * q * SHORT_ROW + ((jcell[q] + 8u) << 4)) = pre[1][q];
-    }
+    for (int q = 0; q < CELLS; q++)
+        if ((mine >> q) & 1u) *reinterpret_cast<uint4 *>(move + PER * q * ROW) = pre[q];
     wave_sync();
-    uint8_t *row = tile + lane * SHORT_ROW;
     // block b's four cells with keystream ks
     auto crypt_block = [&](uint32_t b, const uint32_t (&ks)[16], const uint4 (&v)[4]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const uint32_t kc = 4u * b + j;
-            if (LEAN && kc == 0u) {
-                // (the packet's first cell: the MAC has nothing to multiply yet)
-                uint4 c = v[0];
-                if (len_in < 16u) c = keep_bytes(c, len_in);
-                uint4 o = make_uint4(c.x ^ ks[0], c.y ^ ks[1], c.z ^ ks[2], c.w ^ ks[3]);
-                if (len < 16u) o = keep_bytes(o, len);
-                mac.start(OPEN ? c.x : o.x, OPEN ? c.y : o.y, OPEN ? c.z : o.z, OPEN ? c.w : o.w);
-                if (len < 16u) st_partial(dst, o, len);
-                *reinterpret_cast<uint4 *>(row) = o;
-            } else if (kc < ncell_in) crypt_cell_v<OPEN>(mac, ks, j, v[j], row + (kc << 4));
-            else if (kc < ncell || (kc == ncell && (len & 15u))) {
-                const uint32_t m_out = kc < ncell ? 16u : len & 15u;
-                const uint32_t m_in = len_in > 16u * kc ? min(len_in - 16u * kc, m_out) : 0u;
-                crypt_tail_lds<OPEN>(mac, ks, j, row + (kc << 4), dst + 16u * kc, m_in, m_out);
-            }
+            const uint32_t m_out = min(len > 16u * kc ? len - 16u * kc : 0u, 16u);
+            const uint32_t m_in = min(len_in > 16u * kc ? len_in - 16u * kc : 0u, m_out);
+            if (m_out == 0u) continue;
+            uint4 c = v[j];
+            if (m_in < 16u) c = keep_bytes(c, m_in); // (what follows its bytes in memory has come along)
+            uint4 o = make_uint4(c.x ^ ks[4 * j], c.y ^ ks[4 * j + 1], c.z ^ ks[4 * j + 2], c.w ^ ks[4 * j + 3]);
+            if (m_out < 16u) o = keep_bytes(o, m_out);
+            // (with the packet's first cell the MAC has nothing to multiply yet)
+            if (kc == 0u) mac.start(OPEN ? c.x : o.x, OPEN ? c.y : o.y, OPEN ? c.z : o.z, OPEN ? c.w : o.w);
+            else mac.block(OPEN ? c.x : o.x, OPEN ? c.y : o.y, OPEN ? c.z : o.z, OPEN ? c.w : o.w);
+            *reinterpret_cast<uint4 *>(row + (kc << 4)) = o;
         }
     };
-    static_assert(SHORT_BLOCKS == 2, "the short path is written out for two data blocks");
     uint4 v[4];
     if (len != 0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const uint4 *>(row + (j << 4));
         crypt_block(0, y, v);
     }
-    if (len > 64u) {
+    if (CELLS > 4 && len > 64u) {
         // the second block's cells leave LDS while its keystream is computed
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const uint4 *>(row + ((4 + j) << 4));
@@ -809,41 +811,54 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
         crypt_block(1, x, v);
     }
     if (OPEN) capture_head(head, row, row + 16);
-    if (LEAN) {
-        const uint4 pad = *reinterpret_cast<const uint4 *>(row + 128);
-        mac.pad0 = pad.x; mac.pad1 = pad.y; mac.pad2 = pad.z; mac.pad3 = pad.w;
+    const uint4 pad = *reinterpret_cast<const uint4 *>(row + 16 * CELLS);
+    mac.pad0 = pad.x; mac.pad1 = pad.y; mac.pad2 = pad.z; mac.pad3 = pad.w;
+    const uint32_t out = OPEN ? len : have ? len + 16u : 0u;
+    if (!OPEN && have) {
+        uint32_t tag[4];
+        mac.block(0, 0, len, 0); // LE64(len(aad) = 0) || LE64(len(ciphertext))
+        mac.finish(tag);
+        uint8_t *const at = row + len;
+        if ((len & 3u) == 0u) {
+#pragma unroll
+            for (int w = 0; w < 4; w++) reinterpret_cast<uint32_t *>(at)[w] = tag[w];
+        } else {
+#pragma unroll
+            for (int w = 0; w < 16; w++) at[w] = (uint8_t)(tag[w >> 2] >> (8 * (w & 3)));
+        }
     }
     wave_sync();
-    if (LEAN) {
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const int owner = 8 * q + (int)(lane >> 3);
-            uint8_t *to = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)(dst - skew), owner)) + 16u * sub;
-            const uint32_t jc = sub - (uint32_t)__shfl((int)c0, owner, 64);
-            const uint32_t ns = (uint32_t)__shfl((int)len, owner, 64) >> 4;
-            const uint4 v0 = *reinterpret_cast<const uint4 *>(rows + 8u * q * SHORT_ROW + ((jc < 8u ? jc : 0u) << 4));
-            if (jc < ns) st16a(to, v0);
-            if (two) {
-                const uint32_t j1 = jc + 8u;
-                const uint4 v1 = *reinterpret_cast<const uint4 *>(rows + 8u * q * SHORT_ROW + ((j1 < 8u ? j1 : 0u) << 4));
-                if (j1 < ns) st16a(to + 128u, v1);
-            }
-        }
-        return;
+    for (int q = 0; q < CELLS; q++) {
+        const int owner = PER * q + (int)(lane / CELLS);
+        uint8_t *to = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)dst, owner)) + 16u * sub;
+        const uint32_t whole = (uint32_t)__shfl((int)out, owner, 64) >> 4;
+        const uint4 v0 = *reinterpret_cast<const uint4 *>(move + PER * q * ROW);
+        if (sub < whole) st16a(to, v0);
     }
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        // read first, unconditionally (from cell 0 when mine is not the packet's)
-        const uint4 v = *reinterpret_cast<const uint4 *>(rows + 8u * q * SHORT_ROW + ((jcell[q] < 8u ? jcell[q] : 0u) << 4));
-        if (jcell[q] < nst[q]) st16a(cdst[q], v);
-    }
-    if (two) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const uint32_t j1 = jcell[q] + 8u;
-            const uint4 v = *reinterpret_cast<const uint4 *>(rows + 8u * q * SHORT_ROW + ((j1 < 8u ? j1 : 0u) << 4));
-            if (j1 < nst[q]) st16a(cdst[q] + 128u, v);
+    const uint32_t end = out & ~15u;
+    if (end > 16u * CELLS) st16a(dst + 16 * CELLS, *reinterpret_cast<const uint4 *>(row + 16 * CELLS));
+    if (out != end) {
+        // eight, four, two bytes and one, as many as there are
+        const uint4 v0 = *reinterpret_cast<const uint4 *>(row + end);
+        uint8_t *to = dst + end;
+        uint32_t w = v0.x;
+        if (out & 8u) {
+            st8a(to, make_uint2(v0.x, v0.y));
+            to += 8;
+            w = v0.z;
         }
+        if (out & 4u) {
+            st4a(to, w);
+            to += 4;
+            w = out & 8u ? v0.w : v0.y;
+        }
+        if (out & 2u) {
+            st2a(to, (uint16_t)w);
+            to += 2;
+            w >>= 16;
+        }
+        if (out & 1u) st8(to, (uint8_t)w);
     }
 }
 
@@ -893,7 +908,7 @@ BNK_DEV void decap_result(const AeadArgs &a, uint32_t i, bool have, bool reject,
 template <bool OPEN>
 BNK_DEV bool lane_finish(const AeadArgs &a, uint32_t lane, bool have, uint32_t i, uint32_t len,
                          const uint8_t *src, uint8_t *dst, Poly32 &mac, const Head &head, uint8_t *record,
-                         bool decap = false, uint32_t pr = 0)
+                         bool decap = false, uint32_t pr = 0, const uint4 *tag_here = nullptr)
 {
     bool reject = false;
     if (have) {
@@ -904,7 +919,7 @@ BNK_DEV bool lane_finish(const AeadArgs &a, uint32_t lane, bool have, uint32_t i
         if (!OPEN) {
             st16(dst + len, make_uint4(tag[0], tag[1], tag[2], tag[3]));
         } else {
-            const uint4 tg = ld16(src + len);
+            const uint4 tg = tag_here ? *tag_here : ld16(src + len);
             // all 16 bytes are compared, no early exit
             const uint32_t diff = (tg.x ^ tag[0]) | (tg.y ^ tag[1]) | (tg.z ^ tag[2]) |
                                   (tg.w ^ tag[3]);
@@ -1083,9 +1098,9 @@ BNK_DEV void lane_packet_report(const AeadArgs &a, const LanePacket &p)
     }
 }
 
-// A lane per packet.  SHORT_ONLY: the launch for batches in which every wave
-// takes the short path (see aead_short_kernel).
-template <bool OPEN, bool SHORT_ONLY>
+// A lane per packet.  SHORT_CELLS: of the launch for batches in which every wave takes the
+// short path (see aead_short_kernel), 0 otherwise.
+template <bool OPEN, int SHORT_CELLS>
 BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile, uint2 *aside)
 {
     const uint32_t lane = threadIdx.x & 63u;
@@ -1095,7 +1110,9 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile, uint2 *aside)
                             (((uintptr_t)p.src ^ (uintptr_t)p.dst) & 127u) == 0;
     // which launch does this wave's packets: nothing has been written so far
     const bool all_lines = __ballot(!lane_lines) == 0ull;
-    const bool all_short = all_lines && __ballot(p.len > 64u * SHORT_BLOCKS) == 0ull;
+    constexpr bool SHORT_ONLY = SHORT_CELLS != 0;
+    const bool aligned = (((uintptr_t)p.src | (uintptr_t)p.dst) & 15u) == 0;
+    const bool all_short = __ballot(!aligned || p.len > (SHORT_ONLY ? 16u * SHORT_CELLS : 128u)) == 0ull;
     if (SHORT_ONLY && !all_short) {
         // (the host launches this kernel only where no wave can come here)
         status_raise(a.status, STATUS_INTERNAL);
@@ -1115,8 +1132,10 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile, uint2 *aside)
     head.c0 = head.c1 = make_uint4(0, 0, 0, 0);
     // (which packet it is and whose comes up again only at the end)
     if (OPEN && !SHORT_ONLY) aside[lane] = make_uint2(p.i, p.pr);
-    if (SHORT_ONLY) body_short<OPEN, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
-    else if (all_short) body_short<OPEN>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
+    // (a launch with registers to spare has the tags come with the cells)
+    uint4 tag_here = make_uint4(0, 0, 0, 0);
+    if (OPEN && SHORT_ONLY) tag_here = ld16(p.have ? p.src + p.len : safe);
+    if (all_short) body_short<OPEN, SHORT_ONLY ? SHORT_CELLS : 8>(tile, lane, p.have, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
     else if (!all_lines) {
         if (__ballot(((uintptr_t)p.dst & 3u) != 0) == 0ull)
             body_lines<OPEN, false, true>(tile, lane, p.src, p.dst, p.len, p.len_in, safe, k, n1, n2, mac, x, head);
@@ -1129,9 +1148,12 @@ BNK_DEV void wave_main(const AeadArgs &a, uint8_t *tile, uint2 *aside)
         p.i = aside[lane].x;
         p.pr = aside[lane].y;
     }
-    const bool reject = lane_finish<OPEN>(a, lane, p.have, p.i, p.len, p.src, p.dst, mac, head,
-                                          p.in_batch && a.heads ? a.heads + 32ull * t : nullptr,
-                                          decap && p.in_batch && p.wg_res == BNK_WG_OK, p.pr);
+    bool reject = false;
+    if (OPEN || !all_short)
+        reject = lane_finish<OPEN>(a, lane, p.have, p.i, p.len, p.src, p.dst, mac, head,
+                                   p.in_batch && a.heads ? a.heads + 32ull * t : nullptr,
+                                   decap && p.in_batch && p.wg_res == BNK_WG_OK, p.pr,
+                                   SHORT_ONLY ? &tag_here : nullptr);
     if (!OPEN && a.tally) {
         // an encapsulating launch counting what it sends
         const unsigned long long sent = __ballot(p.have);
@@ -1153,23 +1175,24 @@ __global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2
 {
     __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * RING_ROW];
     __shared__ uint2 aside[OPEN ? LANE_KERNEL_WAVES : 1][OPEN ? 64 : 1];
-    static_assert(RING_ROW >= LDS_ROW && RING_ROW >= SHORT_ROW, "the other paths reuse the tile");
-    wave_main<OPEN, false>(a, tile_all[threadIdx.x >> 6], aside[OPEN ? threadIdx.x >> 6 : 0]);
+    static_assert(RING_ROW >= LDS_ROW && RING_ROW >= short_row<8>(), "the other paths reuse the tile");
+    wave_main<OPEN, 0>(a, tile_all[threadIdx.x >> 6], aside[OPEN ? threadIdx.x >> 6 : 0]);
 }
 
 // Batches in which the host can tell that every wave takes the short path
-// (every_wave_short): without the ring and the line paths' registers three such
-// waves fit a SIMD where the launch above holds two, worth 8-11 % at 60 bytes
-// (2^20 packets seal in 83 us against 93).  Handing the short waves of a mixed
-// batch to this kernel in a second launch was measured too and loses: every wave
-// of both launches walks its metadata before it knows whose it is (IMIX 9 %
+// (every_wave_short): without the ring and the line paths' registers, and with no more of a
+// tile than the packets fill, five (up to 64 bytes) or four such waves fit a SIMD where the launch above holds two.
+// Handing the short waves of a mixed batch to this kernel in a second launch was measured too and
+// loses: every wave of both launches walks its metadata before it knows whose it is (IMIX 9 %
 // slower, the relay 3.5 %).
-template <bool OPEN>
-__global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHORT_WAVES_PER_SIMD, SHORT_WAVES_PER_SIMD)))
+template <int CELLS>
+constexpr int SHORT_WAVES = CELLS == 4 ? 5 : 4;
+template <bool OPEN, int CELLS>
+__global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(SHORT_WAVES<CELLS>, SHORT_WAVES<CELLS>)))
 void aead_short_kernel(AeadArgs a)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * SHORT_ROW];
-    wave_main<OPEN, true>(a, tile_all[threadIdx.x >> 6], nullptr);
+    __shared__ __attribute__((aligned(16))) uint8_t tile_all[LANE_KERNEL_WAVES][64 * short_row<CELLS>()];
+    wave_main<OPEN, CELLS>(a, tile_all[threadIdx.x >> 6], nullptr);
 }
 
 // A few lanes per packet, for batches between the two: too few packets to fill
@@ -1758,11 +1781,11 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
 
 // Can the host tell that every wave of the launch takes the short path?  One
 // common length of at most SHORT_BLOCKS blocks once trimmed, framed and padded,
-// uniform strides, and every packet 16-byte aligned at the same place of a
-// 128-byte line in both arenas.
-static bool every_wave_short(const AeadArgs &a, bool open)
+// uniform strides, and every packet 16-byte aligned in both arenas.  The cells
+// a packet then has at most, 4 or 8; 0: it cannot.
+static int every_wave_short(const AeadArgs &a, bool open)
 {
-    if (a.lens || a.order || a.in_off || a.out_off) return false;
+    if (a.lens || a.order || a.in_off || a.out_off) return 0;
     uint64_t len = a.len;
     if (open) {
         if (a.wg.mode == WG_FUSE_DECAP) len = len >= 16u ? len - 16u : 0u; // the header
@@ -1771,10 +1794,10 @@ static bool every_wave_short(const AeadArgs &a, bool open)
         len = len >= a.trim ? len - a.trim : 0u;
         if (a.wg.mode == WG_FUSE_ENCAP) len += 15u; // at most this much padding
     }
-    if (len > 64u * SHORT_BLOCKS) return false;
+    if (len > 64u * SHORT_BLOCKS) return 0;
     const uint64_t src0 = (uint64_t)(uintptr_t)a.in + a.in_skip, dst0 = (uint64_t)(uintptr_t)a.out + a.out_skip;
-    if (((src0 | dst0 | a.in_stride | a.out_stride) & 15u) != 0) return false;
-    return ((src0 ^ dst0) & 127u) == 0 && ((a.in_stride ^ a.out_stride) & 127u) == 0;
+    if (((src0 | dst0 | a.in_stride | a.out_stride) & 15u) != 0) return 0;
+    return len <= 64u ? 4 : 8;
 }
 
 template <bool OPEN>
@@ -1784,10 +1807,13 @@ static hipError_t launch_wave(const AeadArgs &args, hipStream_t s)
     a.split = aead_split_packets(a);
     if (a.split)
         hipLaunchKernelGGL(aead_split_kernel<OPEN>, dim3((a.n + a.split - 1u) / a.split), dim3(64), 0, s, a);
-    else if (every_wave_short(a, OPEN))
-        hipLaunchKernelGGL(aead_short_kernel<OPEN>, dim3((a.n + LANE_BLOCK - 1u) / LANE_BLOCK), dim3(LANE_BLOCK), 0, s, a);
-    else
-        hipLaunchKernelGGL(aead_wave_kernel<OPEN>, dim3((a.n + LANE_BLOCK - 1u) / LANE_BLOCK), dim3(LANE_BLOCK), 0, s, a);
+    else {
+        const dim3 grid((a.n + LANE_BLOCK - 1u) / LANE_BLOCK);
+        const int cells = every_wave_short(a, OPEN);
+        if (cells == 4) hipLaunchKernelGGL((aead_short_kernel<OPEN, 4>), grid, dim3(LANE_BLOCK), 0, s, a);
+        else if (cells == 8) hipLaunchKernelGGL((aead_short_kernel<OPEN, 8>), grid, dim3(LANE_BLOCK), 0, s, a);
+        else hipLaunchKernelGGL(aead_wave_kernel<OPEN>, grid, dim3(LANE_BLOCK), 0, s, a);
+    }
     return hipGetLastError();
 }
 

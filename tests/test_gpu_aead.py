@@ -696,3 +696,62 @@ def test_uniform_short_device_batches_against_the_oracle(ctx, length, stride, sh
         o = int(off[i])
         expect[o:o + length] = 0 if v[i] == 0 else plain[o:o + length]
     assert np.array_equal(back, expect)
+
+
+@pytest.mark.parametrize("form", ["uniform", "mixed"])
+@pytest.mark.parametrize("longest", [1, 16, 63, 64, 65, 127, 128])
+def test_short_packets_at_different_places_of_a_line(ctx, form, longest):
+    """Short packets that lie 16-byte aligned, but elsewhere in their 128-byte lines in
+    the destination than in the source: of one common length (a launch of their own, up
+    to 64 bytes and up to 128), and of lengths and places of their own (the waves of the
+    common launch).  Every byte of both arenas against the oracle; forged tags among
+    them, and opening in place."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    n = 66000 + 29  # beyond the launches of a wave and of a few lanes per packet; the last wave partly filled
+    rng = np.random.default_rng(2000 + longest)
+    keys = rng.integers(0, 256, (3, 32), dtype=np.uint8)
+    ctx.keys_set(lib.KEYS_SEND, keys)
+    ctx.keys_set(lib.KEYS_RECV, keys)
+    peer = rng.integers(0, 3, n).astype(np.uint32)
+    ctr = rng.integers(0, 1 << 62, n).astype(np.uint64)
+    if form == "uniform":
+        lens = np.full(n, longest, np.uint32)
+        src_off, dst_off = (np.arange(n, dtype=np.uint64) * np.uint64(s) for s in (160, 208))
+    else:
+        lens = rng.integers(0, longest + 1, n).astype(np.uint32)
+        src_off, dst_off = (np.cumsum(144 + 16 * rng.integers(0, 8, n)).astype(np.uint64) for _ in range(2))
+    nb = int(max(src_off[-1], dst_off[-1])) + 256
+    plain = rng.integers(0, 256, nb, dtype=np.uint8)
+    want = np.full(nb, 0xEE, np.uint8)
+    O.seal_batch(keys, peer, ctr, plain, src_off, lens, want, dst_off, 4)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    d_src, d_peer, d_ctr, d_ct = d(plain), d(peer.astype(np.int32)), d(ctr.astype(np.int64)), d(np.full(nb, 0xEE, np.uint8))
+    keep = []
+
+    def batch(t, off, stride, more, **kw):
+        if form == "uniform":
+            return lib.make_batch(t, nb, n, lib.MEM_DEVICE, stride=stride, length=longest + more, **kw)
+        keep.extend([d(off.astype(np.int64)), d((lens + more).astype(np.int32))])
+        torch.cuda.synchronize()
+        return lib.make_batch(t, nb, n, lib.MEM_DEVICE, offsets=keep[-2], lens=keep[-1], **kw)
+
+    torch.cuda.synchronize()
+    ctx.seal(batch(d_src, src_off, 160, 0, peer=d_peer, counters=d_ctr), batch(d_ct, dst_off, 208, 0))
+    ctx.sync()
+    got = d_ct.cpu().numpy()
+    assert np.array_equal(got, want)
+    forged = rng.choice(n, 9, replace=False)
+    got[(dst_off[forged] + lens[forged] + np.uint64(5)).astype(np.int64)] ^= 0x40
+    for to, off, stride in [(d(plain), src_off, 160), (None, dst_off, 208)]:
+        d_from = d(got)
+        to = d_from if to is None else to
+        verdict = torch.full((n,), 7, dtype=torch.uint8, device="cuda:0")
+        before = to.cpu().numpy()
+        torch.cuda.synchronize()
+        ctx.open(batch(d_from, dst_off, 208, 16, peer=d_peer, counters=d_ctr), batch(to, off, stride, 16), verdict)
+        ctx.sync()
+        overdict = O.open_batch(keys, peer, ctr, got, dst_off, lens + np.uint32(16), before, off, 4)
+        assert np.array_equal(verdict.cpu().numpy(), overdict) and int((overdict == 0).sum()) == 9
+        assert np.array_equal(to.cpu().numpy(), before)

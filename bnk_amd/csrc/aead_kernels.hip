@@ -1862,64 +1862,92 @@ BNK_DEV uint32_t len_bin(uint32_t len, uint32_t tag_bytes)
     return nb >= LEN_BINS - 1 ? 0u : (LEN_BINS - 1 - nb);
 }
 
-// Adds one to bins[b] for every participating lane and returns what the
-// lane's own atomicAdd would have returned, with one LDS atomic per distinct
-// bin of the wave instead of one per lane: traffic is a handful of sizes, so
-// most lanes of a wave hit the same bin and would serialise on it.  The
-// leader's values travel through scalar registers (v_readlane), not through
-// LDS.  After eight rounds the remaining lanes (a wave with many distinct
-// sizes) go one by one.
-BNK_DEV uint32_t wave_bin_add(uint32_t *bins, uint32_t b, bool active)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    uint32_t result = 0;
-    bool todo = active;
-    for (int round = 0; round < 8; round++) {
-        const unsigned long long left = __ballot(todo);
-        if (left == 0ull) return result;
-        const int leader = __ffsll((long long)left) - 1;
-        const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)b, leader);
-        const bool mine = todo && b == lb;
-        const unsigned long long same = __ballot(mine);
-        uint32_t old = 0;
-        if ((int)lane == leader) old = atomicAdd(&bins[lb], (uint32_t)__popcll(same));
-        old = (uint32_t)__builtin_amdgcn_readlane((int)old, leader);
-        if (mine) {
-            result = old + (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-            todo = false;
-        }
-    }
-    if (todo) result = atomicAdd(&bins[b], 1u);
-    return result;
-}
-
-// A block of GROUP_THREADS threads takes GROUP_CHUNK consecutive packets, four
-// per thread, loaded together so that their latencies overlap.
+// A block of GROUP_THREADS threads takes ROUNDS times GROUP_CHUNK consecutive packets, each time
+// four consecutive ones per thread, all loaded together.
 constexpr uint32_t GROUP_THREADS = 1024;
 constexpr uint32_t GROUP_PER_THREAD = 4;
 constexpr uint32_t GROUP_CHUNK = GROUP_THREADS * GROUP_PER_THREAD;
+constexpr uint32_t NO_BIN = 0xFFFFFFFFu;
 
+// The bins of packets i to i + 3 (NO_BIN beyond the batch).
+BNK_DEV void len_bins4(const uint32_t *lens, uint32_t i, uint32_t n, uint32_t tag_bytes, uint32_t (&bin)[GROUP_PER_THREAD])
+{
+    typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) u32x4_words;
+    static_assert(GROUP_PER_THREAD == 4, "one load per thread");
+    if (i + 4u <= n) {
+        const u32x4_words v = *reinterpret_cast<const u32x4_words *>(lens + i);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) bin[j] = len_bin(v[j], tag_bytes);
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) bin[j] = i + j < n ? len_bin(lens[i + j], tag_bytes) : NO_BIN;
+    }
+}
+
+// Adds one to bins[b] for each of the lane's bins (NO_BIN: none) and, with RANK, leaves in at[]
+// what each one's own atomicAdd would have returned, the wave's items in their order.  One LDS
+// atomic per distinct bin of the wave's 256 items instead of one per item: traffic is a handful
+// of sizes, so most of them hit the same bin and would serialise on it.  The leader's values
+// travel through scalar registers (v_readlane), not through LDS.  After eight rounds what
+// remains (a wave with many distinct sizes) goes one by one.  (These votes are what the counting
+// launch spends its time on: 0.9 us per item of a thread when each of a thread's four had votes of
+// its own, 2^20 packets of three sizes 8.8 us against 6.4; plain LDS atomics the same 9.0.)
+template <bool RANK>
+BNK_DEV void wave_bins_add(uint32_t *bins, uint32_t (&b)[GROUP_PER_THREAD], uint32_t (&at)[GROUP_PER_THREAD])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    for (int round = 0; round < 8; round++) {
+        const uint32_t next = min(min(b[0], b[1]), min(b[2], b[3]));
+        const unsigned long long left = __ballot(next != NO_BIN);
+        if (left == 0ull) return;
+        const int leader = __ffsll((long long)left) - 1;
+        const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)next, leader);
+        uint32_t c = 0; // how many of mine, 0 to 4
+#pragma unroll
+        for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) c += b[j] == lb ? 1u : 0u;
+        const unsigned long long c0 = __ballot((c & 1u) != 0u), c1 = __ballot((c & 2u) != 0u), c2 = __ballot((c & 4u) != 0u);
+        const uint32_t all = (uint32_t)(__popcll(c0) + 2 * __popcll(c1) + 4 * __popcll(c2));
+        uint32_t old = 0;
+        if ((int)lane == leader) old = atomicAdd(&bins[lb], all);
+        if (RANK) {
+            const unsigned long long below = (1ull << lane) - 1ull;
+            uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)old, leader);
+            r += (uint32_t)(__popcll(c0 & below) + 2 * __popcll(c1 & below) + 4 * __popcll(c2 & below));
+#pragma unroll
+            for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) {
+                at[j] = b[j] == lb ? r : at[j];
+                r += b[j] == lb ? 1u : 0u;
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) b[j] = b[j] == lb ? NO_BIN : b[j];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) {
+        if (b[j] == NO_BIN) continue;
+        const uint32_t old = atomicAdd(&bins[b[j]], 1u);
+        if (RANK) at[j] = old;
+    }
+}
+
+template <uint32_t ROUNDS>
 __global__ __launch_bounds__(GROUP_THREADS) void len_hist_kernel(const uint32_t *lens, uint32_t n,
                                                                  uint32_t tag_bytes, uint32_t *hist,
                                                                  uint32_t *cursor, bool clear_cursor)
 {
     __shared__ uint32_t lh[LEN_BINS];
+    uint32_t bin[ROUNDS][GROUP_PER_THREAD], unused[GROUP_PER_THREAD];
+    const uint32_t first = blockIdx.x * ROUNDS * GROUP_CHUNK + threadIdx.x * GROUP_PER_THREAD;
+#pragma unroll
+    for (uint32_t r = 0; r < ROUNDS; r++) len_bins4(lens, first + r * GROUP_CHUNK, n, tag_bytes, bin[r]);
     for (uint32_t b = threadIdx.x; b < LEN_BINS; b += GROUP_THREADS) lh[b] = 0;
     // a scatter launch that scans for itself counts from zero in cursor[]
     if (clear_cursor && blockIdx.x == 0)
         for (uint32_t b = threadIdx.x; b < LEN_CURSOR_WORDS; b += GROUP_THREADS) cursor[b] = 0;
-    const uint32_t base = blockIdx.x * GROUP_CHUNK + threadIdx.x;
-    uint32_t len[GROUP_PER_THREAD];
-#pragma unroll
-    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) {
-        const uint32_t i = base + j * GROUP_THREADS;
-        len[j] = i < n ? lens[i] : 0u;
-    }
     __syncthreads();
     // whole waves call the helper together (it uses wave-wide votes)
 #pragma unroll
-    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++)
-        (void)wave_bin_add(lh, len_bin(len[j], tag_bytes), base + j * GROUP_THREADS < n);
+    for (uint32_t r = 0; r < ROUNDS; r++) wave_bins_add<false>(lh, bin[r], unused);
     __syncthreads();
     for (uint32_t b = threadIdx.x; b < LEN_BINS; b += GROUP_THREADS)
         if (lh[b]) atomicAdd(&hist[b], lh[b]);
@@ -1976,8 +2004,13 @@ constexpr uint32_t LEN_DONE_WORD = LEN_BINS;
 // up to 2^20 packets: one block per compute unit; measured 1.6 us less than the
 // scan launch per grouping there, 3.6 us more at 2^22 packets
 constexpr uint32_t LEN_FUSED_SCAN_MAX_BLOCKS = 256;
+// beyond them a block takes four times as many packets: fewer blocks add to the same few words
+// of hist[] and cursor[], and up to 2^22 packets still do without the scan launch (2^22: 10.5 us
+// to count and 19.8 to place; with one round and the scan launch 16.0, 4.7 and 20.7, with two
+// 11.8, 4.8 and 15.5, with eight and no scan launch 15.0 and 26.6)
+constexpr uint32_t LEN_MANY_ROUNDS = 4;
 static_assert(LEN_CURSOR_WORDS > LEN_DONE_WORD, "cursor[] holds the count of blocks that have read hist");
-template <bool SCAN>
+template <bool SCAN, uint32_t ROUNDS>
 __global__ __launch_bounds__(GROUP_THREADS) void len_scatter_kernel(const uint32_t *lens, uint32_t n,
                                                                     uint32_t tag_bytes, uint32_t *hist,
                                                                     uint32_t *cursor, uint32_t *order)
@@ -1989,13 +2022,10 @@ __global__ __launch_bounds__(GROUP_THREADS) void len_scatter_kernel(const uint32
     __shared__ uint32_t wave_sum[SCAN_WAVES];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     for (uint32_t b = threadIdx.x; b < LEN_BINS; b += GROUP_THREADS) cnt[b] = 0;
-    const uint32_t first = blockIdx.x * GROUP_CHUNK + threadIdx.x;
-    uint32_t bin[GROUP_PER_THREAD], at[GROUP_PER_THREAD];
+    const uint32_t first = blockIdx.x * ROUNDS * GROUP_CHUNK + threadIdx.x * GROUP_PER_THREAD;
+    uint32_t bin[ROUNDS][GROUP_PER_THREAD], at[ROUNDS][GROUP_PER_THREAD] = {};
 #pragma unroll
-    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) {
-        const uint32_t i = first + j * GROUP_THREADS;
-        bin[j] = len_bin(i < n ? lens[i] : 0u, tag_bytes);
-    }
+    for (uint32_t r = 0; r < ROUNDS; r++) len_bins4(lens, first + r * GROUP_CHUNK, n, tag_bytes, bin[r]);
     // exclusive scan of hist into base[]: PER consecutive bins per thread,
     // inclusive scan within the wave, then across the waves
     uint32_t loc[PER];
@@ -2031,8 +2061,12 @@ __global__ __launch_bounds__(GROUP_THREADS) void len_scatter_kernel(const uint32
     // a packet's place within its block's share of the bin, then one
     // reservation per bin for the whole block
 #pragma unroll
-    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++)
-        at[j] = wave_bin_add(cnt, bin[j], first + j * GROUP_THREADS < n);
+    for (uint32_t r = 0; r < ROUNDS; r++) {
+        uint32_t todo[GROUP_PER_THREAD];
+#pragma unroll
+        for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) todo[j] = bin[r][j];
+        wave_bins_add<true>(cnt, todo, at[r]);
+    }
     __syncthreads();
     for (uint32_t b = threadIdx.x; b < LEN_BINS; b += GROUP_THREADS) {
         const uint32_t c = cnt[b];
@@ -2040,10 +2074,10 @@ __global__ __launch_bounds__(GROUP_THREADS) void len_scatter_kernel(const uint32
     }
     __syncthreads();
 #pragma unroll
-    for (uint32_t j = 0; j < GROUP_PER_THREAD; j++) {
-        const uint32_t i = first + j * GROUP_THREADS;
-        if (i < n) order[base[bin[j]] + at[j]] = i;
-    }
+    for (uint32_t r = 0; r < ROUNDS; r++)
+#pragma unroll
+        for (uint32_t j = 0; j < GROUP_PER_THREAD; j++)
+            if (bin[r][j] != NO_BIN) order[base[bin[r][j]] + at[r][j]] = first + r * GROUP_CHUNK + j;
     if (SCAN && wv == 0 && (uint32_t)__builtin_amdgcn_readfirstlane((int)seen) + 1u == gridDim.x)
         for (uint32_t b = lane; b < LEN_BINS; b += 64u) hist[b] = 0;
 }
@@ -2108,6 +2142,25 @@ hipError_t launch_pull(const void *src, void *dst, uint64_t bytes, hipStream_t s
     return hipGetLastError();
 }
 
+template <uint32_t ROUNDS>
+static hipError_t length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_bytes, uint32_t *order, uint32_t *hist,
+                              uint32_t *cursor, hipStream_t s)
+{
+    const uint32_t blocks = (n + ROUNDS * GROUP_CHUNK - 1u) / (ROUNDS * GROUP_CHUNK);
+    const bool fused = blocks <= LEN_FUSED_SCAN_MAX_BLOCKS;
+    hipLaunchKernelGGL(len_hist_kernel<ROUNDS>, dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n, tag_bytes, hist,
+                       cursor, fused);
+    if (fused) {
+        hipLaunchKernelGGL((len_scatter_kernel<true, ROUNDS>), dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
+                           tag_bytes, hist, cursor, order);
+    } else {
+        hipLaunchKernelGGL(len_scan_kernel, dim3(1), dim3(LEN_SCAN_THREADS), 0, s, hist, cursor);
+        hipLaunchKernelGGL((len_scatter_kernel<false, LEN_MANY_ROUNDS>), dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
+                           tag_bytes, hist, cursor, order);
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_bytes,
                               uint32_t *order, uint32_t *hist, uint32_t *cursor,
                               hipStream_t s)
@@ -2116,19 +2169,9 @@ hipError_t launch_length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_byt
     // hist is all zeros on entry: its owner clears it once when it is allocated
     // and every grouping leaves it cleared (len_scan_kernel, or the scatter
     // launch that scans for itself)
-    const uint32_t blocks = (n + GROUP_CHUNK - 1u) / GROUP_CHUNK;
-    const bool fused = blocks <= LEN_FUSED_SCAN_MAX_BLOCKS;
-    hipLaunchKernelGGL(len_hist_kernel, dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n, tag_bytes, hist,
-                       cursor, fused);
-    if (fused) {
-        hipLaunchKernelGGL(len_scatter_kernel<true>, dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
-                           tag_bytes, hist, cursor, order);
-    } else {
-        hipLaunchKernelGGL(len_scan_kernel, dim3(1), dim3(LEN_SCAN_THREADS), 0, s, hist, cursor);
-        hipLaunchKernelGGL(len_scatter_kernel<false>, dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
-                           tag_bytes, hist, cursor, order);
-    }
-    return hipGetLastError();
+    const uint32_t chunks = (n + GROUP_CHUNK - 1u) / GROUP_CHUNK;
+    return chunks <= LEN_FUSED_SCAN_MAX_BLOCKS ? length_sort<1>(lens, n, tag_bytes, order, hist, cursor, s)
+                                               : length_sort<LEN_MANY_ROUNDS>(lens, n, tag_bytes, order, hist, cursor, s);
 }
 
 } // namespace bnk

@@ -755,3 +755,43 @@ def test_short_packets_at_different_places_of_a_line(ctx, form, longest):
         overdict = O.open_batch(keys, peer, ctr, got, dst_off, lens + np.uint32(16), before, off, 4)
         assert np.array_equal(verdict.cpu().numpy(), overdict) and int((overdict == 0).sum()) == 9
         assert np.array_equal(to.cpu().numpy(), before)
+
+
+@pytest.mark.parametrize("n,longest", [(65, 200), (4095, 1000), (4097, 60), (8193, 1471), ((1 << 20) + 4099, 70),
+                                       ((1 << 20) + (1 << 14), 0)])
+def test_grouping_by_length_keeps_every_packet(ctx, n, longest):
+    """A lane per packet with lengths of their own, grouped by length first: few and many
+    distinct sizes in a wave, a block's last packets, batches whose blocks take one round of packets
+    and several, and lengths that lie at any word of memory."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    key = rng.integers(0, 256, (1, 32), dtype=np.uint8)
+    lens = rng.integers(0, longest + 1, n).astype(np.uint32)
+    if n % 2:
+        lens[rng.random(n) < 0.7] = longest // 3  # (most of one size)
+    room = (lens.astype(np.uint64) + np.uint64(31)) // np.uint64(16) * np.uint64(16)
+    off = np.cumsum(room) - room
+    nb = int(off[-1] + room[-1])
+    plain = rng.integers(0, 256, nb, dtype=np.uint8)
+    want = np.full(nb, 0xEE, np.uint8)
+    counters = np.arange(n, dtype=np.uint64) + np.uint64(7)
+    O.seal_batch(key, np.zeros(n, np.uint32), counters, plain, off, lens, want, off, 4)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    d_plain, d_off, d_got = d(plain), d(off.astype(np.int64)), d(np.full(nb, 0xEE, np.uint8))
+    shift = 1 + n % 3
+    d_lens = d(np.concatenate([np.zeros(shift, np.int32), lens.astype(np.int32)]))[shift:]
+    ctx.keys_set(lib.KEYS_SEND, key)
+    ctx.set_spread_max_packets(0)
+    try:
+        torch.cuda.synchronize()
+        for _ in range(2):  # (a grouping leaves the counts as it found them)
+            ctx.seal(lib.make_batch(d_plain, nb, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens, counter0=7),
+                     lib.make_batch(d_got, nb, n, lib.MEM_DEVICE, offsets=d_off))
+            ctx.sync()
+            assert np.array_equal(d_got.cpu().numpy(), want)
+            d_got.fill_(0xEE)
+            torch.cuda.synchronize()
+    finally:
+        ctx.set_spread_max_packets(4096)

@@ -99,6 +99,7 @@ constexpr uint32_t RANK_TABLE_MAX_KEYS = 4096;
 constexpr uint32_t RANK_ROW_STEP = 256; // 64 lanes x 16 bytes
 constexpr uint32_t RANK_ROW_STEPS = RANK_TABLE_MAX_KEYS / RANK_ROW_STEP;
 constexpr uint32_t TILE_RUNS_MAX = 32;
+constexpr uint32_t TILE_RUNS_FEW = 8; // up to 2^20 packets
 constexpr size_t RANK_TABLE_MAX_BYTES = 64u << 20;
 // Sorting by peer (launch_peer_sort): up to this many keys.  With 4001 of them a tile's row is
 // longer than the tile and it is the library's radix sort or this within 3 % either way.
@@ -346,7 +347,21 @@ __device__ __forceinline__ uint32_t rank_key(uint32_t word, unsigned shift, uint
     return min(word >> shift, n_keys - 1u);
 }
 
-template <bool SHIFTED>
+// A tile's words, 64 to a run, every load on its way before the first is used: no branch
+// around a load (what a branch leaves unloaded the compiler merges with what was loaded, behind a
+// wait in each) but the last word again where a lane has none.  RUNS: the runs that a kernel is
+// compiled for; so few in most batches that a form of their own pays.  Together with the walks
+// below, which wait for LDS at their end instead of in every run: 2^18 packets of 256 peers,
+// assigning 10.8 -> 7.1 us, placing 10.6 -> 9.8, counting 6.4 -> 5.6; 2^22 of 4096 peers,
+// assigning 41.2 -> 39.7 (the table's rows, longer than the tile), counting 12.8 -> 11.4.
+template <uint32_t RUNS>
+__device__ __forceinline__ void tile_words(const uint32_t *words, uint32_t first, uint32_t end, uint32_t (&word)[RUNS])
+{
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) word[r] = words[min(first + r * 64u + threadIdx.x, end - 1u)];
+}
+
+template <bool SHIFTED, uint32_t RUNS>
 __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
                                                         uint32_t cols, uint32_t runs, uint32_t *table,
                                                         uint32_t *status, unsigned shift)
@@ -355,21 +370,17 @@ __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, ui
     const uint32_t lane = threadIdx.x;
     uint4 *cnt4 = reinterpret_cast<uint4 *>(cnt);
     for (uint32_t q = lane; q < cols / 4u; q += 64u) cnt4[q] = make_uint4(0, 0, 0, 0);
-    const uint32_t first = blockIdx.x * runs * 64u;
-    uint32_t key[TILE_RUNS_MAX];
-    // all of the tile's keys are on their way before the first one is counted
-#pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        const uint32_t i = first + r * 64u + lane;
-        key[r] = r < runs && i < n ? keys[i] : NO_PEER;
-    }
+    const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
+    uint32_t word[RUNS];
+    tile_words(keys, first, end, word);
     __syncthreads();
 #pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        if (SHIFTED && r < runs && first + r * 64u + lane < n) key[r] = rank_key(key[r], shift, n_keys);
-        if (key[r] < n_keys) atomicAdd(&cnt[key[r]], 1u);
+    for (uint32_t r = 0; r < RUNS; r++) {
+        if (first + r * 64u + lane >= end) break;
+        const uint32_t key = SHIFTED ? rank_key(word[r], shift, n_keys) : word[r];
+        if (key < n_keys) atomicAdd(&cnt[key], 1u);
         // (keys straight from a caller's peer array: one beyond the table gets no counter and is reported)
-        else if (status && r < runs && first + r * 64u + lane < n) status_raise(status, STATUS_PEER_RANGE);
+        else if (status) status_raise(status, STATUS_PEER_RANGE);
     }
     __syncthreads();
     uint4 *row = reinterpret_cast<uint4 *>(table + (size_t)blockIdx.x * cols);
@@ -434,6 +445,7 @@ __global__ __launch_bounds__(SCAN_PEERS * SCAN_PARTS) void rank_scan_kernel(uint
     }
 }
 
+template <uint32_t RUNS>
 __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
                                                          uint32_t cols, uint32_t runs, const uint32_t *table,
                                                          unsigned bits,
@@ -443,6 +455,10 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
     // packets of each peer ahead of the run at hand
     __shared__ __attribute__((aligned(16))) uint32_t before[RANK_TABLE_MAX_KEYS];
     const uint32_t lane = threadIdx.x;
+    const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
+    // keys and the peers' bases are fetched up front: nothing inside the walk below waits for memory
+    uint32_t key[RUNS];
+    tile_words(keys, first, end, key);
     {
         // the tile's row, every load in flight before the first is used
         const uint4 *row = reinterpret_cast<const uint4 *>(table + (size_t)blockIdx.x * cols);
@@ -454,43 +470,41 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
         for (uint32_t q = 0; q < RANK_ROW_STEPS; q++)
             if (q * RANK_ROW_STEP < cols) reinterpret_cast<uint4 *>(before)[q * 64u + lane] = v[q];
     }
-    const uint32_t first = blockIdx.x * runs * 64u;
-    uint32_t key[TILE_RUNS_MAX];
-    uint64_t base[TILE_RUNS_MAX];
-    // keys and the peers' bases are fetched up front: nothing inside the walk
-    // below waits for memory
+    uint64_t base[RUNS];
 #pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        const uint32_t i = first + r * 64u + lane;
-        key[r] = r < runs && i < n ? keys[i] : NO_PEER;
+    for (uint32_t r = 0; r < RUNS; r++) {
+        if (first + r * 64u + lane >= end) key[r] = NO_PEER;
+        base[r] = ctr_base[min(key[r], n_keys - 1u)];
+    }
+    __syncthreads();
+    uint32_t old[RUNS], lower[RUNS];
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) {
+        old[r] = lower[r] = 0u;
+        if (first + r * 64u < end) {
+            const uint32_t kk = key[r];
+            const bool valid = kk < n_keys;
+            // the lanes of this run with my peer
+            unsigned long long same = __ballot(valid);
+            for (unsigned b = 0; b < bits; b++) {
+                const unsigned long long m = __ballot((kk >> b) & 1u);
+                same &= ((kk >> b) & 1u) ? m : ~m;
+            }
+            lower[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            // every lane reads its entry before the one lane of each peer moves it: LDS serves a
+            // wave's accesses in order, so nothing is waited for from run to run
+            old[r] = before[min(kk, n_keys - 1u)];
+            if (valid && lower[r] == 0u) atomicAdd(&before[kk], (uint32_t)__popcll(same));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
     }
 #pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) base[r] = key[r] < n_keys ? ctr_base[key[r]] : 0ull;
-    __syncthreads();
-#pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        if (r < runs) { // uniform
-        const uint32_t kk = key[r];
-        const bool valid = kk < n_keys;
-        // the lanes of this run with my peer
-        unsigned long long same = __ballot(valid);
-        for (unsigned b = 0; b < bits; b++) {
-            const unsigned long long m = __ballot((kk >> b) & 1u);
-            same &= ((kk >> b) & 1u) ? m : ~m;
-        }
-        if (valid) {
-            const uint32_t lower = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-            const uint32_t rank = before[kk] + lower;
-            ctr_out[first + r * 64u + lane] = ctr_add(base[r], rank, ctr_limit);
-            // every lane has read the entry before any lane writes one: the lanes of a
-            // wave run in lockstep and LDS serves their accesses in order
-            if (lower == 0u) before[kk] += (uint32_t)__popcll(same);
-        } else if (zero_others && first + r * 64u + lane < n) {
-            ctr_out[first + r * 64u + lane] = 0; // a packet without a peer gets no counter
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        }
+    for (uint32_t r = 0; r < RUNS; r++) {
+        const uint32_t i = first + r * 64u + lane;
+        // (a packet without a peer gets no counter)
+        const bool valid = key[r] < n_keys;
+        if (i < end && (valid || zero_others)) ctr_out[i] = valid ? ctr_add(base[r], old[r] + lower[r], ctr_limit) : 0ull;
     }
 }
 
@@ -498,6 +512,7 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
 // library's radix sort takes five to nine with its memsets: a tunnel pass of 16000 packets of
 // 100 bytes 100 -> 92 us, 2^17 151 -> 133, 2^18 201 -> 184, 2^20 472 -> 457): a packet's place is where its
 // key's packets begin (every tile scans the totals for itself) plus its rank among them.
+template <uint32_t RUNS>
 __global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, uint32_t n, uint32_t n_keys,
                                                         uint32_t cols, uint32_t runs, const uint32_t *table,
                                                         const uint32_t *total, unsigned bits, unsigned shift,
@@ -505,13 +520,9 @@ __global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, u
 {
     __shared__ __attribute__((aligned(16))) uint32_t before[RANK_TABLE_MAX_KEYS];
     const uint32_t lane = threadIdx.x;
-    const uint32_t first = blockIdx.x * runs * 64u;
-    uint32_t word[TILE_RUNS_MAX];
-#pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        const uint32_t i = first + r * 64u + lane;
-        word[r] = r < runs && i < n ? words[i] : 0u;
-    }
+    const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
+    uint32_t word[RUNS];
+    tile_words(words, first, end, word);
     {
         const uint4 *const row = reinterpret_cast<const uint4 *>(table + (size_t)blockIdx.x * cols);
         const uint4 *const tot = reinterpret_cast<const uint4 *>(total);
@@ -541,27 +552,29 @@ __global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, u
         }
     }
     __syncthreads();
+    uint32_t at[RUNS], lower[RUNS];
 #pragma unroll
-    for (uint32_t r = 0; r < TILE_RUNS_MAX; r++) {
-        if (r < runs) { // uniform
-            const bool valid = first + r * 64u + lane < n;
+    for (uint32_t r = 0; r < RUNS; r++) {
+        at[r] = lower[r] = 0u;
+        if (first + r * 64u < end) { // uniform
+            const bool valid = first + r * 64u + lane < end;
             const uint32_t kk = rank_key(word[r], shift, n_keys);
             unsigned long long same = __ballot(valid);
             for (unsigned b = 0; b < bits; b++) {
                 const unsigned long long m = __ballot((kk >> b) & 1u);
                 same &= ((kk >> b) & 1u) ? m : ~m;
             }
-            if (valid) {
-                const uint32_t lower = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-                const uint32_t at = before[kk];
-                sorted[at + lower] = word[r];
-                // (see rank_assign_kernel)
-                if (lower == 0u) before[kk] = at + (uint32_t)__popcll(same);
-            }
+            lower[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            // (see rank_assign_kernel)
+            at[r] = before[kk];
+            if (valid && lower[r] == 0u) atomicAdd(&before[kk], (uint32_t)__popcll(same));
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
         }
     }
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++)
+        if (first + r * 64u + lane < end) sorted[at[r] + lower[r]] = word[r];
 }
 
 // One key more than there are peers: the packets without one, last.
@@ -584,11 +597,13 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
     const RankPlan plan = sort_plan(n, n_peers);
     const uint32_t n_keys = n_peers + 1u;
     uint32_t *table = static_cast<uint32_t *>(tmp), *total = table + (size_t)plan.tiles * plan.cols;
-    hipLaunchKernelGGL(rank_count_kernel<true>, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+    const auto count = plan.runs <= TILE_RUNS_FEW ? rank_count_kernel<true, TILE_RUNS_FEW> : rank_count_kernel<true, TILE_RUNS_MAX>;
+    const auto place = plan.runs <= TILE_RUNS_FEW ? rank_place_kernel<TILE_RUNS_FEW> : rank_place_kernel<TILE_RUNS_MAX>;
+    hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
                        (uint32_t *)nullptr, shift);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS), dim3(SCAN_PEERS * SCAN_PARTS), 0, s,
                        table, plan.tiles, n_keys, plan.cols, total, (uint64_t *)nullptr, (uint64_t *)nullptr, 0, 0ull);
-    hipLaunchKernelGGL(rank_place_kernel, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+    hipLaunchKernelGGL(place, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
                        total, key_bits(n_keys), shift, sorted);
     return hipGetLastError();
 }
@@ -601,12 +616,14 @@ static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &p
     uint32_t *table = static_cast<uint32_t *>(tmp);
     uint32_t *total = table + (size_t)plan.tiles * plan.cols;
     uint64_t *base_was = reinterpret_cast<uint64_t *>(total + plan.cols);
-    hipLaunchKernelGGL(rank_count_kernel<false>, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
+    const auto count = plan.runs <= TILE_RUNS_FEW ? rank_count_kernel<false, TILE_RUNS_FEW> : rank_count_kernel<false, TILE_RUNS_MAX>;
+    const auto assign = plan.runs <= TILE_RUNS_FEW ? rank_assign_kernel<TILE_RUNS_FEW> : rank_assign_kernel<TILE_RUNS_MAX>;
+    hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
                        table, status, 0u);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS),
                        dim3(SCAN_PEERS * SCAN_PARTS), 0, s, table, plan.tiles, n_keys, plan.cols, total, ctr_base,
                        base_was, advance ? 1 : 0, ctr_limit);
-    hipLaunchKernelGGL(rank_assign_kernel, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
+    hipLaunchKernelGGL(assign, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
                        table, key_bits(n_keys), base_was, ctr_out, ctr_limit, zero_others ? 1 : 0);
     return hipGetLastError();
 }

@@ -1596,3 +1596,59 @@ def test_uniform_device_batches_between_the_small_and_the_large_launches(n):
     assert (res == 0).all() and (olen == length).all() and np.array_equal(gp.cpu().numpy().view(np.uint32), peer)
     assert np.array_equal(out.cpu().numpy().reshape(n, stride)[:, :length], rows[:, 16:16 + length])
     ctx.close()
+
+
+@pytest.mark.parametrize("n_peers", [3, 300, 4096])
+@pytest.mark.parametrize("n", [64 * 1024 + 1, 1 << 20, (1 << 20) + 77])
+def test_send_counters_follow_batch_order_at_the_sizes_of_a_tile(n, n_peers):
+    """Tiles of a few runs of packets and of many, a last tile of a few packets: every packet
+    gets its peer's next counter in batch order, twice over; received, each is new to its window,
+    once."""
+    import torch
+    from bnk_amd import lib
+    dev = torch.device("cuda:0")
+    stride, plen = 64, 32
+    rng = np.random.default_rng(n + n_peers)
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    table = np.zeros((n_peers, 4), np.uint32)
+    table[:, 0] = np.arange(n_peers, dtype=np.uint32) * 7919 + 3
+    table[:, 1] = np.arange(n_peers, dtype=np.uint32) * 104729 + 11
+    table[:, 3] = 0xFFFFFFFF
+    peer = rng.integers(0, n_peers, n)
+    peer[rng.random(n) < 0.2] = n_peers - 1  # one busy peer
+    order = np.argsort(peer, kind="stable")
+    count = np.bincount(peer, minlength=n_peers)
+    rank = np.empty(n, np.int64)
+    rank[order] = np.arange(n) - np.repeat(np.cumsum(count) - count, count)
+    h = np.zeros((n, stride), np.uint8)
+    h[:, 16] = 0x45
+    h[:, 19] = plen
+    arena = torch.from_numpy(h).to(dev)
+    d_peer = torch.from_numpy(peer.astype(np.int32)).to(dev)
+    d_wl = torch.zeros(n, dtype=torch.int32, device=dev)
+    with lib.Context(0) as ctx:
+        ctx.keys_set(lib.KEYS_SEND, keys)
+        ctx.wg_peers_set(table)
+        for trip in range(2):
+            arena.copy_(torch.from_numpy(h))
+            torch.cuda.synchronize()
+            ctx.wg_encap(lib.make_batch(arena, arena.numel(), n, lib.MEM_DEVICE, stride=stride, length=plen, peer=d_peer),
+                         MTU, d_wl)
+            ctx.sync()
+            head = arena[:, :16].cpu().numpy().copy()
+            assert np.array_equal(head[:, 4:8].copy().view(np.uint32)[:, 0], table[peer, 1])
+            assert np.array_equal(head[:, 8:16].copy().view(np.int64)[:, 0], rank + trip * count[peer])
+        assert np.array_equal(ctx.wg_send_counters(n_peers), (2 * count).astype(np.uint64))
+    results = [torch.zeros(n, dtype=k, device=dev) for k in (torch.uint8, torch.int32, torch.int32, torch.int64)]
+    with lib.Context(0) as ctx:
+        ctx.keys_set(lib.KEYS_RECV, keys)
+        ctx.wg_peers_set(table[:, [1, 0, 2, 3]])
+        back = torch.zeros_like(arena)
+        for want in (lib.WG_OK, lib.WG_REPLAY):
+            torch.cuda.synchronize()
+            ctx.wg_decap(lib.make_batch(arena, arena.numel(), n, lib.MEM_DEVICE, stride=stride, length=64),
+                         lib.make_batch(back, back.numel(), n, lib.MEM_DEVICE, stride=stride), *results)
+            ctx.sync()
+            assert bool((results[0] == want).all())
+            assert np.array_equal(results[2].cpu().numpy(), peer)
+            assert np.array_equal(results[3].cpu().numpy(), rank + count[peer])

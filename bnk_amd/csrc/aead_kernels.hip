@@ -382,7 +382,7 @@ template <bool OPEN, bool ALIGNED, bool SHIFT = false, bool RUNS = false>
 BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_t *dst, uint32_t len,
                         uint32_t len_in, const uint8_t *safe, const uint32_t (&k)[8], uint32_t n1, uint32_t n2,
                         Poly32 &mac, uint32_t (&x)[16], Head &head, uint32_t blk0 = 0, uint32_t lead = 0,
-                        uint32_t key_lane = 0)
+                        uint32_t key_lane = 0, bool one_block = false)
 {
     // len_in <= len: the packet's bytes in memory; the up to 15 between the two
     // are padding that counts as zeros (a sealing WireGuard launch; otherwise
@@ -570,8 +570,9 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
     };
     if (RUNS) {
         // the pair of the first step, which in the packet's first run holds the one-time key
-        uint32_t y[16];
-        chacha_block2(k, blk0, n1, n2, x, y);
+        uint32_t y[16] = {};
+        if (one_block) chacha_block(k, blk0, n1, n2, x); // (see the kernel: a run is a block)
+        else chacha_block2(k, blk0, n1, n2, x, y);
         uint32_t otk[16];
 #pragma unroll
         for (int w = 0; w < 8; w++) otk[w] = w < 4 ? (uint32_t)__shfl((int)x[w], (int)key_lane, 64) : 0u;
@@ -588,10 +589,11 @@ BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_
 #undef BNK_COMMIT2
         wave_sync();
         if (steps != 0u) run_step(0u, x, y);
-        if (OPEN && head.on && lead != 0u) {
+        if (OPEN && head.on && (one_block ? key_lane + 1u == lane : lead != 0u)) {
             // (the plaintext's first cells, for the packet's record; see SplitPacket)
-            *head.keep0 = *reinterpret_cast<const uint4 *>(row + (((c0 + 4u) & 15u) << 4));
-            *head.keep1 = *reinterpret_cast<const uint2 *>(row + (((c0 + 5u) & 15u) << 4));
+            const uint32_t at = c0 + lead;
+            *head.keep0 = *reinterpret_cast<const uint4 *>(row + ((at & 15u) << 4));
+            *head.keep1 = *reinterpret_cast<const uint2 *>(row + (((at + 1u) & 15u) << 4));
         }
         wave_sync();
     } else {
@@ -1210,6 +1212,14 @@ void aead_short_kernel(AeadArgs a)
 // key, comes out of the first piece's pair, whose other half is the packet's first 64
 // bytes, so no lane computes a block for the key alone.  What splitting costs is the
 // lift, some fourteen field multiplications per lane (0.8 of a ChaCha20 block).
+//
+// Where the wave's packets have no more blocks than it has lanes, the keys' included, a run is
+// one block (one_block), the first of them the key alone: such a launch lasts as long as one wave
+// takes, and a wave by itself issues an instruction every five cycles whatever its lanes do, so
+// half the blocks and cells per lane are half of the 5.4 us that they take (600 waves of five IMIX
+// packets: a wave 14.4 -> 12.1 us, of which 2.4 are ChaCha20, 1.0 the cells, 1.5 the lift, 1.5 the
+// lines' way out, 4.7 the packets' metadata, the dealing and the keys; a pair of launches of 4000
+// such packets with three streams at work 13.2 -> 11.6 us, of 8000 23.5 -> 18.9).
 constexpr uint32_t SPLIT_MAX_RUNS = 32; // per packet (split_join)
 
 struct SplitPacket {
@@ -1247,32 +1257,40 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const bool decap = OPEN && a.wg.mode == WG_FUSE_DECAP;
 
     // ---- the packets, a lane each, and how they are dealt out ----
-    uint32_t q, lanes;
+    uint32_t reach, lanes; // bytes of a run; lanes that have one
+    bool one_block;
     {
         const LanePacket p = lane_packet<OPEN>(a, first + lane, lane < count);
         // (the last things a packet is asked for fly while the pieces are dealt out)
         const uint4 tag = ld16(OPEN && p.have ? p.src + p.len : reinterpret_cast<const uint8_t *>(a.keys));
-        const uint32_t pieces = p.have ? ((p.len + 63u) >> 6) / 2u + 1u : 0u;
-        uint32_t total = pieces, most = pieces;
+        const uint32_t blocks = p.have ? ((p.len + 63u) >> 6) + 1u : 0u, pieces = (blocks + 1u) / 2u;
+        uint32_t total = pieces, most = blocks, all = blocks;
 #pragma unroll
         for (int off = 32; off >= 1; off >>= 1) {
             total += (uint32_t)__shfl_xor((int)total, off, 64);
+            all += (uint32_t)__shfl_xor((int)all, off, 64);
             most = max(most, (uint32_t)__shfl_xor((int)most, off, 64));
         }
         // A packet that lands on itself, but not where it is (a datagram's plaintext at the datagram's
         // own offset, 16 bytes ahead of its ciphertext): its runs would overwrite each other's bytes.
         // A lane that goes through it alone reads ahead of what it writes, so such a wave deals out
         // whole packets.
-        const int64_t shift = (int64_t)((uint64_t)(uintptr_t)p.dst - (uint64_t)(uintptr_t)p.src), reach = (int64_t)p.len + 16;
-        const bool onto_itself = __ballot(shift != 0 && shift < reach && -shift < reach) != 0ull;
-        uint32_t runs;
-        for (q = max(onto_itself ? most : max((total + 63u) / 64u, (most + SPLIT_MAX_RUNS - 1u) / SPLIT_MAX_RUNS), 1u);; q++) {
-            lanes = runs = (pieces + q - 1u) / q;
+        const int64_t shift = (int64_t)((uint64_t)(uintptr_t)p.dst - (uint64_t)(uintptr_t)p.src), span = (int64_t)p.len + 16;
+        const bool onto_itself = __ballot(shift != 0 && shift < span && -shift < span) != 0ull;
+        uint32_t q = 0, runs = blocks;
+        lanes = all;
+        most = (most + 1u) / 2u;
+        one_block = !onto_itself && all <= 64u && most <= SPLIT_MAX_RUNS / 2u;
+        if (!one_block) {
+            for (q = max(onto_itself ? most : max((total + 63u) / 64u, (most + SPLIT_MAX_RUNS - 1u) / SPLIT_MAX_RUNS), 1u);; q++) {
+                lanes = runs = (pieces + q - 1u) / q;
 #pragma unroll
-            for (int off = 32; off >= 1; off >>= 1) lanes += (uint32_t)__shfl_xor((int)lanes, off, 64);
-            if (lanes <= 64u) break; // (at q = most every packet has one run)
+                for (int off = 32; off >= 1; off >>= 1) lanes += (uint32_t)__shfl_xor((int)lanes, off, 64);
+                if (lanes <= 64u) break; // (at q = most every packet has one run)
+            }
         }
-        q = __builtin_amdgcn_readfirstlane(q);
+        one_block = __builtin_amdgcn_readfirstlane(one_block);
+        reach = one_block ? 64u : 128u * __builtin_amdgcn_readfirstlane(q);
         lanes = __builtin_amdgcn_readfirstlane(lanes);
         uint32_t upto = runs;
 #pragma unroll
@@ -1320,9 +1338,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     const uint32_t run = on ? lane - my.deal.start : 0u;
     const uint32_t lead = on && run == 0u ? 4u : 0u;
     // (a packet's bytes count from 64 before it, where its key block lies)
-    const uint32_t begin = run * q * 128u;
+    const uint32_t begin = run * reach;
     const uint32_t plen = on ? my.len + 64u : 0u, plen_in = on ? my.deal.len_in + 64u : 0u;
-    const uint32_t len = min(plen - begin, q * 128u);
+    const uint32_t len = min(plen - begin, reach);
     const uint32_t len_in = plen_in > begin ? min(plen_in - begin, len) : 0u;
     const uint8_t *src = on ? my.from.src - 64 + begin : nullptr;
     uint8_t *dst = on ? my.dst - 64 + begin : nullptr;
@@ -1342,11 +1360,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     wave_sync(); // every lane has read what it starts with
     const bool lane_lines = (((uintptr_t)src | (uintptr_t)dst) & 15u) == 0 && (((uintptr_t)src ^ (uintptr_t)dst) & 127u) == 0;
     if (__ballot(!lane_lines) == 0ull)
-        body_lines<OPEN, true, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+        body_lines<OPEN, true, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, begin >> 6, lead, lane - run, one_block);
     else if (__ballot(((uintptr_t)dst & 3u) != 0) == 0ull)
-        body_lines<OPEN, false, true, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+        body_lines<OPEN, false, true, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, begin >> 6, lead, lane - run, one_block);
     else
-        body_lines<OPEN, false, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, 2u * run * q, lead, lane - run);
+        body_lines<OPEN, false, false, true>(tile, lane, src, dst, len, len_in, safe, k, n1, n2, mac, x, head, begin >> 6, lead, lane - run, one_block);
 
     // ---- my share of the tag, lifted over the cells behind my run ----
     {

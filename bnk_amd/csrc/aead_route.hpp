@@ -12,7 +12,8 @@ namespace bnk {
 // Which launch?  Packets in GPU memory (us per launch of n packets in a row, all of
 // them resident at once; seal and open within 2 us of each other):
 //   a wave per packet   9 + 4.2 per 1000 packets at 1420 bytes, 3.3 at 60
-//   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2)
+//   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2), 3 less than
+//                       with q = 1 where every block gets a lane of its own
 //   a lane per packet   5 + 2.75 per ChaCha20 block of the longest packet, and 20 more
 //                       for the grouping where lengths vary
 // so 4096 packets x 1420 take 21 / 18 / 71 us, 16384 66 / 26 / 71, and 24000 packets of 1
@@ -36,9 +37,12 @@ inline bool aead_runs_spread(const AeadArgs &a)
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
         return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
     }
-    // 3072 by default: beyond it the wave-per-packet launch goes over the chip once more (a pair
-    // of launches of 3000 packets of 1 to 1420 bytes 31 us against 32 split, of 3200 42 against 32)
-    const uint64_t most = 3ull * a.spread_max / 4;
+    // 2560 by default.  Pairs of launches of packets of 1 to 1420 bytes, us alone / with three
+    // streams at work, a wave per packet against split: 1500 23.7 / 11.0 against 29.0 / 10.9, 2000
+    // 25.1 / 14.0 against 29.6 / 12.2, 2500 29.6 / 17.2 against 30.9 / 11.6, 3000 31.2 / 20.5
+    // against 32.7 / 12.2 (3200, where the launch goes over the chip once more, 42 against 32);
+    // 3000 of 1420 33 / 21.3 against 32 / 12.5
+    const uint64_t most = 5ull * a.spread_max / 8;
     if (a.lens) return a.n <= most;
     return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);
 }
@@ -78,6 +82,19 @@ inline bool aead_runs_spread(const AeadArgs &a)
 // up to 1471 bytes they are, a piece is then all that a run ever holds, and the launch lasts
 // as long as that (3400 packets of 1 to 1420 bytes 46 -> 32 us a pair against as many as fit on
 // average, 10000 51 -> 40).
+//
+// A wave with a lane for every block of its packets (the kernel deals them out so whenever the
+// lanes allow) is done sooner still, so where that takes no more than a wave per SIMD it gets no
+// more packets than surely fit: two of any lengths up to 1984, five where twice the mean room
+// does, as many as the common length allows.  Pairs, us alone / with three streams at work:
+// tunnel passes of 200 IMIX packets 47.7 / 21.6 -> 42.7 / 19.3, of 900 58.6 / 21.7 -> 54.5 / 21.0, of
+// 2000 of 500 bytes 61 / 22.4 against 65 / 24.2; 3500 packets of 600 bytes 30.8 / 12.0 -> 27.1 / 10.7,
+// 8000 of 300 29.1 / 11.4 -> 26.2 / 10.6.  With more than one such wave per SIMD it only helps a launch
+// that is alone: 4000 packets of 1 to 1420 bytes two to a wave 34.5 / 23.7 against 32.1 / 13.1 five to
+// a wave, 8000 of 600 five to a wave 32.1 / 19.4 against 33.1 / 13.8.  (Not for one or two blocks
+// of data: 4000 of 60 bytes 22.2 / 8.5 against 15.8 / 7.8 a lane per packet, 20000 of 124 28.4 / 12.1
+// against 27.3 / 10.6.)
+
 // Room per packet: what the batch's packets take up on average in an arena that just holds them,
 // as far as the host can tell.  From the lengths themselves where it has them (16 bytes more, for
 // a tag and for the gaps between slots); of a batch in GPU memory it knows the stride, or else
@@ -99,6 +116,7 @@ inline uint32_t aead_room(const bnk_batch &b)
 
 constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
 constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
+constexpr uint32_t SPLIT_ONE_BLOCK_WAVES = 1024;
 inline uint32_t aead_split_packets(const AeadArgs &a)
 {
     // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)
@@ -113,6 +131,11 @@ inline uint32_t aead_split_packets(const AeadArgs &a)
         return k * mean + 0.3 * mean * sqrt((double)k) <= 64.0;
     };
     uint32_t q = 1, k = per;
+    // a lane per block wherever that leaves no more than a wave per SIMD
+    const uint32_t one_block = a.lens ? (5u * ((room + 31u) / 32u + 1u) <= 64u ? SPLIT_ALWAYS_ONE : 2u)
+                                      : std::min(64u / (blocks + 1u), SPLIT_MAX_PACKETS);
+    const bool ahead_of_lanes = a.lens || 150u + 920u < 275u * (blocks + 1u);
+    if (ahead_of_lanes && one_block >= 2u && a.n <= one_block * SPLIT_ONE_BLOCK_WAVES) return one_block;
     if (a.lens && per <= SPLIT_ALWAYS_ONE) return std::max(per, SPLIT_ALWAYS_ONE);
     while (q < pieces && !fits(k, q)) q++;
     while (k < SPLIT_MAX_PACKETS && fits(k + 1u, q)) k++;

@@ -795,3 +795,53 @@ def test_grouping_by_length_keeps_every_packet(ctx, n, longest):
             torch.cuda.synchronize()
     finally:
         ctx.set_spread_max_packets(4096)
+
+
+@pytest.mark.parametrize("layout", ["aligned", "packed"])
+@pytest.mark.parametrize("wave", [(0, 0, 0, 0, 0), (1, 64, 65, 16, 0), (768, 768, 768, 768, 704), (768, 768, 768, 768, 705),
+                                  (1984, 960, 640, 0, 0), (1985, 64, 64, 64, 64), (1420, 60, 576, 60, 60),
+                                  (1420, 1420, 1420, 1420, 1420)])
+def test_a_lane_per_block_or_per_run_of_blocks(ctx, layout, wave):
+    """Split over lanes: five packets of a wave whose blocks, the key's included, are as many as
+    it has lanes or one more, a packet of as many blocks as may be summed or one more, empty
+    packets; sealed, then opened with some tags forged, every byte against the oracle."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    n = 4103  # five to a wave, the last wave not full
+    rng = np.random.default_rng(sum(wave) + len(layout))
+    lens = np.tile(np.array(wave, np.uint32), n // 5 + 1)[:n]
+    keys = rng.integers(0, 256, (3, 32), dtype=np.uint8)
+    peer = rng.integers(0, 3, n).astype(np.uint32)
+    counters = rng.integers(0, 1 << 62, n).astype(np.uint64)
+    step = np.uint64(16 if layout == "aligned" else 1)
+    room = (lens.astype(np.uint64) + np.uint64(16) + step - np.uint64(1)) // step * step
+    off = np.cumsum(room) - room
+    nb = int(off[-1] + room[-1]) + 64
+    plain = rng.integers(0, 256, nb, dtype=np.uint8)
+    want = np.full(nb, 0xEE, np.uint8)
+    O.seal_batch(keys, peer, counters, plain, off, lens, want, off, 4)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    d_plain, d_off, d_got = d(plain), d(off.astype(np.int64)), d(np.full(nb, 0xEE, np.uint8))
+    more = dict(offsets=d_off, peer=d(peer.astype(np.int32)), counters=d(counters.astype(np.int64)))
+    d_lens, d_ct_lens = d(lens.astype(np.int32)), d(lens.astype(np.int32) + 16)
+    ctx.keys_set(lib.KEYS_SEND, keys)
+    ctx.keys_set(lib.KEYS_RECV, keys)
+    torch.cuda.synchronize()
+    ctx.seal(lib.make_batch(d_plain, nb, n, lib.MEM_DEVICE, lens=d_lens, **more),
+             lib.make_batch(d_got, nb, n, lib.MEM_DEVICE, offsets=d_off))
+    ctx.sync()
+    got = d_got.cpu().numpy()
+    assert np.array_equal(got, want)
+    forged = rng.choice(n, 50, replace=False)
+    got[(off[forged] + lens[forged] + np.uint64(9)).astype(np.int64)] ^= 4
+    back = np.full(nb, 0xEE, np.uint8)
+    overdict = O.open_batch(keys, peer, counters, got, off, lens + np.uint32(16), back, off, 4)
+    d_ct, d_back = d(got), d(np.full(nb, 0xEE, np.uint8))
+    verdict = torch.full((n,), 7, dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
+    ctx.open(lib.make_batch(d_ct, nb, n, lib.MEM_DEVICE, lens=d_ct_lens, **more),
+             lib.make_batch(d_back, nb, n, lib.MEM_DEVICE, offsets=d_off), verdict)
+    ctx.sync()
+    assert np.array_equal(verdict.cpu().numpy(), overdict)
+    assert np.array_equal(d_back.cpu().numpy(), back)

@@ -20,28 +20,57 @@ namespace bnk {
 
 constexpr uint32_t NO_PEER = 0xFFFFFFFFu;
 
+// Four packets a thread, and each array in one access where they all lie so that it can be (four
+// byte loads and stores a packet otherwise: 2^22 packets 20 us against 11.5).
+template <bool ALIGNED>
 __global__ __launch_bounds__(256) void relay_verdict_kernel(
     const uint8_t *auth, const uint8_t *pass, const uint32_t *peer_out, uint32_t n_peers_out,
     uint32_t n, uint32_t *keys, uint32_t *idx, uint8_t *verdict, uint64_t *ctr_out, uint32_t *status)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= n) return;
-    uint8_t v = !auth[i] ? BNK_RELAY_FORGED : !pass[i] ? BNK_RELAY_DENIED : BNK_RELAY_OK;
-    uint32_t key = NO_PEER;
-    if (v == BNK_RELAY_OK) {
-        key = peer_out[i];
-        if (key >= n_peers_out) {
-            status_raise(status, STATUS_PEER_RANGE);
-            v = BNK_RELAY_DENIED;
-            key = NO_PEER;
+    const uint32_t first = (blockIdx.x * 256u + threadIdx.x) * 4u;
+    if (first >= n) return;
+    const bool whole = ALIGNED && first + 4u <= n;
+    uint8_t au[4], pa[4], v[4];
+    uint32_t key[4];
+    if (whole) {
+        *reinterpret_cast<uint32_t *>(au) = *reinterpret_cast<const uint32_t *>(auth + first);
+        *reinterpret_cast<uint32_t *>(pa) = *reinterpret_cast<const uint32_t *>(pass + first);
+        *reinterpret_cast<uint4 *>(key) = *reinterpret_cast<const uint4 *>(peer_out + first);
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {
+            const uint32_t i = min(first + j, n - 1u);
+            au[j] = auth[i];
+            pa[j] = pass[i];
+            key[j] = peer_out[i];
         }
     }
-    verdict[i] = v;
-    keys[i] = key;
-    // (the counting kernels need no positions and write every packet's counter themselves)
-    if (idx) {
-        idx[i] = i;
-        ctr_out[i] = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        v[j] = !au[j] ? BNK_RELAY_FORGED : !pa[j] ? BNK_RELAY_DENIED : BNK_RELAY_OK;
+        if (v[j] == BNK_RELAY_OK && key[j] >= n_peers_out && first + j < n) {
+            status_raise(status, STATUS_PEER_RANGE);
+            v[j] = BNK_RELAY_DENIED;
+        }
+        if (v[j] != BNK_RELAY_OK) key[j] = NO_PEER;
+    }
+    if (whole) {
+        *reinterpret_cast<uint32_t *>(verdict + first) = *reinterpret_cast<const uint32_t *>(v);
+        *reinterpret_cast<uint4 *>(keys + first) = *reinterpret_cast<const uint4 *>(key);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t i = first + j;
+        if (i >= n) break;
+        if (!whole) {
+            verdict[i] = v[j];
+            keys[i] = key[j];
+        }
+        // (the counting kernels need no positions and write every packet's counter themselves)
+        if (idx) {
+            idx[i] = i;
+            ctr_out[i] = 0;
+        }
     }
 }
 
@@ -161,12 +190,13 @@ hipError_t launch_relay_assign(const uint8_t *auth, const uint8_t *pass, const u
                                uint64_t *ctr_out, uint32_t *status, bool advance, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    const dim3 grid((n + 255u) / 256u);
     const RankPlan plan = rank_plan(n, n_peers_out);
     const bool one_block = peer_rank_one_block(n, n_peers_out);
     const bool counting = !one_block && plan.fits && plan.bytes <= sort_tmp_bytes;
-    hipLaunchKernelGGL(relay_verdict_kernel, grid, dim3(256), 0, s, auth, pass, peer_out, n_peers_out,
-                       n, keys, counting ? (uint32_t *)nullptr : idx, verdict, ctr_out, status);
+    const bool aligned = (((uintptr_t)auth | (uintptr_t)pass | (uintptr_t)verdict) & 3u) == 0 &&
+                         (((uintptr_t)peer_out | (uintptr_t)keys) & 15u) == 0;
+    hipLaunchKernelGGL(aligned ? relay_verdict_kernel<true> : relay_verdict_kernel<false>, dim3((n + 1023u) / 1024u), dim3(256), 0, s,
+                       auth, pass, peer_out, n_peers_out, n, keys, counting ? (uint32_t *)nullptr : idx, verdict, ctr_out, status);
     // (keys[] is the peer of each survivor and all ones for the rest)
     if (one_block)
         return launch_peer_rank_one_block(keys, n_peers_out, n, const_cast<uint64_t *>(ctr_base_out), ctr_out, advance,

@@ -242,3 +242,48 @@ def test_relay_full_size_device_resident_properties():
         o, L = int(b.off[i]), int(b.lens[i])
         assert (o_host[o:o + L + 16] == 0x77).all()
     ctx.close()
+
+
+@pytest.mark.parametrize("shift", [0, 1, 2])
+@pytest.mark.parametrize("n", [9, 66, 5003, 70001])
+def test_relay_of_device_arrays_that_lie_anywhere(n, shift):
+    """Verdicts and counters of a device batch whose arrays begin at any byte or word, with a
+    number of packets that is no multiple of what a thread takes, against the oracle."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    w = W.relay_workload(n=n, n_peers=7, n_rules=64)
+    b = w.batch
+    keys_in, keys_out = np.ascontiguousarray(b.keys), np.ascontiguousarray(w.keys_out)
+    sealed = np.zeros_like(b.plain)
+    O.seal_batch(keys_in, b.peer, b.counters, b.plain, b.off, b.lens, sealed, b.off, 4)
+    forged = W.forge_tags(5, sealed, b.off, b.lens, 0.1)
+    ct_lens = (b.lens + 16).astype(np.uint32)
+    ora = O.Filter()
+    ora.set_rules(w.rules_ref)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    total = sealed.nbytes
+    with lib.Context(0) as ctx:
+        ctx.filter_set_rules(w.rules_ref)
+        ctx.keys_set(lib.KEYS_RECV, keys_in)
+        ctx.keys_set(lib.KEYS_SEND, keys_out)
+        _note(ctx, ora, w)
+        want_out = np.full_like(b.plain, 0x77)
+        want_v, want_c = ora.relay_fused_batch(keys_in, b.peer, b.counters, keys_out, w.peer_out, w.ctr_base_out, sealed,
+                                               b.off, ct_lens, want_out, b.off, w.now_ns)
+        out = torch.full((total,), 0x77, dtype=torch.uint8, device="cuda:0")
+        verdict = torch.full((n + shift + 1,), 9, dtype=torch.uint8, device="cuda:0")
+        peer_out = d(np.concatenate([np.zeros(shift, np.int32), w.peer_out.astype(np.int32)]))
+        ctr_out = torch.zeros(n, dtype=torch.int64, device="cuda:0")
+        off = d(b.off.astype(np.int64))
+        torch.cuda.synchronize()
+        ctx.relay_fused(lib.make_batch(d(sealed), total, n, lib.MEM_DEVICE, offsets=off, lens=d(ct_lens.astype(np.int32)),
+                                       peer=d(b.peer.astype(np.int32)), counters=d(b.counters.astype(np.int64))),
+                        peer_out[shift:], d(w.ctr_base_out.astype(np.int64)), len(w.ctr_base_out), w.now_ns,
+                        lib.make_batch(out, total, n, lib.MEM_DEVICE, offsets=off), verdict[shift:], ctr_out)
+        ctx.sync()
+        v = verdict.cpu().numpy()
+        assert np.array_equal(v[shift:shift + n], want_v) and np.array_equal(want_v == 1, forged)
+        assert (v[:shift] == 9).all() and v[shift + n] == 9
+        assert np.array_equal(ctr_out.cpu().numpy().astype(np.uint64), want_c)
+        assert np.array_equal(out.cpu().numpy(), want_out)

@@ -1186,10 +1186,12 @@ __global__ __launch_bounds__(LANE_BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2
 
 // Batches in which the host can tell that every wave takes the short path
 // (every_wave_short): without the ring and the line paths' registers, and with no more of a
-// tile than the packets fill, five (up to 64 bytes) or four such waves fit a SIMD where the launch above holds two.
-// Handing the short waves of a mixed batch to this kernel in a second launch was measured too and
-// loses: every wave of both launches walks its metadata before it knows whose it is (IMIX 9 %
-// slower, the relay 3.5 %).
+// tile than the packets fill, five (up to 64 bytes: 85 to 91 registers) or four (up to 128: 102
+// to 111) such waves fit a SIMD where the launch above holds two.  2^20 packets of 60 / 100 / 124
+// bytes, us a pair: four and three 134 / 190 / 212, five and four 131 / 190 / 210, six (spilled)
+// and four 163 / 190 / 210.  Handing the short waves of a mixed batch to this kernel in a second
+// launch was measured too and loses: every wave of both launches walks its metadata before it
+// knows whose it is (IMIX 9 % slower, the relay 3.5 %).
 template <int CELLS>
 constexpr int SHORT_WAVES = CELLS == 4 ? 5 : 4;
 template <bool OPEN, int CELLS>

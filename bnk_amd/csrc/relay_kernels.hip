@@ -30,8 +30,8 @@ __global__ __launch_bounds__(256) void relay_verdict_kernel(
     const uint32_t first = (blockIdx.x * 256u + threadIdx.x) * 4u;
     if (first >= n) return;
     const bool whole = ALIGNED && first + 4u <= n;
-    uint8_t au[4], pa[4], v[4];
-    uint32_t key[4];
+    alignas(4) uint8_t au[4], pa[4], v[4];
+    alignas(16) uint32_t key[4];
     if (whole) {
         *reinterpret_cast<uint32_t *>(au) = *reinterpret_cast<const uint32_t *>(auth + first);
         *reinterpret_cast<uint32_t *>(pa) = *reinterpret_cast<const uint32_t *>(pass + first);

@@ -262,8 +262,7 @@ BNK_DEV QuadBlocks rules_fetch_quad(const RuleIndexDev &ri, uint32_t lane, uint3
                       rules_block<SMALL>(ri, quad_bcast<2>(iv))[part], rules_block<SMALL>(ri, quad_bcast<3>(iv))[part]};
 }
 
-template <bool SMALL>
-BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint32_t lane, uint32_t iv, uint32_t src, uint32_t key)
+BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint32_t lane, uint32_t src, uint32_t key)
 {
     const uint32_t part = lane & 3u;
     // packet j of the quad in the lane's own 16 bytes, and of all that the quad's lanes find the
@@ -276,12 +275,21 @@ BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint3
                    hi = min(odd ? m3 : m2, quad_perm<1, 0, 3, 2>(odd ? m2 : m3));
     bool hit = min(upper ? hi : lo, quad_perm<2, 3, 0, 1>(upper ? lo : hi)) == 0u;
     if (ri.long_lists) {
-        // it shows in the first word of the block, which the quad's first lane holds for packet j
-        // as p<j>.x
+        // A long list shows in the first word of the block, which the quad's first lane holds for packet j
+        // as p<j>.x, next to where the list lies.  Each lane takes its packet's from there: fetching the
+        // block's first words again, by every lane of a wave in which one packet's list is long, were 64
+        // look-ups of 64 lines for the few that need them (4096 rules: the relay's launch over 2^22
+        // records 88.5 us against 70.8, 2^22 plain headers 68.0 against 59.5).
         const bool far = (q.p0.x == RANGE_LONG) | (q.p1.x == RANGE_LONG) | (q.p2.x == RANGE_LONG) | (q.p3.x == RANGE_LONG);
         if (__ballot(far & (part == 0u)) != 0ull) {
-            const uint4 head = *rules_block<SMALL>(ri, iv); // (the line is in L1 by now)
-            if (head.x == RANGE_LONG) hit = long_list_hit(ri, head.y, head.z, key);
+            // (all four exchanges by all lanes, then the choice)
+            auto mine = [&](uint32_t a, uint32_t b, uint32_t c, uint32_t d) __attribute__((always_inline)) {
+                const uint32_t a0 = quad_bcast<0>(a), b0 = quad_bcast<0>(b), c0 = quad_bcast<0>(c), d0 = quad_bcast<0>(d);
+                return upper ? (odd ? d0 : c0) : (odd ? b0 : a0);
+            };
+            const uint32_t head = mine(q.p0.x, q.p1.x, q.p2.x, q.p3.x), first = mine(q.p0.y, q.p1.y, q.p2.y, q.p3.y),
+                           nblk = mine(q.p0.z, q.p1.z, q.p2.z, q.p3.z);
+            if (head == RANGE_LONG) hit = long_list_hit(ri, first, nblk, key);
         }
     }
     if (!hit)
@@ -313,10 +321,11 @@ struct RawHeader {
 
 // Where a launch finds its headers: in packets of one length at one stride and nothing else to
 // look at; in packets with per-packet arrays, whichever of them there are; in the records of
-// FilterArgs::heads.  A launch is compiled for one of them: with all three in one kernel its
-// arguments do not fit the scalar registers and are fetched out of vector registers lane by
-// lane wherever they are used (2^22 plain headers: 510 vector and 280 scalar instructions per
-// 64 packets).
+// FilterArgs::heads.  A launch is compiled for one of them: with all three in one kernel 98 scalar
+// registers do not fit and are fetched out of vector registers lane by lane wherever they are used
+// (278 places; 2^22 plain headers: 510 vector and 280 scalar instructions per 64 packets).  What still
+// does not fit, with a jump table: 20 registers of plain headers (25 places), 34 of records (62), 56 of
+// arrays (144), few of them on a packet's usual way.
 enum HeaderFrom { FROM_PLAIN, FROM_ARRAYS, FROM_RECORDS };
 
 // The loads of one packet, every one issued whether or not the lane needs it (from `safe`, 32
@@ -410,8 +419,9 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     // 65,536 flows took 79.3 us with 510 vector and 280 scalar instructions per 64 packets, the
     // rule lists fetched a word at a time as the tests before it failed; compiled per kind of
     // launch, without branches in the parse and the tests, and with the loads ahead of what
-    // waits for them 355 and 111, and 67.4.  The next header ahead of the flow's look-up as
-    // well: 72 (its loads queue ahead of the look-up's).
+    // waits for them 355 and 111, and 67.4, and 59.5 with a long list's place taken from the quad
+    // (rules_match_quad).  The next header ahead of the flow's look-up as well: 72 against 67.4 (its
+    // loads queue ahead of the look-up's).
     RawHeader raw = fetch_header<FROM>(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
     {
         constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = (SMALL_QUADS + FILTER_THREADS - 1u) / FILTER_THREADS;
@@ -481,7 +491,7 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         asm volatile("" ::: "memory"); // (both are on their way before either is waited for)
         maybe &= ((present >> (s.bit & 31u)) & 1u) != 0u;
         uint8_t pass = 0;
-        if (rules_match_quad<JUMPS>(ri, blocks, lane, iv, h.src, key)) {
+        if (rules_match_quad(ri, blocks, lane, h.src, key)) {
             pass = valid ? 1 : 0;
         } else if (valid) {
             for (uint32_t probe = 0; maybe && probe < a.flows.cap; probe++) {

@@ -20,22 +20,33 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 WAVE_KERNELS = ("_ZN3bnk16aead_wave_kernelILb0EEEvNS_8AeadArgsE", "_ZN3bnk16aead_wave_kernelILb1EEEvNS_8AeadArgsE")
 # the same loop over a run of a packet, with a few lanes per packet
 SPLIT_KERNELS = tuple("_ZN3bnk17aead_split_kernelILb%dEEEvNS_8AeadArgsE" % o for o in (0, 1))
+# CheckInbound over plain headers, per-packet arrays, records; without and with a jump table
+CHECK_KERNELS = tuple("_ZN3bnk19filter_check_kernelILi%dELb%dEEEvNS_10FilterArgsE" % (f, j) for f in (0, 1, 2) for j in (0, 1))
 # seal, open, seal + framing, open + framing of a small batch: a wave per packet
 SPREAD_KERNELS = tuple("_ZN3bnk18aead_spread_kernelILb%dELb%dEEEvNS_8AeadArgsE" % (o, w) for w in (0, 1) for o in (0, 1))
 
 
-@pytest.fixture(scope="module")
-def listing():
+def _listing_of(source):
     if not os.path.exists(HIPCC):
         pytest.skip("no hipcc")
     with tempfile.TemporaryDirectory() as tmp:
-        out = os.path.join(tmp, "aead_kernels.s")
+        out = os.path.join(tmp, source + ".s")
         # the library's own flags (bnk_amd/csrc/Makefile), to a device-side listing instead of an object
         cmd = [HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-               "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, "aead_kernels.hip"), "-o", out]
+               "-packed-fp32-ops", "-S", "--cuda-device-only", os.path.join(CSRC, source), "-o", out]
         r = subprocess.run(cmd, capture_output=True, text=True, timeout=600)
         assert r.returncode == 0, r.stderr[-2000:]
         return open(out).read()
+
+
+@pytest.fixture(scope="module")
+def listing():
+    return _listing_of("aead_kernels.hip")
+
+
+@pytest.fixture(scope="module")
+def filter_listing():
+    return _listing_of("filter_kernels.hip")
 
 
 def _body(listing, name):
@@ -83,3 +94,14 @@ def test_a_small_batch_packet_is_fetched_in_one_go(listing, name):
         elif t.startswith("s_waitcnt") and "vmcnt" in t:
             run = 0
     assert best >= 9, "longest run of loads without a wait for memory is %d in %s" % (best, name)
+
+
+@pytest.mark.parametrize("name", CHECK_KERNELS)
+def test_a_rule_block_is_fetched_once(filter_listing, name):
+    """The first words of a packet's rule block say where a list too long for the block lies.  They
+    come with the block; read from memory again (words 1 and 2 of it, an 8-byte load 4 bytes in, as the
+    kernel did) they cost a look-up for every lane of the wave."""
+    lines = _body(filter_listing, name)
+    assert sum("global_load_dwordx4" in x for x in lines) >= 8, "not the kernel this test was written for"
+    again = [x.strip() for x in lines if re.search(r"global_load_dwordx[24].*offset:4\s*$", x)]
+    assert not again, "%s reads a rule block's pointer words from memory: %r" % (name, again)

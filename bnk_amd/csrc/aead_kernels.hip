@@ -1908,10 +1908,7 @@ BNK_DEV uint32_t len_bin(uint32_t len, uint32_t tag_bytes)
 }
 
 // A block of GROUP_THREADS threads takes ROUNDS times GROUP_CHUNK consecutive packets, each time
-// four consecutive ones per thread, all loaded together.
-constexpr uint32_t GROUP_THREADS = 1024;
-constexpr uint32_t GROUP_PER_THREAD = 4;
-constexpr uint32_t GROUP_CHUNK = GROUP_THREADS * GROUP_PER_THREAD;
+// four consecutive ones per thread, all loaded together (len_sort_plan says how many).
 constexpr uint32_t NO_BIN = 0xFFFFFFFFu;
 
 // The bins of packets i to i + 3 (NO_BIN beyond the batch).
@@ -1919,13 +1916,13 @@ BNK_DEV void len_bins4(const uint32_t *lens, uint32_t i, uint32_t n, uint32_t ta
 {
     typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) u32x4_words;
     static_assert(GROUP_PER_THREAD == 4, "one load per thread");
-    if (i + 4u <= n) {
+    if (has_from(i, 4u, n)) {
         const u32x4_words v = *reinterpret_cast<const u32x4_words *>(lens + i);
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++) bin[j] = len_bin(v[j], tag_bytes);
     } else {
 #pragma unroll
-        for (uint32_t j = 0; j < 4; j++) bin[j] = i + j < n ? len_bin(lens[i + j], tag_bytes) : NO_BIN;
+        for (uint32_t j = 0; j < 4; j++) bin[j] = has_from(i, j + 1u, n) ? len_bin(lens[i + j], tag_bytes) : NO_BIN;
     }
 }
 
@@ -2046,14 +2043,6 @@ __global__ __launch_bounds__(LEN_SCAN_THREADS) void len_scan_kernel(uint32_t *hi
 // block counts itself in cursor[LEN_DONE_WORD] behind the barrier that follows
 // its scan, whose additions consumed the loaded values, so no fence is needed.
 constexpr uint32_t LEN_DONE_WORD = LEN_BINS;
-// up to 2^20 packets: one block per compute unit; measured 1.6 us less than the
-// scan launch per grouping there, 3.6 us more at 2^22 packets
-constexpr uint32_t LEN_FUSED_SCAN_MAX_BLOCKS = 256;
-// beyond them a block takes four times as many packets: fewer blocks add to the same few words
-// of hist[] and cursor[], and up to 2^22 packets still do without the scan launch (2^22: 10.5 us
-// to count and 19.8 to place; with one round and the scan launch 16.0, 4.7 and 20.7, with two
-// 11.8, 4.8 and 15.5, with eight and no scan launch 15.0 and 26.6)
-constexpr uint32_t LEN_MANY_ROUNDS = 4;
 static_assert(LEN_CURSOR_WORDS > LEN_DONE_WORD, "cursor[] holds the count of blocks that have read hist");
 template <bool SCAN, uint32_t ROUNDS>
 __global__ __launch_bounds__(GROUP_THREADS) void len_scatter_kernel(const uint32_t *lens, uint32_t n,
@@ -2187,25 +2176,6 @@ hipError_t launch_pull(const void *src, void *dst, uint64_t bytes, hipStream_t s
     return hipGetLastError();
 }
 
-template <uint32_t ROUNDS>
-static hipError_t length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_bytes, uint32_t *order, uint32_t *hist,
-                              uint32_t *cursor, hipStream_t s)
-{
-    const uint32_t blocks = (n + ROUNDS * GROUP_CHUNK - 1u) / (ROUNDS * GROUP_CHUNK);
-    const bool fused = blocks <= LEN_FUSED_SCAN_MAX_BLOCKS;
-    hipLaunchKernelGGL(len_hist_kernel<ROUNDS>, dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n, tag_bytes, hist,
-                       cursor, fused);
-    if (fused) {
-        hipLaunchKernelGGL((len_scatter_kernel<true, ROUNDS>), dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
-                           tag_bytes, hist, cursor, order);
-    } else {
-        hipLaunchKernelGGL(len_scan_kernel, dim3(1), dim3(LEN_SCAN_THREADS), 0, s, hist, cursor);
-        hipLaunchKernelGGL((len_scatter_kernel<false, LEN_MANY_ROUNDS>), dim3(blocks), dim3(GROUP_THREADS), 0, s, lens, n,
-                           tag_bytes, hist, cursor, order);
-    }
-    return hipGetLastError();
-}
-
 hipError_t launch_length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_bytes,
                               uint32_t *order, uint32_t *hist, uint32_t *cursor,
                               hipStream_t s)
@@ -2214,9 +2184,16 @@ hipError_t launch_length_sort(const uint32_t *lens, uint32_t n, uint32_t tag_byt
     // hist is all zeros on entry: its owner clears it once when it is allocated
     // and every grouping leaves it cleared (len_scan_kernel, or the scatter
     // launch that scans for itself)
-    const uint32_t chunks = (n + GROUP_CHUNK - 1u) / GROUP_CHUNK;
-    return chunks <= LEN_FUSED_SCAN_MAX_BLOCKS ? length_sort<1>(lens, n, tag_bytes, order, hist, cursor, s)
-                                               : length_sort<LEN_MANY_ROUNDS>(lens, n, tag_bytes, order, hist, cursor, s);
+    const LenSortPlan plan = len_sort_plan(n);
+    const dim3 grid(plan.blocks), block(GROUP_THREADS);
+    hipLaunchKernelGGL(plan.rounds == 1u ? len_hist_kernel<1> : len_hist_kernel<LEN_MANY_ROUNDS>, grid, block, 0, s, lens, n,
+                       tag_bytes, hist, cursor, plan.fused);
+    if (!plan.fused) hipLaunchKernelGGL(len_scan_kernel, dim3(1), dim3(LEN_SCAN_THREADS), 0, s, hist, cursor);
+    const auto scatter = plan.rounds == 1u ? len_scatter_kernel<true, 1>
+                         : plan.fused      ? len_scatter_kernel<true, LEN_MANY_ROUNDS>
+                                           : len_scatter_kernel<false, LEN_MANY_ROUNDS>;
+    hipLaunchKernelGGL(scatter, grid, block, 0, s, lens, n, tag_bytes, hist, cursor, order);
+    return hipGetLastError();
 }
 
 } // namespace bnk

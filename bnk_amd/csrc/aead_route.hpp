@@ -148,4 +148,30 @@ inline bool aead_wants_order(const AeadArgs &a)
     return a.lens && a.n > 64 && !aead_runs_spread(a) && aead_split_packets(a) == 0;
 }
 
+// How a batch's lengths are grouped (launch_length_sort).  A block takes GROUP_CHUNK packets at a time,
+// one round of them in batches of up to LEN_FUSED_SCAN_MAX_BLOCKS blocks (2^20 packets, a block per
+// compute unit).  Beyond, a block takes LEN_MANY_ROUNDS: fewer blocks add to the same few words of
+// hist[] and cursor[], and up to 2^22 packets the scatter launch still scans for itself, without a
+// launch for the scan (2^22: 10.5 us to count and 19.8 to place; with one round and the scan launch
+// 16.0, 4.7 and 20.7, with two rounds 11.8, 4.8 and 15.5, with eight and no scan launch 15.0 and 26.6).  Where
+// the blocks are more than that, a launch of its own scans: every block would fetch the same few lines
+// (2^22 packets, one round: 3.6 us more than the scan launch; 2^20: 1.6 less).
+constexpr uint32_t GROUP_THREADS = 1024;
+constexpr uint32_t GROUP_PER_THREAD = 4; // consecutive packets
+constexpr uint32_t GROUP_CHUNK = GROUP_THREADS * GROUP_PER_THREAD;
+constexpr uint32_t LEN_FUSED_SCAN_MAX_BLOCKS = 256;
+constexpr uint32_t LEN_MANY_ROUNDS = 4;
+struct LenSortPlan {
+    uint32_t rounds, blocks;
+    bool fused; // the scatter launch scans
+};
+// (for any n: the packets of a full grid are at most 2^32, so a thread's first one never wraps)
+inline LenSortPlan len_sort_plan(uint32_t n)
+{
+    const uint32_t chunks = n / GROUP_CHUNK + (n % GROUP_CHUNK != 0u);
+    const uint32_t rounds = chunks <= LEN_FUSED_SCAN_MAX_BLOCKS ? 1u : LEN_MANY_ROUNDS;
+    const uint32_t blocks = (chunks + rounds - 1u) / rounds;
+    return {rounds, blocks, blocks <= LEN_FUSED_SCAN_MAX_BLOCKS};
+}
+
 } // namespace bnk

@@ -199,6 +199,8 @@ __host__ __device__ inline bool beyond_arena(uint64_t off, uint32_t skip, uint64
 {
     return beyond_arena(off, skip + len, limit);
 }
+// Are there k elements from number i on, of n?  (i + k would wrap where i lies close to 2^32.)
+__host__ __device__ inline bool has_from(uint32_t i, uint32_t k, uint32_t n) { return i < n && n - i >= k; }
 #if defined(__HIPCC__)
 __device__ inline void status_raise(uint32_t *status, uint32_t condition)
 {

@@ -136,6 +136,25 @@ static void room_per_packet()
         }
 }
 
+// Grouping by length: a grid's threads, four packets each and round, cover the batch, none of them
+// begins beyond 2^32 - 1, and a block more would be one too many.
+static void length_grouping()
+{
+    const uint32_t top = 0xFFFFFFFFu;
+    for (uint32_t n : {1u, 4095u, 4096u, 4097u, 1u << 20, (1u << 20) + 1u, (1u << 20) + 16385u, 1u << 22, (1u << 22) + 1u,
+                       (1u << 22) + 4099u, top - 16384u, top - 16383u, top - 4096u, top - 4095u, top - 1u, top}) {
+        const LenSortPlan p = len_sort_plan(n);
+        const uint64_t per_block = (uint64_t)p.rounds * GROUP_CHUNK, packets = p.blocks * per_block;
+        expect(packets >= n && packets - per_block < n && packets <= 1ull << 32, "the blocks that group a batch");
+        expect(p.rounds == 1u || p.rounds == LEN_MANY_ROUNDS, "a number of rounds that there is a kernel for");
+        expect(p.rounds != 1u || p.fused, "one round only where the scatter launch scans");
+        expect(p.fused == (n <= 1u << 22), "who scans");
+        for (uint32_t k : {1u, 4u})
+            for (uint32_t i : {0u, n - 1u, n - 4u, n - 5u, n, top - 3u, top})
+                expect(has_from(i, k, n) == ((uint64_t)i + k <= n), "packets left from one on");
+    }
+}
+
 // The bound on claimed slots against a model of the launches: never below what is claimed, back
 // down to it once the batches have run, however many batches there have been (the numbers wrap at
 // 2^32, and a table may stay as it is for longer than 2^31 of them).
@@ -176,6 +195,7 @@ int main()
     fetched_batches_stay_with_the_lanes();
     framing_behind_a_header();
     room_per_packet();
+    length_grouping();
     for (uint32_t first_seq : {0u, 1000u, 0x7FFFFFFFu - 2000u, 0x80000001u, 0xFFFFFFFFu - 2000u}) claimed_slots(first_seq);
     if (!failures) printf("PASS launch rules\n");
     return failures;

@@ -758,11 +758,12 @@ def test_short_packets_at_different_places_of_a_line(ctx, form, longest):
 
 
 @pytest.mark.parametrize("n,longest", [(65, 200), (4095, 1000), (4097, 60), (8193, 1471), ((1 << 20) + 4099, 70),
-                                       ((1 << 20) + (1 << 14), 0)])
+                                       ((1 << 20) + (1 << 14), 0), ((1 << 22) + 4099, 16)])
 def test_grouping_by_length_keeps_every_packet(ctx, n, longest):
     """A lane per packet with lengths of their own, grouped by length first: few and many
     distinct sizes in a wave, a block's last packets, batches whose blocks take one round of packets
-    and several, and lengths that lie at any word of memory."""
+    and several, so many blocks that a launch of its own scans the counts, and lengths that lie at any
+    word of memory."""
     import torch
     from bnk_amd import lib
     from oracle import binding as O

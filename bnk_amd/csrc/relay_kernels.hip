@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void relay_verdict_kernel(
 {
     const uint32_t first = (blockIdx.x * 256u + threadIdx.x) * 4u;
     if (first >= n) return;
-    const bool whole = ALIGNED && first + 4u <= n;
+    const bool whole = ALIGNED && has_from(first, 4u, n);
     alignas(4) uint8_t au[4], pa[4], v[4];
     alignas(16) uint32_t key[4];
     if (whole) {
@@ -195,7 +195,7 @@ hipError_t launch_relay_assign(const uint8_t *auth, const uint8_t *pass, const u
     const bool counting = !one_block && plan.fits && plan.bytes <= sort_tmp_bytes;
     const bool aligned = (((uintptr_t)auth | (uintptr_t)pass | (uintptr_t)verdict) & 3u) == 0 &&
                          (((uintptr_t)peer_out | (uintptr_t)keys) & 15u) == 0;
-    hipLaunchKernelGGL(aligned ? relay_verdict_kernel<true> : relay_verdict_kernel<false>, dim3((n + 1023u) / 1024u), dim3(256), 0, s,
+    hipLaunchKernelGGL(aligned ? relay_verdict_kernel<true> : relay_verdict_kernel<false>, dim3(n / 1024u + (n % 1024u != 0u)), dim3(256), 0, s,
                        auth, pass, peer_out, n_peers_out, n, keys, counting ? (uint32_t *)nullptr : idx, verdict, ctr_out, status);
     // (keys[] is the peer of each survivor and all ones for the rest)
     if (one_block)

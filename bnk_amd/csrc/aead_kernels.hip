@@ -768,8 +768,6 @@ BNK_DEV void body_short(uint8_t *tile, uint32_t lane, bool have, const uint8_t *
     static_assert(CELLS == 4 || CELLS == 8, "one data block or two");
     constexpr uint32_t ROW = short_row<CELLS>();
     constexpr int PER = 64 / CELLS; // packets per load
-    const uint32_t ncell_in = len_in >> 4; // see body_lines
-    const uint32_t ncell = len >> 4;       // whole cells, stored cooperatively
     const uint32_t sub = lane % CELLS;
     uint8_t *const move = tile + (lane / CELLS) * ROW + 16u * sub; // my cell of load 0's packet
     uint4 pre[CELLS];

@@ -152,16 +152,19 @@ static void serial_tag(const uint32_t (&otk)[16], const uint8_t *ct, uint32_t le
     mac.finish(tag);
 }
 
-// The same tag the way a few lanes compute it together: `runs` runs of q pieces of 128
-// bytes, each evaluated on its own, lifted to its place and added up.
-static void split_tag(const uint32_t (&otk)[16], const uint8_t *ct, uint32_t len, uint32_t q, uint32_t (&tag)[4])
+// The same tag the way a few lanes compute it together: runs of `reach` bytes, each evaluated on
+// its own, lifted to its place and added up.  key_run: the first run is the key block alone and
+// has nothing of the packet (a lane per block).
+static void split_tag(const uint32_t (&otk)[16], const uint8_t *ct, uint32_t len, uint32_t reach, bool key_run, uint32_t (&tag)[4])
 {
     uint32_t sum[5] = {0, 0, 0, 0, 0};
     Poly32 mac;
     uint32_t begin = 0;
+    bool first = true;
     do {
         mac.init(otk);
-        const uint32_t end = len - begin < 128 * q ? len : begin + 128 * q;
+        const uint32_t end = first && key_run ? 0u : len - begin < reach ? len : begin + reach;
+        first = false;
         for (uint32_t o = begin; o < end; o += 16) {
             uint8_t cell[16] = {0};
             memcpy(cell, ct + o, end - o < 16 ? end - o : 16);
@@ -185,7 +188,7 @@ static void run_spread()
     uint64_t st = 777;
     auto rnd = [&]() { st ^= st << 13; st ^= st >> 7; st ^= st << 17; return st; };
     std::vector<uint8_t> ct(SPREAD_MAX_LEN);
-    int bad = 0, bad_split = 0, cases = 0;
+    int bad = 0, bad_split = 0, bad_by_block = 0, cases = 0, cases_by_block = 0;
     auto check = [&](const uint32_t (&otk)[16], uint32_t len) {
         uint32_t a[4], b[4];
         spread_tag(otk, ct.data(), len, a);
@@ -193,8 +196,14 @@ static void run_spread()
         cases++;
         if (memcmp(a, b, 16) != 0) bad++;
         for (uint32_t q : {1u, 2u, 3u, 7u, 32u}) {
-            split_tag(otk, ct.data(), len, q, a);
+            split_tag(otk, ct.data(), len, 128 * q, false, a);
             if (memcmp(a, b, 16) != 0) bad_split++;
+        }
+        // a lane per block: up to 31 of data and the key's, 32 terms
+        if (len <= 31u * 64u) {
+            split_tag(otk, ct.data(), len, 64, true, a);
+            cases_by_block++;
+            if (memcmp(a, b, 16) != 0) bad_by_block++;
         }
     };
     // every length class around cell, block and lane boundaries, random keys
@@ -216,12 +225,13 @@ static void run_spread()
             if (key == 3) { otk[0] = 0x0fffffffu; otk[1] = otk[2] = otk[3] = 0x0ffffffcu;
                             otk[4] = otk[5] = otk[6] = otk[7] = 0xffffffffu; }
             for (auto &b : ct) b = data == 0 ? 0xff : data == 1 ? 0x00 : (uint8_t)rnd();
-            for (uint32_t len : {0u, 1u, 15u, 16u, 17u, 63u, 64u, 65u, 256u, 1420u, 1436u, 4000u, 4031u, 4032u})
+            for (uint32_t len : {0u, 1u, 15u, 16u, 17u, 63u, 64u, 65u, 256u, 1420u, 1436u, 1920u, 1921u, 1983u, 1984u, 4000u, 4031u, 4032u})
                 check(otk, len);
         }
     printf("spread tags: %d cases, %d differ from the serial form\n", cases, bad);
     expect(bad == 0, "one packet spread over the lanes of a wave");
     expect(bad_split == 0, "one packet split over a few lanes");
+    expect(cases_by_block > 300 && bad_by_block == 0, "one packet split over a lane per block");
 }
 
 int main()

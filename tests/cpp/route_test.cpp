@@ -1,7 +1,9 @@
 // CPU check of the host-side rules around a launch (bnk_amd/csrc): which packets lie in the
-// arena, which AEAD launch a batch gets, how many flow table slots may be claimed.  Prints PASS/FAIL lines; exit status is the number of failures.
+// arena, which AEAD launch a batch gets and how it is dealt out, how lengths are grouped, how many flow
+// table slots may be claimed.  Prints PASS/FAIL lines; exit status is the number of failures.
 #include <stdio.h>
 
+#include <algorithm>
 #include <deque>
 #include <initializer_list>
 #include <random>
@@ -136,6 +138,59 @@ static void room_per_packet()
         }
 }
 
+// Packets per wave of a split launch: what the kernel has lanes and LDS rows for; a lane for every block
+// where the rule counts on it (one common length, two packets of any lengths up to 1984 bytes, five of
+// up to twice the mean); and where a wave per packet ends, 5/8 of the knob.
+static void packets_per_wave()
+{
+    const uint32_t lens[1] = {0};
+    for (uint32_t n = 1; n <= 70000; n += 1 + n / 23)
+        for (uint32_t len : {0u, 1u, 60u, 64u, 65u, 100u, 124u, 128u, 129u, 300u, 500u, 600u, 1000u, 1420u, 1500u, 1984u, 5000u, 65535u})
+            for (int k = 0; k < 8; k++) {
+                AeadArgs a{};
+                a.spread_max = SPREAD_MAX_PACKETS;
+                a.n = n;
+                a.len = len;
+                a.lens = k & 1 ? lens : nullptr;
+                a.room = std::min(len + 16u, SPLIT_ROOM_MAX);
+                a.host_batch = (k & 2) != 0;
+                if (k & 4) { // (framing, which is split from the first packet on)
+                    a.wg.mode = WG_FUSE_ENCAP;
+                    a.in_skip = 16;
+                }
+                const uint32_t per = aead_split_packets(a);
+                if (per == 0) continue;
+                expect(per <= SPLIT_MAX_PACKETS, "no more packets than a wave has rows for");
+                expect(!aead_runs_spread(a), "one launch for a batch");
+                if (a.lens) {
+                    expect(per >= 2u, "packets of any lengths come in company");
+                    // up to 2048 packets a wave has a lane per block, of any two up to 1984 bytes or of five of
+                    // up to twice the mean
+                    if (per == 2u) expect(n <= 2u * SPLIT_ONE_BLOCK_WAVES && per * (1984u / 64u + 1u) <= 64u, "two of any lengths");
+                    else if (n <= 2u * SPLIT_ONE_BLOCK_WAVES)
+                        expect(per == SPLIT_ALWAYS_ONE && per * ((2u * a.room + 63u) / 64u + 1u) <= 64u, "five where twice the mean has room");
+                } else {
+                    const uint32_t blocks = (len + 63u) / 64u;
+                    const bool ahead = 150u + 920u < 275u * (blocks + 1u);
+                    const uint32_t fit = std::min(64u / (blocks + 1u), SPLIT_MAX_PACKETS);
+                    if (ahead && fit >= 2u && n <= fit * SPLIT_ONE_BLOCK_WAVES)
+                        expect(per == fit && per * (blocks + 1u) <= 64u, "a lane for every block of one common length");
+                }
+            }
+    for (uint32_t knob : {64u, 4096u, 16384u})
+        for (int k = 0; k < 2; k++) {
+            AeadArgs a{};
+            a.spread_max = knob;
+            a.lens = k ? lens : nullptr;
+            a.len = 20000; // (one common length ends it there only where packets are long)
+            a.room = SPLIT_ROOM_MAX;
+            a.n = 5u * knob / 8u;
+            expect(aead_runs_spread(a) && aead_split_packets(a) == 0, "a wave per packet up to 5/8 of the knob");
+            a.n++;
+            expect(!aead_runs_spread(a) && aead_split_packets(a) != 0, "and split from there");
+        }
+}
+
 // Grouping by length: a grid's threads, four packets each and round, cover the batch, none of them
 // begins beyond 2^32 - 1, and a block more would be one too many.
 static void length_grouping()
@@ -195,6 +250,7 @@ int main()
     fetched_batches_stay_with_the_lanes();
     framing_behind_a_header();
     room_per_packet();
+    packets_per_wave();
     length_grouping();
     for (uint32_t first_seq : {0u, 1000u, 0x7FFFFFFFu - 2000u, 0x80000001u, 0xFFFFFFFFu - 2000u}) claimed_slots(first_seq);
     if (!failures) printf("PASS launch rules\n");

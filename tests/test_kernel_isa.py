@@ -1,12 +1,12 @@
-"""What the compiler made of the lane-per-packet AEAD kernels, read from its assembly
-listing (no GPU needed: hipcc cross-compiles).
+"""What the compiler made of the AEAD kernels and of CheckInbound's, read from its assembly
+listings (no GPU needed: hipcc cross-compiles).
 
-The kernels prefetch a packet's next line while they work on the current one.  That only
+The lane-per-packet kernels prefetch a packet's next line while they work on the current one.  That only
 overlaps if no wait for *everything* in flight sits inside or right behind the group of
 loads that fetches the line.  The compiler has put one there before (to protect a register
 the last load of the group fills: the sealing launch then sat out a whole trip to memory in
 every step, 5 % of its time), and nothing but its listing shows it.  The same listing says
-whether a kernel spills registers, which at two waves per SIMD it must not."""
+whether a kernel spills registers, which at its number of waves per SIMD it must not."""
 import os
 import re
 import subprocess
@@ -20,6 +20,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 WAVE_KERNELS = ("_ZN3bnk16aead_wave_kernelILb0EEEvNS_8AeadArgsE", "_ZN3bnk16aead_wave_kernelILb1EEEvNS_8AeadArgsE")
 # the same loop over a run of a packet, with a few lanes per packet
 SPLIT_KERNELS = tuple("_ZN3bnk17aead_split_kernelILb%dEEEvNS_8AeadArgsE" % o for o in (0, 1))
+# short packets of one common length, by the 16-byte cells that they fill at most
+SHORT_KERNELS = {c: tuple("_ZN3bnk17aead_short_kernelILb%dELi%dEEEvNS_8AeadArgsE" % (o, c) for o in (0, 1)) for c in (4, 8)}
 # CheckInbound over plain headers, per-packet arrays, records; without and with a jump table
 CHECK_KERNELS = tuple("_ZN3bnk19filter_check_kernelILi%dELb%dEEEvNS_10FilterArgsE" % (f, j) for f in (0, 1, 2) for j in (0, 1))
 # seal, open, seal + framing, open + framing of a small batch: a wave per packet
@@ -68,13 +70,28 @@ def test_no_wait_for_everything_among_the_loads_of_a_line(listing, name):
     assert not bad, "s_waitcnt vmcnt(0) between the loads of a line at listing lines %r of %s" % (bad, name)
 
 
-@pytest.mark.parametrize("name", WAVE_KERNELS + SPLIT_KERNELS)
-def test_the_wave_kernels_spill_nothing(listing, name):
+def _registers(listing, name):
+    """vector registers, how many of them are spilled, bytes of scratch."""
     meta = listing[listing.index(".name:           " + name):]
     meta = meta[:meta.index(".wavefront_size")]
-    get = lambda key: int(re.search(r"\.%s:\s+(\d+)" % key, meta).group(1))  # noqa: E731
-    assert get("vgpr_spill_count") == 0 and get("private_segment_fixed_size") == 0
-    assert get("vgpr_count") <= 256  # two waves per SIMD
+    return tuple(int(re.search(r"\.%s:\s+(\d+)" % key, meta).group(1))
+                 for key in ("vgpr_count", "vgpr_spill_count", "private_segment_fixed_size"))
+
+
+# A SIMD has 512 registers per lane, handed out eight at a time: two waves of the general launches get
+# 256 each, five of short packets up to 64 bytes 96, four of up to 128 bytes 128, eight of CheckInbound 64.
+@pytest.mark.parametrize("name,most", [(k, 256) for k in WAVE_KERNELS + SPLIT_KERNELS] +
+                         [(k, m) for c, m in ((4, 96), (8, 128)) for k in SHORT_KERNELS[c]])
+def test_the_lane_kernels_spill_nothing(listing, name, most):
+    count, spilled, scratch = _registers(listing, name)
+    assert (spilled, scratch) == (0, 0) and count <= most
+
+
+@pytest.mark.parametrize("name", CHECK_KERNELS)
+def test_the_check_kernels_spill_nothing(filter_listing, name):
+    """(Scalar registers that do not fit go to a vector register's lanes; that one is among the 64.)"""
+    count, spilled, scratch = _registers(filter_listing, name)
+    assert (spilled, scratch) == (0, 0) and count <= 64
 
 
 @pytest.mark.parametrize("name", SPREAD_KERNELS)

@@ -386,9 +386,10 @@ BNK_DEV void body_generic(uint8_t *tile, uint32_t lane, const uint8_t *src, uint
 //
 // RUNS: the lane goes through a run of a packet instead of a whole one (see
 // aead_split_kernel).  Positions then count from src and dst, where keystream block
-// blk0 applies; a run begins with an even block, so the first one of a packet begins
-// 64 bytes before it, at the key block, with `lead` = 4 cells that are not the
-// packet's.  key_lane: the lane of the packet's first run, which hands out the
+// blk0 applies; the first run of a packet begins 64 bytes before it, at the key block,
+// with `lead` = 4 cells that are not the packet's.  A run of pieces of 128 bytes begins
+// with an even block; one_block: a run is a block, the first one of a packet its key
+// block alone.  key_lane: the lane of the packet's first run, which hands out the
 // one-time key.
 template <bool OPEN, bool ALIGNED, bool SHIFT = false, bool RUNS = false>
 BNK_DEV void body_lines(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_t *dst, uint32_t len,

@@ -309,7 +309,9 @@ struct Poly32 {
 
     // h = h * r + (w0, w1, w2, w3, top), top 0 or 1.
     //
-    // One carry chain per cell: each column's upper half is added into the next
+    // Additions go 32 bits at a time with an explicit carry (add-with-carry instructions on
+    // the GPU; written as 64-bit sums the compiler builds each zero-extended operand with a
+    // move first).  One carry chain per cell: each column's upper half is added into the next
     // column as it is, and what lies at and above 2^130 (known from the top column
     // and the upper half below it, before any carry) goes in at the bottom of the
     // same chain.  h4 stays below 6: (e4 & 3) and the chain's last carry and `top`.
@@ -343,9 +345,6 @@ struct Poly32 {
     }
 
     // One full 16-byte block (little-endian words w0..w3) with bit 128 set.
-    // Additions go 32 bits at a time with an explicit carry (add-with-carry
-    // instructions on the GPU; written as 64-bit sums the compiler builds each
-    // zero-extended operand with a move first).
     // The block runs at raised wave priority for the same reason as the rotates of
     // ChaCha20: nearly all of it is multiplies and carries, which a SIMD takes
     // from one wave at a time.

@@ -37,15 +37,41 @@ inline bool aead_runs_spread(const AeadArgs &a)
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
         return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
     }
-    // 2560 by default.  Pairs of launches of packets of 1 to 1420 bytes, us alone / with three
-    // streams at work, a wave per packet against split: 1500 23.7 / 11.0 against 29.0 / 10.9, 2000
-    // 25.1 / 14.0 against 29.6 / 12.2, 2500 29.6 / 17.2 against 30.9 / 11.6, 3000 31.2 / 20.5
-    // against 32.7 / 12.2 (3200, where the launch goes over the chip once more, 42 against 32);
-    // 3000 of 1420 33 / 21.3 against 32 / 12.5
+    // 2560 by default: where one stream no longer minds.  Pairs of launches, us alone with a wait behind
+    // each / in a row / with three streams at work, a wave per packet against split, packets of 1 to 1420
+    // bytes: 2000 36.1 / 24.7 / 13.7 against 38.0 / 27.3 / 11.6, 2300 41.0 / 29.4 / 15.7 against 40.4 / 30.0 /
+    // 11.5, 2561 41.2 / 29.6 / 17.4 against 40.4 / 30.0 / 11.6, 2700 41.8 / 30.2 / 18.4 against 40.7 / 30.4 / 11.7, 3000
+    // 42.5 / 31.0 / 20.3 against 41.0 / 30.6 / 11.8; all of 1420 bytes 2300 41.9 / 30.3 against 41.2 / 30.8, 2561
+    // 42.5 / 31.1 against 41.3 / 30.9; IMIX as mixed lengths; of 1 to 600 bytes split is ahead from 2000 on
+    // (35.1 / 23.6 / 13.0 against 34.8 / 24.2 / 9.2).  Runs of one side differ by up to 1.3 alone and 0.9 in a row.
+    // (With several streams alone in view it would end below 2000.)
     const uint64_t most = 5ull * a.spread_max / 8;
     if (a.lens) return a.n <= most;
     return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);
 }
+
+// Room per packet: what the batch's packets take up on average in an arena that just holds them,
+// as far as the host can tell.  From the lengths themselves where it has them (16 bytes more, for
+// a tag and for the gaps between slots); of a batch in GPU memory it knows the stride, or else
+// only the arena, which may hold far more than the batch: room is then too large, and a wave gets
+// fewer packets than would fit.
+constexpr uint32_t SPLIT_ROOM_MAX = 1500; // beyond it one rule holds
+inline uint32_t aead_room(const bnk_batch &b)
+{
+    if (!b.lens || b.n == 0) return 0;
+    uint64_t all = b.bytes;
+    if (b.mem == BNK_MEM_HOST) {
+        all = 16ull * b.n;
+        for (uint32_t i = 0; i < b.n; i++) all += b.lens[i];
+    } else if (!b.offsets) {
+        all = std::min(all, (uint64_t)b.n * b.stride);
+    }
+    return (uint32_t)std::min<uint64_t>(all / b.n, SPLIT_ROOM_MAX);
+}
+
+constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
+constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
+constexpr uint32_t SPLIT_ONE_BLOCK_WAVES = 1024; // a wave per SIMD
 
 // Packets per wave of the launch that splits packets over lanes, 0 where a launch of
 // a lane per packet is the better one.
@@ -94,29 +120,6 @@ inline bool aead_runs_spread(const AeadArgs &a)
 // a wave, 8000 of 600 five to a wave 32.1 / 19.4 against 33.1 / 13.8.  (Not for one or two blocks
 // of data: 4000 of 60 bytes 22.2 / 8.5 against 15.8 / 7.8 a lane per packet, 20000 of 124 28.4 / 12.1
 // against 27.3 / 10.6.)
-
-// Room per packet: what the batch's packets take up on average in an arena that just holds them,
-// as far as the host can tell.  From the lengths themselves where it has them (16 bytes more, for
-// a tag and for the gaps between slots); of a batch in GPU memory it knows the stride, or else
-// only the arena, which may hold far more than the batch: room is then too large, and a wave gets
-// fewer packets than would fit.
-constexpr uint32_t SPLIT_ROOM_MAX = 1500; // beyond it one rule holds
-inline uint32_t aead_room(const bnk_batch &b)
-{
-    if (!b.lens || b.n == 0) return 0;
-    uint64_t all = b.bytes;
-    if (b.mem == BNK_MEM_HOST) {
-        all = 16ull * b.n;
-        for (uint32_t i = 0; i < b.n; i++) all += b.lens[i];
-    } else if (!b.offsets) {
-        all = std::min(all, (uint64_t)b.n * b.stride);
-    }
-    return (uint32_t)std::min<uint64_t>(all / b.n, SPLIT_ROOM_MAX);
-}
-
-constexpr uint32_t SPLIT_MAX_PACKETS = 32; // per wave
-constexpr uint32_t SPLIT_ALWAYS_ONE = 5;
-constexpr uint32_t SPLIT_ONE_BLOCK_WAVES = 1024;
 inline uint32_t aead_split_packets(const AeadArgs &a)
 {
     // (spread_max 0 asks for a lane per packet; order[] is only built for that launch)

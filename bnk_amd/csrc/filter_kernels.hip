@@ -325,7 +325,8 @@ struct RawHeader {
 // registers do not fit and are fetched out of vector registers lane by lane wherever they are used
 // (278 places; 2^22 plain headers: 510 vector and 280 scalar instructions per 64 packets).  What still
 // does not fit, with a jump table: 20 registers of plain headers (25 places), 34 of records (62), 56 of
-// arrays (144), few of them on a packet's usual way.
+// arrays (144).  (The launch over records became a fifth faster with as many, see rules_match_quad:
+// it does not wait for those.)
 enum HeaderFrom { FROM_PLAIN, FROM_ARRAYS, FROM_RECORDS };
 
 // The loads of one packet, every one issued whether or not the lane needs it (from `safe`, 32
@@ -412,9 +413,9 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     // bytes per lane and load, all of them in flight together (word by word, each waited for:
     // 3 us more for 2^22 packets, 1 for 2^14).
     //
-    // What bounds the launch: 8 waves per SIMD, of whose time half is spent waiting for memory
-    // (a packet's rule list, presence word and flow slot come from L2 and beyond, one behind the
-    // other) and a third waiting to issue, half of the VALU's slots taken.  So both count, the
+    // What bounds the launch: 8 waves per SIMD, of whose time more than half is spent waiting for
+    // memory (a packet's rule list, presence word and flow slot come from L2 and beyond, one behind
+    // the other) and a quarter waiting to issue, half of the VALU's slots taken.  So both count, the
     // instructions and the order in which memory is asked: 2^22 plain headers on 4096 rules and
     // 65,536 flows took 79.3 us with 510 vector and 280 scalar instructions per 64 packets, the
     // rule lists fetched a word at a time as the tests before it failed; compiled per kind of

@@ -1418,8 +1418,8 @@ def test_full_size_tunnel_round_trips_device_resident():
 @pytest.mark.parametrize("plen", [20, 40, 60, 100, 113])
 def test_short_uniform_tunnel_batches_device_resident(plen):
     """Device-resident batches of short packets of one common length: the
-    launches in which every wave takes the short path (three waves per SIMD)
-    also do the framing -- header, padding as implied zeros, wire lengths on the
+    launches in which every wave takes the short path (five waves per SIMD up to
+    64 bytes, four up to 128) also do the framing -- header, padding as implied zeros, wire lengths on the
     way out; header checks, index lookup and the checks on the inner header on
     the way in.  Every datagram against the oracle, then decapsulated in line
     with the ciphertext, a forged one and a repeat among them."""

@@ -1465,14 +1465,135 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
 }
 
+// Value of x in lane A, B, C or D of the lane's quad, for its first to fourth lane.
+template <int A, int B, int C, int D>
+BNK_DEV uint32_t quad_from(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, A | B << 2 | C << 4 | D << 6, 0xF, 0xF, true);
+}
+
+// ChaCha20 blocks first .. first + 16 S - 1 of a packet into the rows of `stage`, four lanes a
+// block and S blocks a quad of lanes, side by side.  The lane holds column `lane & 3` of the state,
+// whose words 4.. and 8.. start out as key_b and key_c.
+template <int S>
+BNK_DEV void quad_blocks(uint8_t *stage, uint32_t lane, uint32_t key_b, uint32_t key_c, uint32_t first, uint32_t n1,
+                         uint32_t n2)
+{
+    const uint32_t quad = lane & 3u, row = first + (lane >> 2);
+    const uint32_t sigma = quad < 2u ? (quad == 0u ? 0x61707865u : 0x3320646eu) : quad == 2u ? 0x79622d32u : 0x6b206574u;
+    uint32_t a[S], b[S], c[S], d[S], d0[S];
+    // Rows 1, 2 and 3 move up by one, two and three lanes to make columns of the diagonals; they
+    // enter and leave the loop moved, so that in it every move is part of an addition or a xor.
+    auto diagonal = [&](int s) __attribute__((always_inline)) {
+        b[s] = quad_from<1, 2, 3, 0>(b[s]);
+        c[s] = quad_from<2, 3, 0, 1>(c[s]);
+        d[s] = quad_from<3, 0, 1, 2>(d[s]);
+    };
+    auto columns = [&](int s) __attribute__((always_inline)) {
+        b[s] = quad_from<3, 0, 1, 2>(b[s]);
+        c[s] = quad_from<2, 3, 0, 1>(c[s]);
+        d[s] = quad_from<1, 2, 3, 0>(d[s]);
+    };
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        a[s] = sigma;
+        b[s] = key_b;
+        c[s] = key_c;
+        d[s] = d0[s] = quad < 2u ? (quad == 0u ? row + 16u * s : 0u) : quad == 2u ? n1 : n2;
+        diagonal(s);
+    }
+    auto rounds = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < S; s++) { a[s] += b[s]; d[s] = rotl32(d[s] ^ a[s], 16); }
+#pragma unroll
+        for (int s = 0; s < S; s++) { c[s] += d[s]; b[s] = rotl32(b[s] ^ c[s], 12); }
+#pragma unroll
+        for (int s = 0; s < S; s++) { a[s] += b[s]; d[s] = rotl32(d[s] ^ a[s], 8); }
+#pragma unroll
+        for (int s = 0; s < S; s++) { c[s] += d[s]; b[s] = rotl32(b[s] ^ c[s], 7); }
+    };
+#pragma unroll 1
+    for (int r = 0; r < 10; r++) {
+#pragma unroll
+        for (int s = 0; s < S; s++) columns(s);
+        rounds();
+#pragma unroll
+        for (int s = 0; s < S; s++) diagonal(s);
+        rounds();
+    }
+#pragma unroll
+    for (int s = 0; s < S; s++) {
+        columns(s);
+        uint32_t *to = reinterpret_cast<uint32_t *>(stage + (row + 16u * s) * LDS_ROW) + quad;
+        to[0] = a[s] + sigma;
+        to[4] = b[s] + key_b;
+        to[8] = c[s] + key_c;
+        to[12] = d[s] + d0[s];
+    }
+}
+
+// A value that is the same in every lane, as a scalar.
+BNK_DEV uint32_t wave_value(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+// For cell number `lane` mod 64 of a packet's `cells` (a scalar): r^(1 + cells behind the last such cell), and
+// r^64 in `top` where a lane has more than one.
+//
+// A lane multiplies what it has by r^(2^b) where bit b of its number of cells behind is set.  A lane
+// whose lower bits are all set then holds r^(2^b * 2), the next step's multiplier: no squaring.  (Every
+// residue is some lane's, whether or not that lane has a cell.)
+BNK_DEV Fe26 wave_powers(const Fe26 &r, uint32_t cells, uint32_t lane, Fe26 &top)
+{
+    const uint32_t behind = cells - 1u - lane;
+    const uint32_t most = cells > 64u ? 63u : cells ? cells - 1u : 0u;
+    Fe26 lift = r;
+    top = Fe26{wave_value(r.v0), wave_value(r.v1), wave_value(r.v2), wave_value(r.v3), wave_value(r.v4)};
+#pragma unroll 1
+    for (uint32_t bit = 1; bit <= most; bit <<= 1) {
+        lift = fe_select((behind & bit) != 0u, fe_mul(lift, top), lift);
+        const int from = (int)((cells - 2u * bit) & 63u);
+        top = Fe26{(uint32_t)__builtin_amdgcn_readlane((int)lift.v0, from), (uint32_t)__builtin_amdgcn_readlane((int)lift.v1, from),
+                   (uint32_t)__builtin_amdgcn_readlane((int)lift.v2, from), (uint32_t)__builtin_amdgcn_readlane((int)lift.v3, from),
+                   (uint32_t)__builtin_amdgcn_readlane((int)lift.v4, from)};
+    }
+    return lift;
+}
+
+// The sum of x over lanes 0..31 in lane 31, over lanes 32..63 in lane 63.
+BNK_DEV uint32_t half_wave_sum(uint32_t x)
+{
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xF, 0xF, true); // from 1 lane below, within 16
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true); // 2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true); // 4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true); // 8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, true); // last lane of the 16 before
+    return x;
+}
+
 // One wave = one packet, for batches too small to fill the chip with a packet
 // per lane (there a call lasts as long as one lane needs for a whole packet:
-// about 85 us at 1420 bytes, however few the packets).  Lane 0 computes
-// ChaCha20 block 0 and owns the length block, lane l >= 1 computes block l and
-// moves bytes [64(l-1), 64l) of the packet; the tag is the sum of the lanes'
-// terms (aead_lane.hpp).  All loads of a packet are issued before any store,
-// and a lane stores only what it loaded, so sealing in place is safe.  A
-// packet longer than 63 blocks is done by lane 0 alone, the per-lane way.
+// about 85 us at 1420 bytes, however few the packets).
+//
+// What bounds it is one wave's chain of instructions, one every five cycles whatever
+// its lanes have to do, behind a trip to the packet (over the link, for a host batch).
+// So the chain is as short as the wave can make it, and most of it lies ahead of the
+// packet's arrival:
+// * Four lanes compute a ChaCha20 block, a column each, which become diagonals as the
+//   additions and xors take a neighbour's word (DPP): sixteen blocks in 300 instructions
+//   where a block per lane takes 990, and 24 blocks in 540.  Block 0 is the one-time key.
+// * The keystream goes into LDS.  A cell of 16 bytes of it is read by the lane that has
+//   fetched that cell of the packet (lane l has bytes [16 l, 16 l + 16) of each KB) and
+//   stores it: the packet itself never goes through LDS.
+// * The lane multiplies its cells, 64 apart, by r^64 as it goes along and the result by
+//   r^(1 + cells behind its last one), at most r^64.  Both powers are there before the
+//   packet is (wave_powers), so what follows its arrival is a multiplication per KB, the
+//   sum over the lanes and the tag.
+// Calls that seal and open 1 packet of 1420 bytes in pinned rings 34.5 -> 26.9 us (a block and
+// four cells in a row per lane, each lane's powers by squaring, before), 128 packets through the
+// tunnel 74.7 -> 66.7; launches of 1000 packets in GPU memory 13.2 -> 7.4 us, of 2000 17.4 -> 10.1.
+// (All arguments fetched at once, or the per-packet entries by scalar loads: no different.)
+// All loads of a packet are issued before any store, and a lane stores only what it
+// loaded, so sealing in place is safe.  A packet longer than 63 blocks is done by lane 0
+// alone, the per-lane way.
 //
 // With WG set the wave also does the packet's WireGuard framing (a.wg): on the
 // way out it writes the transport header and treats the bytes between the
@@ -1532,8 +1653,8 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         }
     }
 
-    // ---- my 64 bytes: loads first, they fly while everything below is looked
-    // up and the block is computed.  Where the AEAD data lies and how long it
+    // ---- my cells: loads first, they fly while everything below is looked
+    // up and the keystream is computed.  Where the AEAD data lies and how long it
     // is follows from the length alone, so the loads need not wait for the
     // header, the index search or the key; a packet that is then turned away
     // has loaded bytes of its own datagram for nothing.
@@ -1551,26 +1672,22 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         data_len = (len >= 32u && len - 32u <= WG_FUSE_MAX_LEN) ? len - 32u : 0u;
         data_there = data_len;
     }
-    const uint32_t at = 64u * (lane - 1u);
-    const uint32_t mine = (lane == 0 || at >= data_len) ? 0u : min(data_len - at, 64u);
-    const uint32_t there = (lane == 0 || at >= data_there) ? 0u : min(data_there - at, 64u);
     // The wave fetches the packet in pieces of 1 KB, lane l taking bytes [16 l,
-    // 16 l + 16) of each piece, so that an instruction reads 1 KB in a row; the
-    // lanes pick their own 64-byte blocks out of LDS further down.  (A lane
-    // fetching its own block reads 16 bytes every 64: sixty-four small requests
-    // an instruction, which a packet that lies in host memory pays for with a
-    // read of its own over the link for each.)
+    // 16 l + 16) of each piece, so that an instruction reads 1 KB in a row (64
+    // bytes a lane would be sixty-four small requests an instruction, each of
+    // them a read of its own over the link for a packet in host memory).
     // What the packet's bytes wait for goes out ahead of them, so that a wait for it does
     // not wait for them as well (a wave's loads complete in the order they were issued): the
     // sender's key where the sender is known by now, with the receiver's index for the
     // header on the way out; on the way in the header, which names the sender.
-    uint4 key_lo = make_uint4(0, 0, 0, 0), key_hi = key_lo, wg_head = key_lo;
+    const uint32_t quad = lane & 3u; // the lane's column of its ChaCha20 block
+    uint32_t key_b = 0, key_c = 0;   // and its words of the key
+    uint4 wg_head = make_uint4(0, 0, 0, 0);
     uint32_t wg_remote = 0;
     if (!(WG && OPEN)) {
         const uint32_t known = pr < (WG ? a.wg.n_peers : a.n_peers) ? pr : 0u; // (the table has a row 0)
-        const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * known);
-        key_lo = kp[0];
-        key_hi = kp[1];
+        key_b = a.keys[8u * known + quad];
+        key_c = a.keys[8u * known + 4u + quad];
         if (WG) wg_remote = a.wg.remote_index[known];
     } else {
         wg_head = ld16(len >= 32u && len - 32u <= WG_FUSE_MAX_LEN ? src : safe);
@@ -1668,21 +1785,18 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         len -= 32u; // header and tag
         src += 16;
     }
-    uint32_t k[8];
-    {
-        if (WG && OPEN) { // (the sender has only now been found)
-            const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * pr);
-            key_lo = kp[0];
-            key_hi = kp[1];
-        }
-        k[0] = key_lo.x; k[1] = key_lo.y; k[2] = key_lo.z; k[3] = key_lo.w;
-        k[4] = key_hi.x; k[5] = key_hi.y; k[6] = key_hi.z; k[7] = key_hi.w;
+    if (WG && OPEN) { // (the sender has only now been found)
+        key_b = a.keys[8u * pr + quad];
+        key_c = a.keys[8u * pr + 4u + quad];
     }
     const uint32_t n1 = (uint32_t)ctr, n2 = (uint32_t)(ctr >> 32);
-    uint32_t x[16];
 
     if (!WG && len > SPREAD_MAX_LEN) {
         const bool have = lane == 0;
+        const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * pr);
+        const uint4 k0 = kp[0], k1 = kp[1];
+        const uint32_t k[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+        uint32_t x[16];
         Poly32 mac;
         Head no_head;
         no_head.on = false;
@@ -1693,69 +1807,67 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         return;
     }
 
-    // (the packet's bytes are already on their way: see the top of the kernel)
-    chacha_block(k, lane, n1, n2, x);
-    // Block b of the packet lies at stage + 80 b (rows padded against bank
-    // conflicts): written in the order the pieces came in, read a block per lane.
-    uint8_t *stage = tile_all[threadIdx.x >> 6];
-    if (!tagged) want_tag = make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t off = 1024u * j + 16u * lane;
-        // a cell beyond the packet's whole cells is zeros, but for its last 1-15 bytes
-        if (off + 16u > data_there) pre[j] = make_uint4(0, 0, 0, 0);
-        if (odd_mine && (odd_at >> 10) == (uint32_t)j) pre[j] = odd_cell;
-        if (1024u * j < data_there)
-            *reinterpret_cast<uint4 *>(stage + (16u * j + (lane >> 2)) * LDS_ROW + 16u * (lane & 3u)) = pre[j];
+    // ---- the keystream, block 0 and those of the data (they fly: see the top of the kernel) ----
+    // Block b lies at stage + 80 b (rows padded against bank conflicts).
+    uint8_t *const stage = tile_all[threadIdx.x >> 6];
+    const uint32_t passes = (len + 63u) / 64u / 16u + 1u; // of sixteen blocks
+    if (passes == 1u) {
+        quad_blocks<1>(stage, lane, key_b, key_c, 0u, n1, n2);
+    } else {
+        quad_blocks<2>(stage, lane, key_b, key_c, 0u, n1, n2);
+        if (passes > 2u) quad_blocks<2>(stage, lane, key_b, key_c, 32u, n1, n2);
     }
     wave_sync();
-    uint32_t m[16];
+    uint32_t x[16];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        uint4 v = make_uint4(0, 0, 0, 0);
-        // (bytes of a cell beyond the data were fetched as zeros)
-        if (there > 16u * j) v = *reinterpret_cast<const uint4 *>(stage + (lane - 1u) * LDS_ROW + 16u * j);
-        m[4 * j] = v.x; m[4 * j + 1] = v.y; m[4 * j + 2] = v.z; m[4 * j + 3] = v.w;
+    for (int j = 0; j < 2; j++) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(stage + 16 * j);
+        x[4 * j] = v.x; x[4 * j + 1] = v.y; x[4 * j + 2] = v.z; x[4 * j + 3] = v.w;
     }
-    // the one-time key is lane 0's block
-    const Fe26 r = fe_clamped_r((uint32_t)__builtin_amdgcn_readlane((int)x[0], 0),
-                                (uint32_t)__builtin_amdgcn_readlane((int)x[1], 0),
-                                (uint32_t)__builtin_amdgcn_readlane((int)x[2], 0),
-                                (uint32_t)__builtin_amdgcn_readlane((int)x[3], 0));
-    const uint32_t pad[4] = {(uint32_t)__builtin_amdgcn_readlane((int)x[4], 0),
-                             (uint32_t)__builtin_amdgcn_readlane((int)x[5], 0),
-                             (uint32_t)__builtin_amdgcn_readlane((int)x[6], 0),
-                             (uint32_t)__builtin_amdgcn_readlane((int)x[7], 0)};
+    Poly32 mac;
+    mac.init(x);
+    // ---- the powers of r that my cells take: r^64 from one to the next, r^(1 + cells behind it) the last ----
+    const uint32_t cells = wave_value((len + 15u) >> 4); // (the same in every lane)
+    Fe26 top; // r^64 where a lane has a second cell
+    const Fe26 lift = wave_powers(fe_clamped_r(mac.r0, mac.r1, mac.r2, mac.r3), cells, lane, top);
 
     // ---- crypt: o = m ^ keystream; the MAC reads the ciphertext side ----
-    uint32_t o[16];
+    if (!tagged) want_tag = make_uint4(0, 0, 0, 0);
+    uint4 o[4] = {};
+    Fe26 acc = fe_small(0);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        uint4 v = make_uint4(m[4 * j] ^ x[4 * j], m[4 * j + 1] ^ x[4 * j + 1], m[4 * j + 2] ^ x[4 * j + 2],
-                             m[4 * j + 3] ^ x[4 * j + 3]);
-        const uint32_t have_b = mine > 16u * j ? min(mine - 16u * j, 16u) : 0u;
-        v = keep_bytes(v, have_b);
-        o[4 * j] = v.x; o[4 * j + 1] = v.y; o[4 * j + 2] = v.z; o[4 * j + 3] = v.w;
+        if (64u * j >= cells) break; // (the same for the whole wave)
+        const uint32_t off = 1024u * j + 16u * lane;
+        uint4 m = pre[j];
+        // a cell beyond the packet's whole cells is zeros, but for its last 1-15 bytes
+        if (off + 16u > data_there) m = make_uint4(0, 0, 0, 0);
+        if (odd_mine && (odd_at >> 10) == (uint32_t)j) m = odd_cell;
+        const uint4 ks = *reinterpret_cast<const uint4 *>(stage + (1u + 16u * j + (lane >> 2)) * LDS_ROW + 16u * quad);
+        o[j] = make_uint4(m.x ^ ks.x, m.y ^ ks.y, m.z ^ ks.z, m.w ^ ks.w);
+        if (64u * (j + 1u) >= cells && (len & 15u) != 0u) // the last cell is among these
+            o[j] = o[j] & byte_mask(64u * j + lane == cells - 1u ? len & 15u : 16u);
+        const uint4 mine = OPEN ? m : o[j];
+        Fe26 next = fe_cell(mine.x, mine.y, mine.z, mine.w);
+        if (j != 0) next = fe_add(fe_mul(acc, top), next);
+        acc = fe_select(64u * j + lane < cells, next, acc);
     }
-    if (lane == 0) {
-        // LE64(len(aad) = 0) || LE64(len(ciphertext)) as my only cell
-        m[0] = 0; m[1] = 0; m[2] = len; m[3] = 0;
-        o[0] = 0; o[1] = 0; o[2] = len; o[3] = 0;
-    }
-    const SpreadShare sh = spread_share(lane, len);
-    const Fe26 term = spread_term(r, OPEN ? m : o, sh.k, sh.e, spread_e_max(len));
+    const Fe26 term = fe_mul(acc, lift);
 
-    // ---- add the 64 terms: 32 lanes fit 32 bits per limb, the last step is wider ----
-    uint32_t t32[5] = {term.v0, term.v1, term.v2, term.v3, term.v4};
-#pragma unroll
-    for (int step = 1; step < 32; step <<= 1)
-#pragma unroll
-        for (int q = 0; q < 5; q++) t32[q] += (uint32_t)__shfl_xor((int)t32[q], step, 64);
+    // ---- the sum of the lanes' terms: 32 lanes fit 32 bits per limb ----
+    const uint32_t limb[5] = {term.v0, term.v1, term.v2, term.v3, term.v4};
     uint64_t sum[5];
 #pragma unroll
-    for (int q = 0; q < 5; q++) sum[q] = (uint64_t)t32[q] + (uint32_t)__shfl_xor((int)t32[q], 32, 64);
+    for (int q = 0; q < 5; q++) {
+        const uint32_t v = half_wave_sum(limb[q]);
+        sum[q] = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)v, 31) + (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+    }
+    // LE64(len(aad) = 0) || LE64(len(ciphertext)), the last cell, with its bit 128
+    sum[2] += (uint64_t)len << 12;
+    sum[4] += 1u << 24;
+    split_join(mac, sum);
     uint32_t tag[4];
-    spread_finish(sum, pad, tag);
+    mac.finish(tag);
 
     bool reject = false;
     if (!OPEN) {
@@ -1772,10 +1884,10 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     if (WG && OPEN) {
         // ---- what wireguard-go checks once a packet is authentic: keepalive, IP
         // version, length fields, source inside the sender's allowed prefix.  The
-        // first 16 plaintext bytes (lane 1's first cell) hold every field used.
-        const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)o[0], 1);
-        const uint32_t w1 = (uint32_t)__builtin_amdgcn_readlane((int)o[1], 1);
-        const uint32_t w3 = (uint32_t)__builtin_amdgcn_readlane((int)o[3], 1);
+        // first 16 plaintext bytes (lane 0's first cell) hold every field used.
+        const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].x, 0);
+        const uint32_t w1 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].y, 0);
+        const uint32_t w3 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].w, 0);
         uint8_t res = BNK_WG_OK;
         uint32_t inner = 0;
         const uint32_t version = (w0 >> 4) & 0xFu;
@@ -1802,23 +1914,15 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
             a.wg.counter_out[i] = ctr;
         }
     }
-    // ---- the bytes out, the way they came in: blocks into LDS, pieces of 1 KB in
-    // a row out of it; a rejected packet leaves zeros (chacha20poly1305.Open) ----
-    wave_sync();
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint4 v = reject ? make_uint4(0, 0, 0, 0)
-                               : make_uint4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
-        if (mine > 16u * j) *reinterpret_cast<uint4 *>(stage + (lane - 1u) * LDS_ROW + 16u * j) = v;
-    }
-    wave_sync();
+    // ---- the bytes out, the way they came in; a rejected packet leaves zeros
+    // (chacha20poly1305.Open) ----
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const uint32_t off = 1024u * j + 16u * lane;
-        if (1024u * j < data_len && off < data_len) {
-            const uint4 v = *reinterpret_cast<const uint4 *>(stage + (16u * j + (lane >> 2)) * LDS_ROW + 16u * (lane & 3u));
-            if (off + 16u <= data_len) st16(dst + off, v);
-            else st_partial(dst + off, v, data_len - off);
+        if (off < len) {
+            const uint4 v = reject ? make_uint4(0, 0, 0, 0) : o[j];
+            if (off + 16u <= len) st16(dst + off, v);
+            else st_partial(dst + off, v, len - off);
         }
     }
 }

@@ -385,13 +385,13 @@ struct Poly32 {
 // ---------------------------------------------------------------------------
 // One packet spread over the lanes of a wave (small batches, where a packet
 // per lane would leave the chip empty and a call would last as long as one
-// lane takes for a whole packet).  Lane 0 runs ChaCha20 block 0 (the one-time
-// key) and owns the AEAD length block, lane l >= 1 owns keystream block l and
-// its four 16-byte cells.  With C MAC cells m_0 .. m_{C-1} the tag is
+// lane takes for a whole packet).  With C MAC cells m_0 .. m_{C-1} the tag is
 // sum m_j r^(C-j) + s: each lane evaluates its own cells by Horner's rule,
 // lifts the result by r^(cells after its last one), and the lanes' terms are
 // added.  General multipliers (powers of r are not clamped) need the radix
-// 2^26 form.
+// 2^26 form.  The kernel's lanes take every 64th cell; four in a row each (spread_term),
+// as when a lane computed a block of the keystream for itself, is kept as a
+// cross-check.
 // ---------------------------------------------------------------------------
 
 // Element of GF(2^130 - 5), five limbs of 26 bits; arithmetic keeps limbs
@@ -554,9 +554,9 @@ BNK_DEV Fe26 split_value(const Poly32 &p)
                 funnel(p.h3, p.h2, 14) & 0x3ffffffu, (p.h3 >> 8) | (p.h4 << 24)};
 }
 
-// The sum of up to 32 lifted terms (limb by limb, each below 2^32) back into the
-// accumulator: the length block and the pad follow as for a packet of one lane.
-BNK_DEV void split_join(Poly32 &p, const uint32_t (&sum)[5])
+// The sum of up to 64 lifted terms (limb by limb) back into the accumulator: the
+// length block and the pad follow as for a packet of one lane.
+BNK_DEV void split_join(Poly32 &p, const uint64_t (&sum)[5])
 {
     uint64_t t0 = sum[0], t1 = sum[1], t2 = sum[2], t3 = sum[3], t4 = sum[4];
 #pragma unroll
@@ -573,6 +573,13 @@ BNK_DEV void split_join(Poly32 &p, const uint32_t (&sum)[5])
     p.h2 = (uint32_t)w; w = (w >> 32) + (t4 << 8);
     p.h3 = (uint32_t)w;
     p.h4 = (uint32_t)(w >> 32); // at most 4
+}
+
+// The same for up to 32 terms, whose sums fit 32 bits.
+BNK_DEV void split_join(Poly32 &p, const uint32_t (&sum)[5])
+{
+    const uint64_t wide[5] = {sum[0], sum[1], sum[2], sum[3], sum[4]};
+    split_join(p, wide);
 }
 
 } // namespace bnk

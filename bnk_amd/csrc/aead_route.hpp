@@ -11,12 +11,12 @@ namespace bnk {
 
 // Which launch?  Packets in GPU memory (us per launch of n packets in a row, all of
 // them resident at once; seal and open within 2 us of each other):
-//   a wave per packet   9 + 4.2 per 1000 packets at 1420 bytes, 3.3 at 60
+//   a wave per packet   4.5 + 3.0 per 1000 packets at 1420 bytes, 2.1 at 60
 //   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2), 3 less than
 //                       with q = 1 where every block gets a lane of its own
 //   a lane per packet   5 + 2.75 per ChaCha20 block of the longest packet, and 20 more
 //                       for the grouping where lengths vary
-// so 4096 packets x 1420 take 21 / 18 / 71 us, 16384 66 / 26 / 71, and 24000 packets of 1
+// so 4096 packets x 1420 take 17 / 17 / 71 us, 16384 54 / 26 / 71, and 24000 packets of 1
 // to 1420 bytes - / 35 / 97.
 //
 // Packets in host memory (over_link): a wave per packet reads them where they are, the
@@ -37,14 +37,12 @@ inline bool aead_runs_spread(const AeadArgs &a)
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
         return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
     }
-    // 2560 by default: where one stream no longer minds.  Pairs of launches, us alone with a wait behind
-    // each / in a row / with three streams at work, a wave per packet against split, packets of 1 to 1420
-    // bytes: 2000 36.1 / 24.7 / 13.7 against 38.0 / 27.3 / 11.6, 2300 41.0 / 29.4 / 15.7 against 40.4 / 30.0 /
-    // 11.5, 2561 41.2 / 29.6 / 17.4 against 40.4 / 30.0 / 11.6, 2700 41.8 / 30.2 / 18.4 against 40.7 / 30.4 / 11.7, 3000
-    // 42.5 / 31.0 / 20.3 against 41.0 / 30.6 / 11.8; all of 1420 bytes 2300 41.9 / 30.3 against 41.2 / 30.8, 2561
-    // 42.5 / 31.1 against 41.3 / 30.9; IMIX as mixed lengths; of 1 to 600 bytes split is ahead from 2000 on
-    // (35.1 / 23.6 / 13.0 against 34.8 / 24.2 / 9.2).  Runs of one side differ by up to 1.3 alone and 0.9 in a row.
-    // (With several streams alone in view it would end below 2000.)
+    // 2560 by default: where several streams no longer gain by it.  Pairs of launches, us alone with a
+    // wait behind each / in a row / with three streams at work, a wave per packet against split, packets of
+    // 1 to 1420 bytes: 1000 24.9 / 13.9 / 7.7 against 36.4 / 24.9 / 9.7, 2000 29.5 / 18.7 / 9.7 against 38.8 /
+    // 27.5 / 12.7, 2500 33.6 / 22.3 / 11.7 against 41.7 / 30.1 / 12.1, 3000 35.1 / 23.9 / 13.6 against 42.4 /
+    // 30.7 / 12.4, 4096 41.7 / 31.0 / 17.6 against 42.7 / 31.7 / 13.5; IMIX and one length of 1420 bytes cross
+    // at the same place; of 1 to 600 bytes three streams are even at 2000 and 0.9 apart at 2500.
     const uint64_t most = 5ull * a.spread_max / 8;
     if (a.lens) return a.n <= most;
     return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);

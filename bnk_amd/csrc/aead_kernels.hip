@@ -159,6 +159,7 @@ BNK_DEV uint4 byte_mask(uint32_t m)
     const uint64_t lo = m >= 8u ? ~0ull : some, hi = m >= 16u ? ~0ull : m >= 8u ? some : 0ull;
     return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
 }
+BNK_DEV uint4 operator^(uint4 a, uint4 b) { return make_uint4(a.x ^ b.x, a.y ^ b.y, a.z ^ b.z, a.w ^ b.w); }
 BNK_DEV uint4 operator&(uint4 a, uint4 b) { return make_uint4(a.x & b.x, a.y & b.y, a.z & b.z, a.w & b.w); }
 
 BNK_DEV uint64_t shfl64(uint64_t v, int src_lane)
@@ -178,8 +179,7 @@ BNK_DEV void wave_sync()
 }
 
 // One wave = 64 packets, one lane per packet for the arithmetic.  Memory is
-// touched cooperatively through a per-wave LDS tile (body_lines, body_short,
-// body_generic).
+// touched cooperatively through a per-wave LDS tile (body_lines, body_short).
 //
 // Line path (every packet of the wave 16-byte aligned, source and destination
 // at the same offset within a 128-byte line): the wave moves whole aligned
@@ -196,11 +196,7 @@ BNK_DEV void wave_sync()
 // packet itself, at whatever alignment it has; where every destination of the
 // wave is 4-byte aligned the output still leaves as whole aligned cells of the
 // destination's lines (see body_lines).
-//
-// Generic path (packets beyond the wave-per-packet kernel's reach in small
-// batches): 64 bytes per packet per step, four adjacent lanes per packet, any
-// byte alignment.
-constexpr uint32_t LDS_ROW = 80;    // generic: 64 data bytes + 16 pad
+constexpr uint32_t LDS_ROW = 80;    // wave per packet: a block of keystream + 16 pad
 constexpr uint32_t RING_ROW = 272;  // line path: 2 x 128-byte lines + 16 pad (where the shifted output keeps a copy of the first cell)
 constexpr uint32_t WAVES_PER_BLOCK = 4;
 // The lane-per-packet launches run workgroups of one wave: their waves share nothing, and a
@@ -292,77 +288,6 @@ BNK_DEV void capture_head(Head &h, const uint8_t *c0, const uint8_t *c1)
     if (h.on) {
         h.c0 = *reinterpret_cast<const uint4 *>(c0);
         h.c1 = *reinterpret_cast<const uint4 *>(c1);
-    }
-}
-
-template <bool OPEN>
-BNK_DEV void body_generic(uint8_t *tile, uint32_t lane, const uint8_t *src, uint8_t *dst,
-                          uint32_t len, const uint8_t *safe, const uint32_t (&k)[8], uint32_t n1,
-                          uint32_t n2, Poly32 &mac, uint32_t (&x)[16], Head &head)
-{
-    const uint32_t nfull = len >> 6, rem = len & 63u;
-    const uint32_t steps = nfull + (rem ? 1u : 0u);
-    // the four (packet, 16-byte column) cells this lane moves per step
-    const uint32_t col = lane & 3u;
-    const uint8_t *csrc[4];
-    uint8_t *cdst[4];
-    uint32_t clen[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int owner = 16 * j + (int)(lane >> 2);
-        csrc[j] = reinterpret_cast<const uint8_t *>(shfl64((uint64_t)(uintptr_t)src, owner)) + 16u * col;
-        cdst[j] = reinterpret_cast<uint8_t *>(shfl64((uint64_t)(uintptr_t)dst, owner)) + 16u * col;
-        clen[j] = (uint32_t)__shfl((int)len, owner, 64);
-    }
-    // The cells of step b+1 are fetched into registers while step b is
-    // computed.  Every lane loads every time, from a harmless address (`safe`,
-    // 16 readable bytes) when the cell is not a packet's: a load under a branch
-    // would make the wave wait for it before the branch closes.
-    uint4 pre[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) pre[j] = ld16(16u * col + 16u <= clen[j] ? csrc[j] : safe);
-    chacha_block(k, 0, n1, n2, x);
-    mac.init(x);
-    for (uint32_t b = 0; __ballot(b < steps) != 0ull; b++) {
-        const uint32_t pos = 64u * b + 16u * col;
-        // registers -> LDS, all 64 lanes, only 16-byte cells that lie fully inside a packet
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (pos + 16u <= clen[j])
-                *reinterpret_cast<uint4 *>(tile + (16u * j + (lane >> 2)) * LDS_ROW + 16u * col) = pre[j];
-        }
-        wave_sync();
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            pre[j] = ld16(pos + 64u + 16u <= clen[j] ? csrc[j] + 64u * (b + 1u) : safe);
-        if (b < steps) {
-            chacha_block(k, b + 1, n1, n2, x);
-            uint8_t *row = tile + lane * LDS_ROW;
-            if (b < nfull) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) crypt_cell<OPEN>(mac, x, j, row + 16 * j);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    if (rem >= 16u * (j + 1)) crypt_cell<OPEN>(mac, x, j, row + 16 * j);
-                    else if (rem > 16u * j)
-                        crypt_tail<OPEN>(mac, x, j, src + 64u * b + 16 * j, dst + 64u * b + 16 * j,
-                                         rem - 16u * j, rem - 16u * j, row + 16 * j);
-                }
-            }
-            if (OPEN && b == 0) capture_head(head, row, row + 16);
-        }
-        wave_sync();
-        // LDS -> global
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (pos + 16u <= clen[j]) {
-                const uint4 v = *reinterpret_cast<const uint4 *>(
-                    tile + (16u * j + (lane >> 2)) * LDS_ROW + 16u * col);
-                st16(cdst[j] + 64u * b, v);
-            }
-        }
-        wave_sync();
     }
 }
 
@@ -1472,14 +1397,14 @@ BNK_DEV uint32_t quad_from(uint32_t x)
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, A | B << 2 | C << 4 | D << 6, 0xF, 0xF, true);
 }
 
-// ChaCha20 blocks first .. first + 16 S - 1 of a packet into the rows of `stage`, four lanes a
+// ChaCha20 blocks first .. first + 16 S - 1 of a packet into the rows from `stage` on, four lanes a
 // block and S blocks a quad of lanes, side by side.  The lane holds column `lane & 3` of the state,
 // whose words 4.. and 8.. start out as key_b and key_c.
 template <int S>
 BNK_DEV void quad_blocks(uint8_t *stage, uint32_t lane, uint32_t key_b, uint32_t key_c, uint32_t first, uint32_t n1,
                          uint32_t n2)
 {
-    const uint32_t quad = lane & 3u, row = first + (lane >> 2);
+    const uint32_t quad = lane & 3u, row = lane >> 2;
     const uint32_t sigma = quad < 2u ? (quad == 0u ? 0x61707865u : 0x3320646eu) : quad == 2u ? 0x79622d32u : 0x6b206574u;
     uint32_t a[S], b[S], c[S], d[S], d0[S];
     // Rows 1, 2 and 3 move up by one, two and three lanes to make columns of the diagonals; they
@@ -1499,7 +1424,7 @@ BNK_DEV void quad_blocks(uint8_t *stage, uint32_t lane, uint32_t key_b, uint32_t
         a[s] = sigma;
         b[s] = key_b;
         c[s] = key_c;
-        d[s] = d0[s] = quad < 2u ? (quad == 0u ? row + 16u * s : 0u) : quad == 2u ? n1 : n2;
+        d[s] = d0[s] = quad < 2u ? (quad == 0u ? first + row + 16u * s : 0u) : quad == 2u ? n1 : n2;
         diagonal(s);
     }
     auto rounds = [&]() __attribute__((always_inline)) {
@@ -1558,6 +1483,30 @@ BNK_DEV Fe26 wave_powers(const Fe26 &r, uint32_t cells, uint32_t lane, Fe26 &top
     return lift;
 }
 
+// Cells first + lane, first + 64 + lane and first + 128 + lane of the packet at src, of which `there`
+// bytes are in memory (the rest counts as zeros).
+BNK_DEV void fetch_part(const uint8_t *src, uint32_t there, uint32_t first, uint32_t lane, const uint8_t *safe, uint4 (&m)[3])
+{
+#pragma unroll
+    for (uint32_t j = 0; j < 3; j++) {
+        const uint64_t off = 16ull * (first + 64u * j + lane);
+        m[j] = ld16(off + 16u <= there ? src + off : safe);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 3; j++) {
+        const uint64_t off = 16ull * (first + 64u * j + lane);
+        if (off + 16u > there) m[j] = off < there ? ld_partial(src + off, (uint32_t)(there - off)) : make_uint4(0, 0, 0, 0);
+    }
+}
+
+// Cell number `cell` of a packet of len bytes, its last bytes only where it has no more.
+BNK_DEV void store_cell(uint8_t *dst, uint32_t len, uint32_t cell, uint4 v)
+{
+    const uint64_t off = 16ull * cell;
+    if (off + 16u <= len) st16(dst + off, v);
+    else st_partial(dst + off, v, (uint32_t)(len - off));
+}
+
 // The sum of x over lanes 0..31 in lane 31, over lanes 32..63 in lane 63.
 BNK_DEV uint32_t half_wave_sum(uint32_t x)
 {
@@ -1589,11 +1538,12 @@ BNK_DEV uint32_t half_wave_sum(uint32_t x)
 //   sum over the lanes and the tag.
 // Calls that seal and open 1 packet of 1420 bytes in pinned rings 34.5 -> 26.9 us (a block and
 // four cells in a row per lane, each lane's powers by squaring, before), 128 packets through the
-// tunnel 74.7 -> 66.7; launches of 1000 packets in GPU memory 13.2 -> 7.4 us, of 2000 17.4 -> 10.1.
+// tunnel 74.7 -> 66.7; launches of 1000 packets in GPU memory 13.2 -> 7.4 us, of 2000 17.4 -> 9.9.
 // (All arguments fetched at once, or the per-packet entries by scalar loads: no different.)
-// All loads of a packet are issued before any store, and a lane stores only what it
-// loaded, so sealing in place is safe.  A packet longer than 63 blocks is done by lane 0
-// alone, the per-lane way.
+// All loads of a packet are issued before any store, so that it may lie anywhere, and a lane
+// stores only what it loaded.  A packet longer than 63 blocks goes through in parts of
+// LONG_CELLS cells, the tag first when opening: its parts are then opened in an order in which
+// none is overwritten before it is read, however the packet and its plaintext overlap.
 //
 // With WG set the wave also does the packet's WireGuard framing (a.wg): on the
 // way out it writes the transport header and treats the bytes between the
@@ -1603,8 +1553,9 @@ BNK_DEV uint32_t half_wave_sum(uint32_t x)
 // the tag check looks at the inner IP header while it is still in registers.
 // Same results as wg_parse_kernel / wg_encap_prep_kernel / wg_finish_kernel
 // around a plain launch.
+constexpr uint32_t LONG_CELLS = 192; // with their 48 blocks and block 0 the rows of a wave hold them
 template <bool OPEN, bool WG>
-__global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
+__global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
 {
     __shared__ __attribute__((aligned(16))) uint8_t tile_all[WAVES_PER_BLOCK][64 * LDS_ROW];
     const uint32_t lane = threadIdx.x & 63u;
@@ -1628,29 +1579,43 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     uint32_t len = a.lens ? len_ld : a.len;
     if (!OPEN) len = len >= a.trim ? len - a.trim : 0u;
     uint32_t pr = a.peer ? peer_ld : 0u;
-    const uint8_t *src = a.in + (a.in_off ? in_off_ld : (uint64_t)i * a.in_stride) + a.in_skip;
-    uint8_t *dst = a.out + (a.out_off ? out_off_ld : (uint64_t)i * a.out_stride) + a.out_skip;
+    const uint64_t in_at = a.in_off ? in_off_ld : (uint64_t)i * a.in_stride, out_at = a.out_off ? out_off_ld : (uint64_t)i * a.out_stride;
+    const uint8_t *src = a.in + in_at + a.in_skip;
+    uint8_t *dst = a.out + out_at + a.out_skip;
     const bool skipped = a.skip != nullptr && skip_ld != 0;
     auto refuse = [&]() {
         a.verdict[i] = 0;
         if (a.tally) tally_bump(a.tally, TALLY_REJECTED, 1u);
     };
     uint64_t ctr = 0;
+    uint32_t wire_pad = 0; // (encapsulating)
+    // (a length word of a device-resident batch may be garbage: one so large that lengths made of
+    // it would wrap is beyond any arena)
+    const bool huge = (WG && OPEN && len >= 16u ? len - 16u : len) > MAX_PACKET_BYTES;
+    const bool wraps = huge && (a.in_limit | a.out_limit) != 0;
+    bool outside;
     if (!WG) {
-        // (framing launches only run on layouts the host has checked)
         // (a launch that checks has no skip here: the kernel that framed the packets has looked
         // at their raw offsets.  Taking skip and offset apart costs a launch of 2900 packets 1 %.)
-        const uint64_t in_at = (uint64_t)(src - a.in), out_at = (uint64_t)(dst - a.out);
         const bool short_ct = OPEN && len < 16u;
-        if (beyond_arena(in_at, len, a.in_limit) ||
-            beyond_arena(out_at, OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
-            (len > MAX_PACKET_BYTES && (a.in_limit | a.out_limit) != 0)) {
+        outside = beyond_arena((uint64_t)(src - a.in), len, a.in_limit) ||
+                  beyond_arena((uint64_t)(dst - a.out), OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
+                  wraps;
+        if (outside) {
             if (lane == 0 && !skipped) {
                 status_raise(a.status, STATUS_BOUNDS);
                 if (OPEN) refuse();
             }
             return;
         }
+    } else if (!OPEN) {
+        // the slot from its first byte to the end of the tag
+        wire_pad = huge ? 0u : wg_padding(len, a.wg.mtu);
+        const uint32_t padded = len + wire_pad;
+        outside = wraps || beyond_arena(in_at, 16u, padded, a.in_limit) || beyond_arena(out_at, 16u, (uint64_t)padded + 16u, a.out_limit);
+    } else {
+        // the datagram where it is read, and the plaintext where it would be written
+        outside = beyond_arena(in_at, len, a.in_limit) || beyond_arena(out_at, 0u, len >= 32u ? len - 32u : 0u, a.out_limit);
     }
 
     // ---- my cells: loads first, they fly while everything below is looked
@@ -1661,17 +1626,19 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     const uint8_t *data = src + (WG ? 16 : 0);
     uint32_t data_len; // bytes through the cipher, when the packet is taken at all
     uint32_t data_there; // of which in memory
+    const bool framed = len >= 32u && !outside && !wraps; // (decapsulating)
     if (!WG) {
         data_len = OPEN ? (len >= 16u ? len - 16u : 0u) : len;
-        data_there = data_len <= SPREAD_MAX_LEN ? data_len : 0u; // longer ones go the per-lane way
+        data_there = data_len;
     } else if (!OPEN) {
-        const bool fits = len + 15u <= WG_FUSE_MAX_LEN;
-        data_there = fits ? len : 0u;
-        data_len = fits ? len + wg_padding(len, a.wg.mtu) : 0u;
+        data_there = outside ? 0u : len;
+        data_len = outside ? 0u : len + wire_pad;
     } else {
-        data_len = (len >= 32u && len - 32u <= WG_FUSE_MAX_LEN) ? len - 32u : 0u;
+        data_len = framed ? len - 32u : 0u;
         data_there = data_len;
     }
+    const uint8_t *const tag_at = data + data_len;
+    if (data_len > SPREAD_MAX_LEN) data_there = 0; // (its parts are fetched further down)
     // The wave fetches the packet in pieces of 1 KB, lane l taking bytes [16 l,
     // 16 l + 16) of each piece, so that an instruction reads 1 KB in a row (64
     // bytes a lane would be sixty-four small requests an instruction, each of
@@ -1690,7 +1657,7 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         key_c = a.keys[8u * known + 4u + quad];
         if (WG) wg_remote = a.wg.remote_index[known];
     } else {
-        wg_head = ld16(len >= 32u && len - 32u <= WG_FUSE_MAX_LEN ? src : safe);
+        wg_head = ld16(len >= 32u && !outside ? src : safe);
     }
     // Every load below is issued whatever the lane's share is (from the key table where it
     // has none), so that they are all in flight together: the pieces, the last 1-15 bytes of
@@ -1705,8 +1672,8 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     const uint32_t odd = data_there & 15u, odd_at = data_there & ~15u; // the packet's last, partial cell
     const bool odd_mine = odd != 0u && ((odd_at >> 4) & 63u) == lane;
     const uint4 odd_cell = ld_partial_flat(data + odd_at, odd_mine ? odd : 0u, safe);
-    const bool tagged = OPEN && (WG ? len >= 32u && len - 32u <= WG_FUSE_MAX_LEN : len >= 16u && data_len <= SPREAD_MAX_LEN);
-    uint4 want_tag = ld16(tagged ? data + data_len : safe);
+    const bool tagged = OPEN && (WG ? framed : len >= 16u);
+    uint4 want_tag = ld16(tagged ? tag_at : safe);
     // (what the lanes without a share have fetched is set aside where the pieces are used,
     // further down: looking at it here would make the key wait for the packet)
 
@@ -1727,16 +1694,17 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         ctr = a.counters ? ctr_ld : a.counter0 + i;
     } else if (!OPEN) {
         // ---- encapsulate: header into the headroom, padding as implied zeros ----
-        if (pr >= a.wg.n_peers || len + 15u > WG_FUSE_MAX_LEN) {
-            if (lane == 0) a.wg.wire_len[i] = 0;
-            return;
-        }
         ctr = ctr_ld;
-        if (ctr >= WG_REJECT_AFTER_MESSAGES) { // the keypair has used up its nonces
-            if (lane == 0) a.wg.wire_len[i] = 0;
+        // (a keypair that has used up its nonces sends nothing more)
+        if (pr >= a.wg.n_peers || outside || ctr >= WG_REJECT_AFTER_MESSAGES) {
+            if (lane == 0) {
+                a.wg.wire_len[i] = 0;
+                if (pr >= a.wg.n_peers) status_raise(a.status, STATUS_PEER_RANGE);
+                else if (outside) status_raise(a.status, STATUS_BOUNDS);
+            }
             return;
         }
-        len += wg_padding(len, a.wg.mtu);
+        len += wire_pad;
         if (lane == 0) {
             st16(dst, make_uint4(4u, wg_remote, (uint32_t)ctr, (uint32_t)(ctr >> 32)));
             a.wg.wire_len[i] = 16u + len + 16u;
@@ -1747,8 +1715,9 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
         // ---- decapsulate: header checks and the receiver-index lookup ----
         uint8_t res = BNK_WG_OK;
         uint4 h = make_uint4(0, 0, 0, 0);
-        if (len < 32u || len - 32u > WG_FUSE_MAX_LEN) res = BNK_WG_BAD_HEADER;
+        if (len < 32u || outside) res = BNK_WG_BAD_HEADER;
         else h = wg_head;
+        if (outside && lane == 0) status_raise(a.status, STATUS_BOUNDS);
         if (res == BNK_WG_OK && h.x != 4u) res = BNK_WG_BAD_HEADER;
         if (res == BNK_WG_OK) {
             // narrow [lo, hi) to at most 64 entries, 64 probes at a time
@@ -1782,6 +1751,17 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
             return;
         }
         ctr = (uint64_t)h.z | (uint64_t)h.w << 32;
+        if (lane == 0) {
+            a.wg.peer_out[i] = pr;
+            a.wg.counter_out[i] = ctr;
+        }
+        if (wraps) { // (reported as one that does not verify, by the lane kernels too)
+            if (lane == 0) {
+                status_raise(a.status, STATUS_BOUNDS);
+                decap_result(a, i, false, false, 0u, make_uint4(0, 0, 0, 0), pr);
+            }
+            return;
+        }
         len -= 32u; // header and tag
         src += 16;
     }
@@ -1791,31 +1771,16 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     }
     const uint32_t n1 = (uint32_t)ctr, n2 = (uint32_t)(ctr >> 32);
 
-    if (!WG && len > SPREAD_MAX_LEN) {
-        const bool have = lane == 0;
-        const uint4 *kp = reinterpret_cast<const uint4 *>(a.keys + 8u * pr);
-        const uint4 k0 = kp[0], k1 = kp[1];
-        const uint32_t k[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
-        uint32_t x[16];
-        Poly32 mac;
-        Head no_head;
-        no_head.on = false;
-        body_generic<OPEN>(tile_all[threadIdx.x >> 6], lane, have ? src : nullptr, have ? dst : nullptr,
-                           have ? len : 0u, reinterpret_cast<const uint8_t *>(a.keys), k, n1, n2, mac, x, no_head);
-        const bool bad = lane_finish<OPEN>(a, lane, have, i, len, have ? src : nullptr, have ? dst : nullptr, mac, no_head, nullptr);
-        if (OPEN && have && a.tally) tally_bump(a.tally, bad ? TALLY_REJECTED : TALLY_OPENED, 1u);
-        return;
-    }
-
-    // ---- the keystream, block 0 and those of the data (they fly: see the top of the kernel) ----
+    // ---- the keystream, block 0 and those of the data (whose bytes fly: see the top of the kernel) ----
     // Block b lies at stage + 80 b (rows padded against bank conflicts).
     uint8_t *const stage = tile_all[threadIdx.x >> 6];
-    const uint32_t passes = (len + 63u) / 64u / 16u + 1u; // of sixteen blocks
+    const bool is_long = len > SPREAD_MAX_LEN; // (the same in every lane)
+    const uint32_t passes = is_long ? 4u : (len + 63u) / 64u / 16u + 1u; // of sixteen blocks
     if (passes == 1u) {
         quad_blocks<1>(stage, lane, key_b, key_c, 0u, n1, n2);
     } else {
         quad_blocks<2>(stage, lane, key_b, key_c, 0u, n1, n2);
-        if (passes > 2u) quad_blocks<2>(stage, lane, key_b, key_c, 32u, n1, n2);
+        if (passes > 2u) quad_blocks<2>(stage + 32 * LDS_ROW, lane, key_b, key_c, 32u, n1, n2);
     }
     wave_sync();
     uint32_t x[16];
@@ -1827,30 +1792,62 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
     Poly32 mac;
     mac.init(x);
     // ---- the powers of r that my cells take: r^64 from one to the next, r^(1 + cells behind it) the last ----
-    const uint32_t cells = wave_value((len + 15u) >> 4); // (the same in every lane)
+    const uint32_t cells = wave_value((uint32_t)(((uint64_t)len + 15u) >> 4)); // (the same in every lane)
     Fe26 top; // r^64 where a lane has a second cell
     const Fe26 lift = wave_powers(fe_clamped_r(mac.r0, mac.r1, mac.r2, mac.r3), cells, lane, top);
 
+    // cell number j * 64 + lane of the keystream in `stage`
+    auto keystream = [&](uint32_t j) __attribute__((always_inline)) {
+        return *reinterpret_cast<const uint4 *>(stage + (1u + 16u * j + (lane >> 2)) * LDS_ROW + 16u * quad);
+    };
     // ---- crypt: o = m ^ keystream; the MAC reads the ciphertext side ----
     if (!tagged) want_tag = make_uint4(0, 0, 0, 0);
     uint4 o[4] = {};
     Fe26 acc = fe_small(0);
+    auto take_cell = [&](uint32_t cell, const uint4 &c) __attribute__((always_inline)) {
+        Fe26 next = fe_cell(c.x, c.y, c.z, c.w);
+        if (cell >= 64u) next = fe_add(fe_mul(acc, top), next);
+        acc = fe_select(cell < cells, next, acc);
+    };
+    if (__builtin_expect(!is_long, 1)) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        if (64u * j >= cells) break; // (the same for the whole wave)
-        const uint32_t off = 1024u * j + 16u * lane;
-        uint4 m = pre[j];
-        // a cell beyond the packet's whole cells is zeros, but for its last 1-15 bytes
-        if (off + 16u > data_there) m = make_uint4(0, 0, 0, 0);
-        if (odd_mine && (odd_at >> 10) == (uint32_t)j) m = odd_cell;
-        const uint4 ks = *reinterpret_cast<const uint4 *>(stage + (1u + 16u * j + (lane >> 2)) * LDS_ROW + 16u * quad);
-        o[j] = make_uint4(m.x ^ ks.x, m.y ^ ks.y, m.z ^ ks.z, m.w ^ ks.w);
-        if (64u * (j + 1u) >= cells && (len & 15u) != 0u) // the last cell is among these
-            o[j] = o[j] & byte_mask(64u * j + lane == cells - 1u ? len & 15u : 16u);
-        const uint4 mine = OPEN ? m : o[j];
-        Fe26 next = fe_cell(mine.x, mine.y, mine.z, mine.w);
-        if (j != 0) next = fe_add(fe_mul(acc, top), next);
-        acc = fe_select(64u * j + lane < cells, next, acc);
+        for (uint32_t j = 0; j < 4; j++) {
+            if (64u * j >= cells) break; // (the same for the whole wave)
+            const uint32_t off = 1024u * j + 16u * lane;
+            uint4 m = pre[j];
+            // a cell beyond the packet's whole cells is zeros, but for its last 1-15 bytes
+            if (off + 16u > data_there) m = make_uint4(0, 0, 0, 0);
+            if (odd_mine && (odd_at >> 10) == j) m = odd_cell;
+            o[j] = m ^ keystream(j);
+            if (64u * (j + 1u) >= cells && (len & 15u) != 0u) // the last cell is among these
+                o[j] = o[j] & byte_mask(64u * j + lane == cells - 1u ? len & 15u : 16u);
+            take_cell(64u * j + lane, OPEN ? m : o[j]);
+        }
+    } else {
+        const uint32_t there = WG && !OPEN ? len - wire_pad : len;
+#pragma unroll 1
+        for (uint32_t first = 0; first < cells; first += LONG_CELLS) {
+            if (!OPEN && first != 0u) {
+                quad_blocks<2>(stage, lane, key_b, key_c, first / 4u, n1, n2);
+                quad_blocks<2>(stage + 32 * LDS_ROW, lane, key_b, key_c, first / 4u + 32u, n1, n2);
+                wave_sync();
+            }
+            uint4 m[3];
+            fetch_part(src, there, first, lane, safe, m);
+#pragma unroll
+            for (uint32_t j = 0; j < 3; j++) {
+                const uint32_t cell = first + 64u * j + lane;
+                uint4 out = make_uint4(0, 0, 0, 0);
+                if (!OPEN || first == 0u) out = m[j] ^ keystream(j);
+                if (!OPEN) {
+                    out = out & byte_mask(cell < cells ? min(len - 16u * cell, 16u) : 0u);
+                    if (cell < cells) store_cell(dst, len, cell, out);
+                } else if (first == 0u && j == 0u) {
+                    o[0] = out; // (the inner header, before the plaintext is written)
+                }
+                take_cell(cell, OPEN ? m[j] : out);
+            }
+        }
     }
     const Fe26 term = fe_mul(acc, lift);
 
@@ -1871,7 +1868,10 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
 
     bool reject = false;
     if (!OPEN) {
-        if (lane == 0) st16(dst + len, make_uint4(tag[0], tag[1], tag[2], tag[3]));
+        if (lane == 0) {
+            st16(dst + len, make_uint4(tag[0], tag[1], tag[2], tag[3]));
+            if (WG && a.tally) tally_bump(a.tally, TALLY_SEALED, 1u);
+        }
     } else {
         // all 16 bytes are compared, no early exit
         reject = ((want_tag.x ^ tag[0]) | (want_tag.y ^ tag[1]) | (want_tag.z ^ tag[2]) |
@@ -1881,48 +1881,35 @@ __global__ __launch_bounds__(256) void aead_spread_kernel(AeadArgs a)
             if (a.tally) tally_bump(a.tally, reject ? TALLY_REJECTED : TALLY_OPENED, 1u);
         }
     }
-    if (WG && OPEN) {
-        // ---- what wireguard-go checks once a packet is authentic: keepalive, IP
-        // version, length fields, source inside the sender's allowed prefix.  The
-        // first 16 plaintext bytes (lane 0's first cell) hold every field used.
-        const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].x, 0);
-        const uint32_t w1 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].y, 0);
-        const uint32_t w3 = (uint32_t)__builtin_amdgcn_readlane((int)o[0].w, 0);
-        uint8_t res = BNK_WG_OK;
-        uint32_t inner = 0;
-        const uint32_t version = (w0 >> 4) & 0xFu;
-        if (reject) res = BNK_WG_AUTH_FAIL;
-        else if (len == 0u) res = BNK_WG_KEEPALIVE;
-        else if (len < 16u) res = BNK_WG_BAD_IP;
-        else if (version == 4u) {
-            const uint32_t total = __builtin_bswap32(w0) & 0xFFFFu;
-            const uint2 al = a.wg.allowed[pr];
-            if (len < 20u || total > len || total < 20u) res = BNK_WG_BAD_IP;
-            else if ((__builtin_bswap32(w3) & al.y) != (al.x & al.y)) res = BNK_WG_NOT_ALLOWED;
-            else inner = total;
-        } else if (version == 6u) {
-            // peers own IPv4 addresses only
-            const uint32_t total = (__builtin_bswap32(w1) >> 16) + 40u;
-            res = (len < 40u || total > len) ? BNK_WG_BAD_IP : BNK_WG_NOT_ALLOWED;
-        } else {
-            res = BNK_WG_BAD_IP;
-        }
-        if (lane == 0) {
-            a.wg.result[i] = res;
-            a.wg.out_len[i] = inner;
-            a.wg.peer_out[i] = pr;
-            a.wg.counter_out[i] = ctr;
-        }
-    }
+    // what wireguard-go checks once a packet is authentic (lane 0 has the first 16 plaintext bytes,
+    // which hold every field used)
+    if (WG && OPEN && lane == 0) decap_result(a, i, true, reject, len, o[0], pr);
+
     // ---- the bytes out, the way they came in; a rejected packet leaves zeros
     // (chacha20poly1305.Open) ----
+    if (__builtin_expect(!is_long, 1)) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t off = 1024u * j + 16u * lane;
-        if (off < len) {
-            const uint4 v = reject ? make_uint4(0, 0, 0, 0) : o[j];
-            if (off + 16u <= len) st16(dst + off, v);
-            else st_partial(dst + off, v, len - off);
+        for (uint32_t j = 0; j < 4; j++)
+            if (64u * j + lane < cells) store_cell(dst, len, 64u * j + lane, reject ? make_uint4(0, 0, 0, 0) : o[j]);
+    } else if (OPEN) {
+        const bool backwards = (uintptr_t)dst > (uintptr_t)src;
+        const uint32_t last = (cells - 1u) / LONG_CELLS * LONG_CELLS;
+#pragma unroll 1
+        for (uint32_t done = 0; done < cells; done += LONG_CELLS) {
+            const uint32_t first = backwards ? last - done : done;
+            quad_blocks<2>(stage, lane, key_b, key_c, first / 4u, n1, n2);
+            quad_blocks<2>(stage + 32 * LDS_ROW, lane, key_b, key_c, first / 4u + 32u, n1, n2);
+            wave_sync();
+            uint4 m[3];
+            fetch_part(src, len, first, lane, safe, m);
+            // (the next lane's cell may lie where mine goes: all of them are here before any goes out)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (uint32_t j = 0; j < 3; j++) {
+                const uint32_t cell = first + 64u * j + lane;
+                if (cell < cells) store_cell(dst, len, cell, reject ? make_uint4(0, 0, 0, 0) : m[j] ^ keystream(j));
+            }
         }
     }
 }

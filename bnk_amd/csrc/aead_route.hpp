@@ -11,12 +11,12 @@ namespace bnk {
 
 // Which launch?  Packets in GPU memory (us per launch of n packets in a row, all of
 // them resident at once; seal and open within 2 us of each other):
-//   a wave per packet   4.5 + 3.0 per 1000 packets at 1420 bytes, 2.1 at 60
+//   a wave per packet   4.5 + 2.7 per 1000 packets at 1420 bytes, 1.8 at 60
 //   split over lanes    6.5 + 9.2 q, q = pieces per run (n = 16384 x 1420: q = 2), 3 less than
 //                       with q = 1 where every block gets a lane of its own
 //   a lane per packet   5 + 2.75 per ChaCha20 block of the longest packet, and 20 more
 //                       for the grouping where lengths vary
-// so 4096 packets x 1420 take 17 / 17 / 71 us, 16384 54 / 26 / 71, and 24000 packets of 1
+// so 4096 packets x 1420 take 15 / 17 / 71 us, 16384 50 / 26 / 71, and 24000 packets of 1
 // to 1420 bytes - / 35 / 97.
 //
 // Packets in host memory (over_link): a wave per packet reads them where they are, the
@@ -29,20 +29,19 @@ namespace bnk {
 // not build it).
 inline bool aead_runs_spread(const AeadArgs &a)
 {
-    // (framing behind a header: the host has not seen that every packet fits 63 blocks, and the
-    // wave-per-packet kernel does that framing for no other)
+    // (the wave-per-packet kernel does the framing of whole slots and datagrams, not behind a header)
     if (a.wg.mode != WG_FUSE_OFF && a.in_skip != 0u) return false;
     if (a.over_link) {
         if (a.lens) return a.n <= a.spread_max;
         const uint64_t by_len = 12ull * a.len + a.spread_max / 2;
         return a.n <= std::min<uint64_t>(4ull * a.spread_max, by_len);
     }
-    // 2560 by default: where several streams no longer gain by it.  Pairs of launches, us alone with a
-    // wait behind each / in a row / with three streams at work, a wave per packet against split, packets of
-    // 1 to 1420 bytes: 1000 24.9 / 13.9 / 7.7 against 36.4 / 24.9 / 9.7, 2000 29.5 / 18.7 / 9.7 against 38.8 /
-    // 27.5 / 12.7, 2500 33.6 / 22.3 / 11.7 against 41.7 / 30.1 / 12.1, 3000 35.1 / 23.9 / 13.6 against 42.4 /
-    // 30.7 / 12.4, 4096 41.7 / 31.0 / 17.6 against 42.7 / 31.7 / 13.5; IMIX and one length of 1420 bytes cross
-    // at the same place; of 1 to 600 bytes three streams are even at 2000 and 0.9 apart at 2500.
+    // 2560 by default.  Pairs of launches, us alone with a wait behind each / in a row / with three streams
+    // at work, a wave per packet against split, packets of 1 to 1420 bytes: 1000 25.1 / 13.8 / 7.2 against
+    // 36.1 / 25.0 / 9.4, 2000 29.3 / 18.6 / 8.6 against 38.5 / 27.4 / 11.8, 2500 33.1 / 22.0 / 10.4 against
+    // 41.2 / 30.0 / 11.5, 3000 34.4 / 23.5 / 11.7 against 41.7 / 30.5 / 11.8, 4096 39.3 / 28.4 / 15.3 against
+    // 42.7 / 31.4 / 13.0; IMIX as these, one length of 1420 bytes crosses at 2700 with three streams.  (One
+    // stream alone in view it would end at 5000.)
     const uint64_t most = 5ull * a.spread_max / 8;
     if (a.lens) return a.n <= most;
     return a.n <= std::min<uint64_t>(most, (4ull * a.len + a.spread_max) * 4ull / 10);

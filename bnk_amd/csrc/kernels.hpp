@@ -32,12 +32,11 @@ __host__ __device__ inline uint64_t ctr_add(uint64_t base, uint64_t rank, uint64
     return (c < base || c > limit) ? limit : c;
 }
 
-// WireGuard transport framing done by the AEAD launch itself.  A wave-per-packet
-// launch (small batches): in/out offsets address the slot or datagram
-// (in_skip = out_skip = 0) and every packet must be at most WG_FUSE_MAX_LEN
-// bytes long, padding included.  A lane-per-packet launch: in_skip and
-// out_skip say where the AEAD data starts within the slot or datagram (16 past
-// the header), any length.
+// WireGuard transport framing done by the AEAD launch itself, for packets of any
+// length.  A wave-per-packet launch (small batches): in/out offsets address the
+// slot or datagram (in_skip = out_skip = 0).  A lane-per-packet launch: in_skip
+// and out_skip say where the AEAD data starts within the slot or datagram (16 past
+// the header).
 // Receiver index -> peer row as an open-addressing table of (index, row) pairs
 // with linear probing; an empty slot has row WG_HASH_EMPTY.
 constexpr uint32_t WG_HASH_EMPTY = 0xFFFFFFFFu;
@@ -74,7 +73,6 @@ struct WgFuse {
     uint32_t *wire_len;          // encapsulate: datagram length
 };
 enum : uint32_t { WG_FUSE_OFF = 0, WG_FUSE_ENCAP = 1, WG_FUSE_DECAP = 2 };
-constexpr uint32_t WG_FUSE_MAX_LEN = 63u * 64u;
 // No packet is longer than this: a length word above it (only a device-resident
 // batch can carry one unseen) is treated as reaching beyond the arena, so that
 // length + tag and length + padding never wrap 32 bits.

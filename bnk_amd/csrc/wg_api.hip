@@ -251,11 +251,11 @@ extern "C" int bnk_wg_send_counters(bnk_ctx *ctx, uint64_t *out, uint32_t n)
 }
 
 // Does the launch described by `a` (a plain one over the packets behind their transport
-// headers) do the framing itself?  Wherever it gives a lane a packet or a run of one; and a
-// batch small enough for a wave per packet, which cannot do it over lengths the host has not
-// seen, is split over lanes instead, unless it would be read over the link: one launch in the
-// place of three.  (3000 packets of the internet mix through NoteOutbound + encapsulate and
-// decapsulate + CheckInbound: 117 -> 91 us with the counting launches gone as well.)
+// headers) do the framing itself?  Wherever it gives a lane a packet or a run of one.  (A batch of
+// a wave per packet has been asked for before, in a launch over whole slots or datagrams that does
+// their framing: for one in GPU memory too, up to the same size as without framing.  Tunnel passes of
+// IMIX packets, us in a row / with three streams at work, split over lanes against that: 256 packets
+// 43.3 / 21.8 -> 31.7 / 19.4, 1200 60.2 / 24.4 -> 49.2 / 20.3, 2500 69.0 / 26.7 -> 58.9 / 23.5.)
 static bool wg_framing_fused(const bnk_ctx *ctx, const AeadArgs &a)
 {
     return !ctx->wg_unfused && (!a.over_link || !aead_runs_spread(a));
@@ -289,16 +289,6 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
     Span span;
     HostPipe hp;
     bool chunked = false;
-    // A wave-per-packet launch does the framing itself; it needs every packet to
-    // fit 63 ChaCha20 blocks, which only a host batch can promise.
-    bool fits = host;
-    if (host) {
-        if (slots->lens) {
-            for (uint32_t i = 0; i < n && fits; i++) fits = slots->lens[i] + 15u <= WG_FUSE_MAX_LEN;
-        } else {
-            fits = slots->len + 15u <= WG_FUSE_MAX_LEN;
-        }
-    }
     // Which kernel will read the packets: the framing launch when the batch
     // qualifies for it, else a plain launch over per-packet padded lengths.
     AeadArgs probe{};
@@ -307,7 +297,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
     probe.n = n;
     probe.len = slots->len;
     probe.lens = slots->lens; // only whether there is one matters here
-    const bool wave_per_packet = (fits && aead_runs_spread(probe)) || n <= ctx->spread_max;
+    const bool wave_per_packet = aead_runs_spread(probe) || n <= ctx->spread_max;
 
     // direct route (small batches in a pinned ring): the plaintexts are fetched
     // by a copy kernel, headers and sealed packets go straight into the ring
@@ -478,7 +468,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             fa.record_after = f->record_after && hi == n;
             HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->bound.upper, ctx->stream));
         }
-        if (fits) {
+        if (host || !ctx->wg_unfused) {
             AeadArgs se{};
             se.spread_max = ctx->spread_max;
             se.over_link = over_link;
@@ -495,12 +485,17 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             se.len = slots->len;
             se.peer = d_peer;
             se.counters = d_ctr;
+            se.in_limit = se.out_limit = b.limit;
             if (aead_runs_spread(se)) {
                 se.wg.mode = WG_FUSE_ENCAP;
                 se.wg.n_peers = pe.n;
                 se.wg.mtu = mtu;
                 se.wg.remote_index = pe.remote_index;
                 se.wg.wire_len = d_wire_len;
+                if (!host && counted && ctx->tally_on.load(std::memory_order_relaxed)) {
+                    se.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
+                    *counted = true;
+                }
                 HIPCHK(ctx, launch_aead_seal(se, ctx->stream));
                 return BNK_OK;
             }
@@ -665,16 +660,6 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         const uint64_t l = wire->lens ? wire->lens[i] : wire->len;
         return l >= 32u ? l - 32u : (uint64_t)0;
     };
-    // A wave-per-packet launch does the framing itself; it needs every packet to
-    // fit 63 ChaCha20 blocks, which only a host batch can promise.
-    bool fits = host;
-    if (host) {
-        if (wire->lens) {
-            for (uint32_t i = 0; i < n && fits; i++) fits = wire->lens[i] <= WG_FUSE_MAX_LEN + 32u;
-        } else {
-            fits = wire->len <= WG_FUSE_MAX_LEN + 32u;
-        }
-    }
     // Which kernel will read the datagrams: the framing launch when the batch
     // qualifies for it, else a plain launch over per-packet ciphertext lengths.
     AeadArgs probe{};
@@ -683,7 +668,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     probe.n = n;
     probe.len = wire->len;
     probe.lens = wire->lens; // only whether there is one matters here
-    const bool wave_per_packet = (fits && aead_runs_spread(probe)) || n <= ctx->spread_max;
+    const bool wave_per_packet = aead_runs_spread(probe) || n <= ctx->spread_max;
 
     // direct route (small batches in pinned rings): datagrams fetched by a copy
     // kernel, plaintexts written straight into the out ring, per-packet results
@@ -894,7 +879,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         WgBatch cw = wb, co = ob;
         cw.first = co.first = lo;
         cw.n = co.n = hi - lo;
-        if (fits) {
+        if (host || !ctx->wg_unfused) {
             AeadArgs op{};
             op.spread_max = ctx->spread_max;
             op.over_link = over_link;
@@ -911,6 +896,8 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
             op.out_stride = out->stride;
             op.lens = wb.lens;
             op.len = wire->len;
+            op.in_limit = wb.limit;
+            op.out_limit = ob.limit;
             if (aead_runs_spread(op)) {
                 op.wg.mode = WG_FUSE_DECAP;
                 op.wg.n_peers = pe.n;

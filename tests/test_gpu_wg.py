@@ -1652,3 +1652,86 @@ def test_send_counters_follow_batch_order_at_the_sizes_of_a_tile(n, n_peers):
             assert bool((results[0] == want).all())
             assert np.array_equal(results[2].cpu().numpy(), peer)
             assert np.array_equal(results[3].cpu().numpy(), rank + count[peer])
+
+
+@pytest.mark.parametrize("shift", [-16, 0, 32, 4000])
+def test_small_device_batches_of_any_length(shift):
+    """A wave per packet does the framing of device-resident batches of up to 2560 packets whatever
+    their lengths: keystreams of one, two and four passes, cells on both sides of 1 KB, packets
+    beyond 63 blocks in parts, and plaintexts that overlap the datagram they come out of from
+    ahead or from behind; forged tags and unknown indices among them."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    mtu = 32000
+    lens = np.array([0, 1, 15, 16, 17, 63, 64, 65, 944, 945, 960, 961, 1008, 1024, 1025, 1984, 2047, 2049, 3072, 3073, 4016,
+                     4017, 4032, 4033, 4049, 6143, 6144, 6145, 9000, 20011] * 3, np.uint32)
+    n = len(lens)
+    rng = np.random.default_rng(70 + shift)
+    rng.shuffle(lens)
+    peers = _peers(rng)
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    peer = rng.integers(0, N_PEERS, n).astype(np.uint32)
+    off, total = _layout(rng, lens + 64 + abs(shift), misalign=shift == 32)
+    off += np.uint64(16)  # (room for the plaintext ahead of the first datagram)
+    total += 16
+    arena = np.full(total, 0xEE, np.uint8)
+    want, sent, nxt = arena.copy(), [], np.zeros(N_PEERS, np.int64)
+    for i in range(n):
+        p, o, ln = int(peer[i]), int(off[i]), int(lens[i])
+        pt = _inner(rng, peers, p, ln)
+        arena[o + 16:o + 16 + ln] = np.frombuffer(pt, np.uint8)
+        w = O.wg_encap(pt, mtu, keys[p].tobytes(), peers[p][1], int(nxt[p]))
+        want[o:o + len(w)] = np.frombuffer(w, np.uint8)
+        sent.append(w)
+        nxt[p] += 1
+    dev = torch.device("cuda:0")
+    up = lambda a, t: torch.from_numpy(np.ascontiguousarray(a).view(t)).to(dev)  # noqa: E731
+    d_arena, d_off, d_lens, d_peer = up(arena, np.uint8), up(off, np.int64), up(lens, np.int32), up(peer, np.int32)
+    d_wlen = torch.zeros(n, dtype=torch.int32, device=dev)
+    ctx = _ctx(peers, keys, keys)
+    torch.cuda.synchronize()
+    ctx.wg_encap(lib.make_batch(d_arena, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_lens, peer=d_peer), mtu, d_wlen)
+    ctx.sync()
+    wire_len = d_wlen.cpu().numpy().view(np.uint32)
+    assert np.array_equal(wire_len, np.array([len(w) for w in sent], np.uint32))
+    bad = np.flatnonzero(d_arena.cpu().numpy() != want)
+    assert bad.size == 0, f"first differing byte at {bad[:5]}"
+    # what comes back: the same datagrams under the indices they are received by
+    ctx.wg_peers_set([(b, a, c, d) for a, b, c, d in peers])
+    forged, unknown = np.arange(n) % 11 == 3, np.arange(n) % 17 == 5
+    forged &= ~unknown
+    for i in range(n):
+        o, wl = int(off[i]), int(wire_len[i])
+        if forged[i]:
+            want[o + wl - 1 - int(rng.integers(0, 16))] ^= 1 << int(rng.integers(0, 8))
+        if unknown[i]:
+            want[o + 4:o + 8] ^= 0x5A
+    d_arena.copy_(torch.from_numpy(want))
+    for i in range(n):
+        if unknown[i]:
+            continue
+        o, padded = int(off[i]), int(wire_len[i]) - 32
+        full = bytes(padded) if forged[i] else O.aead_open(keys[int(peer[i])].tobytes(), O.wg_nonce(
+            int(np.frombuffer(sent[i][8:16], np.uint64)[0])), sent[i][16:])[1]
+        want[o + 16 + shift:o + 16 + shift + padded] = np.frombuffer(full, np.uint8)
+    res = torch.full((n,), 99, dtype=torch.uint8, device=dev)
+    olen, gp = torch.zeros(n, dtype=torch.int32, device=dev), torch.zeros(n, dtype=torch.int32, device=dev)
+    gc = torch.zeros(n, dtype=torch.int64, device=dev)
+    d_out = d_off + (16 + shift)
+    torch.cuda.synchronize()
+    ctx.wg_decap(lib.make_batch(d_arena, total, n, lib.MEM_DEVICE, offsets=d_off, lens=d_wlen),
+                 lib.make_batch(d_arena, total, n, lib.MEM_DEVICE, offsets=d_out), res, olen, gp, gc)
+    ctx.sync()
+    res, olen = res.cpu().numpy(), olen.cpu().numpy().view(np.uint32)
+    gp, gc = gp.cpu().numpy().view(np.uint32), gc.cpu().numpy()
+    for i in range(n):
+        if unknown[i]:
+            assert (res[i], olen[i], gp[i], gc[i]) == (O.WG_UNKNOWN_INDEX, 0, 0xFFFFFFFF, 0)
+            continue
+        assert gp[i] == peer[i] and gc[i] == int(np.frombuffer(sent[i][8:16], np.uint64)[0])
+        ok = O.WG_AUTH_FAIL if forged[i] else O.WG_KEEPALIVE if lens[i] == 0 else O.WG_BAD_IP if lens[i] < 20 else O.WG_OK
+        assert res[i] == ok and olen[i] == (lens[i] if ok == O.WG_OK else 0), (i, lens[i], res[i])
+    bad = np.flatnonzero(d_arena.cpu().numpy() != want)
+    assert bad.size == 0, f"first differing byte at {bad[:5]}"
+    ctx.close()

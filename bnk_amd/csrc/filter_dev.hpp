@@ -11,9 +11,10 @@ constexpr int64_t FLOW_TOMB = INT64_MIN; // expiry of a deleted (or never used) 
 // Words of FlowTableDev::counters: entries in the map, slots ever claimed; since the last note
 // launch, whether a sweep ran and how many entries it deleted (FLOW_LIVE still counts those);
 // and two int64, no entry of the map expires before FLOW_MIN_EXP (0: nothing known), or before
-// FLOW_NEXT_EXP if a sweep ran.
+// FLOW_NEXT_EXP if a sweep ran.  FLOW_NOTE_BLOCKS: see FilterArgs::record_blocks (0 between launches).
 enum : uint32_t {
-    FLOW_LIVE = 0, FLOW_CLAIMED = 1, FLOW_SWEPT = 2, FLOW_GONE = 3, FLOW_MIN_EXP = 4, FLOW_NEXT_EXP = 6, FLOW_COUNTERS = 8
+    FLOW_LIVE = 0, FLOW_CLAIMED = 1, FLOW_SWEPT = 2, FLOW_GONE = 3, FLOW_MIN_EXP = 4, FLOW_NEXT_EXP = 6, FLOW_NOTE_BLOCKS = 8,
+    FLOW_COUNTERS = 10
 };
 constexpr int64_t FLOW_TTL_LEAST = 30000000000LL; // filter.go:108-117: nothing is stored for less
 
@@ -102,6 +103,8 @@ struct FilterArgs {
     uint32_t record_seq;  // claimed by the batches up to that number, or more (see flows_reserve)
     bool record_after;    // note only: and record_seq << 32 | slots once this launch, the last of its
                           // batch, has ended
+    uint32_t record_blocks; // set by the launcher: the launch has that many workgroups with packets, and the
+                          // last of them to be done leaves that record (0: it does not)
     RuleIndexDev rules;
     FlowTableDev flows;
 };
@@ -114,6 +117,12 @@ hipError_t launch_filter_check(const FilterArgs &a, uint32_t max_blocks, hipStre
 // claimed_upper: the host's upper bound on claimed slots.  Up to 4096 the
 // sweep cannot fire and its launch is left out.
 hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
+// The sweep alone, behind a launch that has noted the batch.
+hipError_t launch_flow_sweep(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
+// launch_peer_rank_small (kernels.hpp), advancing, and launch_filter_note on the same batch in one launch.
+hipError_t launch_peer_rank_small_note(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
+                                       uint64_t *ctr_out, uint64_t ctr_limit, uint32_t *status, const FilterArgs &note,
+                                       uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
 hipError_t launch_flow_rehash(const FlowTableDev &from, const FlowTableDev &to, uint32_t *status,
                               uint32_t max_blocks, hipStream_t s);
 

@@ -27,132 +27,10 @@
 // expiry FLOW_TOMB.
 #include "../../include/bnkhip.h"
 #include "filter_dev.hpp"
+#include "filter_lane.hpp"
 #include "kernels.hpp"
 
 namespace bnk {
-
-#define BNK_DEV __device__ __forceinline__
-
-BNK_DEV uint32_t ld32u(const uint8_t *p)
-{
-    uint32_t v;
-    __builtin_memcpy(&v, p, 4);
-    return v;
-}
-
-struct Parsed {
-    uint32_t src, dst;
-    uint32_t sport, dport;
-    uint32_t proto;
-};
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef u32x4 __attribute__((aligned(1))) u32x4_unaligned;
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef u32x2 __attribute__((aligned(1))) u32x2_unaligned;
-
-// filter.go:71-106.  Bytes 0-15 come in one load and bytes 16-23 (destination
-// and, without IP options, the ports) in a second when the packet has them:
-// every load instruction here reads 64 different lines, so their number is
-// what the kernel pays for.
-// Where packet i lies in its arena, worked out only when somebody asks.
-struct PacketAt {
-    const uint8_t *pkts;
-    const uint64_t *off;
-    uint32_t stride, i;
-    BNK_DEV const uint8_t *get() const { return pkts + (off ? off[i] : (uint64_t)i * stride); }
-};
-
-// `p`: the packet's first 24 bytes (as many as it has); `full`: the packet
-// where it lies, looked at only for a header with options.
-BNK_DEV bool parse_words(const u32x4 a, uint32_t dst_w, uint32_t l4_w, bool wide, uint32_t len, Parsed &o,
-                         const PacketAt &full)
-{
-    const uint32_t w0 = a.x;
-    if (((w0 >> 4) & 0xFu) != 4u) return false;
-    const uint32_t ihl = (w0 & 0xFu) * 4u;
-    if (ihl < 20u || len < ihl) return false;
-    o.proto = (a.z >> 8) & 0xFFu;
-    o.src = __builtin_bswap32(a.w);
-    o.dst = __builtin_bswap32(dst_w);
-    const uint32_t body = len - ihl;
-    if (o.proto == 6u || o.proto == 17u) {
-        if (body < 4u) return false;
-        const uint32_t w = __builtin_bswap32(wide && ihl == 20u ? l4_w : ld32u(full.get() + ihl));
-        o.sport = w >> 16;
-        o.dport = w & 0xFFFFu;
-        return true;
-    }
-    if (o.proto == 1u) {
-        if (body < 1u) return false;
-        o.sport = 0;
-        o.dport = 0;
-        return true;
-    }
-    return false;
-}
-
-BNK_DEV bool parse_packet(const uint8_t *p, uint32_t len, Parsed &o, const PacketAt &full)
-{
-    if (len < 20u) return false;
-    const u32x4 a = *reinterpret_cast<const u32x4_unaligned *>(p);
-    uint32_t dst_w, l4_w = 0;
-    const bool wide = len >= 24u;
-    if (wide) {
-        const u32x2 b = *reinterpret_cast<const u32x2_unaligned *>(p + 16);
-        dst_w = b.x;
-        l4_w = b.y;
-    } else {
-        dst_w = ld32u(p + 16);
-    }
-    return parse_words(a, dst_w, l4_w, wide, len, o, full);
-}
-
-BNK_DEV uint32_t proto_class(uint32_t proto) { return proto == 1u ? 0u : proto == 6u ? 1u : 2u; }
-
-// filter.go:108-117
-BNK_DEV int64_t flow_ttl_ns(uint32_t proto)
-{
-    return proto == 6u ? 120000000000LL : 30000000000LL;
-}
-
-BNK_DEV uint64_t mix64(uint64_t x)
-{
-    x ^= x >> 33;
-    x *= 0xff51afd7ed558ccdULL;
-    x ^= x >> 33;
-    x *= 0xc4ceb9fe1a85ec53ULL;
-    x ^= x >> 33;
-    return x;
-}
-
-// The two positions of a key in the small presence bitmap (a Bloom filter with
-// two hash functions over SMALL_BITS bits, which is not a power of two).
-BNK_DEV uint32_t small_bit0(uint64_t hsh) { return __umulhi((uint32_t)(hsh >> 32), SMALL_BITS); }
-BNK_DEV uint32_t small_bit1(uint64_t hsh) { return __umulhi((uint32_t)hsh * 0x9E3779B1u, SMALL_BITS); }
-
-struct FlowSlot {
-    uint64_t word;   // stored key word (never 0)
-    uint32_t base;   // first slot of the region
-    uint32_t start;  // probe start within the region
-    uint32_t bit;    // this key's bit in the presence bitmap
-    uint32_t sbit0, sbit1; // and its two bits in the small one
-};
-
-BNK_DEV FlowSlot flow_slot(const FlowTableDev &ft, uint32_t remote, uint32_t rport, uint32_t lport,
-                           uint32_t proto)
-{
-    FlowSlot s;
-    const uint32_t region = proto_class(proto) * 2u + (remote >> 31);
-    s.word = (1ULL << 63) | ((uint64_t)(remote & 0x7FFFFFFFu) << 32) | ((uint64_t)rport << 16) | lport;
-    s.base = region * ft.cap;
-    const uint64_t hsh = mix64(s.word ^ ((uint64_t)region << 59));
-    s.start = (uint32_t)hsh & (ft.cap - 1u);
-    s.bit = (uint32_t)(hsh >> 32) & ft.present_mask;
-    s.sbit0 = small_bit0(hsh);
-    s.sbit1 = small_bit1(hsh);
-    return s;
-}
 
 // ---- rule lookup ----------------------------------------------------------
 
@@ -553,90 +431,16 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     }
 }
 
-// filter.go:189-201 for a batch (the sweep of :202-208 follows as its own
-// kernel because it depends on the entry count after every insert).
-//
-// A packet of a flow that the table has (nearly all of them, on a link that is
-// in use) costs one 16-byte read and at most a plain store: every lane of the
-// batch writes the same expiry for the key, and nothing is deleted in this
-// launch, so a lane may see the old expiry or the new one.  Only a slot that
-// looks empty or deleted is claimed with atomics, whose answers count; such a
-// look may be out of date (the L2s of the eight XCDs are not coherent), then the
-// atomic says so.  2^18 headers of 65,536 flows: 10.6 us (the slots' lines), with a
-// compare-and-swap and an exchange per packet instead 29.1; behind transport headers
-// in a tunnel's slots, 16,384 flows, 11.9 and 32.1.
+// NoteOutbound of a batch (note_packet); the first workgroup has no packets (note_once).
 __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
 {
     const uint32_t stride = (gridDim.x - 1u) * 256u;
-    // The launch's first workgroup has no packets: its few dependent reads, an atomic and a store
-    // to the host would otherwise be one wave's way to its first packet, and the whole launch waits
-    // for the slowest wave.
     if (blockIdx.x == 0u) {
-        if (threadIdx.x != 0u) return;
-        // What the last sweep left behind is folded in here, so that the next one can read the
-        // entry count and the bound without anybody changing them meanwhile.
-        uint32_t *c = a.flows.counters;
-        int64_t *least = reinterpret_cast<int64_t *>(c + FLOW_MIN_EXP), *next = reinterpret_cast<int64_t *>(c + FLOW_NEXT_EXP);
-        int64_t bound = *least;
-        if (c[FLOW_SWEPT] != 0u) {
-            bound = *next;
-            if (c[FLOW_GONE]) atomicSub(&c[FLOW_LIVE], c[FLOW_GONE]);
-            c[FLOW_GONE] = 0u;
-            c[FLOW_SWEPT] = 0u;
-        }
-        *next = INT64_MAX;
-        *least = a.now + FLOW_TTL_LEAST < bound ? a.now + FLOW_TTL_LEAST : bound;
-        // (at least what the batches before this one claimed)
-        if (a.record)
-            __hip_atomic_store(a.record, (uint64_t)(a.record_seq - 1u) << 32 | atomicAdd(&c[FLOW_CLAIMED], 0u),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (threadIdx.x == 0u) note_once(a);
         return;
     }
-    for (uint32_t i = (blockIdx.x - 1u) * 256u + threadIdx.x; i < a.n; i += stride) {
-        const uint64_t at = a.off ? a.off[i] : (uint64_t)i * a.stride;
-        const uint32_t len = a.lens ? a.lens[i] : a.len;
-        if (beyond_arena(at, a.ahead, len, a.limit)) {
-            status_raise(a.status, STATUS_BOUNDS);
-            continue;
-        }
-        const uint8_t *p = a.pkts + at;
-        Parsed h;
-        if (!parse_packet(p, len, h, PacketAt{a.pkts, a.off, a.stride, i})) continue;
-        // remote = dst, remotePort = dstPort, localPort = srcPort
-        const FlowSlot s = flow_slot(a.flows, h.dst, h.dport, h.sport, h.proto);
-        const unsigned long long expiry = (unsigned long long)(a.now + flow_ttl_ns(h.proto));
-        bool placed = false;
-        for (uint32_t probe = 0; probe < a.flows.cap; probe++) {
-            const uint32_t at_slot = s.base + ((s.start + probe) & (a.flows.cap - 1u));
-            FlowSlotMem *slot = a.flows.slots + at_slot;
-            unsigned long long *kp = reinterpret_cast<unsigned long long *>(&slot->key);
-            unsigned long long *ep = reinterpret_cast<unsigned long long *>(&slot->exp);
-            const ulonglong2 cur = *reinterpret_cast<const ulonglong2 *>(slot);
-            if (cur.x != 0ULL && cur.x != s.word) continue; // (a key stays where it is)
-            if (cur.x == s.word && (int64_t)cur.y != FLOW_TOMB) {
-                if (cur.y != expiry) *ep = expiry;
-                placed = true;
-                break;
-            }
-            const unsigned long long old = cur.x ? cur.x : atomicCAS(kp, 0ULL, (unsigned long long)s.word);
-            if (old == 0ULL) {
-                const uint32_t pos = atomicAdd(&a.flows.counters[FLOW_CLAIMED], 1u);
-                if (pos < a.flows.cap / 2u) a.flows.list[pos] = at_slot; // (flows_reserve keeps it below)
-                atomicOr(&a.flows.present[s.bit >> 5], 1u << (s.bit & 31u));
-                atomicOr(&a.flows.present_small[s.sbit0 >> 5], 1u << (s.sbit0 & 31u));
-                atomicOr(&a.flows.present_small[s.sbit1 >> 5], 1u << (s.sbit1 & 31u));
-            }
-            if (old == 0ULL || old == s.word) {
-                // the lane that replaces a tombstone (fresh slots start as
-                // tombstones) brings the entry into the map
-                const int64_t prev = (int64_t)atomicExch(ep, expiry);
-                if (prev == FLOW_TOMB) atomicAdd(&a.flows.counters[FLOW_LIVE], 1u);
-                placed = true;
-                break;
-            }
-        }
-        if (!placed) status_raise(a.status, STATUS_FLOWS_FULL);
-    }
+    for (uint32_t i = (blockIdx.x - 1u) * 256u + threadIdx.x; i < a.n; i += stride) note_packet(a, i);
+    note_block_done(a);
 }
 
 // (FilterArgs::record_after)
@@ -804,12 +608,25 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
     return hipGetLastError();
 }
 
-hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
+// A launch of few workgroups counts them and leaves the record itself (23 ns a workgroup, where a
+// launch for it costs 4 us); of many, a launch behind it does.
+constexpr uint32_t NOTE_COUNTED_BLOCKS = 64;
+
+hipError_t launch_filter_note(const FilterArgs &args, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
 {
-    if (a.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(filter_note_kernel, dim3(grid_for(a.n, max_blocks) + 1u), dim3(256), 0, s, a);
-    if (a.record && a.record_after)
+    if (args.n == 0) return hipSuccess;
+    FilterArgs a = args;
+    const uint32_t blocks = grid_for(a.n, max_blocks);
+    const bool record = a.record && a.record_after;
+    a.record_blocks = record && blocks <= NOTE_COUNTED_BLOCKS ? blocks : 0u;
+    hipLaunchKernelGGL(filter_note_kernel, dim3(blocks + 1u), dim3(256), 0, s, a);
+    if (record && !a.record_blocks)
         hipLaunchKernelGGL(note_record_kernel, dim3(1), dim3(1), 0, s, a.record, a.record_seq, a.flows.counters);
+    return launch_flow_sweep(a, max_blocks, claimed_upper, s);
+}
+
+hipError_t launch_flow_sweep(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
+{
     // filter.go:202: no sweep while the map holds at most 4096 entries
     if (claimed_upper <= 4096u) return hipGetLastError();
     const uint32_t most = (uint32_t)(claimed_upper < a.flows.cap / 2u ? claimed_upper : a.flows.cap / 2u);

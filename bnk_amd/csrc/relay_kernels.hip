@@ -14,6 +14,7 @@
 
 #include "../../include/bnkhip.h"
 #include "block_sort.hpp"
+#include "filter_lane.hpp"
 #include "kernels.hpp"
 
 namespace bnk {
@@ -208,14 +209,22 @@ hipError_t launch_relay_assign(const uint8_t *auth, const uint8_t *pass, const u
                             const_cast<uint64_t *>(ctr_base_out), n_peers_out, n, ctr_out, advance, 0ull, s);
 }
 
-// Batch-order counters for a small batch in one launch of one block, straight
-// from the peer array: a stable block-wide radix sort of (peer, position)
+// The batch-order counters of a small batch, by one workgroup.
+struct RankArgs {
+    const uint32_t *peer; // or nullptr: every packet is peer 0
+    uint32_t n_keys, n;
+    uint64_t *ctr_base, *ctr_out;
+    int advance, no_peer_ok;
+    unsigned bits; // of a key
+    uint64_t ctr_limit;
+    uint32_t *status;
+};
+
+// Straight from the peer array: a stable block-wide radix sort of (peer, position)
 // brings each peer's packets together in batch order; a packet's rank is its
 // distance from the head of its run, and the last packet of a run moves the
 // peer's base.
-__global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
-    const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
-    int advance, int no_peer_ok, unsigned bits, uint64_t ctr_limit, uint32_t *status)
+BNK_DEV void peer_rank_small(const RankArgs &a)
 {
     using Sort = rocprim::block_radix_sort<uint32_t, PEER_RANK_SMALL_MAX, 1, uint32_t>;
     using Scan = rocprim::block_scan<uint32_t, PEER_RANK_SMALL_MAX>;
@@ -226,16 +235,16 @@ __global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
     __shared__ uint32_t sk[PEER_RANK_SMALL_MAX + 1];
     const uint32_t t = threadIdx.x;
     uint32_t key[1] = {NO_PEER}, pos[1] = {t};
-    if (t < n) {
-        key[0] = peer ? peer[t] : 0u;
-        if (key[0] >= n_keys) {
-            if (!(no_peer_ok && key[0] == NO_PEER)) status_raise(status, STATUS_PEER_RANGE);
+    if (t < a.n) {
+        key[0] = a.peer ? a.peer[t] : 0u;
+        if (key[0] >= a.n_keys) {
+            if (!(a.no_peer_ok && key[0] == NO_PEER)) status_raise(a.status, STATUS_PEER_RANGE);
             key[0] = NO_PEER;
         }
     }
     // valid keys are below n_keys < 2^bits and "no peer" is all ones, so the low
     // bits order them the way the full word does, "no peer" last
-    Sort().sort(key, pos, tmp.sort, 0, bits);
+    Sort().sort(key, pos, tmp.sort, 0, a.bits);
     sk[t] = key[0];
     if (t == 0) sk[PEER_RANK_SMALL_MAX] = NO_PEER;
     __syncthreads();
@@ -246,11 +255,11 @@ __global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
     Scan().inclusive_scan(head ? t : 0u, start, tmp.scan, rocprim::maximum<uint32_t>());
     uint64_t mine = 0;
     if (valid) {
-        mine = ctr_add(ctr_base[key[0]], t - start, ctr_limit);
-        ctr_out[pos[0]] = mine;
+        mine = ctr_add(a.ctr_base[key[0]], t - start, a.ctr_limit);
+        a.ctr_out[pos[0]] = mine;
     }
     __syncthreads(); // every base has been read
-    if (advance && valid && last) ctr_base[key[0]] = ctr_add(mine, 1u, ctr_limit);
+    if (a.advance && valid && last) a.ctr_base[key[0]] = ctr_add(mine, 1u, a.ctr_limit);
 }
 
 // The same for up to PEER_RANK_BLOCK_MAX packets, four a thread, peer and position sorted as
@@ -259,10 +268,9 @@ __global__ __launch_bounds__(PEER_RANK_SMALL_MAX) void peer_rank_small_kernel(
 // here 8.)
 constexpr uint32_t PEER_BLOCK_THREADS = BLOCK_SORT_THREADS, PEER_BLOCK_ITEMS = BLOCK_SORT_ITEMS;
 constexpr unsigned PEER_BLOCK_INDEX_BITS = 12;
+static_assert(PEER_RANK_SMALL_MAX == PEER_BLOCK_THREADS, "one launch shape");
 static_assert(PEER_RANK_BLOCK_MAX == 1u << PEER_BLOCK_INDEX_BITS && PEER_RANK_BLOCK_MAX == BLOCK_SORT_WORDS, "packed keys");
-__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
-    const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
-    int advance, int no_peer_ok, unsigned bits, uint64_t ctr_limit, uint32_t *status)
+BNK_DEV void peer_rank_block(const RankArgs &a)
 {
     constexpr uint32_t ROWS = PEER_RANK_BLOCK_MAX / 64u;
     static_assert(ROWS == 64u, "a lane per row");
@@ -270,19 +278,19 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
     __shared__ uint32_t sk[PEER_RANK_BLOCK_MAX + 1];
     __shared__ uint32_t last_head[ROWS];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-    const uint32_t none = (1u << bits) - 1u; // above every peer
+    const uint32_t none = (1u << a.bits) - 1u; // above every peer
     uint32_t word[PEER_BLOCK_ITEMS];
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
         const uint32_t i = block_sort_place(j);
         uint32_t key = NO_PEER;
-        if (i < n) {
-            key = peer ? peer[i] : 0u;
-            if (key >= n_keys && !(no_peer_ok && key == NO_PEER)) status_raise(status, STATUS_PEER_RANGE);
+        if (i < a.n) {
+            key = a.peer ? a.peer[i] : 0u;
+            if (key >= a.n_keys && !(a.no_peer_ok && key == NO_PEER)) status_raise(a.status, STATUS_PEER_RANGE);
         }
-        word[j] = (key < n_keys ? key : none) << PEER_BLOCK_INDEX_BITS | i;
+        word[j] = (key < a.n_keys ? key : none) << PEER_BLOCK_INDEX_BITS | i;
     }
-    block_sort(word, PEER_BLOCK_INDEX_BITS, bits, sort);
+    block_sort(word, PEER_BLOCK_INDEX_BITS, a.bits, sort);
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) sk[j * PEER_BLOCK_THREADS + t] = word[j] >> PEER_BLOCK_INDEX_BITS;
     if (t == 0) sk[PEER_RANK_BLOCK_MAX] = NO_PEER;
@@ -319,14 +327,39 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_block_kernel(
         const uint32_t p = j * PEER_BLOCK_THREADS + t, key = word[j] >> PEER_BLOCK_INDEX_BITS;
         mine[j] = 0;
         if (key == none) continue;
-        mine[j] = ctr_add(ctr_base[key], p - start[j], ctr_limit);
-        ctr_out[word[j] & (PEER_RANK_BLOCK_MAX - 1u)] = mine[j];
+        mine[j] = ctr_add(a.ctr_base[key], p - start[j], a.ctr_limit);
+        a.ctr_out[word[j] & (PEER_RANK_BLOCK_MAX - 1u)] = mine[j];
     }
     __syncthreads(); // every base has been read
 #pragma unroll
     for (uint32_t j = 0; j < PEER_BLOCK_ITEMS; j++) {
         const uint32_t p = j * PEER_BLOCK_THREADS + t, key = word[j] >> PEER_BLOCK_INDEX_BITS;
-        if (advance && key != none && sk[p + 1u] != key) ctr_base[key] = ctr_add(mine[j], 1u, ctr_limit);
+        if (a.advance && key != none && sk[p + 1u] != key) a.ctr_base[key] = ctr_add(mine[j], 1u, a.ctr_limit);
+    }
+}
+
+template <bool SMALL>
+__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_kernel(RankArgs a)
+{
+    SMALL ? peer_rank_small(a) : peer_rank_block(a);
+}
+
+// NoteOutbound on the packets of such a batch as well, which has nothing to do with its counters: the
+// first workgroup ranks, the second does what a note launch does once, the others note.  In launches of
+// their own, one behind the other (4 us each, and 3 for the host to launch one), device-resident tunnel
+// passes of 256 packets took 31.7 us in a row against 29.1, of 3000 70.5 against 65.1; 128 packets in
+// pinned rings through the tunnel 67.5 against 63.7.
+template <bool SMALL>
+__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_note_kernel(RankArgs a, FilterArgs note)
+{
+    if (blockIdx.x == 0u) {
+        SMALL ? peer_rank_small(a) : peer_rank_block(a);
+    } else if (blockIdx.x == 1u) {
+        if (threadIdx.x == 0u) note_once(note);
+    } else {
+        const uint32_t i = (blockIdx.x - 2u) * PEER_BLOCK_THREADS + threadIdx.x;
+        if (i < note.n) note_packet(note, i);
+        note_block_done(note);
     }
 }
 
@@ -339,12 +372,8 @@ static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_ke
                                              uint64_t *ctr_out, bool advance, bool no_peer_ok, uint64_t ctr_limit,
                                              uint32_t *status, hipStream_t s)
 {
-    if (n <= PEER_RANK_SMALL_MAX)
-        hipLaunchKernelGGL(peer_rank_small_kernel, dim3(1), dim3(PEER_RANK_SMALL_MAX), 0, s, peer, n_keys, n,
-                           ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status);
-    else
-        hipLaunchKernelGGL(peer_rank_block_kernel, dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, peer, n_keys, n,
-                           ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status);
+    const RankArgs a{peer, n_keys, n, ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status};
+    hipLaunchKernelGGL(n <= PEER_RANK_SMALL_MAX ? peer_rank_kernel<true> : peer_rank_kernel<false>, dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, a);
     return hipGetLastError();
 }
 
@@ -355,6 +384,21 @@ hipError_t launch_peer_rank_small(const uint32_t *peer, uint32_t n_keys, uint32_
     if (n == 0) return hipSuccess;
     if (!peer_rank_one_block(n, n_keys)) return hipErrorInvalidValue;
     return launch_peer_rank_one_block(peer, n_keys, n, ctr_base, ctr_out, advance, false, ctr_limit, status, s);
+}
+
+hipError_t launch_peer_rank_small_note(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
+                                       uint64_t *ctr_out, uint64_t ctr_limit, uint32_t *status, const FilterArgs &note,
+                                       uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    if (!peer_rank_one_block(n, n_keys) || note.n != n) return hipErrorInvalidValue;
+    const RankArgs a{peer, n_keys, n, ctr_base, ctr_out, 1, 0, key_bits(n_keys), ctr_limit, status};
+    FilterArgs f = note;
+    const uint32_t blocks = (n + PEER_BLOCK_THREADS - 1u) / PEER_BLOCK_THREADS;
+    f.record_blocks = f.record && f.record_after ? blocks : 0u;
+    hipLaunchKernelGGL(n <= PEER_RANK_SMALL_MAX ? peer_rank_note_kernel<true> : peer_rank_note_kernel<false>, dim3(blocks + 2u),
+                       dim3(PEER_BLOCK_THREADS), 0, s, a, f);
+    return launch_flow_sweep(f, max_blocks, claimed_upper, s);
 }
 
 // ---------------------------------------------------------------------------

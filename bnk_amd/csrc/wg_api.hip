@@ -417,11 +417,47 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
     uint32_t *d_padded = ctx->wg_padded.as<uint32_t>();
     uint8_t *d_skip = ctx->wg_skip.as<uint8_t>();
 
+    // filter.go:192-194: NoteOutbound does nothing in allow-all mode
+    const bool note = note_now != nullptr && ctx->filter->enforce;
+    if (note) {
+        rc = flows_reserve(ctx, n);
+        if (rc) return rc;
+    }
+    // NoteOutbound of packets [lo, hi)
+    const auto note_args = [&](uint32_t lo, uint32_t hi) {
+        const FilterState *f = ctx->filter;
+        FilterArgs fa{};
+        fa.pkts = b.base + 16 + (b.off ? 0 : (uint64_t)lo * slots->stride);
+        fa.off = b.off ? b.off + lo : nullptr;
+        fa.lens = b.lens ? b.lens + lo : nullptr;
+        fa.stride = slots->stride;
+        fa.len = slots->len;
+        // (the header's room counts: a slot begins where the arena does)
+        fa.limit = b.limit;
+        fa.ahead = 16;
+        fa.status = ctx->d_status;
+        fa.now = *note_now;
+        fa.n = hi - lo;
+        fa.rules = f->ridx;
+        fa.flows = f->flows;
+        fa.record = f->d_record;
+        fa.record_seq = f->bound.seq;
+        fa.record_after = f->record_after && hi == n;
+        return fa;
+    };
+    bool noted = false;
+
     // counters in batch order per peer, advancing the peers' send counters:
     // needs the peer array only, so it runs ahead of the packet bytes
     if (peer_rank_one_block(n, pe.n)) {
-        HIPCHK(ctx, launch_peer_rank_small(d_peer, pe.n, n, pe.send_ctr, d_ctr, true, WG_REJECT_AFTER_MESSAGES,
-                                           ctx->d_status, ctx->stream));
+        if (note && !chunked) {
+            HIPCHK(ctx, launch_peer_rank_small_note(d_peer, pe.n, n, pe.send_ctr, d_ctr, WG_REJECT_AFTER_MESSAGES, ctx->d_status,
+                                                    note_args(0, n), ctx->filter->max_blocks, ctx->filter->bound.upper, ctx->stream));
+            noted = true;
+        } else {
+            HIPCHK(ctx, launch_peer_rank_small(d_peer, pe.n, n, pe.send_ctr, d_ctr, true, WG_REJECT_AFTER_MESSAGES,
+                                               ctx->d_status, ctx->stream));
+        }
     } else if (d_peer && peer_rank_counts(n, pe.n, tmp_bytes)) {
         HIPCHK(ctx, launch_peer_rank_counting(d_peer, ctx->r_tmp.p, pe.send_ctr, pe.n, n, d_ctr, true,
                                               WG_REJECT_AFTER_MESSAGES, ctx->d_status, ctx->stream));
@@ -434,40 +470,14 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
                                      ctx->stream));
     }
 
-    // filter.go:192-194: NoteOutbound does nothing in allow-all mode
-    const bool note = note_now != nullptr && ctx->filter->enforce;
-    if (note) {
-        rc = flows_reserve(ctx, n);
-        if (rc) return rc;
-    }
-
     // NoteOutbound, then header, padding and seal of packets [lo, hi)
     auto run = [&](uint32_t lo, uint32_t hi) -> int {
         WgBatch c = b;
         c.first = lo;
         c.n = hi - lo;
         uint8_t *sealed = ring_out ? ring_out : const_cast<uint8_t *>(b.base);
-        if (note) {
-            FilterState *f = ctx->filter;
-            FilterArgs fa{};
-            fa.pkts = b.base + 16 + (b.off ? 0 : (uint64_t)lo * slots->stride);
-            fa.off = b.off ? b.off + lo : nullptr;
-            fa.lens = b.lens ? b.lens + lo : nullptr;
-            fa.stride = slots->stride;
-            fa.len = slots->len;
-            // (the header's room counts: a slot begins where the arena does)
-            fa.limit = b.limit;
-            fa.ahead = 16;
-            fa.status = ctx->d_status;
-            fa.now = *note_now;
-            fa.n = hi - lo;
-            fa.rules = f->ridx;
-            fa.flows = f->flows;
-            fa.record = f->d_record;
-            fa.record_seq = f->bound.seq;
-            fa.record_after = f->record_after && hi == n;
-            HIPCHK(ctx, launch_filter_note(fa, f->max_blocks, f->bound.upper, ctx->stream));
-        }
+        if (note && !noted)
+            HIPCHK(ctx, launch_filter_note(note_args(lo, hi), ctx->filter->max_blocks, ctx->filter->bound.upper, ctx->stream));
         if (host || !ctx->wg_unfused) {
             AeadArgs se{};
             se.spread_max = ctx->spread_max;

@@ -15,6 +15,7 @@
 #include "../../include/bnkhip.h"
 #include "aead_route.hpp"
 #include "kernels.hpp"
+#include "wg_small_dev.hpp"
 
 namespace bnk {
 
@@ -826,10 +827,10 @@ BNK_DEV void replay_key(const AeadArgs &a, uint32_t i, uint32_t sender)
 // What WireGuard does with a datagram whose tag has been checked: keepalive, IP
 // version, the trim to the IP header's total length, the sender's allowed prefix.
 // c0: the first 16 bytes of the plaintext, kept when they went through the cipher.
-BNK_DEV void decap_result(const AeadArgs &a, uint32_t i, bool have, bool reject, uint32_t len, const uint4 c0,
-                          uint32_t pr)
+BNK_DEV uint32_t decap_verdict(const AeadArgs &a, bool have, bool reject, uint32_t len, const uint4 c0, uint32_t pr, uint32_t &out_len)
 {
-    uint32_t res = BNK_WG_OK, out_len = 0;
+    uint32_t res = BNK_WG_OK;
+    out_len = 0;
     const uint32_t version = (c0.x >> 4) & 0xFu;
     if (!have || reject) res = BNK_WG_AUTH_FAIL; // (no packet here: it reached beyond the output arena)
     else if (len == 0u) res = BNK_WG_KEEPALIVE;
@@ -845,6 +846,14 @@ BNK_DEV void decap_result(const AeadArgs &a, uint32_t i, bool have, bool reject,
         const uint32_t total = (__builtin_bswap32(c0.y) >> 16) + 40u;
         res = (len < 40u || total > len) ? BNK_WG_BAD_IP : BNK_WG_NOT_ALLOWED;
     } else res = BNK_WG_BAD_IP;
+    return res;
+}
+
+BNK_DEV void decap_result(const AeadArgs &a, uint32_t i, bool have, bool reject, uint32_t len, const uint4 c0,
+                          uint32_t pr)
+{
+    uint32_t out_len;
+    const uint32_t res = decap_verdict(a, have, reject, len, c0, pr, out_len);
     a.wg.result[i] = (uint8_t)res;
     a.wg.out_len[i] = out_len;
     replay_key(a, i, res != BNK_WG_AUTH_FAIL ? pr : 0xFFFFFFFFu);
@@ -1499,6 +1508,14 @@ BNK_DEV void fetch_part(const uint8_t *src, uint32_t there, uint32_t first, uint
     }
 }
 
+// A packet's first 64 bytes in the first four lanes (zeros behind its end).
+BNK_DEV uint4 first_cells(const uint8_t *p, uint32_t len, uint32_t lane)
+{
+    const uint32_t off = 16u * (lane & 3u);
+    if (off + 16u <= len) return ld16(p + off);
+    return off < len ? ld_partial(p + off, len - off) : make_uint4(0, 0, 0, 0);
+}
+
 // Cell number `cell` of a packet of len bytes, its last bytes only where it has no more.
 BNK_DEV void store_cell(uint8_t *dst, uint32_t len, uint32_t cell, uint4 v)
 {
@@ -1554,13 +1571,21 @@ BNK_DEV uint32_t half_wave_sum(uint32_t x)
 // Same results as wg_parse_kernel / wg_encap_prep_kernel / wg_finish_kernel
 // around a plain launch.
 constexpr uint32_t LONG_CELLS = 192; // with their 48 blocks and block 0 the rows of a wave hold them
-template <bool OPEN, bool WG>
-__global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
+// A packet that has been through all of it but for its bytes on the way out.
+struct SpreadPacket {
+    const uint8_t *src;
+    uint8_t *dst;
+    uint32_t len, cells;
+    uint32_t key_b, key_c, n1, n2;
+    uint4 o[4];
+    bool reject, is_long;
+};
+
+// Packet w of the launch, up to its tag and what is said about it; false: there is nothing to store.
+// SMALL: of a launch that does the whole batch (wg_small.hpp), which leaves a record instead.
+template <bool OPEN, bool WG, bool SMALL>
+BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, uint8_t *stage, uint32_t lane, uint32_t w, SpreadPacket &p)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t tile_all[WAVES_PER_BLOCK][64 * LDS_ROW];
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t w = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
-    if (w >= a.n) return;
     // everything up to the per-lane work below is uniform across the wave
     const uint32_t i = a.first + w;
     // The packet's entries in the per-packet arrays, every one loaded whether or not the
@@ -1593,7 +1618,7 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
     // it would wrap is beyond any arena)
     const bool huge = (WG && OPEN && len >= 16u ? len - 16u : len) > MAX_PACKET_BYTES;
     const bool wraps = huge && (a.in_limit | a.out_limit) != 0;
-    bool outside;
+    bool outside, plain_inside = false; // (what NoteOutbound asks for)
     if (!WG) {
         // (a launch that checks has no skip here: the kernel that framed the packets has looked
         // at their raw offsets.  Taking skip and offset apart costs a launch of 2900 packets 1 %.)
@@ -1606,12 +1631,13 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
                 status_raise(a.status, STATUS_BOUNDS);
                 if (OPEN) refuse();
             }
-            return;
+            return false;
         }
     } else if (!OPEN) {
         // the slot from its first byte to the end of the tag
         wire_pad = huge ? 0u : wg_padding(len, a.wg.mtu);
         const uint32_t padded = len + wire_pad;
+        plain_inside = !beyond_arena(in_at, 16u, len, a.in_limit);
         outside = wraps || beyond_arena(in_at, 16u, padded, a.in_limit) || beyond_arena(out_at, 16u, (uint64_t)padded + 16u, a.out_limit);
     } else {
         // the datagram where it is read, and the plaintext where it would be written
@@ -1631,14 +1657,14 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
         data_len = OPEN ? (len >= 16u ? len - 16u : 0u) : len;
         data_there = data_len;
     } else if (!OPEN) {
-        data_there = outside ? 0u : len;
+        data_there = outside && !(SMALL && plain_inside) ? 0u : len;
         data_len = outside ? 0u : len + wire_pad;
     } else {
         data_len = framed ? len - 32u : 0u;
         data_there = data_len;
     }
     const uint8_t *const tag_at = data + data_len;
-    if (data_len > SPREAD_MAX_LEN) data_there = 0; // (its parts are fetched further down)
+    if (data_len > SPREAD_MAX_LEN || data_there > SPREAD_MAX_LEN) data_there = 0; // (its parts are fetched further down)
     // The wave fetches the packet in pieces of 1 KB, lane l taking bytes [16 l,
     // 16 l + 16) of each piece, so that an instruction reads 1 KB in a row (64
     // bytes a lane would be sixty-four small requests an instruction, each of
@@ -1651,11 +1677,17 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
     uint32_t key_b = 0, key_c = 0;   // and its words of the key
     uint4 wg_head = make_uint4(0, 0, 0, 0);
     uint32_t wg_remote = 0;
+    uint64_t ctr_small = 0; // the peer's next counter as the batch found it
+    SendRank rank{0u, false};
     if (!(WG && OPEN)) {
         const uint32_t known = pr < (WG ? a.wg.n_peers : a.n_peers) ? pr : 0u; // (the table has a row 0)
         key_b = a.keys[8u * known + quad];
         key_c = a.keys[8u * known + 4u + quad];
         if (WG) wg_remote = a.wg.remote_index[known];
+        if (WG && SMALL) {
+            ctr_small = t.send_ctr[known];
+            rank = send_rank(a.peer, a.n, i, pr, lane);
+        }
     } else {
         wg_head = ld16(len >= 32u && !outside ? src : safe);
     }
@@ -1678,31 +1710,42 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
     // further down: looking at it here would make the key wait for the packet)
 
     if (!WG) {
-        if (skipped) return;
+        if (skipped) return false;
         if (pr >= a.n_peers) {
             if (lane == 0) {
                 status_raise(a.status, STATUS_PEER_RANGE);
                 if (OPEN) refuse();
             }
-            return;
+            return false;
         }
         if (OPEN && len < 16u) {
             if (lane == 0) refuse();
-            return;
+            return false;
         }
         if (OPEN) len -= 16u;
         ctr = a.counters ? ctr_ld : a.counter0 + i;
     } else if (!OPEN) {
         // ---- encapsulate: header into the headroom, padding as implied zeros ----
-        ctr = ctr_ld;
+        if (SMALL) {
+            const bool known = pr < a.wg.n_peers;
+            ctr = ctr_add(ctr_small, rank.ahead, WG_REJECT_AFTER_MESSAGES);
+            encap_record(t.records, i, lane, known && !rank.later ? pr : 0xFFFFFFFFu, ctr_add(ctr, 1u, WG_REJECT_AFTER_MESSAGES));
+        } else {
+            ctr = ctr_ld;
+        }
         // (a keypair that has used up its nonces sends nothing more)
         if (pr >= a.wg.n_peers || outside || ctr >= WG_REJECT_AFTER_MESSAGES) {
+            if (SMALL && t.filter) {
+                // NoteOutbound comes ahead of all that
+                if (plain_inside) note_end(f, lane, note_begin(f, lane, first_cells(data, len, lane), len));
+                else if (lane == 0) status_raise(a.status, STATUS_BOUNDS);
+            }
             if (lane == 0) {
                 a.wg.wire_len[i] = 0;
                 if (pr >= a.wg.n_peers) status_raise(a.status, STATUS_PEER_RANGE);
                 else if (outside) status_raise(a.status, STATUS_BOUNDS);
             }
-            return;
+            return false;
         }
         len += wire_pad;
         if (lane == 0) {
@@ -1741,6 +1784,10 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
             if (hit == 0ull) res = BNK_WG_UNKNOWN_INDEX;
             else pr = (uint32_t)__shfl((int)e.y, __ffsll((long long)hit) - 1, 64);
         }
+        if (SMALL && res != BNK_WG_OK) {
+            decap_record(t.records, i, lane, 0xFFFFFFFFu, 0ull, res, 0u, CHECK_DENY, 0u);
+            return false;
+        }
         if (res != BNK_WG_OK) {
             if (lane == 0) {
                 a.wg.result[i] = res;
@@ -1748,19 +1795,20 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
                 a.wg.peer_out[i] = 0xFFFFFFFFu;
                 a.wg.counter_out[i] = 0;
             }
-            return;
+            return false;
         }
         ctr = (uint64_t)h.z | (uint64_t)h.w << 32;
-        if (lane == 0) {
+        if (!SMALL && lane == 0) {
             a.wg.peer_out[i] = pr;
             a.wg.counter_out[i] = ctr;
         }
         if (wraps) { // (reported as one that does not verify, by the lane kernels too)
+            if (SMALL) decap_record(t.records, i, lane, pr, ctr, BNK_WG_AUTH_FAIL, 0u, CHECK_DENY, 0u);
             if (lane == 0) {
                 status_raise(a.status, STATUS_BOUNDS);
-                decap_result(a, i, false, false, 0u, make_uint4(0, 0, 0, 0), pr);
+                if (!SMALL) decap_result(a, i, false, false, 0u, make_uint4(0, 0, 0, 0), pr);
             }
-            return;
+            return false;
         }
         len -= 32u; // header and tag
         src += 16;
@@ -1773,7 +1821,6 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
 
     // ---- the keystream, block 0 and those of the data (whose bytes fly: see the top of the kernel) ----
     // Block b lies at stage + 80 b (rows padded against bank conflicts).
-    uint8_t *const stage = tile_all[threadIdx.x >> 6];
     const bool is_long = len > SPREAD_MAX_LEN; // (the same in every lane)
     const uint32_t passes = is_long ? 4u : (len + 63u) / 64u / 16u + 1u; // of sixteen blocks
     if (passes == 1u) {
@@ -1803,6 +1850,7 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
     // ---- crypt: o = m ^ keystream; the MAC reads the ciphertext side ----
     if (!tagged) want_tag = make_uint4(0, 0, 0, 0);
     uint4 o[4] = {};
+    uint4 header = make_uint4(0, 0, 0, 0); // (encapsulating: the packet's first bytes, for NoteOutbound)
     Fe26 acc = fe_small(0);
     auto take_cell = [&](uint32_t cell, const uint4 &c) __attribute__((always_inline)) {
         Fe26 next = fe_cell(c.x, c.y, c.z, c.w);
@@ -1818,6 +1866,7 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
             // a cell beyond the packet's whole cells is zeros, but for its last 1-15 bytes
             if (off + 16u > data_there) m = make_uint4(0, 0, 0, 0);
             if (odd_mine && (odd_at >> 10) == j) m = odd_cell;
+            if (WG && !OPEN && SMALL && j == 0u) header = m;
             o[j] = m ^ keystream(j);
             if (64u * (j + 1u) >= cells && (len & 15u) != 0u) // the last cell is among these
                 o[j] = o[j] & byte_mask(64u * j + lane == cells - 1u ? len & 15u : 16u);
@@ -1825,6 +1874,7 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
         }
     } else {
         const uint32_t there = WG && !OPEN ? len - wire_pad : len;
+        if (WG && !OPEN && SMALL) header = first_cells(src, there, lane);
 #pragma unroll 1
         for (uint32_t first = 0; first < cells; first += LONG_CELLS) {
             if (!OPEN && first != 0u) {
@@ -1849,6 +1899,16 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
             }
         }
     }
+    // (what the filter needs to know is on its way while the tag is worked out)
+    WaveNote note{};
+    if (WG && !OPEN && SMALL && t.filter) note = note_begin(f, lane, header, len - wire_pad);
+    uint4 first_cell = make_uint4(0, 0, 0, 0);
+    WaveCheck check{};
+    if (WG && OPEN && SMALL) {
+        first_cell = make_uint4((uint32_t)__builtin_amdgcn_readlane((int)o[0].x, 0), (uint32_t)__builtin_amdgcn_readlane((int)o[0].y, 0),
+                                (uint32_t)__builtin_amdgcn_readlane((int)o[0].z, 0), (uint32_t)__builtin_amdgcn_readlane((int)o[0].w, 0));
+        if (t.filter) check = check_begin(f, lane, o[0], min(len, __builtin_bswap32(first_cell.x) & 0xFFFFu));
+    }
     const Fe26 term = fe_mul(acc, lift);
 
     // ---- the sum of the lanes' terms: 32 lanes fit 32 bits per limb ----
@@ -1872,6 +1932,7 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
             st16(dst + len, make_uint4(tag[0], tag[1], tag[2], tag[3]));
             if (WG && a.tally) tally_bump(a.tally, TALLY_SEALED, 1u);
         }
+        if (WG && SMALL && t.filter) note_end(f, lane, note);
     } else {
         // all 16 bytes are compared, no early exit
         reject = ((want_tag.x ^ tag[0]) | (want_tag.y ^ tag[1]) | (want_tag.z ^ tag[2]) |
@@ -1883,35 +1944,141 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
     }
     // what wireguard-go checks once a packet is authentic (lane 0 has the first 16 plaintext bytes,
     // which hold every field used)
-    if (WG && OPEN && lane == 0) decap_result(a, i, true, reject, len, o[0], pr);
+    if (WG && OPEN && SMALL) {
+        uint32_t out_len;
+        const uint32_t res = decap_verdict(a, true, reject, len, first_cell, pr, out_len);
+        const uint32_t action = t.filter && res == BNK_WG_OK ? check_end(f, lane, check) : CHECK_DENY;
+        decap_record(t.records, i, lane, pr, ctr, res, out_len, action, check.h.proto);
+    } else if (WG && OPEN && lane == 0) {
+        decap_result(a, i, true, reject, len, o[0], pr);
+    }
+    p.src = src;
+    p.dst = dst;
+    p.len = len;
+    p.cells = cells;
+    p.key_b = key_b;
+    p.key_c = key_c;
+    p.n1 = n1;
+    p.n2 = n2;
+    p.reject = reject;
+    p.is_long = is_long;
+#pragma unroll
+    for (int j = 0; j < 4; j++) p.o[j] = o[j];
+    return true;
+}
 
-    // ---- the bytes out, the way they came in; a rejected packet leaves zeros
-    // (chacha20poly1305.Open) ----
-    if (__builtin_expect(!is_long, 1)) {
+// The bytes out, the way they came in; a rejected packet leaves zeros (chacha20poly1305.Open).
+template <bool OPEN>
+BNK_DEV void spread_store(const SpreadPacket &p, uint8_t *stage, uint32_t lane, const uint8_t *safe)
+{
+    const uint32_t len = p.len, cells = p.cells, quad = lane & 3u;
+    if (__builtin_expect(!p.is_long, 1)) {
 #pragma unroll
         for (uint32_t j = 0; j < 4; j++)
-            if (64u * j + lane < cells) store_cell(dst, len, 64u * j + lane, reject ? make_uint4(0, 0, 0, 0) : o[j]);
+            if (64u * j + lane < cells) store_cell(p.dst, len, 64u * j + lane, p.reject ? make_uint4(0, 0, 0, 0) : p.o[j]);
     } else if (OPEN) {
-        const bool backwards = (uintptr_t)dst > (uintptr_t)src;
+        auto keystream = [&](uint32_t j) __attribute__((always_inline)) {
+            return *reinterpret_cast<const uint4 *>(stage + (1u + 16u * j + (lane >> 2)) * LDS_ROW + 16u * quad);
+        };
+        const bool backwards = (uintptr_t)p.dst > (uintptr_t)p.src;
         const uint32_t last = (cells - 1u) / LONG_CELLS * LONG_CELLS;
 #pragma unroll 1
         for (uint32_t done = 0; done < cells; done += LONG_CELLS) {
             const uint32_t first = backwards ? last - done : done;
-            quad_blocks<2>(stage, lane, key_b, key_c, first / 4u, n1, n2);
-            quad_blocks<2>(stage + 32 * LDS_ROW, lane, key_b, key_c, first / 4u + 32u, n1, n2);
+            quad_blocks<2>(stage, lane, p.key_b, p.key_c, first / 4u, p.n1, p.n2);
+            quad_blocks<2>(stage + 32 * LDS_ROW, lane, p.key_b, p.key_c, first / 4u + 32u, p.n1, p.n2);
             wave_sync();
             uint4 m[3];
-            fetch_part(src, len, first, lane, safe, m);
+            fetch_part(p.src, len, first, lane, safe, m);
             // (the next lane's cell may lie where mine goes: all of them are here before any goes out)
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
             for (uint32_t j = 0; j < 3; j++) {
                 const uint32_t cell = first + 64u * j + lane;
-                if (cell < cells) store_cell(dst, len, cell, reject ? make_uint4(0, 0, 0, 0) : m[j] ^ keystream(j));
+                if (cell < cells) store_cell(p.dst, len, cell, p.reject ? make_uint4(0, 0, 0, 0) : m[j] ^ keystream(j));
             }
         }
     }
+}
+
+template <bool OPEN, bool WG>
+__global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t tile_all[WAVES_PER_BLOCK][64 * LDS_ROW];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
+    if (w >= a.n) return;
+    uint8_t *const stage = tile_all[threadIdx.x >> 6];
+    SpreadPacket p;
+    if (spread_packet<OPEN, WG, false>(a, TunnelSmall{}, FilterArgs{}, stage, lane, w, p))
+        spread_store<OPEN>(p, stage, lane, reinterpret_cast<const uint8_t *>(a.keys));
+}
+
+// A tunnel call of a small batch in one launch (wg_small.hpp).  Encapsulating, every wave notes its
+// packet's flow and counts the packets of its peer ahead of its own (a workgroup behind those with
+// packets does what a note launch does once); decapsulating, every wave looks its packet up in the
+// filter; and the workgroup that has its packets done last moves the peers' counters, or takes the
+// batch through the windows and says what has become of each packet.
+//
+// Launches are what small batches cost: 4 us each in a row, and as much of the chip with several streams
+// at work, whatever is in them.  128 packets in pinned rings out and back 63.7 -> 48.9 us (kernels 13.5
+// and 17, in place of 4.5 + 12 and 12 + 6 + 6.6), device-resident passes of 256 with three streams at
+// work 21.0 -> 12.5.
+template <bool OPEN>
+__global__ __launch_bounds__(256, 4) void tunnel_small_kernel(AeadArgs a, TunnelSmall t, FilterArgs f)
+{
+    static_assert(256u == WG_SMALL_MAX && 64u * WAVES_PER_BLOCK == WG_SMALL_MAX, "a thread per packet at the end");
+    __shared__ union {
+        __attribute__((aligned(16))) uint8_t tile[WAVES_PER_BLOCK][64 * LDS_ROW];
+        SmallWindows windows;
+    } sh;
+    __shared__ bool last;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t blocks = (a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK;
+    if (!OPEN && blockIdx.x >= blocks) {
+        if (threadIdx.x == 0u) note_once(f);
+        return;
+    }
+    const uint32_t w = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
+    uint8_t *const stage = sh.tile[threadIdx.x >> 6];
+    SpreadPacket p;
+    bool out = false;
+    if (w < a.n) out = spread_packet<OPEN, true, true>(a, t, f, stage, lane, w, p);
+    // (the records are where others see them before the workgroup is counted; the packet's bytes go
+    // out meanwhile)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0u) {
+        const bool mine = __hip_atomic_fetch_add(t.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == blocks;
+        if (mine) __hip_atomic_store(t.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = mine;
+    }
+    if (out) spread_store<OPEN>(p, stage, lane, reinterpret_cast<const uint8_t *>(a.keys));
+    __syncthreads();
+    if (!last) return;
+    if (OPEN) decap_finish(t, a, f, sh.windows);
+    else encap_finish(t, f, a.n, a.wg.n_peers);
+}
+
+hipError_t launch_tunnel_seal_small(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, uint32_t max_blocks,
+                                    uint64_t claimed_upper, hipStream_t s)
+{
+    if (a.n == 0) return hipSuccess;
+    if (a.n > WG_SMALL_MAX || a.first != 0u || a.wg.mode != WG_FUSE_ENCAP || a.in_skip != 0u || (t.filter && f.n != a.n)) return hipErrorInvalidValue;
+    FilterArgs note = f;
+    note.record_blocks = f.record && f.record_after ? 1u : 0u; // (the last workgroup leaves the record)
+    const uint32_t blocks = (a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK;
+    hipLaunchKernelGGL(tunnel_small_kernel<false>, dim3(blocks + (t.filter ? 1u : 0u)), dim3(256), 0, s, a, t, note);
+    return t.filter ? launch_flow_sweep(note, max_blocks, claimed_upper, s) : hipGetLastError();
+}
+
+hipError_t launch_tunnel_open_small(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, hipStream_t s)
+{
+    if (a.n == 0) return hipSuccess;
+    if (a.n > WG_SMALL_MAX || a.first != 0u || a.wg.mode != WG_FUSE_DECAP || a.in_skip != 0u) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(tunnel_small_kernel<true>, dim3((a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK), dim3(256), 0, s, a, t, f);
+    return hipGetLastError();
 }
 
 // Can the host tell that every wave of the launch takes the short path?  One

@@ -68,12 +68,6 @@ BNK_DEV uint32_t interval_of_jump(const uint32_t *bounds, const uint16_t *jump, 
     return lo;
 }
 
-// One word holds a range: key_lo << 14 | key_hi - key_lo.  How far the key lies beyond it, 0 in it.
-BNK_DEV uint32_t range_miss(uint32_t e, uint32_t key)
-{
-    return __builtin_elementwise_sub_sat(key - (e >> 14), e & RANGE_MAX_SPAN);
-}
-
 // 0 if one of the four has the key.  (As a chain of comparisons the compiler tests one word,
 // branches, and fetches the next ones only then.)
 BNK_DEV uint32_t quad_miss(uint4 v, uint32_t key)

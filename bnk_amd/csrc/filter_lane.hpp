@@ -132,7 +132,13 @@ BNK_DEV FlowSlot flow_slot(const FlowTableDev &ft, uint32_t remote, uint32_t rpo
     return s;
 }
 
-// filter.go:189-201 for packet i of a batch (the sweep of :202-208 follows as its own
+// One word holds a range: key_lo << 14 | key_hi - key_lo.  How far the key lies beyond it, 0 in it.
+BNK_DEV uint32_t range_miss(uint32_t e, uint32_t key)
+{
+    return __builtin_elementwise_sub_sat(key - (e >> 14), e & RANGE_MAX_SPAN);
+}
+
+// filter.go:195-201 for one packet of a batch (the sweep of :202-208 follows as its own
 // kernel because it depends on the entry count after every insert).
 //
 // A packet of a flow that the table has (nearly all of them, on a link that is
@@ -144,17 +150,8 @@ BNK_DEV FlowSlot flow_slot(const FlowTableDev &ft, uint32_t remote, uint32_t rpo
 // atomic says so.  2^18 headers of 65,536 flows: 10.6 us (the slots' lines), with a
 // compare-and-swap and an exchange per packet instead 29.1; behind transport headers
 // in a tunnel's slots, 16,384 flows, 11.9 and 32.1.
-BNK_DEV void note_packet(const FilterArgs &a, uint32_t i)
+BNK_DEV void note_flow(const FilterArgs &a, const Parsed &h)
 {
-    const uint64_t at = a.off ? a.off[i] : (uint64_t)i * a.stride;
-    const uint32_t len = a.lens ? a.lens[i] : a.len;
-    if (beyond_arena(at, a.ahead, len, a.limit)) {
-        status_raise(a.status, STATUS_BOUNDS);
-        return;
-    }
-    const uint8_t *p = a.pkts + at;
-    Parsed h;
-    if (!parse_packet(p, len, h, PacketAt{a.pkts, a.off, a.stride, i})) return;
     // remote = dst, remotePort = dstPort, localPort = srcPort
     const FlowSlot s = flow_slot(a.flows, h.dst, h.dport, h.sport, h.proto);
     const unsigned long long expiry = (unsigned long long)(a.now + flow_ttl_ns(h.proto));
@@ -189,6 +186,21 @@ BNK_DEV void note_packet(const FilterArgs &a, uint32_t i)
         }
     }
     if (!placed) status_raise(a.status, STATUS_FLOWS_FULL);
+}
+
+// filter.go:189-201 for packet i of a batch.
+BNK_DEV void note_packet(const FilterArgs &a, uint32_t i)
+{
+    const uint64_t at = a.off ? a.off[i] : (uint64_t)i * a.stride;
+    const uint32_t len = a.lens ? a.lens[i] : a.len;
+    if (beyond_arena(at, a.ahead, len, a.limit)) {
+        status_raise(a.status, STATUS_BOUNDS);
+        return;
+    }
+    const uint8_t *p = a.pkts + at;
+    Parsed h;
+    if (!parse_packet(p, len, h, PacketAt{a.pkts, a.off, a.stride, i})) return;
+    note_flow(a, h);
 }
 
 // What a note launch does once, by one thread of a workgroup that has no packets: its few

@@ -5,6 +5,7 @@
 #include "api_common.hpp"
 #include "filter_host.hpp"
 #include "wg_dev.hpp"
+#include "wg_small.hpp"
 
 using namespace bnk;
 
@@ -28,6 +29,18 @@ int upload(bnk_ctx *ctx, DevBuf *dst, const void *src, size_t bytes)
     HIPCHK(ctx, dst->reserve(bytes));
     HIPCHK(ctx, hipMemcpyAsync(dst->p, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return BNK_OK;
+}
+
+// What a launch that does a whole small batch shares among its workgroups.
+TunnelSmall small_view(bnk_ctx *ctx, bool filter)
+{
+    TunnelSmall t{};
+    t.arrived = ctx->wg_small.as<uint32_t>();
+    t.records = t.arrived + 16;
+    t.send_ctr = ctx->wg_send_ctr.as<uint64_t>();
+    t.windows = ctx->wg_replay_on ? ctx->wg_replay : nullptr;
+    t.filter = filter;
+    return t;
 }
 
 } // namespace
@@ -136,6 +149,10 @@ extern "C" int bnk_wg_peers_set(bnk_ctx *ctx, const bnk_wg_peer *peers, uint32_t
                           ctx->wg_rows[i].remote_index == peers[i].remote_index;
         if (!same) ctr[i] = 0;
         fresh[i] = same ? 0 : 1; // the anti-replay window belongs to the keypair as well
+    }
+    if (!ctx->wg_small.p) {
+        HIPCHK(ctx, ctx->wg_small.reserve(WG_SMALL_BYTES));
+        HIPCHK(ctx, launch_fill_u32(ctx->wg_small.as<uint32_t>(), WG_SMALL_BYTES / 4u, 0u, ctx->stream));
     }
     rc = wg_upload_index(ctx, index);
     if (!rc) rc = upload(ctx, &ctx->wg_remote, remote.data(), (size_t)n * 4);
@@ -446,10 +463,41 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         return fa;
     };
     bool noted = false;
+    // A launch of a wave per packet over whole slots, which does the framing itself.
+    const auto whole_slots = [&](uint32_t lo, uint32_t hi) {
+        AeadArgs se{};
+        se.spread_max = ctx->spread_max;
+        se.over_link = over_link;
+        se.keys = ctx->d_keys[BNK_KEYS_SEND];
+        se.n_peers = pe.n;
+        se.status = ctx->d_status;
+        se.first = lo;
+        se.n = hi - lo;
+        se.in = b.base;
+        se.out = ring_out ? ring_out : const_cast<uint8_t *>(b.base);
+        se.in_off = se.out_off = b.off;
+        se.in_stride = se.out_stride = slots->stride;
+        se.lens = b.lens;
+        se.len = slots->len;
+        se.peer = d_peer;
+        se.counters = d_ctr;
+        se.in_limit = se.out_limit = b.limit;
+        se.wg.mode = WG_FUSE_ENCAP;
+        se.wg.n_peers = pe.n;
+        se.wg.mtu = mtu;
+        se.wg.remote_index = pe.remote_index;
+        se.wg.wire_len = d_wire_len;
+        if (!host && counted && ctx->tally_on.load(std::memory_order_relaxed)) se.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
+        if (se.tally && aead_runs_spread(se)) *counted = true;
+        return se;
+    };
 
+    // A small batch in one launch: counters, NoteOutbound and the packets.
+    const bool small = n <= WG_SMALL_MAX && !chunked && !ctx->wg_unfused && aead_runs_spread(whole_slots(0, n));
     // counters in batch order per peer, advancing the peers' send counters:
     // needs the peer array only, so it runs ahead of the packet bytes
-    if (peer_rank_one_block(n, pe.n)) {
+    if (small) {
+    } else if (peer_rank_one_block(n, pe.n)) {
         if (note && !chunked) {
             HIPCHK(ctx, launch_peer_rank_small_note(d_peer, pe.n, n, pe.send_ctr, d_ctr, WG_REJECT_AFTER_MESSAGES, ctx->d_status,
                                                     note_args(0, n), ctx->filter->max_blocks, ctx->filter->bound.upper, ctx->stream));
@@ -476,36 +524,16 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         c.first = lo;
         c.n = hi - lo;
         uint8_t *sealed = ring_out ? ring_out : const_cast<uint8_t *>(b.base);
+        if (small) {
+            HIPCHK(ctx, launch_tunnel_seal_small(whole_slots(lo, hi), small_view(ctx, note), note ? note_args(lo, hi) : FilterArgs{},
+                                                 ctx->filter->max_blocks, ctx->filter->bound.upper, ctx->stream));
+            return BNK_OK;
+        }
         if (note && !noted)
             HIPCHK(ctx, launch_filter_note(note_args(lo, hi), ctx->filter->max_blocks, ctx->filter->bound.upper, ctx->stream));
         if (host || !ctx->wg_unfused) {
-            AeadArgs se{};
-            se.spread_max = ctx->spread_max;
-            se.over_link = over_link;
-            se.keys = ctx->d_keys[BNK_KEYS_SEND];
-            se.n_peers = pe.n;
-            se.status = ctx->d_status;
-            se.first = lo;
-            se.n = hi - lo;
-            se.in = b.base;
-            se.out = sealed;
-            se.in_off = se.out_off = b.off;
-            se.in_stride = se.out_stride = slots->stride;
-            se.lens = b.lens;
-            se.len = slots->len;
-            se.peer = d_peer;
-            se.counters = d_ctr;
-            se.in_limit = se.out_limit = b.limit;
+            const AeadArgs se = whole_slots(lo, hi);
             if (aead_runs_spread(se)) {
-                se.wg.mode = WG_FUSE_ENCAP;
-                se.wg.n_peers = pe.n;
-                se.wg.mtu = mtu;
-                se.wg.remote_index = pe.remote_index;
-                se.wg.wire_len = d_wire_len;
-                if (!host && counted && ctx->tally_on.load(std::memory_order_relaxed)) {
-                    se.tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
-                    *counted = true;
-                }
                 HIPCHK(ctx, launch_aead_seal(se, ctx->stream));
                 return BNK_OK;
             }
@@ -859,16 +887,14 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
 
     // CheckInbound of what packets [lo, hi) delivered: a packet that was not
     // delivered has length 0 here, which the filter refuses without a side effect
-    auto filter_range = [&](uint32_t lo, uint32_t hi) -> int {
-        if (!check) return BNK_OK;
-        FilterState *f = ctx->filter;
-        uint8_t *d_pass = ctx->r_pass.as<uint8_t>();
+    const auto check_args = [&](uint32_t lo, uint32_t hi) {
+        const FilterState *f = ctx->filter;
         FilterArgs fa{};
         fa.pkts = ob.base + (ob.off ? 0 : (uint64_t)lo * out->stride);
         fa.off = ob.off ? ob.off + lo : nullptr;
         fa.lens = d_out_len + lo;
         fa.stride = out->stride;
-        fa.verdict = d_pass + lo;
+        fa.verdict = ctx->r_pass.as<uint8_t>() + lo;
         fa.status = ctx->d_status;
         fa.now = *check_now;
         fa.n = hi - lo;
@@ -880,7 +906,10 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
             fa.wg_tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);
             *counted = true;
         }
-        HIPCHK(ctx, launch_filter_check(fa, f->max_blocks, ctx->stream));
+        return fa;
+    };
+    auto filter_range = [&](uint32_t lo, uint32_t hi) -> int {
+        if (check) HIPCHK(ctx, launch_filter_check(check_args(lo, hi), ctx->filter->max_blocks, ctx->stream));
         return BNK_OK;
     };
 
@@ -917,6 +946,11 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
                 op.wg.out_len = d_out_len;
                 op.wg.peer_out = d_peer;
                 op.wg.counter_out = d_counter;
+                if (n <= WG_SMALL_MAX && !chunked && !ctx->wg_unfused && (replay || check)) {
+                    // a small batch in one launch: the windows and CheckInbound as well
+                    HIPCHK(ctx, launch_tunnel_open_small(op, small_view(ctx, check), check ? check_args(lo, hi) : FilterArgs{}, ctx->stream));
+                    return BNK_OK;
+                }
                 HIPCHK(ctx, launch_aead_open(op, ctx->stream));
                 if (int rr = replay_range(lo, hi)) return rr;
                 return filter_range(lo, hi);

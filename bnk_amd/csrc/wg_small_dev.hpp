@@ -1,0 +1,362 @@
+// The parts of a small tunnel launch (wg_small.hpp) that are not the AEAD's: a packet's send counter,
+// CheckInbound of one packet by a wave, the anti-replay windows of the whole batch by one workgroup.
+//
+// What a wave leaves for the workgroup that ends the launch it stores past the caches (agent scope: the
+// L2s of the eight XCDs are not coherent), waits for, and then its workgroup counts itself in
+// `arrived`; whoever completes the number reads the records the same way.  Nobody waits for anybody.
+#pragma once
+
+#include "filter_lane.hpp"
+#include "wg_small.hpp"
+#include "wg_window.hpp"
+
+namespace bnk {
+
+BNK_DEV void record_put(uint32_t *at, uint32_t v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+BNK_DEV uint32_t record_get(const uint32_t *at) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// How many packets ahead of packet i have its peer, and whether one behind it has.
+struct SendRank {
+    uint32_t ahead;
+    bool later;
+};
+BNK_DEV SendRank send_rank(const uint32_t *peer, uint32_t n, uint32_t i, uint32_t mine, uint32_t lane)
+{
+    static_assert(WG_SMALL_MAX == 256u, "four loads a lane, all in flight together");
+    SendRank r{0u, false};
+    if (!peer) return SendRank{i, i + 1u < n};
+    uint32_t p[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) p[j] = peer[min(64u * j + lane, n - 1u)];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t u = 64u * j + lane;
+        const bool same = u < n && p[j] == mine;
+        r.ahead += (uint32_t)__popcll(__ballot(same && u < i));
+        r.later |= __ballot(same && u > i) != 0ull;
+    }
+    return r;
+}
+
+// The IPv4 header of a packet whose first 64 bytes lie in the first four lanes' cells (parse_words,
+// filter.go:71-106); len: of the packet.  The same for every lane.
+BNK_DEV bool wave_parse(const uint4 &c0, uint32_t len, Parsed &h)
+{
+    const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)c0.x, 0), w2 = (uint32_t)__builtin_amdgcn_readlane((int)c0.z, 0);
+    const uint32_t ihl = (w0 & 0xFu) * 4u;
+    h.proto = (w2 >> 8) & 0xFFu;
+    h.src = __builtin_bswap32((uint32_t)__builtin_amdgcn_readlane((int)c0.w, 0));
+    h.dst = __builtin_bswap32((uint32_t)__builtin_amdgcn_readlane((int)c0.x, 1));
+    const bool ports = h.proto == 6u || h.proto == 17u;
+    // the ports lie behind the header, in a word of their own of one of the first four lanes
+    const uint32_t part = (ihl >> 2) & 3u;
+    const uint32_t word = part < 2u ? (part == 0u ? c0.x : c0.y) : part == 2u ? c0.z : c0.w;
+    const uint32_t p = ports ? __builtin_bswap32((uint32_t)__builtin_amdgcn_readlane((int)word, (int)(ihl >> 4))) : 0u;
+    h.sport = p >> 16;
+    h.dport = p & 0xFFFFu;
+    return len >= 20u && ((w0 >> 4) & 0xFu) == 4u && ihl >= 20u && (ports || h.proto == 1u) && len >= ihl + (ports ? 4u : 1u);
+}
+
+// NoteOutbound of one packet by a wave: a flow that the table has (note_flow) is found with a look at
+// a line of slots that is on its way while the tag is worked out; another is one lane's work.
+struct WaveNote {
+    Parsed h;
+    bool valid;
+    FlowSlot slot;
+    ulonglong2 probe;
+};
+constexpr uint32_t WAVE_PROBES = 8; // lanes, a 128-byte line of slots
+
+BNK_DEV ulonglong2 wave_probe(const FlowTableDev &ft, const FlowSlot &s, uint32_t from, uint32_t lane)
+{
+    return *reinterpret_cast<const ulonglong2 *>(ft.slots + s.base + ((s.start + from + (lane & (WAVE_PROBES - 1u))) & (ft.cap - 1u)));
+}
+
+BNK_DEV WaveNote note_begin(const FilterArgs &f, uint32_t lane, const uint4 &c0, uint32_t len)
+{
+    WaveNote w{};
+    w.valid = wave_parse(c0, len, w.h);
+    // remote = dst, remotePort = dstPort, localPort = srcPort
+    w.slot = flow_slot(f.flows, w.h.dst, w.h.dport, w.h.sport, w.h.proto);
+    w.probe = wave_probe(f.flows, w.slot, 0u, lane);
+    return w;
+}
+
+BNK_DEV void note_end(const FilterArgs &f, uint32_t lane, const WaveNote &w)
+{
+    if (!w.valid) return;
+    const uint64_t expiry = (uint64_t)(f.now + flow_ttl_ns(w.h.proto));
+    const unsigned long long here = __ballot(lane < WAVE_PROBES && (w.probe.x == 0ull || w.probe.x == w.slot.word));
+    const uint32_t at = here ? (uint32_t)__ffsll((long long)here) - 1u : 0u;
+    const bool known = __ballot(lane == at && here != 0ull && w.probe.x == w.slot.word && (int64_t)w.probe.y != FLOW_TOMB) != 0ull;
+    if (!known) {
+        if (lane == 0u) note_flow(f, w.h);
+    } else if (lane == at && w.probe.y != expiry) {
+        f.flows.slots[w.slot.base + ((w.slot.start + at) & (f.flows.cap - 1u))].exp = (int64_t)expiry;
+    }
+}
+
+// CheckInbound (filter.go:121-147) of one packet by a wave.  Three trips to memory at most where one lane takes a dozen: the first probes of
+// the flow table and the place of the source among the cut points at once, the 64 cut points there, and
+// the interval's rule list.  What it would do to the flow table is left for when the packet's counter
+// has been through the window.
+constexpr uint32_t CHECK_DENY = 0u, CHECK_PASS = 1u, CHECK_REFRESH = 2u, CHECK_DELETE = 3u; // low two bits; above them a slot
+struct WaveCheck {
+    Parsed h;
+    bool valid;
+    FlowSlot slot;
+    ulonglong2 probe;  // the first slots, one a lane
+    uint32_t cut;      // bounds[lane] where there are no more than 64
+    uint32_t first, last; // else, with a jump table, where the source's cut points are
+};
+
+BNK_DEV bool few_cuts(const RuleIndexDev &ri) { return ri.n_bounds <= 64u; }
+
+// c0: the lane's first cell; len: of the inner packet.
+BNK_DEV WaveCheck check_begin(const FilterArgs &f, uint32_t lane, const uint4 &c0, uint32_t len)
+{
+    WaveCheck w{};
+    w.valid = wave_parse(c0, len, w.h);
+    // return traffic: remote = src, remotePort = srcPort, localPort = dstPort
+    w.slot = flow_slot(f.flows, w.h.src, w.h.sport, w.h.dport, w.h.proto);
+    w.probe = wave_probe(f.flows, w.slot, 0u, lane);
+    const RuleIndexDev &ri = f.rules;
+    if (few_cuts(ri)) {
+        w.cut = ri.bounds[min(lane, ri.n_bounds - 1u)];
+    } else if (ri.jump) {
+        uint32_t b = (w.h.src - ri.jump_lo) >> ri.jump_shift;
+        b = min(b, JUMP_BUCKETS - 1u);
+        w.first = ri.jump[b];
+        w.last = ri.jump[b + 1u];
+    }
+    return w;
+}
+
+// Largest j in [lo, hi) with word(j) <= v, or lo: words ascend.  64 of them at a time.
+template <class F>
+BNK_DEV uint32_t wave_search(uint32_t lo, uint32_t hi, uint32_t v, uint32_t lane, F word)
+{
+    while (hi - lo > 64u) {
+        const uint32_t step = (hi - lo + 63u) / 64u;
+        const uint32_t at = min(lo + lane * step, hi - 1u);
+        const uint32_t below = (uint32_t)__popcll(__ballot(word(at) <= v));
+        const uint32_t from = min(lo + (below ? below - 1u : 0u) * step, hi - 1u);
+        hi = min(from + step, hi);
+        lo = from;
+    }
+    const bool mine = lo + lane < hi;
+    const uint32_t below = (uint32_t)__popcll(__ballot(mine && word(min(lo + lane, hi - 1u)) <= v));
+    return lo + (below ? below - 1u : 0u);
+}
+
+BNK_DEV uint32_t check_end(const FilterArgs &f, uint32_t lane, const WaveCheck &w)
+{
+    if (!w.valid) return CHECK_DENY;
+    const RuleIndexDev &ri = f.rules;
+    const uint32_t key = proto_class(w.h.proto) << 16 | w.h.dport;
+    uint32_t iv;
+    if (few_cuts(ri)) {
+        const uint32_t below = (uint32_t)__popcll(__ballot(lane < ri.n_bounds && w.cut <= w.h.src));
+        iv = below ? below - 1u : 0u;
+    } else {
+        uint32_t lo = 0, hi = ri.n_bounds;
+        if (ri.jump) { // (see interval_of_jump)
+            const bool in = w.h.src >= ri.jump_lo;
+            lo = in ? w.first : 0u;
+            hi = in ? w.last + 1u : 1u;
+        }
+        const uint32_t *const bounds = ri.bounds;
+        iv = wave_search(lo, hi, w.h.src, lane, [bounds](uint32_t j) { return bounds[j]; });
+    }
+    const uint32_t *list = ri.ranges + (size_t)iv * RANGE_BLOCK;
+    uint32_t mine = list[lane & (RANGE_BLOCK - 1u)];
+    const uint32_t head = (uint32_t)__builtin_amdgcn_readlane((int)mine, 0);
+    if (head == RANGE_LONG) { // (see long_list_hit)
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)mine, 1), blocks = (uint32_t)__builtin_amdgcn_readlane((int)mine, 2);
+        const uint32_t *const all = ri.ranges + (size_t)first * RANGE_BLOCK;
+        const uint32_t b = wave_search(0u, blocks, key, lane, [all](uint32_t j) { return all[(size_t)j * RANGE_BLOCK] >> 14; });
+        mine = all[(size_t)b * RANGE_BLOCK + (lane & (RANGE_BLOCK - 1u))];
+    }
+    bool hit = __ballot(range_miss(mine, key) == 0u) != 0ull;
+    for (uint32_t j = 0; !hit && j < ri.n_wide; j += 64u) {
+        const uint4 r = ri.wide[min(j + lane, ri.n_wide - 1u)];
+        hit = __ballot((w.h.src & r.y) == r.x && key >= r.z && key <= r.w) != 0ull;
+    }
+    if (hit) return CHECK_PASS;
+    ulonglong2 cur = w.probe;
+    for (uint32_t from = 0; from < f.flows.cap; from += WAVE_PROBES) {
+        if (from != 0u) cur = wave_probe(f.flows, w.slot, from, lane);
+        const unsigned long long here = __ballot(lane < WAVE_PROBES && (cur.x == 0ull || cur.x == w.slot.word));
+        if (here == 0ull) continue;
+        const int at = __ffsll((long long)here) - 1;
+        const uint32_t found = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cur.x >> 32), at) | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cur.x, at);
+        const int64_t e = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(cur.y >> 32), at) << 32 |
+                                    (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)cur.y, at));
+        if (found == 0u || e == FLOW_TOMB) return CHECK_DENY; // never stored, or deleted earlier
+        const uint32_t index = w.slot.base + ((w.slot.start + from + (uint32_t)at) & (f.flows.cap - 1u));
+        return index << 2 | (f.now < e ? CHECK_REFRESH : CHECK_DELETE);
+    }
+    return CHECK_DENY;
+}
+
+// What a decapsulated packet's wave leaves: its sender and counter, what the open has made of it, and
+// what the filter would do with it.
+BNK_DEV void decap_record(uint32_t *records, uint32_t i, uint32_t lane, uint32_t peer, uint64_t ctr, uint32_t res, uint32_t out_len,
+                          uint32_t action, uint32_t proto)
+{
+    const uint32_t v = lane < 4u ? (lane < 2u ? (lane == 0u ? peer : out_len) : lane == 2u ? res : 0u)
+                                 : lane < 6u ? (lane == 4u ? action : proto) : (uint32_t)(lane == 6u ? ctr : ctr >> 32);
+    if (lane < WG_SMALL_RECORD) record_put(records + WG_SMALL_RECORD * i + lane, v);
+}
+// And an encapsulated one's: its peer's next counter where it is the peer's last of the batch.
+BNK_DEV void encap_record(uint32_t *records, uint32_t i, uint32_t lane, uint32_t peer, uint64_t next)
+{
+    const uint32_t v = lane == 0u ? peer : lane == 1u ? (uint32_t)next : (uint32_t)(next >> 32);
+    if (lane < 3u) record_put(records + WG_SMALL_RECORD * i + lane, v);
+}
+
+BNK_DEV void encap_finish(const TunnelSmall &t, const FilterArgs &f, uint32_t n, uint32_t n_peers)
+{
+    const uint32_t i = threadIdx.x;
+    if (i >= n) return;
+    const uint32_t *r = t.records + WG_SMALL_RECORD * i;
+    const uint32_t peer = record_get(r), lo = record_get(r + 1), hi = record_get(r + 2);
+    if (peer < n_peers) t.send_ctr[peer] = (uint64_t)hi << 32 | lo;
+    // (FilterArgs::record_after: claims are atomics whose answers their waves have waited for)
+    if (t.filter && i == 0u && f.record && f.record_after)
+        __hip_atomic_store(f.record, (uint64_t)f.record_seq << 32 | atomicAdd(&f.flows.counters[FLOW_CLAIMED], 0u), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+struct SmallWindows {
+    uint64_t ctr[WG_SMALL_MAX];
+    unsigned long long bit[WG_SMALL_MAX / 64u][32]; // which of a row's 64 packets have a bit of the peer number set
+    unsigned long long subject[WG_SMALL_MAX / 64u];
+};
+
+// The batch's packets through their windows, one a thread (replay_small_kernel's steps, but that the
+// packets of a thread's peer are found by votes per bit of the peer number instead of by sorting), then
+// what the filter does with those that are delivered, and the results.
+//
+// One workgroup, so its chain of trips to memory and barriers is what it costs, at the end of everything
+// else: the windows first, the results, which may go over the link, when nothing is left that waits for
+// a store.
+BNK_DEV void decap_finish(const TunnelSmall &t, const AeadArgs &a, const FilterArgs &f, SmallWindows &sh)
+{
+    constexpr uint32_t NONE = 0xFFFFFFFFu, ROWS = WG_SMALL_MAX / 64u;
+    const uint32_t i = threadIdx.x, lane = i & 63u, row = i >> 6, n = a.n;
+    const bool there = i < n;
+    uint64_t v[4] = {NONE, (uint64_t)BNK_WG_BAD_HEADER, 0, 0};
+    if (there) {
+        const uint64_t *r = reinterpret_cast<const uint64_t *>(t.records + WG_SMALL_RECORD * i);
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) v[q] = __hip_atomic_load(r + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const uint32_t peer = (uint32_t)v[0], action = (uint32_t)v[2], proto = (uint32_t)(v[2] >> 32);
+    const uint64_t c = v[3];
+    uint32_t res = (uint32_t)v[1], out_len = (uint32_t)(v[0] >> 32);
+    if (t.windows) {
+        const bool subject = there && replay_subject((uint8_t)res) && peer < a.wg.n_peers;
+        uint64_t *const st = t.windows + (size_t)(subject ? peer : 0u) * WG_REPLAY_WORDS;
+        const uint64_t last0 = st[0];
+        const bool seen = seen_before(st, c);
+        const uint32_t bits = 32u - (uint32_t)__clz((int)(a.wg.n_peers - 1u));
+        sh.ctr[i] = c;
+        for (uint32_t b = 0; b < bits; b++) {
+            const unsigned long long m = __ballot((peer >> b) & 1u);
+            if (lane == 0u) sh.bit[row][b] = m;
+        }
+        {
+            const unsigned long long m = __ballot(subject);
+            if (lane == 0u) sh.subject[row] = m;
+        }
+        __syncthreads();
+        // the packets of my peer, and among them the one ahead of mine
+        unsigned long long mine[ROWS];
+        uint32_t ahead = NONE;
+        bool later = false;
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++) {
+            unsigned long long m = sh.subject[r];
+            for (uint32_t b = 0; b < bits; b++) m &= (peer >> b) & 1u ? sh.bit[r][b] : ~sh.bit[r][b];
+            const unsigned long long below = r < row ? ~0ull : r == row ? (1ull << lane) - 1ull : 0ull;
+            later |= (m & ~below & ~(r == row ? 1ull << lane : 0ull)) != 0ull;
+            mine[r] = m & below;
+            if (mine[r]) ahead = 64u * r + 63u - (uint32_t)__clzll((long long)mine[r]);
+        }
+        // Counters that rise within every peer need no more than that one: it is the highest so far.
+        uint64_t last = last0;
+        bool dup = false, rises = true;
+        if (subject && ahead != NONE) {
+            const uint64_t before = sh.ctr[ahead];
+            rises = before < c && c < WG_REJECT_AFTER_MESSAGES;
+            last = before > last ? before : last;
+        }
+        if (__syncthreads_or(!rises)) {
+            last = last0;
+            if (subject) {
+#pragma unroll 1
+                for (uint32_t r = 0; r <= row; r++) {
+                    unsigned long long m = r == 0u ? mine[0] : r == 1u ? mine[1] : r == 2u ? mine[2] : mine[3];
+                    while (m) {
+                        const uint64_t cu = sh.ctr[64u * r + (uint32_t)__ffsll((long long)m) - 1u];
+                        m &= m - 1ull;
+                        dup |= cu == c;
+                        if (cu < WG_REJECT_AFTER_MESSAGES && cu > last) last = cu;
+                    }
+                }
+            }
+        }
+        const bool reached = subject && reaches_bit_test(c, last);
+        if (subject && (!reached || dup || (c <= last0 && seen))) {
+            res = BNK_WG_REPLAY;
+            out_len = 0;
+        }
+        // (every window has been read as the batch found it: the barrier above lies between)
+        if (subject && !later) {
+            uint64_t to = last;
+            if (c < WG_REJECT_AFTER_MESSAGES && c > to) to = c;
+            advance_window(st, to);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup"); // (see replay_small_kernel)
+        __syncthreads(); // the cleared blocks are in place before bits go in
+        if (reached) {
+            const uint64_t final_last = *reinterpret_cast<volatile uint64_t *>(st);
+            if ((final_last >> 6) - (c >> 6) < WG_REPLAY_BLOCKS)
+                atomicOr(reinterpret_cast<unsigned long long *>(&st[1u + ((c >> 6) & (WG_REPLAY_BLOCKS - 1u))]), 1ull << (c & 63u));
+        }
+    }
+    if (t.filter && there && res == BNK_WG_OK) {
+        const uint32_t what = action & 3u;
+        FlowSlotMem *const slot = f.flows.slots + (action >> 2);
+        if (action == CHECK_DENY || what == CHECK_DELETE) res = BNK_WG_FILTERED;
+        if (what == CHECK_REFRESH) slot->exp = f.now + flow_ttl_ns(proto); // (see filter_check_kernel)
+        if (what == CHECK_DELETE) {
+            const int64_t prev = (int64_t)atomicExch(reinterpret_cast<unsigned long long *>(&slot->exp), (unsigned long long)FLOW_TOMB);
+            if (prev != FLOW_TOMB) atomicSub(&f.flows.counters[FLOW_LIVE], 1u);
+        }
+    }
+    if (there) {
+        a.wg.result[i] = (uint8_t)res;
+        a.wg.out_len[i] = out_len;
+        a.wg.peer_out[i] = peer;
+        a.wg.counter_out[i] = c;
+    }
+    if (t.filter && i == 255u) { // (see filter_check_kernel)
+        const int64_t from = f.now + FLOW_TTL_LEAST;
+        for (const uint32_t w : {FLOW_MIN_EXP, FLOW_NEXT_EXP}) {
+            int64_t *least = reinterpret_cast<int64_t *>(f.flows.counters + w);
+            if (from < *least) (void)__hip_atomic_fetch_min(least, from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (f.wg_tally) {
+        uint32_t votes = 0;
+        tally_vote(res, there, lane, votes);
+        if (lane < 16u && votes != 0u && decap_slot(lane) != TALLY_NONE) {
+            tally_bump(f.wg_tally, decap_slot(lane), votes);
+            if (lane == BNK_WG_OK) tally_bump(f.wg_tally, TALLY_ALLOWED, votes);
+        }
+    }
+}
+
+} // namespace bnk

@@ -1735,3 +1735,103 @@ def test_small_device_batches_of_any_length(shift):
     bad = np.flatnonzero(d_arena.cpu().numpy() != want)
     assert bad.size == 0, f"first differing byte at {bad[:5]}"
     ctx.close()
+
+
+@pytest.mark.parametrize("mem", ["device", "ring"])
+@pytest.mark.parametrize("rules", ["few", "many"])
+@pytest.mark.parametrize("n", [1, 5, 64, 255, 256, 257])
+def test_small_tunnel_batches_in_one_launch(n, rules, mem):
+    """Up to 256 packets NoteOutbound + encapsulate and decapsulate + CheckInbound are a launch each.
+    Against the same calls in launches of their own: datagrams, results, counters, windows, flow
+    table and counts over several rounds, with datagrams that come twice, late and out of order,
+    are forged, or carry headers with options, unknown protocols, and replies to flows that the
+    filter knows, does not, or has let expire."""
+    import torch
+    from bnk_amd import lib
+    rng = np.random.default_rng(n * 2 + (rules == "many"))
+    peers = _peers(rng)
+    peers = [(a, a, c, d) for a, _, c, d in peers]  # (one context is both ends)
+    keys = rng.integers(0, 256, (N_PEERS, 32), dtype=np.uint8)
+    acl = [([(0x64400000, 14)], "tcp", [(22, 22), (80, 80), (8000, 8100)])]
+    if rules == "many":
+        acl += [([(0x64400000 + 7 * k, 29)], "udp", [(50 + k % 40, 52 + k % 40)]) for k in range(900)]
+        acl += [([(0x64400000, 20)], "tcp", [(100 + 3 * k, 101 + 3 * k) for k in range(60)]), ([(0, 0)], "icmp", [])]
+    lens = rng.choice([0, 3, 20, 24, 28, 40, 61, 64, 300, 1400, 4100], n).astype(np.uint32)
+    off, total = _layout(rng, lens + 64)
+    dev = torch.device("cuda:0")
+    now = 1_700_000_000_000_000_000
+    sides = []
+    for fused in (True, False):
+        ctx = _ctx(peers, keys, keys)
+        ctx.wg_set_replay(True)
+        ctx.wg_set_fused(fused)
+        ctx.filter_set_rules(acl)
+        new = (lambda k, t: torch.zeros(k, dtype=t, device=dev)) if mem == "device" else (lambda k, t: np.zeros(k, str(t)[6:]))
+        arena = new(total, torch.uint8) if mem == "device" else ctx.ring_alloc(total)
+        out = new(total, torch.uint8) if mem == "device" else ctx.ring_alloc(total)
+        sides.append((ctx, arena, out, [new(n, torch.int32), new(n, torch.uint8), new(n, torch.int32), new(n, torch.int32), new(n, torch.int64)]))
+    kind = lib.MEM_DEVICE if mem == "device" else lib.MEM_HOST
+    up = lambda a, t: torch.from_numpy(np.ascontiguousarray(a).view(t)).to(dev) if mem == "device" else np.ascontiguousarray(a)  # noqa: E731
+    down = lambda a: a.cpu().numpy() if mem == "device" else np.array(a)  # noqa: E731
+    earlier, seen = None, set()
+    for step in range(5):
+        now += int(rng.choice([1, 20, 70, 200])) * 1_000_000_000
+        peer = rng.integers(0, N_PEERS, n).astype(np.uint32)
+        plain = np.zeros(total, np.uint8)
+        for i in range(n):
+            pt = bytearray(_inner(rng, peers, int(peer[i]), int(lens[i])))
+            if len(pt) >= 20:
+                pt[9] = int(rng.choice([1, 6, 6, 17, 17, 50]))
+                pt[16:20] = struct.pack(">I", peers[int(rng.integers(0, N_PEERS))][2])
+                if len(pt) >= 64 and rng.random() < 0.2:
+                    pt[0] = 0x40 | int(rng.integers(4, 16))
+                at = 4 * (pt[0] & 15)
+                if len(pt) >= at + 4:
+                    port = rng.choice([22, 53, 80, 99, 111, 8050], 2)
+                    pt[at:at + 4] = struct.pack(">HH", *(int(p) for p in port))
+            plain[int(off[i]) + 16:int(off[i]) + 16 + len(pt)] = np.frombuffer(bytes(pt), np.uint8)
+        d_off, d_lens, d_peer = up(off, np.int64 if mem == "device" else np.uint64), up(lens, np.int32 if mem == "device" else np.uint32), \
+            up(peer, np.int32 if mem == "device" else np.uint32)
+        swap, forge = rng.permutation(n), rng.random(n) < 0.1
+        got = []
+        for ctx, arena, out, (wlen, res, olen, gp, gc) in sides:
+            arena[:] = torch.from_numpy(plain).to(dev) if mem == "device" else plain
+            out[:] = 0
+            if mem == "device":
+                torch.cuda.synchronize()
+            ctx.wg_note_encap(lib.make_batch(arena, total, n, kind, offsets=d_off, lens=d_lens, peer=d_peer), MTU, now, wlen)
+            ctx.sync()
+            wire, wl = down(arena), down(wlen).view(np.uint32).copy()
+            got.append([wire.copy(), wl])
+            # datagrams of one slot size trade places, some come a second time, and some of an earlier round
+            for a, b in zip(swap[::2], swap[1::2]):
+                if lens[a] == lens[b] and wl[a] == wl[b]:
+                    x, y, k = int(off[a]), int(off[b]), int(wl[a])
+                    first = wire[x:x + k].copy()
+                    wire[x:x + k] = wire[y:y + k]
+                    if a % 3:
+                        wire[y:y + k] = first
+            if earlier is not None:
+                for i in range(0, n, 9):
+                    k = int(wl[i])
+                    wire[int(off[i]):int(off[i]) + k] = earlier[int(off[i]):int(off[i]) + k]
+            for i in np.flatnonzero(forge):
+                wire[int(off[i]) + int(wl[i]) - 1] ^= 4
+            arena[:] = torch.from_numpy(wire).to(dev) if mem == "device" else wire
+            if mem == "device":
+                torch.cuda.synchronize()
+            d_out = up(off + np.uint64(16), np.int64 if mem == "device" else np.uint64)
+            lens_in = wlen if mem == "device" else wl
+            ctx.wg_decap_filter(lib.make_batch(arena, total, n, kind, offsets=d_off, lens=lens_in),
+                                lib.make_batch(out, total, n, kind, offsets=d_out), now + 1000, res, olen, gp, gc)
+            ctx.sync()
+            got[-1] += [down(t).copy() for t in (res, olen, gp, gc, out)] + [np.array(ctx.wg_send_counters(N_PEERS)), ctx.filter_flows(),
+                                                                          ctx.filter_flow_count(), ctx.counters()]
+        earlier = got[0][0].copy()
+        for k, (a, b) in enumerate(zip(*got)):
+            assert np.array_equal(a, b) if isinstance(a, np.ndarray) else a == b, (step, k)
+        seen |= set(got[0][2].tolist())
+    if n >= 64:
+        assert {lib.WG_OK, lib.WG_AUTH_FAIL, lib.WG_BAD_IP, lib.WG_FILTERED, lib.WG_REPLAY} <= seen
+    for ctx, *_ in sides:
+        ctx.close()

@@ -21,21 +21,18 @@ int aead_batch_host_chunked(bnk_ctx *ctx, bool open, const bnk_batch *in, const 
     hp.ctx = ctx;
     hp.in = in;
     hp.out = out;
-    hp.in_ext = [in](uint32_t i) { return (uint64_t)(in->lens ? in->lens[i] : in->len); };
-    hp.out_ext = [in, out_delta](uint32_t i) {
+    const auto in_ext = [in](uint32_t i) { return (uint64_t)(in->lens ? in->lens[i] : in->len); };
+    const auto out_ext = [in, out_delta](uint32_t i) {
         return (uint64_t)std::max<int64_t>((int64_t)(in->lens ? in->lens[i] : in->len) + out_delta, 0);
     };
-    int rc = hp.plan(in->lens ? 0 : hp.out_ext(0));
+    int rc = hp.plan(in->lens ? 0 : out_ext(0), in_ext, out_ext);
     if (rc) return rc;
     rc = check_index_range(ctx, in->peer, n, a.n_peers, "peer index", "the key table");
     if (rc) return rc;
-    if (open) {
-        HIPCHK(ctx, ctx->verdict.reserve(n));
-        a.verdict = ctx->verdict.as<uint8_t>();
-        hp.add_result(verdict, a.verdict, 1);
-    }
+    if (open) hp.add_written_result(verdict, 1);
     rc = hp.begin();
     if (rc) return rc;
+    if (open) a.verdict = hp.written_result(0);
     // per-packet arrays go up whole, ahead of everything, on the compute stream
     auto up = [&](DevBuf *dst, const void *src, size_t bytes) -> hipError_t {
         hipError_t e = dst->reserve(bytes);

@@ -123,9 +123,8 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         hp.ctx = ctx;
         hp.in = in;
         hp.out = out;
-        hp.in_ext = hp.out_ext = ct_ext;
         hp.max_chunks = RELAY_CHUNKS;
-        rc = hp.plan(in->lens ? 0 : in->len);
+        rc = hp.plan(in->lens ? 0 : in->len, ct_ext, ct_ext);
         if (rc != BNK_OK && rc != 1) return rc;
         chunked = rc == BNK_OK;
     }

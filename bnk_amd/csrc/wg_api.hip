@@ -367,8 +367,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         d_wire_len = ctx->wg_wirelen.as<uint32_t>();
         hp.ctx = ctx;
         hp.in = hp.out = slots;
-        hp.in_ext = hp.out_ext = slot_ext;
-        rc = hp.plan(0);
+        rc = hp.plan(0, slot_ext, slot_ext);
         if (rc != BNK_OK && rc != 1) return rc;
         chunked = rc == BNK_OK;
         if (chunked) {
@@ -769,9 +768,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         hp.ctx = ctx;
         hp.in = &w2;
         hp.out = out;
-        hp.in_ext = wire_ext;
-        hp.out_ext = plain_ext;
-        rc = hp.plan(wire->lens ? 0 : plain_ext(0));
+        rc = hp.plan(wire->lens ? 0 : plain_ext(0), wire_ext, plain_ext);
         if (rc != BNK_OK && rc != 1) return rc;
         chunked = rc == BNK_OK;
         if (chunked) {

@@ -1626,7 +1626,9 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
         outside = beyond_arena((uint64_t)(src - a.in), len, a.in_limit) ||
                   beyond_arena((uint64_t)(dst - a.out), OPEN ? (short_ct ? 0u : len - 16u) : (uint64_t)len + 16u, a.out_limit) ||
                   wraps;
-        if (outside) {
+        // (refusals are marked as rare, here and below: laid out ahead of the loads, their branches
+        // part the fetch)
+        if (__builtin_expect(outside, 0)) {
             if (lane == 0 && !skipped) {
                 status_raise(a.status, STATUS_BOUNDS);
                 if (OPEN) refuse();
@@ -1710,15 +1712,15 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
     // further down: looking at it here would make the key wait for the packet)
 
     if (!WG) {
-        if (skipped) return false;
-        if (pr >= a.n_peers) {
+        if (__builtin_expect(skipped, 0)) return false;
+        if (__builtin_expect(pr >= a.n_peers, 0)) {
             if (lane == 0) {
                 status_raise(a.status, STATUS_PEER_RANGE);
                 if (OPEN) refuse();
             }
             return false;
         }
-        if (OPEN && len < 16u) {
+        if (__builtin_expect(OPEN && len < 16u, 0)) {
             if (lane == 0) refuse();
             return false;
         }
@@ -1734,7 +1736,7 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
             ctr = ctr_ld;
         }
         // (a keypair that has used up its nonces sends nothing more)
-        if (pr >= a.wg.n_peers || outside || ctr >= WG_REJECT_AFTER_MESSAGES) {
+        if (__builtin_expect(pr >= a.wg.n_peers || outside || ctr >= WG_REJECT_AFTER_MESSAGES, 0)) {
             if (SMALL && t.filter) {
                 // NoteOutbound comes ahead of all that
                 if (plain_inside) note_end(f, lane, note_begin(f, lane, first_cells(data, len, lane), len));
@@ -1784,11 +1786,11 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
             if (hit == 0ull) res = BNK_WG_UNKNOWN_INDEX;
             else pr = (uint32_t)__shfl((int)e.y, __ffsll((long long)hit) - 1, 64);
         }
-        if (SMALL && res != BNK_WG_OK) {
+        if (SMALL && __builtin_expect(res != BNK_WG_OK, 0)) {
             decap_record(t.records, i, lane, 0xFFFFFFFFu, 0ull, res, 0u, CHECK_DENY, 0u);
             return false;
         }
-        if (res != BNK_WG_OK) {
+        if (__builtin_expect(res != BNK_WG_OK, 0)) {
             if (lane == 0) {
                 a.wg.result[i] = res;
                 a.wg.out_len[i] = 0;
@@ -1802,7 +1804,7 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
             a.wg.peer_out[i] = pr;
             a.wg.counter_out[i] = ctr;
         }
-        if (wraps) { // (reported as one that does not verify, by the lane kernels too)
+        if (__builtin_expect(wraps, 0)) { // (reported as one that does not verify, by the lane kernels too)
             if (SMALL) decap_record(t.records, i, lane, pr, ctr, BNK_WG_AUTH_FAIL, 0u, CHECK_DENY, 0u);
             if (lane == 0) {
                 status_raise(a.status, STATUS_BOUNDS);

@@ -25,6 +25,7 @@ int aead_batch_host_chunked(bnk_ctx *ctx, bool open, const bnk_batch *in, const 
     const auto out_ext = [in, out_delta](uint32_t i) {
         return (uint64_t)std::max<int64_t>((int64_t)(in->lens ? in->lens[i] : in->len) + out_delta, 0);
     };
+    hp.write_through = true;
     int rc = hp.plan(in->lens ? 0 : out_ext(0), in_ext, out_ext);
     if (rc) return rc;
     rc = check_index_range(ctx, in->peer, n, a.n_peers, "peer index", "the key table");
@@ -58,6 +59,7 @@ int aead_batch_host_chunked(bnk_ctx *ctx, bool open, const bnk_batch *in, const 
     a.out = hp.d_out;
     a.in_off = hp.d_in_off;
     a.out_off = hp.d_out_off;
+    a.out_in_host = hp.out_in_ring;
     rc = hp.open_gate();
     if (rc) return rc;
     for (uint32_t k = 0; k < hp.chunks; k++) {
@@ -135,6 +137,7 @@ int aead_batch_host_direct(bnk_ctx *ctx, bool open, const bnk_batch *in, const b
         a.in = ctx->in_arena.as<uint8_t>() + mis;
     }
     a.out = d_out;
+    a.out_in_host = true;
     if (in->offsets) {
         for (uint32_t i = 0; i < n; i++) p_in_off[i] = in->offsets[i] - sin.lo;
         a.in_off = stage.dev(p_in_off);

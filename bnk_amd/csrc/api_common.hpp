@@ -304,6 +304,8 @@ struct HostPipe {
     Span sin, sout;
     bool in_place = false;
     uint64_t row_width = 0; // > 0: the output comes back row by row (uniform layout, see plan)
+    bool write_through = false; // nothing reads the output on the device: set by the caller, see plan
+    bool out_in_ring = false;   // it goes straight into the ring it lies in
     uint32_t max_chunks = PIPE_MAX_CHUNKS;
     uint8_t *d_in = nullptr, *d_out = nullptr;
     const uint64_t *d_in_off = nullptr, *d_out_off = nullptr;
@@ -383,9 +385,20 @@ struct HostPipe {
             sout = sin;
         }
         row_width = (!in_place && !out->offsets) ? uniform_out_width : 0;
-        HIPCHK(ctx, ctx->in_arena.reserve(sin.size() + 16));
+        HIPCHK(ctx, ctx->in_arena.reserve(sin.size() + 128 + 16));
         d_in = d_out = ctx->in_arena.as<uint8_t>();
-        if (!in_place) {
+        // Output that does not come back row by row would have to go up first, for what lies between its
+        // packets to come back unchanged: where it lies in a ring the kernels write it there instead, and
+        // the link carries it once.  60000 packets out of and into rings, sealed and opened: of 1 to 1420
+        // bytes in slots of 16 bytes 4,850 us before and 3,400 with it, packed without a gap 4,740 and
+        // 3,350, of the mix of sizes 2,930 and 2,305; 20000 of 1 to 1420 bytes 1,840 and 1,390.  (Uniform
+        // layouts come back by rows at 48 GB/s; kernels write into a ring at 43 while as much goes up.)
+        uint8_t *const ring = write_through && !in_place && !row_width ? ring_device_ptr(ctx, out->base, out->bytes) : nullptr;
+        out_in_ring = ring != nullptr;
+        if (out_in_ring) {
+            d_out = ring + sout.lo;
+            d_in += (uintptr_t)d_out & 127u; // the first input as far into its line as the first output
+        } else if (!in_place) {
             HIPCHK(ctx, ctx->out_arena.reserve(sout.size() + 16));
             d_out = ctx->out_arena.as<uint8_t>();
         }
@@ -453,7 +466,7 @@ struct HostPipe {
             HIPCHK(ctx, hipMemcpyAsync(d_in + (u0 - sin.lo), h_in + u0, u1 - u0, hipMemcpyHostToDevice, ctx->s_up));
         // any layout that does not come back row by row first takes the host's
         // output bytes up, so that what lies between packets comes back unchanged
-        if (!in_place && !row_width && o1 > o0)
+        if (!in_place && !row_width && !out_in_ring && o1 > o0)
             HIPCHK(ctx, hipMemcpyAsync(d_out + (o0 - sout.lo), h_out + o0, o1 - o0, hipMemcpyHostToDevice, ctx->s_up));
         HIPCHK(ctx, hipEventRecord(ctx->ev_up[k], ctx->s_up));
         HIPCHK(ctx, hipStreamWaitEvent(ctx->stream, ctx->ev_up[k], 0));
@@ -476,7 +489,7 @@ struct HostPipe {
         if (row_width)
             HIPCHK(ctx, hipMemcpy2DAsync(h_out + o0, out->stride, d_out + (o0 - sout.lo), out->stride, row_width,
                                          hi - lo, hipMemcpyDeviceToHost, ctx->s_down));
-        else if (o1 > o0)
+        else if (!out_in_ring && o1 > o0)
             HIPCHK(ctx, hipMemcpyAsync(h_out + o0, d_out + (o0 - sout.lo), o1 - o0, hipMemcpyDeviceToHost, ctx->s_down));
         for (const Result &r : results)
             if (r.dev) HIPCHK(ctx, hipMemcpyAsync(ctx->pin.as<uint8_t>() + r.pin_off + (size_t)lo * r.elem,

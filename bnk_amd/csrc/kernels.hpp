@@ -113,6 +113,7 @@ struct AeadArgs {
     uint32_t room;             // with lens: bytes of an arena per packet (a hint, see aead_room)
     bool host_batch;           // the call waits for its launch: no other has the chip meanwhile
     bool over_link;            // packets lie in host memory: a wave per packet reads them there
+    bool out_in_host;          // the output does
     uint32_t split;            // set by the launcher: packets per wave of aead_split_kernel
     unsigned long long *tally; // or nullptr: an open without framing counts its own verdicts here
                                // (TALLY_OPENED / TALLY_REJECTED, see tally_bump), an encapsulating

@@ -124,6 +124,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         hp.in = in;
         hp.out = out;
         hp.max_chunks = RELAY_CHUNKS;
+        hp.write_through = true;
         rc = hp.plan(in->lens ? 0 : in->len, ct_ext, ct_ext);
         if (rc != BNK_OK && rc != 1) return rc;
         chunked = rc == BNK_OK;
@@ -298,6 +299,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
         se.in_off = o.in_off;
         se.in_stride = in->stride;
         se.out = d_out;
+        se.out_in_host = direct || hp.out_in_ring;
         se.out_off = d_out_off;
         se.out_stride = out->stride;
         se.lens = o.lens;

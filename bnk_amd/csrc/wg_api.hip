@@ -549,6 +549,7 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         se.n = hi - lo;
         se.in = b.base;
         se.out = sealed;
+        se.out_in_host = ring_out != nullptr;
         se.in_off = se.out_off = b.off;
         se.in_stride = se.out_stride = slots->stride;
         se.in_skip = se.out_skip = 16;
@@ -968,6 +969,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         op.in_stride = wire->stride;
         op.in_skip = 16;
         op.out = const_cast<uint8_t *>(ob.base);
+        op.out_in_host = direct;
         op.out_off = ob.off;
         op.out_stride = out->stride;
         op.lens = d_ctlen;

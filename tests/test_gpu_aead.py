@@ -361,6 +361,52 @@ def test_small_batches_in_pinned_rings(small_ctx, layout, n):
             ctx.ring_free(r)
 
 
+@pytest.mark.parametrize("step,longest,n", [(16, 1420, 20000), (1, 1420, 20000), (4, 700, 60000), (16, 60, 200000)])
+def test_large_host_batches_written_into_rings(ctx, step, longest, n):
+    """Batches of several pieces whose output, of a layout that does not come back row by row, the
+    kernels write into the ring: slots on whole cells, on words and anywhere, and pieces as large as the
+    launches that split a packet over lanes, or give it one, take.  Every byte, those between and around
+    the packets too, against the oracle; a hundred tags forged."""
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(step + longest)
+    lens = rng.integers(1, longest + 1, n).astype(np.uint32)
+    room = (lens.astype(np.uint64) + np.uint64(16 + step - 1)) // np.uint64(step) * np.uint64(step)
+    off = np.cumsum(room) - room + np.uint64(step)
+    nb = int(off[-1] + room[-1]) + 40
+    keys = rng.integers(0, 256, (5, 32), dtype=np.uint8)
+    ctx.keys_set(lib.KEYS_SEND, keys)
+    ctx.keys_set(lib.KEYS_RECV, keys)
+    peer = rng.integers(0, 5, n).astype(np.uint32)
+    counters = rng.integers(0, 1 << 62, n).astype(np.uint64)
+    plain = rng.integers(0, 256, nb, dtype=np.uint8)
+    want = np.full(nb, 0x5A, np.uint8)
+    O.seal_batch(keys, peer, counters, plain, off, lens, want, off, 4)
+    rings = [ctx.ring_alloc(nb + 64) for _ in range(2)]
+    try:
+        src, dst = rings[0][48:48 + nb], rings[1][16:16 + nb]
+        src[:] = plain
+        rings[1][:] = 0x5A
+        ctx.seal(lib.make_batch(src, nb, n, lib.MEM_HOST, offsets=off, lens=lens, peer=peer, counters=counters),
+                 lib.make_batch(dst, nb, n, lib.MEM_HOST, offsets=off))
+        assert np.array_equal(dst, want)
+        assert (rings[1][:16] == 0x5A).all() and (rings[1][16 + nb:] == 0x5A).all()
+        forged = rng.choice(n, 100, replace=False)
+        want[(off[forged] + lens[forged] + np.uint64(9)).astype(np.int64)] ^= 4
+        src[:] = want
+        dst[:] = 0xEE
+        back = np.full(nb, 0xEE, np.uint8)
+        overdict = O.open_batch(keys, peer, counters, want, off, lens + np.uint32(16), back, off, 4)
+        verdict = np.full(n, 7, np.uint8)
+        ctx.open(lib.make_batch(src, nb, n, lib.MEM_HOST, offsets=off, lens=lens + np.uint32(16), peer=peer, counters=counters),
+                 lib.make_batch(dst, nb, n, lib.MEM_HOST, offsets=off), verdict)
+        assert np.array_equal(verdict, overdict)
+        assert np.array_equal(dst, back)
+    finally:
+        for r in rings:
+            ctx.ring_free(r)
+
+
 def test_random_shapes_through_pinned_rings(ctx):
     """Three hundred batches of random size (1 to 5000 packets), length mix,
     alignment and kernel choice, one after the other through the same rings

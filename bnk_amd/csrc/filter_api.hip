@@ -67,7 +67,7 @@ static hipError_t upload_rule_index(FilterState *f, const HostRuleIndex &h, hipS
     f->ridx.wide = f->wide.as<uint4>();
     f->ridx.n_bounds = (uint32_t)nb;
     f->ridx.n_wide = (uint32_t)h.wide.size();
-    f->ridx.long_lists = h.ranges.size() > nb * RANGE_BLOCK; // (they lie behind the intervals' own blocks)
+    f->ridx.long_lists = h.ranges.size() > nb * RANGE_CLASSES * RANGE_BLOCK; // (they lie behind the intervals' own blocks)
     uint32_t step = 0;
     if (nb >= 2) {
         step = 1;

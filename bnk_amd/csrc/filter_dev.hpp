@@ -16,6 +16,7 @@ enum : uint32_t {
     FLOW_LIVE = 0, FLOW_CLAIMED = 1, FLOW_SWEPT = 2, FLOW_GONE = 3, FLOW_MIN_EXP = 4, FLOW_NEXT_EXP = 6, FLOW_NOTE_BLOCKS = 8,
     FLOW_COUNTERS = 10
 };
+constexpr uint32_t FLOW_SWEEP_ABOVE = 4096; // filter.go:202: no sweep while the map holds at most so many entries
 constexpr int64_t FLOW_TTL_LEAST = 30000000000LL; // filter.go:108-117: nothing is stored for less
 
 // One 16-byte slot, so a probe is a single memory transaction.
@@ -43,21 +44,22 @@ constexpr uint32_t SMALL_BITS = 44u * 1024u * 8u; // 44 KiB: leaves 36 KiB of a 
 constexpr uint32_t SMALL_KEYS_MAX = 3u << 16;     // beyond this a clear answer gets too rare (false
                                                   // positives pass 43 %) and the large bitmap is asked
 
-// A key is class << 16 | port with class < 3, so key_lo 0x3FFFF and 0x3FFFE never occur.
-constexpr uint32_t RANGE_PAD = 0x3FFFFu << 14;
-constexpr uint32_t RANGE_LONG = 0x3FFFEu << 14;      // first word of a block that only points on
-constexpr uint32_t RANGE_MAX_SPAN = (1u << 14) - 1u; // largest key_hi - key_lo one entry holds
-constexpr uint32_t RANGE_BLOCK = 16;
-constexpr uint32_t JUMP_BUCKETS = 1024;                 // entries per 64-byte block
+// A range of ports in a word, first | (0xFFFF - last) << 16, with first <= last; so these two are none,
+// and have no port.
+constexpr uint32_t RANGE_PAD = 0xFFFFFFFFu;
+constexpr uint32_t RANGE_LONG = 0xFFFEFFFFu; // first word of a block that only points on
+constexpr uint32_t RANGE_BLOCK = 16;         // entries per 64-byte block
+constexpr uint32_t RANGE_CLASSES = 3;        // icmp, tcp, udp
+constexpr uint32_t JUMP_BUCKETS = 1024;
 
 struct RuleIndexDev {
     const uint32_t *bounds; // [n_bounds] ascending starts of the elementary source intervals
-    const uint32_t *ranges; // 64-byte blocks of RANGE_BLOCK one-word key ranges
-                            // (key_lo << 14 | key_hi - key_lo; wider ranges are cut into
-                            // pieces), sorted, disjoint, padded with RANGE_PAD.  Block j is
-                            // interval j's list, so finding the interval finds the list.  A
-                            // list of more than RANGE_BLOCK pieces lives in blocks past the
-                            // first n_bounds, and block j is {RANGE_LONG, first block, blocks}
+    const uint32_t *ranges; // 64-byte blocks of RANGE_BLOCK one-word ranges of ports, sorted,
+                            // disjoint, padded with RANGE_PAD.  Block RANGE_CLASSES * j + c is
+                            // interval j's list for class c, so finding the interval finds the
+                            // list.  A list of more than RANGE_BLOCK ranges lives in blocks past
+                            // the first RANGE_CLASSES * n_bounds, and its block is {RANGE_LONG,
+                            // first block, blocks}
     const uint4 *wide;      // [n_wide] (net, mask, key_lo, key_hi) scanned by every packet
     const uint16_t *jump;   // [JUMP_BUCKETS + 1] when n_bounds fits 16 bits, else null: the cut
                             // points from bounds[1] up are spread over equal address buckets

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <algorithm>
+#include <iterator>
 #include <string>
 #include <vector>
 
@@ -109,9 +110,6 @@ inline bool build_rule_index(const bnk_rule *rules, uint32_t n, HostRuleIndex &o
     for (const Tuple &t : ts)
         if (!t.wide)
             for (uint32_t j = t.a; j < t.b; j++) raw[fill[j]++] = make_uint2(t.klo, t.khi);
-    // per interval: sort by key_lo, merge overlapping or adjacent key ranges,
-    // cut what is left into one-word pieces; block j takes interval j's pieces,
-    // or points at blocks appended behind the first nb when there are too many
     // jump table over the populated part of the address space
     out.jump.clear();
     if (nb >= 2 && nb <= 0xFFFFu) {
@@ -127,38 +125,34 @@ inline bool build_rule_index(const bnk_rule *rules, uint32_t n, HostRuleIndex &o
             out.jump[b] = (uint16_t)j;
         }
     }
-    out.ranges.assign((size_t)nb * RANGE_BLOCK, RANGE_PAD);
+    // per interval and class: sort by the first port, merge what overlaps or adjoins; its block
+    // takes the ranges, or points at blocks appended behind those when there are too many
+    out.ranges.assign((size_t)nb * RANGE_CLASSES * RANGE_BLOCK, RANGE_PAD);
     std::vector<uint2> merged;
-    std::vector<uint32_t> pieces;
     for (uint32_t j = 0; j < nb; j++) {
         auto lo = raw.begin() + raw_start[j], hi = raw.begin() + raw_start[j + 1];
         std::sort(lo, hi, [](const uint2 &x, const uint2 &y) { return x.x < y.x; });
-        merged.clear();
-        for (auto it = lo; it != hi; ++it) {
-            if (!merged.empty() && it->x <= merged.back().y + 1u) {
-                if (it->y > merged.back().y) merged.back().y = it->y;
+        for (uint32_t cls = 0; cls < RANGE_CLASSES; cls++) {
+            merged.clear();
+            for (; lo != hi && lo->x >> 16 == cls; ++lo) {
+                const uint32_t first = lo->x & 0xFFFFu, last = lo->y & 0xFFFFu;
+                if (!merged.empty() && first <= merged.back().y + 1u) {
+                    if (last > merged.back().y) merged.back().y = last;
+                } else {
+                    merged.push_back(make_uint2(first, last));
+                }
+            }
+            const size_t own = ((size_t)j * RANGE_CLASSES + cls) * RANGE_BLOCK, first = out.ranges.size() / RANGE_BLOCK;
+            const auto word = [](const uint2 &r) { return r.x | (0xFFFFu - r.y) << 16; };
+            if (merged.size() <= RANGE_BLOCK) {
+                std::transform(merged.begin(), merged.end(), out.ranges.begin() + own, word);
             } else {
-                merged.push_back(*it);
+                std::transform(merged.begin(), merged.end(), std::back_inserter(out.ranges), word);
+                while (out.ranges.size() % RANGE_BLOCK) out.ranges.push_back(RANGE_PAD);
+                out.ranges[own] = RANGE_LONG;
+                out.ranges[own + 1] = (uint32_t)first;
+                out.ranges[own + 2] = (uint32_t)(out.ranges.size() / RANGE_BLOCK - first);
             }
-        }
-        pieces.clear();
-        for (const uint2 &r : merged)
-            for (uint32_t at = r.x;; at += RANGE_MAX_SPAN + 1u) {
-                const uint32_t span = std::min(r.y - at, RANGE_MAX_SPAN);
-                pieces.push_back(at << 14 | span);
-                if (at + span == r.y) break;
-            }
-        uint32_t *blk = out.ranges.data() + (size_t)j * RANGE_BLOCK;
-        if (pieces.size() <= RANGE_BLOCK) {
-            std::copy(pieces.begin(), pieces.end(), blk);
-        } else {
-            const size_t first = out.ranges.size() / RANGE_BLOCK;
-            out.ranges.insert(out.ranges.end(), pieces.begin(), pieces.end());
-            while (out.ranges.size() % RANGE_BLOCK) out.ranges.push_back(RANGE_PAD);
-            blk = out.ranges.data() + (size_t)j * RANGE_BLOCK; // the vector may have moved
-            blk[0] = RANGE_LONG;
-            blk[1] = (uint32_t)first;
-            blk[2] = (uint32_t)(out.ranges.size() / RANGE_BLOCK - first);
         }
     }
     return true;

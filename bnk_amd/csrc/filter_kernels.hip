@@ -10,8 +10,8 @@
 // a key interval [class<<16 | first, class<<16 | last] (class 0 icmp, 1 tcp,
 // 2 udp; icmp packets carry key 0 and icmp rules cover the whole class).  The
 // host cuts the 32-bit source space at every interval end into elementary
-// intervals and stores, per elementary interval, the sorted disjoint union of
-// the key intervals of all rules covering it, in 64-byte blocks.  A packet does
+// intervals and stores, per elementary interval and class, the sorted disjoint union of
+// the port intervals of all rules covering it, in 64-byte blocks.  A packet does
 // one binary search over the cut points (staged in LDS together with each
 // interval's block number and length) and then reads its interval's list: one
 // memory transaction when the list fits a block, a binary search otherwise.
@@ -70,9 +70,9 @@ BNK_DEV uint32_t interval_of_jump(const uint32_t *bounds, const uint16_t *jump, 
 
 // 0 if one of the four has the key.  (As a chain of comparisons the compiler tests one word,
 // branches, and fetches the next ones only then.)
-BNK_DEV uint32_t quad_miss(uint4 v, uint32_t key)
+BNK_DEV uint32_t quad_miss(uint4 v, uint32_t ports)
 {
-    return min(min(range_miss(v.x, key), range_miss(v.y, key)), min(range_miss(v.z, key), range_miss(v.w, key)));
+    return min(min(range_miss(v.x, ports), range_miss(v.y, ports)), min(range_miss(v.z, ports), range_miss(v.w, ports)));
 }
 
 // Value of x in lane J of this lane's quad (lanes 4k .. 4k+3).
@@ -89,25 +89,25 @@ BNK_DEV uint32_t quad_perm(uint32_t x)
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, A | B << 2 | C << 4 | D << 6, 0xF, 0xF, true);
 }
 
-// A list of more than 16 pieces: head is the first quad of the interval's own
-// block, {RANGE_LONG, first block, blocks}.  Finds the block by its first key
-// (the ranges are sorted and disjoint, so only that block can hold the key).
-BNK_DEV bool long_list_hit(const RuleIndexDev &ri, uint32_t first, uint32_t nblk, uint32_t key)
+// A list of more than 16 ranges: head is the first quad of the list's own
+// block, {RANGE_LONG, first block, blocks}.  Finds the block by its first port
+// (the ranges are sorted and disjoint, so only that block can hold the packet's).
+BNK_DEV bool long_list_hit(const RuleIndexDev &ri, uint32_t first, uint32_t nblk, uint32_t port, uint32_t ports)
 {
     const uint4 *ob = reinterpret_cast<const uint4 *>(ri.ranges + (size_t)first * RANGE_BLOCK);
     uint32_t lo = 0, hi = nblk;
     while (hi - lo > 1u) {
         const uint32_t mid = (lo + hi) >> 1;
-        if ((ob[4u * mid].x >> 14) <= key) lo = mid;
+        if ((ob[4u * mid].x & 0xFFFFu) <= port) lo = mid;
         else hi = mid;
     }
     const uint4 *b = ob + 4u * lo;
     const uint4 w0 = b[0], w1 = b[1], w2 = b[2], w3 = b[3];
-    return min(min(quad_miss(w0, key), quad_miss(w1, key)), min(quad_miss(w2, key), quad_miss(w3, key))) == 0u;
+    return min(min(quad_miss(w0, ports), quad_miss(w1, ports)), min(quad_miss(w2, ports), quad_miss(w3, ports))) == 0u;
 }
 
 // Rule lookup for the four packets of a quad of lanes at once; every lane of the
-// wave must call it (lanes without a packet pass iv 0 and ignore the answer).
+// wave must call it (lanes without a packet pass block 0 and ignore the answer).
 // The kernel is bound by the cache lookups its scattered loads cause, one per
 // distinct line per load instruction.  A lane fetching its own 64-byte block
 // with four 16-byte loads causes four; here the four lanes of a quad fetch one
@@ -120,28 +120,29 @@ struct QuadBlocks {
 };
 // SMALL: there are at most 2^16 intervals (a byte offset among their blocks has 32 bits).
 template <bool SMALL>
-BNK_DEV const uint4 *rules_block(const RuleIndexDev &ri, uint32_t iv)
+BNK_DEV QuadBlocks rules_fetch_quad(const RuleIndexDev &ri, uint32_t lane, uint32_t block)
 {
+    const uint32_t part = 16u * (lane & 3u);
     const uint8_t *const blocks = reinterpret_cast<const uint8_t *>(ri.ranges);
-    return reinterpret_cast<const uint4 *>(blocks + (SMALL ? iv * (RANGE_BLOCK * 4u) : (size_t)iv * (RANGE_BLOCK * 4u)));
-}
-
-template <bool SMALL>
-BNK_DEV QuadBlocks rules_fetch_quad(const RuleIndexDev &ri, uint32_t lane, uint32_t iv)
-{
-    const uint32_t part = lane & 3u;
-    return QuadBlocks{rules_block<SMALL>(ri, quad_bcast<0>(iv))[part], rules_block<SMALL>(ri, quad_bcast<1>(iv))[part],
-                      rules_block<SMALL>(ri, quad_bcast<2>(iv))[part], rules_block<SMALL>(ri, quad_bcast<3>(iv))[part]};
+    if (SMALL) {
+        const uint32_t at = block * (RANGE_BLOCK * 4u);
+        const auto ld = [&](uint32_t of) __attribute__((always_inline)) { return *reinterpret_cast<const uint4 *>(blocks + (of + part)); };
+        return QuadBlocks{ld(quad_bcast<0>(at)), ld(quad_bcast<1>(at)), ld(quad_bcast<2>(at)), ld(quad_bcast<3>(at))};
+    }
+    const auto ld = [&](uint32_t of) __attribute__((always_inline)) {
+        return *reinterpret_cast<const uint4 *>(blocks + (size_t)of * (RANGE_BLOCK * 4u) + part);
+    };
+    return QuadBlocks{ld(quad_bcast<0>(block)), ld(quad_bcast<1>(block)), ld(quad_bcast<2>(block)), ld(quad_bcast<3>(block))};
 }
 
 BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint32_t lane, uint32_t src, uint32_t key)
 {
-    const uint32_t part = lane & 3u;
+    const uint32_t part = lane & 3u, port = key & 0xFFFFu, ports = range_key(port);
     // packet j of the quad in the lane's own 16 bytes, and of all that the quad's lanes find the
     // least for the lane's own packet: two exchanges, in which a lane hands over what it has
     // found for its neighbours' packets
-    const uint32_t m0 = quad_miss(q.p0, quad_bcast<0>(key)), m1 = quad_miss(q.p1, quad_bcast<1>(key)),
-                   m2 = quad_miss(q.p2, quad_bcast<2>(key)), m3 = quad_miss(q.p3, quad_bcast<3>(key));
+    const uint32_t m0 = quad_miss(q.p0, quad_bcast<0>(ports)), m1 = quad_miss(q.p1, quad_bcast<1>(ports)),
+                   m2 = quad_miss(q.p2, quad_bcast<2>(ports)), m3 = quad_miss(q.p3, quad_bcast<3>(ports));
     const bool odd = (part & 1u) != 0u, upper = (part & 2u) != 0u;
     const uint32_t lo = min(odd ? m1 : m0, quad_perm<1, 0, 3, 2>(odd ? m0 : m1)),
                    hi = min(odd ? m3 : m2, quad_perm<1, 0, 3, 2>(odd ? m2 : m3));
@@ -161,7 +162,7 @@ BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint3
             };
             const uint32_t head = mine(q.p0.x, q.p1.x, q.p2.x, q.p3.x), first = mine(q.p0.y, q.p1.y, q.p2.y, q.p3.y),
                            nblk = mine(q.p0.z, q.p1.z, q.p2.z, q.p3.z);
-            if (head == RANGE_LONG) hit = long_list_hit(ri, first, nblk, key);
+            if (head == RANGE_LONG) hit = long_list_hit(ri, first, nblk, port, ports);
         }
     }
     if (!hit)
@@ -285,16 +286,12 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     // bytes per lane and load, all of them in flight together (word by word, each waited for:
     // 3 us more for 2^22 packets, 1 for 2^14).
     //
-    // What bounds the launch: 8 waves per SIMD, of whose time more than half is spent waiting for
-    // memory (a packet's rule list, presence word and flow slot come from L2 and beyond, one behind
-    // the other) and a quarter waiting to issue, half of the VALU's slots taken.  So both count, the
-    // instructions and the order in which memory is asked: 2^22 plain headers on 4096 rules and
-    // 65,536 flows took 79.3 us with 510 vector and 280 scalar instructions per 64 packets, the
-    // rule lists fetched a word at a time as the tests before it failed; compiled per kind of
-    // launch, without branches in the parse and the tests, and with the loads ahead of what
-    // waits for them 355 and 111, and 67.4, and 59.5 with a long list's place taken from the quad
-    // (rules_match_quad).  The next header ahead of the flow's look-up as well: 72 against 67.4 (its
-    // loads queue ahead of the look-up's).
+    // What bounds the launch: L2's lines and what lies behind it.  2^22 plain headers of 32 bytes, one rule
+    // and 64 flows take 25 us, what a copy of as many bytes takes; with 4096 rules (a 64-byte block of the
+    // rules a packet, from L2) 37.3, and with 65,536 flows too (an eighth of the packets fetch a line of the
+    // table, mostly from beyond L2) 45.5.  Instructions no longer count: the same three took 42.7, 50.5 and
+    // 58.3 with 355 vector instructions per 64 packets instead of 212 and every wave adding its verdicts to
+    // the counters by itself (see the end of the kernel, which was most of it).
     RawHeader raw = fetch_header<FROM>(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
     {
         constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = (SMALL_QUADS + FILTER_THREADS - 1u) / FILTER_THREADS;
@@ -350,7 +347,7 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
                                      : interval_of(ri.bounds, ri.n_bounds, ri.top_step, h.src);
         // What the packet waits for is asked for in the order it is needed, with nothing waited for
         // in between: its rule list, then the word that says whether its flow was ever stored.
-        const QuadBlocks blocks = rules_fetch_quad<JUMPS>(ri, lane, iv);
+        const QuadBlocks blocks = rules_fetch_quad<JUMPS>(ri, lane, range_block(iv, proto_class(h.proto)));
         // return traffic: remote = src, remotePort = srcPort, localPort = dstPort.
         // A clear presence bit means the key was never stored: no probe
         // needed.  The small bitmap is in LDS where it is in use:
@@ -359,10 +356,13 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         const FlowSlot s = flow_slot(a.flows, h.src, h.sport, h.dport, h.proto);
         bool maybe = valid;
         if (small)
-            maybe &= ((lsmall[s.sbit0 >> 5] >> (s.sbit0 & 31u)) & (lsmall[s.sbit1 >> 5] >> (s.sbit1 & 31u)) & 1u) != 0u;
+            maybe &= ((lsmall[small_word(s.small0)] >> (s.small0 & 31u)) & (lsmall[small_word(s.small1)] >> (s.small1 & 31u)) & 1u) != 0u;
         const uint32_t present = a.flows.present[maybe ? s.bit >> 5 : 0u];
         asm volatile("" ::: "memory"); // (both are on their way before either is waited for)
         maybe &= ((present >> (s.bit & 31u)) & 1u) != 0u;
+        // (the next header queues behind those two and ahead of a flow's slot: 46.1 -> 45.5 us)
+        const RawHeader next = fetch_header<FROM>(a, t + stride);
+        asm volatile("" ::: "memory");
         uint8_t pass = 0;
         if (rules_match_quad(ri, blocks, lane, h.src, key)) {
             pass = valid ? 1 : 0;
@@ -389,7 +389,11 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
                     // pushed out to memory for it; this one waits for the end of
                     // the kernel like any other store.
                     // (`volatile` gets the same treatment as an atomic, hence not even that.)
-                    *ep = (unsigned long long)(a.now + flow_ttl_ns(h.proto));
+                    // Left out where it would change nothing: most of a flow's packets, and its
+                    // line need not go back then (2^22 headers, an eighth of them of 65,536
+                    // flows just refreshed: 51.2 us with every store, 46.1).
+                    const unsigned long long expiry = (unsigned long long)(a.now + flow_ttl_ns(h.proto));
+                    if (cur.y != expiry) *ep = expiry;
                     pass = 1;
                 } else {
                     // expired: delete (filter.go:144); only the lane that
@@ -412,16 +416,32 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
             n_pass += (uint32_t)__popcll(ok);
             n_drop += (uint32_t)__popcll(in & ~ok);
         }
-        raw = fetch_header<FROM>(a, t + stride);
+        raw = next;
     }
-    if (a.tally && lane == 0u) {
-        tally_bump(a.tally, TALLY_ALLOWED, n_pass);
-        tally_bump(a.tally, TALLY_DENIED, n_drop);
+    // What the waves have counted goes out once a workgroup: an addition costs 1.35 ns of every other's
+    // time, as all of them meet in a few lines, and the waves of a large launch end together (2 of each of
+    // 8192 waves: 22 us of the launch over 2^22 headers).
+    const bool results = FROM == FROM_ARRAYS && a.wg_tally;
+    if (!a.tally && !results) return;
+    constexpr uint32_t WAVES = FILTER_THREADS / 64u, COUNTS = 18;
+    const uint32_t wave = threadIdx.x / 64u;
+    __syncthreads(); // (nobody looks at the tables any more)
+    if (lane == 0u) {
+        lds[COUNTS * wave + 16u] = n_pass;
+        lds[COUNTS * wave + 17u] = n_drop;
     }
-    if (FROM == FROM_ARRAYS && a.wg_tally && lane < 16u && n_result != 0u && decap_slot(lane) != TALLY_NONE) {
-        tally_bump(a.wg_tally, decap_slot(lane), n_result);
+    if (FROM == FROM_ARRAYS && lane < 16u) lds[COUNTS * wave + lane] = n_result;
+    __syncthreads();
+    if (wave != 0u || lane >= COUNTS) return;
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < WAVES; w++) sum += lds[COUNTS * w + lane];
+    if (lane >= 16u) {
+        if (a.tally) tally_bump(a.tally, lane == 16u ? TALLY_ALLOWED : TALLY_DENIED, sum);
+    } else if (results && decap_slot(lane) != TALLY_NONE) {
+        tally_bump(a.wg_tally, decap_slot(lane), sum);
         // CheckInbound behind a decapsulating call saw exactly what was delivered
-        if (lane == BNK_WG_OK) tally_bump(a.wg_tally, TALLY_ALLOWED, n_result);
+        if (lane == BNK_WG_OK) tally_bump(a.wg_tally, TALLY_ALLOWED, sum);
     }
 }
 
@@ -437,13 +457,6 @@ __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
     note_block_done(a);
 }
 
-// (FilterArgs::record_after)
-__global__ void note_record_kernel(uint64_t *record, uint32_t seq, const uint32_t *counters)
-{
-    const uint32_t claimed = __hip_atomic_load(&counters[FLOW_CLAIMED], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(record, (uint64_t)seq << 32 | claimed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // filter.go:202-207: above 4096 entries, delete those with now.After(exp); there
 // is nothing to delete while no entry can have expired.  Nothing this launch
 // decides by changes while it runs: what it deletes and the bound it finds over
@@ -453,10 +466,13 @@ __global__ void note_record_kernel(uint64_t *record, uint32_t seq, const uint32_
 // Over the list of claimed slots: 14.4 us for 65,536, a gather each, where going through the
 // table they live in (200 MB, sized for batches of 2^18 packets) took 31 us behind every
 // batch.  The host cannot tell that nothing has expired, so the launch is made behind every
-// batch above 4096 entries; it returns at once then (2 to 5 us).
-__global__ __launch_bounds__(256) void flow_sweep_kernel(FlowTableDev ft, int64_t now)
+// batch above 4096 entries; it returns at once then (2 to 5 us).  Being made, it leaves the record of
+// the batch ahead of it (FilterArgs::record_after; record null: not), which a launch for it alone did.
+__global__ __launch_bounds__(256) void flow_sweep_kernel(FlowTableDev ft, int64_t now, uint64_t *record, uint32_t seq)
 {
-    if (ft.counters[FLOW_LIVE] <= 4096u || now <= *reinterpret_cast<const int64_t *>(ft.counters + FLOW_MIN_EXP)) return;
+    if (record && blockIdx.x == 0u && threadIdx.x == 0u)
+        __hip_atomic_store(record, (uint64_t)seq << 32 | ft.counters[FLOW_CLAIMED], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (ft.counters[FLOW_LIVE] <= FLOW_SWEEP_ABOVE || now <= *reinterpret_cast<const int64_t *>(ft.counters + FLOW_MIN_EXP)) return;
     if (blockIdx.x == 0u && threadIdx.x == 0u) ft.counters[FLOW_SWEPT] = 1u;
     const uint32_t claimed = ft.counters[FLOW_CLAIMED];
     const uint32_t total = claimed < ft.cap / 2u ? claimed : ft.cap / 2u;
@@ -501,9 +517,9 @@ __global__ __launch_bounds__(256) void flow_rehash_kernel(FlowTableDev from, Flo
         const int64_t e = from.slots[idx].exp;
         if (word == 0 || e == FLOW_TOMB) continue;
         const uint32_t region = idx / from.cap;
-        const uint64_t hsh = mix64(word ^ ((uint64_t)region << 59));
-        const uint32_t start = (uint32_t)hsh & (to.cap - 1u);
-        const uint32_t bit = (uint32_t)(hsh >> 32) & to.present_mask;
+        const FlowHash h = flow_hash(word, region);
+        const uint32_t start = h.start & (to.cap - 1u);
+        const uint32_t bit = h.bit & to.present_mask;
         bool placed = false;
         for (uint32_t probe = 0; probe < to.cap; probe++) {
             const uint32_t t = region * to.cap + ((start + probe) & (to.cap - 1u));
@@ -511,9 +527,8 @@ __global__ __launch_bounds__(256) void flow_rehash_kernel(FlowTableDev from, Flo
             if (atomicCAS(kp, 0ULL, (unsigned long long)word) == 0ULL) {
                 to.slots[t].exp = e;
                 atomicOr(&to.present[bit >> 5], 1u << (bit & 31u));
-                const uint32_t b0 = small_bit0(hsh), b1 = small_bit1(hsh);
-                atomicOr(&to.present_small[b0 >> 5], 1u << (b0 & 31u));
-                atomicOr(&to.present_small[b1 >> 5], 1u << (b1 & 31u));
+                atomicOr(&to.present_small[small_word(h.small0)], 1u << (h.small0 & 31u));
+                atomicOr(&to.present_small[small_word(h.small1)], 1u << (h.small1 & 31u));
                 const uint32_t pos = atomicAdd(&to.counters[FLOW_CLAIMED], 1u);
                 if (pos < to.cap / 2u) to.list[pos] = t;
                 atomicAdd(&to.counters[FLOW_LIVE], 1u);
@@ -602,29 +617,24 @@ hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipS
     return hipGetLastError();
 }
 
-// A launch of few workgroups counts them and leaves the record itself (23 ns a workgroup, where a
-// launch for it costs 4 us); of many, a launch behind it does.
-constexpr uint32_t NOTE_COUNTED_BLOCKS = 64;
-
 hipError_t launch_filter_note(const FilterArgs &args, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
 {
     if (args.n == 0) return hipSuccess;
     FilterArgs a = args;
     const uint32_t blocks = grid_for(a.n, max_blocks);
-    const bool record = a.record && a.record_after;
-    a.record_blocks = record && blocks <= NOTE_COUNTED_BLOCKS ? blocks : 0u;
+    // A launch with no sweep behind it counts its workgroups and leaves the record itself: they are few,
+    // and cost 23 ns each.
+    a.record_blocks = a.record && a.record_after && claimed_upper <= FLOW_SWEEP_ABOVE ? blocks : 0u;
     hipLaunchKernelGGL(filter_note_kernel, dim3(blocks + 1u), dim3(256), 0, s, a);
-    if (record && !a.record_blocks)
-        hipLaunchKernelGGL(note_record_kernel, dim3(1), dim3(1), 0, s, a.record, a.record_seq, a.flows.counters);
     return launch_flow_sweep(a, max_blocks, claimed_upper, s);
 }
 
 hipError_t launch_flow_sweep(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
 {
-    // filter.go:202: no sweep while the map holds at most 4096 entries
-    if (claimed_upper <= 4096u) return hipGetLastError();
+    if (claimed_upper <= FLOW_SWEEP_ABOVE) return hipGetLastError();
+    uint64_t *const record = a.record_after && !a.record_blocks ? a.record : nullptr;
     const uint32_t most = (uint32_t)(claimed_upper < a.flows.cap / 2u ? claimed_upper : a.flows.cap / 2u);
-    hipLaunchKernelGGL(flow_sweep_kernel, dim3(grid_for(most, max_blocks / 4u)), dim3(256), 0, s, a.flows, a.now);
+    hipLaunchKernelGGL(flow_sweep_kernel, dim3(grid_for(most, max_blocks / 4u)), dim3(256), 0, s, a.flows, a.now, record, a.record_seq);
     return hipGetLastError();
 }
 

@@ -161,7 +161,7 @@ static_assert(TALLY_RELAYED < TALLY_SLOTS, "slots");
 #if defined(__HIPCC__)
 __device__ inline void tally_bump(unsigned long long *tally, uint32_t slot, uint32_t k)
 {
-    if (k != 0u) atomicAdd(&tally[slot * TALLY_LANES + (blockIdx.x & (TALLY_LANES - 1u))], (unsigned long long)k);
+    if (k != 0u) atomicAdd(&tally[(blockIdx.x & (TALLY_LANES - 1u)) * TALLY_SLOTS + slot], (unsigned long long)k);
 }
 
 // The lanes of a wave vote per distinct value below 16 and lane v adds value v's votes to `mine`.

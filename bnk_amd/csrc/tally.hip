@@ -181,7 +181,7 @@ extern "C" int bnk_counters_get(bnk_ctx *ctx, bnk_counters *out)
     uint64_t v[TALLY_SLOTS];
     for (int s = 0; s < TALLY_SLOTS; s++) {
         v[s] = ctx->tally_host[s].load(std::memory_order_relaxed);
-        for (uint32_t l = 0; l < TALLY_LANES; l++) v[s] += dev[s * TALLY_LANES + l];
+        for (uint32_t l = 0; l < TALLY_LANES; l++) v[s] += dev[l * TALLY_SLOTS + s];
     }
     out->sealed = v[TALLY_SEALED];
     out->opened = v[TALLY_OPENED];

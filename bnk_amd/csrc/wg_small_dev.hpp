@@ -168,16 +168,17 @@ BNK_DEV uint32_t check_end(const FilterArgs &f, uint32_t lane, const WaveCheck &
         const uint32_t *const bounds = ri.bounds;
         iv = wave_search(lo, hi, w.h.src, lane, [bounds](uint32_t j) { return bounds[j]; });
     }
-    const uint32_t *list = ri.ranges + (size_t)iv * RANGE_BLOCK;
+    const uint32_t ports = range_key(w.h.dport);
+    const uint32_t *list = ri.ranges + (size_t)range_block(iv, proto_class(w.h.proto)) * RANGE_BLOCK;
     uint32_t mine = list[lane & (RANGE_BLOCK - 1u)];
     const uint32_t head = (uint32_t)__builtin_amdgcn_readlane((int)mine, 0);
     if (head == RANGE_LONG) { // (see long_list_hit)
         const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)mine, 1), blocks = (uint32_t)__builtin_amdgcn_readlane((int)mine, 2);
         const uint32_t *const all = ri.ranges + (size_t)first * RANGE_BLOCK;
-        const uint32_t b = wave_search(0u, blocks, key, lane, [all](uint32_t j) { return all[(size_t)j * RANGE_BLOCK] >> 14; });
+        const uint32_t b = wave_search(0u, blocks, w.h.dport, lane, [all](uint32_t j) { return all[(size_t)j * RANGE_BLOCK] & 0xFFFFu; });
         mine = all[(size_t)b * RANGE_BLOCK + (lane & (RANGE_BLOCK - 1u))];
     }
-    bool hit = __ballot(range_miss(mine, key) == 0u) != 0ull;
+    bool hit = __ballot(range_miss(mine, ports) == 0u) != 0ull;
     for (uint32_t j = 0; !hit && j < ri.n_wide; j += 64u) {
         const uint4 r = ri.wide[min(j + lane, ri.n_wide - 1u)];
         hit = __ballot((w.h.src & r.y) == r.x && key >= r.z && key <= r.w) != 0ull;

@@ -457,3 +457,52 @@ def test_every_form_of_a_device_batch(rules, n):
         assert 0.05 < np.concatenate(passed).mean() < 0.95
     assert ctx.filter_flows() == ora.flows()
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [65, 3000, 600001])
+def test_ranges_of_each_protocol_and_counts_of_large_batches(n):
+    """Ranges that begin at port 0 and end at 65535 or cover every port, lists of one protocol that fill
+    a block, are one longer, or are long, next to none of another; sources on either side of every cut.
+    Verdicts and the flow table against the oracle, and the counters against the verdicts, for batches
+    of part of a workgroup, of a few, and of more packets than the launch has lanes."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n)
+    base = W.CGNAT_BASE
+    net = lambda k: [(base | k << 8, 24)]  # noqa: E731
+    ends = lambda k: [(37 * i + 1, 37 * i + 1 + i % 3) for i in range(k)]  # noqa: E731
+    table = [(net(0), "tcp", [(0, 65535)]), (net(1), "udp", [(0, 65535)]), (net(2), "icmp", []),
+             (net(3), "tcp", [(0, 0), (65535, 65535)]), (net(4), "udp", [(0, 0), (65535, 65535), (1, 1)]),
+             (net(5), "tcp", ends(16)), (net(5), "udp", ends(17)), (net(6), "tcp", ends(17)), (net(6), "icmp", []),
+             (net(7), "udp", ends(300) + [(60000, 65535)]), (net(7), "tcp", [(65534, 65535)]), (net(8), "tcp", ends(33))]
+    ctx, ora = lib.Context(0), O.Filter()
+    ctx.filter_set_rules(table)
+    ora.set_rules(table)
+    proto = rng.choice([6, 6, 17, 17, 1], n).astype(np.uint8)
+    src = (base | rng.integers(0, 10, n) << 8 | rng.choice([0, 1, 255], n)).astype(np.uint32)
+    near = 37 * rng.integers(0, 305, n) + rng.integers(0, 4, n)
+    dport = np.where(rng.integers(0, 4, n) == 0, rng.choice([0, 1, 65534, 65535, 60000, 59999], n), near).astype(np.uint32)
+    sport = rng.integers(0, 65536, n).astype(np.uint32)
+    me = np.full(n, base | 0xFF01, np.uint32)
+    rec = np.ascontiguousarray(W.header_records(proto, src, me, sport, dport))
+    k = np.arange(0, n, 5)
+    out = np.ascontiguousarray(W.header_records(proto[k], me[k], src[k], dport[k], sport[k]))
+    d = torch.from_numpy(np.concatenate([rec.reshape(-1), np.zeros(16, np.uint8)])).to("cuda:0")
+    d_out = torch.from_numpy(out).to("cuda:0")
+    got = torch.full((n,), 9, dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
+    size = lambda m: (np.arange(m, dtype=np.uint64) * 32, np.full(m, 28, np.uint32))  # noqa: E731
+    for j in range(2):  # before the flows are noted, and after
+        want = ora.check_inbound_batch(rec.reshape(-1), *size(n), FC.T0 + j)
+        ctx.counters_reset()
+        ctx.filter_check_inbound(lib.make_batch(d, rec.nbytes, n, lib.MEM_DEVICE, stride=32, length=28), FC.T0 + j, got)
+        ctx.sync()
+        assert np.array_equal(got.cpu().numpy(), want)
+        seen = ctx.counters()
+        assert (seen["allowed"], seen["denied"]) == (int(want.sum()), n - int(want.sum()))
+        if j == 0:
+            ora.note_outbound_batch(out.reshape(-1), *size(k.size), FC.T0)
+            ctx.filter_note_outbound(lib.make_batch(d_out, out.nbytes, k.size, lib.MEM_DEVICE, stride=32, length=28), FC.T0)
+    assert ctx.filter_flows() == ora.flows()
+    ctx.close()

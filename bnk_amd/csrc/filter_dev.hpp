@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "wg_dev.hpp"
+
 namespace bnk {
 
 constexpr uint32_t FLOW_REGIONS = 6;     // protocol class (3) x top address bit (2)
@@ -107,6 +109,7 @@ struct FilterArgs {
                           // batch, has ended
     uint32_t record_blocks; // set by the launcher: the launch has that many workgroups with packets, and the
                           // last of them to be done leaves that record (0: it does not)
+    ReplayMark mark; // check only: bits of the batch's windows that are still to be set (n 0: none)
     RuleIndexDev rules;
     FlowTableDev flows;
 };
@@ -119,12 +122,27 @@ hipError_t launch_filter_check(const FilterArgs &a, uint32_t max_blocks, hipStre
 // claimed_upper: the host's upper bound on claimed slots.  Up to 4096 the
 // sweep cannot fire and its launch is left out.
 hipError_t launch_filter_note(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
-// The sweep alone, behind a launch that has noted the batch.
+// The sweep alone, behind a launch that has noted the batch; or what it does, for a launch of other work
+// with that many workgroups of SWEEP_THREADS more (flow_sweep in filter_lane.hpp; 0: nothing to do).
+struct SweepArgs {
+    FlowTableDev ft;
+    int64_t now;
+    uint64_t *record; // or nullptr
+    uint32_t seq, blocks;
+};
+constexpr uint32_t SWEEP_THREADS = 256;
+SweepArgs flow_sweep_args(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper);
 hipError_t launch_flow_sweep(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
 // launch_peer_rank_small (kernels.hpp), advancing, and launch_filter_note on the same batch in one launch.
 hipError_t launch_peer_rank_small_note(const uint32_t *peer, uint32_t n_keys, uint32_t n, uint64_t *ctr_base,
                                        uint64_t *ctr_out, uint64_t ctr_limit, uint32_t *status, const FilterArgs &note,
                                        uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
+// launch_peer_rank_counting (kernels.hpp), advancing, with launch_filter_note on the same batch in its two
+// launches, where peer_rank_whole says so.
+bool peer_rank_whole(uint32_t n, uint32_t n_keys);
+hipError_t launch_peer_rank_counting_note(const uint32_t *peer, void *tmp, uint64_t *ctr_base, uint32_t n_keys, uint32_t n,
+                                          uint64_t *ctr_out, uint64_t ctr_limit, uint32_t *status, const FilterArgs &note,
+                                          uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s);
 hipError_t launch_flow_rehash(const FlowTableDev &from, const FlowTableDev &to, uint32_t *status,
                               uint32_t max_blocks, hipStream_t s);
 

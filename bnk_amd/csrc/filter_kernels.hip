@@ -25,10 +25,13 @@
 // marker bit form the key word, so 0 can mean "empty" and a slot is claimed
 // with one 64-bit compare-and-swap.  Deleted entries keep their key and carry
 // expiry FLOW_TOMB.
+#include <algorithm>
+
 #include "../../include/bnkhip.h"
 #include "filter_dev.hpp"
 #include "filter_lane.hpp"
 #include "kernels.hpp"
+#include "wg_window.hpp"
 
 namespace bnk {
 
@@ -175,6 +178,12 @@ BNK_DEV bool rules_match_quad(const RuleIndexDev &ri, const QuadBlocks &q, uint3
 
 constexpr uint32_t LDS_BOUNDS_MAX = 24576; // 96 KiB of cut points
 constexpr uint32_t FILTER_THREADS = 1024; // one copy of the index serves 16 waves
+constexpr uint32_t CHECK_FEW_THREADS = 256;
+// filter_check_few_kernel up to here, us a launch against the other's, 6 rules and 64 flows / 4096 and
+// 65,536: 4096 packets 4.0 against 5.3 / 4.9 against 5.8, 32768 4.0, 5.5 / 5.2, 6.4, 131072 4.3, 5.5 / 6.3, 6.3,
+// 262144 5.0, 5.7 / 7.6, 6.8.
+constexpr uint32_t CHECK_FEW_MAX = 1u << 17;
+static_assert(CHECK_FEW_THREADS == REPLAY_MARK_THREADS, "one launch");
 
 // Where the three tables lie in a workgroup's LDS, in words, each on a 16-byte boundary:
 // the small presence bitmap, the jump table, the cut points.
@@ -269,18 +278,19 @@ BNK_DEV bool parse_fetched(const FilterArgs &a, const RawHeader &r, Parsed &o)
 }
 
 // filter.go:121-147 for a batch; enforcement is on (the host short-circuits
-// allow-all mode).  JUMPS: the cut points and the jump table are in LDS.
-template <int FROM, bool JUMPS>
-__global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterArgs a)
+// allow-all mode).  JUMPS: the cut points and the jump table are in LDS.  THREADS: of a workgroup;
+// FEW: of a batch for which the small bitmap is not worth staging.  block: of `blocks`.
+template <int FROM, bool JUMPS, uint32_t THREADS, bool FEW>
+BNK_DEV void check_main(const FilterArgs &a, uint32_t *lds, uint32_t block, uint32_t blocks_of)
 {
-    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
     const RuleIndexDev ri = a.rules;
     const bool in_lds = JUMPS || ri.n_bounds <= LDS_BOUNDS_MAX;
     constexpr bool jumps = JUMPS;
-    const bool small = a.small_in_lds != 0u && a.flows.counters[FLOW_CLAIMED] <= SMALL_KEYS_MAX;
-    uint32_t *lsmall = lds, *ljw = lds + (a.small_in_lds ? LDS_SMALL_WORDS : 0u), *lb = ljw + (jumps ? LDS_JUMP_ROOM : 0u);
+    const bool staged = !FEW && a.small_in_lds != 0u;
+    const bool small = staged && a.flows.counters[FLOW_CLAIMED] <= SMALL_KEYS_MAX;
+    uint32_t *lsmall = lds, *ljw = lds + (staged ? LDS_SMALL_WORDS : 0u), *lb = ljw + (jumps ? LDS_JUMP_ROOM : 0u);
     const uint16_t *lj = reinterpret_cast<const uint16_t *>(ljw);
-    const uint32_t stride = gridDim.x * FILTER_THREADS;
+    const uint32_t stride = blocks_of * THREADS;
     const uint32_t lane = threadIdx.x & 63u;
     // The first packet's header flies while the tables are staged, and theirs is one trip: 16
     // bytes per lane and load, all of them in flight together (word by word, each waited for:
@@ -292,40 +302,45 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     // table, mostly from beyond L2) 45.5.  Instructions no longer count: the same three took 42.7, 50.5 and
     // 58.3 with 355 vector instructions per 64 packets instead of 212 and every wave adding its verdicts to
     // the counters by itself (see the end of the kernel, which was most of it).
-    RawHeader raw = fetch_header<FROM>(a, blockIdx.x * FILTER_THREADS + threadIdx.x);
+    RawHeader raw = fetch_header<FROM>(a, block * THREADS + threadIdx.x);
     {
-        constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = (SMALL_QUADS + FILTER_THREADS - 1u) / FILTER_THREADS;
+        constexpr uint32_t SMALL_QUADS = LDS_SMALL_WORDS / 4u, SMALL_PER = FEW ? 0u : (SMALL_QUADS + THREADS - 1u) / THREADS;
+        constexpr uint32_t BOUND_PER = 8192u / 4u / THREADS; // (beyond 8192 cut points a load at a time)
+        constexpr uint32_t JUMP_PER = (LDS_JUMP_WORDS / 4u + THREADS - 1u) / THREADS;
         static_assert(LDS_SMALL_WORDS % 4u == 0u, "whole quads");
         const uint4 *const s4 = reinterpret_cast<const uint4 *>(a.flows.present_small);
         const uint4 *const b4 = reinterpret_cast<const uint4 *>(ri.bounds), *const j4 = reinterpret_cast<const uint4 *>(ri.jump);
         const uint32_t bq = in_lds ? ri.n_bounds / 4u : 0u, jq = jumps ? LDS_JUMP_WORDS / 4u : 0u;
         const uint32_t t = threadIdx.x;
-        uint4 sv[SMALL_PER], bv[2], jv;
+        uint4 sv[SMALL_PER ? SMALL_PER : 1u], bv[BOUND_PER], jv[JUMP_PER];
         uint32_t btail = 0, jtail = 0;
 #pragma unroll
-        for (uint32_t j = 0; j < SMALL_PER; j++) sv[j] = s4[min(t + j * FILTER_THREADS, SMALL_QUADS - 1u)];
+        for (uint32_t j = 0; j < SMALL_PER; j++) sv[j] = s4[min(t + j * THREADS, SMALL_QUADS - 1u)];
 #pragma unroll
-        for (uint32_t j = 0; j < 2u; j++) bv[j] = *(t + j * FILTER_THREADS < bq ? b4 + t + j * FILTER_THREADS : s4);
-        jv = *(t < jq ? j4 + t : s4);
+        for (uint32_t j = 0; j < BOUND_PER; j++) bv[j] = *(t + j * THREADS < bq ? b4 + t + j * THREADS : s4);
+#pragma unroll
+        for (uint32_t j = 0; j < JUMP_PER; j++) jv[j] = *(t + j * THREADS < jq ? j4 + t + j * THREADS : s4);
         if (in_lds && t < (ri.n_bounds & 3u)) btail = ri.bounds[4u * bq + t];
         if (jumps && t < (LDS_JUMP_WORDS & 3u)) jtail = reinterpret_cast<const uint32_t *>(ri.jump)[4u * jq + t];
-        if (a.small_in_lds) {
+        if (staged) {
 #pragma unroll
             for (uint32_t j = 0; j < SMALL_PER; j++)
-                if (t + j * FILTER_THREADS < SMALL_QUADS) reinterpret_cast<uint4 *>(lsmall)[t + j * FILTER_THREADS] = sv[j];
+                if (t + j * THREADS < SMALL_QUADS) reinterpret_cast<uint4 *>(lsmall)[t + j * THREADS] = sv[j];
         }
 #pragma unroll
-        for (uint32_t j = 0; j < 2u; j++)
-            if (t + j * FILTER_THREADS < bq) reinterpret_cast<uint4 *>(lb)[t + j * FILTER_THREADS] = bv[j];
-        if (t < jq) reinterpret_cast<uint4 *>(ljw)[t] = jv;
+        for (uint32_t j = 0; j < BOUND_PER; j++)
+            if (t + j * THREADS < bq) reinterpret_cast<uint4 *>(lb)[t + j * THREADS] = bv[j];
+#pragma unroll
+        for (uint32_t j = 0; j < JUMP_PER; j++)
+            if (t + j * THREADS < jq) reinterpret_cast<uint4 *>(ljw)[t + j * THREADS] = jv[j];
         if (in_lds && t < (ri.n_bounds & 3u)) lb[4u * bq + t] = btail;
         if (jumps && t < (LDS_JUMP_WORDS & 3u)) ljw[4u * jq + t] = jtail;
-        for (uint32_t q = t + 2u * FILTER_THREADS; q < bq; q += FILTER_THREADS) reinterpret_cast<uint4 *>(lb)[q] = b4[q];
+        for (uint32_t q = t + BOUND_PER * THREADS; q < bq; q += THREADS) reinterpret_cast<uint4 *>(lb)[q] = b4[q];
     }
     __syncthreads();
     uint32_t n_pass = 0, n_drop = 0; // this wave's verdicts (the same in every lane)
     uint32_t n_result = 0;           // with wg_tally: how often lane v's value v came out as the result
-    if (blockIdx.x == 0u && threadIdx.x == FILTER_THREADS - 64u) { // (the wave of a small batch that has nothing else to do)
+    if (block == 0u && threadIdx.x == THREADS - 64u) { // (the wave of a small batch that has nothing else to do)
         // (what this batch refreshes expires no earlier than this: news only if the clock went back)
         const int64_t from = a.now + FLOW_TTL_LEAST;
         for (const uint32_t w : {FLOW_MIN_EXP, FLOW_NEXT_EXP}) {
@@ -334,7 +349,7 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
         }
     }
     // whole waves stay in the loop together: the rule lookup is a joint effort
-    for (uint32_t i0 = blockIdx.x * FILTER_THREADS + (threadIdx.x & ~63u); i0 < a.n; i0 += stride) {
+    for (uint32_t i0 = block * THREADS + (threadIdx.x & ~63u); i0 < a.n; i0 += stride) {
         // t: this lane's place in the sweep; i: the packet it answers for
         const uint32_t t = i0 + lane;
         const uint32_t i = raw.i;
@@ -423,7 +438,7 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     // 8192 waves: 22 us of the launch over 2^22 headers).
     const bool results = FROM == FROM_ARRAYS && a.wg_tally;
     if (!a.tally && !results) return;
-    constexpr uint32_t WAVES = FILTER_THREADS / 64u, COUNTS = 18;
+    constexpr uint32_t WAVES = THREADS / 64u, COUNTS = 18;
     const uint32_t wave = threadIdx.x / 64u;
     __syncthreads(); // (nobody looks at the tables any more)
     if (lane == 0u) {
@@ -445,6 +460,26 @@ __global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterA
     }
 }
 
+template <int FROM, bool JUMPS>
+__global__ __launch_bounds__(FILTER_THREADS, 8) void filter_check_kernel(FilterArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+    check_main<FROM, JUMPS, FILTER_THREADS, false>(a, lds, blockIdx.x, gridDim.x);
+}
+
+// Small batches: without the small bitmap in LDS, whose 44 KiB a workgroup waits for longer than its
+// packets for their words of the large one, in smaller workgroups, and with the packets' bits going into
+// their windows in the same launch, which needs nothing of this and of which this needs nothing
+// (FilterArgs::mark; its workgroups come behind those of the packets).  Behind a decapsulating call of
+// 3000 packets 8.3 -> 5.6 us, of 8192 8.6 -> 5.5 with the 3.1 and the gap of the launch that marked.
+template <int FROM, bool JUMPS>
+__global__ __launch_bounds__(CHECK_FEW_THREADS) void filter_check_few_kernel(FilterArgs a, uint32_t blocks)
+{
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+    if (blockIdx.x < blocks) check_main<FROM, JUMPS, CHECK_FEW_THREADS, true>(a, lds, blockIdx.x, blocks);
+    else replay_mark(a.mark, blockIdx.x - blocks, gridDim.x - blocks);
+}
+
 // NoteOutbound of a batch (note_packet); the first workgroup has no packets (note_once).
 __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
 {
@@ -457,52 +492,7 @@ __global__ __launch_bounds__(256) void filter_note_kernel(FilterArgs a)
     note_block_done(a);
 }
 
-// filter.go:202-207: above 4096 entries, delete those with now.After(exp); there
-// is nothing to delete while no entry can have expired.  Nothing this launch
-// decides by changes while it runs: what it deletes and the bound it finds over
-// what it leaves go into words of their own until the next note launch.  (A
-// counter of finished note blocks in their place costs 23 ns per block.)
-//
-// Over the list of claimed slots: 14.4 us for 65,536, a gather each, where going through the
-// table they live in (200 MB, sized for batches of 2^18 packets) took 31 us behind every
-// batch.  The host cannot tell that nothing has expired, so the launch is made behind every
-// batch above 4096 entries; it returns at once then (2 to 5 us).  Being made, it leaves the record of
-// the batch ahead of it (FilterArgs::record_after; record null: not), which a launch for it alone did.
-__global__ __launch_bounds__(256) void flow_sweep_kernel(FlowTableDev ft, int64_t now, uint64_t *record, uint32_t seq)
-{
-    if (record && blockIdx.x == 0u && threadIdx.x == 0u)
-        __hip_atomic_store(record, (uint64_t)seq << 32 | ft.counters[FLOW_CLAIMED], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    if (ft.counters[FLOW_LIVE] <= FLOW_SWEEP_ABOVE || now <= *reinterpret_cast<const int64_t *>(ft.counters + FLOW_MIN_EXP)) return;
-    if (blockIdx.x == 0u && threadIdx.x == 0u) ft.counters[FLOW_SWEPT] = 1u;
-    const uint32_t claimed = ft.counters[FLOW_CLAIMED];
-    const uint32_t total = claimed < ft.cap / 2u ? claimed : ft.cap / 2u;
-    const uint32_t stride = gridDim.x * 256u;
-    int64_t least = INT64_MAX;
-    uint32_t gone = 0;
-    for (uint32_t idx = blockIdx.x * 256u + threadIdx.x; idx < total; idx += stride) {
-        FlowSlotMem *slot = ft.slots + ft.list[idx];
-        const int64_t e = slot->exp;
-        if (e == FLOW_TOMB) continue;
-        if (now > e) {
-            slot->exp = FLOW_TOMB;
-            gone++;
-        } else if (e < least) {
-            least = e;
-        }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        gone += (uint32_t)__shfl_xor((int)gone, off, 64);
-        const int64_t o = (int64_t)((uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)((uint64_t)least >> 32), off, 64) << 32 |
-                                    (uint32_t)__shfl_xor((int)(uint32_t)least, off, 64));
-        if (o < least) least = o;
-    }
-    if ((threadIdx.x & 63u) != 0u) return;
-    if (gone) atomicAdd(&ft.counters[FLOW_GONE], gone);
-    if (least != INT64_MAX)
-        (void)__hip_atomic_fetch_min(reinterpret_cast<int64_t *>(ft.counters + FLOW_NEXT_EXP), least, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
-}
+__global__ __launch_bounds__(SWEEP_THREADS) void flow_sweep_kernel(SweepArgs a) { flow_sweep(a, blockIdx.x); }
 
 // Moves every entry of the map into a larger table (tombstones are dropped).
 __global__ __launch_bounds__(256) void flow_rehash_kernel(FlowTableDev from, FlowTableDev to,
@@ -588,26 +578,43 @@ hipError_t launch_fill_u8(uint8_t *p, uint32_t n, uint8_t v, hipStream_t s)
     return hipGetLastError();
 }
 
+// (a workgroup's waves leave their counts there)
+constexpr uint32_t CHECK_LDS_LEAST = FILTER_THREADS / 64u * 18u * 4u;
+
 hipError_t launch_filter_check(const FilterArgs &args, uint32_t max_blocks, hipStream_t s)
 {
     if (args.n == 0) return hipSuccess;
     FilterArgs a = args;
+    const bool few = a.n <= CHECK_FEW_MAX;
     uint32_t lds = a.rules.n_bounds <= LDS_BOUNDS_MAX ? a.rules.n_bounds * 4u + (a.rules.jump ? LDS_JUMP_ROOM * 4u : 0u) : 0u;
     // the small bitmap rides along while two workgroups still fit a CU's 160 KiB
-    a.small_in_lds = lds + SMALL_BITS / 8u <= 80u * 1024u ? 1u : 0u;
+    a.small_in_lds = !few && lds + SMALL_BITS / 8u <= 80u * 1024u ? 1u : 0u;
     if (a.small_in_lds) lds += SMALL_BITS / 8u;
+    lds = std::max(lds, CHECK_LDS_LEAST);
     const bool jumps = a.rules.n_bounds <= LDS_BOUNDS_MAX && a.rules.jump != nullptr;
     const bool arrays = a.gate || a.lens || a.off || a.wg_result || a.limit != 0;
     void (*const kernels[3][2])(FilterArgs) = {{filter_check_kernel<FROM_PLAIN, false>, filter_check_kernel<FROM_PLAIN, true>},
                                                {filter_check_kernel<FROM_ARRAYS, false>, filter_check_kernel<FROM_ARRAYS, true>},
                                                {filter_check_kernel<FROM_RECORDS, false>, filter_check_kernel<FROM_RECORDS, true>}};
-    void (*const kernel)(FilterArgs) = kernels[a.heads ? FROM_RECORDS : arrays ? FROM_ARRAYS : FROM_PLAIN][jumps];
+    void (*const few_kernels[3][2])(FilterArgs, uint32_t) = {{filter_check_few_kernel<FROM_PLAIN, false>, filter_check_few_kernel<FROM_PLAIN, true>},
+                                                             {filter_check_few_kernel<FROM_ARRAYS, false>, filter_check_few_kernel<FROM_ARRAYS, true>},
+                                                             {filter_check_few_kernel<FROM_RECORDS, false>, filter_check_few_kernel<FROM_RECORDS, true>}};
+    const int from = a.heads ? FROM_RECORDS : arrays ? FROM_ARRAYS : FROM_PLAIN;
+    void (*const kernel)(FilterArgs) = kernels[from][jumps];
+    void (*const few_kernel)(FilterArgs, uint32_t) = few_kernels[from][jumps];
     if (lds > 48u * 1024u) {
         // more dynamic LDS than the default limit: opt in (gfx950 has 160 KiB per CU)
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipError_t e = hipFuncSetAttribute(few ? reinterpret_cast<const void *>(few_kernel) : reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)(LDS_BOUNDS_MAX * 4u + LDS_JUMP_ROOM * 4u));
         if (e != hipSuccess) return e;
     }
+    if (few) {
+        const uint32_t blocks = (a.n + CHECK_FEW_THREADS - 1u) / CHECK_FEW_THREADS;
+        hipLaunchKernelGGL(few_kernel, dim3(blocks + replay_mark_blocks(a.mark)), dim3(CHECK_FEW_THREADS), lds, s, a, blocks);
+        return hipGetLastError();
+    }
+    if (a.mark.n)
+        if (const hipError_t e = launch_wg_replay_mark(a.mark, s); e != hipSuccess) return e;
     // one index copy per workgroup: as many workgroups per CU as their LDS allows, two at most
     const uint32_t per_cu = lds > 80u * 1024u ? 1u : 2u;
     uint32_t blocks = (a.n + FILTER_THREADS - 1u) / FILTER_THREADS;
@@ -629,12 +636,22 @@ hipError_t launch_filter_note(const FilterArgs &args, uint32_t max_blocks, uint6
     return launch_flow_sweep(a, max_blocks, claimed_upper, s);
 }
 
+SweepArgs flow_sweep_args(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper)
+{
+    SweepArgs w{};
+    if (claimed_upper <= FLOW_SWEEP_ABOVE) return w;
+    w.ft = a.flows;
+    w.now = a.now;
+    w.record = a.record_after && !a.record_blocks ? a.record : nullptr;
+    w.seq = a.record_seq;
+    w.blocks = grid_for((uint32_t)(claimed_upper < a.flows.cap / 2u ? claimed_upper : a.flows.cap / 2u), max_blocks / 4u);
+    return w;
+}
+
 hipError_t launch_flow_sweep(const FilterArgs &a, uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
 {
-    if (claimed_upper <= FLOW_SWEEP_ABOVE) return hipGetLastError();
-    uint64_t *const record = a.record_after && !a.record_blocks ? a.record : nullptr;
-    const uint32_t most = (uint32_t)(claimed_upper < a.flows.cap / 2u ? claimed_upper : a.flows.cap / 2u);
-    hipLaunchKernelGGL(flow_sweep_kernel, dim3(grid_for(most, max_blocks / 4u)), dim3(256), 0, s, a.flows, a.now, record, a.record_seq);
+    const SweepArgs w = flow_sweep_args(a, max_blocks, claimed_upper);
+    if (w.blocks != 0u) hipLaunchKernelGGL(flow_sweep_kernel, dim3(w.blocks), dim3(SWEEP_THREADS), 0, s, w);
     return hipGetLastError();
 }
 

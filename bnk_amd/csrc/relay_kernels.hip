@@ -436,15 +436,14 @@ __device__ __forceinline__ void tile_words(const uint32_t *words, uint32_t first
 }
 
 template <bool SHIFTED, uint32_t RUNS>
-__global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
-                                                        uint32_t cols, uint32_t runs, uint32_t *table,
-                                                        uint32_t *status, unsigned shift)
+__device__ __forceinline__ void rank_count_tile(uint32_t tile, const uint32_t *keys, uint32_t n, uint32_t n_keys, uint32_t cols,
+                                                uint32_t runs, uint32_t *table, uint32_t *status, unsigned shift)
 {
     __shared__ __attribute__((aligned(16))) uint32_t cnt[RANK_TABLE_MAX_KEYS];
     const uint32_t lane = threadIdx.x;
     uint4 *cnt4 = reinterpret_cast<uint4 *>(cnt);
     for (uint32_t q = lane; q < cols / 4u; q += 64u) cnt4[q] = make_uint4(0, 0, 0, 0);
-    const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
+    const uint32_t first = tile * runs * 64u, end = min(n, first + runs * 64u);
     uint32_t word[RUNS];
     tile_words(keys, first, end, word);
     __syncthreads();
@@ -457,8 +456,16 @@ __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, ui
         else if (status) status_raise(status, STATUS_PEER_RANGE);
     }
     __syncthreads();
-    uint4 *row = reinterpret_cast<uint4 *>(table + (size_t)blockIdx.x * cols);
+    uint4 *row = reinterpret_cast<uint4 *>(table + (size_t)tile * cols);
     for (uint32_t q = lane; q < cols / 4u; q += 64u) row[q] = cnt4[q];
+}
+
+template <bool SHIFTED, uint32_t RUNS>
+__global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
+                                                        uint32_t cols, uint32_t runs, uint32_t *table,
+                                                        uint32_t *status, unsigned shift)
+{
+    rank_count_tile<SHIFTED, RUNS>(blockIdx.x, keys, n, n_keys, cols, runs, table, status, shift);
 }
 
 // One block per 16 peers: 64 groups of threads share the tiles between them.
@@ -519,6 +526,37 @@ __global__ __launch_bounds__(SCAN_PEERS * SCAN_PARTS) void rank_scan_kernel(uint
     }
 }
 
+// The walk over a tile, by one wave, in batch order: for every packet what stands at its key in
+// `before` once the lower runs have moved it (old), and how many lower lanes of its run have the key.
+// A key beyond n_keys is nobody's.
+template <uint32_t RUNS>
+__device__ __forceinline__ void tile_walk(uint32_t *before, const uint32_t (&key)[RUNS], uint32_t first, uint32_t end, uint32_t n_keys,
+                                          unsigned bits, uint32_t (&old)[RUNS], uint32_t (&lower)[RUNS])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) {
+        old[r] = lower[r] = 0u;
+        if (first + r * 64u < end) { // uniform
+            const uint32_t kk = key[r];
+            const bool valid = kk < n_keys;
+            // the lanes of this run with my peer
+            unsigned long long same = __ballot(valid);
+            for (unsigned b = 0; b < bits; b++) {
+                const unsigned long long m = __ballot((kk >> b) & 1u);
+                same &= ((kk >> b) & 1u) ? m : ~m;
+            }
+            lower[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+            // every lane reads its entry before the one lane of each peer moves it: LDS serves a
+            // wave's accesses in order, so nothing is waited for from run to run
+            old[r] = before[min(kk, n_keys - 1u)];
+            if (valid && lower[r] == 0u) atomicAdd(&before[kk], (uint32_t)__popcll(same));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
 template <uint32_t RUNS>
 __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, uint32_t n, uint32_t n_keys,
                                                          uint32_t cols, uint32_t runs, const uint32_t *table,
@@ -552,27 +590,7 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
     }
     __syncthreads();
     uint32_t old[RUNS], lower[RUNS];
-#pragma unroll
-    for (uint32_t r = 0; r < RUNS; r++) {
-        old[r] = lower[r] = 0u;
-        if (first + r * 64u < end) {
-            const uint32_t kk = key[r];
-            const bool valid = kk < n_keys;
-            // the lanes of this run with my peer
-            unsigned long long same = __ballot(valid);
-            for (unsigned b = 0; b < bits; b++) {
-                const unsigned long long m = __ballot((kk >> b) & 1u);
-                same &= ((kk >> b) & 1u) ? m : ~m;
-            }
-            lower[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-            // every lane reads its entry before the one lane of each peer moves it: LDS serves a
-            // wave's accesses in order, so nothing is waited for from run to run
-            old[r] = before[min(kk, n_keys - 1u)];
-            if (valid && lower[r] == 0u) atomicAdd(&before[kk], (uint32_t)__popcll(same));
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
+    tile_walk(before, key, first, end, n_keys, bits, old, lower);
 #pragma unroll
     for (uint32_t r = 0; r < RUNS; r++) {
         const uint32_t i = first + r * 64u + lane;
@@ -626,26 +644,171 @@ __global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, u
         }
     }
     __syncthreads();
-    uint32_t at[RUNS], lower[RUNS];
+    uint32_t key[RUNS], at[RUNS], lower[RUNS];
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) key[r] = first + r * 64u + lane < end ? rank_key(word[r], shift, n_keys) : NO_PEER;
+    tile_walk(before, key, first, end, n_keys, bits, at, lower);
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++)
+        if (first + r * 64u + lane < end) sorted[at[r] + lower[r]] = word[r];
+}
+
+// ---------------------------------------------------------------------------
+// The same in two launches, of batches whose table is so short that every tile adds up the rows
+// before its own by itself: up to WHOLE_TILES tiles, as long as a wave keeps their packets' words, and
+// WHOLE_MAX_KEYS keys.  In batches of this size a launch costs more than what it does (the scan by itself 5
+// us and the gap to the next launch 2).  Device-resident tunnel passes of IMIX packets of 64 peers with three
+// streams at work, 15 launches -> 10, together with the windows' bits in the filter's launch: 4097 packets
+// 50.4 -> 37.8 us, 8192 48.6 -> 38.5, 16384 50.1 -> 40.1, 32768 61.6 -> 54.5.  The counting launch leaves the peers' counters as the batch
+// found them, so that the assigning one can move them while it reads; it also takes NoteOutbound of the
+// batch along, which nothing of all this needs, and the assigning one the sweep behind that.
+// ---------------------------------------------------------------------------
+constexpr uint32_t WHOLE_TILES = 64, WHOLE_MAX_KEYS = 1024, WHOLE_THREADS = 256;
+static_assert(WHOLE_THREADS == SWEEP_THREADS && WHOLE_THREADS == RANK_ROW_STEP && WHOLE_TILES % 4u == 0u, "one launch; a thread a column");
+
+static bool rank_whole_plan(uint32_t n, uint32_t n_keys, RankPlan &p)
+{
+    if (n > WHOLE_TILES * 64u * TILE_RUNS_FEW || n_keys > WHOLE_MAX_KEYS) return false;
+    p.runs = (n + 64u * WHOLE_TILES - 1u) / (64u * WHOLE_TILES);
+    p.tiles = (n + 64u * p.runs - 1u) / (64u * p.runs);
+    return true; // (never more tiles than rank_plan has: its scratch holds them)
+}
+
+// What stands in the columns of the first `upto` of the table's rows, and in all of them, by the
+// workgroup's four waves: a quarter of the rows each, all of a step's loads in flight at once.
+template <bool BELOW, bool ALL>
+__device__ __forceinline__ void rows_sum(const uint32_t *table, uint32_t cols, uint32_t tiles, uint32_t upto, uint32_t *below, uint32_t *all)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t part[2][WHOLE_THREADS / 64u][RANK_ROW_STEP];
+    constexpr uint32_t WAVES = WHOLE_THREADS / 64u, PER = WHOLE_TILES / WAVES;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, rows = ALL ? tiles : upto;
+    for (uint32_t q = 0; q < cols; q += RANK_ROW_STEP) {
+        uint4 v[PER];
+#pragma unroll
+        for (uint32_t j = 0; j < PER; j++)
+            v[j] = *reinterpret_cast<const uint4 *>(table + (size_t)min(wave + WAVES * j, tiles - 1u) * cols + q + 4u * lane);
+        uint4 b = make_uint4(0, 0, 0, 0), s = b;
+#pragma unroll
+        for (uint32_t j = 0; j < PER; j++) {
+            const uint32_t row = wave + WAVES * j;
+            if (row < rows) { s.x += v[j].x; s.y += v[j].y; s.z += v[j].z; s.w += v[j].w; }
+            if (BELOW && row < upto) { b.x += v[j].x; b.y += v[j].y; b.z += v[j].z; b.w += v[j].w; }
+        }
+        if (ALL) *reinterpret_cast<uint4 *>(&part[0][wave][4u * lane]) = s;
+        if (BELOW) *reinterpret_cast<uint4 *>(&part[1][wave][4u * lane]) = b;
+        __syncthreads();
+        const uint32_t t = threadIdx.x;
+        if (ALL) all[q + t] = part[0][0][t] + part[0][1][t] + part[0][2][t] + part[0][3][t];
+        if (BELOW) below[q + t] = part[1][0][t] + part[1][1][t] + part[1][2][t] + part[1][3][t];
+        __syncthreads();
+    }
+}
+
+struct WholeArgs {
+    const uint32_t *keys;
+    uint32_t n, n_keys, cols, runs, tiles;
+    uint32_t *table;
+    uint64_t *ctr_base, *base_was;
+    uint32_t *status;
+};
+
+// Workgroups: the tiles, the peers' counters, then those of NoteOutbound (note_once, and a packet a lane).
+template <uint32_t RUNS>
+__global__ __launch_bounds__(64) void rank_count_whole_kernel(WholeArgs a, FilterArgs note)
+{
+    const uint32_t b = blockIdx.x;
+    if (b < a.tiles) {
+        rank_count_tile<false, RUNS>(b, a.keys, a.n, a.n_keys, a.cols, a.runs, a.table, a.status, 0u);
+    } else if (b == a.tiles) {
+        for (uint32_t k = threadIdx.x; k < a.n_keys; k += 64u) a.base_was[k] = a.ctr_base[k];
+    } else if (b == a.tiles + 1u) {
+        if (threadIdx.x == 0u) note_once(note);
+    } else {
+        const uint32_t i = (b - a.tiles - 2u) * 64u + threadIdx.x;
+        if (i < note.n) note_packet(note, i);
+        note_block_done(note);
+    }
+}
+
+// Workgroups: the tiles, one that moves the peers' counters (with advance), the sweep's.
+template <uint32_t RUNS>
+__global__ __launch_bounds__(WHOLE_THREADS) void rank_assign_whole_kernel(WholeArgs a, unsigned bits, uint64_t *ctr_out, uint64_t ctr_limit,
+                                                                          int zero_others, int advance, SweepArgs sweep)
+{
+    __shared__ uint32_t before[WHOLE_MAX_KEYS];
+    const uint32_t b = blockIdx.x;
+    if (b > a.tiles) {
+        flow_sweep(sweep, b - a.tiles - 1u);
+        return;
+    }
+    if (b == a.tiles) {
+        if (!advance) return;
+        rows_sum<false, true>(a.table, a.cols, a.tiles, 0u, nullptr, before);
+        for (uint32_t k = threadIdx.x; k < a.n_keys; k += WHOLE_THREADS)
+            if (before[k] != 0u) a.ctr_base[k] = ctr_add(a.base_was[k], before[k], ctr_limit);
+        return;
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t first = b * a.runs * 64u, end = min(a.n, first + a.runs * 64u);
+    uint32_t key[RUNS];
+    uint64_t base[RUNS];
 #pragma unroll
     for (uint32_t r = 0; r < RUNS; r++) {
-        at[r] = lower[r] = 0u;
-        if (first + r * 64u < end) { // uniform
-            const bool valid = first + r * 64u + lane < end;
-            const uint32_t kk = rank_key(word[r], shift, n_keys);
-            unsigned long long same = __ballot(valid);
-            for (unsigned b = 0; b < bits; b++) {
-                const unsigned long long m = __ballot((kk >> b) & 1u);
-                same &= ((kk >> b) & 1u) ? m : ~m;
-            }
-            lower[r] = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
-            // (see rank_assign_kernel)
-            at[r] = before[kk];
-            if (valid && lower[r] == 0u) atomicAdd(&before[kk], (uint32_t)__popcll(same));
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
+        const uint32_t i = first + r * 64u + lane, k = a.keys[min(i, end - 1u)];
+        key[r] = i < end ? k : NO_PEER;
     }
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) base[r] = a.base_was[min(key[r], a.n_keys - 1u)];
+    rows_sum<true, false>(a.table, a.cols, a.tiles, b, before, nullptr);
+    if (threadIdx.x >= 64u) return;
+    uint32_t old[RUNS], lower[RUNS];
+    tile_walk(before, key, first, end, a.n_keys, bits, old, lower);
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) {
+        const uint32_t i = first + r * 64u + lane;
+        const bool valid = key[r] < a.n_keys;
+        if (i < end && (valid || zero_others)) ctr_out[i] = valid ? ctr_add(base[r], old[r] + lower[r], ctr_limit) : 0ull;
+    }
+}
+
+// The second launch when the batch is to be sorted (rank_place_kernel).
+template <uint32_t RUNS>
+__global__ __launch_bounds__(WHOLE_THREADS) void rank_place_whole_kernel(const uint32_t *words, uint32_t n, uint32_t n_keys, uint32_t cols,
+                                                                         uint32_t runs, uint32_t tiles, const uint32_t *table,
+                                                                         unsigned bits, unsigned shift, uint32_t *sorted)
+{
+    __shared__ uint32_t before[WHOLE_MAX_KEYS], total[WHOLE_MAX_KEYS];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
+    uint32_t word[RUNS];
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) word[r] = words[min(first + r * 64u + lane, end - 1u)];
+    rows_sum<true, true>(table, cols, tiles, blockIdx.x, before, total);
+    if (threadIdx.x >= 64u) return;
+    // where each key's packets begin
+    uint32_t base = 0;
+    for (uint32_t q = 0; q < cols; q += RANK_ROW_STEP) {
+        const uint32_t c = q + 4u * lane; // (columns beyond the keys are all 0)
+        const uint32_t t0 = total[c], t1 = total[c + 1u], t2 = total[c + 2u], t3 = total[c + 3u], mine = t0 + t1 + t2 + t3;
+        uint32_t inc = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)inc, off, 64);
+            if ((int)lane >= off) inc += o;
+        }
+        const uint32_t s0 = base + inc - mine;
+        before[c] += s0;
+        before[c + 1u] += s0 + t0;
+        before[c + 2u] += s0 + t0 + t1;
+        before[c + 3u] += s0 + t0 + t1 + t2;
+        base += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t key[RUNS], at[RUNS], lower[RUNS];
+#pragma unroll
+    for (uint32_t r = 0; r < RUNS; r++) key[r] = first + r * 64u + lane < end ? rank_key(word[r], shift, n_keys) : NO_PEER;
+    tile_walk(before, key, first, end, n_keys, bits, at, lower);
 #pragma unroll
     for (uint32_t r = 0; r < RUNS; r++)
         if (first + r * 64u + lane < end) sorted[at[r] + lower[r]] = word[r];
@@ -668,8 +831,16 @@ size_t peer_sort_tmp_bytes(uint32_t n, uint32_t n_peers)
 hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n, uint32_t n_peers, unsigned shift,
                             void *tmp, hipStream_t s)
 {
-    const RankPlan plan = sort_plan(n, n_peers);
+    RankPlan plan = sort_plan(n, n_peers);
     const uint32_t n_keys = n_peers + 1u;
+    if (rank_whole_plan(n, n_keys, plan)) {
+        uint32_t *const table = static_cast<uint32_t *>(tmp);
+        hipLaunchKernelGGL((rank_count_kernel<true, TILE_RUNS_FEW>), dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs,
+                           table, (uint32_t *)nullptr, shift);
+        hipLaunchKernelGGL(rank_place_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles), dim3(WHOLE_THREADS), 0, s, words, n, n_keys, plan.cols,
+                           plan.runs, plan.tiles, table, key_bits(n_keys), shift, sorted);
+        return hipGetLastError();
+    }
     uint32_t *table = static_cast<uint32_t *>(tmp), *total = table + (size_t)plan.tiles * plan.cols;
     const auto count = plan.runs <= TILE_RUNS_FEW ? rank_count_kernel<true, TILE_RUNS_FEW> : rank_count_kernel<true, TILE_RUNS_MAX>;
     const auto place = plan.runs <= TILE_RUNS_FEW ? rank_place_kernel<TILE_RUNS_FEW> : rank_place_kernel<TILE_RUNS_MAX>;
@@ -682,11 +853,49 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
     return hipGetLastError();
 }
 
+// note: null, or the batch's NoteOutbound, with the sweep behind it.
+static hipError_t launch_peer_rank_whole(const uint32_t *keys, const RankPlan &plan, void *tmp, uint64_t *ctr_base, uint32_t n_keys,
+                                         uint32_t n, uint64_t *ctr_out, bool advance, uint64_t ctr_limit, bool zero_others,
+                                         uint32_t *status, const FilterArgs *note, const SweepArgs &sweep, hipStream_t s)
+{
+    uint32_t *const table = static_cast<uint32_t *>(tmp);
+    uint64_t *const base_was = reinterpret_cast<uint64_t *>(table + (size_t)plan.tiles * plan.cols);
+    const WholeArgs a{keys, n, n_keys, plan.cols, plan.runs, plan.tiles, table, ctr_base, base_was, status};
+    const uint32_t noting = note ? 1u + (note->n + 63u) / 64u : 0u;
+    hipLaunchKernelGGL(rank_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + noting), dim3(64), 0, s, a, note ? *note : FilterArgs{});
+    hipLaunchKernelGGL(rank_assign_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + sweep.blocks), dim3(WHOLE_THREADS), 0, s, a,
+                       key_bits(n_keys), ctr_out, ctr_limit, zero_others ? 1 : 0, advance ? 1 : 0, sweep);
+    return hipGetLastError();
+}
+
+bool peer_rank_whole(uint32_t n, uint32_t n_keys)
+{
+    RankPlan p{};
+    return rank_whole_plan(n, n_keys, p);
+}
+
+hipError_t launch_peer_rank_counting_note(const uint32_t *peer, void *tmp, uint64_t *ctr_base, uint32_t n_keys, uint32_t n,
+                                          uint64_t *ctr_out, uint64_t ctr_limit, uint32_t *status, const FilterArgs &note,
+                                          uint32_t max_blocks, uint64_t claimed_upper, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    RankPlan plan = rank_plan(n, n_keys);
+    if (!rank_whole_plan(n, n_keys, plan) || note.n != n) return hipErrorInvalidValue;
+    FilterArgs f = note;
+    const SweepArgs sweep = flow_sweep_args(f, max_blocks, claimed_upper);
+    f.record_blocks = f.record && f.record_after && sweep.blocks == 0u ? (n + 63u) / 64u : 0u;
+    return launch_peer_rank_whole(peer, plan, tmp, ctr_base, n_keys, n, ctr_out, true, ctr_limit, true, status, &f, sweep, s);
+}
+
 static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &plan, void *tmp,
                                          uint64_t *ctr_base, uint32_t n_keys, uint32_t n, uint64_t *ctr_out,
                                          bool advance, uint64_t ctr_limit, bool zero_others, uint32_t *status,
                                          hipStream_t s)
 {
+    RankPlan whole = plan;
+    if (rank_whole_plan(n, n_keys, whole))
+        return launch_peer_rank_whole(keys, whole, tmp, ctr_base, n_keys, n, ctr_out, advance, ctr_limit, zero_others, status, nullptr,
+                                      SweepArgs{}, s);
     uint32_t *table = static_cast<uint32_t *>(tmp);
     uint32_t *total = table + (size_t)plan.tiles * plan.cols;
     uint64_t *base_was = reinterpret_cast<uint64_t *>(total + plan.cols);

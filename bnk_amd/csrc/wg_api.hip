@@ -505,6 +505,11 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
             HIPCHK(ctx, launch_peer_rank_small(d_peer, pe.n, n, pe.send_ctr, d_ctr, true, WG_REJECT_AFTER_MESSAGES,
                                                ctx->d_status, ctx->stream));
         }
+    } else if (d_peer && peer_rank_counts(n, pe.n, tmp_bytes) && note && !chunked && peer_rank_whole(n, pe.n)) {
+        HIPCHK(ctx, launch_peer_rank_counting_note(d_peer, ctx->r_tmp.p, pe.send_ctr, pe.n, n, d_ctr, WG_REJECT_AFTER_MESSAGES,
+                                                   ctx->d_status, note_args(0, n), ctx->filter->max_blocks, ctx->filter->bound.upper,
+                                                   ctx->stream));
+        noted = true;
     } else if (d_peer && peer_rank_counts(n, pe.n, tmp_bytes)) {
         HIPCHK(ctx, launch_peer_rank_counting(d_peer, ctx->r_tmp.p, pe.send_ctr, pe.n, n, d_ctr, true,
                                               WG_REJECT_AFTER_MESSAGES, ctx->d_status, ctx->stream));
@@ -872,14 +877,17 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     }
     // wireguard-go's sequential receiver validates the counter of every
     // authentic packet before it looks inside: ahead of the inbound filter
+    // (with the filter behind it, it sets the last of the windows' bits)
+    ReplayMark rest{};
     auto replay_range = [&](uint32_t lo, uint32_t hi, bool keys_from_open = false) -> int {
+        rest.n = 0;
         if (!replay) return BNK_OK;
         WgReplayScratch c = rsc;
         c.table_slots = wg_replay_one_block(hi - lo, pe.n) ? 0 : wg_replay_table_slots(hi - lo);
         if (c.table_slots) c.parity = ctx->wg_replay_parity++ & 1u;
         c.keys_ready = keys_from_open;
         HIPCHK(ctx, launch_wg_replay(d_result + lo, d_out_len + lo, d_peer + lo, d_counter + lo, hi - lo, rpd, c,
-                                     ctx->stream));
+                                     check ? &rest : nullptr, ctx->stream));
         return BNK_OK;
     };
 
@@ -899,6 +907,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         fa.rules = f->ridx;
         fa.flows = f->flows;
         fa.wg_result = d_result + lo;
+        fa.mark = rest;
         if (!host && counted && ctx->tally_on.load(std::memory_order_relaxed)) {
             // (every result is final once the filter has seen it)
             fa.wg_tally = reinterpret_cast<unsigned long long *>(ctx->d_tally);

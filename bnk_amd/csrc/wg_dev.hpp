@@ -66,6 +66,19 @@ struct WgReplayScratch {
     void *tmp;                             // wg_replay_tmp_bytes(n, n_peers)
     size_t tmp_bytes;
 };
+// The last part of a pass over more packets than that: the bits of what reached the bit test, and the
+// scratch made ready for the next pass (replay_mark in wg_window.hpp).
+struct ReplayMark {
+    const uint32_t *skeys;
+    const uint64_t *sctr;
+    const uint8_t *cls;
+    uint64_t *state;
+    uint32_t *table, *flags;
+    uint32_t n, slots, parity;
+};
+constexpr uint32_t REPLAY_MARK_THREADS = 256;
+inline uint32_t replay_mark_blocks(const ReplayMark &m) { return m.n / REPLAY_MARK_THREADS + (m.n % REPLAY_MARK_THREADS != 0u); }
+hipError_t launch_wg_replay_mark(const ReplayMark &m, hipStream_t s);
 size_t wg_replay_tmp_bytes(uint32_t n, uint32_t n_peers);
 // When a sender and a position within a pass of n packets fit one word together: the bits
 // the position takes (the sender sits above them; see wg_replay_pack), else 0.  With it
@@ -76,9 +89,10 @@ uint32_t wg_replay_table_slots(uint32_t n);
 // Runs every packet whose result so far says "authentic" (anything but
 // BAD_HEADER, UNKNOWN_INDEX, AUTH_FAIL) through its peer's window, in batch
 // order per peer; a packet the window turns away gets BNK_WG_REPLAY and
-// out_len 0.  The arrays are indexed from the first packet of the pass.
+// out_len 0.  The arrays are indexed from the first packet of the pass.  rest: null, or what is left to
+// do goes there (n 0: nothing), for a launch that the caller makes next on the stream.
 hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *peer, const uint64_t *counter,
-                            uint32_t n, const WgReplayDev &rp, const WgReplayScratch &sc, hipStream_t s);
+                            uint32_t n, const WgReplayDev &rp, const WgReplayScratch &sc, ReplayMark *rest, hipStream_t s);
 // Clears the windows of the rows whose flag is set.
 hipError_t launch_wg_replay_reset(uint64_t *state, const uint8_t *flags, uint32_t n_peers, hipStream_t s);
 

@@ -260,14 +260,6 @@ __device__ __forceinline__ uint64_t seg_handed(const uint64_t *carry_x, const ui
     return acc;
 }
 
-// What the window decides about a packet without looking at other packets'
-// counters: turned away outright, ahead of everything before it (fresh for
-// certain), inside the window with its bit set before the batch (a repeat for
-// certain), or inside the window at or below an earlier counter with the bit
-// clear ("late": fresh unless an earlier packet of the batch carried the
-// counter too).
-enum : uint8_t { RP_NONE = 0, RP_AHEAD = 1, RP_LATE = 2, RP_SEEN = 3 };
-
 __device__ __forceinline__ uint32_t table_home(uint32_t key, uint64_t c, uint32_t mask)
 {
     return (uint32_t)mix(c ^ ((uint64_t)key << 40) ^ key) & mask;
@@ -397,66 +389,7 @@ __global__ __launch_bounds__(256) void replay_late_advance_kernel(const uint32_t
     advance_window(state + (size_t)key * WG_REPLAY_WORDS, last);
 }
 
-// Sets `bit` of `block` in the window of peer `key` for every lane that has one (key NO_PEER:
-// none).  A lane whose left neighbour differs gathers the bits of the lanes behind it that
-// agree with it in peer and block and issues one atomic for all of them.
-__device__ __forceinline__ void mark_bits(uint64_t *state, uint32_t key, uint64_t block, uint64_t bit)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    // runs of equal (peer, block) among neighbouring lanes
-    const uint32_t pkey = (uint32_t)__shfl_up((int)key, 1, 64);
-    const uint32_t pblo = (uint32_t)__shfl_up((int)(uint32_t)block, 1, 64);
-    const uint32_t pbhi = (uint32_t)__shfl_up((int)(uint32_t)(block >> 32), 1, 64);
-    const bool head = lane == 0 || pkey != key || pblo != (uint32_t)block || pbhi != (uint32_t)(block >> 32);
-    const unsigned long long heads = __ballot(head);
-    // my run ends before the next head after me
-    const unsigned long long after = lane == 63u ? 0ull : heads & ~((2ull << lane) - 1ull);
-    const uint32_t end = after ? (uint32_t)__ffsll((long long)after) - 1u : 64u;
-    uint64_t acc = bit;
-    // suffix OR within the run: six doubling steps cover 64 lanes
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t lo = (uint32_t)__shfl_down((int)(uint32_t)acc, off, 64);
-        const uint32_t hi = (uint32_t)__shfl_down((int)(uint32_t)(acc >> 32), off, 64);
-        if (lane + (uint32_t)off < end) acc |= (uint64_t)hi << 32 | lo;
-    }
-    if (head && key != NO_PEER && acc != 0)
-        atomicOr(reinterpret_cast<unsigned long long *>(
-                     &state[(size_t)key * WG_REPLAY_WORDS + 1u + (block & (WG_REPLAY_BLOCKS - 1u))]),
-                 (unsigned long long)acc);
-}
-
-// Sets the bit of every packet that reached the bit test and still lies in the
-// window its peer ends the batch with.  Neighbours in sorted order mostly
-// share their peer and their block of 64 counters.
-//
-// The same launch leaves the first-occurrence table empty for the next pass
-// (nothing to do when this pass had no late packet, the usual case) and clears
-// the flag word the next pass will use (nobody reads that one now).
-__global__ __launch_bounds__(256) void replay_mark_kernel(const uint32_t *skeys, const uint64_t *sctr,
-                                                          const uint8_t *cls, uint64_t *state, uint32_t n,
-                                                          uint32_t *table, uint32_t slots, uint32_t *flags,
-                                                          uint32_t parity)
-{
-    if (blockIdx.x == 0 && threadIdx.x == 0) flags[parity ^ 1u] = 0u;
-    if (flags[parity] != 0u)
-        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < slots; i += gridDim.x * 256u) table[i] = HASH_EMPTY;
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
-    uint32_t key = NO_PEER;
-    uint64_t block = ~0ull, bit = 0;
-    if (p < n && cls[p] != RP_NONE) {
-        key = skeys[p];
-        const uint64_t c = sctr[p];
-        const uint64_t final_last = state[(size_t)key * WG_REPLAY_WORDS];
-        if ((final_last >> 6) - (c >> 6) < WG_REPLAY_BLOCKS) { // else its slot now belongs to a later block
-            block = c >> 6;
-            bit = 1ull << (c & 63u);
-        } else {
-            key = NO_PEER;
-        }
-    }
-    mark_bits(state, key, block, bit);
-}
+__global__ __launch_bounds__(REPLAY_MARK_THREADS) void replay_mark_kernel(ReplayMark m) { replay_mark(m, blockIdx.x, gridDim.x); }
 
 unsigned key_bits(uint32_t n_keys)
 {
@@ -776,8 +709,9 @@ bool wg_replay_one_block(uint32_t n, uint32_t n_peers)
 }
 
 hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *peer, const uint64_t *counter,
-                            uint32_t n, const WgReplayDev &rp, const WgReplayScratch &sc, hipStream_t s)
+                            uint32_t n, const WgReplayDev &rp, const WgReplayScratch &sc, ReplayMark *rest, hipStream_t s)
 {
+    if (rest) rest->n = 0;
     if (n == 0) return hipSuccess;
     if (n <= 256u) {
         hipLaunchKernelGGL(replay_small_kernel<256>, dim3(1), dim3(256), 0, s, result, out_len, peer, counter,
@@ -833,8 +767,15 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
                        out_len);
     hipLaunchKernelGGL(replay_late_advance_kernel, grid, dim3(256), 0, s, sc.skeys, sc.sidx, sc.sctr, sc.pmax, sc.cls,
                        rp.state, n, sc.table, mask, late_flag, result, out_len);
-    hipLaunchKernelGGL(replay_mark_kernel, grid, dim3(256), 0, s, sc.skeys, sc.sctr, sc.cls, rp.state, n, sc.table,
-                       sc.table_slots, sc.flags, sc.parity);
+    const ReplayMark m{sc.skeys, sc.sctr, sc.cls, rp.state, sc.table, sc.flags, n, sc.table_slots, sc.parity};
+    if (!rest) return launch_wg_replay_mark(m, s);
+    *rest = m;
+    return hipGetLastError();
+}
+
+hipError_t launch_wg_replay_mark(const ReplayMark &m, hipStream_t s)
+{
+    hipLaunchKernelGGL(replay_mark_kernel, dim3(replay_mark_blocks(m)), dim3(REPLAY_MARK_THREADS), 0, s, m);
     return hipGetLastError();
 }
 

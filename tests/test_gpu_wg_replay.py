@@ -540,3 +540,99 @@ def test_counters_and_windows_of_one_workgroup_over_the_peers_digits(n_peers, n)
             assert np.array_equal(res.cpu().numpy(), want)
             assert np.array_equal(olen.cpu().numpy(), np.where(want == lib.WG_OK, length, 0))
             assert len(np.unique(want)) == 2
+
+
+@pytest.mark.parametrize("n_peers,n", [(1, 4097), (255, 5000), (256, 8191), (1023, 32768), (1024, 6000), (3, 32769)])
+def test_tunnel_batches_whose_tiles_add_up_the_rows_before_theirs(n_peers, n):
+    """NoteOutbound and encapsulation, then decapsulation, windows and CheckInbound of device-resident
+    batches between those of one workgroup and those with a launch for the scan: tables of one row of
+    columns, of several and of one key too many, batches of one run a tile and of as many as a wave
+    keeps; counters against the count of earlier packets, windows (repeats, old packets, jumps, two
+    batches in a row) against the sequential filter, verdicts and the flow tables against the oracle."""
+    import torch
+    from bnk_amd import lib
+    from bnk_amd import workloads as W
+    from oracle import binding as O
+    rng = np.random.default_rng(n_peers + n)
+    base, t0 = 0x64400000, 1_700_000_000 * 10**9
+    tx = [(10 + 3 * i, 500000 + 5 * i, base + i, 0xFFFFFFFF) for i in range(n_peers)]
+    rx = [(p[1], p[0], p[2], p[3]) for p in tx]
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    rules = [([(base, 10)], "tcp", [(0, 999)]), ([(base, 10)], "udp", [(65000, 65535)])]
+    peer = rng.integers(0, n_peers, n).astype(np.uint32)
+    peer[:n // 3] = n_peers - 1
+    rng.shuffle(peer)
+    slot, length = 96, 40
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    i32 = lambda: torch.full((n,), 99, dtype=torch.int32, device="cuda:0")  # noqa: E731
+    at = lambda m: (np.arange(m, dtype=np.uint64) * slot, np.full(m, length, np.uint32))  # noqa: E731
+    with lib.Context(0) as txc, lib.Context(0) as rxc:
+        sent, flows_in = O.Filter(), O.Filter()
+        for c, o, k in ((txc, sent, lib.KEYS_SEND), (rxc, flows_in, lib.KEYS_RECV)):
+            c.keys_set(k, keys)
+            c.wg_peers_set(tx if c is txc else rx)
+            c.filter_set_rules(rules)
+            o.set_rules(rules)
+        first = {int(p): 9000 + int(p) % 7 for p in rng.choice(n_peers, min(n_peers, 40), replace=False)}
+        for p, c in first.items():
+            txc.wg_send_counter_set(p, c)
+        nxt = np.array([first.get(p, 0) for p in range(n_peers)], np.uint64)
+        wires, inner, ctrs = [], [], []
+        for k in range(2):
+            src = (base + peer).astype(np.uint32)
+            proto = rng.choice([6, 17, 1], n).astype(np.uint8)
+            rec = W.header_records(proto, src, np.full(n, base | 0xFFFF, np.uint32), rng.integers(0, 2000, n).astype(np.uint32),
+                                   rng.choice([0, 999, 1000, 64999, 65000, 65535], n).astype(np.uint32))
+            rows = rng.integers(0, 256, (n, slot), dtype=np.uint8)
+            rows[:, 16:16 + 28] = rec[:, :28]
+            rows[:, 18], rows[:, 19] = 0, length
+            want = np.zeros(n, np.uint64)
+            for i in range(n):
+                want[i] = nxt[peer[i]]
+                nxt[peer[i]] += 1
+            sent.note_outbound_batch(np.ascontiguousarray(rows[:, 16:]).reshape(-1), np.arange(n, dtype=np.uint64) * (slot - 16),
+                                     at(n)[1], t0 + k)
+            buf, wl = d(rows.reshape(-1)), i32()
+            torch.cuda.synchronize()
+            txc.wg_note_encap(lib.make_batch(buf, n * slot, n, lib.MEM_DEVICE, stride=slot, length=length, peer=d(peer.view(np.int32))),
+                              1420, t0 + k, wl)
+            txc.sync()
+            assert (wl == 80).all()
+            wires.append(buf.cpu().numpy().reshape(n, slot))
+            assert np.array_equal(wires[-1][:, 8:16].copy().view("<u8").reshape(-1), want)
+            inner.append(rows[:, 16:16 + length].copy())
+            ctrs.append(want)
+            assert txc.filter_flows() == sent.flows()
+        assert np.array_equal(txc.wg_send_counters(n_peers), nxt)
+        # some of the flows are ours: what comes back on them passes whatever the rules say
+        back = np.concatenate(inner)[::7].copy()
+        back[:, 12:16], back[:, 16:20] = np.concatenate(inner)[::7, 16:20], np.concatenate(inner)[::7, 12:16]
+        back[:, 20:22], back[:, 22:24] = np.concatenate(inner)[::7, 22:24], np.concatenate(inner)[::7, 20:22]
+        flat = np.ascontiguousarray(back).reshape(-1)
+        offs = np.arange(len(back), dtype=np.uint64) * length
+        flows_in.note_outbound_batch(flat, offs, np.full(len(back), length, np.uint32), t0)
+        rxc.filter_note_outbound(lib.make_batch(flat, flat.nbytes, len(back), lib.MEM_HOST, offsets=offs,
+                                                lens=np.full(len(back), length, np.uint32)), t0)
+        both, who, ctr, plain = np.concatenate(wires), np.concatenate([peer, peer]), np.concatenate(ctrs), np.concatenate(inner)
+        filters = {}
+        # the second half in order, then any of both again and again
+        for k, pick in enumerate([np.arange(n, 2 * n), rng.integers(0, 2 * n, n), rng.integers(0, 2 * n, n)]):
+            fresh = np.array([filters.setdefault(int(who[i]), O.ReplayFilter()).validate(int(ctr[i])) for i in pick])
+            rows = both[pick].copy()
+            want = np.full(n, lib.WG_REPLAY, np.uint8)
+            got_in = np.flatnonzero(fresh)
+            passed = flows_in.check_inbound_batch(np.ascontiguousarray(plain[pick[got_in]]).reshape(-1),
+                                                  np.arange(got_in.size, dtype=np.uint64) * length,
+                                                  np.full(got_in.size, length, np.uint32), t0 + 5 + k)
+            want[got_in] = np.where(passed != 0, lib.WG_OK, lib.WG_FILTERED)
+            wire, out = d(rows.reshape(-1)), torch.zeros(n * slot, dtype=torch.uint8, device="cuda:0")
+            res, olen, gp = torch.full((n,), 99, dtype=torch.uint8, device="cuda:0"), i32(), i32()
+            gc = torch.zeros(n, dtype=torch.int64, device="cuda:0")
+            torch.cuda.synchronize()
+            rxc.wg_decap_filter(lib.make_batch(wire, n * slot, n, lib.MEM_DEVICE, stride=slot, length=80),
+                                lib.make_batch(out, n * slot, n, lib.MEM_DEVICE, stride=slot), t0 + 5 + k, res, olen, gp, gc)
+            rxc.sync()
+            assert np.array_equal(gc.cpu().numpy().view(np.uint64), ctr[pick])
+            assert np.array_equal(res.cpu().numpy(), want)
+            assert len(np.unique(want)) >= 2
+            assert rxc.filter_flows() == flows_in.flows()

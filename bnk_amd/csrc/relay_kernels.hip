@@ -13,6 +13,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "../../include/bnkhip.h"
+#include "block_rows.hpp"
 #include "block_sort.hpp"
 #include "filter_lane.hpp"
 #include "kernels.hpp"
@@ -338,22 +339,88 @@ BNK_DEV void peer_rank_block(const RankArgs &a)
     }
 }
 
-template <bool SMALL>
-__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_kernel(RankArgs a)
+// The same without a sort (block_rows.hpp), for tables of fewer than ROW_DIGITS peers.
+static_assert(PEER_BLOCK_THREADS == ROW_THREADS && PEER_RANK_BLOCK_MAX == ROW_PACKETS, "one launch shape");
+BNK_DEV void peer_rank_rows(const RankArgs &a)
 {
-    SMALL ? peer_rank_small(a) : peer_rank_block(a);
+    __shared__ uint32_t count[ROW_WAVES][ROW_DIGITS];
+    __shared__ uint64_t base[ROW_DIGITS];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const uint32_t rows = (a.n + ROW_THREADS - 1u) / ROW_THREADS, none = ROW_DIGITS - 1u;
+    uint32_t *const mine = count[wave];
+    uint32_t key[ROWS_MOST];
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        const uint32_t i = row_place(rows, j);
+        key[j] = j < rows && i < a.n ? (a.peer ? a.peer[i] : 0u) : NO_PEER;
+    }
+    uint64_t was = 0;
+    if (t < a.n_keys) was = a.ctr_base[t];
+#pragma unroll
+    for (uint32_t k = 0; k < ROW_DIGITS / 64u; k++) mine[k * 64u + lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    uint32_t rank[ROWS_MOST]; // among the wave's packets of the peer
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        if (j >= rows) break; // (the same for every lane)
+        if (key[j] >= a.n_keys) {
+            if (row_place(rows, j) < a.n && !(a.no_peer_ok && key[j] == NO_PEER)) status_raise(a.status, STATUS_PEER_RANGE);
+            key[j] = none;
+        }
+        const unsigned long long same = row_same(key[j], ROW_BITS);
+        const uint32_t lower = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+        const uint32_t before = mine[key[j]];
+        rank[j] = before + lower;
+        // (LDS answers a wave's accesses in order: every lane has read)
+        if (lower == 0u) mine[key[j]] = before + (uint32_t)__popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    if (t < a.n_keys) { // (fewer than ROW_DIGITS)
+        uint32_t c[ROW_WAVES], upto = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < ROW_WAVES; w++) c[w] = count[w][t];
+#pragma unroll
+        for (uint32_t w = 0; w < ROW_WAVES; w++) {
+            count[w][t] = upto;
+            upto += c[w];
+        }
+        base[t] = was;
+        if (a.advance && upto != 0u) a.ctr_base[t] = ctr_add(was, upto, a.ctr_limit);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++)
+        if (j < rows && key[j] != none) a.ctr_out[row_place(rows, j)] = ctr_add(base[key[j]], mine[key[j]] + rank[j], a.ctr_limit);
 }
+
+// The form for a batch: a packet a thread, four, or rows.
+enum RankForm : uint32_t { RANK_SMALL, RANK_BLOCK, RANK_ROWS };
+static RankForm rank_form(uint32_t n, uint32_t n_keys)
+{
+    return n_keys < ROW_DIGITS ? RANK_ROWS : n <= PEER_RANK_SMALL_MAX ? RANK_SMALL : RANK_BLOCK;
+}
+template <uint32_t FORM>
+BNK_DEV void peer_rank(const RankArgs &a)
+{
+    FORM == RANK_ROWS ? peer_rank_rows(a) : FORM == RANK_SMALL ? peer_rank_small(a) : peer_rank_block(a);
+}
+
+template <uint32_t FORM>
+__global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_kernel(RankArgs a) { peer_rank<FORM>(a); }
 
 // NoteOutbound on the packets of such a batch as well, which has nothing to do with its counters: the
 // first workgroup ranks, the second does what a note launch does once, the others note.  In launches of
 // their own, one behind the other (4 us each, and 3 for the host to launch one), device-resident tunnel
 // passes of 256 packets took 31.7 us in a row against 29.1, of 3000 70.5 against 65.1; 128 packets in
 // pinned rings through the tunnel 67.5 against 63.7.
-template <bool SMALL>
+template <uint32_t FORM>
 __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_note_kernel(RankArgs a, FilterArgs note)
 {
     if (blockIdx.x == 0u) {
-        SMALL ? peer_rank_small(a) : peer_rank_block(a);
+        peer_rank<FORM>(a);
     } else if (blockIdx.x == 1u) {
         if (threadIdx.x == 0u) note_once(note);
     } else {
@@ -373,7 +440,8 @@ static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_ke
                                              uint32_t *status, hipStream_t s)
 {
     const RankArgs a{peer, n_keys, n, ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status};
-    hipLaunchKernelGGL(n <= PEER_RANK_SMALL_MAX ? peer_rank_kernel<true> : peer_rank_kernel<false>, dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, a);
+    void (*const kernels[])(RankArgs) = {peer_rank_kernel<RANK_SMALL>, peer_rank_kernel<RANK_BLOCK>, peer_rank_kernel<RANK_ROWS>};
+    hipLaunchKernelGGL(kernels[rank_form(n, n_keys)], dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, a);
     return hipGetLastError();
 }
 
@@ -396,8 +464,9 @@ hipError_t launch_peer_rank_small_note(const uint32_t *peer, uint32_t n_keys, ui
     FilterArgs f = note;
     const uint32_t blocks = (n + PEER_BLOCK_THREADS - 1u) / PEER_BLOCK_THREADS;
     f.record_blocks = f.record && f.record_after ? blocks : 0u;
-    hipLaunchKernelGGL(n <= PEER_RANK_SMALL_MAX ? peer_rank_note_kernel<true> : peer_rank_note_kernel<false>, dim3(blocks + 2u),
-                       dim3(PEER_BLOCK_THREADS), 0, s, a, f);
+    void (*const kernels[])(RankArgs, FilterArgs) = {peer_rank_note_kernel<RANK_SMALL>, peer_rank_note_kernel<RANK_BLOCK>,
+                                                     peer_rank_note_kernel<RANK_ROWS>};
+    hipLaunchKernelGGL(kernels[rank_form(n, n_keys)], dim3(blocks + 2u), dim3(PEER_BLOCK_THREADS), 0, s, a, f);
     return launch_flow_sweep(f, max_blocks, claimed_upper, s);
 }
 

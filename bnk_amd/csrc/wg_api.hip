@@ -846,18 +846,22 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
     const bool replay = ctx->wg_replay_on;
     WgReplayDev rpd{ctx->wg_replay, pe.n};
     WgReplayScratch rsc{};
+    if (replay) {
+        // the flag words and the first-occurrence table keep their resting state from pass
+        // to pass: set it when they are first allocated or grow
+        const void *had = ctx->wg_lastb.p;
+        HIPCHK(ctx, ctx->wg_lastb.reserve((size_t)(chunked ? hp.per : n) + 64));
+        if (ctx->wg_lastb.p != had) HIPCHK(ctx, hipMemsetAsync(ctx->wg_lastb.p, 0, 64, ctx->stream));
+        rsc.cls = ctx->wg_lastb.as<uint8_t>() + 64;
+        rsc.flags = ctx->wg_lastb.as<uint32_t>();
+    }
     if (replay && !wg_replay_one_block(n, pe.n)) {
         const uint32_t biggest = chunked ? hp.per : n;
         for (DevBuf *buf : {&ctx->r_keys, &ctx->r_idx, &ctx->r_skeys, &ctx->r_sidx})
             HIPCHK(ctx, buf->reserve((size_t)biggest * 4));
         for (DevBuf *buf : {&ctx->wg_sctr, &ctx->wg_sval, &ctx->wg_pmax}) HIPCHK(ctx, buf->reserve((size_t)biggest * 8));
-        // the flag words and the first-occurrence table keep their resting state from pass
-        // to pass: set it when they are first allocated or grow
-        const void *had = ctx->wg_lastb.p;
-        HIPCHK(ctx, ctx->wg_lastb.reserve((size_t)biggest + 64));
-        if (ctx->wg_lastb.p != had) HIPCHK(ctx, hipMemsetAsync(ctx->wg_lastb.p, 0, 64, ctx->stream));
         rsc.table_slots = wg_replay_table_slots(biggest);
-        had = ctx->wg_rtable.p;
+        const void *const had = ctx->wg_rtable.p;
         HIPCHK(ctx, ctx->wg_rtable.reserve((size_t)rsc.table_slots * 4));
         if (ctx->wg_rtable.p != had)
             HIPCHK(ctx, hipMemsetAsync(ctx->wg_rtable.p, 0xFF, ctx->wg_rtable.cap, ctx->stream));
@@ -870,8 +874,6 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
         rsc.sctr = ctx->wg_sctr.as<uint64_t>();
         rsc.sval = ctx->wg_sval.as<uint64_t>();
         rsc.pmax = ctx->wg_pmax.as<uint64_t>();
-        rsc.cls = ctx->wg_lastb.as<uint8_t>() + 64;
-        rsc.flags = ctx->wg_lastb.as<uint32_t>();
         rsc.table = ctx->wg_rtable.as<uint32_t>();
         rsc.tmp = ctx->r_tmp.p;
     }

@@ -51,7 +51,7 @@ struct WgReplayDev {
     uint32_t n_peers;
 };
 
-// Device scratch of one replay pass over n packets (not needed where wg_replay_one_block).
+// Device scratch of one replay pass over n packets (where wg_replay_one_block, cls alone).
 struct WgReplayScratch {
     uint32_t *keys, *idx, *skeys, *sidx;   // n words each
     uint64_t *sctr, *sval, *pmax;          // n each
@@ -73,7 +73,7 @@ struct ReplayMark {
     const uint64_t *sctr;
     const uint8_t *cls;
     uint64_t *state;
-    uint32_t *table, *flags;
+    uint32_t *table, *flags; // null where the pass has none
     uint32_t n, slots, parity;
 };
 constexpr uint32_t REPLAY_MARK_THREADS = 256;

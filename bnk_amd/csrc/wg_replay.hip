@@ -40,6 +40,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include "../../include/bnkhip.h"
+#include "block_rows.hpp"
 #include "block_sort.hpp"
 #include "kernels.hpp"
 #include "wg_dev.hpp"
@@ -97,6 +98,13 @@ __global__ __launch_bounds__(256) void replay_keys_packed_kernel(const uint8_t *
 // inside replay_classify_kernel, which needs the values).
 // ---------------------------------------------------------------------------
 constexpr uint32_t SEG_BLOCK = 1024;
+
+__device__ __forceinline__ uint64_t shfl64(uint64_t v, int lane)
+{
+    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)v, lane, 64);
+    const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(v >> 32), lane, 64);
+    return (uint64_t)hi << 32 | lo;
+}
 
 __device__ __forceinline__ uint64_t shfl_up64(uint64_t v, unsigned off)
 {
@@ -659,6 +667,172 @@ __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *re
     }
 }
 
+// The same in batch order, without a sort (block_rows.hpp), for tables of fewer than ROW_DIGITS peers; the
+// packets' bits go into their windows in a launch behind it (cls; see replay_mark).
+static_assert(WG_REPLAY_BLOCK_MAX == ROW_PACKETS, "one workgroup");
+__global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *result, uint32_t *out_len, const uint32_t *peer,
+                                                                  const uint64_t *counter, uint32_t n_peers, uint32_t n,
+                                                                  uint64_t *state, unsigned bits, uint8_t *cls_out)
+{
+    __shared__ union {
+        uint64_t most[ROW_WAVES][ROW_DIGITS]; // of a peer's counters so far, of the wave; then of the waves before
+        uint32_t table[BLOCK_TABLE];
+    } tmp;
+    __shared__ uint64_t last_was[ROW_DIGITS];
+    __shared__ uint64_t sc[ROW_PACKETS];
+    __shared__ uint8_t sk[ROW_PACKETS];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    const uint32_t rows = (n + ROW_THREADS - 1u) / ROW_THREADS, none = ROW_DIGITS - 1u;
+    uint32_t key[ROWS_MOST];
+    uint64_t c[ROWS_MOST];
+    {
+        uint8_t res[ROWS_MOST];
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            const uint32_t at = min(row_place(rows, j), n - 1u);
+            key[j] = peer[at];
+            res[j] = result[at];
+            c[j] = counter[at];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++)
+            if (j >= rows || row_place(rows, j) >= n || !replay_subject(res[j]) || key[j] >= n_peers) key[j] = none;
+    }
+    uint64_t was = 0;
+    if (t < n_peers) was = state[(size_t)t * WG_REPLAY_WORDS];
+    uint64_t *const mine = tmp.most[wave];
+#pragma unroll
+    for (uint32_t k = 0; k < ROW_DIGITS / 64u; k++) mine[k * 64u + lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    // The running maximum of the peer's counters ahead of each packet, among the wave's (a counter the
+    // filter turns away outright never moves last).
+    uint64_t before[ROWS_MOST];
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        before[j] = 0;
+        if (j >= rows) break; // (the same for every lane)
+        const uint64_t v = c[j] < WG_REJECT_AFTER_MESSAGES ? c[j] : 0;
+        const unsigned long long same = row_same(key[j], bits), lower = same & ((1ull << lane) - 1ull);
+        int from = lower ? 63 - __clzll((long long)lower) : -1; // the lane before this one with the key
+        uint64_t m = shfl64(v, from < 0 ? 0 : from);
+        if (from < 0) m = 0;
+        // (counters that rise from packet to packet: that lane's is the most of them)
+        if (__ballot(from >= 0 && v < m) != 0ull) {
+#pragma unroll
+            for (int step = 0; step < 6; step++) {
+                const uint64_t o = shfl64(m, from < 0 ? 0 : from);
+                const int further = __shfl(from, from < 0 ? 0 : from, 64);
+                if (from >= 0) {
+                    m = o > m ? o : m;
+                    from = further;
+                }
+            }
+        }
+        const uint64_t m0 = mine[key[j]];
+        before[j] = m0 > m ? m0 : m;
+        // (LDS answers a wave's accesses in order: every lane has read)
+        if ((same >> lane) == 1ull) mine[key[j]] = v > before[j] ? v : before[j];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint64_t upto = 0; // of peer t, over all
+    if (t < n_peers) { // (fewer than ROW_DIGITS)
+        uint64_t m[ROW_WAVES];
+#pragma unroll
+        for (uint32_t w = 0; w < ROW_WAVES; w++) m[w] = tmp.most[w][t];
+#pragma unroll
+        for (uint32_t w = 0; w < ROW_WAVES; w++) {
+            tmp.most[w][t] = upto;
+            upto = m[w] > upto ? m[w] : upto;
+        }
+        last_was[t] = was;
+    }
+    __syncthreads();
+    uint8_t cls[ROWS_MOST];
+    bool any_late = false;
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        cls[j] = RP_NONE;
+        if (key[j] == none) continue;
+        const uint64_t last0 = last_was[key[j]], ahead = mine[key[j]];
+        uint64_t last = last0 > ahead ? last0 : ahead;
+        if (before[j] > last) last = before[j];
+        if (reaches_bit_test(c[j], last)) cls[j] = c[j] > last ? RP_AHEAD : RP_LATE;
+        if (cls[j] == RP_LATE && c[j] <= last0 && seen_before(state + (size_t)key[j] * WG_REPLAY_WORDS, c[j])) cls[j] = RP_SEEN;
+        any_late |= cls[j] == RP_LATE;
+    }
+    bool repeat[ROWS_MOST];
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) repeat[j] = false;
+    // (the windows have been read as the batch found them behind this)
+    if (__syncthreads_or(any_late)) {
+        // The first packet that carries a late one's counter: the late ones' places in a table, then those
+        // that were ahead when they came (never after a late one of the same counter) where it is there.
+        constexpr uint32_t mask = BLOCK_TABLE - 1u;
+        for (uint32_t h = t; h < BLOCK_TABLE; h += ROW_THREADS) tmp.table[h] = HASH_EMPTY;
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            const uint32_t i = row_place(rows, j);
+            if (j < rows && i < n) {
+                sk[i] = (uint8_t)key[j];
+                sc[i] = c[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            if (cls[j] != RP_LATE) continue;
+            for (uint32_t h = table_home(key[j], c[j], mask);; h = (h + 1u) & mask) {
+                const uint32_t old = atomicCAS(&tmp.table[h], HASH_EMPTY, row_place(rows, j));
+                if (old == HASH_EMPTY) break;
+                if (sk[old] == key[j] && sc[old] == c[j]) {
+                    atomicMin(&tmp.table[h], row_place(rows, j));
+                    break;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            if (cls[j] != RP_AHEAD) continue;
+            for (uint32_t h = table_home(key[j], c[j], mask);; h = (h + 1u) & mask) {
+                const uint32_t at = tmp.table[h];
+                if (at == HASH_EMPTY) break; // (the table has twice as many slots as there are packets)
+                if (sk[at] == key[j] && sc[at] == c[j]) {
+                    atomicMin(&tmp.table[h], row_place(rows, j));
+                    break;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            if (cls[j] != RP_LATE) continue;
+            for (uint32_t h = table_home(key[j], c[j], mask);; h = (h + 1u) & mask) {
+                const uint32_t at = tmp.table[h];
+                if (at == HASH_EMPTY) break; // cannot happen: it was entered
+                if (sk[at] == key[j] && sc[at] == c[j]) {
+                    repeat[j] = at != row_place(rows, j);
+                    break;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        const uint32_t i = row_place(rows, j);
+        if (j >= rows || i >= n) continue;
+        cls_out[i] = cls[j];
+        if (key[j] != none && (cls[j] == RP_NONE || cls[j] == RP_SEEN || repeat[j])) {
+            result[i] = BNK_WG_REPLAY;
+            out_len[i] = 0;
+        }
+    }
+    if (t < n_peers && upto > was) advance_window(state + (size_t)t * WG_REPLAY_WORDS, upto);
+}
+
 __global__ __launch_bounds__(256) void replay_reset_kernel(uint64_t *state, const uint8_t *flags, uint32_t n_peers)
 {
     const uint32_t total = n_peers * WG_REPLAY_WORDS;
@@ -716,6 +890,14 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
     if (n <= 256u) {
         hipLaunchKernelGGL(replay_small_kernel<256>, dim3(1), dim3(256), 0, s, result, out_len, peer, counter,
                            rp.n_peers, n, rp.state, key_bits(rp.n_peers));
+        return hipGetLastError();
+    }
+    if (n <= WG_REPLAY_BLOCK_MAX && rp.n_peers < ROW_DIGITS) {
+        hipLaunchKernelGGL(replay_rows_kernel, dim3(1), dim3(ROW_THREADS), 0, s, result, out_len, peer, counter, rp.n_peers, n, rp.state,
+                           ROW_BITS, sc.cls);
+        const ReplayMark m{peer, counter, sc.cls, rp.state, nullptr, nullptr, n, 0u, 0u};
+        if (!rest) return launch_wg_replay_mark(m, s);
+        *rest = m;
         return hipGetLastError();
     }
     if (n <= WG_REPLAY_SMALL_MAX) {

@@ -77,7 +77,7 @@ __device__ __forceinline__ void mark_bits(uint64_t *state, uint32_t key, uint64_
 
 // Sets the bit of every packet that reached the bit test and still lies in the
 // window its peer ends the batch with.  Neighbours in sorted order mostly
-// share their peer and their block of 64 counters.  By workgroup `b` of `blocks`, each of
+// share their peer and their block of 64 counters (small batches come in batch order).  By workgroup `b` of `blocks`, each of
 // REPLAY_MARK_THREADS.
 //
 // The same launch leaves the first-occurrence table empty for the next pass
@@ -86,9 +86,11 @@ __device__ __forceinline__ void mark_bits(uint64_t *state, uint32_t key, uint64_
 __device__ __forceinline__ void replay_mark(const ReplayMark &m, uint32_t b, uint32_t blocks)
 {
     const uint32_t p = b * REPLAY_MARK_THREADS + threadIdx.x;
-    if (p == 0u) m.flags[m.parity ^ 1u] = 0u;
-    if (m.flags[m.parity] != 0u)
-        for (uint32_t i = p; i < m.slots; i += blocks * REPLAY_MARK_THREADS) m.table[i] = 0xFFFFFFFFu;
+    if (m.flags) {
+        if (p == 0u) m.flags[m.parity ^ 1u] = 0u;
+        if (m.flags[m.parity] != 0u)
+            for (uint32_t i = p; i < m.slots; i += blocks * REPLAY_MARK_THREADS) m.table[i] = 0xFFFFFFFFu;
+    }
     uint32_t key = 0xFFFFFFFFu;
     uint64_t block = ~0ull, bit = 0;
     if (p < m.n && m.cls[p] != RP_NONE) {

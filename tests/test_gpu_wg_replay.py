@@ -636,3 +636,10 @@ def test_tunnel_batches_whose_tiles_add_up_the_rows_before_theirs(n_peers, n):
             assert np.array_equal(res.cpu().numpy(), want)
             assert len(np.unique(want)) >= 2
             assert rxc.filter_flows() == flows_in.flows()
+
+
+@pytest.mark.parametrize("n_peers,n", [(1, 257), (255, 300), (3, 1023), (254, 1024), (256, 700), (40, 2049), (255, 4096)])
+def test_counters_and_windows_by_rows_of_a_workgroup(n_peers, n):
+    """One row of 64 packets a wave and as many as four, the last ones part full, as few peers as one
+    and as many as fit, and one more (which are sorted): the checks are those of the test above."""
+    test_counters_and_windows_of_one_workgroup_over_the_peers_digits(n_peers, n)

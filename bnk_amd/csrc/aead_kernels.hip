@@ -1599,8 +1599,9 @@ struct SpreadPacket {
 };
 
 // Packet w of the launch, up to its tag and what is said about it; false: there is nothing to store.
-// SMALL: of a launch that does the whole batch (wg_small.hpp), which leaves a record instead.
-template <bool OPEN, bool WG, bool SMALL>
+// SMALL: of a launch that does the whole batch (wg_small.hpp), which leaves a record instead; MANY: of more
+// than WG_SMALL_MAX packets.
+template <bool OPEN, bool WG, bool SMALL, bool MANY = false>
 BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, uint8_t *stage, uint32_t lane, uint32_t w, SpreadPacket &p)
 {
     // everything up to the per-lane work below is uniform across the wave
@@ -1705,7 +1706,7 @@ BNK_DEV bool spread_packet(const AeadArgs &a, const TunnelSmall &t, const Filter
         if (WG) wg_remote = a.wg.remote_index[known];
         if (WG && SMALL) {
             ctr_small = t.send_ctr[known];
-            rank = send_rank(a.peer, a.n, i, pr, lane);
+            rank = send_rank<MANY>(a.peer, a.n, i, pr, lane);
         }
     } else {
         wg_head = ld16(len >= 32u && !outside ? src : safe);
@@ -2044,10 +2045,10 @@ __global__ __launch_bounds__(256, 5) void aead_spread_kernel(AeadArgs a)
 // at work, whatever is in them.  128 packets in pinned rings out and back 63.7 -> 48.9 us (kernels 13.5
 // and 17, in place of 4.5 + 12 and 12 + 6 + 6.6), device-resident passes of 256 with three streams at
 // work 21.0 -> 12.5.
-template <bool OPEN>
+template <bool OPEN, bool MANY>
 __global__ __launch_bounds__(256, 4) void tunnel_small_kernel(AeadArgs a, TunnelSmall t, FilterArgs f)
 {
-    static_assert(256u == WG_SMALL_MAX && 64u * WAVES_PER_BLOCK == WG_SMALL_MAX, "a thread per packet at the end");
+    static_assert(256u == WG_SMALL_MAX && 64u * WAVES_PER_BLOCK == WG_SMALL_MAX, "decap_finish: a thread per packet");
     __shared__ union {
         __attribute__((aligned(16))) uint8_t tile[WAVES_PER_BLOCK][64 * LDS_ROW];
         SmallWindows windows;
@@ -2063,40 +2064,55 @@ __global__ __launch_bounds__(256, 4) void tunnel_small_kernel(AeadArgs a, Tunnel
     uint8_t *const stage = sh.tile[threadIdx.x >> 6];
     SpreadPacket p;
     bool out = false;
-    if (w < a.n) out = spread_packet<OPEN, true, true>(a, t, f, stage, lane, w, p);
+    if (w < a.n) out = spread_packet<OPEN, true, true, MANY>(a, t, f, stage, lane, w, p);
     // (the records are where others see them before the workgroup is counted; the packet's bytes go
     // out meanwhile)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0u) {
-        const bool mine = __hip_atomic_fetch_add(t.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == blocks;
-        if (mine) __hip_atomic_store(t.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = mine;
-    }
+    if (threadIdx.x == 0u) last = arrive(t.arrived, blockIdx.x, blocks);
     if (out) spread_store<OPEN>(p, stage, lane, reinterpret_cast<const uint8_t *>(a.keys));
     __syncthreads();
     if (!last) return;
     if (OPEN) decap_finish(t, a, f, sh.windows);
-    else encap_finish(t, f, a.n, a.wg.n_peers);
+    else encap_finish<MANY>(t, f, a.n, a.wg.n_peers);
+}
+
+// The first launch of a decapsulating call of more packets than that: the records alone.
+__global__ __launch_bounds__(256, 4) void tunnel_open_waves_kernel(AeadArgs a, TunnelSmall t, FilterArgs f)
+{
+    __shared__ __attribute__((aligned(16))) uint8_t tile_all[WAVES_PER_BLOCK][64 * LDS_ROW];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = blockIdx.x * WAVES_PER_BLOCK + (threadIdx.x >> 6);
+    if (w >= a.n) return;
+    uint8_t *const stage = tile_all[threadIdx.x >> 6];
+    SpreadPacket p;
+    if (spread_packet<true, true, true, true>(a, t, f, stage, lane, w, p))
+        spread_store<true>(p, stage, lane, reinterpret_cast<const uint8_t *>(a.keys));
 }
 
 hipError_t launch_tunnel_seal_small(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, uint32_t max_blocks,
                                     uint64_t claimed_upper, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    if (a.n > WG_SMALL_MAX || a.first != 0u || a.wg.mode != WG_FUSE_ENCAP || a.in_skip != 0u || (t.filter && f.n != a.n)) return hipErrorInvalidValue;
+    if (a.n > WG_WAVES_MAX || a.first != 0u || a.wg.mode != WG_FUSE_ENCAP || a.in_skip != 0u || (t.filter && f.n != a.n)) return hipErrorInvalidValue;
     FilterArgs note = f;
     note.record_blocks = f.record && f.record_after ? 1u : 0u; // (the last workgroup leaves the record)
     const uint32_t blocks = (a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK;
-    hipLaunchKernelGGL(tunnel_small_kernel<false>, dim3(blocks + (t.filter ? 1u : 0u)), dim3(256), 0, s, a, t, note);
+    hipLaunchKernelGGL((a.n > WG_SMALL_MAX ? tunnel_small_kernel<false, true> : tunnel_small_kernel<false, false>), dim3(blocks + (t.filter ? 1u : 0u)), dim3(256), 0, s, a, t, note);
     return t.filter ? launch_flow_sweep(note, max_blocks, claimed_upper, s) : hipGetLastError();
 }
 
 hipError_t launch_tunnel_open_small(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    if (a.n > WG_SMALL_MAX || a.first != 0u || a.wg.mode != WG_FUSE_DECAP || a.in_skip != 0u) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(tunnel_small_kernel<true>, dim3((a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK), dim3(256), 0, s, a, t, f);
+    if (a.n > WG_WAVES_MAX || (a.n > WG_SMALL_MAX && a.wg.n_peers > WG_WAVES_PEERS) || a.first != 0u || a.wg.mode != WG_FUSE_DECAP || a.in_skip != 0u)
+        return hipErrorInvalidValue;
+    const dim3 grid((a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK);
+    if (a.n > WG_SMALL_MAX) {
+        hipLaunchKernelGGL(tunnel_open_waves_kernel, grid, dim3(256), 0, s, a, t, f);
+        return launch_tunnel_open_rest(a, t, f, s);
+    }
+    hipLaunchKernelGGL((tunnel_small_kernel<true, false>), grid, dim3(256), 0, s, a, t, f);
     return hipGetLastError();
 }
 

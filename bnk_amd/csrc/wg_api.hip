@@ -36,7 +36,7 @@ TunnelSmall small_view(bnk_ctx *ctx, bool filter)
 {
     TunnelSmall t{};
     t.arrived = ctx->wg_small.as<uint32_t>();
-    t.records = t.arrived + 16;
+    t.records = t.arrived + WG_ARRIVE_WORDS;
     t.send_ctr = ctx->wg_send_ctr.as<uint64_t>();
     t.windows = ctx->wg_replay_on ? ctx->wg_replay : nullptr;
     t.filter = filter;
@@ -491,8 +491,9 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         return se;
     };
 
-    // A small batch in one launch: counters, NoteOutbound and the packets.
-    const bool small = n <= WG_SMALL_MAX && !chunked && !ctx->wg_unfused && aead_runs_spread(whole_slots(0, n));
+    // A small batch in one launch: counters, NoteOutbound and the packets.  (Every wave goes through the
+    // whole peer array, which of a batch in a ring lies in the host's staging.)
+    const bool small = n <= (ring_out ? WG_SMALL_MAX : WG_WAVES_MAX) && !chunked && !ctx->wg_unfused && aead_runs_spread(whole_slots(0, n));
     // counters in batch order per peer, advancing the peers' send counters:
     // needs the peer array only, so it runs ahead of the packet bytes
     if (small) {
@@ -955,8 +956,8 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
                 op.wg.out_len = d_out_len;
                 op.wg.peer_out = d_peer;
                 op.wg.counter_out = d_counter;
-                if (n <= WG_SMALL_MAX && !chunked && !ctx->wg_unfused && (replay || check)) {
-                    // a small batch in one launch: the windows and CheckInbound as well
+                if (n <= (pe.n <= WG_WAVES_PEERS ? WG_WAVES_MAX : WG_SMALL_MAX) && !chunked && !ctx->wg_unfused && (replay || check)) {
+                    // a small batch in one launch, or two: the windows and CheckInbound as well
                     HIPCHK(ctx, launch_tunnel_open_small(op, small_view(ctx, check), check ? check_args(lo, hi) : FilterArgs{}, ctx->stream));
                     return BNK_OK;
                 }

@@ -44,6 +44,7 @@
 #include "block_sort.hpp"
 #include "kernels.hpp"
 #include "wg_dev.hpp"
+#include "wg_small_dev.hpp"
 #include "wg_window.hpp"
 
 namespace bnk {
@@ -670,9 +671,11 @@ __global__ __launch_bounds__(BLOCK_THREADS) void replay_block_kernel(uint8_t *re
 // The same in batch order, without a sort (block_rows.hpp), for tables of fewer than ROW_DIGITS peers; the
 // packets' bits go into their windows in a launch behind it (cls; see replay_mark).
 static_assert(WG_REPLAY_BLOCK_MAX == ROW_PACKETS, "one workgroup");
-__global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *result, uint32_t *out_len, const uint32_t *peer,
-                                                                  const uint64_t *counter, uint32_t n_peers, uint32_t n,
-                                                                  uint64_t *state, unsigned bits, uint8_t *cls_out)
+// key: the packets' peers, or 255; c: their counters.  What the window says of each (RP_LATE: a repeat
+// that the batch itself holds is RP_SEEN by then), and the windows moved, but for the batch's bits;
+// last: what the window of thread t's peer ends with.
+__device__ __forceinline__ void replay_rows(const uint32_t (&key)[ROWS_MOST], const uint64_t (&c)[ROWS_MOST], uint32_t n_peers,
+                                            uint32_t n, uint64_t *state, uint8_t (&cls)[ROWS_MOST], uint64_t &last_out)
 {
     __shared__ union {
         uint64_t most[ROW_WAVES][ROW_DIGITS]; // of a peer's counters so far, of the wave; then of the waves before
@@ -683,21 +686,6 @@ __global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *resul
     __shared__ uint8_t sk[ROW_PACKETS];
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     const uint32_t rows = (n + ROW_THREADS - 1u) / ROW_THREADS, none = ROW_DIGITS - 1u;
-    uint32_t key[ROWS_MOST];
-    uint64_t c[ROWS_MOST];
-    {
-        uint8_t res[ROWS_MOST];
-#pragma unroll
-        for (uint32_t j = 0; j < ROWS_MOST; j++) {
-            const uint32_t at = min(row_place(rows, j), n - 1u);
-            key[j] = peer[at];
-            res[j] = result[at];
-            c[j] = counter[at];
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < ROWS_MOST; j++)
-            if (j >= rows || row_place(rows, j) >= n || !replay_subject(res[j]) || key[j] >= n_peers) key[j] = none;
-    }
     uint64_t was = 0;
     if (t < n_peers) was = state[(size_t)t * WG_REPLAY_WORDS];
     uint64_t *const mine = tmp.most[wave];
@@ -713,7 +701,7 @@ __global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *resul
         before[j] = 0;
         if (j >= rows) break; // (the same for every lane)
         const uint64_t v = c[j] < WG_REJECT_AFTER_MESSAGES ? c[j] : 0;
-        const unsigned long long same = row_same(key[j], bits), lower = same & ((1ull << lane) - 1ull);
+        const unsigned long long same = row_same(key[j], ROW_BITS), lower = same & ((1ull << lane) - 1ull);
         int from = lower ? 63 - __clzll((long long)lower) : -1; // the lane before this one with the key
         uint64_t m = shfl64(v, from < 0 ? 0 : from);
         if (from < 0) m = 0;
@@ -750,7 +738,6 @@ __global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *resul
         last_was[t] = was;
     }
     __syncthreads();
-    uint8_t cls[ROWS_MOST];
     bool any_late = false;
 #pragma unroll
     for (uint32_t j = 0; j < ROWS_MOST; j++) {
@@ -763,9 +750,6 @@ __global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *resul
         if (cls[j] == RP_LATE && c[j] <= last0 && seen_before(state + (size_t)key[j] * WG_REPLAY_WORDS, c[j])) cls[j] = RP_SEEN;
         any_late |= cls[j] == RP_LATE;
     }
-    bool repeat[ROWS_MOST];
-#pragma unroll
-    for (uint32_t j = 0; j < ROWS_MOST; j++) repeat[j] = false;
     // (the windows have been read as the batch found them behind this)
     if (__syncthreads_or(any_late)) {
         // The first packet that carries a late one's counter: the late ones' places in a table, then those
@@ -814,23 +798,115 @@ __global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *resul
                 const uint32_t at = tmp.table[h];
                 if (at == HASH_EMPTY) break; // cannot happen: it was entered
                 if (sk[at] == key[j] && sc[at] == c[j]) {
-                    repeat[j] = at != row_place(rows, j);
+                    if (at != row_place(rows, j)) cls[j] = RP_SEEN;
                     break;
                 }
             }
         }
     }
+    last_out = upto > was ? upto : was;
+    if (t < n_peers && upto > was) advance_window(state + (size_t)t * WG_REPLAY_WORDS, upto);
+}
+
+__global__ __launch_bounds__(ROW_THREADS) void replay_rows_kernel(uint8_t *result, uint32_t *out_len, const uint32_t *peer,
+                                                                  const uint64_t *counter, uint32_t n_peers, uint32_t n,
+                                                                  uint64_t *state, uint8_t *cls_out)
+{
+    const uint32_t rows = (n + ROW_THREADS - 1u) / ROW_THREADS, none = ROW_DIGITS - 1u;
+    uint32_t key[ROWS_MOST];
+    uint64_t c[ROWS_MOST];
+    {
+        uint8_t res[ROWS_MOST];
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            const uint32_t at = min(row_place(rows, j), n - 1u);
+            key[j] = peer[at];
+            res[j] = result[at];
+            c[j] = counter[at];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++)
+            if (j >= rows || row_place(rows, j) >= n || !replay_subject(res[j]) || key[j] >= n_peers) key[j] = none;
+    }
+    uint8_t cls[ROWS_MOST];
+    uint64_t last;
+    replay_rows(key, c, n_peers, n, state, cls, last);
 #pragma unroll
     for (uint32_t j = 0; j < ROWS_MOST; j++) {
         const uint32_t i = row_place(rows, j);
         if (j >= rows || i >= n) continue;
         cls_out[i] = cls[j];
-        if (key[j] != none && (cls[j] == RP_NONE || cls[j] == RP_SEEN || repeat[j])) {
+        if (key[j] != none && (cls[j] == RP_NONE || cls[j] == RP_SEEN)) {
             result[i] = BNK_WG_REPLAY;
             out_len[i] = 0;
         }
     }
-    if (t < n_peers && upto > was) advance_window(state + (size_t)t * WG_REPLAY_WORDS, upto);
+}
+
+// What is left of a decapsulating call whose packets' waves have left records (TunnelSmall): the windows,
+// what the filter does with the packets that are delivered, and the results.  With the counters of an
+// encapsulating call counted by its packets' waves, a pass makes three launches instead of five.
+__global__ __launch_bounds__(ROW_THREADS) void tunnel_rest_kernel(AeadArgs a, TunnelSmall t, FilterArgs f)
+{
+    __shared__ uint64_t last_is[ROW_DIGITS];
+    const uint32_t n = a.n, lane = threadIdx.x & 63u;
+    const uint32_t rows = (n + ROW_THREADS - 1u) / ROW_THREADS, none = ROW_DIGITS - 1u;
+    uint32_t peer[ROWS_MOST], out_len[ROWS_MOST], res[ROWS_MOST], action[ROWS_MOST], proto[ROWS_MOST], key[ROWS_MOST];
+    uint64_t c[ROWS_MOST];
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        const uint4 *const r = reinterpret_cast<const uint4 *>(t.records + (size_t)WG_SMALL_RECORD * min(row_place(rows, j), n - 1u));
+        const uint4 u = r[0], v = r[1];
+        peer[j] = u.x;
+        out_len[j] = u.y;
+        res[j] = u.z;
+        action[j] = v.x;
+        proto[j] = v.y;
+        c[j] = (uint64_t)v.w << 32 | v.z;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        const bool there = j < rows && row_place(rows, j) < n;
+        key[j] = there && replay_subject((uint8_t)res[j]) && peer[j] < a.wg.n_peers ? peer[j] : none;
+    }
+    if (t.windows) {
+        uint8_t cls[ROWS_MOST];
+        uint64_t last;
+        replay_rows(key, c, a.wg.n_peers, n, t.windows, cls, last);
+        if (threadIdx.x < a.wg.n_peers) last_is[threadIdx.x] = last;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup"); // (see replay_small_kernel)
+        __syncthreads(); // the cleared blocks are in place before bits go in
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            if (j >= rows) break; // (the same for every lane)
+            if (key[j] != none && (cls[j] == RP_NONE || cls[j] == RP_SEEN)) {
+                res[j] = BNK_WG_REPLAY;
+                out_len[j] = 0;
+            }
+            const bool set = cls[j] != RP_NONE && (last_is[key[j]] >> 6) - (c[j] >> 6) < WG_REPLAY_BLOCKS;
+            mark_bits(t.windows, set ? key[j] : NO_PEER, set ? c[j] >> 6 : ~0ull, set ? 1ull << (c[j] & 63u) : 0ull);
+        }
+    }
+    uint32_t votes = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < ROWS_MOST; j++) {
+        if (j >= rows) break; // (the same for every lane)
+        const uint32_t i = row_place(rows, j);
+        const bool there = i < n;
+        if (t.filter && there && res[j] == BNK_WG_OK) check_apply(f, action[j], proto[j], res[j]);
+        if (there) {
+            a.wg.result[i] = (uint8_t)res[j];
+            a.wg.out_len[i] = out_len[j];
+            a.wg.peer_out[i] = peer[j];
+            a.wg.counter_out[i] = c[j];
+        }
+        if (f.wg_tally) tally_vote(res[j], there, lane, votes);
+    }
+    if (t.filter && threadIdx.x == ROW_THREADS - 1u) check_once(f);
+    if (f.wg_tally && lane < 16u && votes != 0u && decap_slot(lane) != TALLY_NONE) {
+        tally_bump(f.wg_tally, decap_slot(lane), votes);
+        if (lane == BNK_WG_OK) tally_bump(f.wg_tally, TALLY_ALLOWED, votes);
+    }
 }
 
 __global__ __launch_bounds__(256) void replay_reset_kernel(uint64_t *state, const uint8_t *flags, uint32_t n_peers)
@@ -894,7 +970,7 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
     }
     if (n <= WG_REPLAY_BLOCK_MAX && rp.n_peers < ROW_DIGITS) {
         hipLaunchKernelGGL(replay_rows_kernel, dim3(1), dim3(ROW_THREADS), 0, s, result, out_len, peer, counter, rp.n_peers, n, rp.state,
-                           ROW_BITS, sc.cls);
+                           sc.cls);
         const ReplayMark m{peer, counter, sc.cls, rp.state, nullptr, nullptr, n, 0u, 0u};
         if (!rest) return launch_wg_replay_mark(m, s);
         *rest = m;
@@ -952,6 +1028,13 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
     const ReplayMark m{sc.skeys, sc.sctr, sc.cls, rp.state, sc.table, sc.flags, n, sc.table_slots, sc.parity};
     if (!rest) return launch_wg_replay_mark(m, s);
     *rest = m;
+    return hipGetLastError();
+}
+
+hipError_t launch_tunnel_open_rest(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, hipStream_t s)
+{
+    static_assert(WG_WAVES_MAX <= ROW_PACKETS && WG_WAVES_PEERS == ROW_DIGITS - 1u, "one workgroup");
+    hipLaunchKernelGGL(tunnel_rest_kernel, dim3(1), dim3(ROW_THREADS), 0, s, a, t, f);
     return hipGetLastError();
 }
 

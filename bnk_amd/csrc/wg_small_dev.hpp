@@ -15,26 +15,50 @@ namespace bnk {
 BNK_DEV void record_put(uint32_t *at, uint32_t v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 BNK_DEV uint32_t record_get(const uint32_t *at) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+// One thread of workgroup `block` of `blocks`, all of whose records are out: is it the last?
+BNK_DEV bool arrive_one(uint32_t *at, uint32_t of)
+{
+    const bool last = __hip_atomic_fetch_add(at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == of;
+    if (last) __hip_atomic_store(at, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return last;
+}
+BNK_DEV bool arrive(uint32_t *arrived, uint32_t block, uint32_t blocks)
+{
+    if (blocks <= WG_ARRIVE_GROUP) return arrive_one(arrived, blocks);
+    const uint32_t group = block / WG_ARRIVE_GROUP, groups = (blocks + WG_ARRIVE_GROUP - 1u) / WG_ARRIVE_GROUP;
+    return arrive_one(arrived + (1u + group) * WG_ARRIVE_LINE, min(WG_ARRIVE_GROUP, blocks - group * WG_ARRIVE_GROUP)) &&
+           arrive_one(arrived, groups);
+}
+
 // How many packets ahead of packet i have its peer, and whether one behind it has.
 struct SendRank {
     uint32_t ahead;
     bool later;
 };
-BNK_DEV SendRank send_rank(const uint32_t *peer, uint32_t n, uint32_t i, uint32_t mine, uint32_t lane)
+// `LOADS` a lane, all in flight together, of packets `from` on.
+template <uint32_t LOADS>
+BNK_DEV void send_rank_part(const uint32_t *peer, uint32_t n, uint32_t from, uint32_t i, uint32_t mine, uint32_t lane, SendRank &r)
 {
-    static_assert(WG_SMALL_MAX == 256u, "four loads a lane, all in flight together");
-    SendRank r{0u, false};
-    if (!peer) return SendRank{i, i + 1u < n};
-    uint32_t p[4];
+    uint32_t p[LOADS];
 #pragma unroll
-    for (uint32_t j = 0; j < 4; j++) p[j] = peer[min(64u * j + lane, n - 1u)];
+    for (uint32_t j = 0; j < LOADS; j++) p[j] = peer[min(from + 64u * j + lane, n - 1u)];
 #pragma unroll
-    for (uint32_t j = 0; j < 4; j++) {
-        const uint32_t u = 64u * j + lane;
+    for (uint32_t j = 0; j < LOADS; j++) {
+        const uint32_t u = from + 64u * j + lane;
         const bool same = u < n && p[j] == mine;
         r.ahead += (uint32_t)__popcll(__ballot(same && u < i));
         r.later |= __ballot(same && u > i) != 0ull;
     }
+}
+// MANY: there may be more than WG_SMALL_MAX.
+template <bool MANY>
+BNK_DEV SendRank send_rank(const uint32_t *peer, uint32_t n, uint32_t i, uint32_t mine, uint32_t lane)
+{
+    SendRank r{0u, false};
+    if (!peer) return SendRank{i, i + 1u < n};
+    static_assert(WG_SMALL_MAX == 256u, "one part");
+    if (!MANY) send_rank_part<4>(peer, n, 0u, i, mine, lane, r);
+    else for (uint32_t from = 0; from < n; from += 1024u) send_rank_part<16>(peer, n, from, i, mine, lane, r);
     return r;
 }
 
@@ -212,21 +236,58 @@ BNK_DEV void decap_record(uint32_t *records, uint32_t i, uint32_t lane, uint32_t
 // And an encapsulated one's: its peer's next counter where it is the peer's last of the batch.
 BNK_DEV void encap_record(uint32_t *records, uint32_t i, uint32_t lane, uint32_t peer, uint64_t next)
 {
-    const uint32_t v = lane == 0u ? peer : lane == 1u ? (uint32_t)next : (uint32_t)(next >> 32);
-    if (lane < 3u) record_put(records + WG_SMALL_RECORD * i + lane, v);
+    const uint32_t v = lane == 0u ? peer : lane == 2u ? (uint32_t)next : (uint32_t)(next >> 32);
+    if (lane < 4u) record_put(records + WG_SMALL_RECORD * i + lane, v);
 }
 
+// The peers' counters moved, by WG_SMALL_MAX threads, PER packets each, whose records are on their way
+// together: they come from beyond L2, and nothing else is left of the launch.
+template <uint32_t PER>
+BNK_DEV void counters_move(const TunnelSmall &t, uint32_t n, uint32_t n_peers)
+{
+    uint32_t peer[PER];
+    uint64_t next[PER];
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++) {
+        const uint32_t *const r = t.records + WG_SMALL_RECORD * min(threadIdx.x + WG_SMALL_MAX * j, n - 1u);
+        peer[j] = record_get(r);
+        next[j] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(r + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < PER; j++)
+        if (threadIdx.x + WG_SMALL_MAX * j < n && peer[j] < n_peers) t.send_ctr[peer[j]] = next[j];
+}
+
+template <bool MANY>
 BNK_DEV void encap_finish(const TunnelSmall &t, const FilterArgs &f, uint32_t n, uint32_t n_peers)
 {
-    const uint32_t i = threadIdx.x;
-    if (i >= n) return;
-    const uint32_t *r = t.records + WG_SMALL_RECORD * i;
-    const uint32_t peer = record_get(r), lo = record_get(r + 1), hi = record_get(r + 2);
-    if (peer < n_peers) t.send_ctr[peer] = (uint64_t)hi << 32 | lo;
+    counters_move<MANY ? WG_WAVES_MAX / WG_SMALL_MAX : 1u>(t, n, n_peers);
     // (FilterArgs::record_after: claims are atomics whose answers their waves have waited for)
-    if (t.filter && i == 0u && f.record && f.record_after)
+    if (t.filter && threadIdx.x == 0u && f.record && f.record_after)
         __hip_atomic_store(f.record, (uint64_t)f.record_seq << 32 | atomicAdd(&f.flows.counters[FLOW_CLAIMED], 0u), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// What the filter does with a packet that is delivered (action: of check_end), by a lane.
+BNK_DEV void check_apply(const FilterArgs &f, uint32_t action, uint32_t proto, uint32_t &res)
+{
+    const uint32_t what = action & 3u;
+    FlowSlotMem *const slot = f.flows.slots + (action >> 2);
+    if (action == CHECK_DENY || what == CHECK_DELETE) res = BNK_WG_FILTERED;
+    if (what == CHECK_REFRESH) slot->exp = f.now + flow_ttl_ns(proto); // (see check_main)
+    if (what == CHECK_DELETE) {
+        const int64_t prev = (int64_t)atomicExch(reinterpret_cast<unsigned long long *>(&slot->exp), (unsigned long long)FLOW_TOMB);
+        if (prev != FLOW_TOMB) atomicSub(&f.flows.counters[FLOW_LIVE], 1u);
+    }
+}
+// And once a batch, by one lane: see check_main.
+BNK_DEV void check_once(const FilterArgs &f)
+{
+    const int64_t from = f.now + FLOW_TTL_LEAST;
+    for (const uint32_t w : {FLOW_MIN_EXP, FLOW_NEXT_EXP}) {
+        int64_t *least = reinterpret_cast<int64_t *>(f.flows.counters + w);
+        if (from < *least) (void)__hip_atomic_fetch_min(least, from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 struct SmallWindows {
@@ -327,29 +388,14 @@ BNK_DEV void decap_finish(const TunnelSmall &t, const AeadArgs &a, const FilterA
                 atomicOr(reinterpret_cast<unsigned long long *>(&st[1u + ((c >> 6) & (WG_REPLAY_BLOCKS - 1u))]), 1ull << (c & 63u));
         }
     }
-    if (t.filter && there && res == BNK_WG_OK) {
-        const uint32_t what = action & 3u;
-        FlowSlotMem *const slot = f.flows.slots + (action >> 2);
-        if (action == CHECK_DENY || what == CHECK_DELETE) res = BNK_WG_FILTERED;
-        if (what == CHECK_REFRESH) slot->exp = f.now + flow_ttl_ns(proto); // (see filter_check_kernel)
-        if (what == CHECK_DELETE) {
-            const int64_t prev = (int64_t)atomicExch(reinterpret_cast<unsigned long long *>(&slot->exp), (unsigned long long)FLOW_TOMB);
-            if (prev != FLOW_TOMB) atomicSub(&f.flows.counters[FLOW_LIVE], 1u);
-        }
-    }
+    if (t.filter && there && res == BNK_WG_OK) check_apply(f, action, proto, res);
     if (there) {
         a.wg.result[i] = (uint8_t)res;
         a.wg.out_len[i] = out_len;
         a.wg.peer_out[i] = peer;
         a.wg.counter_out[i] = c;
     }
-    if (t.filter && i == 255u) { // (see filter_check_kernel)
-        const int64_t from = f.now + FLOW_TTL_LEAST;
-        for (const uint32_t w : {FLOW_MIN_EXP, FLOW_NEXT_EXP}) {
-            int64_t *least = reinterpret_cast<int64_t *>(f.flows.counters + w);
-            if (from < *least) (void)__hip_atomic_fetch_min(least, from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    if (t.filter && i == 255u) check_once(f);
     if (f.wg_tally) {
         uint32_t votes = 0;
         tally_vote(res, there, lane, votes);

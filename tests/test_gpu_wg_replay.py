@@ -643,3 +643,11 @@ def test_counters_and_windows_by_rows_of_a_workgroup(n_peers, n):
     """One row of 64 packets a wave and as many as four, the last ones part full, as few peers as one
     and as many as fit, and one more (which are sorted): the checks are those of the test above."""
     test_counters_and_windows_of_one_workgroup_over_the_peers_digits(n_peers, n)
+
+
+@pytest.mark.parametrize("n_peers,n", [(1, 257), (255, 1025), (256, 1024), (40, 2048), (40, 2049), (255, 2047), (1024, 2048)])
+def test_tunnel_batches_of_a_wave_per_packet_in_three_launches(n_peers, n):
+    """The fewest and the most packets that are encapsulated in one launch and decapsulated in two, one
+    more, as many peers as the second of those takes and more: the checks are those of the test of
+    larger batches above."""
+    test_tunnel_batches_whose_tiles_add_up_the_rows_before_theirs(n_peers, n)

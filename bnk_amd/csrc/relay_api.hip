@@ -231,6 +231,9 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
     }
     FilterState *f = ctx->filter;
     uint8_t *d_pass = ctx->r_pass.as<uint8_t>();
+    // (a host batch's verdicts are counted where they arrive)
+    unsigned long long *const tally =
+        !host && ctx->tally_on.load(std::memory_order_relaxed) ? reinterpret_cast<unsigned long long *>(ctx->d_tally) : nullptr;
 
     // packets [lo, hi): open -> filter -> verdicts and counters -> re-seal
     auto run = [&](uint32_t lo, uint32_t hi, bool advance) -> int {
@@ -283,7 +286,7 @@ static int relay_impl(bnk_ctx *ctx, const bnk_batch *in, const uint32_t *peer_ou
                                         ctx->r_keys.as<uint32_t>(), ctx->r_idx.as<uint32_t>(),
                                         ctx->r_skeys.as<uint32_t>(), ctx->r_sidx.as<uint32_t>(),
                                         ctx->r_tmp.p, tmp_bytes, d_verdict + lo, d_ctr_out + lo, ctx->d_status,
-                                        advance, ctx->stream));
+                                        tally, advance, ctx->stream));
 
         // ---- 4. re-seal the survivors under the outbound keys ----
         AeadArgs se{};
@@ -362,7 +365,8 @@ extern "C" int bnk_relay_fused_batch(bnk_ctx *ctx, const bnk_batch *in, const ui
     if (g.rc) return g.rc;
     const int rc = relay_impl(ctx, in, peer_out, ctr_base_out, n_peers_out, now_ns, out, verdict, ctr_out);
     // (every packet relayed was opened and re-sealed on the way)
-    if (rc == BNK_OK) return tally_results(ctx, TALLY_RELAY, verdict, in->n, in->mem);
+    // (a device-resident batch has counted its own)
+    if (rc == BNK_OK && in->mem == BNK_MEM_HOST) return tally_results(ctx, TALLY_RELAY, verdict, in->n, in->mem);
     return rc;
     BNK_API_CATCH(ctx)
 }

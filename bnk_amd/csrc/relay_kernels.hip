@@ -22,15 +22,58 @@ namespace bnk {
 
 constexpr uint32_t NO_PEER = 0xFFFFFFFFu;
 
-// Four packets a thread, and each array in one access where they all lie so that it can be (four
-// byte loads and stores a packet otherwise: 2^22 packets 20 us against 11.5).
-template <bool ALIGNED>
-__global__ __launch_bounds__(256) void relay_verdict_kernel(
-    const uint8_t *auth, const uint8_t *pass, const uint32_t *peer_out, uint32_t n_peers_out,
-    uint32_t n, uint32_t *keys, uint32_t *idx, uint8_t *verdict, uint64_t *ctr_out, uint32_t *status)
+// What a relayed packet's verdict and key come from, and where they go: keys[] is the outbound peer of each
+// survivor and all ones for the rest.  tally: null, or the launch counts the verdicts.
+// (With a launch of their own for the verdicts and one that counted them at the end, relayed batches of 1000
+// packets with three streams at work took 17.3 us against 12.6, of 4000 22.5 against 18.6, of 100000 76.5
+// against 74.4.)
+struct RelayIn {
+    const uint8_t *auth, *pass;
+    const uint32_t *peer_out;
+    uint8_t *verdict;
+    uint32_t *keys;
+    uint32_t *status;
+    unsigned long long *tally;
+};
+
+// The verdict of a packet of the batch, and its key.
+__device__ __forceinline__ uint8_t relay_verdict(const RelayIn &in, uint8_t auth, uint8_t pass, uint32_t n_peers_out, uint32_t &key)
 {
+    uint8_t v = !auth ? BNK_RELAY_FORGED : !pass ? BNK_RELAY_DENIED : BNK_RELAY_OK;
+    if (v == BNK_RELAY_OK && key >= n_peers_out) {
+        status_raise(in.status, STATUS_PEER_RANGE);
+        v = BNK_RELAY_DENIED;
+    }
+    if (v != BNK_RELAY_OK) key = NO_PEER;
+    return v;
+}
+
+// The votes of a wave, one a lane (there: it has one), added to what it has of the three verdicts.
+__device__ __forceinline__ void relay_vote(uint8_t v, bool there, uint32_t (&votes)[3])
+{
+    votes[0] += (uint32_t)__popcll(__ballot(there && v == BNK_RELAY_OK));
+    votes[1] += (uint32_t)__popcll(__ballot(there && v == BNK_RELAY_FORGED));
+    votes[2] += (uint32_t)__popcll(__ballot(there && v == BNK_RELAY_DENIED));
+}
+__device__ __forceinline__ void relay_tally(unsigned long long *tally, const uint32_t (&votes)[3])
+{
+    tally_bump(tally, TALLY_RELAYED, votes[0]);
+    tally_bump(tally, TALLY_REJECTED, votes[1]);
+    tally_bump(tally, TALLY_DENIED, votes[2]);
+}
+
+// Four packets a thread, and each array in one access where they all lie so that it can be (four
+// byte loads and stores a packet otherwise: 2^22 packets 20 us against 11.5).  For batches whose counters
+// come from a sort; the others' first launch does this along the way (rank_count_tile, peer_rank_rows).
+template <bool ALIGNED>
+__global__ __launch_bounds__(256) void relay_verdict_kernel(RelayIn in, uint32_t n_peers_out, uint32_t n, uint32_t *idx, uint64_t *ctr_out)
+{
+    const uint8_t *const auth = in.auth, *const pass = in.pass;
+    const uint32_t *const peer_out = in.peer_out;
+    uint32_t *const keys = in.keys;
+    uint8_t *const verdict = in.verdict;
     const uint32_t first = (blockIdx.x * 256u + threadIdx.x) * 4u;
-    if (first >= n) return;
+    if (__ballot(first < n) == 0ull) return;
     const bool whole = ALIGNED && has_from(first, 4u, n);
     alignas(4) uint8_t au[4], pa[4], v[4];
     alignas(16) uint32_t key[4];
@@ -49,13 +92,15 @@ __global__ __launch_bounds__(256) void relay_verdict_kernel(
     }
 #pragma unroll
     for (uint32_t j = 0; j < 4; j++) {
-        v[j] = !au[j] ? BNK_RELAY_FORGED : !pa[j] ? BNK_RELAY_DENIED : BNK_RELAY_OK;
-        if (v[j] == BNK_RELAY_OK && key[j] >= n_peers_out && first + j < n) {
-            status_raise(status, STATUS_PEER_RANGE);
-            v[j] = BNK_RELAY_DENIED;
-        }
-        if (v[j] != BNK_RELAY_OK) key[j] = NO_PEER;
+        v[j] = relay_verdict(in, au[j], pa[j], n_peers_out, key[j]); // (beyond the end: the last packet's again)
     }
+    if (in.tally) {
+        uint32_t votes[3] = {0, 0, 0};
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) relay_vote(v[j], first < n && first + j < n, votes);
+        if ((threadIdx.x & 63u) == 0u) relay_tally(in.tally, votes);
+    }
+    if (first >= n) return;
     if (whole) {
         *reinterpret_cast<uint32_t *>(verdict + first) = *reinterpret_cast<const uint32_t *>(v);
         *reinterpret_cast<uint4 *>(keys + first) = *reinterpret_cast<const uint4 *>(key);
@@ -68,11 +113,8 @@ __global__ __launch_bounds__(256) void relay_verdict_kernel(
             verdict[i] = v[j];
             keys[i] = key[j];
         }
-        // (the counting kernels need no positions and write every packet's counter themselves)
-        if (idx) {
-            idx[i] = i;
-            ctr_out[i] = 0;
-        }
+        idx[i] = i;
+        ctr_out[i] = 0;
     }
 }
 
@@ -183,31 +225,37 @@ static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_ke
 static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &plan, void *tmp,
                                          uint64_t *ctr_base, uint32_t n_keys, uint32_t n, uint64_t *ctr_out,
                                          bool advance, uint64_t ctr_limit, bool zero_others, uint32_t *status,
-                                         hipStream_t s);
+                                         const RelayIn *relay, hipStream_t s);
+static hipError_t launch_relay_rank_rows(const RelayIn &in, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
+                                         bool advance, hipStream_t s);
+
+// The form for a batch of one workgroup: a packet a thread, four, or rows.
+enum RankForm : uint32_t { RANK_SMALL, RANK_BLOCK, RANK_ROWS };
+static RankForm rank_form(uint32_t n, uint32_t n_keys)
+{
+    return n_keys < ROW_DIGITS ? RANK_ROWS : n <= PEER_RANK_SMALL_MAX ? RANK_SMALL : RANK_BLOCK;
+}
 
 hipError_t launch_relay_assign(const uint8_t *auth, const uint8_t *pass, const uint32_t *peer_out,
                                const uint64_t *ctr_base_out, uint32_t n_peers_out, uint32_t n,
                                uint32_t *keys, uint32_t *idx, uint32_t *skeys, uint32_t *sidx,
                                void *sort_tmp, size_t sort_tmp_bytes, uint8_t *verdict,
-                               uint64_t *ctr_out, uint32_t *status, bool advance, hipStream_t s)
+                               uint64_t *ctr_out, uint32_t *status, unsigned long long *tally, bool advance, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     const RankPlan plan = rank_plan(n, n_peers_out);
     const bool one_block = peer_rank_one_block(n, n_peers_out);
-    const bool counting = !one_block && plan.fits && plan.bytes <= sort_tmp_bytes;
+    const RelayIn in{auth, pass, peer_out, verdict, keys, status, tally};
+    uint64_t *const ctr_base = const_cast<uint64_t *>(ctr_base_out);
+    if (one_block && rank_form(n, n_peers_out) == RANK_ROWS) return launch_relay_rank_rows(in, n_peers_out, n, ctr_base, ctr_out, advance, s);
+    if (!one_block && plan.fits && plan.bytes <= sort_tmp_bytes)
+        return launch_peer_rank_table(keys, plan, sort_tmp, ctr_base, n_peers_out, n, ctr_out, advance, 0ull, true, nullptr, &in, s);
     const bool aligned = (((uintptr_t)auth | (uintptr_t)pass | (uintptr_t)verdict) & 3u) == 0 &&
                          (((uintptr_t)peer_out | (uintptr_t)keys) & 15u) == 0;
     hipLaunchKernelGGL(aligned ? relay_verdict_kernel<true> : relay_verdict_kernel<false>, dim3(n / 1024u + (n % 1024u != 0u)), dim3(256), 0, s,
-                       auth, pass, peer_out, n_peers_out, n, keys, counting ? (uint32_t *)nullptr : idx, verdict, ctr_out, status);
-    // (keys[] is the peer of each survivor and all ones for the rest)
-    if (one_block)
-        return launch_peer_rank_one_block(keys, n_peers_out, n, const_cast<uint64_t *>(ctr_base_out), ctr_out, advance,
-                                          true, 0ull, status, s);
-    if (counting)
-        return launch_peer_rank_table(keys, plan, sort_tmp, const_cast<uint64_t *>(ctr_base_out), n_peers_out, n,
-                                      ctr_out, advance, 0ull, true, nullptr, s);
-    return launch_peer_rank(keys, idx, skeys, sidx, sort_tmp, sort_tmp_bytes,
-                            const_cast<uint64_t *>(ctr_base_out), n_peers_out, n, ctr_out, advance, 0ull, s);
+                       in, n_peers_out, n, idx, ctr_out);
+    if (one_block) return launch_peer_rank_one_block(keys, n_peers_out, n, ctr_base, ctr_out, advance, true, 0ull, status, s);
+    return launch_peer_rank(keys, idx, skeys, sidx, sort_tmp, sort_tmp_bytes, ctr_base, n_peers_out, n, ctr_out, advance, 0ull, s);
 }
 
 // The batch-order counters of a small batch, by one workgroup.
@@ -341,7 +389,9 @@ BNK_DEV void peer_rank_block(const RankArgs &a)
 
 // The same without a sort (block_rows.hpp), for tables of fewer than ROW_DIGITS peers.
 static_assert(PEER_BLOCK_THREADS == ROW_THREADS && PEER_RANK_BLOCK_MAX == ROW_PACKETS, "one launch shape");
-BNK_DEV void peer_rank_rows(const RankArgs &a)
+// RELAY: of a relay's batch, whose verdicts come first (a.peer is not read).
+template <bool RELAY>
+BNK_DEV void peer_rank_rows(const RankArgs &a, const RelayIn &in)
 {
     __shared__ uint32_t count[ROW_WAVES][ROW_DIGITS];
     __shared__ uint64_t base[ROW_DIGITS];
@@ -352,7 +402,32 @@ BNK_DEV void peer_rank_rows(const RankArgs &a)
 #pragma unroll
     for (uint32_t j = 0; j < ROWS_MOST; j++) {
         const uint32_t i = row_place(rows, j);
-        key[j] = j < rows && i < a.n ? (a.peer ? a.peer[i] : 0u) : NO_PEER;
+        if (!RELAY) key[j] = j < rows && i < a.n ? (a.peer ? a.peer[i] : 0u) : NO_PEER;
+    }
+    if (RELAY) {
+        uint8_t au[ROWS_MOST], pa[ROWS_MOST];
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            const uint32_t i = min(row_place(rows, j), a.n - 1u);
+            au[j] = in.auth[i];
+            pa[j] = in.pass[i];
+            key[j] = in.peer_out[i];
+        }
+        uint32_t votes[3] = {0, 0, 0};
+#pragma unroll
+        for (uint32_t j = 0; j < ROWS_MOST; j++) {
+            const uint32_t i = row_place(rows, j);
+            const bool there = j < rows && i < a.n;
+            const uint8_t v = relay_verdict(in, au[j], pa[j], a.n_keys, key[j]); // (elsewhere: the last packet's again)
+            if (there) {
+                in.verdict[i] = v;
+                if (key[j] == NO_PEER) a.ctr_out[i] = 0;
+            } else {
+                key[j] = NO_PEER;
+            }
+            if (in.tally) relay_vote(v, there, votes);
+        }
+        if (in.tally && lane == 0u) relay_tally(in.tally, votes);
     }
     uint64_t was = 0;
     if (t < a.n_keys) was = a.ctr_base[t];
@@ -365,7 +440,7 @@ BNK_DEV void peer_rank_rows(const RankArgs &a)
     for (uint32_t j = 0; j < ROWS_MOST; j++) {
         if (j >= rows) break; // (the same for every lane)
         if (key[j] >= a.n_keys) {
-            if (row_place(rows, j) < a.n && !(a.no_peer_ok && key[j] == NO_PEER)) status_raise(a.status, STATUS_PEER_RANGE);
+            if (!RELAY && row_place(rows, j) < a.n && !(a.no_peer_ok && key[j] == NO_PEER)) status_raise(a.status, STATUS_PEER_RANGE);
             key[j] = none;
         }
         const unsigned long long same = row_same(key[j], ROW_BITS);
@@ -396,20 +471,16 @@ BNK_DEV void peer_rank_rows(const RankArgs &a)
         if (j < rows && key[j] != none) a.ctr_out[row_place(rows, j)] = ctr_add(base[key[j]], mine[key[j]] + rank[j], a.ctr_limit);
 }
 
-// The form for a batch: a packet a thread, four, or rows.
-enum RankForm : uint32_t { RANK_SMALL, RANK_BLOCK, RANK_ROWS };
-static RankForm rank_form(uint32_t n, uint32_t n_keys)
-{
-    return n_keys < ROW_DIGITS ? RANK_ROWS : n <= PEER_RANK_SMALL_MAX ? RANK_SMALL : RANK_BLOCK;
-}
 template <uint32_t FORM>
 BNK_DEV void peer_rank(const RankArgs &a)
 {
-    FORM == RANK_ROWS ? peer_rank_rows(a) : FORM == RANK_SMALL ? peer_rank_small(a) : peer_rank_block(a);
+    FORM == RANK_ROWS ? peer_rank_rows<false>(a, RelayIn{}) : FORM == RANK_SMALL ? peer_rank_small(a) : peer_rank_block(a);
 }
 
 template <uint32_t FORM>
 __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_kernel(RankArgs a) { peer_rank<FORM>(a); }
+
+__global__ __launch_bounds__(PEER_BLOCK_THREADS) void relay_rank_rows_kernel(RankArgs a, RelayIn in) { peer_rank_rows<true>(a, in); }
 
 // NoteOutbound on the packets of such a batch as well, which has nothing to do with its counters: the
 // first workgroup ranks, the second does what a note launch does once, the others note.  In launches of
@@ -442,6 +513,14 @@ static hipError_t launch_peer_rank_one_block(const uint32_t *peer, uint32_t n_ke
     const RankArgs a{peer, n_keys, n, ctr_base, ctr_out, advance ? 1 : 0, no_peer_ok ? 1 : 0, key_bits(n_keys), ctr_limit, status};
     void (*const kernels[])(RankArgs) = {peer_rank_kernel<RANK_SMALL>, peer_rank_kernel<RANK_BLOCK>, peer_rank_kernel<RANK_ROWS>};
     hipLaunchKernelGGL(kernels[rank_form(n, n_keys)], dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, a);
+    return hipGetLastError();
+}
+
+static hipError_t launch_relay_rank_rows(const RelayIn &in, uint32_t n_keys, uint32_t n, uint64_t *ctr_base, uint64_t *ctr_out,
+                                         bool advance, hipStream_t s)
+{
+    const RankArgs a{nullptr, n_keys, n, ctr_base, ctr_out, advance ? 1 : 0, 1, key_bits(n_keys), 0ull, in.status};
+    hipLaunchKernelGGL(relay_rank_rows_kernel, dim3(1), dim3(PEER_BLOCK_THREADS), 0, s, a, in);
     return hipGetLastError();
 }
 
@@ -504,9 +583,10 @@ __device__ __forceinline__ void tile_words(const uint32_t *words, uint32_t first
     for (uint32_t r = 0; r < RUNS; r++) word[r] = words[min(first + r * 64u + threadIdx.x, end - 1u)];
 }
 
-template <bool SHIFTED, uint32_t RUNS>
+// RELAY: of a relay's batch, whose verdicts come first, and whose keys[] are written here.
+template <bool SHIFTED, bool RELAY, uint32_t RUNS>
 __device__ __forceinline__ void rank_count_tile(uint32_t tile, const uint32_t *keys, uint32_t n, uint32_t n_keys, uint32_t cols,
-                                                uint32_t runs, uint32_t *table, uint32_t *status, unsigned shift)
+                                                uint32_t runs, uint32_t *table, uint32_t *status, unsigned shift, const RelayIn &in)
 {
     __shared__ __attribute__((aligned(16))) uint32_t cnt[RANK_TABLE_MAX_KEYS];
     const uint32_t lane = threadIdx.x;
@@ -514,7 +594,29 @@ __device__ __forceinline__ void rank_count_tile(uint32_t tile, const uint32_t *k
     for (uint32_t q = lane; q < cols / 4u; q += 64u) cnt4[q] = make_uint4(0, 0, 0, 0);
     const uint32_t first = tile * runs * 64u, end = min(n, first + runs * 64u);
     uint32_t word[RUNS];
-    tile_words(keys, first, end, word);
+    tile_words(RELAY ? in.peer_out : keys, first, end, word);
+    if (RELAY) {
+        uint8_t au[RUNS], pa[RUNS];
+#pragma unroll
+        for (uint32_t r = 0; r < RUNS; r++) {
+            const uint32_t i = min(first + r * 64u + lane, end - 1u);
+            au[r] = in.auth[i];
+            pa[r] = in.pass[i];
+        }
+        uint32_t votes[3] = {0, 0, 0};
+#pragma unroll
+        for (uint32_t r = 0; r < RUNS; r++) {
+            if (first + r * 64u >= end) break; // (the same for every lane)
+            const uint32_t i = first + r * 64u + lane;
+            const uint8_t v = relay_verdict(in, au[r], pa[r], n_keys, word[r]); // (beyond the end: the last packet's again)
+            if (i < end) {
+                in.verdict[i] = v;
+                in.keys[i] = word[r];
+            }
+            if (in.tally) relay_vote(v, i < end, votes);
+        }
+        if (in.tally && lane == 0u) relay_tally(in.tally, votes);
+    }
     __syncthreads();
 #pragma unroll
     for (uint32_t r = 0; r < RUNS; r++) {
@@ -534,7 +636,13 @@ __global__ __launch_bounds__(64) void rank_count_kernel(const uint32_t *keys, ui
                                                         uint32_t cols, uint32_t runs, uint32_t *table,
                                                         uint32_t *status, unsigned shift)
 {
-    rank_count_tile<SHIFTED, RUNS>(blockIdx.x, keys, n, n_keys, cols, runs, table, status, shift);
+    rank_count_tile<SHIFTED, false, RUNS>(blockIdx.x, keys, n, n_keys, cols, runs, table, status, shift, RelayIn{});
+}
+
+template <uint32_t RUNS>
+__global__ __launch_bounds__(64) void relay_count_kernel(RelayIn in, uint32_t n, uint32_t n_keys, uint32_t cols, uint32_t runs, uint32_t *table)
+{
+    rank_count_tile<false, true, RUNS>(blockIdx.x, nullptr, n, n_keys, cols, runs, table, nullptr, 0u, in);
 }
 
 // One block per 16 peers: 64 groups of threads share the tiles between them.
@@ -787,7 +895,7 @@ __global__ __launch_bounds__(64) void rank_count_whole_kernel(WholeArgs a, Filte
 {
     const uint32_t b = blockIdx.x;
     if (b < a.tiles) {
-        rank_count_tile<false, RUNS>(b, a.keys, a.n, a.n_keys, a.cols, a.runs, a.table, a.status, 0u);
+        rank_count_tile<false, false, RUNS>(b, a.keys, a.n, a.n_keys, a.cols, a.runs, a.table, a.status, 0u, RelayIn{});
     } else if (b == a.tiles) {
         for (uint32_t k = threadIdx.x; k < a.n_keys; k += 64u) a.base_was[k] = a.ctr_base[k];
     } else if (b == a.tiles + 1u) {
@@ -797,6 +905,15 @@ __global__ __launch_bounds__(64) void rank_count_whole_kernel(WholeArgs a, Filte
         if (i < note.n) note_packet(note, i);
         note_block_done(note);
     }
+}
+
+// The same of a relay's batch, with its verdicts.
+template <uint32_t RUNS>
+__global__ __launch_bounds__(64) void relay_count_whole_kernel(WholeArgs a, RelayIn in)
+{
+    if (blockIdx.x < a.tiles) rank_count_tile<false, true, RUNS>(blockIdx.x, nullptr, a.n, a.n_keys, a.cols, a.runs, a.table, nullptr, 0u, in);
+    else
+        for (uint32_t k = threadIdx.x; k < a.n_keys; k += 64u) a.base_was[k] = a.ctr_base[k];
 }
 
 // Workgroups: the tiles, one that moves the peers' counters (with advance), the sweep's.
@@ -925,13 +1042,15 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
 // note: null, or the batch's NoteOutbound, with the sweep behind it.
 static hipError_t launch_peer_rank_whole(const uint32_t *keys, const RankPlan &plan, void *tmp, uint64_t *ctr_base, uint32_t n_keys,
                                          uint32_t n, uint64_t *ctr_out, bool advance, uint64_t ctr_limit, bool zero_others,
-                                         uint32_t *status, const FilterArgs *note, const SweepArgs &sweep, hipStream_t s)
+                                         uint32_t *status, const FilterArgs *note, const SweepArgs &sweep, const RelayIn *relay,
+                                         hipStream_t s)
 {
     uint32_t *const table = static_cast<uint32_t *>(tmp);
     uint64_t *const base_was = reinterpret_cast<uint64_t *>(table + (size_t)plan.tiles * plan.cols);
     const WholeArgs a{keys, n, n_keys, plan.cols, plan.runs, plan.tiles, table, ctr_base, base_was, status};
     const uint32_t noting = note ? 1u + (note->n + 63u) / 64u : 0u;
-    hipLaunchKernelGGL(rank_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + noting), dim3(64), 0, s, a, note ? *note : FilterArgs{});
+    if (relay) hipLaunchKernelGGL(relay_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u), dim3(64), 0, s, a, *relay);
+    else hipLaunchKernelGGL(rank_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + noting), dim3(64), 0, s, a, note ? *note : FilterArgs{});
     hipLaunchKernelGGL(rank_assign_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + sweep.blocks), dim3(WHOLE_THREADS), 0, s, a,
                        key_bits(n_keys), ctr_out, ctr_limit, zero_others ? 1 : 0, advance ? 1 : 0, sweep);
     return hipGetLastError();
@@ -953,25 +1072,28 @@ hipError_t launch_peer_rank_counting_note(const uint32_t *peer, void *tmp, uint6
     FilterArgs f = note;
     const SweepArgs sweep = flow_sweep_args(f, max_blocks, claimed_upper);
     f.record_blocks = f.record && f.record_after && sweep.blocks == 0u ? (n + 63u) / 64u : 0u;
-    return launch_peer_rank_whole(peer, plan, tmp, ctr_base, n_keys, n, ctr_out, true, ctr_limit, true, status, &f, sweep, s);
+    return launch_peer_rank_whole(peer, plan, tmp, ctr_base, n_keys, n, ctr_out, true, ctr_limit, true, status, &f, sweep, nullptr, s);
 }
 
 static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &plan, void *tmp,
                                          uint64_t *ctr_base, uint32_t n_keys, uint32_t n, uint64_t *ctr_out,
                                          bool advance, uint64_t ctr_limit, bool zero_others, uint32_t *status,
-                                         hipStream_t s)
+                                         const RelayIn *relay, hipStream_t s)
 {
     RankPlan whole = plan;
     if (rank_whole_plan(n, n_keys, whole))
         return launch_peer_rank_whole(keys, whole, tmp, ctr_base, n_keys, n, ctr_out, advance, ctr_limit, zero_others, status, nullptr,
-                                      SweepArgs{}, s);
+                                      SweepArgs{}, relay, s);
     uint32_t *table = static_cast<uint32_t *>(tmp);
     uint32_t *total = table + (size_t)plan.tiles * plan.cols;
     uint64_t *base_was = reinterpret_cast<uint64_t *>(total + plan.cols);
     const auto count = plan.runs <= TILE_RUNS_FEW ? rank_count_kernel<false, TILE_RUNS_FEW> : rank_count_kernel<false, TILE_RUNS_MAX>;
     const auto assign = plan.runs <= TILE_RUNS_FEW ? rank_assign_kernel<TILE_RUNS_FEW> : rank_assign_kernel<TILE_RUNS_MAX>;
-    hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
-                       table, status, 0u);
+    if (relay)
+        hipLaunchKernelGGL((plan.runs <= TILE_RUNS_FEW ? relay_count_kernel<TILE_RUNS_FEW> : relay_count_kernel<TILE_RUNS_MAX>), dim3(plan.tiles),
+                           dim3(64), 0, s, *relay, n, n_keys, plan.cols, plan.runs, table);
+    else
+        hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs, table, status, 0u);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS),
                        dim3(SCAN_PEERS * SCAN_PARTS), 0, s, table, plan.tiles, n_keys, plan.cols, total, ctr_base,
                        base_was, advance ? 1 : 0, ctr_limit);
@@ -993,7 +1115,7 @@ hipError_t launch_peer_rank_counting(const uint32_t *peer, void *tmp, uint64_t *
     if (n == 0) return hipSuccess;
     // (a packet whose peer lies beyond the table gets counter 0, as one without a peer does)
     return launch_peer_rank_table(peer, rank_plan(n, n_keys), tmp, ctr_base, n_keys, n, ctr_out, advance, ctr_limit,
-                                  true, status, s);
+                                  true, status, nullptr, s);
 }
 
 hipError_t launch_peer_rank(uint32_t *keys, uint32_t *idx, uint32_t *skeys, uint32_t *sidx,
@@ -1004,7 +1126,7 @@ hipError_t launch_peer_rank(uint32_t *keys, uint32_t *idx, uint32_t *skeys, uint
     const RankPlan plan = rank_plan(n, n_keys);
     if (plan.fits && plan.bytes <= sort_tmp_bytes)
         return launch_peer_rank_table(keys, plan, sort_tmp, ctr_base, n_keys, n, ctr_out, advance, ctr_limit, false,
-                                      nullptr, s);
+                                      nullptr, nullptr, s);
     const dim3 grid((n + 255u) / 256u);
     hipError_t e = rocprim::radix_sort_pairs<SortConfig>(sort_tmp, sort_tmp_bytes, keys, skeys, idx, sidx, (size_t)n,
                                              0, key_bits(n_keys), s);

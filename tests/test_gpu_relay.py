@@ -287,3 +287,47 @@ def test_relay_of_device_arrays_that_lie_anywhere(n, shift):
         assert (v[:shift] == 9).all() and v[shift + n] == 9
         assert np.array_equal(ctr_out.cpu().numpy().astype(np.uint64), want_c)
         assert np.array_equal(out.cpu().numpy(), want_out)
+
+
+@pytest.mark.parametrize("n,n_peers", [(70, 255), (700, 256), (4096, 64), (4097, 1024), (32769, 300), (9000, 1025)])
+def test_device_relay_of_every_form_of_the_counters(n, n_peers):
+    """Batches whose verdicts come with the ranks of one workgroup, with the counting launch of two or of
+    three, and ahead of a sort: outputs, verdicts and outbound counters against the oracle, and what the
+    context has counted against the verdicts."""
+    import torch
+    from bnk_amd import lib
+    from oracle import binding as O
+    w = W.relay_workload(n=n, n_peers=n_peers, n_rules=64)
+    b = w.batch
+    keys_in, keys_out = np.ascontiguousarray(b.keys), np.ascontiguousarray(w.keys_out)
+    sealed = np.zeros_like(b.plain)
+    O.seal_batch(keys_in, b.peer, b.counters, b.plain, b.off, b.lens, sealed, b.off, 4)
+    W.forge_tags(5, sealed, b.off, b.lens, w.forged_fraction)
+    ct_lens = (b.lens + 16).astype(np.uint32)
+    ora, ctx = O.Filter(), lib.Context(0)
+    ora.set_rules(w.rules_ref)
+    ctx.filter_set_rules(w.rules_ref)
+    ctx.keys_set(lib.KEYS_RECV, keys_in)
+    ctx.keys_set(lib.KEYS_SEND, keys_out)
+    _note(ctx, ora, w)
+    want_out = np.full_like(b.plain, 0x77)
+    want_v, want_c = ora.relay_fused_batch(keys_in, b.peer, b.counters, keys_out, w.peer_out, w.ctr_base_out, sealed, b.off,
+                                           ct_lens, want_out, b.off, w.now_ns)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")  # noqa: E731
+    i64, i32 = lambda a: d(a.astype(np.int64)), lambda a: d(a.view(np.int32))  # noqa: E731
+    off = i64(b.off)
+    got, v, c = d(np.full_like(b.plain, 0x77)), d(np.full(n, 9, np.uint8)), d(np.full(n, 123, np.int64))
+    arena, base, peer_out = d(sealed), d(w.ctr_base_out.view(np.int64)), i32(w.peer_out.astype(np.uint32))
+    more = dict(lens=i32(ct_lens), peer=i32(b.peer.astype(np.uint32)), counters=d(b.counters.view(np.int64)))
+    torch.cuda.synchronize()
+    ctx.counters_reset()
+    ctx.relay_fused(lib.make_batch(arena, sealed.nbytes, n, lib.MEM_DEVICE, offsets=off, **more), peer_out, base,
+                    len(w.ctr_base_out), w.now_ns, lib.make_batch(got, sealed.nbytes, n, lib.MEM_DEVICE, offsets=off), v, c)
+    ctx.sync()
+    assert np.array_equal(v.cpu().numpy(), want_v)
+    assert np.array_equal(c.cpu().numpy().view(np.uint64), want_c)
+    assert np.array_equal(got.cpu().numpy(), want_out)
+    seen = ctx.counters()
+    assert [seen["relayed"], seen["rejected"], seen["denied"]] == [int((want_v == k).sum()) for k in (0, 1, 2)]
+    assert ctx.filter_flows() == ora.flows()
+    ctx.close()

@@ -487,6 +487,12 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void relay_rank_rows_kernel(Ran
 // their own, one behind the other (4 us each, and 3 for the host to launch one), device-resident tunnel
 // passes of 256 packets took 31.7 us in a row against 29.1, of 3000 70.5 against 65.1; 128 packets in
 // pinned rings through the tunnel 67.5 against 63.7.
+//
+// A workgroup notes no more packets than one of its waves has lanes: the packets' headers are a line each,
+// over the link for a batch in a ring, and a compute unit has only so many of them in flight.  With 1024
+// a workgroup tunnel calls of 1024 packets in a ring took 162 us out and back against 154, of 2500 163.5
+// against 158, device-resident passes of 3000 50.0 against 47.6 in a row.
+constexpr uint32_t NOTE_PER_BLOCK = 64;
 template <uint32_t FORM>
 __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_note_kernel(RankArgs a, FilterArgs note)
 {
@@ -495,8 +501,8 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_note_kernel(Rank
     } else if (blockIdx.x == 1u) {
         if (threadIdx.x == 0u) note_once(note);
     } else {
-        const uint32_t i = (blockIdx.x - 2u) * PEER_BLOCK_THREADS + threadIdx.x;
-        if (i < note.n) note_packet(note, i);
+        const uint32_t i = (blockIdx.x - 2u) * NOTE_PER_BLOCK + threadIdx.x;
+        if (threadIdx.x < NOTE_PER_BLOCK && i < note.n) note_packet(note, i);
         note_block_done(note);
     }
 }
@@ -541,7 +547,7 @@ hipError_t launch_peer_rank_small_note(const uint32_t *peer, uint32_t n_keys, ui
     if (!peer_rank_one_block(n, n_keys) || note.n != n) return hipErrorInvalidValue;
     const RankArgs a{peer, n_keys, n, ctr_base, ctr_out, 1, 0, key_bits(n_keys), ctr_limit, status};
     FilterArgs f = note;
-    const uint32_t blocks = (n + PEER_BLOCK_THREADS - 1u) / PEER_BLOCK_THREADS;
+    const uint32_t blocks = (n + NOTE_PER_BLOCK - 1u) / NOTE_PER_BLOCK;
     f.record_blocks = f.record && f.record_after ? blocks : 0u;
     void (*const kernels[])(RankArgs, FilterArgs) = {peer_rank_note_kernel<RANK_SMALL>, peer_rank_note_kernel<RANK_BLOCK>,
                                                      peer_rank_note_kernel<RANK_ROWS>};

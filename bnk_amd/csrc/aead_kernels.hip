@@ -2094,7 +2094,7 @@ hipError_t launch_tunnel_seal_small(const AeadArgs &a, const TunnelSmall &t, con
                                     uint64_t claimed_upper, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    if (a.n > WG_WAVES_MAX || a.first != 0u || a.wg.mode != WG_FUSE_ENCAP || a.in_skip != 0u || (t.filter && f.n != a.n)) return hipErrorInvalidValue;
+    if (a.n > WG_RING_WAVES_MAX || a.first != 0u || a.wg.mode != WG_FUSE_ENCAP || a.in_skip != 0u || (t.filter && f.n != a.n)) return hipErrorInvalidValue;
     FilterArgs note = f;
     note.record_blocks = f.record && f.record_after ? 1u : 0u; // (the last workgroup leaves the record)
     const uint32_t blocks = (a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK;
@@ -2105,7 +2105,7 @@ hipError_t launch_tunnel_seal_small(const AeadArgs &a, const TunnelSmall &t, con
 hipError_t launch_tunnel_open_small(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    if (a.n > WG_WAVES_MAX || (a.n > WG_SMALL_MAX && a.wg.n_peers > WG_WAVES_PEERS) || a.first != 0u || a.wg.mode != WG_FUSE_DECAP || a.in_skip != 0u)
+    if (a.n > WG_RING_WAVES_MAX || (a.n > WG_SMALL_MAX && a.wg.n_peers > WG_WAVES_PEERS) || a.first != 0u || a.wg.mode != WG_FUSE_DECAP || a.in_skip != 0u)
         return hipErrorInvalidValue;
     const dim3 grid((a.n + WAVES_PER_BLOCK - 1u) / WAVES_PER_BLOCK);
     if (a.n > WG_SMALL_MAX) {

@@ -158,7 +158,7 @@ struct bnk_ctx {
     uint64_t *wg_replay = nullptr;
     uint32_t wg_replay_rows = 0;
     bnk::DevBuf wg_hash;      // receiver index -> row, hash table form
-    bnk::DevBuf wg_small;     // TunnelSmall::arrived and its records
+    bnk::DevBuf wg_small;     // TunnelSmall::arrived and its records; a ring batch's peers
     uint32_t wg_hash_bits = 0;
     uint32_t wg_replay_parity = 0; // WgReplayScratch::parity of the next pass over a large batch
     bool wg_replay_on = true;

@@ -491,9 +491,14 @@ int bnk::wg_encap_impl(bnk_ctx *ctx, const bnk_batch *slots, uint32_t mtu, uint3
         return se;
     };
 
-    // A small batch in one launch: counters, NoteOutbound and the packets.  (Every wave goes through the
-    // whole peer array, which of a batch in a ring lies in the host's staging.)
-    const bool small = n <= (ring_out ? WG_SMALL_MAX : WG_WAVES_MAX) && !chunked && !ctx->wg_unfused && aead_runs_spread(whole_slots(0, n));
+    // A small batch in one launch: counters, NoteOutbound and the packets.
+    const bool small = n <= (ring_out ? WG_RING_WAVES_MAX : WG_WAVES_MAX) && !chunked && !ctx->wg_unfused && aead_runs_spread(whole_slots(0, n));
+    if (small && ring_out && d_peer && n > WG_SMALL_MAX) {
+        // (every wave goes through the whole peer array, which of a batch in a ring lies in the host's staging)
+        uint8_t *const here = ctx->wg_small.as<uint8_t>() + WG_SMALL_PEERS + ((uintptr_t)d_peer & 15u);
+        HIPCHK(ctx, launch_pull(d_peer, here, (uint64_t)n * 4, ctx->stream));
+        d_peer = reinterpret_cast<const uint32_t *>(here);
+    }
     // counters in batch order per peer, advancing the peers' send counters:
     // needs the peer array only, so it runs ahead of the packet bytes
     if (small) {
@@ -956,7 +961,7 @@ int bnk::wg_decap_impl(bnk_ctx *ctx, const bnk_batch *wire, const bnk_batch *out
                 op.wg.out_len = d_out_len;
                 op.wg.peer_out = d_peer;
                 op.wg.counter_out = d_counter;
-                if (n <= (pe.n <= WG_WAVES_PEERS ? WG_WAVES_MAX : WG_SMALL_MAX) && !chunked && !ctx->wg_unfused && (replay || check)) {
+                if (n <= (pe.n > WG_WAVES_PEERS ? WG_SMALL_MAX : direct ? WG_RING_WAVES_MAX : WG_WAVES_MAX) && !chunked && !ctx->wg_unfused && (replay || check)) {
                     // a small batch in one launch, or two: the windows and CheckInbound as well
                     HIPCHK(ctx, launch_tunnel_open_small(op, small_view(ctx, check), check ? check_args(lo, hi) : FilterArgs{}, ctx->stream));
                     return BNK_OK;

@@ -1033,7 +1033,7 @@ hipError_t launch_wg_replay(uint8_t *result, uint32_t *out_len, const uint32_t *
 
 hipError_t launch_tunnel_open_rest(const AeadArgs &a, const TunnelSmall &t, const FilterArgs &f, hipStream_t s)
 {
-    static_assert(WG_WAVES_MAX <= ROW_PACKETS && WG_WAVES_PEERS == ROW_DIGITS - 1u, "one workgroup");
+    static_assert(WG_RING_WAVES_MAX <= ROW_PACKETS && WG_WAVES_PEERS == ROW_DIGITS - 1u, "one workgroup");
     hipLaunchKernelGGL(tunnel_rest_kernel, dim3(1), dim3(ROW_THREADS), 0, s, a, t, f);
     return hipGetLastError();
 }

@@ -240,28 +240,29 @@ BNK_DEV void encap_record(uint32_t *records, uint32_t i, uint32_t lane, uint32_t
     if (lane < 4u) record_put(records + WG_SMALL_RECORD * i + lane, v);
 }
 
-// The peers' counters moved, by WG_SMALL_MAX threads, PER packets each, whose records are on their way
+// The peers' counters moved, by WG_SMALL_MAX threads, PER packets each from packet `from` on, whose records are on their way
 // together: they come from beyond L2, and nothing else is left of the launch.
 template <uint32_t PER>
-BNK_DEV void counters_move(const TunnelSmall &t, uint32_t n, uint32_t n_peers)
+BNK_DEV void counters_move(const TunnelSmall &t, uint32_t from, uint32_t n, uint32_t n_peers)
 {
     uint32_t peer[PER];
     uint64_t next[PER];
 #pragma unroll
     for (uint32_t j = 0; j < PER; j++) {
-        const uint32_t *const r = t.records + WG_SMALL_RECORD * min(threadIdx.x + WG_SMALL_MAX * j, n - 1u);
+        const uint32_t *const r = t.records + WG_SMALL_RECORD * min(from + threadIdx.x + WG_SMALL_MAX * j, n - 1u);
         peer[j] = record_get(r);
         next[j] = __hip_atomic_load(reinterpret_cast<const uint64_t *>(r + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 #pragma unroll
     for (uint32_t j = 0; j < PER; j++)
-        if (threadIdx.x + WG_SMALL_MAX * j < n && peer[j] < n_peers) t.send_ctr[peer[j]] = next[j];
+        if (from + threadIdx.x + WG_SMALL_MAX * j < n && peer[j] < n_peers) t.send_ctr[peer[j]] = next[j];
 }
 
 template <bool MANY>
 BNK_DEV void encap_finish(const TunnelSmall &t, const FilterArgs &f, uint32_t n, uint32_t n_peers)
 {
-    counters_move<MANY ? WG_WAVES_MAX / WG_SMALL_MAX : 1u>(t, n, n_peers);
+    if (!MANY) counters_move<1>(t, 0u, n, n_peers);
+    else for (uint32_t from = 0; from < n; from += 8u * WG_SMALL_MAX) counters_move<8>(t, from, n, n_peers);
     // (FilterArgs::record_after: claims are atomics whose answers their waves have waited for)
     if (t.filter && threadIdx.x == 0u && f.record && f.record_after)
         __hip_atomic_store(f.record, (uint64_t)f.record_seq << 32 | atomicAdd(&f.flows.counters[FLOW_CLAIMED], 0u), __ATOMIC_RELAXED,

@@ -1835,3 +1835,46 @@ def test_small_tunnel_batches_in_one_launch(n, rules, mem):
         assert {lib.WG_OK, lib.WG_AUTH_FAIL, lib.WG_BAD_IP, lib.WG_FILTERED, lib.WG_REPLAY} <= seen
     for ctx, *_ in sides:
         ctx.close()
+
+
+@pytest.mark.parametrize("n,rules", [(300, "few"), (2048, "many"), (2049, "many"), (4095, "few"), (4096, "many"), (4097, "few")])
+def test_ring_batches_of_a_wave_per_packet(n, rules):
+    """Up to 4096 packets of a ring are encapsulated in one launch behind the one that fetches their peers,
+    and decapsulated in two: the checks are those of the test above."""
+    test_small_tunnel_batches_in_one_launch(n, rules, "ring")
+
+
+@pytest.mark.parametrize("n_peers", [1, 257])
+@pytest.mark.parametrize("first", [0, 1, 3])
+def test_ring_batches_of_many_peers_or_none(n_peers, first):
+    """A batch without a peer array, and one of more peers than the launch behind an open takes, whose peer
+    array starts at any place of 16 bytes: datagrams against the oracle, and back."""
+    from bnk_amd import lib
+    from oracle import binding as O
+    rng = np.random.default_rng(n_peers + first)
+    n, length, slot = 1021 + first, 100, 160
+    rows = [(5 + 3 * i, 5 + 3 * i, 0x64400000 + i, 0xFFFFFFFF) for i in range(n_peers)]
+    keys = rng.integers(0, 256, (n_peers, 32), dtype=np.uint8)
+    peer = rng.integers(0, n_peers, n).astype(np.uint32)
+    ctx = _ctx(rows, keys, keys)
+    ring, out = ctx.ring_alloc(n * slot), ctx.ring_alloc(n * slot)
+    ring[:] = 0
+    out[:] = 0
+    want, nxt = np.zeros(n * slot, np.uint8), np.zeros(n_peers, np.int64)
+    for i in range(n):
+        p = int(peer[i])
+        pt = _inner(rng, rows, p, length)
+        ring[i * slot + 16:i * slot + 16 + length] = np.frombuffer(pt, np.uint8)
+        want[i * slot:i * slot + 144] = np.frombuffer(O.wg_encap(pt, MTU, keys[p].tobytes(), rows[p][1], int(nxt[p])), np.uint8)
+        nxt[p] += 1
+    plain = np.array(ring).reshape(n, slot)[:, 16:16 + length].copy()
+    wl = np.zeros(n, np.uint32)
+    ctx.wg_encap(lib.make_batch(ring, n * slot, n, lib.MEM_HOST, stride=slot, length=length, peer=peer if n_peers > 1 else None), MTU, wl)
+    assert (wl == 144).all() and np.array_equal(np.array(ring), want)
+    assert np.array_equal(ctx.wg_send_counters(n_peers), nxt.astype(np.uint64))
+    res, olen, gp, gc = np.full(n, 99, np.uint8), np.zeros(n, np.uint32), np.zeros(n, np.uint32), np.zeros(n, np.uint64)
+    ctx.wg_decap(lib.make_batch(ring, n * slot, n, lib.MEM_HOST, stride=slot, length=144),
+                 lib.make_batch(out, n * slot, n, lib.MEM_HOST, stride=slot), res, olen, gp, gc)
+    assert (res == lib.WG_OK).all() and (olen == length).all() and np.array_equal(gp, peer)
+    assert np.array_equal(np.array(out).reshape(n, slot)[:, :length], plain)
+    ctx.close()

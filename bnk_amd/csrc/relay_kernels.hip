@@ -489,9 +489,9 @@ __global__ __launch_bounds__(PEER_BLOCK_THREADS) void relay_rank_rows_kernel(Ran
 // pinned rings through the tunnel 67.5 against 63.7.
 //
 // A workgroup notes no more packets than one of its waves has lanes: the packets' headers are a line each,
-// over the link for a batch in a ring, and a compute unit has only so many of them in flight.  With 1024
-// a workgroup tunnel calls of 1024 packets in a ring took 162 us out and back against 154, of 2500 163.5
-// against 158, device-resident passes of 3000 50.0 against 47.6 in a row.
+// and a compute unit has only so many of them in flight.  With 1024 a workgroup device-resident passes of
+// 3000 packets took 50.0 us in a row against 47.6; over the link (a ring's packets, as far as no wave of
+// their own notes them) a launch for 1024 took 34 us, and a pass 162 against 154.
 constexpr uint32_t NOTE_PER_BLOCK = 64;
 template <uint32_t FORM>
 __global__ __launch_bounds__(PEER_BLOCK_THREADS) void peer_rank_note_kernel(RankArgs a, FilterArgs note)

@@ -589,12 +589,18 @@ __device__ __forceinline__ void tile_words(const uint32_t *words, uint32_t first
     for (uint32_t r = 0; r < RUNS; r++) word[r] = words[min(first + r * 64u + threadIdx.x, end - 1u)];
 }
 
+// A row of the table, in as much LDS as its columns take: beside a launch of a lane per packet, which leaves
+// a compute unit 21 KiB, room for the longest row would be room for one wave of these.  With other streams at
+// work, against 16 KiB for every table: a relay of 2.7 million packets of 5 peers 1346 -> 1340 us, tunnel passes
+// of 2^18 packets of 1024 peers 440.7 -> 437.8, the relay of 4096 peers, whose rows are that long, the same.
+extern __shared__ __attribute__((aligned(16))) uint32_t rank_row[];
+
 // RELAY: of a relay's batch, whose verdicts come first, and whose keys[] are written here.
 template <bool SHIFTED, bool RELAY, uint32_t RUNS>
 __device__ __forceinline__ void rank_count_tile(uint32_t tile, const uint32_t *keys, uint32_t n, uint32_t n_keys, uint32_t cols,
                                                 uint32_t runs, uint32_t *table, uint32_t *status, unsigned shift, const RelayIn &in)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t cnt[RANK_TABLE_MAX_KEYS];
+    uint32_t *const cnt = rank_row;
     const uint32_t lane = threadIdx.x;
     uint4 *cnt4 = reinterpret_cast<uint4 *>(cnt);
     for (uint32_t q = lane; q < cols / 4u; q += 64u) cnt4[q] = make_uint4(0, 0, 0, 0);
@@ -748,7 +754,7 @@ __global__ __launch_bounds__(64) void rank_assign_kernel(const uint32_t *keys, u
                                                          uint64_t ctr_limit, int zero_others)
 {
     // packets of each peer ahead of the run at hand
-    __shared__ __attribute__((aligned(16))) uint32_t before[RANK_TABLE_MAX_KEYS];
+    uint32_t *const before = rank_row;
     const uint32_t lane = threadIdx.x;
     const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
     // keys and the peers' bases are fetched up front: nothing inside the walk below waits for memory
@@ -793,7 +799,7 @@ __global__ __launch_bounds__(64) void rank_place_kernel(const uint32_t *words, u
                                                         const uint32_t *total, unsigned bits, unsigned shift,
                                                         uint32_t *sorted)
 {
-    __shared__ __attribute__((aligned(16))) uint32_t before[RANK_TABLE_MAX_KEYS];
+    uint32_t *const before = rank_row;
     const uint32_t lane = threadIdx.x;
     const uint32_t first = blockIdx.x * runs * 64u, end = min(n, first + runs * 64u);
     uint32_t word[RUNS];
@@ -1027,7 +1033,7 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
     const uint32_t n_keys = n_peers + 1u;
     if (rank_whole_plan(n, n_keys, plan)) {
         uint32_t *const table = static_cast<uint32_t *>(tmp);
-        hipLaunchKernelGGL((rank_count_kernel<true, TILE_RUNS_FEW>), dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs,
+        hipLaunchKernelGGL((rank_count_kernel<true, TILE_RUNS_FEW>), dim3(plan.tiles), dim3(64), plan.cols * 4u, s, words, n, n_keys, plan.cols, plan.runs,
                            table, (uint32_t *)nullptr, shift);
         hipLaunchKernelGGL(rank_place_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles), dim3(WHOLE_THREADS), 0, s, words, n, n_keys, plan.cols,
                            plan.runs, plan.tiles, table, key_bits(n_keys), shift, sorted);
@@ -1036,11 +1042,11 @@ hipError_t launch_peer_sort(const uint32_t *words, uint32_t *sorted, uint32_t n,
     uint32_t *table = static_cast<uint32_t *>(tmp), *total = table + (size_t)plan.tiles * plan.cols;
     const auto count = plan.runs <= TILE_RUNS_FEW ? rank_count_kernel<true, TILE_RUNS_FEW> : rank_count_kernel<true, TILE_RUNS_MAX>;
     const auto place = plan.runs <= TILE_RUNS_FEW ? rank_place_kernel<TILE_RUNS_FEW> : rank_place_kernel<TILE_RUNS_MAX>;
-    hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+    hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), plan.cols * 4u, s, words, n, n_keys, plan.cols, plan.runs, table,
                        (uint32_t *)nullptr, shift);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS), dim3(SCAN_PEERS * SCAN_PARTS), 0, s,
                        table, plan.tiles, n_keys, plan.cols, total, (uint64_t *)nullptr, (uint64_t *)nullptr, 0, 0ull);
-    hipLaunchKernelGGL(place, dim3(plan.tiles), dim3(64), 0, s, words, n, n_keys, plan.cols, plan.runs, table,
+    hipLaunchKernelGGL(place, dim3(plan.tiles), dim3(64), plan.cols * 4u, s, words, n, n_keys, plan.cols, plan.runs, table,
                        total, key_bits(n_keys), shift, sorted);
     return hipGetLastError();
 }
@@ -1055,8 +1061,8 @@ static hipError_t launch_peer_rank_whole(const uint32_t *keys, const RankPlan &p
     uint64_t *const base_was = reinterpret_cast<uint64_t *>(table + (size_t)plan.tiles * plan.cols);
     const WholeArgs a{keys, n, n_keys, plan.cols, plan.runs, plan.tiles, table, ctr_base, base_was, status};
     const uint32_t noting = note ? 1u + (note->n + 63u) / 64u : 0u;
-    if (relay) hipLaunchKernelGGL(relay_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u), dim3(64), 0, s, a, *relay);
-    else hipLaunchKernelGGL(rank_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + noting), dim3(64), 0, s, a, note ? *note : FilterArgs{});
+    if (relay) hipLaunchKernelGGL(relay_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u), dim3(64), plan.cols * 4u, s, a, *relay);
+    else hipLaunchKernelGGL(rank_count_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + noting), dim3(64), plan.cols * 4u, s, a, note ? *note : FilterArgs{});
     hipLaunchKernelGGL(rank_assign_whole_kernel<TILE_RUNS_FEW>, dim3(plan.tiles + 1u + sweep.blocks), dim3(WHOLE_THREADS), 0, s, a,
                        key_bits(n_keys), ctr_out, ctr_limit, zero_others ? 1 : 0, advance ? 1 : 0, sweep);
     return hipGetLastError();
@@ -1097,13 +1103,13 @@ static hipError_t launch_peer_rank_table(const uint32_t *keys, const RankPlan &p
     const auto assign = plan.runs <= TILE_RUNS_FEW ? rank_assign_kernel<TILE_RUNS_FEW> : rank_assign_kernel<TILE_RUNS_MAX>;
     if (relay)
         hipLaunchKernelGGL((plan.runs <= TILE_RUNS_FEW ? relay_count_kernel<TILE_RUNS_FEW> : relay_count_kernel<TILE_RUNS_MAX>), dim3(plan.tiles),
-                           dim3(64), 0, s, *relay, n, n_keys, plan.cols, plan.runs, table);
+                           dim3(64), plan.cols * 4u, s, *relay, n, n_keys, plan.cols, plan.runs, table);
     else
-        hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs, table, status, 0u);
+        hipLaunchKernelGGL(count, dim3(plan.tiles), dim3(64), plan.cols * 4u, s, keys, n, n_keys, plan.cols, plan.runs, table, status, 0u);
     hipLaunchKernelGGL(rank_scan_kernel, dim3((n_keys + SCAN_PEERS - 1u) / SCAN_PEERS),
                        dim3(SCAN_PEERS * SCAN_PARTS), 0, s, table, plan.tiles, n_keys, plan.cols, total, ctr_base,
                        base_was, advance ? 1 : 0, ctr_limit);
-    hipLaunchKernelGGL(assign, dim3(plan.tiles), dim3(64), 0, s, keys, n, n_keys, plan.cols, plan.runs,
+    hipLaunchKernelGGL(assign, dim3(plan.tiles), dim3(64), plan.cols * 4u, s, keys, n, n_keys, plan.cols, plan.runs,
                        table, key_bits(n_keys), base_was, ctr_out, ctr_limit, zero_others ? 1 : 0);
     return hipGetLastError();
 }
